@@ -1,24 +1,7 @@
 // Matrix products over groups (one weight matrix per group: an expert and the tokens routed to it, or a head and
 // its slice of every token's row), the router's choice of experts, the sort of tokens by expert, the weighted sum
 // of the chosen experts' outputs, and the elementwise activation of a dense feed-forward.  Sums are float.
-#include "common.h"
-
-#define ACT_NONE 0
-#define ACT_RELU2 1
-#define ACT_SILU 2
-#define ACT_GELU_TANH 3
-#define ACT_GELU 4        // the exact form, with the error function
-#define ACT_PAIRS 16      // added to one of the above: the product's columns 2i and 2i + 1 are a gate and an up value, the output act(gate) * up
-
-__device__ __forceinline__ float activate(float v, int act) {
-    if (act == ACT_RELU2) { v = fmaxf(v, 0.f); return v * v; }
-    if (act == ACT_SILU) return v / (1.f + expf(-v));
-    if (act == ACT_GELU_TANH) return gelu_tanh(v);
-    if (act == ACT_GELU) return 0.5f * v * (1.f + erff(v * 0.7071067811865476f));
-    return v;
-}
-
-__host__ __device__ __forceinline__ bool known_activation(int act) { return (act & ~ACT_PAIRS) >= ACT_NONE && (act & ~ACT_PAIRS) <= ACT_GELU; }
+#include "direct_tile.h"
 
 // ------------------------------------------------------------------ grouped product
 // out[row(m), g_out + n] = act(sum_k a[src(m), g_a + k] * w[g][n][k]) for the rows m of group g, in tiles of 64 x 64
@@ -214,6 +197,195 @@ grouped_gemm_mfma_kernel(const bf16_t* __restrict__ a, int a_ld, int a_group, co
     }
 }
 
+// ------------------------------------------------------------------ products over the experts' rows (bfloat16, K a multiple of 64)
+// Two kernels beside the one above, which keeps the heads' products and what these refuse.
+//
+// Few rows per expert (a decode step): what counts is the stream of the weights, and a stream needs work-groups enough to have tens of KB on their
+// way from every compute unit.  A work-group owns a strip of 16 weight rows of one expert and up to 16 of its slots; its waves deal K out
+// in steps of 64 (a lane fetches 32 bytes of its weight row and of its x row, a row's 128 bytes lie in one line; the order of k inside a step is
+// the same for both operands and so does not matter), FEW_DEPTH steps on their way at once, and their sums meet in shared memory in the order of
+// the waves.  Slots beyond the group's are copies of its last one and are not stored.
+#define FEW_DEPTH 4
+
+template <int FEW_WAVES>
+__global__ void __launch_bounds__(FEW_WAVES * 64)
+experts_few_rows_kernel(const bf16_t* __restrict__ a, int a_ld, const int* __restrict__ src, const bf16_t* __restrict__ w, bf16_t* __restrict__ out,
+                        int out_ld, const int* __restrict__ offsets, int groups, int N, int K, int act) {
+    __shared__ __attribute__((aligned(16))) float red[FEW_WAVES][256];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, kg = lane >> 4;
+    // this work-group's tile among the groups', found by a prefix sum over the lanes
+    int g = -1, m0 = 0, m_end = 0, first = 0;
+    for (int base = 0; base < groups && g < 0; base += TL_WAVE) {
+        const int e = base + lane;
+        const int from = e < groups ? offsets[e] : 0, to = e < groups ? offsets[e + 1] : 0;
+        const int mine = (to - from + 15) / 16;
+        int upto = mine;
+#pragma unroll
+        for (int o = 1; o < TL_WAVE; o <<= 1) {
+            const int t = __shfl_up(upto, o, TL_WAVE);
+            if (lane >= o) upto += t;
+        }
+        const unsigned long long past = __ballot(first + upto > (int)blockIdx.y);
+        if (past) {
+            const int l = __builtin_amdgcn_readfirstlane(__ffsll(past) - 1);
+            g = base + l;
+            const int before = first + __builtin_amdgcn_readlane(upto, l) - __builtin_amdgcn_readlane(mine, l);
+            m0 = __builtin_amdgcn_readlane(from, l) + ((int)blockIdx.y - before) * 16;
+            m_end = __builtin_amdgcn_readlane(to, l);
+        }
+        first += __builtin_amdgcn_readlane(upto, TL_WAVE - 1);
+    }
+    if (g < 0) return;
+    const int n0 = blockIdx.x * 16;
+    const bf16_t* wrow = w + ((size_t)g * N + min(n0 + li, N - 1)) * K + 16 * kg;
+    const int mine = min(m0 + li, m_end - 1);
+    const bf16_t* xrow = a + (size_t)(src ? src[mine] : mine) * a_ld + 16 * kg;
+    f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const int steps = K / 64;
+    for (int s0 = wave; s0 < steps; s0 += FEW_WAVES * FEW_DEPTH) {
+        Frag16 wf[FEW_DEPTH][2], xf[FEW_DEPTH][2];
+#pragma unroll
+        for (int u = 0; u < FEW_DEPTH; ++u) {
+            const int k = min(s0 + u * FEW_WAVES, steps - 1) * 64;          // (beyond the end: fetched again, not used)
+            wf[u][0].u = *(const uint4*)(wrow + k);
+            wf[u][1].u = *(const uint4*)(wrow + k + 8);
+            xf[u][0].u = *(const uint4*)(xrow + k);
+            xf[u][1].u = *(const uint4*)(xrow + k + 8);
+        }
+#pragma unroll
+        for (int u = 0; u < FEW_DEPTH; ++u) {
+            if (s0 + u * FEW_WAVES < steps) {
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][0].v, xf[u][0].v, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][1].v, xf[u][1].v, acc, 0, 0, 0);
+            }
+        }
+    }
+    *(f32x4_t*)&red[wave][lane * 4] = acc;
+    __syncthreads();
+    if (wave > 0) return;
+    f32x4_t sum = acc;
+#pragma unroll
+    for (int v = 1; v < FEW_WAVES; ++v) sum += *(const f32x4_t*)&red[v][lane * 4];
+    // sum[v] = out[slot m0 + li][column n0 + 4 kg + v]
+    const int m = m0 + li, n = n0 + 4 * kg, base_act = act & ~ACT_PAIRS;
+    if (m >= m_end) return;
+    bf16_t* orow = out + (size_t)m * out_ld;
+    if (act & ACT_PAIRS) {
+#pragma unroll
+        for (int v = 0; v < 4; v += 2)
+            if (n + v + 1 < N) orow[(n + v) / 2] = from_float<bf16_t>(activate(sum[v], base_act) * sum[v + 1]);
+    } else {
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            if (n + v < N) orow[n + v] = from_float<bf16_t>(activate(sum[v], base_act));
+    }
+}
+
+// Many rows per expert (a prompt): the tile kernel with operands fetched straight into shared memory, over groups of rows.
+static int experts_units = 256;       // compute units the tiles are dealt to
+extern "C" void tl_experts_set_compute_units(int units) { if (units > 0) experts_units = units; }
+
+struct ExpertsCall {
+    const bf16_t* a;
+    int a_ld;
+    const int* src;
+    const bf16_t* w;
+    bf16_t* out;
+    int out_ld;
+    const int* offsets;
+    int groups, rows, N, K, act;
+};
+
+template <int WAVES>
+static int launch_experts_few(const ExpertsCall& c, hipStream_t stream) {
+    const dim3 grid((c.N + 15) / 16, c.rows / 16 + (c.groups < c.rows ? c.groups : c.rows));
+    experts_few_rows_kernel<WAVES><<<grid, WAVES * 64, 0, stream>>>(c.a, c.a_ld, c.src, c.w, c.out, c.out_ld, c.offsets, c.groups, c.N, c.K, c.act);
+    return TL_OK;
+}
+
+template <int BM, int BN, int WGM, int WGN, int STAGES, bool PAIRS>
+static int launch_experts_tile_t(const ExpertsCall& c, hipStream_t stream) {
+    constexpr size_t lds = (size_t)STAGES * dl_slab_rows(BM, BN, WGM * WGN, 64) * 64 * sizeof(bf16_t);
+    auto kernel = gemm_dl_tile_kernel<BM, BN, WGM, WGN, STAGES, bf16_t, 0, 64, ExpertRows<PAIRS>>;
+    static hipError_t allowed = allow_lds(kernel, lds);
+    if (allowed != hipSuccess) {
+        tl_set_error("experts_tile: cannot get %zu bytes of shared memory: %s", lds, hipGetErrorString(allowed));
+        return TL_ERR_HIP;
+    }
+    const long tiles = ((long)c.rows / BM + (c.groups < c.rows ? c.groups : c.rows)) * ((c.N + BN - 1) / BN);
+    kernel<<<dim3(tiles), 64 * WGM * WGN, lds, stream>>>(c.a, c.w, nullptr, 0, c.out, 0, c.N, c.K, c.a_ld, c.out_ld, 0, 0,
+                                                         ExpertRows<PAIRS>{c.offsets, c.src, c.groups, c.act});
+    return TL_OK;
+}
+
+template <int BM, int BN, int WGM, int WGN, int STAGES>
+static int launch_experts_tile(const ExpertsCall& c, hipStream_t stream) {
+    return c.act & ACT_PAIRS ? launch_experts_tile_t<BM, BN, WGM, WGN, STAGES, true>(c, stream) : launch_experts_tile_t<BM, BN, WGM, WGN, STAGES, false>(c, stream);
+}
+
+enum ExpertsKernel { EX_FEW_8, EX_FEW_4, EX_TILE_64x128, EX_TILE_128x128, EX_TILE_128x256, EX_TILE_256x256, EX_KERNELS };
+
+static int launch_experts(int which, const ExpertsCall& c, hipStream_t stream) {
+    int rc = TL_OK;
+    switch (which) {
+    case EX_FEW_8: rc = launch_experts_few<8>(c, stream); break;
+    case EX_FEW_4: rc = launch_experts_few<4>(c, stream); break;
+    case EX_TILE_64x128: rc = launch_experts_tile<64, 128, 1, 2, 3>(c, stream); break;
+    case EX_TILE_128x128: rc = launch_experts_tile<128, 128, 2, 2, 2>(c, stream); break;
+    case EX_TILE_128x256: rc = launch_experts_tile<128, 256, 2, 4, 3>(c, stream); break;
+    case EX_TILE_256x256: rc = launch_experts_tile<256, 256, 4, 2, 2>(c, stream); break;
+    default: TL_REQUIRE(false, "experts_gemm: no kernel %d", which);
+    }
+    if (rc != TL_OK) return rc;
+    TL_CHECK_LAUNCH("experts_gemm");
+    return TL_OK;
+}
+
+// Which kernel a call gets, by what the host knows: the slots of all groups together (how they are dealt to the groups only the GPU knows).
+//
+// Up to 8 slots a group on average (4 where K is beyond 2048: a strip's rows of x, read once per strip, outgrow the caches) the weights' stream
+// sets the time: the few-rows kernel, with waves enough to leave each a few steps of K.  Measured (us; few rows with 8 waves / with 4 / the
+// tiles of 64 x 128; groups x N x K, every call on other weights):
+//   16 x 1024 x 2048, 16 slots 11.8 / 13.8 / 20.9, 128 slots 17.7 / 20.9 / 22.1, 256 slots 26.4 / 26.7 / 22.5
+//   16 x 2048 x 1024, 16 slots 15.7 / 9.8 / 13.6, 64 slots 25.2 / 15.0 / 16.0, 128 slots 28.2 / 17.0 / 16.1, 256 slots 43.9 / 26.3 / 16.0
+//   32 x 4096 x 4096, 16 slots 77 / 82 / 84, 128 slots 181 / 191 / 178, 256 slots 208 / 213 / 179 (229 us at the rate of a large copy)
+// (the kernel without shared memory, which had these calls, took 37 us for the first and 134 at 4096 slots, where the tiles take 37).
+//
+// Beyond that, tiles: rounds of work-groups (two of the two smaller tiles to a compute unit) times a tile's time, fitted to single rounds at K of
+// 1024 and 2048; every group ends in a tile that is half empty on average.  Measured (us; 64 x 128 / 128 x 128 / 128 x 256 / 256 x 256):
+//   16 x 1024 x 2048, 2048 slots 35 / 36 / 37 / 50, 4096 slots 49 / 42 / 37 / 53, 16384 slots 121 / 110 / 92 / 107
+//   16 x 2048 x 1024, 2048 slots 31 / 25 / 23 / 31, 4096 slots 45 / 47 / 43 / 34, 16384 slots 134 / 110 / 104 / 95
+//   32 x 4096 x 4096, 2048 slots 219 / 192 / 190 / 254, 16384 slots 873 / 693 / 630 / 654
+static int pick_experts(const ExpertsCall& c) {
+    if ((long)c.rows <= (c.K > 2048 ? 4L : 8L) * c.groups) return c.K < 2048 ? EX_FEW_4 : EX_FEW_8;
+    static const struct { int kernel, bm, bn, per_unit; double fixed, per_k; } tiles[] = {
+        {EX_TILE_64x128, 64, 128, 2, 9e-6, 6.5e-6}, {EX_TILE_128x128, 128, 128, 2, 7e-6, 13e-6},
+        {EX_TILE_128x256, 128, 256, 1, 8e-6, 10.2e-6}, {EX_TILE_256x256, 256, 256, 1, 9e-6, 20e-6}};       // seconds of a tile: fixed, and per 1024 columns of K
+    int best = EX_TILE_64x128;
+    double best_t = 1e30;
+    for (const auto& t : tiles) {
+        const long groups = c.groups < c.rows ? c.groups : c.rows;
+        const long count = ((long)c.rows + groups * (t.bm / 2) + t.bm - 1) / t.bm * ((c.N + t.bn - 1) / t.bn), slots = (long)t.per_unit * experts_units;
+        const double est = (double)((count + slots - 1) / slots) * (t.fixed + t.per_k * c.K / 1024.0);
+        if (est < best_t) { best_t = est; best = t.kernel; }
+    }
+    return best;
+}
+
+static bool experts_fit(const ExpertsCall& c) {
+    // (a lane's offset from the first row of x, and of w from its tile's, is kept in 32 bits)
+    return c.K % 64 == 0 && c.a_ld % 8 == 0 && ((uintptr_t)c.a % 16) == 0 && ((uintptr_t)c.w % 16) == 0 && (long)c.rows * c.a_ld * 2 < (1L << 31) &&
+           256L * c.K * 2 < (1L << 31) && (long)(c.rows / 16 + c.groups) <= 65535;
+}
+
+// One named kernel of the two (tests cover each; tuning times them).
+extern "C" int tl_experts_variant(const void* a, int a_ld, const void* src, const void* w, void* out, int out_ld, const void* offsets, int groups, int rows,
+                                  int N, int K, int act, int which, hipStream_t stream) {
+    const ExpertsCall c{(const bf16_t*)a, a_ld, (const int*)src, (const bf16_t*)w, (bf16_t*)out, out_ld, (const int*)offsets, groups, rows, N, K, act};
+    TL_REQUIRE(groups > 0 && rows > 0 && N > 0 && K > 0 && offsets && known_activation(act) && (!(act & ACT_PAIRS) || N % 2 == 0) && experts_fit(c), "experts_variant: bad arguments");
+    return launch_experts(which, c, stream);
+}
+
 extern "C" int tl_grouped_gemm(const void* a, int a_ld, int a_group, const void* src, const void* w, void* out, int out_ld, int out_group,
                                const void* offsets, int groups, int rows, int N, int K, int act, const void* gate, int gate_ld, int dtype, int general,
                                hipStream_t stream) {
@@ -226,6 +398,8 @@ extern "C" int tl_grouped_gemm(const void* a, int a_ld, int a_group, const void*
     dim3 grid(offsets ? (rows + GG_T - 1) / GG_T + groups : (rows + GG_T - 1) / GG_T, (N + GG_T - 1) / GG_T, offsets ? 1 : groups), block(256);
     const bool aligned = K % 32 == 0 && a_ld % 8 == 0 && a_group % 8 == 0 && ((uintptr_t)a % 16) == 0 && ((uintptr_t)w % 16) == 0 &&
                          ((uintptr_t)out % 8) == 0;
+    const ExpertsCall experts{(const bf16_t*)a, a_ld, (const int*)src, (const bf16_t*)w, (bf16_t*)out, out_ld, (const int*)offsets, groups, rows, N, K, act};
+    if (dtype == TL_DT_BF16 && offsets && !general && experts_fit(experts)) return launch_experts(pick_experts(experts), experts, stream);
     if (dtype == TL_DT_BF16 && aligned && !general) {
         dim3 mgrid(offsets ? (rows + GM_BM - 1) / GM_BM + groups : (rows + GM_BM - 1) / GM_BM, (N + GM_BN - 1) / GM_BN, offsets ? 1 : groups);
         grouped_gemm_mfma_kernel<<<mgrid, block, 0, stream>>>((const bf16_t*)a, a_ld, a_group, (const int*)src, (const bf16_t*)w, (bf16_t*)out, out_ld,

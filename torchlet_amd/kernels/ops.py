@@ -45,6 +45,8 @@ def _lib(name: str) -> ctypes.CDLL:
             lib.tl_gemm_set_compute_units(c_int(compute_units()))
         if name == "recurrent" and torch.cuda.is_available():
             lib.tl_mlstm_set_compute_units(c_int(compute_units()))
+        if name == "experts" and torch.cuda.is_available():
+            lib.tl_experts_set_compute_units(c_int(compute_units()))
     return lib
 
 
@@ -1592,6 +1594,22 @@ def experts_linear(x: torch.Tensor, slot_token: torch.Tensor | None, weight: tor
     _check(lib, lib.tl_grouped_gemm(_ptr(x), c_int(x.stride(0)), c_int(0), _ptr(slot_token), _ptr(weight), _ptr(out), c_int(out.shape[1]), c_int(0),
                                     _ptr(offsets), c_int(G), c_int(S), c_int(N), c_int(K), c_int(ACTIVATIONS[activation]), c_void_p(0), c_int(0),
                                     c_int(_dt(x, "experts_linear")), c_int(1 if general else 0), _stream()))
+
+
+def experts_linear_variant(x: torch.Tensor, slot_token: torch.Tensor | None, weight: torch.Tensor, offsets: torch.Tensor, out: torch.Tensor,
+                           activation: str, which: int) -> None:
+    """:func:`experts_linear` with the kernel named (0, 1: few rows with 8 or 4 waves; 2 to 5: tiles of 64 x 128, 128 x 128, 128 x 256, 256 x 256),
+    for tests and tuning: bfloat16, K a multiple of 64."""
+    G, N, K = weight.shape
+    S, pairs = out.shape[0], ACTIVATIONS[activation] >= 16
+    if x.dtype != torch.bfloat16 or weight.dtype != x.dtype or out.dtype != x.dtype or x.stride(1) != 1 or x.shape[1] != K or out.shape != (S, N // 2 if pairs else N) \
+            or not out.is_contiguous() or not weight.is_contiguous() or (slot_token is None and x.shape[0] != S):
+        raise KernelError("experts_linear_variant: shapes or dtypes do not fit")
+    _i32(offsets, "offsets", G + 1)
+    _i32(slot_token, "slot_token", S)
+    lib = _lib("experts")
+    _check(lib, lib.tl_experts_variant(_ptr(x), c_int(x.stride(0)), _ptr(slot_token), _ptr(weight), _ptr(out), c_int(out.shape[1]), _ptr(offsets), c_int(G),
+                                       c_int(S), c_int(N), c_int(K), c_int(ACTIVATIONS[activation]), c_int(which), _stream()))
 
 
 ROUTER_SCORES = {"chosen": 0, "all": 1, "sigmoid": 2}
