@@ -519,14 +519,17 @@ extern "C" int tl_delta_prepare(const void* proj, int ld, const void* conv_w, vo
 //   S <- g S;   u = beta (v - S^T k);   S <- S + k u^T;   o = S^T q.
 // Column j of S needs only its own a_j = sum_r S[r][j] k[r] and b_j = sum_r S[r][j] q[r] (of the state before the decay) and k . q:
 //   u_j = beta (v_j - g a_j);   o_j = g b_j + (k . q) u_j;   S[r][j] <- g S[r][j] + k[r] u_j.
-// The 16 lanes of a row of the wave share a column: lane i of them owns the rows i RPL .. i RPL + RPL - 1 of it in registers for all
-// tokens of the step (RPL = 4, 8, 12 or 16, fixed by dim alone), and they add their sums with four exchanges inside the row (pairs,
-// quads, halves, the row: every lane gets the same bits).  The order of every sum is fixed by dim, so a token's result depends neither
-// on how its request was cut into steps nor on what else the step holds.  A wave has 4 columns, a work-group of four waves 16.  The
-// state of a head lies column by column ([vdim][dim]), so a lane's rows are side by side in memory and a wave fetches whole lines.
-// Tokens are taken TB at a time (1, 4 or 16, by the longest portion of the step): their q, k, v, beta and g go to shared memory (the
-// next batch is fetched into registers while this one is worked on) and every lane runs the TB updates of its rows; a request's last
-// batch is filled up with tokens that change nothing (k = 0, beta = 0, decay 1), so the loop has no branch.
+// The 16 lanes of a row of the wave share a column: lane i of them owns the rows 64 q + 4 i .. + 3 (q < RPL / 4; RPL = 4, 8, 12 or 16, fixed
+// by dim alone) of it in registers for all tokens of the step, so the lanes' pieces of q and k lie side by side in shared memory and those of
+// the state side by side in memory ([vdim][dim] per head), and they add their sums with four exchanges inside the row (pairs, quads, halves,
+// the row: every lane gets the same bits).  k . q, which all columns share, is made once a token.  The order of every sum is fixed by dim, so a
+// token's result depends neither on how its request was cut into steps nor on what else the step holds.  A wave has 4 CPL columns, a work-group
+// of four waves 16 CPL.  Tokens are taken TB at a time (1, 4 or 16, by the longest portion of the step): their q, k, v, beta and g are fetched
+// into registers one batch ahead, as whole pieces of four where the rows allow it, and go to shared memory; a request's last batch is filled up
+// with tokens that change nothing (k = 0, beta = 0, decay 1), so the loop has no branch.
+// What bounds it: a token is a chain (S -> a -> u -> S) of some 50 vector instructions a wave beside six reads of shared memory; the fetches and
+// their address arithmetic must stay small beside that (number by number, each under a condition of its own, they were five sixths of the
+// instructions and held a work-group at 256 registers).  Measured: see launch_delta_scan.
 #define DELTA_L 16
 #define DELTA_COLS 16           // columns of a work-group
 #define DELTA_TB 16
@@ -549,134 +552,208 @@ __device__ __forceinline__ float row16_sum(float v) {
 // head (`head_decay`) in place of the tokens' gates: the decayed linear attention.  MODE 2: without the correction, with the tokens' own
 // decays and step sizes, S <- g S + k (beta v)^T and o = S^T q + skip v with one skip factor per head (`head_decay` holds them): a
 // selective state-space recurrence (k: the input matrix's row B, q: the output matrix's row C, beta: the step size, v: the input).
-template <int RPL, int TB, int MODE>
-__global__ void __launch_bounds__(256)
+template <int RPL, int TB, int MODE, int CPL>
+__global__ void __launch_bounds__(256, RPL * CPL <= 16 ? 4 : 2)
 delta_scan_kernel(const float* __restrict__ qkv, const float* __restrict__ gates, const float* __restrict__ head_decay,
                   float* __restrict__ state, size_t slot_stride,
                   const int* __restrict__ slots, const int* __restrict__ req_indptr, float* __restrict__ out,
-                  int heads, int kv_heads, int dim, int vdim) {
-    constexpr int tb = TB;
-    extern __shared__ float smem[];
-    constexpr int ROWS = DELTA_L * RPL;                // >= dim
-    float* sq = smem;                                  // [tb][ROWS]
-    float* sk = sq + tb * ROWS;                        // [tb][ROWS]
-    float* sv = sk + tb * ROWS;                        // [tb][DELTA_COLS]
-    float* sg = sv + tb * DELTA_COLS;                  // [tb][2]: beta, decay
-    const int req = blockIdx.z, head = blockIdx.y, col0 = blockIdx.x * DELTA_COLS;
+                  int heads, int kv_heads, int dim, int vdim, int vec) {
+    constexpr int ROWS = DELTA_L * RPL, Q = RPL / 4, COLS = DELTA_COLS * CPL;          // ROWS >= dim
+    constexpr int PPT = ROWS / 4, NP = (TB * PPT + 255) / 256, NV = (TB * COLS + 255) / 256;      // pieces of four: per token, per thread and batch
+    __shared__ __attribute__((aligned(16))) float sq[TB * ROWS], sk[TB * ROWS], sg[TB * 4];       // sg: beta, decay, k . q
+    __shared__ float sv[TB * COLS];
+    const int req = blockIdx.z, head = blockIdx.y, col0 = blockIdx.x * COLS;
     const int tok0 = req_indptr[req], tok1 = req_indptr[req + 1];
     if (tok0 >= tok1) return;
-    const int wave = threadIdx.x / TL_WAVE, lane = threadIdx.x % TL_WAVE;
-    const int rg = lane & 15, cw = wave * 4 + (lane >> 4);       // the lane's group of rows and its column within the work-group
-    const int col = col0 + cw, row0 = rg * RPL;
-    const bool col_ok = col < vdim;
+    const int tid = threadIdx.x, wave = tid / TL_WAVE, lane = tid % TL_WAVE;
+    const int rg = lane & 15, cw = wave * 4 + (lane >> 4);       // the lane's place in its columns, and the first of them within the work-group
     const int C = 2 * kv_heads * dim + heads * vdim;
     const int qk_head = head / (heads / kv_heads);
     const int q_at = qk_head * dim, k_at = kv_heads * dim + qk_head * dim, v_at = 2 * kv_heads * dim + head * vdim + col0;
-    float* st = state + (size_t)slots[req] * slot_stride + ((size_t)head * vdim + col) * dim + row0;
+    float* st = state + (size_t)slots[req] * slot_stride + (size_t)head * vdim * dim;
 
-    float S[RPL];
-    const bool whole = col_ok && row0 + RPL <= dim && (dim & 3) == 0 && ((uintptr_t)state & 15) == 0 && (slot_stride & 3) == 0;
-    if (whole) {
+    float S[CPL][RPL];
+    const bool vec_state = (dim & 3) == 0 && ((uintptr_t)state & 15) == 0 && (slot_stride & 3) == 0;
 #pragma unroll
-        for (int r = 0; r < RPL; r += 4) {
-            const float4 x = *(const float4*)(st + r);
-            S[r] = x.x; S[r + 1] = x.y; S[r + 2] = x.z; S[r + 3] = x.w;
+    for (int c = 0; c < CPL; ++c) {
+        const int col = col0 + cw + c * DELTA_COLS;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int row = 64 * q + 4 * rg;
+            const float* from = st + (size_t)col * dim + row;
+            if (vec_state && col < vdim && row + 4 <= dim) {
+                const float4 x = *(const float4*)from;
+                S[c][4 * q] = x.x; S[c][4 * q + 1] = x.y; S[c][4 * q + 2] = x.z; S[c][4 * q + 3] = x.w;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) S[c][4 * q + e] = (col < vdim && row + e < dim) ? from[e] : 0.f;
+            }
         }
-    } else {
-#pragma unroll
-        for (int r = 0; r < RPL; ++r) S[r] = (col_ok && row0 + r < dim) ? st[r] : 0.f;
     }
 
-    // a batch's numbers, fetched into registers one batch ahead: per token 2 * ROWS of q and k (zeros beyond dim), 16 of v, 2 gates
-    constexpr int PER_TOKEN = 2 * ROWS + DELTA_COLS + 2;
-    constexpr int STAGE = (TB * PER_TOKEN + 255) / 256;
-    float stage[STAGE];
-    auto fetch = [&](int base) {
-        const int nb = min(tb, tok1 - base);
+    // The state is waited for here: left to the token loop, the wait at its head would be one for every fetch on its way, the next batch's too.
 #pragma unroll
-        for (int j = 0; j < STAGE; ++j) {
-            const int idx = threadIdx.x + j * 256;
-            float v = 0.f;
-            if (idx < TB * PER_TOKEN) {
-                const int t = idx / PER_TOKEN, e = idx % PER_TOKEN;
-                if (t < nb) {
-                    const float* row = qkv + (size_t)(base + t) * C;
-                    if (e < ROWS) v = e < dim ? row[q_at + e] : 0.f;
-                    else if (e < 2 * ROWS) v = e - ROWS < dim ? row[k_at + e - ROWS] : 0.f;
-                    else if (e < 2 * ROWS + DELTA_COLS) v = col0 + e - 2 * ROWS < vdim ? row[v_at + e - 2 * ROWS] : 0.f;
-                    else if (MODE != 0) v = gates[(size_t)(base + t) * 2 * heads + (e - 2 * ROWS - DELTA_COLS) * heads + head];
-                    else v = e == PER_TOKEN - 1 ? head_decay[head] : 1.f;
-                } else if (e == PER_TOKEN - 1) v = 1.f;        // beyond the request's last token: k = 0, beta = 0 and a decay of 1 leave the state as it is, to the bit
+    for (int c = 0; c < CPL; ++c)
+#pragma unroll
+        for (int r = 0; r < RPL; ++r) asm volatile("" : "+v"(S[c][r]));
+
+    float4 pq[NP], pk[NP];
+    float pv[NV], pg = 0.f;
+    auto fetch = [&](int base) {
+        const int nb = min(TB, tok1 - base);
+        if (vec && nb == TB && (TB * PPT) % 256 == 0) {           // whole pieces of whole tokens, and one for every thread
+#pragma unroll
+            for (int j = 0; j < NP; ++j) {
+                const int idx = tid + j * 256;
+                const float* row = qkv + (size_t)(base + idx / PPT) * C + (idx % PPT) * 4;
+                pq[j] = *(const float4*)(row + q_at);
+                pk[j] = *(const float4*)(row + k_at);
             }
-            stage[j] = v;
+        } else if (vec) {
+#pragma unroll
+            for (int j = 0; j < NP; ++j) {
+                const int idx = tid + j * 256, t = idx / PPT;
+                const float* row = qkv + (size_t)(base + t) * C + (idx % PPT) * 4;
+                pq[j] = pk[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (idx < TB * PPT && t < nb) {
+                    pq[j] = *(const float4*)(row + q_at);
+                    pk[j] = *(const float4*)(row + k_at);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < NP; ++j) {
+                const int idx = tid + j * 256, t = idx / PPT, e = (idx % PPT) * 4;
+                pq[j] = pk[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (idx < TB * PPT && t < nb && e < dim) {
+                    const float* row = qkv + (size_t)(base + t) * C + e;
+                    float a[4], b[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        a[u] = e + u < dim ? row[q_at + u] : 0.f;
+                        b[u] = e + u < dim ? row[k_at + u] : 0.f;
+                    }
+                    pq[j] = make_float4(a[0], a[1], a[2], a[3]);
+                    pk[j] = make_float4(b[0], b[1], b[2], b[3]);
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            const int idx = tid + j * 256, t = idx / COLS, c = idx % COLS;
+            pv[j] = (idx < TB * COLS && t < nb && col0 + c < vdim) ? qkv[(size_t)(base + t) * C + v_at + c] : 0.f;
+        }
+        if (tid < 2 * TB) {                            // beyond the request's last token: k = 0, beta = 0 and a decay of 1 leave the state as it is, to the bit
+            const int t = tid >> 1, which = tid & 1;
+            if (t >= nb) pg = which ? 1.f : 0.f;
+            else if (MODE != 0) pg = gates[(size_t)(base + t) * 2 * heads + which * heads + head];
+            else pg = which ? head_decay[head] : 1.f;
         }
     };
     const float skip = MODE == 2 ? head_decay[head] : 0.f;
     fetch(tok0);
-    for (int base = tok0; base < tok1; base += tb) {
-        const int nb = min(tb, tok1 - base);
-        __syncthreads();                               // the batch before has been worked on
+    for (int base = tok0; base < tok1; base += TB) {
+        const int nb = min(TB, tok1 - base);
+        shared_barrier();                              // the batch before has been worked on
 #pragma unroll
-        for (int j = 0; j < STAGE; ++j) {
-            const int idx = threadIdx.x + j * 256;
-            if (idx < TB * PER_TOKEN) {
-                const int t = idx / PER_TOKEN, e = idx % PER_TOKEN;
-                if (e < ROWS) sq[t * ROWS + e] = stage[j];
-                else if (e < 2 * ROWS) sk[t * ROWS + e - ROWS] = stage[j];
-                else if (e < 2 * ROWS + DELTA_COLS) sv[t * DELTA_COLS + e - 2 * ROWS] = stage[j];
-                else sg[t * 2 + e - 2 * ROWS - DELTA_COLS] = stage[j];
+        for (int j = 0; j < NP; ++j) {
+            const int idx = tid + j * 256;
+            if (idx < TB * PPT) {
+                *(float4*)(sq + idx * 4) = pq[j];
+                *(float4*)(sk + idx * 4) = pk[j];
             }
         }
-        if (base + tb < tok1) fetch(base + tb);
-        __syncthreads();
-        // the batch's tokens one after the other, the loop written out without a branch (a batch is always whole: see above): nothing
-        // in it writes memory, so the fetches of the tokens to come move ahead of the sums of the token at hand; the outputs wait in
-        // registers for the end of the batch
-        float obuf[TB];
 #pragma unroll
+        for (int j = 0; j < NV; ++j)
+            if (tid + j * 256 < TB * COLS) sv[tid + j * 256] = pv[j];
+        if (tid < 2 * TB) sg[(tid >> 1) * 4 + (tid & 1)] = pg;
+        if (base + TB < tok1) fetch(base + TB);
+        shared_barrier();
+        // k . q: the 16 lanes of column cw make token cw's
+        if (cw < TB) {
+            float c4[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                const float4 k4 = *(const float4*)(sk + cw * ROWS + 64 * q + 4 * rg), q4 = *(const float4*)(sq + cw * ROWS + 64 * q + 4 * rg);
+                c4[0] = fmaf(k4.x, q4.x, c4[0]);
+                c4[1] = fmaf(k4.y, q4.y, c4[1]);
+                c4[2] = fmaf(k4.z, q4.z, c4[2]);
+                c4[3] = fmaf(k4.w, q4.w, c4[3]);
+            }
+            const float kq = row16_sum((c4[0] + c4[1]) + (c4[2] + c4[3]));
+            if (rg == 0) sg[cw * 4 + 2] = kq;
+        }
+        shared_barrier();
+        float mine[CPL];                               // the outputs of token rg of the batch
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) mine[c] = 0.f;
+        // a token's operands are read from shared memory one token ahead, beside the sums of the token at hand (asked for when they are needed,
+        // four tokens' at a time, they and the sums took turns)
+        float4 kn[Q], qn[Q], gn;
+        float vn[CPL];
+        auto ahead = [&](int t) {
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                kn[q] = *(const float4*)(sk + t * ROWS + 64 * q + 4 * rg);
+                qn[q] = *(const float4*)(sq + t * ROWS + 64 * q + 4 * rg);
+            }
+            gn = *(const float4*)(sg + t * 4);
+#pragma unroll
+            for (int c = 0; c < CPL; ++c) vn[c] = sv[t * COLS + cw + c * DELTA_COLS];
+        };
+        ahead(0);
+#pragma unroll 4
         for (int t = 0; t < TB; ++t) {
-            {
-                const float* kt = sk + t * ROWS + row0;
-                const float* qt = sq + t * ROWS + row0;
-                float kr[RPL], qr[RPL];
+            float kr[RPL], qr[RPL], vr[CPL];
 #pragma unroll
-                for (int r = 0; r < RPL; r += 4) {
-                    const float4 k4 = *(const float4*)(kt + r), q4 = *(const float4*)(qt + r);
-                    kr[r] = k4.x; kr[r + 1] = k4.y; kr[r + 2] = k4.z; kr[r + 3] = k4.w;
-                    qr[r] = q4.x; qr[r + 1] = q4.y; qr[r + 2] = q4.z; qr[r + 3] = q4.w;
-                }
-                const float beta = sg[t * 2], g = sg[t * 2 + 1], vt = sv[t * DELTA_COLS + cw];
+            for (int q = 0; q < Q; ++q) {
+                kr[4 * q] = kn[q].x; kr[4 * q + 1] = kn[q].y; kr[4 * q + 2] = kn[q].z; kr[4 * q + 3] = kn[q].w;
+                qr[4 * q] = qn[q].x; qr[4 * q + 1] = qn[q].y; qr[4 * q + 2] = qn[q].z; qr[4 * q + 3] = qn[q].w;
+            }
+#pragma unroll
+            for (int c = 0; c < CPL; ++c) vr[c] = vn[c];
+            const float beta = gn.x, g = gn.y, kq = gn.z;
+            ahead(min(t + 1, TB - 1));
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int c = 0; c < CPL; ++c) {
+                const float vt = vr[c];
                 // four chains of additions each, joined in a fixed order
-                float a4[4] = {0.f, 0.f, 0.f, 0.f}, b4[4] = {0.f, 0.f, 0.f, 0.f}, c4[4] = {0.f, 0.f, 0.f, 0.f};
+                float a4[4] = {0.f, 0.f, 0.f, 0.f}, b4[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int r = 0; r < RPL; ++r) {
-                    if (MODE == 1) a4[r & 3] = fmaf(S[r], kr[r], a4[r & 3]);
-                    b4[r & 3] = fmaf(S[r], qr[r], b4[r & 3]);
-                    c4[r & 3] = fmaf(kr[r], qr[r], c4[r & 3]);
+                    if (MODE == 1) a4[r & 3] = fmaf(S[c][r], kr[r], a4[r & 3]);
+                    b4[r & 3] = fmaf(S[c][r], qr[r], b4[r & 3]);
                 }
                 const float a = MODE == 1 ? row16_sum((a4[0] + a4[1]) + (a4[2] + a4[3])) : 0.f;
                 const float b = row16_sum((b4[0] + b4[1]) + (b4[2] + b4[3]));
-                const float kq = row16_sum((c4[0] + c4[1]) + (c4[2] + c4[3]));
-                const float u = MODE == 1 ? beta * (vt - g * a) : (MODE == 2 ? beta * vt : vt);
+                const float u = MODE == 1 ? beta * fmaf(-g, a, vt) : (MODE == 2 ? beta * vt : vt);
 #pragma unroll
-                for (int r = 0; r < RPL; ++r) S[r] = fmaf(kr[r], u, g * S[r]);
-                obuf[t] = MODE == 2 ? fmaf(skip, vt, fmaf(kq, u, g * b)) : fmaf(kq, u, g * b);
+                for (int r = 0; r < RPL; ++r) S[c][r] = fmaf(kr[r], u, g * S[c][r]);
+                const float o = MODE == 2 ? fmaf(skip, vt, fmaf(kq, u, g * b)) : fmaf(kq, u, g * b);
+                if (rg == t) mine[c] = o;
             }
         }
-        if (rg == 0 && col_ok) {
-            float* orow = out + ((size_t)base * heads + head) * vdim + col;
 #pragma unroll
-            for (int t = 0; t < TB; ++t)
-                if (t < nb) orow[(size_t)t * heads * vdim] = obuf[t];
+        for (int c = 0; c < CPL; ++c) {
+            const int col = col0 + cw + c * DELTA_COLS;
+            if (rg < nb && col < vdim) out[((size_t)(base + rg) * heads + head) * vdim + col] = mine[c];
         }
     }
-    if (whole) {
 #pragma unroll
-        for (int r = 0; r < RPL; r += 4) *(float4*)(st + r) = make_float4(S[r], S[r + 1], S[r + 2], S[r + 3]);
-    } else if (col_ok) {
+    for (int c = 0; c < CPL; ++c) {
+        const int col = col0 + cw + c * DELTA_COLS;
 #pragma unroll
-        for (int r = 0; r < RPL; ++r)
-            if (row0 + r < dim) st[r] = S[r];
+        for (int q = 0; q < Q; ++q) {
+            const int row = 64 * q + 4 * rg;
+            float* to = st + (size_t)col * dim + row;
+            if (vec_state && col < vdim && row + 4 <= dim) *(float4*)to = make_float4(S[c][4 * q], S[c][4 * q + 1], S[c][4 * q + 2], S[c][4 * q + 3]);
+            else if (col < vdim) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (row + e < dim) to[e] = S[c][4 * q + e];
+            }
+        }
     }
 }
 
@@ -687,16 +764,25 @@ static int launch_delta_scan(const void* qkv, const void* gates, const void* hea
     const int rpl = dim <= 64 ? 4 : dim <= 128 ? 8 : dim <= 192 ? 12 : 16;
     // tokens of a batch: 1 for a step of single tokens, 4 for short portions, else 16 (a batch is always worked through whole)
     const int tb = longest <= 1 ? 1 : (longest <= 4 ? 4 : DELTA_TB);
-    const size_t smem = sizeof(float) * (size_t)tb * (2 * DELTA_L * rpl + DELTA_COLS + 2);
-    dim3 grid((vdim + DELTA_COLS - 1) / DELTA_COLS, heads, requests), block(256);
-#define TL_DELTA_B(R, B)                                                                                                                   \
-    delta_scan_kernel<R, B, MODE><<<grid, block, smem, stream>>>((const float*)qkv, (const float*)gates, (const float*)head_decay, (float*)state, \
-                                                           (size_t)slot_stride, (const int*)slots, (const int*)req_indptr, (float*)out, heads, kv_heads, dim, vdim)
-#define TL_DELTA(R)                        \
-    if (tb == 1) TL_DELTA_B(R, 1);         \
-    else if (tb == 4) TL_DELTA_B(R, 4);    \
-    else TL_DELTA_B(R, DELTA_TB)
-    if (rpl == 4) { TL_DELTA(4); }
+    const int vec = dim == DELTA_L * rpl && vdim % 4 == 0 && ((uintptr_t)qkv & 15) == 0;       // (a token's numbers are then a multiple of four)
+    const long groups = (long)((vdim + DELTA_COLS - 1) / DELTA_COLS) * heads * requests;
+    // two columns to a lane (half the reads of shared memory a column) where one to a lane would not all be on the GPU at once, four work-groups to a
+    // compute unit; up to there more waves win.  Measured (us, one column / two; number-by-number fetches before): the delta rule, 16 heads of 128 x
+    // 128, one prompt of 2048 tokens 405 / 603 (1533), eight prompts of 175 to 700 tokens 189 / 230 (1328); the selective recurrence, 128 heads of 128 x
+    // 64, four prompts of 275 to 1100 tokens 467 / 342 (3780); fixed decays, 16 heads of 128 x 128, 2048 tokens 366 / 492 (1342).  Portions of 4
+    // tokens and single ones (8 requests, 9 us) as before.
+    const int cpl = groups > 4L * tl_mlstm_units && rpl <= 8 && tb == DELTA_TB ? 2 : 1;
+    dim3 grid((vdim + DELTA_COLS * cpl - 1) / (DELTA_COLS * cpl), heads, requests), block(256);
+#define TL_DELTA_B(R, B, P)                                                                                                                \
+    delta_scan_kernel<R, B, MODE, P><<<grid, block, 0, stream>>>((const float*)qkv, (const float*)gates, (const float*)head_decay, (float*)state, \
+                                                           (size_t)slot_stride, (const int*)slots, (const int*)req_indptr, (float*)out, heads, kv_heads, dim, vdim, vec)
+#define TL_DELTA(R)                           \
+    if (tb == 1) TL_DELTA_B(R, 1, 1);         \
+    else if (tb == 4) TL_DELTA_B(R, 4, 1);    \
+    else TL_DELTA_B(R, DELTA_TB, 1)
+    if (cpl == 2 && rpl == 4) TL_DELTA_B(4, DELTA_TB, 2);
+    else if (cpl == 2 && rpl == 8) TL_DELTA_B(8, DELTA_TB, 2);
+    else if (rpl == 4) { TL_DELTA(4); }
     else if (rpl == 8) { TL_DELTA(8); }
     else if (rpl == 12) { TL_DELTA(12); }
     else { TL_DELTA(16); }
@@ -929,6 +1015,9 @@ wkv_scan_kernel(const T* __restrict__ rkv, int ld, int k_off, int v_off, const f
         for (int e = 0; e < 4; ++e) ub[4 * q + e] = row + e < dim ? bonus[head * dim + row + e] : 0.f;
     }
 
+    // (the state and the bonuses are waited for here: left to the token loop, the wait at its head would cover the next batch's fetches too)
+#pragma unroll
+    for (int r = 0; r < RPL; ++r) asm volatile("" : "+v"(S[r]), "+v"(ub[r]));
     float4 pr[NP], pk[NP], pw[NP];
     float pv = 0.f;
     auto fetch = [&](int base) {
