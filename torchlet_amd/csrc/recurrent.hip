@@ -1,6 +1,8 @@
 // Recurrent mixers with a fixed-size state per request: the matrix-memory recurrence (mLSTM), the gated delta rule behind its
 // short convolutions, a recurrence whose decays are each key channel's and each token's own (the time mixing of RWKV), and the gated per-head norm of their outputs.  State, gates, decays and the output's quotient are float whatever the
 // activation type; queries, keys and values come in the activation type as the projection left them.
+#include <limits.h>
+
 #include "common.h"
 
 // A barrier that orders shared memory only: __syncthreads() also waits for every fetch from memory that is on its
@@ -39,7 +41,7 @@ mlstm_scan_kernel(const T* __restrict__ qkv, int ld, int k_off, int v_off,
                   const float* __restrict__ gates,          // [tokens, 2 * heads]: raw input gates, raw forget gates
                   float* __restrict__ state, size_t slot_stride, const int* __restrict__ slots, const float* __restrict__ before,
                   const int* __restrict__ req_indptr, float* __restrict__ out, int heads, int dim, int vdim,
-                  float cap, float qscale, float denom_eps, int tb) {
+                  float cap, float qscale, float denom_eps, int tb, int below) {
     constexpr int RG = TL_WAVE / COLS;                 // groups of RPT rows a wave holds side by side
     extern __shared__ float smem[];
     const int waves = blockDim.x / TL_WAVE, wave = threadIdx.x / TL_WAVE, lane = threadIdx.x % TL_WAVE;
@@ -55,7 +57,7 @@ mlstm_scan_kernel(const T* __restrict__ qkv, int ld, int k_off, int v_off,
 
     const int req = blockIdx.z, head = blockIdx.y, col0 = blockIdx.x * (COLS - 1);
     const int tok0 = req_indptr[req], tok1 = req_indptr[req + 1];
-    if (tok0 >= tok1) return;
+    if (tok0 >= tok1 || tok1 - tok0 >= below) return;  // (a long portion goes through the chunks)
     const int c = lane % COLS, share = (wave * RG + lane / COLS) * SPL;     // the first of this lane's shares
     const bool is_n = c == COLS - 1;
     const int col = col0 + c;
@@ -221,7 +223,7 @@ __global__ void mlstm_before_kernel(const float* __restrict__ state, size_t slot
 template <typename T, int RPT, int COLS>
 static int launch_mlstm_scan(const void* qkv, int ld, int k_off, int v_off, const void* gates, void* state, size_t slot_stride,
                              const void* slots, const void* before, const void* req_indptr, void* out, int requests, int heads, int dim, int vdim,
-                             float cap, float qscale, float denom_eps, int tb, hipStream_t stream) {
+                             float cap, float qscale, float denom_eps, int tb, int below, hipStream_t stream) {
     constexpr int RG = TL_WAVE / COLS;
     const int waves = (dim + RPT * RG - 1) / (RPT * RG);
     TL_REQUIRE(waves <= 16, "mlstm_scan: %d rows of a head do not fit a work-group of %d rows a lane and %d columns", dim, RPT, COLS);
@@ -241,7 +243,7 @@ static int launch_mlstm_scan(const void* qkv, int ld, int k_off, int v_off, cons
     mlstm_before_kernel<<<requests * heads, 128, 0, stream>>>((const float*)state, slot_stride, (const int*)slots, (float*)before, heads, dim, vdim);
     TL_CHECK_LAUNCH("mlstm_before");
     kernel<<<grid, block, smem, stream>>>((const T*)qkv, ld, k_off, v_off, (const float*)gates, (float*)state, slot_stride,
-                                           (const int*)slots, (const float*)before, (const int*)req_indptr, (float*)out, heads, dim, vdim, cap, qscale, denom_eps, tb);
+                                           (const int*)slots, (const float*)before, (const int*)req_indptr, (float*)out, heads, dim, vdim, cap, qscale, denom_eps, tb, below);
     TL_CHECK_LAUNCH("mlstm_scan");
     return TL_OK;
 }
@@ -249,13 +251,10 @@ static int launch_mlstm_scan(const void* qkv, int ld, int k_off, int v_off, cons
 static int tl_mlstm_units = 256;       // compute units the column tiles are dealt to
 extern "C" void tl_mlstm_set_compute_units(int units) { if (units > 0) tl_mlstm_units = units; }
 
-// qkv [tokens, ld]: queries at column 0 (heads * dim), keys at k_off, values at v_off (heads * vdim); gates float
-// [tokens, 2 * heads]; state float [slots, heads, dim * vdim + dim + 1] with slot_stride floats between slots;
-// out float [tokens, heads * vdim]; before: scratch of requests * heads * (dim + 1) floats.  Requests whose req_indptr range
-// is empty are left alone.
-extern "C" int tl_mlstm_scan(const void* qkv, int ld, int k_off, int v_off, const void* gates, void* state, long slot_stride,
-                             const void* slots, const void* before, const void* req_indptr, void* out, int requests, int heads, int dim, int vdim,
-                             float cap, float qscale, float denom_eps, int longest, int dtype, hipStream_t stream) {
+// The token loop: requests of `below` tokens or more are left alone.
+static int mlstm_token_loop(const void* qkv, int ld, int k_off, int v_off, const void* gates, void* state, long slot_stride,
+                            const void* slots, const void* before, const void* req_indptr, void* out, int requests, int heads, int dim, int vdim,
+                            float cap, float qscale, float denom_eps, int longest, int below, int dtype, hipStream_t stream) {
     TL_REQUIRE(requests >= 0 && heads > 0 && dim > 0 && vdim > 0 && ld > 0, "mlstm_scan: bad sizes");
     const int tb = longest < 1 ? 1 : (longest < MLSTM_TB ? longest : MLSTM_TB);       // longest: the most tokens a request of the step brings
     TL_REQUIRE(dim <= 1024, "mlstm_scan: built for up to 1024 query/key dimensions per head, got %d", dim);
@@ -271,9 +270,9 @@ extern "C" int tl_mlstm_scan(const void* qkv, int ld, int k_off, int v_off, cons
 #define TL_MLSTM_C(R, C)                                                                                                       \
     return dtype == TL_DT_F32                                                                                                  \
         ? launch_mlstm_scan<float, R, C>(qkv, ld, k_off, v_off, gates, state, (size_t)slot_stride, slots, before, req_indptr, out,    \
-                                         requests, heads, dim, vdim, cap, qscale, denom_eps, tb, stream)                      \
+                                         requests, heads, dim, vdim, cap, qscale, denom_eps, tb, below, stream)                      \
         : launch_mlstm_scan<bf16_t, R, C>(qkv, ld, k_off, v_off, gates, state, (size_t)slot_stride, slots, before, req_indptr, out,   \
-                                          requests, heads, dim, vdim, cap, qscale, denom_eps, tb, stream)
+                                          requests, heads, dim, vdim, cap, qscale, denom_eps, tb, below, stream)
 #define TL_MLSTM(R)                                  \
     if (cols == 64) { TL_MLSTM_C(R, 64); }           \
     else if (cols == 32) { TL_MLSTM_C(R, 32); }      \
@@ -557,14 +556,14 @@ __global__ void __launch_bounds__(256, RPL * CPL <= 16 ? 4 : 2)
 delta_scan_kernel(const float* __restrict__ qkv, const float* __restrict__ gates, const float* __restrict__ head_decay,
                   float* __restrict__ state, size_t slot_stride,
                   const int* __restrict__ slots, const int* __restrict__ req_indptr, float* __restrict__ out,
-                  int heads, int kv_heads, int dim, int vdim, int vec) {
+                  int heads, int kv_heads, int dim, int vdim, int vec, int below) {
     constexpr int ROWS = DELTA_L * RPL, Q = RPL / 4, COLS = DELTA_COLS * CPL;          // ROWS >= dim
     constexpr int PPT = ROWS / 4, NP = (TB * PPT + 255) / 256, NV = (TB * COLS + 255) / 256;      // pieces of four: per token, per thread and batch
     __shared__ __attribute__((aligned(16))) float sq[TB * ROWS], sk[TB * ROWS], sg[TB * 4];       // sg: beta, decay, k . q
     __shared__ float sv[TB * COLS];
     const int req = blockIdx.z, head = blockIdx.y, col0 = blockIdx.x * COLS;
     const int tok0 = req_indptr[req], tok1 = req_indptr[req + 1];
-    if (tok0 >= tok1) return;
+    if (tok0 >= tok1 || tok1 - tok0 >= below) return;            // (a long portion goes through the chunks)
     const int tid = threadIdx.x, wave = tid / TL_WAVE, lane = tid % TL_WAVE;
     const int rg = lane & 15, cw = wave * 4 + (lane >> 4);       // the lane's place in its columns, and the first of them within the work-group
     const int C = 2 * kv_heads * dim + heads * vdim;
@@ -760,7 +759,7 @@ delta_scan_kernel(const float* __restrict__ qkv, const float* __restrict__ gates
 // state: per slot, from its start, heads x [vdim][dim] floats (a head's state column by column).
 template <int MODE>
 static int launch_delta_scan(const void* qkv, const void* gates, const void* head_decay, void* state, long slot_stride, const void* slots,
-                             const void* req_indptr, void* out, int requests, int heads, int kv_heads, int dim, int vdim, int longest, hipStream_t stream) {
+                             const void* req_indptr, void* out, int requests, int heads, int kv_heads, int dim, int vdim, int longest, int below, hipStream_t stream) {
     const int rpl = dim <= 64 ? 4 : dim <= 128 ? 8 : dim <= 192 ? 12 : 16;
     // tokens of a batch: 1 for a step of single tokens, 4 for short portions, else 16 (a batch is always worked through whole)
     const int tb = longest <= 1 ? 1 : (longest <= 4 ? 4 : DELTA_TB);
@@ -775,7 +774,7 @@ static int launch_delta_scan(const void* qkv, const void* gates, const void* hea
     dim3 grid((vdim + DELTA_COLS * cpl - 1) / (DELTA_COLS * cpl), heads, requests), block(256);
 #define TL_DELTA_B(R, B, P)                                                                                                                \
     delta_scan_kernel<R, B, MODE, P><<<grid, block, 0, stream>>>((const float*)qkv, (const float*)gates, (const float*)head_decay, (float*)state, \
-                                                           (size_t)slot_stride, (const int*)slots, (const int*)req_indptr, (float*)out, heads, kv_heads, dim, vdim, vec)
+                                                           (size_t)slot_stride, (const int*)slots, (const int*)req_indptr, (float*)out, heads, kv_heads, dim, vdim, vec, below)
 #define TL_DELTA(R)                           \
     if (tb == 1) TL_DELTA_B(R, 1, 1);         \
     else if (tb == 4) TL_DELTA_B(R, 4, 1);    \
@@ -798,43 +797,13 @@ extern "C" int tl_delta_scan(const void* qkv, const void* gates, void* state, lo
     TL_REQUIRE(slot_stride >= (long)heads * dim * vdim, "delta_scan: the state rows are too short");
     TL_REQUIRE(requests <= 65535 && heads <= 65535, "delta_scan: too many requests or heads for one launch");
     if (requests == 0) return TL_OK;
-    launch_delta_scan<1>(qkv, gates, nullptr, state, slot_stride, slots, req_indptr, out, requests, heads, kv_heads, dim, vdim, longest, stream);
+    launch_delta_scan<1>(qkv, gates, nullptr, state, slot_stride, slots, req_indptr, out, requests, heads, kv_heads, dim, vdim, longest, INT_MAX, stream);
     TL_CHECK_LAUNCH("delta_scan");
     return TL_OK;
 }
 
-// ------------------------------------------------------------------ decayed linear attention
-// Per head S <- decay[head] S + k v^T, o = S^T q over the step's tokens, request by request from the state its slot holds: qkv float
-// [T, 2 * heads * dim + heads * vdim] (queries, keys, values, head by head), state as the delta rule's, out float [T, heads * vdim].
-extern "C" int tl_decay_scan(const void* qkv, const void* decay, void* state, long slot_stride, const void* slots, const void* req_indptr,
-                             void* out, int requests, int heads, int dim, int vdim, int longest, hipStream_t stream) {
-    TL_REQUIRE(requests >= 0 && heads > 0 && dim > 0 && vdim > 0 && decay, "decay_scan: bad sizes");
-    TL_REQUIRE(dim <= DELTA_L * 16, "decay_scan: built for up to %d query/key dimensions per head, got %d", DELTA_L * 16, dim);
-    TL_REQUIRE(slot_stride >= (long)heads * dim * vdim, "decay_scan: the state rows are too short");
-    TL_REQUIRE(requests <= 65535 && heads <= 65535, "decay_scan: too many requests or heads for one launch");
-    if (requests == 0) return TL_OK;
-    launch_delta_scan<0>(qkv, nullptr, decay, state, slot_stride, slots, req_indptr, out, requests, heads, heads, dim, vdim, longest, stream);
-    TL_CHECK_LAUNCH("decay_scan");
-    return TL_OK;
-}
-
-// ------------------------------------------------------------------ selective state-space recurrence (Mamba-2)
-// Per head S <- decay S + dt B x^T (S: state x vdim), y = S^T C + D x, with B and C shared by the heads of a group.  qkv float [T, 2 * groups *
-// state + heads * vdim] as selective_prepare leaves it (C, B, x), gates float [T, 2 * heads] (dt, decay), skip float [heads] (D); the
-// state as the delta rule's ([vdim][state] per head), out float [T, heads * vdim].
-extern "C" int tl_selective_scan(const void* qkv, const void* gates, const void* skip, void* state, long slot_stride, const void* slots,
-                                 const void* req_indptr, void* out, int requests, int heads, int groups, int dim, int vdim, int longest, hipStream_t stream) {
-    TL_REQUIRE(requests >= 0 && heads > 0 && groups > 0 && heads % groups == 0 && dim > 0 && vdim > 0 && gates && skip, "selective_scan: bad sizes");
-    TL_REQUIRE(dim <= DELTA_L * 16, "selective_scan: built for states of up to %d numbers per column, got %d", DELTA_L * 16, dim);
-    TL_REQUIRE(slot_stride >= (long)heads * dim * vdim, "selective_scan: the state rows are too short");
-    TL_REQUIRE(requests <= 65535 && heads <= 65535, "selective_scan: too many requests or heads for one launch");
-    if (requests == 0) return TL_OK;
-    launch_delta_scan<2>(qkv, gates, skip, state, slot_stride, slots, req_indptr, out, requests, heads, groups, dim, vdim, longest, stream);
-    TL_CHECK_LAUNCH("selective_scan");
-    return TL_OK;
-}
-
-// What that recurrence reads, made from the projection of the step's tokens.  proj [T, ld] holds per token, from column x_off on, the
+// ------------------------------------------------------------------ what the selective state-space recurrence reads
+// Made from the projection of the step's tokens.  proj [T, ld] holds per token, from column x_off on, the
 // `channels` = inner + 2 * groups * state convolved channels [x | B | C] and after them `heads` raw step sizes.  Channel c at the request's
 // i-th token of the step: y = silu(bias[c] + sum_j w[c][j] * in[i - (taps - 1) + j][c]) with in[i'] the projection of the step's token
 // i' >= 0, else tail[taps - 1 + i'][c] (the slot's last taps - 1 inputs from before the step; zero for a new request).  y goes to qkv
@@ -1162,5 +1131,579 @@ extern "C" int tl_wkv_scan(const void* rkv, int ld, int k_off, int v_off, const 
     else if (dtype == TL_DT_BF16) launch_wkv_scan<bf16_t>(rkv, ld, k_off, v_off, decay, bonus, state, slot_stride, slots, req_indptr, out, requests, heads, dim, vdim, longest, last_rows, row_width, tail_off, stream);
     else TL_REQUIRE(false, "wkv_scan: unknown dtype %d", dtype);
     TL_CHECK_LAUNCH("wkv_scan");
+    return TL_OK;
+}
+
+// ------------------------------------------------------------------ long portions in chunks: recurrences with one decay per head and token
+// S <- g S + b k v^T, o = S^T q (the matrix memory; the decayed linear attention; the selective recurrence) over the tokens of a long portion.
+// Token by token the work of a head is a chain that a few compute units walk (four heads of 256 x 512 over 2048 tokens: 1.2 ms, a prompt's
+// largest item; in chunks 0.17); cut into chunks of 64 tokens nearly all of it is products of matrices that every chunk can take at once:
+//   chunk_states:  D_c = sum_j w_j v_j k_j^T with w_j = b_j prod_{l > j} g_l, and the chunk's decay G_c = prod g;     (all chunks at once)
+//   chunk_pass:    S_c, the state before chunk c, from S_0 and the D_c, S_{c+1} = G_c S_c + D_c;                      (a stream over the chunks)
+//   chunk_outputs: o_i = G_i S_c^T q_i + sum_{j <= i} b_j (prod_{j < l <= i} g_l) (q_i . k_j) v_j.                     (all chunks at once)
+// Products and sums in true 32-bit on v_mfma_f32_32x32x2_f32; decays enter as products of the same numbers the token loop multiplies by (no
+// logarithms, no quotients: a decay of zero is one).  Errors against 64 bits are no larger than the token loop's (median per token and head, at 2000 tokens: the matrix memory 1.2e-7 against 1.7e-7, fixed decays 0.70e-7 against 0.79e-7).
+// Requests of few tokens in the step (decoded ones) stay with the token loop, which leaves the others out.
+#define CK_T 64                 // tokens of a chunk
+#define CK_D 64                 // query/key dimensions of a slab in shared memory
+#define CK_V 128                // value columns of a work-group
+#define CK_LD (CK_D + 4)        // row pitches in shared memory: rows read 16 bytes a lane fall on all banks
+#define CK_LV (CK_V + 4)
+
+typedef float ck_f32x16 __attribute__((ext_vector_type(16)));
+
+struct ChunkArgs {
+    const void* qkv;            // a token's row: ld numbers; queries of head h from column q_off + qk(h) * dim on, keys from k_off, values from v_off + h * vdim
+    int ld, q_off, k_off, v_off, heads, qk_share;      // qk(h) = h / qk_share
+    int dim, vdim;
+    const float* gates;         // [tokens][gate_ld]: b at column h * gate_step + b_at, g at h * gate_step + g_at; null: b = 1, g = head_decay[h]
+    int gate_ld, gate_step, b_at, g_at;
+    const float* head_decay;    // fixed decays, or the skip factors
+    float qscale, denom_eps;
+    float* state;
+    size_t slot_stride;
+    const int *slots, *req_indptr;
+    float* out;                 // [tokens][heads * vdim]
+    float *states, *sums, *decays;      // scratch: [chunks][heads][vdim][dim], [chunks][heads][dim] (matrix memory), [chunks][heads]
+    int requests, least, seg0, seg_len;      // the tokens seg0 .. seg0 + seg_len - 1 of every request of at least `least` tokens
+};
+
+__device__ __forceinline__ int ck_chunks(const ChunkArgs& a, int n) { return n >= a.least && n > a.seg0 ? (min(n - a.seg0, a.seg_len) + CK_T - 1) / CK_T : 0; }
+
+// The request of chunk `want` among all requests' chunks and its first chunk, by a prefix sum over the lanes; -1 beyond the last chunk.
+__device__ __forceinline__ int ck_find(const ChunkArgs& a, int want, int& first_chunk) {
+    const int lane = threadIdx.x % TL_WAVE;
+    int first = 0;
+    for (int base = 0; base < a.requests; base += TL_WAVE) {
+        const int r = base + lane;
+        const int mine = r < a.requests ? ck_chunks(a, a.req_indptr[r + 1] - a.req_indptr[r]) : 0;
+        int upto = mine;
+#pragma unroll
+        for (int o = 1; o < TL_WAVE; o <<= 1) {
+            const int t = __shfl_up(upto, o, TL_WAVE);
+            if (lane >= o) upto += t;
+        }
+        const unsigned long long past = __ballot(first + upto > want);
+        if (past) {
+            const int l = __builtin_amdgcn_readfirstlane(__ffsll(past) - 1);
+            first_chunk = first + __builtin_amdgcn_readlane(upto, l) - __builtin_amdgcn_readlane(mine, l);
+            return base + l;
+        }
+        first += __builtin_amdgcn_readlane(upto, TL_WAVE - 1);
+    }
+    return -1;
+}
+
+template <typename T> __device__ __forceinline__ float4 ck_load4(const T* p) { return wkv_load4<T>(p); }
+
+// MODE 0: fixed decays.  MODE 3: the matrix memory (b, g and the running maximum per
+// token; outputs over max(|n . q|, exp(-m)) + denom_eps).
+template <typename T, int MODE>
+__global__ void __launch_bounds__(256)
+chunk_states_kernel(ChunkArgs a) {
+    __shared__ __attribute__((aligned(16))) float sk[CK_T * CK_LD], sv[CK_T * CK_LV];
+    __shared__ float sw[CK_T], sn[4 * CK_D];
+    const int tid = threadIdx.x, wave = tid / TL_WAVE, lane = tid % TL_WAVE, li = lane & 31, half = lane >> 5;
+    int chunk0 = 0;
+    const int chunk = blockIdx.x, req = ck_find(a, chunk, chunk0);
+    if (req < 0) return;
+    const int head = blockIdx.y, v0 = blockIdx.z * CK_V;
+    const int tok0 = a.req_indptr[req] + a.seg0 + (chunk - chunk0) * CK_T;
+    const int nt = min(min(CK_T, a.req_indptr[req + 1] - tok0), a.seg_len - (chunk - chunk0) * CK_T);
+    if (wave == 0) {                                   // the tokens' weights: a product over the tokens behind them, taken from the back
+        float b = 0.f, g = 1.f;
+        if (lane < nt) {
+            if (MODE == 0) { b = 1.f; g = a.head_decay[head]; }
+            else {
+                const float* row = a.gates + (size_t)(tok0 + lane) * a.gate_ld + head * a.gate_step;
+                b = row[a.b_at];
+                g = row[a.g_at];
+            }
+        }
+        double p = g;
+#pragma unroll
+        for (int o = 1; o < TL_WAVE; o <<= 1) {
+            const double t = __shfl_down(p, o, TL_WAVE);
+            if (lane + o < TL_WAVE) p *= t;
+        }
+        const double behind = __shfl_down(p, 1, TL_WAVE);
+        sw[lane] = (float)(b * (lane + 1 < TL_WAVE ? behind : 1.0));
+        if (lane == 0 && blockIdx.z == 0) a.decays[(size_t)chunk * a.heads + head] = (float)p;
+    }
+    __syncthreads();
+    const T* base = (const T*)a.qkv + (size_t)tok0 * a.ld;
+    const T* vsrc = base + a.v_off + head * a.vdim + v0;
+#pragma unroll
+    for (int j = 0; j < CK_T * CK_V / 4 / 256; ++j) {
+        const int idx = tid + j * 256, t = idx / (CK_V / 4), c = (idx % (CK_V / 4)) * 4;
+        float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (t < nt && v0 + c < a.vdim) {
+            x = ck_load4<T>(vsrc + (size_t)t * a.ld + c);
+            const float w = sw[t];
+            x.x *= w; x.y *= w; x.z *= w; x.w *= w;
+        }
+        *(float4*)(sv + t * CK_LV + c) = x;
+    }
+    const T* ksrc = base + a.k_off + head / a.qk_share * a.dim;
+    float* dst = a.states + ((size_t)chunk * a.heads + head) * a.vdim * a.dim;
+    for (int d0 = 0; d0 < a.dim; d0 += CK_D) {
+        if (d0 > 0) __syncthreads();
+#pragma unroll
+        for (int j = 0; j < CK_T * CK_D / 4 / 256; ++j) {
+            const int idx = tid + j * 256, t = idx / (CK_D / 4), c = (idx % (CK_D / 4)) * 4;
+            *(float4*)(sk + t * CK_LD + c) = t < nt && d0 + c < a.dim ? ck_load4<T>(ksrc + (size_t)t * a.ld + d0 + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        __syncthreads();
+        if (v0 + wave * 32 < a.vdim) {
+            ck_f32x16 acc[2], more[2];                 // two chains of sums each
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[0][i] = acc[1][i] = more[0][i] = more[1][i] = 0.f;
+#pragma unroll 4
+            for (int t = 0; t < CK_T; t += 4) {
+                const float x = sv[(t + half) * CK_LV + wave * 32 + li], y = sv[(t + 2 + half) * CK_LV + wave * 32 + li];
+                acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, sk[(t + half) * CK_LD + li], acc[0], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, sk[(t + half) * CK_LD + 32 + li], acc[1], 0, 0, 0);
+                more[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(y, sk[(t + 2 + half) * CK_LD + li], more[0], 0, 0, 0);
+                more[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(y, sk[(t + 2 + half) * CK_LD + 32 + li], more[1], 0, 0, 0);
+            }
+            acc[0] += more[0];
+            acc[1] += more[1];
+#pragma unroll
+            for (int n = 0; n < 2; ++n)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int v = v0 + wave * 32 + 8 * (i / 4) + 4 * half + i % 4, d = d0 + 32 * n + li;
+                    if (v < a.vdim && d < a.dim) dst[(size_t)v * a.dim + d] = acc[n][i];
+                }
+        }
+        if (MODE == 3 && blockIdx.z == 0) {            // the keys' own weighted sum (the memory's column of ones)
+            const int d = tid % CK_D, part = tid / CK_D;
+            float s = 0.f;
+#pragma unroll
+            for (int t = 0; t < CK_T / 4; ++t) s = fmaf(sw[part * (CK_T / 4) + t], sk[(part * (CK_T / 4) + t) * CK_LD + d], s);
+            sn[part * CK_D + d] = s;
+            __syncthreads();
+            if (tid < CK_D && d0 + tid < a.dim)
+                a.sums[((size_t)chunk * a.heads + head) * a.dim + d0 + tid] = ((sn[tid] + sn[CK_D + tid]) + sn[2 * CK_D + tid]) + sn[3 * CK_D + tid];
+        }
+    }
+}
+
+// The states before every chunk, in place of the chunks' own sums, and the state after the last one in the request's slot.  A thread owns four
+// neighbouring numbers of a column.  ROWS: the slot holds the state row by row ([dim][vdim], and behind it the keys' sums and the running maximum),
+// so a work-group takes a tile of 32 x 32 and turns it in shared memory on its way from and to the slot; otherwise column by column, as the scratch does.
+template <bool ROWS>
+__global__ void __launch_bounds__(256)
+chunk_pass_kernel(ChunkArgs a) {
+    __shared__ float turn[32][33];
+    const int req = blockIdx.z, head = blockIdx.y, tid = threadIdx.x, lane = tid % TL_WAVE;
+    const int count = ck_chunks(a, a.req_indptr[req + 1] - a.req_indptr[req]);
+    if (count == 0) return;
+    int first = 0;
+    for (int base = 0; base < req; base += TL_WAVE) {
+        const int r = base + lane;
+        int mine = r < req ? ck_chunks(a, a.req_indptr[r + 1] - a.req_indptr[r]) : 0;
+#pragma unroll
+        for (int o = TL_WAVE / 2; o > 0; o >>= 1) mine += __shfl_xor(mine, o, TL_WAVE);
+        first += mine;
+    }
+    const size_t slot_head = ROWS ? (size_t)a.dim * a.vdim + a.dim + 1 : (size_t)a.dim * a.vdim;
+    float* st = a.state + (size_t)a.slots[req] * a.slot_stride + head * slot_head;
+    const float* gs = a.decays + (size_t)first * a.heads + head;
+    const size_t step = (size_t)a.heads * a.vdim * a.dim;
+    const int tiles_d = (a.dim + 31) / 32;
+    if (ROWS && (int)blockIdx.x == tiles_d * ((a.vdim + 31) / 32)) {      // the keys' sums and the running maximum
+        for (int d = tid; d < a.dim; d += 256) {
+            float n = st[(size_t)a.dim * a.vdim + d];
+            for (int c = 0; c < count; ++c) {
+                float* p = a.sums + ((size_t)(first + c) * a.heads + head) * a.dim + d;
+                const float x = *p;
+                *p = n;
+                n = fmaf(gs[(size_t)c * a.heads], n, x);
+            }
+            st[(size_t)a.dim * a.vdim + d] = n;
+        }
+        if (tid == 0) {
+            const int end = min(a.req_indptr[req + 1], a.req_indptr[req] + a.seg0 + a.seg_len);
+            st[(size_t)a.dim * a.vdim + a.dim] = a.gates[(size_t)(end - 1) * a.gate_ld + head * a.gate_step + 2];
+        }
+        return;
+    }
+    int v, d;
+    if (ROWS) {
+        const int tv = blockIdx.x / tiles_d * 32, td = blockIdx.x % tiles_d * 32;
+        v = tv + tid / 8;
+        d = td + tid % 8 * 4;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int dd = td + tid / 32 + 8 * j, vv = tv + tid % 32;
+            turn[tid / 32 + 8 * j][tid % 32] = dd < a.dim && vv < a.vdim ? st[(size_t)dd * a.vdim + vv] : 0.f;
+        }
+        __syncthreads();
+    } else {
+        const int idx = (blockIdx.x * 256 + tid) * 4;
+        v = idx / a.dim;
+        d = idx % a.dim;
+    }
+    const bool ok = v < a.vdim && d < a.dim;
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (ok) {
+        if (ROWS) s = make_float4(turn[tid % 8 * 4][tid / 8], turn[tid % 8 * 4 + 1][tid / 8], turn[tid % 8 * 4 + 2][tid / 8], turn[tid % 8 * 4 + 3][tid / 8]);
+        else s = *(const float4*)(st + (size_t)v * a.dim + d);
+        float* p = a.states + ((size_t)first * a.heads + head) * a.vdim * a.dim + (size_t)v * a.dim + d;
+        constexpr int AHEAD = 8;                       // chunks' numbers requested together
+        for (int c0 = 0; c0 < count; c0 += AHEAD) {
+            float4 x[AHEAD];
+            float g[AHEAD];
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) {
+                const int c = min(c0 + u, count - 1);
+                x[u] = *(const float4*)(p + c * step);
+                g[u] = gs[(size_t)c * a.heads];
+            }
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) {
+                if (c0 + u < count) {
+                    *(float4*)(p + (c0 + u) * step) = s;
+                    s.x = fmaf(g[u], s.x, x[u].x);
+                    s.y = fmaf(g[u], s.y, x[u].y);
+                    s.z = fmaf(g[u], s.z, x[u].z);
+                    s.w = fmaf(g[u], s.w, x[u].w);
+                }
+            }
+        }
+        if (!ROWS) *(float4*)(st + (size_t)v * a.dim + d) = s;
+    }
+    if (ROWS) {
+        __syncthreads();
+        turn[tid % 8 * 4][tid / 8] = s.x; turn[tid % 8 * 4 + 1][tid / 8] = s.y; turn[tid % 8 * 4 + 2][tid / 8] = s.z; turn[tid % 8 * 4 + 3][tid / 8] = s.w;
+        __syncthreads();
+        const int tv = blockIdx.x / tiles_d * 32, td = blockIdx.x % tiles_d * 32;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int dd = td + tid / 32 + 8 * j, vv = tv + tid % 32;
+            if (dd < a.dim && vv < a.vdim) st[(size_t)dd * a.vdim + vv] = turn[tid / 32 + 8 * j][tid % 32];
+        }
+    }
+}
+
+template <typename T, int MODE>
+__global__ void __launch_bounds__(256, 2)
+chunk_outputs_kernel(ChunkArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float ck_smem[];
+    float* sq = ck_smem;                               // [64][CK_LD] queries of a slab; after the slabs the weighted scores
+    float* sk = sq + CK_T * CK_LD;                     // [64][CK_LD] keys of a slab
+    float* ss = sk + CK_T * CK_LD;                     // [CK_V][CK_LD] the state's columns of a slab; after the slabs [64][CK_LV] values
+    float* sg = ss + CK_V * CK_LD;                     // [64] g, [64] b, [64] G (products up to the token), [64] 1 / denominator, [64] keys' sums of a slab
+    const int tid = threadIdx.x, wave = tid / TL_WAVE, lane = tid % TL_WAVE, li = lane & 31, half = lane >> 5;
+    int chunk0 = 0;
+    const int chunk = blockIdx.x, req = ck_find(a, chunk, chunk0);
+    if (req < 0) return;
+    const int head = blockIdx.y, v0 = blockIdx.z * CK_V;
+    const int tok0 = a.req_indptr[req] + a.seg0 + (chunk - chunk0) * CK_T;
+    const int nt = min(min(CK_T, a.req_indptr[req + 1] - tok0), a.seg_len - (chunk - chunk0) * CK_T);
+    float m_mine = 0.f;                                // the running maximum after token tid / 4
+    if (wave == 0) {
+        float b = 0.f, g = 1.f;
+        if (lane < nt) {
+            if (MODE == 0) { b = 1.f; g = a.head_decay[head]; }
+            else {
+                const float* row = a.gates + (size_t)(tok0 + lane) * a.gate_ld + head * a.gate_step;
+                b = row[a.b_at];
+                g = row[a.g_at];
+            }
+        }
+        double p = g;
+#pragma unroll
+        for (int o = 1; o < TL_WAVE; o <<= 1) {
+            const double t = __shfl_up(p, o, TL_WAVE);
+            if (lane >= o) p *= t;
+        }
+        sg[lane] = g; sg[CK_T + lane] = b; sg[2 * CK_T + lane] = (float)p;
+    }
+    if (MODE == 3 && tid / 4 < nt) m_mine = a.gates[(size_t)(tok0 + tid / 4) * a.gate_ld + head * a.gate_step + 2];
+    const T* base = (const T*)a.qkv + (size_t)tok0 * a.ld;
+    const T* qsrc = base + a.q_off + head / a.qk_share * a.dim;
+    const T* ksrc = base + a.k_off + head / a.qk_share * a.dim;
+    const T* vsrc = base + a.v_off + head * a.vdim + v0;
+    const float* src = a.states + ((size_t)chunk * a.heads + head) * a.vdim * a.dim;
+    const float* nsrc = a.sums + ((size_t)chunk * a.heads + head) * a.dim;
+    const bool cols = v0 + wave * 32 < a.vdim;         // this wave's 32 columns hold some of the head's
+    const int ti = wave >> 1, tj = wave & 1;           // this wave's block of the scores
+    // sums over 32 dimensions (and below over 32 tokens) in a chain, the chains added up: a single chain over 256 lost more than the token loop's sums
+    ck_f32x16 sc, so[2];                               // scores of the wave's block; the state's share of the outputs
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sc[i] = so[0][i] = so[1][i] = 0.f;
+    float qn = 0.f;
+    for (int d0 = 0; d0 < a.dim; d0 += CK_D) {
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < CK_T * CK_D / 4 / 256; ++j) {
+            const int idx = tid + j * 256, t = idx / (CK_D / 4), c = (idx % (CK_D / 4)) * 4;
+            float4 x = make_float4(0.f, 0.f, 0.f, 0.f), y = x;
+            if (t < nt && d0 + c < a.dim) {
+                x = ck_load4<T>(qsrc + (size_t)t * a.ld + d0 + c);
+                y = ck_load4<T>(ksrc + (size_t)t * a.ld + d0 + c);
+                x.x *= a.qscale; x.y *= a.qscale; x.z *= a.qscale; x.w *= a.qscale;
+            }
+            *(float4*)(sq + t * CK_LD + c) = x;
+            *(float4*)(sk + t * CK_LD + c) = y;
+        }
+#pragma unroll
+        for (int j = 0; j < CK_V * CK_D / 4 / 256; ++j) {
+            const int idx = tid + j * 256, v = idx / (CK_D / 4), c = (idx % (CK_D / 4)) * 4;
+            *(float4*)(ss + v * CK_LD + c) = v0 + v < a.vdim && d0 + c < a.dim ? *(const float4*)(src + (size_t)(v0 + v) * a.dim + d0 + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        if (MODE == 3 && tid < CK_D) sg[4 * CK_T + tid] = d0 + tid < a.dim ? nsrc[d0 + tid] : 0.f;
+        __syncthreads();
+        if (MODE == 3) {
+            const float* qr = sq + (tid / 4) * CK_LD + 16 * (tid % 4);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) qn = fmaf(qr[e], sg[4 * CK_T + 16 * (tid % 4) + e], qn);
+        }
+        // a lane reads four neighbouring dimensions at once, the two halves of the wave alternate groups of four
+        for (int dh = 0; dh < CK_D; dh += 32) {
+            ck_f32x16 scx, sox[2];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) scx[i] = sox[0][i] = sox[1][i] = 0.f;
+#pragma unroll
+            for (int d = dh; d < dh + 32; d += 8) {
+                const float4 q0 = *(const float4*)(sq + li * CK_LD + d + 4 * half), q1 = *(const float4*)(sq + (32 + li) * CK_LD + d + 4 * half);
+                const float4 kk = *(const float4*)(sk + (32 * tj + li) * CK_LD + d + 4 * half), sv4 = *(const float4*)(ss + (32 * wave + li) * CK_LD + d + 4 * half);
+                const float qa[2][4] = {{q0.x, q0.y, q0.z, q0.w}, {q1.x, q1.y, q1.z, q1.w}}, ka[4] = {kk.x, kk.y, kk.z, kk.w}, va[4] = {sv4.x, sv4.y, sv4.z, sv4.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (tj <= ti) scx = __builtin_amdgcn_mfma_f32_32x32x2f32(ti ? qa[1][e] : qa[0][e], ka[e], scx, 0, 0, 0);
+                    if (cols) {
+                        sox[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(qa[0][e], va[e], sox[0], 0, 0, 0);
+                        sox[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(qa[1][e], va[e], sox[1], 0, 0, 0);
+                    }
+                }
+            }
+            sc += scx;
+            so[0] += sox[0];
+            so[1] += sox[1];
+        }
+    }
+    __syncthreads();
+    // the weights b_j prod_{j < l <= i} g_l of every pair of tokens, lane j's column row after row (each wave the rows of its quarter), and the values
+    {
+        double r = 0.0;
+        const double bj = sg[CK_T + lane];
+        const int end = 16 * wave + 16;
+#pragma unroll 4
+        for (int i = 0; i < end; ++i) {
+            r = i == lane ? bj : r * sg[i];
+            if (i >= end - 16) sq[i * CK_LD + lane] = i < lane ? 0.f : (float)r;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < CK_T * CK_V / 4 / 256; ++j) {
+        const int idx = tid + j * 256, t = idx / (CK_V / 4), c = (idx % (CK_V / 4)) * 4;
+        *(float4*)(ss + t * CK_LV + c) = t < nt && v0 + c < a.vdim ? ck_load4<T>(vsrc + (size_t)t * a.ld + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        float* w = sq + (32 * ti + 8 * (i / 4) + 4 * half + i % 4) * CK_LD + 32 * tj + li;
+        if (tj <= ti) *w *= sc[i];
+    }
+    ck_f32x16 o[2], o1;                                // the chunk's own share, apart from the state's: of its first 32 tokens, of its last
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[0][i] = o[1][i] = o1[i] = 0.f;
+    __syncthreads();
+    if (MODE == 3) {
+        // n . q after every token: the state's share and the chunk's, four lanes a token
+        const float* w = sq + (tid / 4) * CK_LD + 16 * (tid % 4);
+        float rs = 0.f;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) rs += w[e];
+        float den = fmaf(sg[2 * CK_T + tid / 4], qn, rs);
+        den += row_exchange<0xB1>(den);
+        den += row_exchange<0x4E>(den);
+        if (tid % 4 == 0) sg[3 * CK_T + tid / 4] = fmaxf(fabsf(den), expf(-m_mine)) + a.denom_eps;
+        __syncthreads();
+    }
+    if (!cols) return;
+#pragma unroll 4
+    for (int t = 0; t < CK_T; t += 8) {
+        const float4 w1 = *(const float4*)(sq + (32 + li) * CK_LD + t + 4 * half);
+        const float wa[4] = {w1.x, w1.y, w1.z, w1.w};
+        float x[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = ss[(t + 4 * half + e) * CK_LV + wave * 32 + li];
+        if (t < 32) {                                  // (the first 32 tokens see none of the last 32)
+            const float4 w0 = *(const float4*)(sq + li * CK_LD + t + 4 * half);
+            const float wb[4] = {w0.x, w0.y, w0.z, w0.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                o[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(wb[e], x[e], o[0], 0, 0, 0);
+                o[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(wa[e], x[e], o[1], 0, 0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o1 = __builtin_amdgcn_mfma_f32_32x32x2f32(wa[e], x[e], o1, 0, 0, 0);
+        }
+    }
+    o[1] += o1;
+    const int v = v0 + wave * 32 + li;
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int row = 32 * n + 8 * (i / 4) + 4 * half + i % 4;
+            if (row >= nt || v >= a.vdim) continue;
+            float y = fmaf(sg[2 * CK_T + row], so[n][i], o[n][i]);
+            if (MODE == 3) y /= sg[3 * CK_T + row];
+            a.out[((size_t)(tok0 + row) * a.heads + head) * a.vdim + v] = y;
+        }
+}
+
+// Tokens of a request that one pass over the chunks takes, so that the chunks' states fit the scratch.
+static int chunk_segment(size_t scratch_floats, size_t per_chunk, int requests, int tokens, int longest) {
+    const long fit = (long)(scratch_floats / per_chunk);                     // chunks
+    long len = (longest + CK_T - 1) / CK_T;
+    const long all = tokens / CK_T + requests;                               // most chunks of the step
+    if (all > fit) len = fit / requests < len ? fit / requests : len;
+    return (int)(len * CK_T);
+}
+
+template <typename T, int MODE>
+static int launch_chunks(ChunkArgs a, int tokens, int longest, float* scratch, size_t scratch_floats, hipStream_t stream) {
+    const size_t per_chunk = (size_t)a.heads * ((size_t)a.vdim * a.dim + (MODE == 3 ? a.dim : 0) + 1);
+    a.seg_len = chunk_segment(scratch_floats, per_chunk, a.requests, tokens, longest);
+    TL_REQUIRE(a.seg_len > 0, "chunked scan: scratch of %zu numbers does not hold a chunk of every request", scratch_floats);
+    const long chunks = (long)a.seg_len / CK_T * a.requests < (long)tokens / CK_T + a.requests ? (long)a.seg_len / CK_T * a.requests : (long)tokens / CK_T + a.requests;
+    a.states = scratch;
+    a.sums = scratch + (size_t)chunks * a.heads * a.vdim * a.dim;
+    a.decays = a.sums + (MODE == 3 ? (size_t)chunks * a.heads * a.dim : 0);
+    constexpr size_t smem = sizeof(float) * (2 * CK_T * CK_LD + CK_V * CK_LD + 5 * CK_T);
+    auto outputs = chunk_outputs_kernel<T, MODE>;
+    static hipError_t allowed = hipFuncSetAttribute((const void*)outputs, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    if (allowed != hipSuccess) { tl_set_error("chunked scan: cannot get %zu bytes of shared memory: %s", smem, hipGetErrorString(allowed)); return TL_ERR_HIP; }
+    const dim3 grid(chunks, a.heads, (a.vdim + CK_V - 1) / CK_V);
+    const dim3 pass(MODE == 3 ? (a.dim + 31) / 32 * ((a.vdim + 31) / 32) + 1 : (a.vdim * a.dim / 4 + 255) / 256, a.heads, a.requests);
+    for (a.seg0 = 0; a.seg0 < longest; a.seg0 += a.seg_len) {
+        chunk_states_kernel<T, MODE><<<grid, 256, 0, stream>>>(a);
+        TL_CHECK_LAUNCH("chunk_states");
+        chunk_pass_kernel<MODE == 3><<<pass, 256, 0, stream>>>(a);
+        TL_CHECK_LAUNCH("chunk_pass");
+        outputs<<<grid, 256, smem, stream>>>(a);
+        TL_CHECK_LAUNCH("chunk_outputs");
+    }
+    return TL_OK;
+}
+
+// What the matrix memory's chunks read: per token and head (decay, input factor, running maximum, 0), the maximum taken from the slot's on as a
+// scan over 64 tokens at a time (max-plus: a stretch is the pair (sum of the log forget gates, maximum it brings)), one wave a request and head.
+__global__ void __launch_bounds__(64)
+mlstm_gates_kernel(const float* __restrict__ gates, const float* __restrict__ state, size_t slot_stride, const int* __restrict__ slots,
+                   const int* __restrict__ req_indptr, float4* __restrict__ factors, int heads, int dim, int vdim, float cap, int least) {
+    const int req = blockIdx.y, head = blockIdx.x, lane = threadIdx.x;
+    const int tok0 = req_indptr[req], tok1 = req_indptr[req + 1];
+    if (tok1 - tok0 < least) return;
+    float m = state[(size_t)slots[req] * slot_stride + (size_t)(head + 1) * ((size_t)dim * vdim + dim + 1) - 1];
+    for (int base = tok0; base < tok1; base += TL_WAVE) {
+        const float* g = gates + (size_t)min(base + lane, tok1 - 1) * 2 * heads;
+        const float gi = soft_cap(g[head], cap), gf = log_sigmoid(soft_cap(g[heads + head], cap));
+        float f = gf, i = gi;                          // of the stretch that ends with this lane's token
+#pragma unroll
+        for (int o = 1; o < TL_WAVE; o <<= 1) {
+            const float pf = __shfl_up(f, o, TL_WAVE), pi = __shfl_up(i, o, TL_WAVE);
+            if (lane >= o) { i = fmaxf(pi + f, i); f += pf; }
+        }
+        const float mine = fmaxf(f + m, i);
+        float before = __shfl_up(mine, 1, TL_WAVE);
+        if (lane == 0) before = m;
+        if (base + lane < tok1) factors[(size_t)(base + lane) * heads + head] = make_float4(expf(gf + before - mine), expf(gi - mine), mine, 0.f);
+        m = __shfl(mine, min(TL_WAVE, tok1 - base) - 1, TL_WAVE);
+    }
+}
+
+// Whether a step's long portions go through the chunks: two estimates in us, fitted to the measurements (dim x vdim states; memory: the matrix memory).
+//   token loop, a token: fixed decays 0.18 while the work-groups fit twice on every compute unit, in proportion beyond (one prompt of 512 / 2048 tokens
+//   of 16 heads of 128 x 128: 97 / 372; eight of 400: 141; 16 of 200: 123); the matrix memory 0.58, or 1 per million numbers of state (one prompt of 300
+//   / 2048 tokens of 4 heads of 256 x 512: 189 / 1193; 16 of 130: 1145; 4 of 200 of 8 heads: 1149; 64 of 40: 1136);
+//   chunks: their launches, and the tokens (the same: 54 / 80, 151, 172; 93 / 172, 241, 148, 382).
+extern "C" int tl_chunks_pay(int memory, int tokens, int requests, int longest, int heads, int dim, int vdim) {
+    const double state = (double)heads * dim * vdim, groups = (double)((vdim + DELTA_COLS - 1) / DELTA_COLS) * heads * requests;
+    const double loop = memory ? longest * fmax(0.58, requests * state / 1e6) : longest * 0.18 * fmax(1.0, groups / (2.0 * tl_mlstm_units));
+    const double chunks = memory ? 60 + tokens * 0.08 * state / 524288 : 45 + tokens * 0.038 * state / 262144;
+    return chunks < loop;
+}
+
+// Whether the chunks can be read in whole pieces of four numbers.
+static bool chunks_fit(const void* qkv, int ld, int q_off, int k_off, int v_off, int dim, int vdim, const void* state, long slot_stride, bool columns) {
+    return dim % 4 == 0 && vdim % 4 == 0 && ld % 4 == 0 && q_off % 4 == 0 && k_off % 4 == 0 && v_off % 4 == 0 && ((uintptr_t)qkv & 15) == 0 &&
+           (!columns || (((uintptr_t)state & 15) == 0 && slot_stride % 4 == 0));
+}
+
+// qkv [tokens, ld]: queries at column 0 (heads * dim), keys at k_off, values at v_off (heads * vdim); gates float
+// [tokens, 2 * heads]; state float [slots, heads, dim * vdim + dim + 1] with slot_stride floats between slots;
+// out float [tokens, heads * vdim]; before: scratch of requests * heads * (dim + 1) floats.  Requests whose req_indptr range
+// is empty are left alone.  Requests of at least `least` tokens go through the chunks where the sizes allow it; longest: no fewer tokens than any request of
+// the step brings; scratch (null: the token loop alone): the chunks' states and, from scratch_floats on, the tokens' factors (4 * tokens * heads floats).
+extern "C" int tl_mlstm_scan(const void* qkv, int ld, int k_off, int v_off, const void* gates, void* state, long slot_stride,
+                             const void* slots, const void* before, const void* req_indptr, void* out, int requests, int heads, int dim, int vdim,
+                             float cap, float qscale, float denom_eps, int longest, int tokens, int least, void* scratch, long scratch_floats, int dtype,
+                             hipStream_t stream) {
+    TL_REQUIRE(requests >= 0 && heads > 0 && dim > 0 && vdim > 0 && ld > 0, "mlstm_scan: bad sizes");
+    TL_REQUIRE(dim <= 1024, "mlstm_scan: built for up to 1024 query/key dimensions per head, got %d", dim);
+    TL_REQUIRE(slot_stride >= (long)heads * ((long)dim * vdim + dim + 1), "mlstm_scan: the state rows are too short");
+    TL_REQUIRE(dtype == TL_DT_F32 || dtype == TL_DT_BF16, "mlstm_scan: unknown dtype %d", dtype);
+    if (requests == 0) return TL_OK;
+    const bool chunks = scratch && longest >= least && chunks_fit(qkv, ld, 0, k_off, v_off, dim, vdim, state, slot_stride, false);
+    if (chunks) {
+        float4* factors = (float4*)((float*)scratch + scratch_floats);
+        mlstm_gates_kernel<<<dim3(heads, requests), 64, 0, stream>>>((const float*)gates, (const float*)state, (size_t)slot_stride, (const int*)slots,
+                                                                     (const int*)req_indptr, factors, heads, dim, vdim, cap, least);
+        TL_CHECK_LAUNCH("mlstm_gates");
+        const ChunkArgs a{qkv, ld, 0, k_off, v_off, heads, 1, dim, vdim, (const float*)factors, 4 * heads, 4, 1, 0, nullptr, qscale, denom_eps, (float*)state,
+                          (size_t)slot_stride, (const int*)slots, (const int*)req_indptr, (float*)out, nullptr, nullptr, nullptr, requests, least, 0, 0};
+        const int rc = dtype == TL_DT_F32 ? launch_chunks<float, 3>(a, tokens, longest, (float*)scratch, (size_t)scratch_floats, stream)
+                                          : launch_chunks<bf16_t, 3>(a, tokens, longest, (float*)scratch, (size_t)scratch_floats, stream);
+        if (rc != TL_OK || requests == 1) return rc;
+    }
+    return mlstm_token_loop(qkv, ld, k_off, v_off, gates, state, slot_stride, slots, before, req_indptr, out, requests, heads, dim, vdim, cap, qscale, denom_eps,
+                            chunks ? min(longest, least - 1) : longest, chunks ? least : INT_MAX, dtype, stream);
+}
+
+// ------------------------------------------------------------------ decayed linear attention
+// Per head S <- decay[head] S + k v^T, o = S^T q over the step's tokens, request by request from the state its slot holds: qkv float
+// [T, 2 * heads * dim + heads * vdim] (queries, keys, values, head by head), state as the delta rule's, out float [T, heads * vdim].
+extern "C" int tl_decay_scan(const void* qkv, const void* decay, void* state, long slot_stride, const void* slots, const void* req_indptr,
+                             void* out, int requests, int heads, int dim, int vdim, int longest, int tokens, int least,
+                             void* scratch, long scratch_floats, hipStream_t stream) {
+    TL_REQUIRE(requests >= 0 && heads > 0 && dim > 0 && vdim > 0 && decay, "decay_scan: bad sizes");
+    TL_REQUIRE(dim <= DELTA_L * 16, "decay_scan: built for up to %d query/key dimensions per head, got %d", DELTA_L * 16, dim);
+    TL_REQUIRE(slot_stride >= (long)heads * dim * vdim, "decay_scan: the state rows are too short");
+    TL_REQUIRE(requests <= 65535 && heads <= 65535, "decay_scan: too many requests or heads for one launch");
+    if (requests == 0) return TL_OK;
+    const bool chunks = scratch && longest >= least && chunks_fit(qkv, 2 * heads * dim + heads * vdim, 0, 0, 0, dim, vdim, state, slot_stride, true);
+    if (chunks) {
+        const int rc = launch_chunks<float, 0>(ChunkArgs{qkv, 2 * heads * dim + heads * vdim, 0, heads * dim, 2 * heads * dim, heads, 1, dim, vdim, nullptr, 0, 0, 0, 0,
+            (const float*)decay, 1.f, 0.f, (float*)state, (size_t)slot_stride, (const int*)slots, (const int*)req_indptr, (float*)out, nullptr, nullptr, nullptr,
+            requests, least, 0, 0}, tokens, longest, (float*)scratch, (size_t)scratch_floats, stream);
+        if (rc != TL_OK || requests == 1) return rc;
+    }
+    launch_delta_scan<0>(qkv, nullptr, decay, state, slot_stride, slots, req_indptr, out, requests, heads, heads, dim, vdim, chunks ? min(longest, least - 1) : longest,
+                         chunks ? least : INT_MAX, stream);
+    TL_CHECK_LAUNCH("decay_scan");
+    return TL_OK;
+}
+
+// ------------------------------------------------------------------ selective state-space recurrence (Mamba-2)
+// Per head S <- decay S + dt B x^T (S: state x vdim), y = S^T C + D x, with B and C shared by the heads of a group.  qkv float [T, 2 * groups *
+// state + heads * vdim] as selective_prepare leaves it (C, B, x), gates float [T, 2 * heads] (dt, decay), skip float [heads] (D); the
+// state as the delta rule's ([vdim][state] per head), out float [T, heads * vdim].
+extern "C" int tl_selective_scan(const void* qkv, const void* gates, const void* skip, void* state, long slot_stride, const void* slots,
+                                 const void* req_indptr, void* out, int requests, int heads, int groups, int dim, int vdim, int longest, hipStream_t stream) {
+    TL_REQUIRE(requests >= 0 && heads > 0 && groups > 0 && heads % groups == 0 && dim > 0 && vdim > 0 && gates && skip, "selective_scan: bad sizes");
+    TL_REQUIRE(dim <= DELTA_L * 16, "selective_scan: built for states of up to %d numbers per column, got %d", DELTA_L * 16, dim);
+    TL_REQUIRE(slot_stride >= (long)heads * dim * vdim, "selective_scan: the state rows are too short");
+    TL_REQUIRE(requests <= 65535 && heads <= 65535, "selective_scan: too many requests or heads for one launch");
+    if (requests == 0) return TL_OK;
+    launch_delta_scan<2>(qkv, gates, skip, state, slot_stride, slots, req_indptr, out, requests, heads, groups, dim, vdim, longest, INT_MAX, stream);
+    TL_CHECK_LAUNCH("selective_scan");
     return TL_OK;
 }

@@ -953,9 +953,27 @@ def scaled_add_rmsnorm(residual: torch.Tensor, pending: torch.Tensor | None, alp
 
 # ------------------------------------------------------------- matrix-memory recurrence
 
+# Portions of at least so many tokens go through chunks of 64 tokens in the recurrences with one decay per head and token (the matrix memory, fixed
+# decays), where a step's sizes make that the faster way; the chunks' states stand in scratch of at most so many 32-bit numbers (256 MiB), and tokens
+# beyond wait for another pass over it.
+CHUNKED_FROM = 32
+CHUNK_SCRATCH = 1 << 26
+
+
+def _chunk_scratch(lib, memory: bool, tokens: int, requests: int, longest: int, heads: int, dim: int, vdim: int, more: int, device):
+    """Scratch for the chunks of a step's long portions (``None``: the token loop takes them all), and how many of its numbers are the chunks'."""
+    if longest < CHUNKED_FROM or not lib.tl_chunks_pay(c_int(1 if memory else 0), c_int(tokens), c_int(requests), c_int(longest), c_int(heads), c_int(dim), c_int(vdim)):
+        return None, 0
+    per_chunk = heads * (dim * vdim + (dim if memory else 0) + 1)
+    chunks = min(-(-longest // 64) * requests, tokens // 64 + requests)
+    floats = max(min(chunks, CHUNK_SCRATCH // per_chunk), requests) * per_chunk
+    floats = -(-floats // 4) * 4
+    return torch.empty(floats + more, dtype=torch.float32, device=device), floats
+
+
 def mlstm_scan(qkv: torch.Tensor, k_off: int, v_off: int, gates: torch.Tensor, state: torch.Tensor, slots: torch.Tensor,
                req_indptr: torch.Tensor, out: torch.Tensor, heads: int, dim: int, vdim: int, cap: float | None,
-               qscale: float, denom_eps: float) -> None:
+               qscale: float, denom_eps: float, max_new_tokens: int | None = None) -> None:
     """The matrix-memory recurrence over the step's tokens, request by request from the state its slot holds:
     ``qkv [T, >=]`` holds per token the queries at column 0 (``heads * dim``), the keys at ``k_off`` and the values at
     ``v_off`` (``heads * vdim``); ``gates`` float32 ``[T, 2 * heads]`` the raw input and forget gates (bias added);
@@ -976,10 +994,12 @@ def mlstm_scan(qkv: torch.Tensor, k_off: int, v_off: int, gates: torch.Tensor, s
     _i32(req_indptr, "req_indptr", R + 1)
     lib = _lib("recurrent")
     before = torch.empty((R, heads, dim + 1), dtype=torch.float32, device=qkv.device)      # n and m as the step finds them
+    longest = max(1, T - R + 1) if max_new_tokens is None else max_new_tokens
+    scratch, floats = _chunk_scratch(lib, True, T, R, longest, heads, dim, vdim, 4 * T * heads, qkv.device)
     _check(lib, lib.tl_mlstm_scan(_ptr(qkv), c_int(qkv.stride(0)), c_int(k_off), c_int(v_off), _ptr(gates), _ptr(state),
                                   ctypes.c_long(state.stride(0)), _ptr(slots), _ptr(before), _ptr(req_indptr), _ptr(out), c_int(R), c_int(heads),
                                   c_int(dim), c_int(vdim), c_float(cap if cap else 0.0), c_float(qscale), c_float(denom_eps),
-                                  c_int(max(1, T - R + 1)), c_int(_dt(qkv, "mlstm_scan")), _stream()))
+                                  c_int(longest), c_int(T), c_int(CHUNKED_FROM), _ptr(scratch), ctypes.c_long(floats), c_int(_dt(qkv, "mlstm_scan")), _stream()))
 
 
 GATES = {"sigmoid": 0, "silu": 1}
@@ -1090,9 +1110,11 @@ def decay_scan(qkv: torch.Tensor, decay: torch.Tensor, state: torch.Tensor, slot
     _i32(slots, "slots", R)
     _i32(req_indptr, "req_indptr", R + 1)
     lib = _lib("recurrent")
+    longest = max(1, T - R + 1) if max_new_tokens is None else max_new_tokens
+    scratch, floats = _chunk_scratch(lib, False, T, R, longest, heads, dim, vdim, 0, qkv.device)
     _check(lib, lib.tl_decay_scan(_ptr(qkv), _ptr(decay), _ptr(state), ctypes.c_long(state.stride(0)), _ptr(slots), _ptr(req_indptr), _ptr(out),
-                                  c_int(R), c_int(heads), c_int(dim), c_int(vdim),
-                                  c_int(max(1, T - R + 1) if max_new_tokens is None else max_new_tokens), _stream()))
+                                  c_int(R), c_int(heads), c_int(dim), c_int(vdim), c_int(longest), c_int(T), c_int(CHUNKED_FROM), _ptr(scratch),
+                                  ctypes.c_long(floats), _stream()))
 
 
 def selective_prepare(proj: torch.Tensor, x_off: int, conv_w: torch.Tensor, conv_b: torch.Tensor, gates: torch.Tensor, a_log: torch.Tensor,
