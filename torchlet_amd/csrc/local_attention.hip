@@ -11,6 +11,8 @@
 // row b of planes of their own with a block table of their own (pool_blocks_kernel makes them when a step brings a block's last token).
 // A third one: values that lie in the cache turned by their own positions; a head's output at position p is turned back by p.
 // A fourth one: a gate per head; a token's output of head h is multiplied by sigmoid(gate[token, h]).
+#include <limits.h>
+
 #include "common.h"
 
 // ------------------------------------------------------------------ cache write
@@ -238,7 +240,7 @@ local_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __re
                             const int* __restrict__ tile_tok0, int heads, int kv_heads, int page_size, float scale, float cap,
                             LocalMask mask, float gain, const float* __restrict__ sink, const bf16_t* __restrict__ pk_plane,
                             const bf16_t* __restrict__ pv_plane, const int* __restrict__ pool_table, int pool_table_ld, int pool_table_width, int pool,
-                            OutputTurn back, const bf16_t* __restrict__ gate, int gate_ld) {
+                            OutputTurn back, const bf16_t* __restrict__ gate, int gate_ld, int below) {
     constexpr int dim = DK * 32, vdim = DV * 16;
     extern __shared__ float la_smem[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, kq = lane >> 4;
@@ -248,7 +250,7 @@ local_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __re
     const int first = req_indptr[req], n_new = req_indptr[req + 1] - first;
     const int tok0 = tile_tok0 ? tile_tok0[tile] : 0;
     const int n_tile = min(LAM_TOKENS, n_new - tok0);            // tokens of this tile
-    if (n_tile <= 0) return;
+    if (n_tile <= 0 || n_new >= below) return;                   // (requests of `below` tokens or more are local_prompt_kernel's)
     const int g = head / (heads / kv_heads);
     const int p0 = ctx_lens[req] + tok0;                         // position of the tile's first token
     const int my_tok = min(li, n_tile - 1);                      // (lanes beyond the tile's tokens repeat its last one and store nothing)
@@ -435,7 +437,7 @@ static void launch_local_mfma(const void* q, int q_ld, void* out, int out_ld, co
                               int table_ld, int table_width, const void* req_indptr, const void* ctx_lens, const void* tile_req,
                               const void* tile_tok0, int tiles, int heads, int kv_heads, int page_size, float scale, float cap, LocalMask mask,
                               float gain, const void* sink, const void* pk_plane, const void* pv_plane, const void* pool_table, int pool_table_ld,
-                              int pool_table_width, int pool, OutputTurn back, const void* gate, int gate_ld, hipStream_t stream) {
+                              int pool_table_width, int pool, OutputTurn back, const void* gate, int gate_ld, int below, hipStream_t stream) {
     dim3 grid(tiles, heads), block(LAM_WAVES * TL_WAVE);
     const size_t smem = sizeof(float) * LAM_WAVES * LAM_TOKENS * (2 + DV * 16);
     auto kernel = local_attention_mfma_kernel<DK, DV>;
@@ -447,7 +449,7 @@ static void launch_local_mfma(const void* q, int q_ld, void* out, int out_ld, co
     kernel<<<grid, block, smem, stream>>>((const bf16_t*)q, q_ld, (bf16_t*)out, out_ld, (const bf16_t*)k_plane, (const bf16_t*)v_plane,
         (const int*)block_table, table_ld, table_width, (const int*)req_indptr, (const int*)ctx_lens, (const int*)tile_req, (const int*)tile_tok0,
         heads, kv_heads, page_size, scale, cap, mask, gain, (const float*)sink, (const bf16_t*)pk_plane, (const bf16_t*)pv_plane, (const int*)pool_table,
-        pool_table_ld, pool_table_width, pool, back, (const bf16_t*)gate, gate_ld);
+        pool_table_ld, pool_table_width, pool, back, (const bf16_t*)gate, gate_ld, below);
 }
 
 // Whether the matrix-core kernel is built for these sizes.
@@ -455,6 +457,416 @@ extern "C" int tl_local_attention_mfma_fits(int dim, int vdim, int page_size) {
     const bool dk = dim == 32 || dim == 64 || dim == 96 || dim == 128 || dim == 192 || dim == 256;
     const bool dv = vdim > 0 && vdim % 16 == 0 && (vdim <= 128 || vdim == 160 || vdim == 192 || vdim == 256);
     return dk && dv && page_size % 8 == 0;
+}
+
+// ------------------------------------------------------------------ long portions of prompts: 128 rows a work-group
+// The same attention for requests that bring LP_LEAST tokens or more in a step that is large enough (local_prompt_pays).  A row is a token and one of up to gcap heads of a key/value
+// head; four waves of 32 rows share steps of KEYS keys, which go from the pages straight into shared memory (STAGES steps of it, so that the next
+// ones are on their way while this one is multiplied; 16-byte pieces whose slot in a row is exclusive-ored with the row against bank conflicts).
+// Both products run transposed on v_mfma_f32_32x32x16_bf16: a lane owns one row (its maximum, sum and output), and the keys are dealt to the
+// rows of the first product so that the weights a lane holds are the second product's operand as they stand (row 8 a + 4 h + b of a block of 32
+// carries key 16 (a / 2) + 8 h + 4 (a % 2) + b).  The tile kernel above reads its operands from the caches for every 16 tokens of every head, and that
+// traffic set its time; here 128 rows share them, and the matrix and vector units take turns at being the bound (0.8 PFLOP/s on long prompts).
+// Measured against it, 32 heads of 128 over 8: a prompt of 4096 tokens 918 -> 172 us, 2048 305 -> 58, with a window of 512 181 -> 36; 64 heads of
+// 192 / 128, 2048 tokens 817 -> 123.
+// A tile takes up to three stretches of keys one after the other, each with limits of its own per row: the pooled blocks before the window, the
+// kept first tokens, the tokens themselves.  Late tiles start first.
+#define LP_ROWS 128
+#define LP_BT_MAX 2048               // block-table entries of a stretch in shared memory
+#define LP_LEAST 32                  // tokens of a request in a step
+#define LP_HEADS_MOST 16             // heads of a tile
+#define LP_SLACK 8.f                 // powers of two a row's scores may rise above its reference before it is moved
+
+typedef float la_f32x16 __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ void lp_load_to_lds(const void* base, unsigned offset, unsigned lds_addr) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(offset), "s"(base), "s"(lds_addr) : "memory", "m0");
+}
+
+struct LocalArgs {
+    const bf16_t* q;
+    int q_ld;
+    bf16_t* out;
+    int out_ld;
+    const bf16_t *k_plane, *v_plane;
+    const int* block_table;
+    int table_ld, table_width;
+    const int *req_indptr, *ctx_lens;
+    int requests, heads, kv_heads, gcap, page_size, page_shift;
+    float scale, cap;
+    LocalMask mask;
+    float gain;
+    const float* sink;
+    const bf16_t *pk_plane, *pv_plane;
+    const int* pool_table;
+    int pool_table_ld, pool_table_width, pool;
+    OutputTurn back;
+    const bf16_t* gate;
+    int gate_ld, least;
+};
+
+template <int DIM, int VDIM, int KEYS, int STAGES, bool CAP>
+__global__ void __launch_bounds__(256, 2)
+local_prompt_kernel(LocalArgs a) {
+    constexpr int KB = KEYS / 32, NC = DIM / 16, NB = VDIM / 32;      // blocks of keys; pieces of a score's sum; blocks of output columns
+    constexpr int KPP = DIM / 8, VPP = KEYS / 8;                      // 16-byte pieces of a key row, of a row of transposed values
+    constexpr int KBYTES = KEYS * DIM * 2, STAGE = KBYTES + VDIM * KEYS * 2;
+    constexpr int KI = KBYTES / 4096, VI = VDIM * KEYS * 2 / 4096, NI = KI + VI;      // load instructions of a wave and step
+    static_assert(KBYTES % 4096 == 0 && (VDIM * KEYS * 2) % 4096 == 0 && NI * (STAGES - 1) < 64, "whole instructions of four waves");
+    extern __shared__ __attribute__((aligned(16))) unsigned char lp_smem[];
+    int* bt = (int*)(lp_smem + STAGES * STAGE);
+    const unsigned lds_base = (unsigned)(uintptr_t)((void __attribute__((address_space(3)))*)lp_smem);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 31, h = lane >> 5;
+    auto key_slot = [](int piece, int key) { return DIM == 128 ? (piece ^ (key & 15)) : ((piece & ~7) | ((piece ^ (key >> 1)) & 7)); };
+    auto value_slot = [](int piece, int d) { return KEYS == 64 ? (piece ^ ((d >> 1) & 7)) : (piece ^ ((d >> 2) & 3)); };
+
+    // ---- which tile: the requests' tiles are counted by a prefix sum over the lanes; the last tile first, each with all its heads
+    const int group = a.heads / a.kv_heads, chunks_h = (group + a.gcap - 1) / a.gcap, per_tile = a.kv_heads * chunks_h, tq = LP_ROWS / a.gcap;
+    int total = 0;
+    for (int base = 0; base < a.requests; base += TL_WAVE) {
+        const int r = base + lane;
+        const int n = r < a.requests ? a.req_indptr[r + 1] - a.req_indptr[r] : 0;
+        int mine = n >= a.least ? (n + tq - 1) / tq : 0;
+#pragma unroll
+        for (int o = TL_WAVE / 2; o > 0; o >>= 1) mine += __shfl_xor(mine, o, TL_WAVE);
+        total += __builtin_amdgcn_readfirstlane(mine);
+    }
+    if ((int)blockIdx.x >= total * per_tile) return;
+    const int want = total - 1 - (int)blockIdx.x / per_tile, by = blockIdx.x % per_tile;
+    int req = 0, tok0 = 0;
+    {
+        int first = 0;
+        for (int base = 0; base < a.requests; base += TL_WAVE) {
+            const int r = base + lane;
+            const int n = r < a.requests ? a.req_indptr[r + 1] - a.req_indptr[r] : 0;
+            const int mine = n >= a.least ? (n + tq - 1) / tq : 0;
+            int upto = mine;
+#pragma unroll
+            for (int o = 1; o < TL_WAVE; o <<= 1) {
+                const int t = __shfl_up(upto, o, TL_WAVE);
+                if (lane >= o) upto += t;
+            }
+            const unsigned long long past = __ballot(first + upto > want);
+            if (past) {
+                const int l = __builtin_amdgcn_readfirstlane(__ffsll(past) - 1);
+                req = base + l;
+                tok0 = (want - first - __builtin_amdgcn_readlane(upto, l) + __builtin_amdgcn_readlane(mine, l)) * tq;
+                break;
+            }
+            first += __builtin_amdgcn_readlane(upto, TL_WAVE - 1);
+        }
+    }
+    const int g = by / chunks_h, g0 = by % chunks_h * a.gcap, gcount = min(a.gcap, group - g0);
+    const int first = a.req_indptr[req], n_new = a.req_indptr[req + 1] - first, ctx = a.ctx_lens[req];
+    const int ntok = min(tq, n_new - tok0), p0 = ctx + tok0, p_last = p0 + ntok - 1;
+
+    const int row = wave * 32 + lr, r_tok = row / a.gcap, r_g = row % a.gcap;
+    const bool row_ok = r_tok < ntok && r_g < gcount;
+    const int r_pos = p0 + r_tok, r_head = g * group + g0 + r_g, r_token = first + tok0 + r_tok;
+    const bool wave_has_rows = (wave * 32) / a.gcap < ntok;
+    const int w_pos_min = p0 + min((wave * 32) / a.gcap, ntok - 1), w_pos_max = p0 + min((wave * 32 + 31) / a.gcap, ntok - 1);
+
+    la_bf16x8 qf[NC];                        // my row's query: d = 16 c + 8 h .. + 7
+    {
+        const bf16_t* q = a.q + (size_t)r_token * a.q_ld + (size_t)r_head * DIM;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            LaFrag f;
+            f.u = row_ok ? *(const uint4*)(q + 16 * c + 8 * h) : make_uint4(0, 0, 0, 0);
+            qf[c] = f.v;
+        }
+    }
+    // (waited for here, once: see the wait at a loop's head that the compiler would otherwise place)
+#pragma unroll
+    for (int c = 0; c < NC; ++c) asm volatile("" : "+v"(qf[c]));
+
+    // what of a piece's address does not change from step to step: its key within the step, and bytes from the start of its page
+    const int shift = a.page_shift, pmask = a.page_size - 1;
+    unsigned k_off[KI], v_off[VI];
+    int k_x[KI];
+    int v_x;                                 // (the same in every value load of a lane: a piece's slot depends on the row's low bits alone)
+#pragma unroll
+    for (int j = 0; j < KI; ++j) {
+        const int piece = (wave + 4 * j) * 64 + lane, kx = piece / KPP;
+        k_x[j] = kx;
+        k_off[j] = (unsigned)((g * a.page_size + (kx & pmask)) * DIM + key_slot(piece % KPP, kx) * 8) * 2u;
+    }
+#pragma unroll
+    for (int j = 0; j < VI; ++j) {
+        const int piece = (wave + 4 * j) * 64 + lane, d = piece / VPP, x = 8 * value_slot(piece % VPP, d);
+        if (j == 0) v_x = x;
+        v_off[j] = (unsigned)((g * VDIM + d) * a.page_size + (x & pmask)) * 2u;
+    }
+    const unsigned kpage = (unsigned)(a.kv_heads * a.page_size * DIM) * 2u, vpage = (unsigned)(a.kv_heads * a.page_size * VDIM) * 2u;
+    const int krow = 16 * (lr >> 4) + 8 * ((lr >> 2) & 1) + 4 * ((lr >> 3) & 1) + (lr & 3);      // key that row lr of the first product carries
+
+    // scores in units of log 2: with a cap they are capped first and then stand as they are, without one the factor goes into the exponent
+    const float inv_cap = CAP ? 2.f * LA_LOG2E / a.cap : 0.f, scale2 = CAP ? 1.f : a.scale * LA_LOG2E;
+    float m = -INFINITY, l = 0.f;
+    la_f32x16 acc[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[b][v] = 0.f;
+
+    for (int phase = 0; phase < 3; ++phase) {
+        const bf16_t *kp = a.k_plane, *vp = a.v_plane;
+        const int* tbl = a.block_table + (size_t)req * a.table_ld;
+        int width = a.table_width, key_lo = 0, key_hi = 0;            // the tile reads keys key_lo .. key_hi - 1, ...
+        int r_lo = 0, r_hi = -1, w_lo_max = 0, w_lo_min = 0, w_hi_min = -1, w_hi_max = -1;      // ... a row r_lo .. r_hi, and over the wave's rows
+        if (phase == 0) {
+            if (a.pool == 0 || a.mask.window == 0) continue;
+            kp = a.pk_plane; vp = a.pv_plane;
+            tbl = a.pool_table + (size_t)req * a.pool_table_ld;
+            width = a.pool_table_width;
+            auto blocks = [&](int p) { return max(0, p - a.mask.window + 1) / a.pool; };
+            key_hi = blocks(p_last);
+            r_hi = blocks(r_pos) - 1; w_hi_min = blocks(w_pos_min) - 1; w_hi_max = blocks(w_pos_max) - 1;
+        } else if (phase == 1) {
+            if (a.mask.keep_first == 0 || a.mask.window == 0) continue;
+            auto kept = [&](int p) { return min(a.mask.keep_first, a.mask.first(p)); };
+            key_hi = kept(p_last);
+            r_hi = kept(r_pos) - 1; w_hi_min = kept(w_pos_min) - 1; w_hi_max = kept(w_pos_max) - 1;
+        } else {
+            key_lo = a.mask.first(p0);
+            key_hi = p_last + 1;
+            r_lo = a.mask.first(r_pos); r_hi = r_pos;
+            w_lo_min = a.mask.first(w_pos_min); w_lo_max = a.mask.first(w_pos_max);
+            w_hi_min = w_pos_min; w_hi_max = w_pos_max;
+        }
+        if (key_hi <= key_lo) continue;
+        const int st_first = key_lo / KEYS, st_last = (key_hi + KEYS - 1) / KEYS;
+        const int blk0 = (st_first * KEYS) >> shift, blk_n = ((key_hi - 1) >> shift) - blk0 + 1, blk_last = blk_n - 1;
+        if (blk_n > LP_BT_MAX || blk0 + blk_n > width) continue;      // (the host has seen to it that this cannot be)
+        __syncthreads();                                              // the stretch before has been worked on
+        for (int i = threadIdx.x; i < blk_n; i += 256) bt[i] = tbl[max(blk0 + i, key_lo >> shift)];      // (pages before the first key may be gone)
+        __syncthreads();
+        int pg_k[KI], pg_v;
+        auto look_up_one = [&](int st, int j) {
+            const int first_key = st * KEYS - (blk0 << shift);
+            if (j < KI) pg_k[j] = bt[min((first_key + k_x[j]) >> shift, blk_last)];
+            else pg_v = bt[min((first_key + v_x) >> shift, blk_last)];
+        };
+        auto request_one = [&](int st, int buf, int j) {              // (after the step's look-ups)
+            const unsigned sb = lds_base + buf * STAGE;
+            const unsigned uin = KEYS < a.page_size ? (unsigned)((st * KEYS) & pmask) : 0u;      // the step's first key's place in a longer page
+            if (j < KI) lp_load_to_lds(kp + (size_t)uin * DIM, (unsigned)pg_k[j] * kpage + k_off[j], sb + (wave + 4 * j) * 1024);
+            else lp_load_to_lds(vp + uin, (unsigned)pg_v * vpage + v_off[j - KI], sb + KBYTES + (wave + 4 * (j - KI)) * 1024);
+        };
+        auto look_up = [&](int st) {
+#pragma unroll
+            for (int j = 0; j <= KI; ++j) look_up_one(st, j);
+        };
+        // steps are requested STAGES - 1 ahead; past the end the last one again (nobody reads it), so that every wait is for the same count
+#pragma unroll
+        for (int i = 0; i < STAGES - 1; ++i) {
+            const int st = min(st_first + i, st_last - 1);
+            look_up(st);
+#pragma unroll
+            for (int j = 0; j < NI; ++j) request_one(st, i, j);
+        }
+        look_up(min(st_first + STAGES - 1, st_last - 1));
+        asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NI * (STAGES - 2)) : "memory");
+        __syncthreads();
+        for (int st = st_first; st < st_last; ++st) {
+            const int buf = (st - st_first) % STAGES, buf_req = (st - st_first + STAGES - 1) % STAGES;
+            const int st_req = min(st + STAGES - 1, st_last - 1), st_look = min(st + STAGES, st_last - 1), kbase = st * KEYS;
+            unsigned char *kb_s = lp_smem + buf * STAGE, *vb_s = kb_s + KBYTES;
+            if (kbase + KEYS > key_hi || kbase < key_lo) {
+                // keys beyond the stretch's last may not be written yet, and the pages of those before its first may be gone: whatever lies there
+                // must not reach the second product (0 * Inf), so their values count as zero
+                for (int i = threadIdx.x; i < VDIM * VPP; i += 256) {
+                    const int d = i / VPP, piece = i % VPP, k0 = kbase + 8 * piece;
+                    if (k0 + 8 > key_hi || k0 < key_lo) {
+                        LaFrag f;
+                        uint4* ptr = (uint4*)(vb_s + d * (KEYS * 2) + value_slot(piece, d) * 16);
+                        f.u = *ptr;
+#pragma unroll
+                        for (int e = 0; e < 8; ++e)
+                            if (k0 + e >= key_hi || k0 + e < key_lo) f.e[e] = 0;
+                        *ptr = f.u;
+                    }
+                }
+                __syncthreads();
+            }
+            if (wave_has_rows && kbase <= w_hi_max && kbase + KEYS > w_lo_min) {
+                la_f32x16 sc[KB];
+#pragma unroll
+                for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) sc[kb][v] = 0.f;
+                constexpr int KAHEAD = 2;                 // a block's keys are read two products ahead
+                LaFrag kf[KAHEAD + 1][KB];
+                auto read_keys = [&](int c, int kb) {
+                    const int kl = 32 * kb + krow;
+                    kf[c % (KAHEAD + 1)][kb].u = *(const uint4*)(kb_s + kl * (DIM * 2) + key_slot(2 * c + h, kl) * 16);
+                };
+#pragma unroll
+                for (int c = 0; c < KAHEAD; ++c)
+#pragma unroll
+                    for (int kb = 0; kb < KB; ++kb) read_keys(c, kb);
+                __builtin_amdgcn_sched_barrier(0);
+                constexpr int EVERY = NC * KB / NI;       // a request beside every so many products
+                static_assert(EVERY >= 1, "a product for every request");
+#pragma unroll
+                for (int c = 0; c < NC; ++c)
+#pragma unroll
+                    for (int kb = 0; kb < KB; ++kb) {
+                        sc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[c % (KAHEAD + 1)][kb].v, qf[c], sc[kb], 0, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (c + KAHEAD < NC) read_keys(c + KAHEAD, kb);
+                        const int at = c * KB + kb;
+                        if (at % EVERY == 0 && at / EVERY < NI) request_one(st_req, buf_req, at / EVERY);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                if (CAP) {
+#pragma unroll
+                    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) sc[kb][e] = cap_score_fast(sc[kb][e] * a.scale, a.cap, inv_cap) * LA_LOG2E;
+                }
+                float mloc = -INFINITY;
+                if (kbase + KEYS - 1 <= w_hi_min && kbase >= w_lo_max) {
+#pragma unroll
+                    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) mloc = fmaxf(mloc, sc[kb][e]);
+                } else {
+#pragma unroll
+                    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) {
+                            const int key = kbase + 32 * kb + 16 * (e >> 3) + 8 * h + 4 * ((e >> 2) & 1) + (e & 3);
+                            sc[kb][e] = (row_ok && key <= r_hi && key >= r_lo) ? sc[kb][e] : -INFINITY;
+                            mloc = fmaxf(mloc, sc[kb][e]);
+                        }
+                }
+                {
+                    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(mloc), __float_as_uint(mloc), false, false);
+                    mloc = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])) * scale2;
+                }
+                // m is the row's reference for the exponents, not its maximum: it moves only when some row of the wave rises more than LP_SLACK above
+                // its own, so most steps rescale nothing; the quotient at the end is the same
+                if (__any(mloc > m + LP_SLACK)) {
+                    const float m_new = fmaxf(m, mloc);
+                    const float alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - m_new);
+                    m = m_new;
+                    l *= alpha;
+#pragma unroll
+                    for (int b = 0; b < NB; ++b) acc[b] *= alpha;
+                }
+                const float m_use = m == -INFINITY ? 0.f : -m;      // (nothing seen yet: every score is -inf)
+                LaFrag pf[2 * KB];
+                float psum = 0.f;
+                auto weights = [&](int kb, int e0, int n) {
+#pragma unroll
+                    for (int e = e0; e < e0 + n; ++e) {
+                        const __bf16 w = (__bf16)__builtin_amdgcn_exp2f(__builtin_fmaf(sc[kb][e], scale2, m_use));
+                        psum += (float)w;                            // the sum of what the second product sees
+                        pf[2 * kb + (e >> 3)].v[e & 7] = w;
+                    }
+                };
+                // values: product i takes the columns 32 (i % NB) .. + 31 for the 16 keys of chunk i / NB, read two products ahead; the weights of a later
+                // block and the next step's look-ups stand beside the products
+                constexpr int NPV = 2 * KB * NB, VAHEAD = 2, PER = 16 / (2 * NB);
+                LaFrag vf[VAHEAD + 1];
+                auto read_values = [&](int i) {
+                    const int d = 32 * (i % NB) + lr;
+                    vf[i % (VAHEAD + 1)].u = *(const uint4*)(vb_s + d * (KEYS * 2) + value_slot(2 * (i / NB) + h, d) * 16);
+                };
+#pragma unroll
+                for (int i = 0; i < VAHEAD; ++i) read_values(i);
+                weights(0, 0, 16);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < NPV; ++i) {
+                    acc[i % NB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i % (VAHEAD + 1)].v, pf[i / NB].v, acc[i % NB], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (i + VAHEAD < NPV) read_values(i + VAHEAD);
+                    const int kb = i / (2 * NB), within = i % (2 * NB);
+                    if (kb + 1 < KB) weights(kb + 1, within * PER, PER);
+                    else {
+                        constexpr int LOOKS = (KI + 1 + 2 * NB - 1) / (2 * NB);
+#pragma unroll
+                        for (int u = 0; u < LOOKS; ++u)
+                            if (within * LOOKS + u <= KI) look_up_one(st_look, within * LOOKS + u);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                l += psum;
+            } else {
+#pragma unroll
+                for (int j = 0; j < NI; ++j) request_one(st_req, buf_req, j);
+                look_up(st_look);
+            }
+            asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NI * (STAGES - 2)) : "memory");
+            __syncthreads();
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    l += __shfl_xor(l, 32, TL_WAVE);
+    if (!row_ok) return;
+    // lane holds column 32 b + 8 q + 4 h + v of its row
+    float norm = a.gain;
+    if (a.sink) {
+        const float sink2 = a.sink[r_head] * LA_LOG2E, top = fmaxf(m, sink2), keep = __builtin_amdgcn_exp2f(m - top);
+        l = l * keep + __builtin_amdgcn_exp2f(sink2 - top);
+        norm *= keep;
+    }
+    norm /= l;
+    if (a.gate) norm *= sigmoid(to_float(a.gate[(size_t)r_token * a.gate_ld + r_head]));
+    bf16_t* o = a.out + (size_t)r_token * a.out_ld + (size_t)r_head * VDIM;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int col = 32 * b + 8 * q + 4 * h;
+            float y[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) y[v] = acc[b][4 * q + v] * norm;
+            if (a.back.freq) {                           // (pairs of neighbours: the host has seen to it)
+                a.back.turn(col / 2, r_pos, y[0], y[1]);
+                a.back.turn(col / 2 + 1, r_pos, y[2], y[3]);
+            }
+            union { uint2 u; uint16_t e[4]; } pk;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) pk.e[v] = from_float<bf16_t>(y[v]).bits;
+            *(uint2*)(o + col) = pk.u;
+        }
+}
+
+template <int DIM, int VDIM, int KEYS, int STAGES>
+static int launch_local_prompt(const LocalArgs& a, long tokens, hipStream_t stream) {
+    constexpr size_t smem = (size_t)STAGES * (KEYS * DIM * 2 + VDIM * KEYS * 2) + LP_BT_MAX * 4;
+    auto kernel = a.cap > 0.f ? local_prompt_kernel<DIM, VDIM, KEYS, STAGES, true> : local_prompt_kernel<DIM, VDIM, KEYS, STAGES, false>;
+    static const hipError_t allowed[2] = {
+        hipFuncSetAttribute((const void*)local_prompt_kernel<DIM, VDIM, KEYS, STAGES, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem),
+        hipFuncSetAttribute((const void*)local_prompt_kernel<DIM, VDIM, KEYS, STAGES, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem)};
+    if (allowed[0] != hipSuccess || allowed[1] != hipSuccess) { tl_set_error("local_prompt: cannot get %zu bytes of shared memory", smem); return TL_ERR_HIP; }
+    const int group = a.heads / a.kv_heads, tq = LP_ROWS / a.gcap;
+    const long tiles = tokens / tq + (a.requests < tokens / a.least ? a.requests : tokens / a.least);
+    if (tiles > 0) kernel<<<dim3((unsigned)(tiles * a.kv_heads * ((group + a.gcap - 1) / a.gcap))), 256, smem, stream>>>(a);
+    TL_CHECK_LAUNCH("local_prompt");
+    return TL_OK;
+}
+
+// From where the kernel of 128 rows is the faster one: three of the tile kernel's work-groups (16 tokens of a head) to a CU.  That kernel deals a
+// tile's keys to four waves and so fills the chip with few tokens already: with 32 heads over 8, 4000 cached tokens, 128 new ones take 55 us in it and
+// 83 us here, 256 take 110 / 87, 512 take 206 / 94; 256 new ones beside 31 decoded tokens at 2000, where both kernels run, 189 / 207.  Tokens that
+// must be decoded ones (all requests' but one each) do not count; a request of LP_LEAST tokens is where a step may hold no decoded ones at all
+// (8 x 32 tokens of 64 heads after 1000: 94 / 54 us; below, most of a tile's rows would be empty).
+static bool local_prompt_pays(const LocalArgs& a, long tokens) {
+    const long more = tokens - a.requests + 1;
+    return more >= LP_LEAST && more * a.heads >= 12288;
+}
+
+// Whether the kernel of 128 rows is built for these sizes: pages of a power of two of 8 keys or more, planes whose bytes 32 bits count, a request's
+// blocks in its shared memory, a positive factor on the scores, outputs turned in neighbouring pairs.
+static bool local_prompt_fits(const LocalArgs& a, int dim, int vdim, int pages, int pool_pages) {
+    const bool sizes = (dim == 128 && vdim == 128) || (dim == 64 && vdim == 64) || (dim == 192 && vdim == 128);
+    const long most = (long)(pages > pool_pages ? pages : pool_pages) * a.kv_heads * a.page_size * (dim > vdim ? dim : vdim) * 2;
+    return sizes && a.page_size >= 8 && (a.page_size & (a.page_size - 1)) == 0 && most < (1L << 32) && a.table_width <= LP_BT_MAX &&
+           a.pool_table_width <= LP_BT_MAX && a.scale > 0.f && !(a.back.freq && a.back.halves) && a.out_ld % 4 == 0 && ((uintptr_t)a.out % 8) == 0;
 }
 
 // Tiles of up to 16 consecutive tokens of one request: tile i belongs to request tile_req[i] (null: request i) and starts at that
@@ -465,7 +877,7 @@ extern "C" int tl_local_attention_tiles(const void* q, int q_ld, void* out, int 
                                         int page_size, float scale, float cap, int chunk, int window, float gain, const void* sink,
                                         const void* pk_plane, const void* pv_plane, const void* pool_table, int pool_table_ld, int pool_table_width,
                                         int pool, int keep_first, const void* turn_freq, int turn_dims, int turn_halves, const void* gate, int gate_ld,
-                                        hipStream_t stream) {
+                                        int tokens, int requests, int pool_pages, hipStream_t stream) {
     TL_REQUIRE(!gate || gate_ld >= heads, "local_attention_tiles: a gate has a number per head");
     TL_REQUIRE(!turn_freq || (turn_dims > 0 && turn_dims % 2 == 0 && turn_dims <= vdim && vdim % 2 == 0), "local_attention_tiles: an output of %d columns turned over %d", vdim, turn_dims);
     TL_REQUIRE(keep_first >= 0 && (keep_first == 0 || (window > 0 && chunk == 0)), "local_attention_tiles: kept first tokens stand beside a window, without chunks");
@@ -478,10 +890,24 @@ extern "C" int tl_local_attention_tiles(const void* q, int q_ld, void* out, int 
     if (tiles == 0) return TL_OK;
     const LocalMask mask{chunk, window, keep_first};
     const OutputTurn back{(const float*)turn_freq, turn_dims, turn_halves};
+    TL_REQUIRE(tokens >= 0 && requests >= 0 && pool_pages >= 0, "local_attention_tiles: bad sizes");
+    const int group = heads / kv_heads, cut = (group + LP_HEADS_MOST - 1) / LP_HEADS_MOST;
+    const LocalArgs a{(const bf16_t*)q, q_ld, (bf16_t*)out, out_ld, (const bf16_t*)k_plane, (const bf16_t*)v_plane, (const int*)block_table, table_ld,
+                      table_width, (const int*)req_indptr, (const int*)ctx_lens, requests, heads, kv_heads, (group + cut - 1) / cut, page_size,
+                      __builtin_ctz(page_size), scale, cap, mask, gain, (const float*)sink, (const bf16_t*)pk_plane, (const bf16_t*)pv_plane,
+                      (const int*)pool_table, pool_table_ld, pool_table_width, pool, back, (const bf16_t*)gate, gate_ld, LP_LEAST};
+    int below = INT_MAX;
+    if (tile_req && (long)tiles * LAM_TOKENS >= tokens && local_prompt_pays(a, tokens) && local_prompt_fits(a, dim, vdim, pages, pool_pages)) {
+        const int rc = dim == 192 ? launch_local_prompt<192, 128, 32, 3>(a, tokens, stream)
+                       : dim == 128 ? launch_local_prompt<128, 128, 64, 2>(a, tokens, stream) : launch_local_prompt<64, 64, 64, 2>(a, tokens, stream);
+        if (rc != TL_OK) return rc;
+        if (requests == 1) return TL_OK;
+        below = LP_LEAST;
+    }
 #define TL_LAM(DK, DV)                                                                                                                      \
     launch_local_mfma<DK, DV>(q, q_ld, out, out_ld, k_plane, v_plane, block_table, table_ld, table_width, req_indptr, ctx_lens, tile_req,  \
                               tile_tok0, tiles, heads, kv_heads, page_size, scale, cap, mask, gain, sink, pk_plane, pv_plane, pool_table,        \
-                              pool_table_ld, pool_table_width, pool, back, gate, gate_ld, stream)
+                              pool_table_ld, pool_table_width, pool, back, gate, gate_ld, below, stream)
 #define TL_LAM_V(DK)                                     \
     switch (vdim) {                                      \
         case 16: TL_LAM(DK, 1); break;                   \

@@ -1342,7 +1342,8 @@ def local_attention(q: torch.Tensor, out: torch.Tensor, k_plane: torch.Tensor, v
                                                  _ptr(req_indptr), _ptr(ctx_lens), _ptr(tile_req), _ptr(tile_tok0), c_int(n_tiles), c_int(heads),
                                                  c_int(kv_heads), c_int(dim), c_int(vdim), c_int(page_size), c_float(scale), c_float(softcap),
                                                  c_int(chunk), c_int(window), c_float(gain), *pool_args, c_int(pool_table.shape[1] if pool else 0),
-                                                 c_int(pool), c_int(keep_first), *turn_args, *gate_args, _stream()))
+                                                 c_int(pool), c_int(keep_first), *turn_args, *gate_args, c_int(T), c_int(R),
+                                                 c_int(pk_plane.shape[0] if pool else 0), _stream()))
         return
     _i32(token_req, "token_req", T)
     _i32(positions, "positions", T)
