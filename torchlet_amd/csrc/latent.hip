@@ -155,6 +155,43 @@ extern "C" int tl_rotate_pairs(const void* src, int src_ld, int src_head, int sr
     return TL_OK;
 }
 
+// ------------------------------------------------------------------ cached rows side by side
+// Row i of `latents` [rows, rank] and `rotated` [rows, rot]: portion_at[p] <= i < portion_at[p + 1] is portion p's row of the position
+// portion_low[p] + i - portion_at[p] of request portion_req[p]; zeros for positions that the portion does not read (before its window, from
+// the request's end on).  A wave copies a row in 16-byte pieces.
+__global__ void __launch_bounds__(256)
+latent_rows_kernel(const uint4* __restrict__ plane, int page_size, const int* __restrict__ block_table, int bt_stride, const int* __restrict__ req_indptr,
+                   const int* __restrict__ ctx_lens, const int* __restrict__ portion_req, const int* __restrict__ portion_at,
+                   const int* __restrict__ portion_low, int portions, int window, int rank8, int rot8, uint4* __restrict__ latents, uint4* __restrict__ rotated,
+                   int rows) {
+    const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (row >= rows) return;
+    int p = 0;
+    while (p + 1 < portions && portion_at[p + 1] <= row) ++p;
+    const int req = portion_req[p], ctx = ctx_lens[req], pos = portion_low[p] + row - portion_at[p];
+    const int first = window > 0 ? max(0, ctx - window + 1) : 0, end = ctx + req_indptr[req + 1] - req_indptr[req];
+    const bool read = pos >= first && pos < end;
+    const int page = read ? block_table[(size_t)req * bt_stride + pos / page_size] : 0;
+    const uint4* src = plane + ((size_t)page * page_size + pos % page_size) * (rank8 + rot8);
+    for (int i = lane; i < rank8 + rot8; i += TL_WAVE) {
+        const uint4 x = read ? src[i] : make_uint4(0, 0, 0, 0);
+        if (i < rank8) latents[(size_t)row * rank8 + i] = x; else rotated[(size_t)row * rot8 + i - rank8] = x;
+    }
+}
+
+extern "C" int tl_latent_rows(const void* plane, int page_size, const void* block_table, int bt_stride, const void* req_indptr, const void* ctx_lens,
+                              const void* portion_req, const void* portion_at, const void* portion_low, int portions, int window, int rank, int rot,
+                              void* latents, void* rotated, int rows, hipStream_t stream) {
+    TL_REQUIRE(page_size > 0 && portions >= 0 && window >= 0 && rows >= 0 && rank > 0 && rank % 8 == 0 && rot >= 0 && rot % 8 == 0, "latent_rows: bad sizes");
+    TL_REQUIRE((((uintptr_t)plane | (uintptr_t)latents | (uintptr_t)rotated) & 15) == 0 && (rot == 0 || rotated), "latent_rows: rows not aligned");
+    if (rows == 0 || portions == 0) return TL_OK;
+    latent_rows_kernel<<<(rows + 3) / 4, 256, 0, stream>>>((const uint4*)plane, page_size, (const int*)block_table, bt_stride, (const int*)req_indptr,
+        (const int*)ctx_lens, (const int*)portion_req, (const int*)portion_at, (const int*)portion_low, portions, window, rank / 8, rot / 8, (uint4*)latents,
+        (uint4*)rotated, rows);
+    TL_CHECK_LAUNCH("latent_rows");
+    return TL_OK;
+}
+
 // ------------------------------------------------------------------ attention
 // A tile is up to `tile_tokens` consecutive new tokens of one request times a chunk of up to 16 heads: one wave per
 // row (token, head).  The keys pass through shared memory KT at a time, shared by all rows of the tile; a lane takes the

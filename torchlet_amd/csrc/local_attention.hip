@@ -503,11 +503,20 @@ struct LocalArgs {
     OutputTurn back;
     const bf16_t* gate;
     int gate_ld, least;
+    // keys and values in rows side by side instead of pages (LINEAR): the i-th of `requests` portions is request portion_req[i]'s, whose key at
+    // position p is row portion_at[i] + p - portion_low[i] (both multiples of 64); rows hold keys of all heads, k_ld numbers apart, then, from
+    // shared_at bytes after k_plane, shared_ld numbers apart, the last dimensions of every head's key; values lie transposed, v_ld keys to a row
+    const int *portion_req, *portion_at, *portion_low;
+    int k_ld, shared_ld, v_ld;
+    unsigned shared_at;
+    const bf16_t* value_gate;            // every output number times the sigmoid of its own
+    int value_gate_ld;
 };
 
-template <int DIM, int VDIM, int KEYS, int STAGES, bool CAP>
+template <int DIM, int VDIM, int KEYS, int STAGES, bool CAP, bool LINEAR>
 __global__ void __launch_bounds__(256, 2)
 local_prompt_kernel(LocalArgs a) {
+    constexpr int OWN = LINEAR && DIM > VDIM ? VDIM / 8 : DIM / 8;    // (LINEAR) pieces of a key row that are the head's own
     constexpr int KB = KEYS / 32, NC = DIM / 16, NB = VDIM / 32;      // blocks of keys; pieces of a score's sum; blocks of output columns
     constexpr int KPP = DIM / 8, VPP = KEYS / 8;                      // 16-byte pieces of a key row, of a row of transposed values
     constexpr int KBYTES = KEYS * DIM * 2, STAGE = KBYTES + VDIM * KEYS * 2;
@@ -523,9 +532,13 @@ local_prompt_kernel(LocalArgs a) {
     // ---- which tile: the requests' tiles are counted by a prefix sum over the lanes; the last tile first, each with all its heads
     const int group = a.heads / a.kv_heads, chunks_h = (group + a.gcap - 1) / a.gcap, per_tile = a.kv_heads * chunks_h, tq = LP_ROWS / a.gcap;
     int total = 0;
+    auto new_tokens = [&](int i) {
+        if (i >= a.requests) return 0;
+        const int r = LINEAR ? a.portion_req[i] : i;
+        return a.req_indptr[r + 1] - a.req_indptr[r];
+    };
     for (int base = 0; base < a.requests; base += TL_WAVE) {
-        const int r = base + lane;
-        const int n = r < a.requests ? a.req_indptr[r + 1] - a.req_indptr[r] : 0;
+        const int n = new_tokens(base + lane);
         int mine = n >= a.least ? (n + tq - 1) / tq : 0;
 #pragma unroll
         for (int o = TL_WAVE / 2; o > 0; o >>= 1) mine += __shfl_xor(mine, o, TL_WAVE);
@@ -533,12 +546,11 @@ local_prompt_kernel(LocalArgs a) {
     }
     if ((int)blockIdx.x >= total * per_tile) return;
     const int want = total - 1 - (int)blockIdx.x / per_tile, by = blockIdx.x % per_tile;
-    int req = 0, tok0 = 0;
+    int portion = 0, tok0 = 0;
     {
         int first = 0;
         for (int base = 0; base < a.requests; base += TL_WAVE) {
-            const int r = base + lane;
-            const int n = r < a.requests ? a.req_indptr[r + 1] - a.req_indptr[r] : 0;
+            const int n = new_tokens(base + lane);
             const int mine = n >= a.least ? (n + tq - 1) / tq : 0;
             int upto = mine;
 #pragma unroll
@@ -549,7 +561,7 @@ local_prompt_kernel(LocalArgs a) {
             const unsigned long long past = __ballot(first + upto > want);
             if (past) {
                 const int l = __builtin_amdgcn_readfirstlane(__ffsll(past) - 1);
-                req = base + l;
+                portion = base + l;
                 tok0 = (want - first - __builtin_amdgcn_readlane(upto, l) + __builtin_amdgcn_readlane(mine, l)) * tq;
                 break;
             }
@@ -557,6 +569,7 @@ local_prompt_kernel(LocalArgs a) {
         }
     }
     const int g = by / chunks_h, g0 = by % chunks_h * a.gcap, gcount = min(a.gcap, group - g0);
+    const int req = LINEAR ? __builtin_amdgcn_readfirstlane(a.portion_req[portion]) : portion;
     const int first = a.req_indptr[req], n_new = a.req_indptr[req + 1] - first, ctx = a.ctx_lens[req];
     const int ntok = min(tq, n_new - tok0), p0 = ctx + tok0, p_last = p0 + ntok - 1;
 
@@ -582,20 +595,25 @@ local_prompt_kernel(LocalArgs a) {
 
     // what of a piece's address does not change from step to step: its key within the step, and bytes from the start of its page
     const int shift = a.page_shift, pmask = a.page_size - 1;
-    unsigned k_off[KI], v_off[VI];
+    unsigned k_off[KI], v_off[VI], k_step[LINEAR ? KI : 1];      // (LINEAR: bytes from one step's key to the next one's)
     int k_x[KI];
     int v_x;                                 // (the same in every value load of a lane: a piece's slot depends on the row's low bits alone)
 #pragma unroll
     for (int j = 0; j < KI; ++j) {
         const int piece = (wave + 4 * j) * 64 + lane, kx = piece / KPP;
         k_x[j] = kx;
-        k_off[j] = (unsigned)((g * a.page_size + (kx & pmask)) * DIM + key_slot(piece % KPP, kx) * 8) * 2u;
+        const int slot = key_slot(piece % KPP, kx);
+        if (LINEAR) {
+            const bool own = slot < OWN;
+            k_step[j] = (unsigned)(KEYS * (own ? a.k_ld : a.shared_ld)) * 2u;
+            k_off[j] = own ? (unsigned)(kx * a.k_ld + g * (OWN * 8) + slot * 8) * 2u : a.shared_at + (unsigned)(kx * a.shared_ld + (slot - OWN) * 8) * 2u;
+        } else k_off[j] = (unsigned)((g * a.page_size + (kx & pmask)) * DIM + slot * 8) * 2u;
     }
 #pragma unroll
     for (int j = 0; j < VI; ++j) {
         const int piece = (wave + 4 * j) * 64 + lane, d = piece / VPP, x = 8 * value_slot(piece % VPP, d);
         if (j == 0) v_x = x;
-        v_off[j] = (unsigned)((g * VDIM + d) * a.page_size + (x & pmask)) * 2u;
+        v_off[j] = LINEAR ? ((unsigned)(g * VDIM + d) * (unsigned)a.v_ld + (unsigned)x) * 2u : (unsigned)((g * VDIM + d) * a.page_size + (x & pmask)) * 2u;
     }
     const unsigned kpage = (unsigned)(a.kv_heads * a.page_size * DIM) * 2u, vpage = (unsigned)(a.kv_heads * a.page_size * VDIM) * 2u;
     const int krow = 16 * (lr >> 4) + 8 * ((lr >> 2) & 1) + 4 * ((lr >> 3) & 1) + (lr & 3);      // key that row lr of the first product carries
@@ -609,9 +627,9 @@ local_prompt_kernel(LocalArgs a) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[b][v] = 0.f;
 
-    for (int phase = 0; phase < 3; ++phase) {
+    for (int phase = LINEAR ? 2 : 0; phase < 3; ++phase) {
         const bf16_t *kp = a.k_plane, *vp = a.v_plane;
-        const int* tbl = a.block_table + (size_t)req * a.table_ld;
+        const int* tbl = LINEAR ? nullptr : a.block_table + (size_t)req * a.table_ld;
         int width = a.table_width, key_lo = 0, key_hi = 0;            // the tile reads keys key_lo .. key_hi - 1, ...
         int r_lo = 0, r_hi = -1, w_lo_max = 0, w_lo_min = 0, w_hi_min = -1, w_hi_max = -1;      // ... a row r_lo .. r_hi, and over the wave's rows
         if (phase == 0) {
@@ -636,19 +654,27 @@ local_prompt_kernel(LocalArgs a) {
         }
         if (key_hi <= key_lo) continue;
         const int st_first = key_lo / KEYS, st_last = (key_hi + KEYS - 1) / KEYS;
+        const int row0 = LINEAR ? a.portion_at[portion] - a.portion_low[portion] : 0;
         const int blk0 = (st_first * KEYS) >> shift, blk_n = ((key_hi - 1) >> shift) - blk0 + 1, blk_last = blk_n - 1;
-        if (blk_n > LP_BT_MAX || blk0 + blk_n > width) continue;      // (the host has seen to it that this cannot be)
+        if (!LINEAR && (blk_n > LP_BT_MAX || blk0 + blk_n > width)) continue;      // (the host has seen to it that this cannot be)
         __syncthreads();                                              // the stretch before has been worked on
-        for (int i = threadIdx.x; i < blk_n; i += 256) bt[i] = tbl[max(blk0 + i, key_lo >> shift)];      // (pages before the first key may be gone)
+        if (!LINEAR) for (int i = threadIdx.x; i < blk_n; i += 256) bt[i] = tbl[max(blk0 + i, key_lo >> shift)];      // (pages before the first key may be gone)
         __syncthreads();
         int pg_k[KI], pg_v;
         auto look_up_one = [&](int st, int j) {
+            if (LINEAR) return;
             const int first_key = st * KEYS - (blk0 << shift);
             if (j < KI) pg_k[j] = bt[min((first_key + k_x[j]) >> shift, blk_last)];
             else pg_v = bt[min((first_key + v_x) >> shift, blk_last)];
         };
         auto request_one = [&](int st, int buf, int j) {              // (after the step's look-ups)
             const unsigned sb = lds_base + buf * STAGE;
+            if (LINEAR) {
+                const unsigned at = (unsigned)(row0 + st * KEYS);
+                if (j < KI) lp_load_to_lds(kp, at / KEYS * k_step[j] + k_off[j], sb + (wave + 4 * j) * 1024);
+                else lp_load_to_lds(vp + at, v_off[j - KI], sb + KBYTES + (wave + 4 * (j - KI)) * 1024);
+                return;
+            }
             const unsigned uin = KEYS < a.page_size ? (unsigned)((st * KEYS) & pmask) : 0u;      // the step's first key's place in a longer page
             if (j < KI) lp_load_to_lds(kp + (size_t)uin * DIM, (unsigned)pg_k[j] * kpage + k_off[j], sb + (wave + 4 * j) * 1024);
             else lp_load_to_lds(vp + uin, (unsigned)pg_v * vpage + v_off[j - KI], sb + KBYTES + (wave + 4 * (j - KI)) * 1024);
@@ -672,7 +698,7 @@ local_prompt_kernel(LocalArgs a) {
             const int buf = (st - st_first) % STAGES, buf_req = (st - st_first + STAGES - 1) % STAGES;
             const int st_req = min(st + STAGES - 1, st_last - 1), st_look = min(st + STAGES, st_last - 1), kbase = st * KEYS;
             unsigned char *kb_s = lp_smem + buf * STAGE, *vb_s = kb_s + KBYTES;
-            if (kbase + KEYS > key_hi || kbase < key_lo) {
+            if (!LINEAR && (kbase + KEYS > key_hi || kbase < key_lo)) {      // (LINEAR: such rows are zeros)
                 // keys beyond the stretch's last may not be written yet, and the pages of those before its first may be gone: whatever lies there
                 // must not reach the second product (0 * Inf), so their values count as zero
                 for (int i = threadIdx.x; i < VDIM * VPP; i += 256) {
@@ -824,7 +850,13 @@ local_prompt_kernel(LocalArgs a) {
             float y[4];
 #pragma unroll
             for (int v = 0; v < 4; ++v) y[v] = acc[b][4 * q + v] * norm;
-            if (a.back.freq) {                           // (pairs of neighbours: the host has seen to it)
+            if (LINEAR && a.value_gate) {
+                union { uint2 u; bf16_t e[4]; } vg;
+                vg.u = *(const uint2*)(a.value_gate + (size_t)r_token * a.value_gate_ld + r_head * VDIM + col);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) y[v] *= sigmoid(to_float(vg.e[v]));
+            }
+            if (!LINEAR && a.back.freq) {                // (pairs of neighbours: the host has seen to it)
                 a.back.turn(col / 2, r_pos, y[0], y[1]);
                 a.back.turn(col / 2 + 1, r_pos, y[2], y[3]);
             }
@@ -835,16 +867,14 @@ local_prompt_kernel(LocalArgs a) {
         }
 }
 
-template <int DIM, int VDIM, int KEYS, int STAGES>
-static int launch_local_prompt(const LocalArgs& a, long tokens, hipStream_t stream) {
-    constexpr size_t smem = (size_t)STAGES * (KEYS * DIM * 2 + VDIM * KEYS * 2) + LP_BT_MAX * 4;
-    auto kernel = a.cap > 0.f ? local_prompt_kernel<DIM, VDIM, KEYS, STAGES, true> : local_prompt_kernel<DIM, VDIM, KEYS, STAGES, false>;
-    static const hipError_t allowed[2] = {
-        hipFuncSetAttribute((const void*)local_prompt_kernel<DIM, VDIM, KEYS, STAGES, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem),
-        hipFuncSetAttribute((const void*)local_prompt_kernel<DIM, VDIM, KEYS, STAGES, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem)};
-    if (allowed[0] != hipSuccess || allowed[1] != hipSuccess) { tl_set_error("local_prompt: cannot get %zu bytes of shared memory", smem); return TL_ERR_HIP; }
-    const int group = a.heads / a.kv_heads, tq = LP_ROWS / a.gcap;
-    const long tiles = tokens / tq + (a.requests < tokens / a.least ? a.requests : tokens / a.least);
+// `tiles`: at most so many of LP_ROWS / gcap tokens (those beyond the last leave at once).
+template <int DIM, int VDIM, int KEYS, int STAGES, bool CAP, bool LINEAR>
+static int launch_local_prompt(const LocalArgs& a, long tiles, hipStream_t stream) {
+    constexpr size_t smem = (size_t)STAGES * (KEYS * DIM * 2 + VDIM * KEYS * 2) + (LINEAR ? 0 : LP_BT_MAX * 4);
+    auto kernel = local_prompt_kernel<DIM, VDIM, KEYS, STAGES, CAP, LINEAR>;
+    static const hipError_t allowed = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    if (allowed != hipSuccess) { tl_set_error("local_prompt: cannot get %zu bytes of shared memory", smem); return TL_ERR_HIP; }
+    const int group = a.heads / a.kv_heads;
     if (tiles > 0) kernel<<<dim3((unsigned)(tiles * a.kv_heads * ((group + a.gcap - 1) / a.gcap))), 256, smem, stream>>>(a);
     TL_CHECK_LAUNCH("local_prompt");
     return TL_OK;
@@ -895,11 +925,16 @@ extern "C" int tl_local_attention_tiles(const void* q, int q_ld, void* out, int 
     const LocalArgs a{(const bf16_t*)q, q_ld, (bf16_t*)out, out_ld, (const bf16_t*)k_plane, (const bf16_t*)v_plane, (const int*)block_table, table_ld,
                       table_width, (const int*)req_indptr, (const int*)ctx_lens, requests, heads, kv_heads, (group + cut - 1) / cut, page_size,
                       __builtin_ctz(page_size), scale, cap, mask, gain, (const float*)sink, (const bf16_t*)pk_plane, (const bf16_t*)pv_plane,
-                      (const int*)pool_table, pool_table_ld, pool_table_width, pool, back, (const bf16_t*)gate, gate_ld, LP_LEAST};
+                      (const int*)pool_table, pool_table_ld, pool_table_width, pool, back, (const bf16_t*)gate, gate_ld, LP_LEAST, nullptr, nullptr, nullptr, 0, 0, 0, 0u, nullptr, 0};
     int below = INT_MAX;
     if (tile_req && (long)tiles * LAM_TOKENS >= tokens && local_prompt_pays(a, tokens) && local_prompt_fits(a, dim, vdim, pages, pool_pages)) {
-        const int rc = dim == 192 ? launch_local_prompt<192, 128, 32, 3>(a, tokens, stream)
-                       : dim == 128 ? launch_local_prompt<128, 128, 64, 2>(a, tokens, stream) : launch_local_prompt<64, 64, 64, 2>(a, tokens, stream);
+        const long most = tokens / LP_LEAST, tiles_most = tokens / (LP_ROWS / a.gcap) + (requests < most ? requests : most);
+        int rc;
+#define TL_LP(DIM, VDIM, KEYS, STAGES)                                                                        \
+    rc = cap > 0.f ? launch_local_prompt<DIM, VDIM, KEYS, STAGES, true, false>(a, tiles_most, stream)         \
+                   : launch_local_prompt<DIM, VDIM, KEYS, STAGES, false, false>(a, tiles_most, stream)
+        if (dim == 192) TL_LP(192, 128, 32, 3); else if (dim == 128) TL_LP(128, 128, 64, 2); else TL_LP(64, 64, 64, 2);
+#undef TL_LP
         if (rc != TL_OK) return rc;
         if (requests == 1) return TL_OK;
         below = LP_LEAST;
@@ -934,6 +969,35 @@ extern "C" int tl_local_attention_tiles(const void* q, int q_ld, void* out, int 
 #undef TL_LAM
     TL_CHECK_LAUNCH("local_attention_mfma");
     return TL_OK;
+}
+
+// ------------------------------------------------------------------ portions of prompts over rows of keys and values
+// The kernel of 128 rows over keys and values that lie side by side for the step (LocalArgs: LINEAR), every head with keys and values of its own.  dim =
+// own + shared numbers a key, own == vdim where a part is shared.  portion_* int32 [portions]; rows: of keys, a multiple of 64, zeros where no key is.
+extern "C" int tl_prompt_rows_fits(int own, int shared, int vdim) {
+    return (own == 128 && vdim == 128 && (shared == 0 || shared == 64)) || (own == 64 && vdim == 64 && shared == 0);
+}
+
+extern "C" int tl_prompt_rows(const void* q, int q_ld, void* out, int out_ld, const void* keys, int k_ld, long shared_at, int shared_ld, const void* values,
+                              long rows, const void* portion_req, const void* portion_at, const void* portion_low, int portions, const void* req_indptr,
+                              const void* ctx_lens, int tiles, int heads, int own, int shared, int vdim, float scale, int window, const void* sink,
+                              const void* gate, int gate_ld, const void* value_gate, int value_gate_ld, hipStream_t stream) {
+    TL_REQUIRE(tl_prompt_rows_fits(own, shared, vdim) && heads > 0 && scale > 0.f && window >= 0 && tiles >= 0 && portions >= 0, "prompt_rows: not built for these sizes");
+    TL_REQUIRE(q_ld >= heads * (own + shared) && q_ld % 8 == 0 && ((uintptr_t)q & 15) == 0 && out_ld >= heads * vdim && out_ld % 4 == 0 && ((uintptr_t)out & 7) == 0,
+               "prompt_rows: queries or output too short or not aligned");
+    TL_REQUIRE(rows % 64 == 0 && k_ld >= heads * own && k_ld % 8 == 0 && ((uintptr_t)keys & 15) == 0 && ((uintptr_t)values & 15) == 0 &&
+                   (shared == 0 || (shared_ld >= shared && shared_ld % 8 == 0 && shared_at % 16 == 0 && shared_at >= rows * k_ld * 2)),
+               "prompt_rows: keys or values not aligned");
+    TL_REQUIRE((shared ? shared_at + rows * shared_ld * 2 : rows * k_ld * 2) < (1L << 32) && rows * heads * vdim * 2 < (1L << 32), "prompt_rows: more keys than 32 bits count");
+    TL_REQUIRE((!gate || gate_ld >= heads) && (!value_gate || (value_gate_ld >= heads * vdim && value_gate_ld % 4 == 0 && ((uintptr_t)value_gate & 7) == 0)),
+               "prompt_rows: a gate that does not fit");
+    if (tiles == 0 || portions == 0) return TL_OK;
+    const LocalArgs a{(const bf16_t*)q, q_ld, (bf16_t*)out, out_ld, (const bf16_t*)keys, (const bf16_t*)values, nullptr, 0, 0, (const int*)req_indptr,
+                      (const int*)ctx_lens, portions, heads, heads, 1, 64, 6, scale, 0.f, LocalMask{0, window, 0}, 1.f, (const float*)sink, nullptr, nullptr,
+                      nullptr, 0, 0, 0, OutputTurn{nullptr, 0, 0}, (const bf16_t*)gate, gate_ld, 1, (const int*)portion_req, (const int*)portion_at,
+                      (const int*)portion_low, k_ld, shared_ld, (int)rows, (unsigned)shared_at, (const bf16_t*)value_gate, value_gate_ld};
+    if (shared) return launch_local_prompt<192, 128, 32, 3, false, true>(a, tiles, stream);
+    return own == 128 ? launch_local_prompt<128, 128, 64, 2, false, true>(a, tiles, stream) : launch_local_prompt<64, 64, 64, 2, false, true>(a, tiles, stream);
 }
 
 extern "C" int tl_local_attention(const void* q, int q_ld, void* out, int out_ld, const void* k_plane, const void* v_plane, int pages,

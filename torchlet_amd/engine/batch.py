@@ -141,6 +141,28 @@ class StepContext:
                                     (v["lr"], v["l0"], len(lr), v["lt"], len(long_tokens), shortest))
         return t
 
+    def long_portions(self, least: int, window: int = 0, tile: int = 128):
+        """The requests that bring ``least`` tokens or more, and where the rows of the positions that each reads lie side by side (from the first one inside
+        the ``window`` on, 0: all; starts and counts rounded to multiples of 64): ``(portion_req [n], portion_at [n + 1], portion_low [n], n, rows,
+        tiles of `tile` new tokens, others, pairs, tokens)``, the first three int32 on the device; ``None`` without such requests.  ``others``: the ``req_indptr`` of a step that
+        held the other requests' tokens alone (int32 ``[R + 1]`` on the device), ``None`` if there are none; ``pairs``: the portions' tokens times the rows they read; ``tokens``: theirs."""
+        key = ("portions", least, window, tile)
+        if key not in self._tiles:
+            req = np.nonzero(self._host_new_lens >= least)[0].astype(np.int32)
+            if not len(req):
+                self._tiles[key] = None
+            else:
+                new, ctx = self._host_new_lens[req].astype(np.int64), self._host_ctx_lens[req].astype(np.int64)
+                low = np.maximum(0, ctx - window + 1) // 64 * 64 if window else np.zeros_like(ctx)
+                at = np.zeros(len(req) + 1, dtype=np.int64)
+                np.cumsum(-(-(ctx + new - low) // 64) * 64, out=at[1:])
+                others = np.zeros(self.num_requests + 1, dtype=np.int32)
+                np.cumsum(np.where(self._host_new_lens < least, self._host_new_lens, 0), out=others[1:])
+                v = self._upload({"r": req, "a": at.astype(np.int32), "l": low.astype(np.int32), "o": others})
+                self._tiles[key] = (v["r"], v["a"], v["l"], len(req), int(at[-1]), int((-(-new // tile)).sum()), v["o"] if others[-1] else None,
+                                    int((new * np.diff(at)).sum()), int(new.sum()))
+        return self._tiles[key]
+
 
 class StaticDecodeContext:
     """A step context of fixed shape for decode-only steps: ``width`` requests with one new

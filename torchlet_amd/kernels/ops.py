@@ -1574,6 +1574,58 @@ def latent_attention(q: torch.Tensor, out: torch.Tensor, plane: torch.Tensor, bl
                                         c_int(window), _ptr(gate), c_int(gate.stride(0) if gate is not None else 0), _stream()))
 
 
+PROMPT_ROWS_SCRATCH_BYTES = 512 << 20     # keys and values of a group of heads that a step may hold beside the cache
+
+
+def prompt_rows_fits(dtype: torch.dtype, own: int, shared: int, vdim: int) -> bool:
+    """Whether :func:`prompt_rows_attention` is built for keys of ``own`` numbers a head and ``shared`` ones for all heads, and values of ``vdim``."""
+    return dtype == torch.bfloat16 and bool(_lib("local_attention").tl_prompt_rows_fits(c_int(own), c_int(shared), c_int(vdim)))
+
+
+def latent_rows(plane: torch.Tensor, block_table: torch.Tensor, req_indptr: torch.Tensor, ctx_lens: torch.Tensor, portions, rank: int, rot: int,
+                latents: torch.Tensor, rotated: torch.Tensor | None, window: int = 0) -> None:
+    """The cached rows that the step's long portions read, side by side: ``latents [rows, rank]`` and ``rotated [rows, rot]`` (bfloat16, contiguous);
+    ``portions = (portion_req, portion_at, portion_low, portions, rows, tiles, ..)`` as a step context makes them; rows that are no key are zeros."""
+    req, at, low, count, rows = portions[:5]
+    if plane.dtype != torch.bfloat16 or plane.dim() != 4 or plane.shape[1] != 1 or plane.shape[3] != rank + rot or not plane.is_contiguous() \
+            or latents.shape != (rows, rank) or latents.dtype != plane.dtype or not latents.is_contiguous() \
+            or (rot > 0 and (rotated is None or rotated.shape != (rows, rot) or rotated.dtype != plane.dtype or not rotated.is_contiguous())):
+        raise KernelError("latent_rows: shapes or dtypes do not fit")
+    for name, t, n in (("portion_req", req, count), ("portion_at", at, count + 1), ("portion_low", low, count)):
+        _i32(t, name, n)
+    lib = _lib("latent")
+    _check(lib, lib.tl_latent_rows(_ptr(plane), c_int(plane.shape[2]), _ptr(block_table), c_int(block_table.stride(0)), _ptr(req_indptr), _ptr(ctx_lens), _ptr(req),
+                                   _ptr(at), _ptr(low), c_int(count), c_int(window), c_int(rank), c_int(rot), _ptr(latents), _ptr(rotated), c_int(rows), _stream()))
+
+
+def prompt_rows_attention(q: torch.Tensor, out: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, rows: int, req_indptr: torch.Tensor,
+                          ctx_lens: torch.Tensor, portions, heads: int, own: int, shared: int, vdim: int, scale: float, sink: torch.Tensor | None = None,
+                          window: int = 0, gate: torch.Tensor | None = None, value_gate: torch.Tensor | None = None) -> None:
+    """Causal attention of the step's long portions (:func:`latent_rows`) over keys and values of their own for every head: ``q [T, heads * (own + shared)]`` and
+    ``out [T, heads * vdim]`` (rows may be strided; other requests' rows are left alone); ``keys`` holds, flat, ``[rows, heads, own]`` and, behind them,
+    ``[rows, shared]`` for all heads; ``values [heads * vdim, rows]``.  ``sink``, ``window`` and ``gate`` as in :func:`latent_attention`; ``value_gate [T, heads
+    * vdim]``: every output number is multiplied by the sigmoid of its own.  bfloat16, where :func:`prompt_rows_fits`."""
+    req, at, low, count, total, tiles = portions[:6]
+    T = q.shape[0]
+    if total != rows or keys.numel() != rows * (heads * own + shared) or not keys.is_contiguous() or values.shape != (heads * vdim, rows) or not values.is_contiguous() \
+            or q.shape[1] != heads * (own + shared) or out.shape != (T, heads * vdim) or q.stride(1) != 1 or out.stride(1) != 1 \
+            or any(t.dtype != torch.bfloat16 for t in (q, out, keys, values)):
+        raise KernelError("prompt_rows_attention: shapes or dtypes do not fit")
+    if sink is not None and (sink.dtype != torch.float32 or sink.numel() != heads or not sink.is_contiguous()):
+        raise KernelError("prompt_rows_attention: sink must be float32 [heads]")
+    for t, n in ((gate, heads), (value_gate, heads * vdim)):
+        if t is not None and (t.dtype != q.dtype or t.shape != (T, n) or t.stride(1) != 1):
+            raise KernelError("prompt_rows_attention: a gate that does not fit")
+    for name, t, n in (("portion_req", req, count), ("portion_at", at, count + 1), ("portion_low", low, count)):
+        _i32(t, name, n)
+    lib = _lib("local_attention")
+    _check(lib, lib.tl_prompt_rows(_ptr(q), c_int(q.stride(0)), _ptr(out), c_int(out.stride(0)), _ptr(keys), c_int(heads * own), ctypes.c_long(rows * heads * own * 2),
+                                   c_int(shared), _ptr(values), ctypes.c_long(rows), _ptr(req), _ptr(at), _ptr(low), c_int(count), _ptr(req_indptr), _ptr(ctx_lens),
+                                   c_int(tiles), c_int(heads), c_int(own), c_int(shared), c_int(vdim), c_float(scale), c_int(window), _ptr(sink), _ptr(gate),
+                                   c_int(gate.stride(0) if gate is not None else 0), _ptr(value_gate),
+                                   c_int(value_gate.stride(0) if value_gate is not None else 0), _stream()))
+
+
 # ------------------------------------------------------------- products over groups, routing
 
 # ``*_pairs``: the product's columns come in pairs (gate, up) and the output, half as wide, is ``act(gate) * up``

@@ -16,8 +16,13 @@ latent the kernel that writes the cache row turns the queries' rotated parts as 
 Only ``c`` and the rotated key part are cached: one page plane whose rows hold ``kv_rank + rot_dim`` numbers.  The key
 up-projection is taken to the query's side, ``q_t . (W_uk c_s) = (W_uk^T q_t) . c_s``, so a head's query becomes a vector
 of the cache row's shape and all heads read the same rows: the attention kernel is one dot product per key and its
-weighted sum runs over the latents; the value up-projection ``W_uv`` is applied to that sum.  Prompts and decode steps
-take the same path, so how a request is cut cannot change what it computes beyond the order of the sums.
+weighted sum runs over the latents; the value up-projection ``W_uv`` is applied to that sum.
+
+Long portions of prompts (bfloat16, the head sizes the kernel is built for) go the other way: the cached rows that they read are brought side by side, keys
+and values are projected up for all heads, and an ordinary attention runs over them.  A score then costs ``dim + rot_dim`` products instead of ``kv_rank +
+rot_dim``, and a value ``vdim`` instead of ``kv_rank``; the projection costs ``kv_rank * (dim + vdim)`` for every key once, which a portion of _PROMPT_LEAST tokens or
+more earns back where there is work enough.  The two ways differ in what is rounded between the products (the projected query and the mixed latent, or keys and values), not in what is
+held in 32-bit: scores, softmax and sums.
 """
 from __future__ import annotations
 
@@ -28,6 +33,12 @@ from ..kernels import ops
 from .base import KEEP_COMPUTE, KEEP_FLOAT32, KEEP_STORED, MIXERS, POSITION_ENCODINGS, Mixer, PagedNeed, WeightSpec
 
 _MIN_KEYS_PER_SPLIT = 64        # two steps of the matrix-core kernel
+_PROMPT_LEAST = 64              # tokens of a portion from which its keys and values may be projected up
+# ... and the least work for which they are: (token, key) pairs times heads, a token itself counting like so many keys (its way through the two absorbed
+# projections).  Measured with 32 / 16 / 8 heads, us of the whole mixer, absorbed against projected: 256 tokens after none 135 / 134, 92 / 105, 88 / 118; 512
+# after none 221 / 131, 141 / 105, 112 / 116; 64 after 4000 193 / 193, 124 / 135; 128 after 4000 297 / 211, 177 / 138; 8 x 128 after none 215 / 132, 123 / 108, 117 / 117.
+# Beside 31 decoded tokens, which then take kernels of their own, 256 after 2000 516 / 301, 282 / 205, 130 / 198.
+_TOKEN_AS_KEYS, _UP_LEAST, _UP_LEAST_BESIDE = 256, 5 << 20, 8 << 20
 
 
 @MIXERS.register("latent_attention")
@@ -62,19 +73,22 @@ class LatentAttention(Mixer):
         self.tile_tokens = ops.latent_tile_tokens(self.heads, ops.LATENT_MFMA_ROWS if on_matrix_cores else ops.LATENT_ATTENTION_ROWS)
         self.general_tile_tokens = ops.latent_tile_tokens(self.heads, ops.LATENT_ATTENTION_ROWS)
         self.compute_units = ops.compute_units()
-        self.w_down = self.w_dq_norm = self.w_dkv_norm = self.w_uq = self.w_uk_t = self.w_uv = self.sink = self.w_o = None
+        self.w_down = self.w_dq_norm = self.w_dkv_norm = self.w_uq = self.w_uk = self.w_uk_t = self.w_uv = self.sink = self.w_o = None
         # the columns of the fused first projection: [query latent, or the queries themselves | latent | rotated key part | gate], filled up with
         # zero rows of the matrix so that a token's row stays aligned
         self.q_cols = self.q_rank if self.q_rank else self.heads * (self.dim + self.rot)
         self.gate_at = self.q_cols + self.row
         self.gate_cols = self.heads if spec.gate else self.heads * self.vdim if spec.gate_values else 0
         self.down_cols = -(-(self.gate_at + self.gate_cols) // 8) * 8
+        # long portions' keys and values are projected up where that attention is built for the sizes
+        self.project_up = on_matrix_cores and self.rank % 64 == 0 and self.rot % 8 == 0 and self.scale > 0 and (not spec.gate_values or self.gate_at % 4 == 0) \
+            and ops.prompt_rows_fits(dtype, self.dim, self.rot, self.vdim)
 
     def paged_need(self):
         return PagedNeed(num_heads=1, head_dim=self.row, planes=((1, self.row),), window=self.spec.window)
 
     def kernel_libraries(self):
-        return ["latent", "experts"]
+        return ["latent", "experts", "local_attention"]
 
     def parts(self):
         yield self
@@ -112,6 +126,8 @@ class LatentAttention(Mixer):
             self.w_uq = self._place(tensors["uq"], KEEP_COMPUTE)
         # per head the key up-projection transposed, [rank, dim]: it multiplies the unrotated query
         self.w_uk_t = self._place(tensors["uk"].view(n, self.dim, self.rank).transpose(1, 2).contiguous(), KEEP_COMPUTE)
+        if self.project_up:
+            self.w_uk = self._place(tensors["uk"], KEEP_COMPUTE)
         self.w_uv = self._place(tensors["uv"].view(n, self.vdim, self.rank).contiguous(), KEEP_COMPUTE)
         self.sink = self._place(tensors["sink"], KEEP_FLOAT32) if self.spec.sink else None
         self.w_o = self._place(tensors["o"], KEEP_COMPUTE)
@@ -121,6 +137,42 @@ class LatentAttention(Mixer):
         groups = max(1, tiles * -(-self.heads // ops.LATENT_ATTENTION_ROWS))
         keys = ctx.max_total_len if not self.window else min(ctx.max_total_len, self.window + ctx.max_new_tokens - 1)
         return max(1, min(self.compute_units // groups, keys // _MIN_KEYS_PER_SPLIT, 64))
+
+    def _portions(self, ctx):
+        """The step's long portions and the heads whose keys and values are held at once, or ``None``."""
+        if not self.project_up or ctx.max_new_tokens < _PROMPT_LEAST:
+            return None
+        portions = ctx.long_portions(_PROMPT_LEAST, self.window)
+        work = (portions[7] + _TOKEN_AS_KEYS * portions[8]) * self.heads
+        if work < (_UP_LEAST if portions[6] is None else _UP_LEAST_BESIDE):
+            return None
+        most = ops.PROMPT_ROWS_SCRATCH_BYTES // (portions[4] * (self.dim + self.vdim) * 2)
+        if most < 1:
+            return None
+        return portions, -(-self.heads // -(-self.heads // min(most, self.heads)))
+
+    def _attend_up(self, q, values, down, plane, table, ctx, portions, at_once):
+        """The long portions' rows of ``values``, from queries ``q`` whose rotated parts are turned."""
+        rows, dev = portions[4], q.device
+        latents = torch.empty((rows, self.rank), dtype=self.dtype, device=dev)
+        keys = torch.empty(rows * (at_once * self.dim + self.rot), dtype=self.dtype, device=dev)
+        up = torch.empty((at_once * self.vdim, rows), dtype=self.dtype, device=dev)
+        w_uv = self.w_uv.view(self.heads * self.vdim, self.rank)
+        gate = down[:, self.gate_at: self.gate_at + self.gate_cols] if self.gate_cols else None
+        width = self.dim + self.rot
+        for a in range(0, self.heads, at_once):
+            b = min(a + at_once, self.heads)
+            own = rows * (b - a) * self.dim
+            part = keys[: own + rows * self.rot]
+            if a == 0 or b - a < at_once:      # (the rotated parts lie behind the heads' own)
+                ops.latent_rows(plane, table, ctx.req_indptr, ctx.ctx_lens, portions, self.rank, self.rot, latents,
+                                part[own:].view(rows, self.rot) if self.rot else None, self.window)
+            ops.linear(latents, self.w_uk[a * self.dim: b * self.dim], None, part[:own].view(rows, (b - a) * self.dim))
+            ops.linear(w_uv[a * self.vdim: b * self.vdim], latents, None, up[: (b - a) * self.vdim])
+            ops.prompt_rows_attention(q[:, a * width: b * width], values[:, a * self.vdim: b * self.vdim], part, up[: (b - a) * self.vdim], rows, ctx.req_indptr,
+                                      ctx.ctx_lens, portions, b - a, self.dim, self.rot, self.vdim, self.scale, self.sink[a:b] if self.sink is not None else None,
+                                      self.window, gate[:, a:b] if self.spec.gate else None,
+                                      gate[:, a * self.vdim: b * self.vdim] if self.spec.gate_values else None)
 
     def forward(self, h, ctx, cache):
         T, n = h.shape[0], self.heads
@@ -132,38 +184,71 @@ class LatentAttention(Mixer):
         down = torch.empty((T, self.down_cols), dtype=self.dtype, device=dev)
         ops.linear(h, self.w_down, None, down)
         write = (ctx.token_req, table, plane, cache.page_size) if cache.writable else (None, None, None, 0)
-        # the query against a cache row: [W_uk^T q_unrotated, rotated part], head by head
-        qrow = torch.empty((T, n * self.row), dtype=self.dtype, device=dev)
+        long = self._portions(ctx)
         if self.q_rank:
             cq = torch.empty((T, self.q_rank), dtype=self.dtype, device=dev)
             ops.latent_prepare(down, self.q_rank, self.rank, self.rot, rot_dims, self.w_dq_norm, self.w_dkv_norm, float(self.spec.norm_eps),
                                ctx.positions, inv_freq, cq, *write, halves=self.halves)
             q = torch.empty((T, n * (self.dim + self.rot)), dtype=self.dtype, device=dev)
             ops.linear(cq, self.w_uq, None, q)
-            if self.rot:
-                ops.rotate_pairs(q, self.dim + self.rot, self.dim, qrow, self.row, self.rank, ctx.positions, inv_freq, n, self.rot, self.halves)
         else:                       # the queries are the first columns of the projection
-            ops.latent_prepare(down, 0, self.rank, self.rot, rot_dims, None, self.w_dkv_norm, float(self.spec.norm_eps),
-                               ctx.positions, inv_freq, None, *write, kv_off=self.q_cols, halves=self.halves,
-                               queries=(qrow, n, self.dim + self.rot, self.dim) if self.rot else None)
             q = down[:, : self.q_cols]
-        ops.heads_linear(q, self.dim + self.rot, self.w_uk_t, qrow, self.row)
-        # (sequences whose block table the matrix-core kernel cannot keep in shared memory go to the general kernel and its tiles)
-        general = table.shape[1] > ops.LATENT_MFMA_MAX_BLOCKS
-        tq = self.general_tile_tokens if general else self.tile_tokens
-        tile_req, tile_tok0, tiles = ctx.tiles(tq)
-        if ctx.decode_only and tiles == T:          # one token per request: no tile list to look up
-            tile_req = tile_tok0 = None
-        mixed_latent = torch.empty((T, n * self.rank), dtype=self.dtype, device=dev)
-        ops.latent_attention(qrow, mixed_latent, plane, table, ctx.req_indptr, ctx.ctx_lens, tile_req, tile_tok0, tiles, tq,
-                             n, self.rank, self.rot, cache.page_size, self.scale, self.sink, self._splits(ctx, tiles),
-                             general=general, max_new_tokens=ctx.max_new_tokens, window=self.window,
-                             gate=down[:, self.gate_at:] if self.spec.gate else None)
         values = torch.empty((T, n * self.vdim), dtype=self.dtype, device=dev)
-        ops.heads_linear(mixed_latent, self.rank, self.w_uv, values, self.vdim,
-                         gate=down[:, self.gate_at: self.gate_at + self.gate_cols] if self.spec.gate_values else None)
+        # the query against a cache row: [W_uk^T q_unrotated, rotated part], head by head
+        if long is None:
+            qrow = torch.empty((T, n * self.row), dtype=self.dtype, device=dev)
+            if not self.q_rank:
+                ops.latent_prepare(down, 0, self.rank, self.rot, rot_dims, None, self.w_dkv_norm, float(self.spec.norm_eps),
+                                   ctx.positions, inv_freq, None, *write, kv_off=self.q_cols, halves=self.halves,
+                                   queries=(qrow, n, self.dim + self.rot, self.dim) if self.rot else None)
+            elif self.rot:
+                ops.rotate_pairs(q, self.dim + self.rot, self.dim, qrow, self.row, self.rank, ctx.positions, inv_freq, n, self.rot, self.halves)
+            # (sequences whose block table the matrix-core kernel cannot keep in shared memory go to the general kernel and its tiles)
+            general = table.shape[1] > ops.LATENT_MFMA_MAX_BLOCKS
+            tq = self.general_tile_tokens if general else self.tile_tokens
+            tile_req, tile_tok0, tiles = ctx.tiles(tq)
+            if ctx.decode_only and tiles == T:          # one token per request: no tile list to look up
+                tile_req = tile_tok0 = None
+            self._attend_absorbed(q, qrow, values, down, plane, table, ctx, ctx.req_indptr, tile_req, tile_tok0, tiles, tq, general, ctx.max_new_tokens)
+        else:
+            portions, at_once = long
+            if not self.q_rank:
+                ops.latent_prepare(down, 0, self.rank, self.rot, rot_dims, None, self.w_dkv_norm, float(self.spec.norm_eps),
+                                   ctx.positions, inv_freq, None, *write, kv_off=self.q_cols, halves=self.halves)
+            if self.rot:
+                ops.rotate_pairs(q, self.dim + self.rot, self.dim, q, self.dim + self.rot, self.dim, ctx.positions, inv_freq, n, self.rot, self.halves)
+            if portions[6] is not None:
+                self._attend_others(q, values, down, plane, table, ctx, portions)
+            self._attend_up(q, values, down, plane, table, ctx, portions, at_once)
         if self.dtype == torch.bfloat16 and ops.linear_partials_pay(T, self.hidden, n * self.vdim):
             return ops.linear_partials(values, self.w_o)      # few rows against a narrow matrix: the next norm adds the slabs up
         out = torch.empty((T, self.hidden), dtype=self.dtype, device=dev)
         ops.linear(values, self.w_o, None, out)
         return out
+
+    def _attend_others(self, q, values, down, plane, table, ctx, portions):
+        """The rows of ``values`` of the requests beside the long portions, their tokens taken out of the step, from queries whose rotated parts are turned."""
+        general = table.shape[1] > ops.LATENT_MFMA_MAX_BLOCKS
+        tq = self.general_tile_tokens if general else self.tile_tokens
+        tile_req, tile_tok0, tiles, tokens, count, _ = ctx.tiles_by_length(tq, tq, _PROMPT_LEAST)[0]
+        few = q.index_select(0, tokens)
+        qrow = torch.empty((count, self.heads * self.row), dtype=self.dtype, device=q.device)
+        if self.rot:
+            qrow.view(count, self.heads, self.row)[:, :, self.rank:] = few.view(count, self.heads, self.dim + self.rot)[:, :, self.dim:]
+        out = torch.empty((count, self.heads * self.vdim), dtype=self.dtype, device=q.device)
+        most = 1 if count == ctx.num_requests - portions[3] else tq
+        self._attend_absorbed(few, qrow, out, down.index_select(0, tokens) if self.gate_cols else down, plane, table, ctx, portions[6], tile_req, tile_tok0,
+                              tiles, tq, general, most)
+        values.index_copy_(0, tokens.long(), out)
+
+    def _attend_absorbed(self, q, qrow, values, down, plane, table, ctx, indptr, tile_req, tile_tok0, tiles, tq, general, most_new):
+        """``values`` of queries whose rotated parts lie in ``qrow`` already, against the cached rows as they are."""
+        T, n = q.shape[0], self.heads
+        ops.heads_linear(q, self.dim + self.rot, self.w_uk_t, qrow, self.row)
+        mixed_latent = torch.empty((T, n * self.rank), dtype=self.dtype, device=q.device)
+        ops.latent_attention(qrow, mixed_latent, plane, table, indptr, ctx.ctx_lens, tile_req, tile_tok0, tiles, tq,
+                             n, self.rank, self.rot, plane.shape[2], self.scale, self.sink, self._splits(ctx, tiles),
+                             general=general, max_new_tokens=most_new, window=self.window,
+                             gate=down[:, self.gate_at:] if self.spec.gate else None)
+        ops.heads_linear(mixed_latent, self.rank, self.w_uv, values, self.vdim,
+                         gate=down[:, self.gate_at: self.gate_at + self.gate_cols] if self.spec.gate_values else None)
