@@ -1,4 +1,4 @@
-"""Attention over a paged cache for long portions of prompts (tiles of 128 rows) against the kernel that walks the keys of one token and head.
+"""Attention over a paged cache for long portions of prompts (tiles of 128 rows) and for decoded tokens (heads together, keys split) against the kernel that walks the keys of one token and head.
 
 Both get the same bfloat16 queries, keys and values.  The tiles round a weight to bfloat16 (half a unit: 2^-9 of it) and sum the rounded ones, so a
 column moves by at most 2^-8 of the weights' mean of |value| (which the largest |value| bounds), and both round what they store (2^-9 of it each);
@@ -88,3 +88,19 @@ def test_long_portions_against_the_token_kernel(H, G, dim, vdim, page, form):
     times = -(-12288 // (H * (sum(new) - len(new))))
     _close(*_both(H, G, dim, vdim, page, ctx * times, new * times, g, **more))
     _close(*_both(H, G, dim, vdim, page, [11], [-(-12288 // H) + 1], g, spread=2.0, **more))
+
+
+@pytest.mark.parametrize("H, G, dim, vdim", [(4, 4, 128, 128), (16, 2, 64, 64), (6, 1, 192, 64), (34, 2, 128, 128), (5, 1, 64, 128), (20, 1, 192, 128)])
+@pytest.mark.parametrize("page", [8, 24])
+@pytest.mark.parametrize("form", ["plain", "window", "chunk", "kept", "pooled", "capped", "halves"])
+@pytest.mark.parametrize("ctx", [[0], [700], [0, 1, 127, 128, 1500, 33], [40] * 70])
+@pytest.mark.parametrize("splits", [None, 1, 5])
+def test_decoded_tokens_with_their_heads_together_against_the_token_kernel(H, G, dim, vdim, page, form, ctx, splits, monkeypatch):
+    if splits:
+        monkeypatch.setattr(ops, "local_decode_splits", lambda *a: splits)
+    g = torch.Generator(device="cuda").manual_seed(H + page)
+    freq = torch.rand(vdim // 4, generator=g, device="cuda")
+    more = {"plain": {}, "window": dict(window=450, sink=torch.linspace(-3, 8, H, device="cuda")), "chunk": dict(chunk=352, gain=0.7),
+            "kept": dict(window=170, keep=21, gated=True), "pooled": dict(window=333, pool=4, sink=torch.zeros(H, device="cuda"), gated=True),
+            "capped": dict(cap=5.0, turn=(freq, vdim // 2, False)), "halves": dict(turn=(freq, vdim // 2, True), window=300)}[form]
+    _close(*_both(H, G, dim, vdim, page, ctx, [1] * len(ctx), g, **more))

@@ -232,7 +232,11 @@ __device__ __forceinline__ float cap_score_fast(float s, float cap, float two_lo
     return cap * (1.f - 2.f * __builtin_amdgcn_rcpf(e + 1.f));
 }
 
-template <int DK, int DV>          // dim / 32 and vdim / 16
+// HEADS: every request brings one token; a tile's 16 columns are heads of one key/value head (chunks of up to 16) instead of tokens of one head, so the
+// heads read their keys and values once, and with splits > 1 a tile's keys are dealt to that many work-groups, each of which leaves its sums for
+// local_merge_kernel.  Splits are what one request needs: a work-group's CU fetches at most 64 bytes a clock, 2 MB of a head's keys and values at 4000
+// tokens take it 14 us.
+template <int DK, int DV, bool HEADS>          // dim / 32 and vdim / 16
 __global__ void __launch_bounds__(256)
 local_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __restrict__ out, int out_ld, const bf16_t* __restrict__ k_plane,
                             const bf16_t* __restrict__ v_plane, const int* __restrict__ block_table, int table_ld, int table_width,
@@ -240,20 +244,25 @@ local_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __re
                             const int* __restrict__ tile_tok0, int heads, int kv_heads, int page_size, float scale, float cap,
                             LocalMask mask, float gain, const float* __restrict__ sink, const bf16_t* __restrict__ pk_plane,
                             const bf16_t* __restrict__ pv_plane, const int* __restrict__ pool_table, int pool_table_ld, int pool_table_width, int pool,
-                            OutputTurn back, const bf16_t* __restrict__ gate, int gate_ld, int below) {
+                            OutputTurn back, const bf16_t* __restrict__ gate, int gate_ld, int below, float* __restrict__ part_o,
+                            float2* __restrict__ part_ml) {
     constexpr int dim = DK * 32, vdim = DV * 16;
     extern __shared__ float la_smem[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, kq = lane >> 4;
-    const int head = blockIdx.y;
+    const int group = heads / kv_heads, chunks = (group + 15) / 16;
+    const int g = HEADS ? blockIdx.y / chunks : blockIdx.y / group;
+    const int head0 = HEADS ? g * group + blockIdx.y % chunks * 16 : blockIdx.y;      // the head of the first column
+    const int split = HEADS ? blockIdx.z : 0, splits = HEADS ? gridDim.z : 1;
     const int tile = blockIdx.x;
     const int req = tile_req ? tile_req[tile] : tile;
     const int first = req_indptr[req], n_new = req_indptr[req + 1] - first;
     const int tok0 = tile_tok0 ? tile_tok0[tile] : 0;
     const int n_tile = min(LAM_TOKENS, n_new - tok0);            // tokens of this tile
     if (n_tile <= 0 || n_new >= below) return;                   // (requests of `below` tokens or more are local_prompt_kernel's)
-    const int g = head / (heads / kv_heads);
+    const int n_cols = HEADS ? min(16, group - blockIdx.y % chunks * 16) : n_tile;
     const int p0 = ctx_lens[req] + tok0;                         // position of the tile's first token
-    const int my_tok = min(li, n_tile - 1);                      // (lanes beyond the tile's tokens repeat its last one and store nothing)
+    const int my_tok = HEADS ? 0 : min(li, n_cols - 1);          // (lanes beyond the tile's columns repeat its last one and store nothing)
+    const int my_head = HEADS ? head0 + min(li, n_cols - 1) : head0;
     const int my_p = p0 + my_tok, my_lo = mask.first(my_p);
     const int* table = block_table + (size_t)req * table_ld;
     const float inv_cap = cap > 0.f ? 2.f * LA_LOG2E / cap : 0.f;
@@ -264,7 +273,7 @@ local_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __re
 
     LaFrag qf[DK];
     {
-        const bf16_t* qrow = q + (size_t)(first + tok0 + my_tok) * q_ld + head * dim + 8 * kq;
+        const bf16_t* qrow = q + (size_t)(first + tok0 + my_tok) * q_ld + my_head * dim + 8 * kq;
 #pragma unroll
         for (int s = 0; s < DK; ++s) qf[s].u = *(const uint4*)(qrow + 32 * s);
     }
@@ -281,10 +290,11 @@ local_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __re
     auto run = [&](const bf16_t* __restrict__ kp, const bf16_t* __restrict__ vp, const int* __restrict__ tbl, int tbl_width, int lo_valid, int hi_valid,
                    int my_first, int my_last) {
         const int base0 = lo_valid / LAM_KEYS * LAM_KEYS;
-        if (base0 + LAM_KEYS * wave > hi_valid) return;
+        const int mine = base0 + LAM_KEYS * (split * LAM_WAVES + wave), stride = splits * LAM_STRIDE;      // (key steps are dealt to the splits' waves in turn)
+        if (mine > hi_valid) return;
         // The pages of up to 64 blocks of the request lie in a register across the wave (lane i: block tab_first + i) and are read from
         // there, so that no fetch waits for a look-up in memory; the window moves on every 64 blocks.
-        int tab_first = page_of(base0);
+        int tab_first = page_of(mine);
         int tab_reg = tbl[min(tab_first + lane, tbl_width - 1)];
         auto page_at = [&](int key) { return __shfl(tab_reg, page_of(key) - tab_first, TL_WAVE); };
         // The keys and values of a step are fetched one step ahead, while the step before is worked on.
@@ -315,7 +325,7 @@ local_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __re
                 s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[s].v, qf[s].v, s0, 0, 0, 0);
                 s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[s].v, qf[s].v, s1, 0, 0, 0);
             }
-            if (base + LAM_STRIDE <= hi_valid) fetch(base + LAM_STRIDE, vnext);
+            if (base + stride <= hi_valid) fetch(base + stride, vnext);
             // ---- cap, mask, running maximum (scores in units of log 2 from here on, so that the weights are plain powers of two)
             float sc[8];
             float mx = -INFINITY;
@@ -358,10 +368,10 @@ local_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __re
 #pragma unroll
             for (int j = 0; j < DV; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[j].v, pf.v, acc[j], 0, 0, 0);
         };
-        fetch(base0 + LAM_KEYS * wave, va);
-        for (int base = base0 + LAM_KEYS * wave; base <= hi_valid; base += 2 * LAM_STRIDE) {
+        fetch(mine, va);
+        for (int base = mine; base <= hi_valid; base += 2 * stride) {
             step(base, va, vb);
-            if (base + LAM_STRIDE <= hi_valid) step(base + LAM_STRIDE, vb, va);
+            if (base + stride <= hi_valid) step(base + stride, vb, va);
         }
     };
     if (pool > 0 && mask.window > 0) {
@@ -389,9 +399,31 @@ local_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __re
     for (int j = 0; j < DV; ++j)
         *(float4*)(sm_o + ((size_t)wave * LAM_TOKENS + li) * vdim + 16 * j + 4 * kq) = make_float4(acc[j][0], acc[j][1], acc[j][2], acc[j][3]);
     __syncthreads();
-    const float sink2 = sink ? sink[head] * LA_LOG2E : -INFINITY;       // in units of log 2, like the maxima
-    // columns ca and cb of a token (cb < 0: ca alone)
+    if (HEADS && splits > 1) {
+        // this work-group's share: maximum, sum and weighted sum of the values, not yet divided
+        for (int idx = threadIdx.x; idx < n_cols * vdim; idx += blockDim.x) {
+            const int c = idx / vdim, col = idx % vdim;
+            float top = sm_m[c];
+#pragma unroll
+            for (int w = 1; w < LAM_WAVES; ++w) top = fmaxf(top, sm_m[w * LAM_TOKENS + c]);
+            const float use = top == -INFINITY ? 0.f : top;      // (a share without keys: zeros)
+            float den = 0.f, o = 0.f;
+#pragma unroll
+            for (int w = 0; w < LAM_WAVES; ++w) {
+                const float f = __builtin_amdgcn_exp2f(sm_m[w * LAM_TOKENS + c] - use);
+                den = fmaf(sm_l[w * LAM_TOKENS + c], f, den);
+                o = fmaf(sm_o[((size_t)w * LAM_TOKENS + c) * vdim + col], f, o);
+            }
+            const size_t at = ((size_t)first * heads + head0 + c) * splits + split;
+            part_o[at * vdim + col] = o;
+            if (col == 0) part_ml[at] = make_float2(top, den);
+        }
+        return;
+    }
+    // columns ca and cb of a token or head (cb < 0: ca alone)
     auto joined = [&](int tok, int ca, int cb, float& u, float& v) {
+        const int head = HEADS ? head0 + tok : head0;
+        const float sink2 = sink ? sink[head] * LA_LOG2E : -INFINITY;       // in units of log 2, like the maxima
         float top = sm_m[tok];
 #pragma unroll
         for (int w = 1; w < LAM_WAVES; ++w) top = fmaxf(top, sm_m[w * LAM_TOKENS + tok]);
@@ -407,40 +439,79 @@ local_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __re
             if (cb >= 0) v = fmaf(o[cb], f, v);
         }
         float norm = gain / den;
-        if (gate) norm *= sigmoid(to_float(gate[(size_t)(first + tok0 + tok) * gate_ld + head]));
+        if (gate) norm *= sigmoid(to_float(gate[(size_t)(first + tok0 + (HEADS ? 0 : tok)) * gate_ld + head]));
         u *= norm;
         v *= norm;
     };
-    bf16_t* const orow0 = out + (size_t)(first + tok0) * out_ld + head * vdim;
+    bf16_t* const orow0 = out + (size_t)(first + tok0) * out_ld + head0 * vdim;
+    const size_t col_ld = HEADS ? vdim : out_ld;
     if (back.freq) {
-        for (int idx = threadIdx.x; idx < n_tile * (vdim / 2); idx += blockDim.x) {
+        for (int idx = threadIdx.x; idx < n_cols * (vdim / 2); idx += blockDim.x) {
             const int tok = idx / (vdim / 2), m = idx % (vdim / 2);
             const int ca = back.column_a(m), cb = back.column_b(m);
             float u, v;
             joined(tok, ca, cb, u, v);
-            back.turn(m, p0 + tok, u, v);
-            orow0[(size_t)tok * out_ld + ca] = from_float<bf16_t>(u);
-            orow0[(size_t)tok * out_ld + cb] = from_float<bf16_t>(v);
+            back.turn(m, HEADS ? p0 : p0 + tok, u, v);
+            orow0[tok * col_ld + ca] = from_float<bf16_t>(u);
+            orow0[tok * col_ld + cb] = from_float<bf16_t>(v);
         }
         return;
     }
-    for (int idx = threadIdx.x; idx < n_tile * vdim; idx += blockDim.x) {
+    for (int idx = threadIdx.x; idx < n_cols * vdim; idx += blockDim.x) {
         const int tok = idx / vdim, col = idx % vdim;
         float u, v;
         joined(tok, col, -1, u, v);
-        orow0[(size_t)tok * out_ld + col] = from_float<bf16_t>(u);
+        orow0[tok * col_ld + col] = from_float<bf16_t>(u);
     }
 }
 
-template <int DK, int DV>
+// A token's head from the shares of its splits: weights exp(m_s - M) in the order of the splits, the sink's term, then what the tile kernel does as it stores.
+// A wave per token and head, lanes over pairs of columns; the shares are read with nothing in between that waits.
+__global__ void __launch_bounds__(TL_WAVE)
+local_merge_kernel(const float* __restrict__ part_o, const float2* __restrict__ part_ml, bf16_t* __restrict__ out, int out_ld, const int* __restrict__ req_indptr,
+                   const int* __restrict__ ctx_lens, const int* __restrict__ tile_req, int heads, int vdim, int splits, float gain, const float* __restrict__ sink,
+                   OutputTurn back, const bf16_t* __restrict__ gate, int gate_ld) {
+    const int req = tile_req ? tile_req[blockIdx.x] : blockIdx.x, head = blockIdx.y, lane = threadIdx.x;
+    const int token = req_indptr[req];
+    if (req_indptr[req + 1] <= token) return;
+    const size_t at = ((size_t)token * heads + head) * splits;
+    const float2 ml = lane < splits ? part_ml[at + lane] : make_float2(-INFINITY, 0.f);
+    const float sink2 = sink ? sink[head] * LA_LOG2E : -INFINITY;
+    const float top = fmaxf(wave_max(ml.x), sink2);
+    const float f = __builtin_amdgcn_exp2f(ml.x - top);             // (0 for a share without keys)
+    const float den = wave_sum(ml.y * f) + __builtin_amdgcn_exp2f(sink2 - top);
+    float norm = gain / den;
+    if (gate) norm *= sigmoid(to_float(gate[(size_t)token * gate_ld + head]));
+    bf16_t* o = out + (size_t)token * out_ld + (size_t)head * vdim;
+    const float* po = part_o + at * vdim;
+    for (int m = lane; m < vdim / 2; m += TL_WAVE) {
+        const int ca = back.freq ? back.column_a(m) : 2 * m, cb = back.freq ? back.column_b(m) : 2 * m + 1;
+        float u = 0.f, v = 0.f;
+#pragma unroll 8
+        for (int s = 0; s < splits; ++s) {
+            const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), s));
+            u = fmaf(w, po[(size_t)s * vdim + ca], u);
+            v = fmaf(w, po[(size_t)s * vdim + cb], v);
+        }
+        u *= norm;
+        v *= norm;
+        if (back.freq) back.turn(m, ctx_lens[req], u, v);
+        o[ca] = from_float<bf16_t>(u);
+        o[cb] = from_float<bf16_t>(v);
+    }
+}
+
+template <int DK, int DV, bool HEADS = false>
 static void launch_local_mfma(const void* q, int q_ld, void* out, int out_ld, const void* k_plane, const void* v_plane, const void* block_table,
                               int table_ld, int table_width, const void* req_indptr, const void* ctx_lens, const void* tile_req,
                               const void* tile_tok0, int tiles, int heads, int kv_heads, int page_size, float scale, float cap, LocalMask mask,
                               float gain, const void* sink, const void* pk_plane, const void* pv_plane, const void* pool_table, int pool_table_ld,
-                              int pool_table_width, int pool, OutputTurn back, const void* gate, int gate_ld, int below, hipStream_t stream) {
-    dim3 grid(tiles, heads), block(LAM_WAVES * TL_WAVE);
+                              int pool_table_width, int pool, OutputTurn back, const void* gate, int gate_ld, int below, hipStream_t stream, int splits = 1, void* part_o = nullptr,
+                              void* part_ml = nullptr) {
+    const int group = heads / kv_heads;
+    dim3 grid(tiles, HEADS ? kv_heads * ((group + 15) / 16) : heads, splits), block(LAM_WAVES * TL_WAVE);
     const size_t smem = sizeof(float) * LAM_WAVES * LAM_TOKENS * (2 + DV * 16);
-    auto kernel = local_attention_mfma_kernel<DK, DV>;
+    auto kernel = local_attention_mfma_kernel<DK, DV, HEADS>;
     static bool raised = false;                      // (per instance of the template)
     if (smem > 48 * 1024 && !raised) {
         hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
@@ -449,7 +520,7 @@ static void launch_local_mfma(const void* q, int q_ld, void* out, int out_ld, co
     kernel<<<grid, block, smem, stream>>>((const bf16_t*)q, q_ld, (bf16_t*)out, out_ld, (const bf16_t*)k_plane, (const bf16_t*)v_plane,
         (const int*)block_table, table_ld, table_width, (const int*)req_indptr, (const int*)ctx_lens, (const int*)tile_req, (const int*)tile_tok0,
         heads, kv_heads, page_size, scale, cap, mask, gain, (const float*)sink, (const bf16_t*)pk_plane, (const bf16_t*)pv_plane, (const int*)pool_table,
-        pool_table_ld, pool_table_width, pool, back, (const bf16_t*)gate, gate_ld, below);
+        pool_table_ld, pool_table_width, pool, back, (const bf16_t*)gate, gate_ld, below, (float*)part_o, (float2*)part_ml);
 }
 
 // Whether the matrix-core kernel is built for these sizes.
@@ -901,13 +972,16 @@ static bool local_prompt_fits(const LocalArgs& a, int dim, int vdim, int pages, 
 
 // Tiles of up to 16 consecutive tokens of one request: tile i belongs to request tile_req[i] (null: request i) and starts at that
 // request's token tile_tok0[i] of the step (null: 0).
+// Whether decoded tokens' heads go together (HEADS) at these sizes.
+extern "C" int tl_local_heads_fits(int dim, int vdim) { return (dim == 64 || dim == 128 || dim == 192) && (vdim == 64 || vdim == 128); }
+
 extern "C" int tl_local_attention_tiles(const void* q, int q_ld, void* out, int out_ld, const void* k_plane, const void* v_plane, int pages,
                                         const void* block_table, int table_ld, int table_width, const void* req_indptr, const void* ctx_lens,
                                         const void* tile_req, const void* tile_tok0, int tiles, int heads, int kv_heads, int dim, int vdim,
                                         int page_size, float scale, float cap, int chunk, int window, float gain, const void* sink,
                                         const void* pk_plane, const void* pv_plane, const void* pool_table, int pool_table_ld, int pool_table_width,
                                         int pool, int keep_first, const void* turn_freq, int turn_dims, int turn_halves, const void* gate, int gate_ld,
-                                        int tokens, int requests, int pool_pages, hipStream_t stream) {
+                                        int tokens, int requests, int pool_pages, int splits, void* part_o, void* part_ml, hipStream_t stream) {
     TL_REQUIRE(!gate || gate_ld >= heads, "local_attention_tiles: a gate has a number per head");
     TL_REQUIRE(!turn_freq || (turn_dims > 0 && turn_dims % 2 == 0 && turn_dims <= vdim && vdim % 2 == 0), "local_attention_tiles: an output of %d columns turned over %d", vdim, turn_dims);
     TL_REQUIRE(keep_first >= 0 && (keep_first == 0 || (window > 0 && chunk == 0)), "local_attention_tiles: kept first tokens stand beside a window, without chunks");
@@ -926,6 +1000,24 @@ extern "C" int tl_local_attention_tiles(const void* q, int q_ld, void* out, int 
                       table_width, (const int*)req_indptr, (const int*)ctx_lens, requests, heads, kv_heads, (group + cut - 1) / cut, page_size,
                       __builtin_ctz(page_size), scale, cap, mask, gain, (const float*)sink, (const bf16_t*)pk_plane, (const bf16_t*)pv_plane,
                       (const int*)pool_table, pool_table_ld, pool_table_width, pool, back, (const bf16_t*)gate, gate_ld, LP_LEAST, nullptr, nullptr, nullptr, 0, 0, 0, 0u, nullptr, 0};
+    if (splits > 0) {        // one token a request, its heads together
+        TL_REQUIRE(tl_local_heads_fits(dim, vdim) && tiles == tokens && splits <= TL_WAVE && (splits == 1 || (part_o && part_ml)), "local_attention_tiles: not built for these splits");
+#define TL_LAH(DK, DV)                                                                                                                       \
+    launch_local_mfma<DK, DV, true>(q, q_ld, out, out_ld, k_plane, v_plane, block_table, table_ld, table_width, req_indptr, ctx_lens,         \
+                                    tile_req, tile_tok0, tiles, heads, kv_heads, page_size, scale, cap, mask, gain, sink, pk_plane, pv_plane, \
+                                    pool_table, pool_table_ld, pool_table_width, pool, back, gate, gate_ld, INT_MAX, stream, splits, part_o, part_ml)
+        if (dim == 64) { if (vdim == 64) TL_LAH(2, 4); else TL_LAH(2, 8); }
+        else if (dim == 128) { if (vdim == 64) TL_LAH(4, 4); else TL_LAH(4, 8); }
+        else { if (vdim == 64) TL_LAH(6, 4); else TL_LAH(6, 8); }
+#undef TL_LAH
+        TL_CHECK_LAUNCH("local_attention_heads");
+        if (splits > 1) {
+            local_merge_kernel<<<dim3(tiles, heads), TL_WAVE, 0, stream>>>((const float*)part_o, (const float2*)part_ml, (bf16_t*)out, out_ld, (const int*)req_indptr,
+                (const int*)ctx_lens, (const int*)tile_req, heads, vdim, splits, gain, (const float*)sink, back, (const bf16_t*)gate, gate_ld);
+            TL_CHECK_LAUNCH("local_merge");
+        }
+        return TL_OK;
+    }
     int below = INT_MAX;
     if (tile_req && (long)tiles * LAM_TOKENS >= tokens && local_prompt_pays(a, tokens) && local_prompt_fits(a, dim, vdim, pages, pool_pages)) {
         const long most = tokens / LP_LEAST, tiles_most = tokens / (LP_ROWS / a.gcap) + (requests < most ? requests : most);

@@ -1279,6 +1279,21 @@ def local_attention_mfma_fits(dtype: torch.dtype, dim: int, vdim: int, page_size
     return dtype == torch.bfloat16 and bool(_lib("local_attention").tl_local_attention_mfma_fits(c_int(dim), c_int(vdim), c_int(page_size)))
 
 
+def local_decode_splits(tokens: int, heads: int, kv_heads: int, keys: int, units: int) -> int:
+    """How :func:`local_attention` takes a step of one token a request, ``keys`` the most that a query can read: 0 for a work-group per token and head, else
+    the work-groups that share the keys of one token's tile of heads (up to 16 heads of a key/value head): one to a compute unit and no more, 256 keys each
+    where that leaves four, never under 128 (a step of 32 for each of its four waves), 32 at most.
+
+    The heads together pay from where the heads' own work-groups are two to a compute unit (32 heads over 8, 60 keys, us: 32 requests 15.4 against 5.4; 8 requests 5.0
+    against 5.4), or one with 512 keys (8 requests 10.6 against 8.4); the splits from 1024 keys on, also for one request (4000 keys 48 against 15, 16 heads of 64 over 4
+    36 against 13; 512 keys 8.6 against 9.0).  More splits cost their merge: 4000 keys with 32 of them 17.4."""
+    group = heads // kv_heads
+    if not (keys >= 1024 or (group > 1 and (tokens * heads >= 2 * units or (tokens * heads >= units and keys >= 512)))):
+        return 0
+    tiles = tokens * kv_heads * -(-group // 16)
+    return max(1, min(units // tiles, max(4, keys // 256), keys // 128, 32))
+
+
 def local_attention(q: torch.Tensor, out: torch.Tensor, k_plane: torch.Tensor, v_plane: torch.Tensor, block_table: torch.Tensor,
                     token_req: torch.Tensor, positions: torch.Tensor, heads: int, kv_heads: int, dim: int, vdim: int, page_size: int,
                     scale: float, softcap: float = 0.0, chunk: int = 0, window: int = 0, gain: float = 1.0, tiles=None,
@@ -1337,13 +1352,22 @@ def local_attention(q: torch.Tensor, out: torch.Tensor, k_plane: torch.Tensor, v
         _i32(tile_tok0, "tile_tok0", n_tiles)
         if tile_req is None and n_tiles > R:
             raise KernelError("local_attention: without a tile list there is one tile per request")
+        # one token a request: the heads of a key/value head together, and its keys dealt to enough work-groups to fill the chip
+        splits, part_o, part_ml = 0, None, None
+        if tile_req is not None and n_tiles == T and T > 0 and lib.tl_local_heads_fits(c_int(dim), c_int(vdim)):
+            keys = block_table.shape[1] * page_size if not (window or chunk) else min(block_table.shape[1] * page_size, max(window, chunk))
+            keys += keep_first + (pool_table.shape[1] * page_size if pool else 0)
+            splits = local_decode_splits(T, heads, kv_heads, keys, compute_units())
+            if splits > 1:
+                part_o = torch.empty((T * heads * splits, vdim), dtype=torch.float32, device=q.device)
+                part_ml = torch.empty((T * heads * splits, 2), dtype=torch.float32, device=q.device)
         _check(lib, lib.tl_local_attention_tiles(_ptr(q), c_int(q.stride(0)), _ptr(out), c_int(out.stride(0)), _ptr(k_plane), _ptr(v_plane),
                                                  c_int(k_plane.shape[0]), _ptr(block_table), c_int(block_table.stride(0)), c_int(block_table.shape[1]),
                                                  _ptr(req_indptr), _ptr(ctx_lens), _ptr(tile_req), _ptr(tile_tok0), c_int(n_tiles), c_int(heads),
                                                  c_int(kv_heads), c_int(dim), c_int(vdim), c_int(page_size), c_float(scale), c_float(softcap),
                                                  c_int(chunk), c_int(window), c_float(gain), *pool_args, c_int(pool_table.shape[1] if pool else 0),
                                                  c_int(pool), c_int(keep_first), *turn_args, *gate_args, c_int(T), c_int(R),
-                                                 c_int(pk_plane.shape[0] if pool else 0), _stream()))
+                                                 c_int(pk_plane.shape[0] if pool else 0), c_int(splits), _ptr(part_o), _ptr(part_ml), _stream()))
         return
     _i32(token_req, "token_req", T)
     _i32(positions, "positions", T)
