@@ -984,9 +984,6 @@ wkv_scan_kernel(const T* __restrict__ rkv, int ld, int k_off, int v_off, const f
         for (int e = 0; e < 4; ++e) ub[4 * q + e] = row + e < dim ? bonus[head * dim + row + e] : 0.f;
     }
 
-    // (the state and the bonuses are waited for here: left to the token loop, the wait at its head would cover the next batch's fetches too)
-#pragma unroll
-    for (int r = 0; r < RPL; ++r) asm volatile("" : "+v"(S[r]), "+v"(ub[r]));
     float4 pr[NP], pk[NP], pw[NP];
     float pv = 0.f;
     auto fetch = [&](int base) {
