@@ -562,16 +562,80 @@ __global__ void scaled_add_rmsnorm_kernel(float* __restrict__ residual, const vo
     }
 }
 
+// The same with a row in registers, four neighbouring numbers to a piece and IT pieces to a thread: everything a row needs is requested at once (slabs four at a
+// time, added up in their order), where the kernel above fetches the row again after the sum and the slabs one after the other.  Measured, rows of 2048
+// numbers: one row 5.2 -> 2.4 us, with four slabs 7.4 -> 2.5; 2048 rows 11.4 -> 7.9, with four slabs 22.4 -> 17.3.
+template <typename T, int IT>
+__global__ void scaled_add_rmsnorm_reg_kernel(float* __restrict__ residual, const void* __restrict__ pending, int parts, size_t part_stride, float alpha,
+                                              const void* __restrict__ weight, int weight_f32, float eps, T* __restrict__ out, int hidden) {
+    __shared__ float red[16];
+    const size_t at = (size_t)blockIdx.x * hidden;
+    float r[IT][4], wv[IT][4];
+    float ss = 0.f;
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+        const int i = (it * blockDim.x + threadIdx.x) * 4;
+        if (i < hidden) {
+            float x[4], y[4] = {0.f, 0.f, 0.f, 0.f};
+            Vec4<float>::load(residual + at + i, x);
+            if (weight_f32) Vec4<float>::load((const float*)weight + i, wv[it]);
+            else Vec4<bf16_t>::load((const bf16_t*)weight + i, wv[it]);
+            if (pending && parts == 0) Vec4<T>::load((const T*)pending + at + i, y);
+            if (pending && parts > 0) {
+                const float* slabs = (const float*)pending + at + i;
+                int q = 0;
+                for (; q + 4 <= parts; q += 4) add_slabs<4>(slabs + q * part_stride, part_stride, y);
+                if (parts - q == 3) add_slabs<3>(slabs + q * part_stride, part_stride, y);
+                else if (parts - q == 2) add_slabs<2>(slabs + q * part_stride, part_stride, y);
+                else if (parts - q == 1) add_slabs<1>(slabs + q * part_stride, part_stride, y);
+            }
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                r[it][v] = alpha * x[v] + y[v];
+                ss = fmaf(r[it][v], r[it][v], ss);
+            }
+        }
+    }
+    ss = block_sum(ss, red);
+    const float inv = 1.f / sqrtf(ss / (float)hidden + eps);
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+        const int i = (it * blockDim.x + threadIdx.x) * 4;
+        if (i < hidden) {
+            float y[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) y[v] = r[it][v] * inv * wv[it][v];
+            Vec4<float>::store(residual + at + i, y);
+            if (out) Vec4<T>::store(out + at + i, y);
+        }
+    }
+}
+
+// Rows of a multiple of four numbers up to 16384, everything on 16 bytes; others keep the kernel above.
+template <typename T>
+static void launch_scaled_add_rmsnorm(float* residual, const void* pending, int parts, size_t part_stride, float alpha, const void* weight, int weight_f32,
+                                      float eps, T* out, int rows, int hidden, hipStream_t stream) {
+    const bool aligned = hidden % 4 == 0 && (((uintptr_t)residual | (uintptr_t)pending | (uintptr_t)weight | (uintptr_t)out) & 15) == 0;
+#define TL_SAR(IT, THREADS) scaled_add_rmsnorm_reg_kernel<T, IT><<<rows, THREADS, 0, stream>>>(residual, pending, parts, part_stride, alpha, weight, weight_f32, eps, out, hidden)
+    if (aligned && hidden <= 1024) TL_SAR(1, 256);
+    else if (aligned && hidden <= 2048) TL_SAR(1, 512);
+    else if (aligned && hidden <= 4096) TL_SAR(2, 512);
+    else if (aligned && hidden <= 8192) TL_SAR(4, 512);
+    else if (aligned && hidden <= 16384) TL_SAR(4, 1024);
+    else
+        scaled_add_rmsnorm_kernel<T><<<rows, hidden <= 512 ? 128 : hidden <= 2048 ? 256 : 512, 0, stream>>>(residual, pending, parts, part_stride, alpha, weight, weight_f32,
+                                                                                                         eps, out, hidden);
+#undef TL_SAR
+}
+
 extern "C" int tl_scaled_add_rmsnorm(void* residual, const void* pending, int parts, int total_rows, float alpha, const void* weight,
                                      int weight_f32, float eps, void* out, int rows, int hidden, int dtype, hipStream_t stream) {
     TL_REQUIRE(rows >= 0 && hidden > 0 && parts >= 0, "scaled_add_rmsnorm: bad sizes rows=%d hidden=%d", rows, hidden);
     if (rows == 0) return TL_OK;
     const size_t part_stride = (size_t)total_rows * hidden;
-    dim3 grid(rows), block(hidden <= 512 ? 128 : hidden <= 2048 ? 256 : 512);
-    if (dtype == TL_DT_F32)
-        scaled_add_rmsnorm_kernel<float><<<grid, block, 0, stream>>>((float*)residual, pending, parts, part_stride, alpha, weight, weight_f32, eps, (float*)out, hidden);
+    if (dtype == TL_DT_F32) launch_scaled_add_rmsnorm<float>((float*)residual, pending, parts, part_stride, alpha, weight, weight_f32, eps, (float*)out, rows, hidden, stream);
     else if (dtype == TL_DT_BF16)
-        scaled_add_rmsnorm_kernel<bf16_t><<<grid, block, 0, stream>>>((float*)residual, pending, parts, part_stride, alpha, weight, weight_f32, eps, (bf16_t*)out, hidden);
+        launch_scaled_add_rmsnorm<bf16_t>((float*)residual, pending, parts, part_stride, alpha, weight, weight_f32, eps, (bf16_t*)out, rows, hidden, stream);
     else TL_REQUIRE(false, "scaled_add_rmsnorm: unknown dtype %d", dtype);
     TL_CHECK_LAUNCH("scaled_add_rmsnorm");
     return TL_OK;
