@@ -123,6 +123,18 @@ __device__ __forceinline__ void add_slabs(const float* src, size_t stride, float
         for (int v = 0; v < 4; ++v) r[v] += p[u][v];
 }
 
+// The same for the eight elements at src.
+template <int N>
+__device__ __forceinline__ void add_slab_pairs(const float* src, size_t stride, float (&lo)[4], float (&hi)[4]) {
+    float p[N][4], q[N][4];
+#pragma unroll
+    for (int u = 0; u < N; ++u) { Vec4<float>::load(src + u * stride, p[u]); Vec4<float>::load(src + u * stride + 4, q[u]); }
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) { lo[v] += p[u][v]; hi[v] += q[u][v]; }
+}
+
 template <typename T, int IT>
 __global__ void add_rmsnorm_reg_kernel(float* __restrict__ residual, const void* __restrict__ pending, int parts, size_t part_stride,
                                        const void* __restrict__ weight, int weight_f32, float eps, float gain,
@@ -350,12 +362,16 @@ void rope_cache_write_kernel(T* __restrict__ qkv, int row_stride, int q_heads, i
 // time: a work-group owns one token, a thread one 16-byte piece (four pairs of one head) per round.
 // Queries are rotated in place, keys rotated and copied to their page in whole pieces, values
 // scattered to their transposed place.  (One wave per head, as above, moved 1.7 TB/s on a prompt of
-// 2048 tokens; this is for steps of many tokens.)
-__global__ __launch_bounds__(256)
+// 2048 tokens; this is for steps of many tokens.)  PARTS: the row is the sum of float slabs and the bias, as above; a thread requests its piece's eight numbers of four
+// slabs together, and the work-group is as wide as the row has pieces, up to 1024 threads (512 tokens of 40 + 16 heads of 128, three slabs: 17.5 -> 12.5 us, of which
+// the slabs' 44 MB are nine).
+template <bool PARTS>
+__global__ __launch_bounds__(PARTS ? 1024 : 256)
 void rope_cache_write_rows_kernel(bf16_t* __restrict__ qkv, int row_stride, int q_heads, int kv_heads, int head_dim,
                                   int rot_heads, const int* __restrict__ positions, const float* __restrict__ inv_freq,
                                   const int* __restrict__ token_req, const int* __restrict__ block_table, int bt_stride,
-                                  bf16_t* __restrict__ k_plane, bf16_t* __restrict__ v_plane, int page_size) {
+                                  bf16_t* __restrict__ k_plane, bf16_t* __restrict__ v_plane, int page_size, const float* __restrict__ parts,
+                                  int num_parts, size_t part_stride, int parts_ld, const void* __restrict__ bias, int bias_f32) {
     const int t = blockIdx.x;
     const int pos = positions[t];
     const int heads = q_heads + kv_heads + (k_plane ? kv_heads : 0);
@@ -369,16 +385,41 @@ void rope_cache_write_rows_kernel(bf16_t* __restrict__ qkv, int row_stride, int 
     // back from shared memory by every head's threads (28 query heads and 4 key heads of 128: 2048 tokens 17 -> 12 us).
     __shared__ float2 turn[128];                                   // (head_dim <= 256: the host checks)
     if (inv_freq) {
-        for (int j = threadIdx.x; j < head_dim / 2; j += 256) {
+        for (int j = threadIdx.x; j < head_dim / 2; j += blockDim.x) {
             const float angle = (float)pos * inv_freq[j];
             turn[j] = make_float2(cosf(angle), sinf(angle));
         }
         __syncthreads();
     }
-    for (int p = threadIdx.x; p < heads * pph; p += 256) {
+    for (int p = threadIdx.x; p < heads * pph; p += blockDim.x) {
         const int head = p / pph, d0 = (p % pph) * 8;
         union { uint4 u; uint16_t e[8]; } piece;
-        piece.u = *(const uint4*)(row + (size_t)head * head_dim + d0);
+        float x[8];
+        if (PARTS) {
+            const size_t col = (size_t)head * head_dim + d0;
+            const float* src = parts + (size_t)t * parts_ld + col;
+            float lo[4] = {0.f, 0.f, 0.f, 0.f}, hi[4] = {0.f, 0.f, 0.f, 0.f};
+            if (bias && bias_f32) {
+                Vec4<float>::load((const float*)bias + col, lo);
+                Vec4<float>::load((const float*)bias + col + 4, hi);
+            } else if (bias) {
+                Vec4<bf16_t>::load((const bf16_t*)bias + col, lo);
+                Vec4<bf16_t>::load((const bf16_t*)bias + col + 4, hi);
+            }
+            int q = 0;
+            for (; q + 4 <= num_parts; q += 4) add_slab_pairs<4>(src + q * part_stride, part_stride, lo, hi);
+            if (num_parts - q == 3) add_slab_pairs<3>(src + q * part_stride, part_stride, lo, hi);
+            else if (num_parts - q == 2) add_slab_pairs<2>(src + q * part_stride, part_stride, lo, hi);
+            else if (num_parts - q == 1) add_slab_pairs<1>(src + q * part_stride, part_stride, lo, hi);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { x[e] = lo[e]; x[4 + e] = hi[e]; }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) piece.e[e] = from_float<bf16_t>(x[e]).bits;
+        } else {
+            piece.u = *(const uint4*)(row + (size_t)head * head_dim + d0);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) { bf16_t b; b.bits = piece.e[e]; x[e] = to_float(b); }
+        }
         if (head >= q_heads + kv_heads) {                          // value head: [head_dim, page] inside the page
             bf16_t* dst = v_plane + page_base + (size_t)(head - q_heads - kv_heads) * page_size * head_dim + off;
             if (stores) {
@@ -391,17 +432,14 @@ void rope_cache_write_rows_kernel(bf16_t* __restrict__ qkv, int row_stride, int 
         if (rotate) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                bf16_t a, b;
-                a.bits = piece.e[2 * j];
-                b.bits = piece.e[2 * j + 1];
-                float x1 = to_float(a), x2 = to_float(b);
+                float x1 = x[2 * j], x2 = x[2 * j + 1];
                 const float2 cs = turn[d0 / 2 + j];
                 rope_turn(x1, x2, cs.x, cs.y);
                 piece.e[2 * j] = from_float<bf16_t>(x1).bits;
                 piece.e[2 * j + 1] = from_float<bf16_t>(x2).bits;
             }
-            *(uint4*)(row + (size_t)head * head_dim + d0) = piece.u;
         }
+        if (rotate || PARTS) *(uint4*)(row + (size_t)head * head_dim + d0) = piece.u;
         if (head >= q_heads && stores)
             *(uint4*)(k_plane + page_base + ((size_t)(head - q_heads) * page_size + off) * head_dim + d0) = piece.u;
     }
@@ -427,11 +465,14 @@ extern "C" int tl_rope_cache_write(void* qkv, int row_stride, int tokens, int q_
     const int heads = q_heads + kv_heads + (k_plane ? kv_heads : 0);
     // pairs as one access: rows and planes start on a multiple of two elements (eight bytes covers both dtypes)
     const int pair_aligned = row_stride % 2 == 0 && ((uintptr_t)qkv % 8) == 0 && ((uintptr_t)k_plane % 8) == 0;
-    if (act_dtype == TL_DT_BF16 && pairs && !parts && tokens >= 64 && head_dim % 8 == 0 && row_stride % 8 == 0 &&
+    const uintptr_t slab_bits = (uintptr_t)parts | (uintptr_t)bias;
+    if (act_dtype == TL_DT_BF16 && pairs && tokens >= 64 && (!parts || (slab_bits % 16 == 0 && parts_ld % 4 == 0 && part_stride % 4 == 0)) && head_dim % 8 == 0 && row_stride % 8 == 0 &&
         ((uintptr_t)qkv % 16) == 0 && ((uintptr_t)k_plane % 16) == 0 && (!inv_freq || ((uintptr_t)inv_freq % 16) == 0)) {
-        rope_cache_write_rows_kernel<<<dim3(tokens), dim3(256), 0, stream>>>((bf16_t*)qkv, row_stride, q_heads, kv_heads, head_dim, rot_heads,
-            (const int*)positions, (const float*)inv_freq, (const int*)token_req, (const int*)block_table, bt_stride,
-            (bf16_t*)k_plane, (bf16_t*)v_plane, page_size);
+        const int pieces = heads * (head_dim / 8);
+        auto kernel = parts ? rope_cache_write_rows_kernel<true> : rope_cache_write_rows_kernel<false>;
+        kernel<<<dim3(tokens), dim3(!parts ? 256 : pieces >= 1024 ? 1024 : (pieces + 63) / 64 * 64), 0, stream>>>((bf16_t*)qkv, row_stride, q_heads, kv_heads, head_dim,
+            rot_heads, (const int*)positions, (const float*)inv_freq, (const int*)token_req, (const int*)block_table, bt_stride, (bf16_t*)k_plane, (bf16_t*)v_plane,
+            page_size, (const float*)parts, num_parts, part_stride, parts_ld, bias, bias_f32);
         TL_CHECK_LAUNCH("rope_cache_write");
         return TL_OK;
     }
