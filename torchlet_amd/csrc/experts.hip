@@ -548,16 +548,65 @@ __global__ void combine_kernel(const T* __restrict__ y, const int* __restrict__ 
     }
 }
 
+// The same, 16 bytes of a row to a thread and four choices requested before the first is added (the sums keep their order): a number at a time every choice was a
+// trip to memory of its own (eight tokens, 8 choices 7.9 -> 4.6 us on average; over a pass of prompts of 4 x 1100 tokens, 6 choices and a shared expert, and
+// decoded tokens 33 -> 7.3).
+template <typename T>
+__global__ void __launch_bounds__(128)
+combine_pieces_kernel(const T* __restrict__ y, const int* __restrict__ pair_slot, const float* __restrict__ weights, T* __restrict__ out, const T* __restrict__ x,
+                      const int* __restrict__ offsets, int real, int top, int width, const T* __restrict__ addend) {
+    constexpr int VEC = 16 / sizeof(T);
+    struct __attribute__((aligned(16))) Piece { T v[VEC]; };
+    const int t = blockIdx.x, i = (blockIdx.y * 128 + threadIdx.x) * VEC;
+    if (i >= width) return;
+    const int own_from = x ? offsets[real] : 0x7fffffff;
+    const int* slots = pair_slot + (size_t)t * top;
+    const float* w = weights + (size_t)t * top;
+    auto row = [&](int slot) { return *(const Piece*)((slot >= own_from ? x + (size_t)t * width : y + (size_t)slot * width) + i); };
+    Piece last;
+    if (addend) last = *(const Piece*)(addend + (size_t)t * width + i);
+    float a[VEC] = {};
+    int j = 0;
+    for (; j + 4 <= top; j += 4) {
+        Piece p[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) p[u] = row(slots[j + u]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int v = 0; v < VEC; ++v) a[v] = fmaf(w[j + u], to_float(p[u].v[v]), a[v]);
+    }
+    for (; j < top; ++j) {
+        const Piece p = row(slots[j]);
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) a[v] = fmaf(w[j], to_float(p.v[v]), a[v]);
+    }
+    Piece o;
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) o.v[v] = from_float<T>(addend ? a[v] + to_float(last.v[v]) : a[v]);
+    *(Piece*)(out + (size_t)t * width + i) = o;
+}
+
+// Rows of whole 16-byte pieces on 16 bytes; others keep the kernel of single numbers.
+template <typename T>
+static void launch_combine(const T* y, const int* pair_slot, const float* weights, T* out, const T* x, const int* offsets, int real, int tokens, int top, int width,
+                           const T* addend, hipStream_t stream) {
+    constexpr int VEC = 16 / sizeof(T);
+    if (width % VEC == 0 && (((uintptr_t)y | (uintptr_t)out | (uintptr_t)x | (uintptr_t)addend) & 15) == 0 && width / VEC <= 128 * 65535)
+        combine_pieces_kernel<T><<<dim3(tokens, (width / VEC + 127) / 128), 128, 0, stream>>>(y, pair_slot, weights, out, x, offsets, real, top, width, addend);
+    else combine_kernel<T><<<tokens, 256, 0, stream>>>(y, pair_slot, weights, out, x, offsets, real, top, width, addend);
+}
+
 extern "C" int tl_combine(const void* y, const void* pair_slot, const void* weights, void* out, const void* x, const void* offsets, int real,
                           int tokens, int top, int width, const void* addend, int dtype, hipStream_t stream) {
     TL_REQUIRE(tokens >= 0 && top > 0 && width > 0 && real >= 0 && (!x || offsets), "combine: bad sizes");
     if (tokens == 0) return TL_OK;
     if (dtype == TL_DT_F32)
-        combine_kernel<float><<<tokens, 256, 0, stream>>>((const float*)y, (const int*)pair_slot, (const float*)weights, (float*)out, (const float*)x,
-                                                          (const int*)offsets, real, top, width, (const float*)addend);
+        launch_combine<float>((const float*)y, (const int*)pair_slot, (const float*)weights, (float*)out, (const float*)x, (const int*)offsets, real, tokens, top, width,
+                              (const float*)addend, stream);
     else if (dtype == TL_DT_BF16)
-        combine_kernel<bf16_t><<<tokens, 256, 0, stream>>>((const bf16_t*)y, (const int*)pair_slot, (const float*)weights, (bf16_t*)out, (const bf16_t*)x,
-                                                           (const int*)offsets, real, top, width, (const bf16_t*)addend);
+        launch_combine<bf16_t>((const bf16_t*)y, (const int*)pair_slot, (const float*)weights, (bf16_t*)out, (const bf16_t*)x, (const int*)offsets, real, tokens, top,
+                               width, (const bf16_t*)addend, stream);
     else TL_REQUIRE(false, "combine: unknown dtype %d", dtype);
     TL_CHECK_LAUNCH("combine");
     return TL_OK;
