@@ -29,9 +29,10 @@ __device__ __forceinline__ float log_sigmoid(float z) { return fminf(z, 0.f) - l
 // gates and the exponentials side by side, the running maximum one token after the other, as it is defined), every
 // lane runs the TB updates of its rows and leaves its rows' shares of each token's sums, and the shares are added in the
 // order of the rows.  A share is always that of four rows, whatever RPT and COLS are (a lane with RPT rows leaves RPT / 4
-// of them), so a token's result does not depend on how the step was cut or on what else is in it: a prompt is run with
+// of them), so a token's result does not depend on the tile's shape: a prompt is run with
 // few rows to a lane, because the time of a token is the chain of one lane's updates, a decode step with many rows and
-// wide tiles, because its time is the stream of the states.
+// wide tiles, because its time is the stream of the states.  Long portions leave this loop for the chunks at the end of this file, whose sums are
+// in another order: a portion equals single steps to the bit up to the length where that starts, and within rounding beyond it.
 #define MLSTM_TB 16
 #define MLSTM_SHARE 4
 
