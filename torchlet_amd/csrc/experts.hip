@@ -198,24 +198,31 @@ grouped_gemm_mfma_kernel(const bf16_t* __restrict__ a, int a_ld, int a_group, co
 }
 
 // ------------------------------------------------------------------ products over the experts' rows (bfloat16, K a multiple of 64)
-// Two kernels beside the one above, which keeps the heads' products and what these refuse.
+// Two kernels beside the one above, which keeps the heads' products of many rows and what these refuse.
 //
 // Few rows per expert (a decode step): what counts is the stream of the weights, and a stream needs work-groups enough to have tens of KB on their
 // way from every compute unit.  A work-group owns a strip of 16 weight rows of one expert and up to 16 of its slots; its waves deal K out
 // in steps of 64 (a lane fetches 32 bytes of its weight row and of its x row, a row's 128 bytes lie in one line; the order of k inside a step is
 // the same for both operands and so does not matter), FEW_DEPTH steps on their way at once, and their sums meet in shared memory in the order of
 // the waves.  Slots beyond the group's are copies of its last one and are not stored.
+// HEADS: the same for groups that all have the step's rows (a head's columns of x and out a_group and out_group numbers apart), with a gate per output number:
+// a decode step's products over heads, which one wave of the kernel above took whole (few work-groups, K one piece after the other).
 #define FEW_DEPTH 4
+struct HeadColumns {
+    int a_group, out_group, rows;
+    const bf16_t* gate;
+    int gate_ld;
+};
 
-template <int FEW_WAVES>
+template <int FEW_WAVES, bool HEADS>
 __global__ void __launch_bounds__(FEW_WAVES * 64)
 experts_few_rows_kernel(const bf16_t* __restrict__ a, int a_ld, const int* __restrict__ src, const bf16_t* __restrict__ w, bf16_t* __restrict__ out,
-                        int out_ld, const int* __restrict__ offsets, int groups, int N, int K, int act) {
+                        int out_ld, const int* __restrict__ offsets, int groups, int N, int K, int act, HeadColumns heads) {
     __shared__ __attribute__((aligned(16))) float red[FEW_WAVES][256];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, kg = lane >> 4;
     // this work-group's tile among the groups', found by a prefix sum over the lanes
-    int g = -1, m0 = 0, m_end = 0, first = 0;
-    for (int base = 0; base < groups && g < 0; base += TL_WAVE) {
+    int g = HEADS ? blockIdx.z : -1, m0 = HEADS ? blockIdx.y * 16 : 0, m_end = HEADS ? heads.rows : 0, first = 0;
+    for (int base = 0; !HEADS && base < groups && g < 0; base += TL_WAVE) {
         const int e = base + lane;
         const int from = e < groups ? offsets[e] : 0, to = e < groups ? offsets[e + 1] : 0;
         const int mine = (to - from + 15) / 16;
@@ -239,7 +246,7 @@ experts_few_rows_kernel(const bf16_t* __restrict__ a, int a_ld, const int* __res
     const int n0 = blockIdx.x * 16;
     const bf16_t* wrow = w + ((size_t)g * N + min(n0 + li, N - 1)) * K + 16 * kg;
     const int mine = min(m0 + li, m_end - 1);
-    const bf16_t* xrow = a + (size_t)(src ? src[mine] : mine) * a_ld + 16 * kg;
+    const bf16_t* xrow = a + (size_t)(!HEADS && src ? src[mine] : mine) * a_ld + (HEADS ? (size_t)g * heads.a_group : 0) + 16 * kg;
     f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
     const int steps = K / 64;
     for (int s0 = wave; s0 < steps; s0 += FEW_WAVES * FEW_DEPTH) {
@@ -269,8 +276,13 @@ experts_few_rows_kernel(const bf16_t* __restrict__ a, int a_ld, const int* __res
     // sum[v] = out[slot m0 + li][column n0 + 4 kg + v]
     const int m = m0 + li, n = n0 + 4 * kg, base_act = act & ~ACT_PAIRS;
     if (m >= m_end) return;
-    bf16_t* orow = out + (size_t)m * out_ld;
-    if (act & ACT_PAIRS) {
+    bf16_t* orow = out + (size_t)m * out_ld + (HEADS ? (size_t)g * heads.out_group : 0);
+    if (HEADS) {
+        const bf16_t* grow = heads.gate ? heads.gate + (size_t)m * heads.gate_ld + (size_t)g * heads.out_group : nullptr;
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            if (n + v < N) orow[n + v] = from_float<bf16_t>(grow ? sum[v] * sigmoid(to_float(grow[n + v])) : sum[v]);
+    } else if (act & ACT_PAIRS) {
 #pragma unroll
         for (int v = 0; v < 4; v += 2)
             if (n + v + 1 < N) orow[(n + v) / 2] = from_float<bf16_t>(activate(sum[v], base_act) * sum[v + 1]);
@@ -299,7 +311,7 @@ struct ExpertsCall {
 template <int WAVES>
 static int launch_experts_few(const ExpertsCall& c, hipStream_t stream) {
     const dim3 grid((c.N + 15) / 16, c.rows / 16 + (c.groups < c.rows ? c.groups : c.rows));
-    experts_few_rows_kernel<WAVES><<<grid, WAVES * 64, 0, stream>>>(c.a, c.a_ld, c.src, c.w, c.out, c.out_ld, c.offsets, c.groups, c.N, c.K, c.act);
+    experts_few_rows_kernel<WAVES, false><<<grid, WAVES * 64, 0, stream>>>(c.a, c.a_ld, c.src, c.w, c.out, c.out_ld, c.offsets, c.groups, c.N, c.K, c.act, HeadColumns{});
     return TL_OK;
 }
 
@@ -386,6 +398,13 @@ extern "C" int tl_experts_variant(const void* a, int a_ld, const void* src, cons
     return launch_experts(which, c, stream);
 }
 
+// Whether products over heads go to the few-rows kernel: up to eight of its work-groups to a compute unit, 64 rows at most (beyond, every strip of 16 rows reads the
+// weights again).  Measured against the kernel without shared memory (us; heads x N x K): 32 x 512 x 128, 1 row 4.2 / 6.4, 32 rows 8.1 / 8.8, 48 rows (twelve to a
+// unit) 10.9 / 8.9; 32 x 128 x 512, 1 row 3.8 / 11.1, 64 rows 9.7 / 15.4; 16 x 512 x 128, 64 rows 8.1 / 8.9; 8 x 192 x 64, 1 row 2.4 / 4.5.
+static bool heads_few_rows(int rows, int groups, int N, int K) {
+    return K % 64 == 0 && rows <= 64 && groups <= 65535 && (long)((N + 15) / 16) * ((rows + 15) / 16) * groups <= 8L * experts_units;
+}
+
 extern "C" int tl_grouped_gemm(const void* a, int a_ld, int a_group, const void* src, const void* w, void* out, int out_ld, int out_group,
                                const void* offsets, int groups, int rows, int N, int K, int act, const void* gate, int gate_ld, int dtype, int general,
                                hipStream_t stream) {
@@ -400,6 +419,14 @@ extern "C" int tl_grouped_gemm(const void* a, int a_ld, int a_group, const void*
                          ((uintptr_t)out % 8) == 0;
     const ExpertsCall experts{(const bf16_t*)a, a_ld, (const int*)src, (const bf16_t*)w, (bf16_t*)out, out_ld, (const int*)offsets, groups, rows, N, K, act};
     if (dtype == TL_DT_BF16 && offsets && !general && experts_fit(experts)) return launch_experts(pick_experts(experts), experts, stream);
+    if (dtype == TL_DT_BF16 && aligned && !general && !offsets && act == ACT_NONE && heads_few_rows(rows, groups, N, K)) {
+        const HeadColumns heads{a_group, out_group, rows, (const bf16_t*)gate, gate_ld};
+        const dim3 fgrid((N + 15) / 16, (rows + 15) / 16, groups);
+        auto kernel = K >= 512 ? experts_few_rows_kernel<4, true> : experts_few_rows_kernel<2, true>;      // (two steps of 64 to a wave, where there are so many)
+        kernel<<<fgrid, K >= 512 ? 256 : 128, 0, stream>>>((const bf16_t*)a, a_ld, nullptr, (const bf16_t*)w, (bf16_t*)out, out_ld, nullptr, groups, N, K, act, heads);
+        TL_CHECK_LAUNCH("heads_few_rows");
+        return TL_OK;
+    }
     if (dtype == TL_DT_BF16 && aligned && !general) {
         dim3 mgrid(offsets ? (rows + GM_BM - 1) / GM_BM + groups : (rows + GM_BM - 1) / GM_BM, (N + GM_BN - 1) / GM_BN, offsets ? 1 : groups);
         grouped_gemm_mfma_kernel<<<mgrid, block, 0, stream>>>((const bf16_t*)a, a_ld, a_group, (const int*)src, (const bf16_t*)w, (bf16_t*)out, out_ld,
