@@ -1,0 +1,63 @@
+"""The chunked recurrences where the host knows a step's portions only as a bound, and beside requests of few tokens."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _pays(monkeypatch):
+    """Chunks wherever the sizes allow them, whatever the estimates say."""
+    from torchlet_amd.kernels import ops
+    real = ops._chunk_scratch
+
+    class Pays:
+        @staticmethod
+        def tl_chunks_pay(*_):
+            return 1
+    monkeypatch.setattr(ops, "_chunk_scratch", lambda lib, *a, **k: real(Pays, *a, **k))
+
+
+class _Step:
+    """The matrix memory or fixed decays over random numbers, requests of `lens` tokens in the first rows of a step of `rows`."""
+
+    def __init__(self, memory, lens, rows=None, H=2, dim=64, vdim=128):
+        self.memory, self.lens, self.H, self.dim, self.vdim = memory, lens, H, dim, vdim
+        g = torch.Generator().manual_seed(sum(lens))
+        T = rows or sum(lens)
+        self.qkv = torch.randn(T, 2 * H * dim + H * vdim, generator=g).cuda()
+        self.gates = (torch.randn(T, 2 * H, generator=g) + 1.0).cuda()
+        self.decay = torch.tensor([0.97, 0.999])[:H].cuda()
+        self.start = torch.randn(len(lens), H, dim * vdim + (dim + 1 if memory else 0), generator=g).cuda()
+        self.slots = torch.arange(len(lens), dtype=torch.int32, device="cuda")
+        self.indptr = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device="cuda")
+
+    def run(self, qkv=None, gates=None, start=None, slots=None, indptr=None, **more):
+        from torchlet_amd.kernels import ops
+        qkv, gates = (self.qkv if qkv is None else qkv), (self.gates if gates is None else gates)
+        state = (self.start if start is None else start).clone()
+        slots, indptr = (self.slots if slots is None else slots), (self.indptr if indptr is None else indptr)
+        out = torch.full((qkv.shape[0], self.H * self.vdim), float("nan"), device="cuda")
+        H, dim, vdim = self.H, self.dim, self.vdim
+        if self.memory:
+            ops.mlstm_scan(qkv, H * dim, 2 * H * dim, gates, state, slots, indptr, out, H, dim, vdim, 9.0, dim ** -0.5, 1e-6, **more)
+        else:
+            ops.decay_scan(qkv, self.decay, state.view(state.shape[0], -1), slots, indptr, out, H, dim, vdim, **more)
+        return out, state
+
+    def alone(self, r):
+        """Request r's tokens and nothing else in the step, and its own length given."""
+        rows = slice(int(self.indptr[r]), int(self.indptr[r + 1]))
+        n = self.lens[r]
+        return self.run(self.qkv[rows].contiguous(), self.gates[rows].contiguous(), self.start[r: r + 1], self.slots[:1],
+                        torch.tensor([0, n], dtype=torch.int32, device="cuda"), max_new_tokens=n)
+
+
+@pytest.mark.parametrize("memory", [True, False])
+@pytest.mark.parametrize("lens, rows, most", [([20], 20, 300), ([20], 400, None), ([31], 31, 32), ([40], 400, None)])
+def test_a_request_shorter_than_the_bound_is_not_left_out(monkeypatch, memory, lens, rows, most):
+    _pays(monkeypatch)
+    step = _Step(memory, lens, rows)
+    out, state = step.run(max_new_tokens=most)
+    want, left = step.alone(0)
+    assert torch.equal(out[: lens[0]], want) and torch.equal(state, left)
+    assert bool(torch.isnan(out[lens[0]:]).all())

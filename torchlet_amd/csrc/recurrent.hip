@@ -1640,7 +1640,7 @@ static bool chunks_fit(const void* qkv, int ld, int q_off, int k_off, int v_off,
 // [tokens, 2 * heads]; state float [slots, heads, dim * vdim + dim + 1] with slot_stride floats between slots;
 // out float [tokens, heads * vdim]; before: scratch of requests * heads * (dim + 1) floats.  Requests whose req_indptr range
 // is empty are left alone.  Requests of at least `least` tokens go through the chunks where the sizes allow it; longest: no fewer tokens than any request of
-// the step brings; scratch (null: the token loop alone): the chunks' states and, from scratch_floats on, the tokens' factors (4 * tokens * heads floats).
+// the step brings, and more in some calls, so the token loop always follows; scratch (null: the token loop alone): the chunks' states and, from scratch_floats on, the tokens' factors (4 * tokens * heads floats).
 extern "C" int tl_mlstm_scan(const void* qkv, int ld, int k_off, int v_off, const void* gates, void* state, long slot_stride,
                              const void* slots, const void* before, const void* req_indptr, void* out, int requests, int heads, int dim, int vdim,
                              float cap, float qscale, float denom_eps, int longest, int tokens, int least, void* scratch, long scratch_floats, int dtype,
@@ -1660,7 +1660,7 @@ extern "C" int tl_mlstm_scan(const void* qkv, int ld, int k_off, int v_off, cons
                           (size_t)slot_stride, (const int*)slots, (const int*)req_indptr, (float*)out, nullptr, nullptr, nullptr, requests, least, 0, 0};
         const int rc = dtype == TL_DT_F32 ? launch_chunks<float, 3>(a, tokens, longest, (float*)scratch, (size_t)scratch_floats, stream)
                                           : launch_chunks<bf16_t, 3>(a, tokens, longest, (float*)scratch, (size_t)scratch_floats, stream);
-        if (rc != TL_OK || requests == 1) return rc;
+        if (rc != TL_OK) return rc;
     }
     return mlstm_token_loop(qkv, ld, k_off, v_off, gates, state, slot_stride, slots, before, req_indptr, out, requests, heads, dim, vdim, cap, qscale, denom_eps,
                             chunks ? min(longest, least - 1) : longest, chunks ? least : INT_MAX, dtype, stream);
@@ -1682,7 +1682,7 @@ extern "C" int tl_decay_scan(const void* qkv, const void* decay, void* state, lo
         const int rc = launch_chunks<float, 0>(ChunkArgs{qkv, 2 * heads * dim + heads * vdim, 0, heads * dim, 2 * heads * dim, heads, 1, dim, vdim, nullptr, 0, 0, 0, 0,
             (const float*)decay, 1.f, 0.f, (float*)state, (size_t)slot_stride, (const int*)slots, (const int*)req_indptr, (float*)out, nullptr, nullptr, nullptr,
             requests, least, 0, 0}, tokens, longest, (float*)scratch, (size_t)scratch_floats, stream);
-        if (rc != TL_OK || requests == 1) return rc;
+        if (rc != TL_OK) return rc;
     }
     launch_delta_scan<0>(qkv, nullptr, decay, state, slot_stride, slots, req_indptr, out, requests, heads, heads, dim, vdim, chunks ? min(longest, least - 1) : longest,
                          chunks ? least : INT_MAX, stream);
