@@ -61,3 +61,30 @@ def test_a_request_shorter_than_the_bound_is_not_left_out(monkeypatch, memory, l
     want, left = step.alone(0)
     assert torch.equal(out[: lens[0]], want) and torch.equal(state, left)
     assert bool(torch.isnan(out[lens[0]:]).all())
+
+
+@pytest.mark.parametrize("memory", [True, False])
+@pytest.mark.parametrize("where", ["query", "key", "value", "input gate"])
+@pytest.mark.parametrize("token", [0, 5, 40, 63, 64, 100])
+def test_infinities_and_nans_do_not_reach_the_tokens_before_them(monkeypatch, memory, where, token):
+    from torchlet_amd.kernels import ops
+    if where == "input gate" and not memory:
+        pytest.skip("fixed decays have no gates")
+    _pays(monkeypatch)
+    step = _Step(memory, [130])
+    clean, _ = step.run(max_new_tokens=130)
+    H, dim = step.H, step.dim
+    for bad in (float("inf"), float("nan")):
+        qkv, gates = step.qkv.clone(), step.gates.clone()
+        if where == "input gate":
+            gates[token, 1] = float("nan")
+        else:
+            qkv[token, {"query": 3, "key": H * dim + 3, "value": 2 * H * dim + 3}[where]] = bad
+        got, _ = step.run(qkv, gates, max_new_tokens=130)
+        # (a chunk with such a value adds its tokens up in another order: 130 terms of like size, each rounding at most 2^-24 of a partial sum)
+        assert float((got[:token] - clean[:token]).norm()) <= 130 * 2.0 ** -24 * float(clean[:token].norm()), bad
+        assert not bool(torch.isfinite(got[token]).all()), bad
+        monkeypatch.setattr(ops, "CHUNKED_FROM", 1 << 30)
+        loop, _ = step.run(qkv, gates, max_new_tokens=130)
+        monkeypatch.setattr(ops, "CHUNKED_FROM", 32)
+        assert torch.equal(torch.isfinite(got), torch.isfinite(loop)), bad

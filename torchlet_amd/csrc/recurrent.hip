@@ -1393,6 +1393,7 @@ chunk_outputs_kernel(ChunkArgs a) {
     float* sk = sq + CK_T * CK_LD;                     // [64][CK_LD] keys of a slab
     float* ss = sk + CK_T * CK_LD;                     // [CK_V][CK_LD] the state's columns of a slab; after the slabs [64][CK_LV] values
     float* sg = ss + CK_V * CK_LD;                     // [64] g, [64] b, [64] G (products up to the token), [64] 1 / denominator, [64] keys' sums of a slab
+    int* odd = (int*)(sg + 5 * CK_T);                  // whether some value of the chunk is an infinity or a NaN
     const int tid = threadIdx.x, wave = tid / TL_WAVE, lane = tid % TL_WAVE, li = lane & 31, half = lane >> 5;
     int chunk0 = 0;
     const int chunk = blockIdx.x, req = ck_find(a, chunk, chunk0);
@@ -1401,6 +1402,7 @@ chunk_outputs_kernel(ChunkArgs a) {
     const int tok0 = a.req_indptr[req] + a.seg0 + (chunk - chunk0) * CK_T;
     const int nt = min(min(CK_T, a.req_indptr[req + 1] - tok0), a.seg_len - (chunk - chunk0) * CK_T);
     float m_mine = 0.f;                                // the running maximum after token tid / 4
+    if (tid == 0) *odd = 0;
     if (wave == 0) {
         float b = 0.f, g = 1.f;
         if (lane < nt) {
@@ -1498,13 +1500,16 @@ chunk_outputs_kernel(ChunkArgs a) {
 #pragma unroll
     for (int j = 0; j < CK_T * CK_V / 4 / 256; ++j) {
         const int idx = tid + j * 256, t = idx / (CK_V / 4), c = (idx % (CK_V / 4)) * 4;
-        *(float4*)(ss + t * CK_LV + c) = t < nt && v0 + c < a.vdim ? ck_load4<T>(vsrc + (size_t)t * a.ld + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+        const float4 x = t < nt && v0 + c < a.vdim ? ck_load4<T>(vsrc + (size_t)t * a.ld + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+        *(float4*)(ss + t * CK_LV + c) = x;
+        if (fmaf(x.x, 0.f, fmaf(x.y, 0.f, fmaf(x.z, 0.f, x.w * 0.f))) != 0.f) *odd = 1;      // an infinity or a NaN
     }
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        float* w = sq + (32 * ti + 8 * (i / 4) + 4 * half + i % 4) * CK_LD + 32 * tj + li;
-        if (tj <= ti) *w *= sc[i];
+    for (int i = 0; i < 16; ++i) {                     // (a score of a later token, which may be anything, is put aside and not multiplied by zero)
+        const int row = 32 * ti + 8 * (i / 4) + 4 * half + i % 4, col = 32 * tj + li;
+        float* w = sq + row * CK_LD + col;
+        if (tj <= ti && col <= row) *w *= sc[i];
     }
     ck_f32x16 o[2], o1;                                // the chunk's own share, apart from the state's: of its first 32 tokens, of its last
 #pragma unroll
@@ -1523,27 +1528,41 @@ chunk_outputs_kernel(ChunkArgs a) {
         __syncthreads();
     }
     if (!cols) return;
-#pragma unroll 4
-    for (int t = 0; t < CK_T; t += 8) {
-        const float4 w1 = *(const float4*)(sq + (32 + li) * CK_LD + t + 4 * half);
-        const float wa[4] = {w1.x, w1.y, w1.z, w1.w};
-        float x[4];
+    if (*odd) {
+        // some value is an infinity or a NaN: the matrix products would carry it, times a weight of zero, to the tokens before it as well
+        for (int t = 0; t < nt; ++t) {
+            const float x = ss[t * CK_LV + wave * 32 + li];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) x[e] = ss[(t + 4 * half + e) * CK_LV + wave * 32 + li];
-        if (t < 32) {                                  // (the first 32 tokens see none of the last 32)
-            const float4 w0 = *(const float4*)(sq + li * CK_LD + t + 4 * half);
-            const float wb[4] = {w0.x, w0.y, w0.z, w0.w};
+            for (int n = 0; n < 2; ++n)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                o[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(wb[e], x[e], o[0], 0, 0, 0);
-                o[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(wa[e], x[e], o[1], 0, 0, 0);
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o1 = __builtin_amdgcn_mfma_f32_32x32x2f32(wa[e], x[e], o1, 0, 0, 0);
+                for (int i = 0; i < 16; ++i) {
+                    const int row = 32 * n + 8 * (i / 4) + 4 * half + i % 4;
+                    if (row >= t) o[n][i] = fmaf(sq[row * CK_LD + t], x, o[n][i]);
+                }
         }
+    } else {
+#pragma unroll 4
+        for (int t = 0; t < CK_T; t += 8) {
+            const float4 w1 = *(const float4*)(sq + (32 + li) * CK_LD + t + 4 * half);
+            const float wa[4] = {w1.x, w1.y, w1.z, w1.w};
+            float x[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = ss[(t + 4 * half + e) * CK_LV + wave * 32 + li];
+            if (t < 32) {                                  // (the first 32 tokens see none of the last 32)
+                const float4 w0 = *(const float4*)(sq + li * CK_LD + t + 4 * half);
+                const float wb[4] = {w0.x, w0.y, w0.z, w0.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    o[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(wb[e], x[e], o[0], 0, 0, 0);
+                    o[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(wa[e], x[e], o[1], 0, 0, 0);
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o1 = __builtin_amdgcn_mfma_f32_32x32x2f32(wa[e], x[e], o1, 0, 0, 0);
+            }
+        }
+        o[1] += o1;
     }
-    o[1] += o1;
     const int v = v0 + wave * 32 + li;
 #pragma unroll
     for (int n = 0; n < 2; ++n)
@@ -1575,7 +1594,7 @@ static int launch_chunks(ChunkArgs a, int tokens, int longest, float* scratch, s
     a.states = scratch;
     a.sums = scratch + (size_t)chunks * a.heads * a.vdim * a.dim;
     a.decays = a.sums + (MODE == 3 ? (size_t)chunks * a.heads * a.dim : 0);
-    constexpr size_t smem = sizeof(float) * (2 * CK_T * CK_LD + CK_V * CK_LD + 5 * CK_T);
+    constexpr size_t smem = sizeof(float) * (2 * CK_T * CK_LD + CK_V * CK_LD + 5 * CK_T + 4);
     auto outputs = chunk_outputs_kernel<T, MODE>;
     static hipError_t allowed = hipFuncSetAttribute((const void*)outputs, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     if (allowed != hipSuccess) { tl_set_error("chunked scan: cannot get %zu bytes of shared memory: %s", smem, hipGetErrorString(allowed)); return TL_ERR_HIP; }
