@@ -88,3 +88,31 @@ def test_infinities_and_nans_do_not_reach_the_tokens_before_them(monkeypatch, me
         loop, _ = step.run(qkv, gates, max_new_tokens=130)
         monkeypatch.setattr(ops, "CHUNKED_FROM", 32)
         assert torch.equal(torch.isfinite(got), torch.isfinite(loop)), bad
+
+
+def _portions(lens):
+    from torchlet_amd.kernels import ops
+    return ops.Portions.of(lens, ops.CHUNKED_FROM)
+
+
+@pytest.mark.parametrize("memory", [True, False])
+@pytest.mark.parametrize("lens", [[65, 0], [0, 0, 130, 0], [4] * 40, [1] * 9 + [65] + [31], [200, 33, 1, 64], [5, 1]])
+@pytest.mark.parametrize("exact", [True, False])
+@pytest.mark.parametrize("passes", [True, False])
+def test_every_request_moves_as_it_does_alone(monkeypatch, memory, lens, exact, passes):
+    """With the lengths given and without, empty requests and decoded tokens beside long portions, in one pass over the chunks and in several."""
+    from torchlet_amd.kernels import ops
+    _pays(monkeypatch)
+    step = _Step(memory, lens)
+    want = {r: step.alone(r) for r, n in enumerate(lens) if n}
+    if passes:                                         # (room for one chunk of every portion)
+        per_chunk = step.H * (step.dim * step.vdim + (step.dim if memory else 0) + 1)
+        monkeypatch.setattr(ops, "CHUNK_SCRATCH", per_chunk * max(1, sum(n >= 32 for n in lens) if exact else len(lens)))
+    out, state = step.run(**({"portions": _portions(lens), "max_new_tokens": max(lens)} if exact else {}))
+    at = 0
+    for r, n in enumerate(lens):
+        if n:
+            assert torch.equal(out[at: at + n], want[r][0]) and torch.equal(state[r], want[r][1][0]), r
+        else:
+            assert torch.equal(state[r], step.start[r]), r
+        at += n

@@ -1576,21 +1576,21 @@ chunk_outputs_kernel(ChunkArgs a) {
         }
 }
 
-// Tokens of a request that one pass over the chunks takes, so that the chunks' states fit the scratch.
-static int chunk_segment(size_t scratch_floats, size_t per_chunk, int requests, int tokens, int longest) {
-    const long fit = (long)(scratch_floats / per_chunk);                     // chunks
-    long len = (longest + CK_T - 1) / CK_T;
-    const long all = tokens / CK_T + requests;                               // most chunks of the step
-    if (all > fit) len = fit / requests < len ? fit / requests : len;
-    return (int)(len * CK_T);
-}
+// How the long portions of a step go through the chunks: `segment` tokens of every portion a pass, `grid` chunks of them all in a pass at most, whose
+// states and sums stand in `scratch` (`floats` numbers).
+struct ChunkPlan {
+    int segment, grid;
+    float* scratch;
+    long floats;
+};
 
 template <typename T, int MODE>
-static int launch_chunks(ChunkArgs a, int tokens, int longest, float* scratch, size_t scratch_floats, hipStream_t stream) {
+static int launch_chunks(ChunkArgs a, const ChunkPlan& p, int longest, hipStream_t stream) {
     const size_t per_chunk = (size_t)a.heads * ((size_t)a.vdim * a.dim + (MODE == 3 ? a.dim : 0) + 1);
-    a.seg_len = chunk_segment(scratch_floats, per_chunk, a.requests, tokens, longest);
-    TL_REQUIRE(a.seg_len > 0, "chunked scan: scratch of %zu numbers does not hold a chunk of every request", scratch_floats);
-    const long chunks = (long)a.seg_len / CK_T * a.requests < (long)tokens / CK_T + a.requests ? (long)a.seg_len / CK_T * a.requests : (long)tokens / CK_T + a.requests;
+    TL_REQUIRE(p.segment > 0 && p.segment % CK_T == 0 && p.grid > 0 && p.floats >= (long)(p.grid * per_chunk), "chunked scan: scratch of %ld numbers does not hold %d chunks", p.floats, p.grid);
+    const int chunks = p.grid;
+    float* scratch = p.scratch;
+    a.seg_len = p.segment;
     a.states = scratch;
     a.sums = scratch + (size_t)chunks * a.heads * a.vdim * a.dim;
     a.decays = a.sums + (MODE == 3 ? (size_t)chunks * a.heads * a.dim : 0);
@@ -1658,12 +1658,14 @@ static bool chunks_fit(const void* qkv, int ld, int q_off, int k_off, int v_off,
 // qkv [tokens, ld]: queries at column 0 (heads * dim), keys at k_off, values at v_off (heads * vdim); gates float
 // [tokens, 2 * heads]; state float [slots, heads, dim * vdim + dim + 1] with slot_stride floats between slots;
 // out float [tokens, heads * vdim]; before: scratch of requests * heads * (dim + 1) floats.  Requests whose req_indptr range
-// is empty are left alone.  Requests of at least `least` tokens go through the chunks where the sizes allow it; longest: no fewer tokens than any request of
-// the step brings, and more in some calls, so the token loop always follows; scratch (null: the token loop alone): the chunks' states and, from scratch_floats on, the tokens' factors (4 * tokens * heads floats).
+// is empty are left alone.  longest: no fewer tokens than any request of the step brings.  With scratch (null: the token loop alone) requests of at least `least`
+// tokens go through the chunks where the rows allow it: `segment` tokens of each a pass, chunk_grid chunks a pass at most; the chunks' states come first in
+// scratch and from scratch_floats on the tokens' factors (4 * tokens * heads floats).  The token loop then takes the others (rest: how many there are, or more if
+// the caller cannot tell; 0 only if there are none), of about rest_longest tokens at most, which sizes its batches.
 extern "C" int tl_mlstm_scan(const void* qkv, int ld, int k_off, int v_off, const void* gates, void* state, long slot_stride,
                              const void* slots, const void* before, const void* req_indptr, void* out, int requests, int heads, int dim, int vdim,
-                             float cap, float qscale, float denom_eps, int longest, int tokens, int least, void* scratch, long scratch_floats, int dtype,
-                             hipStream_t stream) {
+                             float cap, float qscale, float denom_eps, int longest, int segment, int chunk_grid, int least, int rest, int rest_longest,
+                             void* scratch, long scratch_floats, int dtype, hipStream_t stream) {
     TL_REQUIRE(requests >= 0 && heads > 0 && dim > 0 && vdim > 0 && ld > 0, "mlstm_scan: bad sizes");
     TL_REQUIRE(dim <= 1024, "mlstm_scan: built for up to 1024 query/key dimensions per head, got %d", dim);
     TL_REQUIRE(slot_stride >= (long)heads * ((long)dim * vdim + dim + 1), "mlstm_scan: the state rows are too short");
@@ -1677,20 +1679,20 @@ extern "C" int tl_mlstm_scan(const void* qkv, int ld, int k_off, int v_off, cons
         TL_CHECK_LAUNCH("mlstm_gates");
         const ChunkArgs a{qkv, ld, 0, k_off, v_off, heads, 1, dim, vdim, (const float*)factors, 4 * heads, 4, 1, 0, nullptr, qscale, denom_eps, (float*)state,
                           (size_t)slot_stride, (const int*)slots, (const int*)req_indptr, (float*)out, nullptr, nullptr, nullptr, requests, least, 0, 0};
-        const int rc = dtype == TL_DT_F32 ? launch_chunks<float, 3>(a, tokens, longest, (float*)scratch, (size_t)scratch_floats, stream)
-                                          : launch_chunks<bf16_t, 3>(a, tokens, longest, (float*)scratch, (size_t)scratch_floats, stream);
-        if (rc != TL_OK) return rc;
+        const ChunkPlan plan{segment, chunk_grid, (float*)scratch, scratch_floats};
+        const int rc = dtype == TL_DT_F32 ? launch_chunks<float, 3>(a, plan, longest, stream) : launch_chunks<bf16_t, 3>(a, plan, longest, stream);
+        if (rc != TL_OK || rest == 0) return rc;
     }
     return mlstm_token_loop(qkv, ld, k_off, v_off, gates, state, slot_stride, slots, before, req_indptr, out, requests, heads, dim, vdim, cap, qscale, denom_eps,
-                            chunks ? min(longest, least - 1) : longest, chunks ? least : INT_MAX, dtype, stream);
+                            chunks ? rest_longest : longest, chunks ? least : INT_MAX, dtype, stream);
 }
 
 // ------------------------------------------------------------------ decayed linear attention
 // Per head S <- decay[head] S + k v^T, o = S^T q over the step's tokens, request by request from the state its slot holds: qkv float
 // [T, 2 * heads * dim + heads * vdim] (queries, keys, values, head by head), state as the delta rule's, out float [T, heads * vdim].
 extern "C" int tl_decay_scan(const void* qkv, const void* decay, void* state, long slot_stride, const void* slots, const void* req_indptr,
-                             void* out, int requests, int heads, int dim, int vdim, int longest, int tokens, int least,
-                             void* scratch, long scratch_floats, hipStream_t stream) {
+                             void* out, int requests, int heads, int dim, int vdim, int longest, int segment, int chunk_grid, int least, int rest,
+                             int rest_longest, void* scratch, long scratch_floats, hipStream_t stream) {
     TL_REQUIRE(requests >= 0 && heads > 0 && dim > 0 && vdim > 0 && decay, "decay_scan: bad sizes");
     TL_REQUIRE(dim <= DELTA_L * 16, "decay_scan: built for up to %d query/key dimensions per head, got %d", DELTA_L * 16, dim);
     TL_REQUIRE(slot_stride >= (long)heads * dim * vdim, "decay_scan: the state rows are too short");
@@ -1700,10 +1702,10 @@ extern "C" int tl_decay_scan(const void* qkv, const void* decay, void* state, lo
     if (chunks) {
         const int rc = launch_chunks<float, 0>(ChunkArgs{qkv, 2 * heads * dim + heads * vdim, 0, heads * dim, 2 * heads * dim, heads, 1, dim, vdim, nullptr, 0, 0, 0, 0,
             (const float*)decay, 1.f, 0.f, (float*)state, (size_t)slot_stride, (const int*)slots, (const int*)req_indptr, (float*)out, nullptr, nullptr, nullptr,
-            requests, least, 0, 0}, tokens, longest, (float*)scratch, (size_t)scratch_floats, stream);
-        if (rc != TL_OK) return rc;
+            requests, least, 0, 0}, ChunkPlan{segment, chunk_grid, (float*)scratch, scratch_floats}, longest, stream);
+        if (rc != TL_OK || rest == 0) return rc;
     }
-    launch_delta_scan<0>(qkv, nullptr, decay, state, slot_stride, slots, req_indptr, out, requests, heads, heads, dim, vdim, chunks ? min(longest, least - 1) : longest,
+    launch_delta_scan<0>(qkv, nullptr, decay, state, slot_stride, slots, req_indptr, out, requests, heads, heads, dim, vdim, chunks ? rest_longest : longest,
                          chunks ? least : INT_MAX, stream);
     TL_CHECK_LAUNCH("decay_scan");
     return TL_OK;

@@ -16,6 +16,8 @@ from dataclasses import dataclass, field
 import numpy as np
 import torch
 
+from ..kernels.ops import Portions
+
 
 @dataclass
 class StepEntry:
@@ -141,6 +143,13 @@ class StepContext:
                                     (v["lr"], v["l0"], len(lr), v["lt"], len(long_tokens), shortest))
         return t
 
+    def portions(self, least: int) -> Portions:
+        """How many requests bring ``least`` tokens or more, and how many tokens these and the others."""
+        key = ("lengths", least)
+        if key not in self._tiles:
+            self._tiles[key] = Portions.of(self._host_new_lens.tolist(), least)
+        return self._tiles[key]
+
     def long_portions(self, least: int, window: int = 0, tile: int = 128):
         """The requests that bring ``least`` tokens or more, and where the rows of the positions that each reads lie side by side (from the first one inside
         the ``window`` on, 0: all; starts and counts rounded to multiples of 64): ``(portion_req [n], portion_at [n + 1], portion_low [n], n, rows,
@@ -215,6 +224,9 @@ class StaticDecodeContext:
         o, n = self._offsets[key]
         self._np[o: o + n] = 0
         self._np[o: o + len(values)] = values
+
+    def portions(self, least: int) -> Portions:
+        return Portions(0, 0, 0, 0, self.width, self.width, 1)
 
     def tiles(self, tq: int):
         return self._tile                 # one token per request: a tile per request whatever its height

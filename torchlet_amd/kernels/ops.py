@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import ctypes
 from ctypes import c_float, c_int, c_void_p
+from typing import NamedTuple
 
 import torch
 
@@ -960,25 +961,75 @@ CHUNKED_FROM = 32
 CHUNK_SCRATCH = 1 << 26
 
 
-def _chunk_scratch(lib, memory: bool, tokens: int, requests: int, longest: int, heads: int, dim: int, vdim: int, more: int, device):
-    """Scratch for the chunks of a step's long portions (``None``: the token loop takes them all), and how many of its numbers are the chunks'."""
-    if longest < CHUNKED_FROM or not lib.tl_chunks_pay(c_int(1 if memory else 0), c_int(tokens), c_int(requests), c_int(longest), c_int(heads), c_int(dim), c_int(vdim)):
-        return None, 0
+class Portions(NamedTuple):
+    """What the host knows of a step's lengths: the requests of `least` tokens or more (how many, their tokens, the chunks of 64 that these make, the most
+    tokens of one), and the others."""
+    count: int
+    tokens: int
+    chunks: int
+    longest: int
+    rest: int
+    rest_tokens: int
+    rest_longest: int
+
+    @classmethod
+    def of(cls, lengths, least: int) -> "Portions":
+        long, rest = [n for n in lengths if n >= least], [n for n in lengths if 0 < n < least]
+        return cls(len(long), sum(long), sum(-(-n // 64) for n in long), max(long, default=0), len(rest), sum(rest), max(rest, default=0))
+
+    @classmethod
+    def bound(cls, tokens: int, requests: int, longest: int | None, least: int) -> "Portions":
+        """For callers that know their rows and requests alone, and maybe a bound on a request's tokens: no fewer of anything than there are."""
+        longest = tokens if longest is None else longest
+        if longest < least:
+            return cls(0, 0, 0, 0, requests, tokens, longest)
+        count = min(requests, tokens // least)
+        return cls(count, tokens, tokens // 64 + count, longest, requests, 0, least - 1)
+
+
+class _Chunks(NamedTuple):
+    """How a step's long portions go through the chunks: `segment` tokens of every portion a pass, `grid` chunks of all portions at most, their scratch and
+    the numbers of it that are the chunks'."""
+    segment: int
+    grid: int
+    scratch: torch.Tensor
+    floats: int
+
+
+def _chunk_scratch(lib, memory: bool, requests: int, heads: int, dim: int, vdim: int, more: int, device, portions: Portions) -> _Chunks | None:
+    """``None``: the token loop takes all of the step."""
+    if portions.count == 0 or portions.longest < CHUNKED_FROM:
+        return None
     per_chunk = heads * (dim * vdim + (dim if memory else 0) + 1)
-    chunks = min(-(-longest // 64) * requests, tokens // 64 + requests)
-    floats = max(min(chunks, CHUNK_SCRATCH // per_chunk), requests) * per_chunk
-    floats = -(-floats // 4) * 4
-    return torch.empty(floats + more, dtype=torch.float32, device=device), floats
+    fit, longest = CHUNK_SCRATCH // per_chunk, -(-portions.longest // 64)
+    if fit < portions.count:
+        return None
+    each = longest if portions.chunks <= fit else min(longest, fit // portions.count)
+    grid = min(portions.chunks, each * portions.count)
+    if not lib.tl_chunks_pay(c_int(1 if memory else 0), c_int(portions.tokens + portions.rest_tokens), c_int(requests), c_int(portions.longest), c_int(heads), c_int(dim), c_int(vdim)):
+        return None
+    floats = -(-grid * per_chunk // 4) * 4
+    return _Chunks(64 * each, grid, torch.empty(floats + more, dtype=torch.float32, device=device), floats)
+
+
+def _chunk_args(chunks: _Chunks | None, portions: Portions, most: int):
+    """Of the C entries: the most tokens of a request, whether and how the portions go through the chunks, what is left for the token loop.  ``most``: the
+    tokens of a request by which the loop alone sizes its batches."""
+    if chunks is None:
+        return c_int(most), c_int(0), c_int(0), c_int(CHUNKED_FROM), c_int(0), c_int(0), c_void_p(0), ctypes.c_long(0)
+    return (c_int(portions.longest), c_int(chunks.segment), c_int(chunks.grid), c_int(CHUNKED_FROM), c_int(portions.rest),
+            c_int(min(portions.rest_longest, most)), _ptr(chunks.scratch), ctypes.c_long(chunks.floats))
 
 
 def mlstm_scan(qkv: torch.Tensor, k_off: int, v_off: int, gates: torch.Tensor, state: torch.Tensor, slots: torch.Tensor,
                req_indptr: torch.Tensor, out: torch.Tensor, heads: int, dim: int, vdim: int, cap: float | None,
-               qscale: float, denom_eps: float, max_new_tokens: int | None = None) -> None:
+               qscale: float, denom_eps: float, max_new_tokens: int | None = None, portions: Portions | None = None) -> None:
     """The matrix-memory recurrence over the step's tokens, request by request from the state its slot holds:
     ``qkv [T, >=]`` holds per token the queries at column 0 (``heads * dim``), the keys at ``k_off`` and the values at
     ``v_off`` (``heads * vdim``); ``gates`` float32 ``[T, 2 * heads]`` the raw input and forget gates (bias added);
     ``state`` float32 ``[slots, heads, dim * vdim + dim + 1]`` (S, n, m per head) is updated in place; ``out`` float32
-    ``[T, heads * vdim]`` receives ``S^T q / (max(|n.q|, exp(-m)) + denom_eps)``."""
+    ``[T, heads * vdim]`` receives ``S^T q / (max(|n.q|, exp(-m)) + denom_eps)``.  ``max_new_tokens``: no fewer tokens than any request brings; ``portions``
+    (of :data:`CHUNKED_FROM` tokens or more): what the host knows of the requests' lengths, exactly."""
     T = qkv.shape[0]
     R = req_indptr.numel() - 1
     if qkv.stride(1) != 1 or qkv.shape[1] < max(heads * dim, k_off + heads * dim, v_off + heads * vdim):
@@ -994,12 +1045,13 @@ def mlstm_scan(qkv: torch.Tensor, k_off: int, v_off: int, gates: torch.Tensor, s
     _i32(req_indptr, "req_indptr", R + 1)
     lib = _lib("recurrent")
     before = torch.empty((R, heads, dim + 1), dtype=torch.float32, device=qkv.device)      # n and m as the step finds them
-    longest = max(1, T - R + 1) if max_new_tokens is None else max_new_tokens
-    scratch, floats = _chunk_scratch(lib, True, T, R, longest, heads, dim, vdim, 4 * T * heads, qkv.device)
+    most = max(1, T - R + 1) if max_new_tokens is None else max_new_tokens
+    portions = portions or Portions.bound(T, R, max_new_tokens, CHUNKED_FROM)
+    chunks = _chunk_scratch(lib, True, R, heads, dim, vdim, 4 * T * heads, qkv.device, portions)
     _check(lib, lib.tl_mlstm_scan(_ptr(qkv), c_int(qkv.stride(0)), c_int(k_off), c_int(v_off), _ptr(gates), _ptr(state),
                                   ctypes.c_long(state.stride(0)), _ptr(slots), _ptr(before), _ptr(req_indptr), _ptr(out), c_int(R), c_int(heads),
                                   c_int(dim), c_int(vdim), c_float(cap if cap else 0.0), c_float(qscale), c_float(denom_eps),
-                                  c_int(longest), c_int(T), c_int(CHUNKED_FROM), _ptr(scratch), ctypes.c_long(floats), c_int(_dt(qkv, "mlstm_scan")), _stream()))
+                                  *_chunk_args(chunks, portions, most), c_int(_dt(qkv, "mlstm_scan")), _stream()))
 
 
 GATES = {"sigmoid": 0, "silu": 1}
@@ -1091,11 +1143,12 @@ def delta_scan(qkv: torch.Tensor, gates: torch.Tensor, state: torch.Tensor, slot
 
 
 def decay_scan(qkv: torch.Tensor, decay: torch.Tensor, state: torch.Tensor, slots: torch.Tensor, req_indptr: torch.Tensor, out: torch.Tensor,
-               heads: int, dim: int, vdim: int, max_new_tokens: int | None = None) -> None:
+               heads: int, dim: int, vdim: int, max_new_tokens: int | None = None, portions: Portions | None = None) -> None:
     """Linear attention with one fixed decay per head over the step's tokens, request by request from the state its slot holds: ``qkv``
     float32 ``[T, 2 * heads * dim + heads * vdim]`` (queries, keys, values, head by head), ``decay`` float32 ``[heads]``; head ``h`` of
     ``state[slot]`` (float32, laid out as :func:`delta_scan`'s) moves by ``S <- decay[h] S + k v^T`` and ``out`` float32 ``[T, heads * vdim]``
-    receives ``S^T q``."""
+    receives ``S^T q``.  ``max_new_tokens``: no fewer tokens than any request brings; ``portions`` (of :data:`CHUNKED_FROM` tokens or more): what
+    the host knows of the requests' lengths, exactly."""
     T = qkv.shape[0]
     R = req_indptr.numel() - 1
     C = 2 * heads * dim + heads * vdim
@@ -1110,11 +1163,11 @@ def decay_scan(qkv: torch.Tensor, decay: torch.Tensor, state: torch.Tensor, slot
     _i32(slots, "slots", R)
     _i32(req_indptr, "req_indptr", R + 1)
     lib = _lib("recurrent")
-    longest = max(1, T - R + 1) if max_new_tokens is None else max_new_tokens
-    scratch, floats = _chunk_scratch(lib, False, T, R, longest, heads, dim, vdim, 0, qkv.device)
+    most = max(1, T - R + 1) if max_new_tokens is None else max_new_tokens
+    portions = portions or Portions.bound(T, R, max_new_tokens, CHUNKED_FROM)
+    chunks = _chunk_scratch(lib, False, R, heads, dim, vdim, 0, qkv.device, portions)
     _check(lib, lib.tl_decay_scan(_ptr(qkv), _ptr(decay), _ptr(state), ctypes.c_long(state.stride(0)), _ptr(slots), _ptr(req_indptr), _ptr(out),
-                                  c_int(R), c_int(heads), c_int(dim), c_int(vdim), c_int(longest), c_int(T), c_int(CHUNKED_FROM), _ptr(scratch),
-                                  ctypes.c_long(floats), _stream()))
+                                  c_int(R), c_int(heads), c_int(dim), c_int(vdim), *_chunk_args(chunks, portions, most), _stream()))
 
 
 def selective_prepare(proj: torch.Tensor, x_off: int, conv_w: torch.Tensor, conv_b: torch.Tensor, gates: torch.Tensor, a_log: torch.Tensor,

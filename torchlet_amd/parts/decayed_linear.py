@@ -58,7 +58,8 @@ class DecayedLinearAttention(StagedMixer):
         qkv = torch.empty((T, self.channels), dtype=torch.float32, device=h.device)
         ops.silu_float(proj[:, : self.channels], qkv)
         o = torch.empty((T, self.v_width), dtype=torch.float32, device=h.device)
+        lengths = {"portions": ctx.portions(ops.CHUNKED_FROM)} if h.is_cuda else {}      # (which kernels take the step's requests)
         ops.decay_scan(qkv, self.decay, cache.state, ctx.slots, ctx.req_indptr, o, self.heads, self.dim, self.vdim,
-                       max_new_tokens=ctx.max_new_tokens)
+                       max_new_tokens=ctx.max_new_tokens, **lengths)
         # the heads side by side are one vector for the norm
         ops.gated_head_norm(o, proj[:, self.channels:], self.w_norm, float(self.spec.norm_eps), out, 1, self.v_width, gate="sigmoid", gain=gain)

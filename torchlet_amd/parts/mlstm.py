@@ -65,8 +65,10 @@ class MLSTM(Mixer):
         gates = torch.empty((T, 2 * self.heads), dtype=torch.float32, device=h.device)
         ops.linear(h, self.w_gates, self.b_gates, gates)
         o = torch.empty((T, self.v_width), dtype=torch.float32, device=h.device)
+        # (what the kernels need to know of the requests' lengths)
+        lengths = {"max_new_tokens": ctx.max_new_tokens, "portions": ctx.portions(ops.CHUNKED_FROM)} if h.is_cuda else {}
         ops.mlstm_scan(proj, self.qk_width, 2 * self.qk_width, gates, cache.state, ctx.slots, ctx.req_indptr, o,
-                       self.heads, self.dim, self.vdim, self.spec.gate_cap, self.qscale, float(self.spec.denom_eps))
+                       self.heads, self.dim, self.vdim, self.spec.gate_cap, self.qscale, float(self.spec.denom_eps), **lengths)
         y = torch.empty((T, self.v_width), dtype=self.dtype, device=h.device)
         ops.gated_head_norm(o, proj[:, 2 * self.qk_width + self.v_width:], self.w_norm, float(self.spec.norm_eps), y, self.heads, self.vdim)
         if self.dtype == torch.bfloat16 and ops.linear_partials_pay(T, self.hidden, self.v_width):
