@@ -757,21 +757,29 @@ delta_scan_kernel(const float* __restrict__ qkv, const float* __restrict__ gates
     }
 }
 
+// Columns of a lane: two (half the reads of shared memory a column) where one to a lane would not all be on the GPU at once, four work-groups to a
+// compute unit; up to there more waves win.  What counts as on the GPU at once is the step's work over that of its longest request (a request's last batch is
+// worked through whole): beside a long prompt the work-groups of decoded requests are gone after one batch.  Measured (us, one column / two; number-by-number
+// fetches before): the delta rule, 16 heads of 128 x 128, one prompt of 2048 tokens 405 / 603 (1533), beside 8 decoded tokens 418 / 605, eight prompts of 175 to 700
+// tokens 189 / 230 (1328); the selective recurrence, 128 heads of 128 x 64, four prompts of 275 to 1100 tokens 467 / 342 (3780); fixed decays, 16 heads of
+// 128 x 128, 2048 tokens 366 / 492 (1342).  Portions of 4 tokens and single ones (8 requests, 9 us) as before.
+static int delta_columns(int dim, int vdim, int heads, int requests, int tokens, int longest) {
+    if (dim > 128 || longest <= 4) return 1;
+    const double longs = ((double)tokens + (DELTA_TB - 1.0) * requests) / (longest < DELTA_TB ? DELTA_TB : longest);
+    return (double)((vdim + DELTA_COLS - 1) / DELTA_COLS) * heads * longs > 4.0 * tl_mlstm_units ? 2 : 1;
+}
+// (the rule alone, for tests)
+extern "C" int tl_delta_columns(int dim, int vdim, int heads, int requests, int tokens, int longest) { return delta_columns(dim, vdim, heads, requests, tokens, longest); }
+
 // state: per slot, from its start, heads x [vdim][dim] floats (a head's state column by column).
 template <int MODE>
 static int launch_delta_scan(const void* qkv, const void* gates, const void* head_decay, void* state, long slot_stride, const void* slots,
-                             const void* req_indptr, void* out, int requests, int heads, int kv_heads, int dim, int vdim, int longest, int below, hipStream_t stream) {
+                             const void* req_indptr, void* out, int requests, int heads, int kv_heads, int dim, int vdim, int tokens, int longest, int below, hipStream_t stream) {
     const int rpl = dim <= 64 ? 4 : dim <= 128 ? 8 : dim <= 192 ? 12 : 16;
     // tokens of a batch: 1 for a step of single tokens, 4 for short portions, else 16 (a batch is always worked through whole)
     const int tb = longest <= 1 ? 1 : (longest <= 4 ? 4 : DELTA_TB);
     const int vec = dim == DELTA_L * rpl && vdim % 4 == 0 && ((uintptr_t)qkv & 15) == 0;       // (a token's numbers are then a multiple of four)
-    const long groups = (long)((vdim + DELTA_COLS - 1) / DELTA_COLS) * heads * requests;
-    // two columns to a lane (half the reads of shared memory a column) where one to a lane would not all be on the GPU at once, four work-groups to a
-    // compute unit; up to there more waves win.  Measured (us, one column / two; number-by-number fetches before): the delta rule, 16 heads of 128 x
-    // 128, one prompt of 2048 tokens 405 / 603 (1533), eight prompts of 175 to 700 tokens 189 / 230 (1328); the selective recurrence, 128 heads of 128 x
-    // 64, four prompts of 275 to 1100 tokens 467 / 342 (3780); fixed decays, 16 heads of 128 x 128, 2048 tokens 366 / 492 (1342).  Portions of 4
-    // tokens and single ones (8 requests, 9 us) as before.
-    const int cpl = groups > 4L * tl_mlstm_units && rpl <= 8 && tb == DELTA_TB ? 2 : 1;
+    const int cpl = delta_columns(dim, vdim, heads, requests, tokens, longest);
     dim3 grid((vdim + DELTA_COLS * cpl - 1) / (DELTA_COLS * cpl), heads, requests), block(256);
 #define TL_DELTA_B(R, B, P)                                                                                                                \
     delta_scan_kernel<R, B, MODE, P><<<grid, block, 0, stream>>>((const float*)qkv, (const float*)gates, (const float*)head_decay, (float*)state, \
@@ -792,13 +800,13 @@ static int launch_delta_scan(const void* qkv, const void* gates, const void* hea
 }
 
 extern "C" int tl_delta_scan(const void* qkv, const void* gates, void* state, long slot_stride, const void* slots, const void* req_indptr,
-                             void* out, int requests, int heads, int kv_heads, int dim, int vdim, int longest, hipStream_t stream) {
+                             void* out, int requests, int heads, int kv_heads, int dim, int vdim, int tokens, int longest, hipStream_t stream) {
     TL_REQUIRE(requests >= 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && dim > 0 && vdim > 0, "delta_scan: bad sizes");
     TL_REQUIRE(dim <= DELTA_L * 16, "delta_scan: built for up to %d query/key dimensions per head, got %d", DELTA_L * 16, dim);
     TL_REQUIRE(slot_stride >= (long)heads * dim * vdim, "delta_scan: the state rows are too short");
     TL_REQUIRE(requests <= 65535 && heads <= 65535, "delta_scan: too many requests or heads for one launch");
     if (requests == 0) return TL_OK;
-    launch_delta_scan<1>(qkv, gates, nullptr, state, slot_stride, slots, req_indptr, out, requests, heads, kv_heads, dim, vdim, longest, INT_MAX, stream);
+    launch_delta_scan<1>(qkv, gates, nullptr, state, slot_stride, slots, req_indptr, out, requests, heads, kv_heads, dim, vdim, tokens, longest, INT_MAX, stream);
     TL_CHECK_LAUNCH("delta_scan");
     return TL_OK;
 }
@@ -1691,7 +1699,7 @@ extern "C" int tl_mlstm_scan(const void* qkv, int ld, int k_off, int v_off, cons
 // Per head S <- decay[head] S + k v^T, o = S^T q over the step's tokens, request by request from the state its slot holds: qkv float
 // [T, 2 * heads * dim + heads * vdim] (queries, keys, values, head by head), state as the delta rule's, out float [T, heads * vdim].
 extern "C" int tl_decay_scan(const void* qkv, const void* decay, void* state, long slot_stride, const void* slots, const void* req_indptr,
-                             void* out, int requests, int heads, int dim, int vdim, int longest, int segment, int chunk_grid, int least, int rest,
+                             void* out, int requests, int heads, int dim, int vdim, int tokens, int longest, int segment, int chunk_grid, int least, int rest,
                              int rest_longest, void* scratch, long scratch_floats, hipStream_t stream) {
     TL_REQUIRE(requests >= 0 && heads > 0 && dim > 0 && vdim > 0 && decay, "decay_scan: bad sizes");
     TL_REQUIRE(dim <= DELTA_L * 16, "decay_scan: built for up to %d query/key dimensions per head, got %d", DELTA_L * 16, dim);
@@ -1705,8 +1713,8 @@ extern "C" int tl_decay_scan(const void* qkv, const void* decay, void* state, lo
             requests, least, 0, 0}, ChunkPlan{segment, chunk_grid, (float*)scratch, scratch_floats}, longest, stream);
         if (rc != TL_OK || rest == 0) return rc;
     }
-    launch_delta_scan<0>(qkv, nullptr, decay, state, slot_stride, slots, req_indptr, out, requests, heads, heads, dim, vdim, chunks ? rest_longest : longest,
-                         chunks ? least : INT_MAX, stream);
+    launch_delta_scan<0>(qkv, nullptr, decay, state, slot_stride, slots, req_indptr, out, requests, heads, heads, dim, vdim, chunks ? rest * rest_longest : tokens,
+                         chunks ? rest_longest : longest, chunks ? least : INT_MAX, stream);
     TL_CHECK_LAUNCH("decay_scan");
     return TL_OK;
 }
@@ -1716,13 +1724,13 @@ extern "C" int tl_decay_scan(const void* qkv, const void* decay, void* state, lo
 // state + heads * vdim] as selective_prepare leaves it (C, B, x), gates float [T, 2 * heads] (dt, decay), skip float [heads] (D); the
 // state as the delta rule's ([vdim][state] per head), out float [T, heads * vdim].
 extern "C" int tl_selective_scan(const void* qkv, const void* gates, const void* skip, void* state, long slot_stride, const void* slots,
-                                 const void* req_indptr, void* out, int requests, int heads, int groups, int dim, int vdim, int longest, hipStream_t stream) {
+                                 const void* req_indptr, void* out, int requests, int heads, int groups, int dim, int vdim, int tokens, int longest, hipStream_t stream) {
     TL_REQUIRE(requests >= 0 && heads > 0 && groups > 0 && heads % groups == 0 && dim > 0 && vdim > 0 && gates && skip, "selective_scan: bad sizes");
     TL_REQUIRE(dim <= DELTA_L * 16, "selective_scan: built for states of up to %d numbers per column, got %d", DELTA_L * 16, dim);
     TL_REQUIRE(slot_stride >= (long)heads * dim * vdim, "selective_scan: the state rows are too short");
     TL_REQUIRE(requests <= 65535 && heads <= 65535, "selective_scan: too many requests or heads for one launch");
     if (requests == 0) return TL_OK;
-    launch_delta_scan<2>(qkv, gates, skip, state, slot_stride, slots, req_indptr, out, requests, heads, groups, dim, vdim, longest, INT_MAX, stream);
+    launch_delta_scan<2>(qkv, gates, skip, state, slot_stride, slots, req_indptr, out, requests, heads, groups, dim, vdim, tokens, longest, INT_MAX, stream);
     TL_CHECK_LAUNCH("selective_scan");
     return TL_OK;
 }

@@ -1138,7 +1138,7 @@ def delta_scan(qkv: torch.Tensor, gates: torch.Tensor, state: torch.Tensor, slot
     _i32(req_indptr, "req_indptr", R + 1)
     lib = _lib("recurrent")
     _check(lib, lib.tl_delta_scan(_ptr(qkv), _ptr(gates), _ptr(state), ctypes.c_long(state.stride(0)), _ptr(slots), _ptr(req_indptr), _ptr(out),
-                                  c_int(R), c_int(heads), c_int(kv_heads), c_int(dim), c_int(vdim),
+                                  c_int(R), c_int(heads), c_int(kv_heads), c_int(dim), c_int(vdim), c_int(T),
                                   c_int(max(1, T - R + 1) if max_new_tokens is None else max_new_tokens), _stream()))
 
 
@@ -1167,7 +1167,7 @@ def decay_scan(qkv: torch.Tensor, decay: torch.Tensor, state: torch.Tensor, slot
     portions = portions or Portions.bound(T, R, max_new_tokens, CHUNKED_FROM)
     chunks = _chunk_scratch(lib, False, R, heads, dim, vdim, 0, qkv.device, portions)
     _check(lib, lib.tl_decay_scan(_ptr(qkv), _ptr(decay), _ptr(state), ctypes.c_long(state.stride(0)), _ptr(slots), _ptr(req_indptr), _ptr(out),
-                                  c_int(R), c_int(heads), c_int(dim), c_int(vdim), *_chunk_args(chunks, portions, most), _stream()))
+                                  c_int(R), c_int(heads), c_int(dim), c_int(vdim), c_int(T), *_chunk_args(chunks, portions, most), _stream()))
 
 
 def selective_prepare(proj: torch.Tensor, x_off: int, conv_w: torch.Tensor, conv_b: torch.Tensor, gates: torch.Tensor, a_log: torch.Tensor,
@@ -1229,7 +1229,7 @@ def selective_scan(qkv: torch.Tensor, gates: torch.Tensor, skip: torch.Tensor, s
     _i32(req_indptr, "req_indptr", R + 1)
     lib = _lib("recurrent")
     _check(lib, lib.tl_selective_scan(_ptr(qkv), _ptr(gates), _ptr(skip), _ptr(state), ctypes.c_long(state.stride(0)), _ptr(slots), _ptr(req_indptr),
-                                      _ptr(out), c_int(R), c_int(heads), c_int(groups), c_int(dim), c_int(vdim),
+                                      _ptr(out), c_int(R), c_int(heads), c_int(groups), c_int(dim), c_int(vdim), c_int(T),
                                       c_int(max(1, T - R + 1) if max_new_tokens is None else max_new_tokens), _stream()))
 
 
