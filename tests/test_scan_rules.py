@@ -18,3 +18,31 @@ def lib():
     ([1] * 64, 128, 128, 64, 1), ([4] * 64, 128, 128, 64, 1), ([512] * 16, 16, 256, 128, 1)])
 def test_two_columns_a_lane_where_the_prompts_fill_the_gpu(lib, lens, heads, dim, vdim, want):
     assert lib.tl_delta_columns(*(c_int(x) for x in (dim, vdim, heads, len(lens), sum(lens), max(lens)))) == want
+
+
+def _pays(lib, memory, lens, heads, dim, vdim):
+    from torchlet_amd.kernels import ops
+    p = ops.Portions.of(lens, 32)
+    passes = -(-p.chunks * heads * (dim * vdim + dim + 1) // ops.CHUNK_SCRATCH)
+    return bool(lib.tl_chunks_pay(*(c_int(x) for x in (memory, p.count, p.tokens, p.chunks, passes, p.longest, p.rest, p.rest_tokens, p.rest_longest, len(lens),
+                                                       heads, dim, vdim))))
+
+
+# steps whose two ways differ by a fifth or more where both were measured
+@pytest.mark.parametrize("lens, heads, dim, vdim, want", [
+    ([128], 16, 128, 128, False), ([512], 16, 128, 128, True), ([2048], 16, 128, 128, True), ([100] * 4, 16, 128, 128, False), ([33] * 40, 16, 128, 128, False),
+    ([1] * 8 + [128], 16, 128, 128, False), ([1] * 31 + [64], 16, 128, 128, False), ([1] * 31 + [128], 16, 128, 128, False), ([1] * 31 + [512], 16, 128, 128, True),
+    ([1] * 63 + [64], 16, 128, 128, False), ([1] * 63 + [512], 16, 128, 128, True), ([1] * 31 + [64] * 4, 16, 128, 128, False), ([1] * 31 + [2017], 16, 128, 128, True),
+    ([1] * 8 + [64], 32, 128, 128, False), ([1] * 31 + [32], 32, 128, 128, False), ([20] * 8 + [128], 32, 128, 128, False), ([1] * 63 + [512], 32, 128, 128, True),
+    ([128], 4, 64, 64, False), ([512], 4, 64, 64, True), ([1] * 63 + [128], 4, 64, 64, False), ([1] * 31 + [2017], 4, 64, 64, True)])
+def test_fixed_decays_take_the_faster_way(lib, lens, heads, dim, vdim, want):
+    assert _pays(lib, 0, lens, heads, dim, vdim) == want
+
+
+@pytest.mark.parametrize("lens, heads, dim, vdim, want", [
+    ([32], 4, 256, 512, False), ([64], 4, 256, 512, False), ([512], 4, 256, 512, True), ([100] * 4, 4, 256, 512, True), ([1] * 8 + [64], 4, 256, 512, True),
+    ([1] * 31 + [64], 4, 256, 512, True), ([1] * 63 + [128], 4, 256, 512, True), ([1] * 31 + [2017], 8, 256, 512, True), ([20] * 8 + [32], 4, 256, 512, False),
+    ([20] * 8 + [128], 4, 256, 512, True), ([1] * 200 + [256], 8, 256, 512, True), ([32], 2, 128, 128, False), ([1] * 31 + [64], 2, 128, 128, False),
+    ([1] * 63 + [64], 2, 128, 128, True), ([1] * 31 + [64] * 4, 2, 128, 128, False), ([256], 2, 128, 128, True), ([1] * 200 + [256], 2, 128, 128, True)])
+def test_the_matrix_memory_takes_the_faster_way(lib, lens, heads, dim, vdim, want):
+    assert _pays(lib, 1, lens, heads, dim, vdim) == want

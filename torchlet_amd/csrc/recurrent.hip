@@ -252,6 +252,16 @@ static int launch_mlstm_scan(const void* qkv, int ld, int k_off, int v_off, cons
 static int tl_mlstm_units = 256;       // compute units the column tiles are dealt to
 extern "C" void tl_mlstm_set_compute_units(int units) { if (units > 0) tl_mlstm_units = units; }
 
+// Columns of a work-group: as few as it takes to give every compute unit one (the sums do not depend on the choice); rows a lane keeps: as few as 16 waves
+// of such lanes can hold the head's rows with, four at least.
+struct MlstmShape { int cols, rpt; };
+static MlstmShape mlstm_shape(int requests, int heads, int dim, int vdim) {
+    const long heads_reqs = (long)heads * requests;
+    const int cols = heads_reqs * ((vdim + 62) / 63) >= tl_mlstm_units ? 64 : heads_reqs * ((vdim + 30) / 31) >= tl_mlstm_units ? 32 : 16;
+    const int need = (dim * cols + 16 * TL_WAVE - 1) / (16 * TL_WAVE);
+    return {cols, need <= 4 ? 4 : need <= 8 ? 8 : need <= 16 ? 16 : need <= 32 ? 32 : 64};
+}
+
 // The token loop: requests of `below` tokens or more are left alone.
 static int mlstm_token_loop(const void* qkv, int ld, int k_off, int v_off, const void* gates, void* state, long slot_stride,
                             const void* slots, const void* before, const void* req_indptr, void* out, int requests, int heads, int dim, int vdim,
@@ -262,12 +272,8 @@ static int mlstm_token_loop(const void* qkv, int ld, int k_off, int v_off, const
     TL_REQUIRE(slot_stride >= (long)heads * ((long)dim * vdim + dim + 1), "mlstm_scan: the state rows are too short");
     TL_REQUIRE(dtype == TL_DT_F32 || dtype == TL_DT_BF16, "mlstm_scan: unknown dtype %d", dtype);
     if (requests == 0) return TL_OK;
-    // columns of a work-group: as few as it takes to give every compute unit one (the sums do not depend on the choice)
-    const long heads_reqs = (long)heads * requests;
-    const int cols = heads_reqs * ((vdim + 62) / 63) >= tl_mlstm_units ? 64 : heads_reqs * ((vdim + 30) / 31) >= tl_mlstm_units ? 32 : 16;
-    // rows a lane keeps: as few as 16 waves of such lanes can hold the head's rows with, four at least
-    const int need = (dim * cols + 16 * TL_WAVE - 1) / (16 * TL_WAVE);
-    const int rpt = need <= 4 ? 4 : need <= 8 ? 8 : need <= 16 ? 16 : need <= 32 ? 32 : 64;
+    const MlstmShape shape = mlstm_shape(requests, heads, dim, vdim);
+    const int cols = shape.cols, rpt = shape.rpt;
 #define TL_MLSTM_C(R, C)                                                                                                       \
     return dtype == TL_DT_F32                                                                                                  \
         ? launch_mlstm_scan<float, R, C>(qkv, ld, k_off, v_off, gates, state, (size_t)slot_stride, slots, before, req_indptr, out,    \
@@ -1645,16 +1651,36 @@ mlstm_gates_kernel(const float* __restrict__ gates, const float* __restrict__ st
     }
 }
 
-// Whether a step's long portions go through the chunks: two estimates in us, fitted to the measurements (dim x vdim states; memory: the matrix memory).
-//   token loop, a token: fixed decays 0.18 while the work-groups fit twice on every compute unit, in proportion beyond (one prompt of 512 / 2048 tokens
-//   of 16 heads of 128 x 128: 97 / 372; eight of 400: 141; 16 of 200: 123); the matrix memory 0.58, or 1 per million numbers of state (one prompt of 300
-//   / 2048 tokens of 4 heads of 256 x 512: 189 / 1193; 16 of 130: 1145; 4 of 200 of 8 heads: 1149; 64 of 40: 1136);
-//   chunks: their launches, and the tokens (the same: 54 / 80, 151, 172; 93 / 172, 241, 148, 382).
-extern "C" int tl_chunks_pay(int memory, int tokens, int requests, int longest, int heads, int dim, int vdim) {
-    const double state = (double)heads * dim * vdim, groups = (double)((vdim + DELTA_COLS - 1) / DELTA_COLS) * heads * requests;
-    const double loop = memory ? longest * fmax(0.58, requests * state / 1e6) : longest * 0.18 * fmax(1.0, groups / (2.0 * tl_mlstm_units));
-    const double chunks = memory ? 60 + tokens * 0.08 * state / 524288 : 45 + tokens * 0.038 * state / 262144;
-    return chunks < loop;
+// Whether a step's long portions (count of them, tokens in all, `chunks` chunks in `passes` passes, the longest of so many tokens) go through the chunks, beside
+// `rest` requests of rest_tokens tokens, rest_longest at most: two estimates in us, fitted to the device's times below.
+//   The token loop.  Fixed decays: a token of the longest portion 0.18 (0.115 with states of 64 rows), or all portions' work-groups over 2.8 of them a compute
+//     unit, and behind it the others' over 2.4, whose one token is a batch of 16 like any.  The matrix memory: a token 0.58, 1.2 or 2.8 by the rows a lane keeps, once for
+//     every round of work-groups (16 waves a compute unit); the decoded requests' states cost the same on both ways.
+//   The chunks: their launches, a little for every chunk of the longest portion, the chunks' sums and products; then the others go through the loop alone, decoded ones in
+//     batches of one token.
+// Measured (us, loop / chunks): fixed decays, 16 heads of 128 x 128: 128 tokens 24 / 45, 256 51 / 47, 2048 367 / 80; 16 x 128 78 / 83; 64 beside 31 decoded 38 / 65, 128 beside
+// 31 47 / 66, 512 beside 31 114 / 70, 256 beside 200 158 / 133; 32 heads: 256 51 / 52, 256 beside 31 93 / 79; 4 heads of 64 x 64: 256 32 / 32, beside 8 32 / 35.  The matrix memory, 4
+// heads of 256 x 512: 64 tokens 49 / 77, 128 85 / 79, 2048 1191 / 170; 32 beside 8 decoded 127 / 122, 64 beside 31 278 / 194, 32 beside 63 269 / 269, 32 beside 8 of 20 176 / 220, 128 beside them
+// 445 / 229; 8 heads: 64 91 / 80, 32 beside 63 521 / 541; 2 heads of 128 x 128: 64 44 / 52, 128 80 / 54, 64 beside 31 57 / 76, 64 beside 63 103 / 84, 16 x 64 52 / 56.
+extern "C" int tl_chunks_pay(int memory, int count, int tokens, int chunks, int passes, int longest, int rest, int rest_tokens, int rest_longest, int requests, int heads,
+                             int dim, int vdim) {
+    const double state = (double)heads * dim * vdim;
+    if (rest_tokens == 0) rest = rest_longest = 0;                 // (none, or the caller cannot tell)
+    if (memory) {
+        const MlstmShape shape = mlstm_shape(requests, heads, dim, vdim);
+        const int waves = (dim + shape.rpt * (TL_WAVE / shape.cols) - 1) / (shape.rpt * (TL_WAVE / shape.cols));
+        const double token = shape.rpt <= 4 ? 0.58 : shape.rpt <= 8 ? 1.2 : 0.175 * shape.rpt, tiles = (double)heads * ((vdim + shape.cols - 2) / (shape.cols - 1));
+        const double at_once = (double)tl_mlstm_units * (waves < 16 ? 16 / waves : 1);
+        auto loop = [&](int n, int most) { return n > 0 && most > 1 ? most * token * ceil(n * tiles / at_once) : 0.0; };
+        const double others = loop(rest, rest_longest), together = loop(count + (rest_longest > 1 ? rest : 0), longest > rest_longest ? longest : rest_longest);
+        const double all = fmin(loop(count, longest) + others, together) + (rest > 0 ? 0 : 10);
+        return 50 + 25 * fmin(1.0, state / 5e5) + longest * 0.02 + chunks * 64 * state * 5e-8 + (passes - 1) * 50.0 + (rest > 0 ? 15 + others : 0) < all;
+    }
+    const double groups = (double)((vdim + DELTA_COLS - 1) / DELTA_COLS) * heads, token = dim <= 64 ? 0.115 : 0.18;
+    auto batches = [&](int n, int t, double per_unit) { return token * groups * (t + (DELTA_TB - 1.0) * n) / (per_unit * tl_mlstm_units); };
+    const double all = 3 + fmax(token * longest, batches(count, tokens, 2.8)) + batches(rest, rest_tokens, 2.4);
+    const double others = rest == 0 ? 0 : 5 + (rest_longest <= 1 ? 1.4e-6 * rest * state : batches(rest, rest_tokens, 2.4));
+    return 30 + 12 * fmin(1.0, state / 262144) + longest * 0.003 + chunks * 64 * state * 1e-7 + (passes - 1) * 30.0 + others < all;
 }
 
 // Whether the chunks can be read in whole pieces of four numbers.

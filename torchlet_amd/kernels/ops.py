@@ -979,9 +979,11 @@ class Portions(NamedTuple):
 
     @classmethod
     def bound(cls, tokens: int, requests: int, longest: int | None, least: int) -> "Portions":
-        """For callers that know their rows and requests alone, and maybe a bound on a request's tokens: no fewer of anything than there are."""
+        """For callers that know their rows and requests alone, and maybe a bound on a request's tokens: no fewer of
+        anything than there are, or none for the chunks where there will hardly be any."""
+        likely = tokens - requests + 1 if longest is None else longest      # (none of them empty)
         longest = tokens if longest is None else longest
-        if longest < least:
+        if likely < least:
             return cls(0, 0, 0, 0, requests, tokens, longest)
         count = min(requests, tokens // least)
         return cls(count, tokens, tokens // 64 + count, longest, requests, 0, least - 1)
@@ -1006,7 +1008,8 @@ def _chunk_scratch(lib, memory: bool, requests: int, heads: int, dim: int, vdim:
         return None
     each = longest if portions.chunks <= fit else min(longest, fit // portions.count)
     grid = min(portions.chunks, each * portions.count)
-    if not lib.tl_chunks_pay(c_int(1 if memory else 0), c_int(portions.tokens + portions.rest_tokens), c_int(requests), c_int(portions.longest), c_int(heads), c_int(dim), c_int(vdim)):
+    if not lib.tl_chunks_pay(*(c_int(x) for x in (1 if memory else 0, portions.count, portions.tokens, portions.chunks, -(-longest // each), portions.longest,
+                                                  portions.rest, portions.rest_tokens, portions.rest_longest, requests, heads, dim, vdim))):
         return None
     floats = -(-grid * per_chunk // 4) * 4
     return _Chunks(64 * each, grid, torch.empty(floats + more, dtype=torch.float32, device=device), floats)
