@@ -192,6 +192,55 @@ extern "C" int tl_latent_rows(const void* plane, int page_size, const void* bloc
     return TL_OK;
 }
 
+// ------------------------------------------------------------------ some tokens' rows side by side, and back
+// Row i of `own` [count, heads * dim] and the places from `rank` on of every head's `row` numbers of qrow [count, heads * row] are the two parts of token
+// tokens[i]'s queries (dim and rot numbers a head), row i of `gates` [count, gate_cols] its gates.  16 bytes to a thread, the gates'
+// numbers one by one where they do not all start on 16 bytes.
+__global__ void __launch_bounds__(256)
+latent_take_kernel(const bf16_t* __restrict__ q, int q_ld, int heads, int dim8, int rot8, const int* __restrict__ tokens, uint4* __restrict__ own, bf16_t* __restrict__ qrow,
+                   int rank, int row, const bf16_t* __restrict__ gate, int gate_ld, int gate_cols, bf16_t* __restrict__ gates) {
+    const int i = blockIdx.x, t = tokens[i], width8 = dim8 + rot8;
+    const uint4* src = (const uint4*)(q + (size_t)t * q_ld);
+    for (int p = threadIdx.x; p < heads * width8; p += blockDim.x) {
+        const int h = p / width8, c = p % width8;
+        if (c < dim8) own[((size_t)i * heads + h) * dim8 + c] = src[p];
+        else *(uint4*)(qrow + ((size_t)i * heads + h) * row + rank + (c - dim8) * 8) = src[p];
+    }
+    if (!gate) return;
+    const bf16_t* from = gate + (size_t)t * gate_ld;
+    bf16_t* to = gates + (size_t)i * gate_cols;
+    if (gate_cols % 8 == 0 && gate_ld % 8 == 0 && (((uintptr_t)gate | (uintptr_t)gates) & 15) == 0)
+        for (int c = threadIdx.x * 8; c < gate_cols; c += blockDim.x * 8) *(uint4*)(to + c) = *(const uint4*)(from + c);
+    else
+        for (int c = threadIdx.x; c < gate_cols; c += blockDim.x) to[c] = from[c];
+}
+
+extern "C" int tl_latent_take(const void* q, int q_ld, int heads, int dim, int rot, const void* tokens, int count, void* own, void* qrow, int rank, const void* gate,
+                              int gate_ld, int gate_cols, void* gates, hipStream_t stream) {
+    TL_REQUIRE(heads > 0 && dim > 0 && dim % 8 == 0 && rot >= 0 && rot % 8 == 0 && rank % 8 == 0 && count >= 0 && q_ld >= heads * (dim + rot) && q_ld % 8 == 0, "latent_take: bad sizes");
+    TL_REQUIRE((((uintptr_t)q | (uintptr_t)own | (uintptr_t)qrow) & 15) == 0 && (!gate || (gates && gate_ld >= gate_cols)), "latent_take: rows not aligned");
+    if (count == 0) return TL_OK;
+    latent_take_kernel<<<count, 256, 0, stream>>>((const bf16_t*)q, q_ld, heads, dim / 8, rot / 8, (const int*)tokens, (uint4*)own, (bf16_t*)qrow, rank, rank + rot,
+                                                  (const bf16_t*)gate, gate_ld, gate_cols, (bf16_t*)gates);
+    TL_CHECK_LAUNCH("latent_take");
+    return TL_OK;
+}
+
+// Row tokens[i] of dst becomes row i of src [count, cols].
+__global__ void __launch_bounds__(256)
+put_rows_kernel(const uint4* __restrict__ src, const int* __restrict__ tokens, bf16_t* __restrict__ dst, int dst_ld, int cols8) {
+    uint4* to = (uint4*)(dst + (size_t)tokens[blockIdx.x] * dst_ld);
+    for (int c = threadIdx.x; c < cols8; c += blockDim.x) to[c] = src[(size_t)blockIdx.x * cols8 + c];
+}
+
+extern "C" int tl_put_rows(const void* src, const void* tokens, void* dst, int dst_ld, int count, int cols, hipStream_t stream) {
+    TL_REQUIRE(count >= 0 && cols > 0 && cols % 8 == 0 && dst_ld >= cols && dst_ld % 8 == 0 && (((uintptr_t)src | (uintptr_t)dst) & 15) == 0, "put_rows: rows not aligned");
+    if (count == 0) return TL_OK;
+    put_rows_kernel<<<count, 256, 0, stream>>>((const uint4*)src, (const int*)tokens, (bf16_t*)dst, dst_ld, cols / 8);
+    TL_CHECK_LAUNCH("put_rows");
+    return TL_OK;
+}
+
 // ------------------------------------------------------------------ attention
 // A tile is up to `tile_tokens` consecutive new tokens of one request times a chunk of up to 16 heads: one wave per
 // row (token, head).  The keys pass through shared memory KT at a time, shared by all rows of the tile; a lane takes the

@@ -1678,6 +1678,33 @@ def latent_rows(plane: torch.Tensor, block_table: torch.Tensor, req_indptr: torc
                                    _ptr(at), _ptr(low), c_int(count), c_int(window), c_int(rank), c_int(rot), _ptr(latents), _ptr(rotated), c_int(rows), _stream()))
 
 
+def latent_take(q: torch.Tensor, heads: int, dim: int, rot: int, tokens: torch.Tensor, own: torch.Tensor, qrow: torch.Tensor, rank: int,
+                gate: torch.Tensor | None = None, gates: torch.Tensor | None = None) -> None:
+    """Some tokens' queries (``q [T, heads * (dim + rot)]``) side by side: row ``i`` of ``own [count, heads * dim]`` and the places behind every head's first ``rank`` of
+    ``qrow [count, heads * (rank + rot)]`` are those of token ``tokens[i]`` (int32 ``[count]``), row ``i`` of ``gates`` is row ``tokens[i]`` of ``gate``.  bfloat16, sizes
+    multiples of 8."""
+    count = own.shape[0]
+    if q.shape[1] != heads * (dim + rot) or q.stride(1) != 1 or own.shape != (count, heads * dim) or qrow.shape != (count, heads * (rank + rot)) \
+            or not own.is_contiguous() or not qrow.is_contiguous() or any(t.dtype != torch.bfloat16 for t in (q, own, qrow)) \
+            or (gate is not None and (gates is None or gates.shape != (count, gate.shape[1]) or gate.shape[0] != q.shape[0] or gate.stride(1) != 1
+                                      or not gates.is_contiguous() or gate.dtype != q.dtype or gates.dtype != q.dtype)):
+        raise KernelError("latent_take: shapes or dtypes do not fit")
+    _i32(tokens, "tokens", count)
+    lib = _lib("latent")
+    _check(lib, lib.tl_latent_take(_ptr(q), c_int(q.stride(0)), c_int(heads), c_int(dim), c_int(rot), _ptr(tokens), c_int(count), _ptr(own), _ptr(qrow), c_int(rank),
+                                   _ptr(gate), c_int(gate.stride(0) if gate is not None else 0), c_int(gate.shape[1] if gate is not None else 0), _ptr(gates), _stream()))
+
+
+def put_rows(src: torch.Tensor, tokens: torch.Tensor, dst: torch.Tensor) -> None:
+    """``dst[tokens[i]] = src[i]``: ``src [count, cols]`` contiguous, ``dst [T, cols]`` (rows may be strided), bfloat16, ``cols`` a multiple of 8."""
+    count, cols = src.shape
+    if dst.shape[1] != cols or dst.stride(1) != 1 or not src.is_contiguous() or src.dtype != torch.bfloat16 or dst.dtype != src.dtype:
+        raise KernelError("put_rows: shapes or dtypes do not fit")
+    _i32(tokens, "tokens", count)
+    lib = _lib("latent")
+    _check(lib, lib.tl_put_rows(_ptr(src), _ptr(tokens), _ptr(dst), c_int(dst.stride(0)), c_int(count), c_int(cols), _stream()))
+
+
 def prompt_rows_attention(q: torch.Tensor, out: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, rows: int, req_indptr: torch.Tensor,
                           ctx_lens: torch.Tensor, portions, heads: int, own: int, shared: int, vdim: int, scale: float, sink: torch.Tensor | None = None,
                           window: int = 0, gate: torch.Tensor | None = None, value_gate: torch.Tensor | None = None) -> None:

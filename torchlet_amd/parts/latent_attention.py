@@ -158,7 +158,7 @@ class LatentAttention(Mixer):
         keys = torch.empty(rows * (at_once * self.dim + self.rot), dtype=self.dtype, device=dev)
         up = torch.empty((at_once * self.vdim, rows), dtype=self.dtype, device=dev)
         w_uv = self.w_uv.view(self.heads * self.vdim, self.rank)
-        gate = down[:, self.gate_at: self.gate_at + self.gate_cols] if self.gate_cols else None
+        gate = self._gates(down)
         width = self.dim + self.rot
         for a in range(0, self.heads, at_once):
             b = min(a + at_once, self.heads)
@@ -209,7 +209,8 @@ class LatentAttention(Mixer):
             tile_req, tile_tok0, tiles = ctx.tiles(tq)
             if ctx.decode_only and tiles == T:          # one token per request: no tile list to look up
                 tile_req = tile_tok0 = None
-            self._attend_absorbed(q, qrow, values, down, plane, table, ctx, ctx.req_indptr, tile_req, tile_tok0, tiles, tq, general, ctx.max_new_tokens)
+            self._attend_absorbed(q, self.dim + self.rot, qrow, self._gates(down), values, plane, table, ctx, ctx.req_indptr, tile_req, tile_tok0, tiles, tq, general,
+                                  ctx.max_new_tokens)
         else:
             portions, at_once = long
             if not self.q_rank:
@@ -231,24 +232,24 @@ class LatentAttention(Mixer):
         general = table.shape[1] > ops.LATENT_MFMA_MAX_BLOCKS
         tq = self.general_tile_tokens if general else self.tile_tokens
         tile_req, tile_tok0, tiles, tokens, count, _ = ctx.tiles_by_length(tq, tq, _PROMPT_LEAST)[0]
-        few = q.index_select(0, tokens)
+        own = torch.empty((count, self.heads * self.dim), dtype=self.dtype, device=q.device)
         qrow = torch.empty((count, self.heads * self.row), dtype=self.dtype, device=q.device)
-        if self.rot:
-            qrow.view(count, self.heads, self.row)[:, :, self.rank:] = few.view(count, self.heads, self.dim + self.rot)[:, :, self.dim:]
+        gates = torch.empty((count, self.gate_cols), dtype=self.dtype, device=q.device) if self.gate_cols else None
+        ops.latent_take(q, self.heads, self.dim, self.rot, tokens, own, qrow, self.rank, self._gates(down), gates)
         out = torch.empty((count, self.heads * self.vdim), dtype=self.dtype, device=q.device)
         most = 1 if count == ctx.num_requests - portions[3] else tq
-        self._attend_absorbed(few, qrow, out, down.index_select(0, tokens) if self.gate_cols else down, plane, table, ctx, portions[6], tile_req, tile_tok0,
-                              tiles, tq, general, most)
-        values.index_copy_(0, tokens.long(), out)
+        self._attend_absorbed(own, self.dim, qrow, gates, out, plane, table, ctx, portions[6], tile_req, tile_tok0, tiles, tq, general, most)
+        ops.put_rows(out, tokens, values)
 
-    def _attend_absorbed(self, q, qrow, values, down, plane, table, ctx, indptr, tile_req, tile_tok0, tiles, tq, general, most_new):
-        """``values`` of queries whose rotated parts lie in ``qrow`` already, against the cached rows as they are."""
+    def _gates(self, down):
+        return down[:, self.gate_at: self.gate_at + self.gate_cols] if self.gate_cols else None
+
+    def _attend_absorbed(self, q, q_head, qrow, gates, values, plane, table, ctx, indptr, tile_req, tile_tok0, tiles, tq, general, most_new):
+        """``values`` of queries (``q_head`` numbers from one head's to the next one's) whose rotated parts lie in ``qrow`` already, against the cached rows as they are."""
         T, n = q.shape[0], self.heads
-        ops.heads_linear(q, self.dim + self.rot, self.w_uk_t, qrow, self.row)
+        ops.heads_linear(q, q_head, self.w_uk_t, qrow, self.row)
         mixed_latent = torch.empty((T, n * self.rank), dtype=self.dtype, device=q.device)
         ops.latent_attention(qrow, mixed_latent, plane, table, indptr, ctx.ctx_lens, tile_req, tile_tok0, tiles, tq,
                              n, self.rank, self.rot, plane.shape[2], self.scale, self.sink, self._splits(ctx, tiles),
-                             general=general, max_new_tokens=most_new, window=self.window,
-                             gate=down[:, self.gate_at:] if self.spec.gate else None)
-        ops.heads_linear(mixed_latent, self.rank, self.w_uv, values, self.vdim,
-                         gate=down[:, self.gate_at: self.gate_at + self.gate_cols] if self.spec.gate_values else None)
+                             general=general, max_new_tokens=most_new, window=self.window, gate=gates if self.spec.gate else None)
+        ops.heads_linear(mixed_latent, self.rank, self.w_uv, values, self.vdim, gate=gates if self.spec.gate_values else None)
