@@ -116,6 +116,10 @@ class StepContext:
             t = self._tiles[tq] = (v["r"], v["t"], len(tr))
         return t
 
+    def tile_count(self, tq: int) -> int:
+        """The number of tiles of ``tq`` tokens."""
+        return int((-(-self._host_new_lens // tq)).sum())
+
     def tiles_by_length(self, tq_short: int, tq_long: int, threshold: int):
         """Two tile lists: requests that bring fewer than ``threshold`` tokens in tiles of
         ``tq_short`` tokens, the others in tiles of ``tq_long``.  The first list comes with the
@@ -153,8 +157,9 @@ class StepContext:
     def long_portions(self, least: int, window: int = 0, tile: int = 128):
         """The requests that bring ``least`` tokens or more, and where the rows of the positions that each reads lie side by side (from the first one inside
         the ``window`` on, 0: all; starts and counts rounded to multiples of 64): ``(portion_req [n], portion_at [n + 1], portion_low [n], n, rows,
-        tiles of `tile` new tokens, others, pairs, tokens)``, the first three int32 on the device; ``None`` without such requests.  ``others``: the ``req_indptr`` of a step that
-        held the other requests' tokens alone (int32 ``[R + 1]`` on the device), ``None`` if there are none; ``pairs``: the portions' tokens times the rows they read; ``tokens``: theirs."""
+        tiles of `tile` new tokens, others, pairs, tokens, most)``, the first three int32 on the device; ``None`` without such requests.  ``others``: the ``req_indptr`` of a step that
+        held the other requests' tokens alone (int32 ``[R + 1]`` on the device), ``None`` if there are none; ``pairs``: the portions' tokens times the rows they read; ``tokens``: theirs;
+        ``most``: the rows of the portion that reads the most."""
         key = ("portions", least, window, tile)
         if key not in self._tiles:
             req = np.nonzero(self._host_new_lens >= least)[0].astype(np.int32)
@@ -169,7 +174,7 @@ class StepContext:
                 np.cumsum(np.where(self._host_new_lens < least, self._host_new_lens, 0), out=others[1:])
                 v = self._upload({"r": req, "a": at.astype(np.int32), "l": low.astype(np.int32), "o": others})
                 self._tiles[key] = (v["r"], v["a"], v["l"], len(req), int(at[-1]), int((-(-new // tile)).sum()), v["o"] if others[-1] else None,
-                                    int((new * np.diff(at)).sum()), int(new.sum()))
+                                    int((new * np.diff(at)).sum()), int(new.sum()), int(np.diff(at).max()))
         return self._tiles[key]
 
 

@@ -39,6 +39,13 @@ _PROMPT_LEAST = 64              # tokens of a portion from which its keys and va
 # after none 221 / 131, 141 / 105, 112 / 116; 64 after 4000 193 / 193, 124 / 135; 128 after 4000 297 / 211, 177 / 138; 8 x 128 after none 215 / 132, 123 / 108, 117 / 117.
 # Beside 31 decoded tokens, which then take kernels of their own, 256 after 2000 516 / 301, 282 / 205, 130 / 198.
 _TOKEN_AS_KEYS, _UP_LEAST, _UP_LEAST_BESIDE = 256, 5 << 20, 8 << 20
+# What a long context adds is not in those: every key is projected once, whatever the number of tokens that read it, and a portion's 128 tokens walk it in one work-group.
+# So the absorbed way must also cost no less than the projected one up to _UP_SLACK, in the same unit (12 ps): its pairs, or the longest context over the splits that the
+# step's tiles leave, 64 rows a tile; against a key's projection for a head and a key's way through the walk of the portion that reads the most, in steps of 32 keys (with
+# a shared part) or 64.  Measured on the device with 32 / 16 / 8 heads, absorbed against projected: 64 tokens after 4000 188 / 197, 123 / 180, 82 / 162; after 8000 285 / 349,
+# 168 / 287, 107 / 259; after 16000 477 / 649, 272 / 536, 156 / 468; 128 after 8000 490 / 361, 290 / 297, 178 / 270; 256 after 16000 1641 / 695, 876 / 562, 481 / 487; 64 after 8000 beside
+# 31 decoded tokens after 2000 850 / 490, 400 / 367, 329 / 327.  The kernel that takes what the matrix cores' cannot costs 24 times as much.
+_KEY_PROJECTED, _KEY_WALKED, _UP_SLACK, _GENERAL = 51, (1110, 1670), 1_700_000, 24
 
 
 @MIXERS.register("latent_attention")
@@ -138,15 +145,21 @@ class LatentAttention(Mixer):
         keys = ctx.max_total_len if not self.window else min(ctx.max_total_len, self.window + ctx.max_new_tokens - 1)
         return max(1, min(self.compute_units // groups, keys // _MIN_KEYS_PER_SPLIT, 64))
 
-    def _portions(self, ctx):
-        """The step's long portions and the heads whose keys and values are held at once, or ``None``."""
+    def _portions(self, ctx, blocks: int = 0):
+        """The step's long portions (``blocks``: the width of its block table) and the heads whose keys and values are held at once, or ``None``."""
         if not self.project_up or ctx.max_new_tokens < _PROMPT_LEAST:
             return None
         portions = ctx.long_portions(_PROMPT_LEAST, self.window)
-        work = (portions[7] + _TOKEN_AS_KEYS * portions[8]) * self.heads
-        if work < (_UP_LEAST if portions[6] is None else _UP_LEAST_BESIDE):
+        rows, pairs, tokens, longest = portions[4], portions[7], portions[8], portions[9]
+        if (pairs + _TOKEN_AS_KEYS * tokens) * self.heads < (_UP_LEAST if portions[6] is None else _UP_LEAST_BESIDE):
             return None
-        most = ops.PROMPT_ROWS_SCRATCH_BYTES // (portions[4] * (self.dim + self.vdim) * 2)
+        tiles = ctx.tile_count(self.tile_tokens)
+        splits = self._splits(ctx, tiles)
+        keys = ctx.max_total_len if not self.window else min(ctx.max_total_len, self.window + ctx.max_new_tokens - 1)
+        absorbed = max(pairs * self.heads, keys // splits * 64 * min(self.compute_units, tiles * splits)) + _TOKEN_AS_KEYS * tokens * self.heads
+        if absorbed * (_GENERAL if blocks > ops.LATENT_MFMA_MAX_BLOCKS else 1) + _UP_SLACK < rows * self.heads * _KEY_PROJECTED + longest * _KEY_WALKED[self.rot > 0]:
+            return None
+        most = ops.PROMPT_ROWS_SCRATCH_BYTES // (rows * (self.dim + self.vdim) * 2)
         if most < 1:
             return None
         return portions, -(-self.heads // -(-self.heads // min(most, self.heads)))
@@ -184,7 +197,7 @@ class LatentAttention(Mixer):
         down = torch.empty((T, self.down_cols), dtype=self.dtype, device=dev)
         ops.linear(h, self.w_down, None, down)
         write = (ctx.token_req, table, plane, cache.page_size) if cache.writable else (None, None, None, 0)
-        long = self._portions(ctx)
+        long = self._portions(ctx, table.shape[1])
         if self.q_rank:
             cq = torch.empty((T, self.q_rank), dtype=self.dtype, device=dev)
             ops.latent_prepare(down, self.q_rank, self.rank, self.rot, rot_dims, self.w_dq_norm, self.w_dkv_norm, float(self.spec.norm_eps),
