@@ -45,7 +45,7 @@ _TOKEN_AS_KEYS, _UP_LEAST, _UP_LEAST_BESIDE = 256, 5 << 20, 8 << 20
 # a shared part) or 64.  Measured on the device with 32 / 16 / 8 heads, absorbed against projected: 64 tokens after 4000 188 / 197, 123 / 180, 82 / 162; after 8000 285 / 349,
 # 168 / 287, 107 / 259; after 16000 477 / 649, 272 / 536, 156 / 468; 128 after 8000 490 / 361, 290 / 297, 178 / 270; 256 after 16000 1641 / 695, 876 / 562, 481 / 487; 64 after 8000 beside
 # 31 decoded tokens after 2000 850 / 490, 400 / 367, 329 / 327.  The kernel that takes what the matrix cores' cannot costs 24 times as much.
-_KEY_PROJECTED, _KEY_WALKED, _UP_SLACK, _GENERAL = 51, (1110, 1670), 1_700_000, 24
+_KEY_PROJECTED, _KEY_WALKED, _UP_SLACK, _GENERAL = 51, (1110, 1580), 1_700_000, 24
 
 
 @MIXERS.register("latent_attention")
@@ -156,7 +156,7 @@ class LatentAttention(Mixer):
         tiles = ctx.tile_count(self.tile_tokens)
         splits = self._splits(ctx, tiles)
         keys = ctx.max_total_len if not self.window else min(ctx.max_total_len, self.window + ctx.max_new_tokens - 1)
-        absorbed = max(pairs * self.heads, keys // splits * 64 * min(self.compute_units, tiles * splits)) + _TOKEN_AS_KEYS * tokens * self.heads
+        absorbed = max(pairs * self.heads, keys // splits * 64 * min(self.compute_units, tiles * -(-self.heads // ops.LATENT_ATTENTION_ROWS) * splits)) + _TOKEN_AS_KEYS * tokens * self.heads
         if absorbed * (_GENERAL if blocks > ops.LATENT_MFMA_MAX_BLOCKS else 1) + _UP_SLACK < rows * self.heads * _KEY_PROJECTED + longest * _KEY_WALKED[self.rot > 0]:
             return None
         most = ops.PROMPT_ROWS_SCRATCH_BYTES // (rows * (self.dim + self.vdim) * 2)
