@@ -305,7 +305,7 @@ struct ExpertsCall {
     bf16_t* out;
     int out_ld;
     const int* offsets;
-    int groups, rows, N, K, act;
+    int groups, rows, x_rows, N, K, act;      // rows: of out; x_rows: of a
 };
 
 template <int WAVES>
@@ -386,14 +386,14 @@ static int pick_experts(const ExpertsCall& c) {
 
 static bool experts_fit(const ExpertsCall& c) {
     // (a lane's offset from the first row of x, and of w from its tile's, is kept in 32 bits)
-    return c.K % 64 == 0 && c.a_ld % 8 == 0 && ((uintptr_t)c.a % 16) == 0 && ((uintptr_t)c.w % 16) == 0 && (long)c.rows * c.a_ld * 2 < (1L << 31) &&
+    return c.K % 64 == 0 && c.a_ld % 8 == 0 && ((uintptr_t)c.a % 16) == 0 && ((uintptr_t)c.w % 16) == 0 && (long)c.x_rows * c.a_ld * 2 < (1L << 31) &&
            256L * c.K * 2 < (1L << 31) && (long)(c.rows / 16 + c.groups) <= 65535;
 }
 
 // One named kernel of the two (tests cover each; tuning times them).
 extern "C" int tl_experts_variant(const void* a, int a_ld, const void* src, const void* w, void* out, int out_ld, const void* offsets, int groups, int rows,
-                                  int N, int K, int act, int which, hipStream_t stream) {
-    const ExpertsCall c{(const bf16_t*)a, a_ld, (const int*)src, (const bf16_t*)w, (bf16_t*)out, out_ld, (const int*)offsets, groups, rows, N, K, act};
+                                  int x_rows, int N, int K, int act, int which, hipStream_t stream) {
+    const ExpertsCall c{(const bf16_t*)a, a_ld, (const int*)src, (const bf16_t*)w, (bf16_t*)out, out_ld, (const int*)offsets, groups, rows, x_rows, N, K, act};
     TL_REQUIRE(groups > 0 && rows > 0 && N > 0 && K > 0 && offsets && known_activation(act) && (!(act & ACT_PAIRS) || N % 2 == 0) && experts_fit(c), "experts_variant: bad arguments");
     return launch_experts(which, c, stream);
 }
@@ -406,9 +406,9 @@ static bool heads_few_rows(int rows, int groups, int N, int K) {
 }
 
 extern "C" int tl_grouped_gemm(const void* a, int a_ld, int a_group, const void* src, const void* w, void* out, int out_ld, int out_group,
-                               const void* offsets, int groups, int rows, int N, int K, int act, const void* gate, int gate_ld, int dtype, int general,
+                               const void* offsets, int groups, int rows, int x_rows, int N, int K, int act, const void* gate, int gate_ld, int dtype, int general,
                                hipStream_t stream) {
-    TL_REQUIRE(groups > 0 && rows >= 0 && N > 0 && K > 0 && a_ld > 0 && out_ld > 0, "grouped_gemm: bad sizes");
+    TL_REQUIRE(groups > 0 && rows >= 0 && x_rows >= 0 && N > 0 && K > 0 && a_ld > 0 && out_ld > 0, "grouped_gemm: bad sizes");
     TL_REQUIRE(known_activation(act), "grouped_gemm: unknown activation %d", act);
     TL_REQUIRE(!(act & ACT_PAIRS) || (N % 2 == 0 && out_group == 0), "grouped_gemm: an activation in pairs needs an even number of columns");
     TL_REQUIRE(!gate || (!offsets && act == ACT_NONE && gate_ld >= (groups - 1) * out_group + N), "grouped_gemm: a gate stands beside groups of equal rows, with a number per output column");
@@ -417,7 +417,7 @@ extern "C" int tl_grouped_gemm(const void* a, int a_ld, int a_group, const void*
     dim3 grid(offsets ? (rows + GG_T - 1) / GG_T + groups : (rows + GG_T - 1) / GG_T, (N + GG_T - 1) / GG_T, offsets ? 1 : groups), block(256);
     const bool aligned = K % 32 == 0 && a_ld % 8 == 0 && a_group % 8 == 0 && ((uintptr_t)a % 16) == 0 && ((uintptr_t)w % 16) == 0 &&
                          ((uintptr_t)out % 8) == 0;
-    const ExpertsCall experts{(const bf16_t*)a, a_ld, (const int*)src, (const bf16_t*)w, (bf16_t*)out, out_ld, (const int*)offsets, groups, rows, N, K, act};
+    const ExpertsCall experts{(const bf16_t*)a, a_ld, (const int*)src, (const bf16_t*)w, (bf16_t*)out, out_ld, (const int*)offsets, groups, rows, x_rows, N, K, act};
     if (dtype == TL_DT_BF16 && offsets && !general && experts_fit(experts)) return launch_experts(pick_experts(experts), experts, stream);
     if (dtype == TL_DT_BF16 && aligned && !general && !offsets && act == ACT_NONE && heads_few_rows(rows, groups, N, K)) {
         const HeadColumns heads{a_group, out_group, rows, (const bf16_t*)gate, gate_ld};

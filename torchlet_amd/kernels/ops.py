@@ -1754,7 +1754,7 @@ def heads_linear(x: torch.Tensor, x_head: int, weight: torch.Tensor, out: torch.
         raise KernelError("heads_linear: shapes or dtypes do not fit")
     lib = _lib("experts")
     _check(lib, lib.tl_grouped_gemm(_ptr(x), c_int(x.stride(0)), c_int(x_head), c_void_p(0), _ptr(weight), _ptr(out), c_int(out.stride(0)),
-                                    c_int(out_head), c_void_p(0), c_int(G), c_int(T), c_int(N), c_int(K), c_int(0), _ptr(gate),
+                                    c_int(out_head), c_void_p(0), c_int(G), c_int(T), c_int(T), c_int(N), c_int(K), c_int(0), _ptr(gate),
                                     c_int(gate.stride(0) if gate is not None else 0), c_int(_dt(x, "heads_linear")), c_int(1 if general else 0), _stream()))
 
 
@@ -1774,7 +1774,7 @@ def experts_linear(x: torch.Tensor, slot_token: torch.Tensor | None, weight: tor
     _i32(slot_token, "slot_token", S)
     lib = _lib("experts")
     _check(lib, lib.tl_grouped_gemm(_ptr(x), c_int(x.stride(0)), c_int(0), _ptr(slot_token), _ptr(weight), _ptr(out), c_int(out.shape[1]), c_int(0),
-                                    _ptr(offsets), c_int(G), c_int(S), c_int(N), c_int(K), c_int(ACTIVATIONS[activation]), c_void_p(0), c_int(0),
+                                    _ptr(offsets), c_int(G), c_int(S), c_int(x.shape[0]), c_int(N), c_int(K), c_int(ACTIVATIONS[activation]), c_void_p(0), c_int(0),
                                     c_int(_dt(x, "experts_linear")), c_int(1 if general else 0), _stream()))
 
 
@@ -1791,7 +1791,7 @@ def experts_linear_variant(x: torch.Tensor, slot_token: torch.Tensor | None, wei
     _i32(slot_token, "slot_token", S)
     lib = _lib("experts")
     _check(lib, lib.tl_experts_variant(_ptr(x), c_int(x.stride(0)), _ptr(slot_token), _ptr(weight), _ptr(out), c_int(out.shape[1]), _ptr(offsets), c_int(G),
-                                       c_int(S), c_int(N), c_int(K), c_int(ACTIVATIONS[activation]), c_int(which), _stream()))
+                                       c_int(S), c_int(x.shape[0]), c_int(N), c_int(K), c_int(ACTIVATIONS[activation]), c_int(which), _stream()))
 
 
 ROUTER_SCORES = {"chosen": 0, "all": 1, "sigmoid": 2}
