@@ -1028,7 +1028,7 @@ extern "C" int tl_local_attention_tiles(const void* q, int q_ld, void* out, int 
         if (dim == 192) TL_LP(192, 128, 32, 3); else if (dim == 128) TL_LP(128, 128, 64, 2); else TL_LP(64, 64, 64, 2);
 #undef TL_LP
         if (rc != TL_OK) return rc;
-        if (requests == 1) return TL_OK;
+        if (requests == 1 && (tiles - 1) * LAM_TOKENS + 1 >= LP_LEAST) return TL_OK;      // (its tiles show that it is a long one)
         below = LP_LEAST;
     }
 #define TL_LAM(DK, DV)                                                                                                                      \
