@@ -537,16 +537,16 @@ extern "C" int tl_local_attention_mfma_fits(int dim, int vdim, int page_size) {
 // Both products run transposed on v_mfma_f32_32x32x16_bf16: a lane owns one row (its maximum, sum and output), and the keys are dealt to the
 // rows of the first product so that the weights a lane holds are the second product's operand as they stand (row 8 a + 4 h + b of a block of 32
 // carries key 16 (a / 2) + 8 h + 4 (a % 2) + b).  The tile kernel above reads its operands from the caches for every 16 tokens of every head, and that
-// traffic set its time; here 128 rows share them, and the matrix and vector units take turns at being the bound (0.8 PFLOP/s on long prompts).
-// Measured against it, 32 heads of 128 over 8: a prompt of 4096 tokens 918 -> 172 us, 2048 305 -> 58, with a window of 512 181 -> 36; 64 heads of
-// 192 / 128, 2048 tokens 817 -> 123.
+// traffic set its time; here 128 rows share them, and the matrix and vector units take turns at being the bound (0.77 PFLOP/s on long prompts).
+// Measured against it, 32 heads of 128 over 8: a prompt of 4096 tokens 918 -> 178 us, 2048 305 -> 60, with a window of 512 181 -> 39; 64 heads of
+// 192 / 128, 2048 tokens 817 -> 130.
 // A tile takes up to three stretches of keys one after the other, each with limits of its own per row: the pooled blocks before the window, the
 // kept first tokens, the tokens themselves.  Late tiles start first.
 #define LP_ROWS 128
 #define LP_BT_MAX 2048               // block-table entries of a stretch in shared memory
 #define LP_LEAST 32                  // tokens of a request in a step
 #define LP_HEADS_MOST 16             // heads of a tile
-#define LP_SLACK 8.f                 // powers of two a row's scores may rise above its reference before it is moved
+#define LP_DEEP 12.f                 // powers of two a step's reference may lie under the largest score so far
 
 typedef float la_f32x16 __attribute__((ext_vector_type(16)));
 
@@ -691,7 +691,7 @@ local_prompt_kernel(LocalArgs a) {
 
     // scores in units of log 2: with a cap they are capped first and then stand as they are, without one the factor goes into the exponent
     const float inv_cap = CAP ? 2.f * LA_LOG2E / a.cap : 0.f, scale2 = CAP ? 1.f : a.scale * LA_LOG2E;
-    float m = -INFINITY, l = 0.f;
+    float m = -INFINITY, top = -INFINITY, l = 0.f;      // m: the reference of l and acc; top: the largest score so far
     la_f32x16 acc[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b)
@@ -842,10 +842,13 @@ local_prompt_kernel(LocalArgs a) {
                     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(mloc), __float_as_uint(mloc), false, false);
                     mloc = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])) * scale2;
                 }
-                // m is the row's reference for the exponents, not its maximum: it moves only when some row of the wave rises more than LP_SLACK above
-                // its own, so most steps rescale nothing; the quotient at the end is the same
-                if (__any(mloc > m + LP_SLACK)) {
-                    const float m_new = fmaxf(m, mloc);
+                // The weights' rounding to bfloat16 is the largest error here, and it is least for those at and next below 1, so a step's weights are taken from the
+                // step's own maximum (no more than LP_DEEP powers of two under the row's), and what stands in the sums is brought to that reference.  Error of the
+                // output against 64 bits, 2048 tokens after 2000: 2.09e-3; 2.20e-3 in the tile kernel above, whose waves have a maximum each; 2.26e-3 with the row's running
+                // maximum, and 2.34e-3 where the reference moved only when a row had risen by eight powers of two, which took 2 to 8 % less time.
+                top = fmaxf(top, mloc);
+                {
+                    const float m_new = fmaxf(mloc, top - LP_DEEP);
                     const float alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - m_new);
                     m = m_new;
                     l *= alpha;
@@ -953,7 +956,7 @@ static int launch_local_prompt(const LocalArgs& a, long tiles, hipStream_t strea
 
 // From where the kernel of 128 rows is the faster one: three of the tile kernel's work-groups (16 tokens of a head) to a CU.  That kernel deals a
 // tile's keys to four waves and so fills the chip with few tokens already: with 32 heads over 8, 4000 cached tokens, 128 new ones take 55 us in it and
-// 83 us here, 256 take 110 / 87, 512 take 206 / 94; 256 new ones beside 31 decoded tokens at 2000, where both kernels run, 189 / 207.  Tokens that
+// 83 us here, 256 take 110 / 87, 512 take 206 / 98; 256 new ones beside 31 decoded tokens at 2000, where both kernels run, 189 / 207.  Tokens that
 // must be decoded ones (all requests' but one each) do not count; a request of LP_LEAST tokens is where a step may hold no decoded ones at all
 // (8 x 32 tokens of 64 heads after 1000: 94 / 54 us; below, most of a tile's rows would be empty).
 static bool local_prompt_pays(const LocalArgs& a, long tokens) {
