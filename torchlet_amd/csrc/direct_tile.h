@@ -127,8 +127,7 @@ __device__ __forceinline__ void store_expert_tile(const f32x16_t (&acc)[FM][FN],
 // N, K]; `src` (optional) maps an output row to the row of x it reads.  How many rows a group has is known on the GPU alone, so the grid is an
 // upper bound: a work-group adds up the groups' tiles, finds its own among them and ends at once if there is none.  The tiles of a group follow
 // each other, those that read the same weight rows side by side, and each XCD gets a stretch of them, so a group's matrix passes through one L2.
-// Measured at 4096 slots, 16 experts, 2048 x 1024 each, against a kernel whose waves fetch their operands from memory into registers: see
-// tl_experts_gemm.
+// Measured against a kernel whose waves fetch their operands from memory into registers: see pick_experts.
 template <bool PAIRS_>
 struct ExpertRows {
     static constexpr bool PAIRS = PAIRS_;      // the activation joins the columns 2i and 2i + 1 into one output column

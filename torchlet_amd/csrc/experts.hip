@@ -390,7 +390,7 @@ static bool experts_fit(const ExpertsCall& c) {
            256L * c.K * 2 < (1L << 31) && (long)(c.rows / 16 + c.groups) <= 65535;
 }
 
-// One named kernel of the two (tests cover each; tuning times them).
+// One kernel of ExpertsKernel by its number (tests cover each; tuning times them).
 extern "C" int tl_experts_variant(const void* a, int a_ld, const void* src, const void* w, void* out, int out_ld, const void* offsets, int groups, int rows,
                                   int x_rows, int N, int K, int act, int which, hipStream_t stream) {
     const ExpertsCall c{(const bf16_t*)a, a_ld, (const int*)src, (const bf16_t*)w, (bf16_t*)out, out_ld, (const int*)offsets, groups, rows, x_rows, N, K, act};

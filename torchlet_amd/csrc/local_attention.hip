@@ -973,11 +973,11 @@ static bool local_prompt_fits(const LocalArgs& a, int dim, int vdim, int pages, 
            a.pool_table_width <= LP_BT_MAX && a.scale > 0.f && !(a.back.freq && a.back.halves) && a.out_ld % 4 == 0 && ((uintptr_t)a.out % 8) == 0;
 }
 
-// Tiles of up to 16 consecutive tokens of one request: tile i belongs to request tile_req[i] (null: request i) and starts at that
-// request's token tile_tok0[i] of the step (null: 0).
 // Whether decoded tokens' heads go together (HEADS) at these sizes.
 extern "C" int tl_local_heads_fits(int dim, int vdim) { return (dim == 64 || dim == 128 || dim == 192) && (vdim == 64 || vdim == 128); }
 
+// Tiles of up to 16 consecutive tokens of one request: tile i belongs to request tile_req[i] (null: request i) and starts at that
+// request's token tile_tok0[i] of the step (null: 0).
 extern "C" int tl_local_attention_tiles(const void* q, int q_ld, void* out, int out_ld, const void* k_plane, const void* v_plane, int pages,
                                         const void* block_table, int table_ld, int table_width, const void* req_indptr, const void* ctx_lens,
                                         const void* tile_req, const void* tile_tok0, int tiles, int heads, int kv_heads, int dim, int vdim,

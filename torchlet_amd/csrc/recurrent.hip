@@ -529,7 +529,8 @@ extern "C" int tl_delta_prepare(const void* proj, int ld, const void* conv_w, vo
 // by dim alone) of it in registers for all tokens of the step, so the lanes' pieces of q and k lie side by side in shared memory and those of
 // the state side by side in memory ([vdim][dim] per head), and they add their sums with four exchanges inside the row (pairs, quads, halves,
 // the row: every lane gets the same bits).  k . q, which all columns share, is made once a token.  The order of every sum is fixed by dim, so a
-// token's result depends neither on how its request was cut into steps nor on what else the step holds.  A wave has 4 CPL columns, a work-group
+// token's result in this loop depends neither on how its request was cut into steps nor on what else the step holds (fixed decays leave it for long portions: see the
+// chunks below).  A wave has 4 CPL columns, a work-group
 // of four waves 16 CPL.  Tokens are taken TB at a time (1, 4 or 16, by the longest portion of the step): their q, k, v, beta and g are fetched
 // into registers one batch ahead, as whole pieces of four where the rows allow it, and go to shared memory; a request's last batch is filled up
 // with tokens that change nothing (k = 0, beta = 0, decay 1), so the loop has no branch.
@@ -1147,7 +1148,7 @@ extern "C" int tl_wkv_scan(const void* rkv, int ld, int k_off, int v_off, const 
 }
 
 // ------------------------------------------------------------------ long portions in chunks: recurrences with one decay per head and token
-// S <- g S + b k v^T, o = S^T q (the matrix memory; the decayed linear attention; the selective recurrence) over the tokens of a long portion.
+// S <- g S + b k v^T, o = S^T q (the matrix memory; the decayed linear attention) over the tokens of a long portion.
 // Token by token the work of a head is a chain that a few compute units walk (four heads of 256 x 512 over 2048 tokens: 1.2 ms, a prompt's
 // largest item; in chunks 0.17); cut into chunks of 64 tokens nearly all of it is products of matrices that every chunk can take at once:
 //   chunk_states:  D_c = sum_j w_j v_j k_j^T with w_j = b_j prod_{l > j} g_l, and the chunk's decay G_c = prod g;     (all chunks at once)
@@ -1165,12 +1166,12 @@ extern "C" int tl_wkv_scan(const void* rkv, int ld, int k_off, int v_off, const 
 typedef float ck_f32x16 __attribute__((ext_vector_type(16)));
 
 struct ChunkArgs {
-    const void* qkv;            // a token's row: ld numbers; queries of head h from column q_off + qk(h) * dim on, keys from k_off, values from v_off + h * vdim
-    int ld, q_off, k_off, v_off, heads, qk_share;      // qk(h) = h / qk_share
+    const void* qkv;            // a token's row: ld numbers; queries of head h from column h * dim on, keys from k_off + h * dim, values from v_off + h * vdim
+    int ld, k_off, v_off, heads;
     int dim, vdim;
     const float* gates;         // [tokens][gate_ld]: b at column h * gate_step + b_at, g at h * gate_step + g_at; null: b = 1, g = head_decay[h]
     int gate_ld, gate_step, b_at, g_at;
-    const float* head_decay;    // fixed decays, or the skip factors
+    const float* head_decay;    // fixed decays
     float qscale, denom_eps;
     float* state;
     size_t slot_stride;
@@ -1208,9 +1209,8 @@ __device__ __forceinline__ int ck_find(const ChunkArgs& a, int want, int& first_
 
 template <typename T> __device__ __forceinline__ float4 ck_load4(const T* p) { return wkv_load4<T>(p); }
 
-// MODE 0: fixed decays.  MODE 3: the matrix memory (b, g and the running maximum per
-// token; outputs over max(|n . q|, exp(-m)) + denom_eps).
-template <typename T, int MODE>
+// MEMORY: the matrix memory (b, g and the running maximum per token; outputs over max(|n . q|, exp(-m)) + denom_eps); otherwise fixed decays.
+template <typename T, bool MEMORY>
 __global__ void __launch_bounds__(256)
 chunk_states_kernel(ChunkArgs a) {
     __shared__ __attribute__((aligned(16))) float sk[CK_T * CK_LD], sv[CK_T * CK_LV];
@@ -1225,7 +1225,7 @@ chunk_states_kernel(ChunkArgs a) {
     if (wave == 0) {                                   // the tokens' weights: a product over the tokens behind them, taken from the back
         float b = 0.f, g = 1.f;
         if (lane < nt) {
-            if (MODE == 0) { b = 1.f; g = a.head_decay[head]; }
+            if (!MEMORY) { b = 1.f; g = a.head_decay[head]; }
             else {
                 const float* row = a.gates + (size_t)(tok0 + lane) * a.gate_ld + head * a.gate_step;
                 b = row[a.b_at];
@@ -1256,7 +1256,7 @@ chunk_states_kernel(ChunkArgs a) {
         }
         *(float4*)(sv + t * CK_LV + c) = x;
     }
-    const T* ksrc = base + a.k_off + head / a.qk_share * a.dim;
+    const T* ksrc = base + a.k_off + head * a.dim;
     float* dst = a.states + ((size_t)chunk * a.heads + head) * a.vdim * a.dim;
     for (int d0 = 0; d0 < a.dim; d0 += CK_D) {
         if (d0 > 0) __syncthreads();
@@ -1288,7 +1288,7 @@ chunk_states_kernel(ChunkArgs a) {
                     if (v < a.vdim && d < a.dim) dst[(size_t)v * a.dim + d] = acc[n][i];
                 }
         }
-        if (MODE == 3 && blockIdx.z == 0) {            // the keys' own weighted sum (the memory's column of ones)
+        if (MEMORY && blockIdx.z == 0) {            // the keys' own weighted sum (the memory's column of ones)
             const int d = tid % CK_D, part = tid / CK_D;
             float s = 0.f;
 #pragma unroll
@@ -1399,7 +1399,7 @@ chunk_pass_kernel(ChunkArgs a) {
     }
 }
 
-template <typename T, int MODE>
+template <typename T, bool MEMORY>
 __global__ void __launch_bounds__(256, 2)
 chunk_outputs_kernel(ChunkArgs a) {
     extern __shared__ __attribute__((aligned(16))) float ck_smem[];
@@ -1420,7 +1420,7 @@ chunk_outputs_kernel(ChunkArgs a) {
     if (wave == 0) {
         float b = 0.f, g = 1.f;
         if (lane < nt) {
-            if (MODE == 0) { b = 1.f; g = a.head_decay[head]; }
+            if (!MEMORY) { b = 1.f; g = a.head_decay[head]; }
             else {
                 const float* row = a.gates + (size_t)(tok0 + lane) * a.gate_ld + head * a.gate_step;
                 b = row[a.b_at];
@@ -1435,10 +1435,10 @@ chunk_outputs_kernel(ChunkArgs a) {
         }
         sg[lane] = g; sg[CK_T + lane] = b; sg[2 * CK_T + lane] = (float)p;
     }
-    if (MODE == 3 && tid / 4 < nt) m_mine = a.gates[(size_t)(tok0 + tid / 4) * a.gate_ld + head * a.gate_step + 2];
+    if (MEMORY && tid / 4 < nt) m_mine = a.gates[(size_t)(tok0 + tid / 4) * a.gate_ld + head * a.gate_step + 2];
     const T* base = (const T*)a.qkv + (size_t)tok0 * a.ld;
-    const T* qsrc = base + a.q_off + head / a.qk_share * a.dim;
-    const T* ksrc = base + a.k_off + head / a.qk_share * a.dim;
+    const T* qsrc = base + head * a.dim;
+    const T* ksrc = base + a.k_off + head * a.dim;
     const T* vsrc = base + a.v_off + head * a.vdim + v0;
     const float* src = a.states + ((size_t)chunk * a.heads + head) * a.vdim * a.dim;
     const float* nsrc = a.sums + ((size_t)chunk * a.heads + head) * a.dim;
@@ -1468,9 +1468,9 @@ chunk_outputs_kernel(ChunkArgs a) {
             const int idx = tid + j * 256, v = idx / (CK_D / 4), c = (idx % (CK_D / 4)) * 4;
             *(float4*)(ss + v * CK_LD + c) = v0 + v < a.vdim && d0 + c < a.dim ? *(const float4*)(src + (size_t)(v0 + v) * a.dim + d0 + c) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
-        if (MODE == 3 && tid < CK_D) sg[4 * CK_T + tid] = d0 + tid < a.dim ? nsrc[d0 + tid] : 0.f;
+        if (MEMORY && tid < CK_D) sg[4 * CK_T + tid] = d0 + tid < a.dim ? nsrc[d0 + tid] : 0.f;
         __syncthreads();
-        if (MODE == 3) {
+        if (MEMORY) {
             const float* qr = sq + (tid / 4) * CK_LD + 16 * (tid % 4);
 #pragma unroll
             for (int e = 0; e < 16; ++e) qn = fmaf(qr[e], sg[4 * CK_T + 16 * (tid % 4) + e], qn);
@@ -1529,7 +1529,7 @@ chunk_outputs_kernel(ChunkArgs a) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[0][i] = o[1][i] = o1[i] = 0.f;
     __syncthreads();
-    if (MODE == 3) {
+    if (MEMORY) {
         // n . q after every token: the state's share and the chunk's, four lanes a token
         const float* w = sq + (tid / 4) * CK_LD + 16 * (tid % 4);
         float rs = 0.f;
@@ -1585,7 +1585,7 @@ chunk_outputs_kernel(ChunkArgs a) {
             const int row = 32 * n + 8 * (i / 4) + 4 * half + i % 4;
             if (row >= nt || v >= a.vdim) continue;
             float y = fmaf(sg[2 * CK_T + row], so[n][i], o[n][i]);
-            if (MODE == 3) y /= sg[3 * CK_T + row];
+            if (MEMORY) y /= sg[3 * CK_T + row];
             a.out[((size_t)(tok0 + row) * a.heads + head) * a.vdim + v] = y;
         }
 }
@@ -1598,26 +1598,26 @@ struct ChunkPlan {
     long floats;
 };
 
-template <typename T, int MODE>
+template <typename T, bool MEMORY>
 static int launch_chunks(ChunkArgs a, const ChunkPlan& p, int longest, hipStream_t stream) {
-    const size_t per_chunk = (size_t)a.heads * ((size_t)a.vdim * a.dim + (MODE == 3 ? a.dim : 0) + 1);
+    const size_t per_chunk = (size_t)a.heads * ((size_t)a.vdim * a.dim + (MEMORY ? a.dim : 0) + 1);
     TL_REQUIRE(p.segment > 0 && p.segment % CK_T == 0 && p.grid > 0 && p.floats >= (long)(p.grid * per_chunk), "chunked scan: scratch of %ld numbers does not hold %d chunks", p.floats, p.grid);
     const int chunks = p.grid;
     float* scratch = p.scratch;
     a.seg_len = p.segment;
     a.states = scratch;
     a.sums = scratch + (size_t)chunks * a.heads * a.vdim * a.dim;
-    a.decays = a.sums + (MODE == 3 ? (size_t)chunks * a.heads * a.dim : 0);
+    a.decays = a.sums + (MEMORY ? (size_t)chunks * a.heads * a.dim : 0);
     constexpr size_t smem = sizeof(float) * (2 * CK_T * CK_LD + CK_V * CK_LD + 5 * CK_T + 4);
-    auto outputs = chunk_outputs_kernel<T, MODE>;
+    auto outputs = chunk_outputs_kernel<T, MEMORY>;
     static hipError_t allowed = hipFuncSetAttribute((const void*)outputs, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     if (allowed != hipSuccess) { tl_set_error("chunked scan: cannot get %zu bytes of shared memory: %s", smem, hipGetErrorString(allowed)); return TL_ERR_HIP; }
     const dim3 grid(chunks, a.heads, (a.vdim + CK_V - 1) / CK_V);
-    const dim3 pass(MODE == 3 ? (a.dim + 31) / 32 * ((a.vdim + 31) / 32) + 1 : (a.vdim * a.dim / 4 + 255) / 256, a.heads, a.requests);
+    const dim3 pass(MEMORY ? (a.dim + 31) / 32 * ((a.vdim + 31) / 32) + 1 : (a.vdim * a.dim / 4 + 255) / 256, a.heads, a.requests);
     for (a.seg0 = 0; a.seg0 < longest; a.seg0 += a.seg_len) {
-        chunk_states_kernel<T, MODE><<<grid, 256, 0, stream>>>(a);
+        chunk_states_kernel<T, MEMORY><<<grid, 256, 0, stream>>>(a);
         TL_CHECK_LAUNCH("chunk_states");
-        chunk_pass_kernel<MODE == 3><<<pass, 256, 0, stream>>>(a);
+        chunk_pass_kernel<MEMORY><<<pass, 256, 0, stream>>>(a);
         TL_CHECK_LAUNCH("chunk_pass");
         outputs<<<grid, 256, smem, stream>>>(a);
         TL_CHECK_LAUNCH("chunk_outputs");
@@ -1684,8 +1684,8 @@ extern "C" int tl_chunks_pay(int memory, int count, int tokens, int chunks, int 
 }
 
 // Whether the chunks can be read in whole pieces of four numbers.
-static bool chunks_fit(const void* qkv, int ld, int q_off, int k_off, int v_off, int dim, int vdim, const void* state, long slot_stride, bool columns) {
-    return dim % 4 == 0 && vdim % 4 == 0 && ld % 4 == 0 && q_off % 4 == 0 && k_off % 4 == 0 && v_off % 4 == 0 && ((uintptr_t)qkv & 15) == 0 &&
+static bool chunks_fit(const void* qkv, int ld, int k_off, int v_off, int dim, int vdim, const void* state, long slot_stride, bool columns) {
+    return dim % 4 == 0 && vdim % 4 == 0 && ld % 4 == 0 && k_off % 4 == 0 && v_off % 4 == 0 && ((uintptr_t)qkv & 15) == 0 &&
            (!columns || (((uintptr_t)state & 15) == 0 && slot_stride % 4 == 0));
 }
 
@@ -1705,16 +1705,16 @@ extern "C" int tl_mlstm_scan(const void* qkv, int ld, int k_off, int v_off, cons
     TL_REQUIRE(slot_stride >= (long)heads * ((long)dim * vdim + dim + 1), "mlstm_scan: the state rows are too short");
     TL_REQUIRE(dtype == TL_DT_F32 || dtype == TL_DT_BF16, "mlstm_scan: unknown dtype %d", dtype);
     if (requests == 0) return TL_OK;
-    const bool chunks = scratch && longest >= least && chunks_fit(qkv, ld, 0, k_off, v_off, dim, vdim, state, slot_stride, false);
+    const bool chunks = scratch && longest >= least && chunks_fit(qkv, ld, k_off, v_off, dim, vdim, state, slot_stride, false);
     if (chunks) {
         float4* factors = (float4*)((float*)scratch + scratch_floats);
         mlstm_gates_kernel<<<dim3(heads, requests), 64, 0, stream>>>((const float*)gates, (const float*)state, (size_t)slot_stride, (const int*)slots,
                                                                      (const int*)req_indptr, factors, heads, dim, vdim, cap, least);
         TL_CHECK_LAUNCH("mlstm_gates");
-        const ChunkArgs a{qkv, ld, 0, k_off, v_off, heads, 1, dim, vdim, (const float*)factors, 4 * heads, 4, 1, 0, nullptr, qscale, denom_eps, (float*)state,
+        const ChunkArgs a{qkv, ld, k_off, v_off, heads, dim, vdim, (const float*)factors, 4 * heads, 4, 1, 0, nullptr, qscale, denom_eps, (float*)state,
                           (size_t)slot_stride, (const int*)slots, (const int*)req_indptr, (float*)out, nullptr, nullptr, nullptr, requests, least, 0, 0};
         const ChunkPlan plan{segment, chunk_grid, (float*)scratch, scratch_floats};
-        const int rc = dtype == TL_DT_F32 ? launch_chunks<float, 3>(a, plan, longest, stream) : launch_chunks<bf16_t, 3>(a, plan, longest, stream);
+        const int rc = dtype == TL_DT_F32 ? launch_chunks<float, true>(a, plan, longest, stream) : launch_chunks<bf16_t, true>(a, plan, longest, stream);
         if (rc != TL_OK || rest == 0) return rc;
     }
     return mlstm_token_loop(qkv, ld, k_off, v_off, gates, state, slot_stride, slots, before, req_indptr, out, requests, heads, dim, vdim, cap, qscale, denom_eps,
@@ -1732,9 +1732,9 @@ extern "C" int tl_decay_scan(const void* qkv, const void* decay, void* state, lo
     TL_REQUIRE(slot_stride >= (long)heads * dim * vdim, "decay_scan: the state rows are too short");
     TL_REQUIRE(requests <= 65535 && heads <= 65535, "decay_scan: too many requests or heads for one launch");
     if (requests == 0) return TL_OK;
-    const bool chunks = scratch && longest >= least && chunks_fit(qkv, 2 * heads * dim + heads * vdim, 0, 0, 0, dim, vdim, state, slot_stride, true);
+    const bool chunks = scratch && longest >= least && chunks_fit(qkv, 2 * heads * dim + heads * vdim, 0, 0, dim, vdim, state, slot_stride, true);
     if (chunks) {
-        const int rc = launch_chunks<float, 0>(ChunkArgs{qkv, 2 * heads * dim + heads * vdim, 0, heads * dim, 2 * heads * dim, heads, 1, dim, vdim, nullptr, 0, 0, 0, 0,
+        const int rc = launch_chunks<float, false>(ChunkArgs{qkv, 2 * heads * dim + heads * vdim, heads * dim, 2 * heads * dim, heads, dim, vdim, nullptr, 0, 0, 0, 0,
             (const float*)decay, 1.f, 0.f, (float*)state, (size_t)slot_stride, (const int*)slots, (const int*)req_indptr, (float*)out, nullptr, nullptr, nullptr,
             requests, least, 0, 0}, ChunkPlan{segment, chunk_grid, (float*)scratch, scratch_floats}, longest, stream);
         if (rc != TL_OK || rest == 0) return rc;

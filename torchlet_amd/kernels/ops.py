@@ -956,7 +956,7 @@ def scaled_add_rmsnorm(residual: torch.Tensor, pending: torch.Tensor | None, alp
 
 # Portions of at least so many tokens go through chunks of 64 tokens in the recurrences with one decay per head and token (the matrix memory, fixed
 # decays), where a step's sizes make that the faster way; the chunks' states stand in scratch of at most so many 32-bit numbers (256 MiB), and tokens
-# beyond wait for another pass over it.
+# beyond wait for another pass over it; where one chunk of every portion does not fit, the token loop takes them.
 CHUNKED_FROM = 32
 CHUNK_SCRATCH = 1 << 26
 
@@ -1654,7 +1654,9 @@ def latent_attention(q: torch.Tensor, out: torch.Tensor, plane: torch.Tensor, bl
                                         c_int(window), _ptr(gate), c_int(gate.stride(0) if gate is not None else 0), _stream()))
 
 
-PROMPT_ROWS_SCRATCH_BYTES = 512 << 20     # keys and values of a group of heads that a step may hold beside the cache
+# Projected keys and values of a group of heads that a step may hold beside the cache (the cached rows side by side, one for all heads, come on top: 1.2 GB at the most
+# rows that leave room for one head of 128 + 128 numbers).
+PROMPT_ROWS_SCRATCH_BYTES = 512 << 20
 
 
 def prompt_rows_fits(dtype: torch.dtype, own: int, shared: int, vdim: int) -> bool:
