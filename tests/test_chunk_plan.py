@@ -41,4 +41,5 @@ def test_portions_that_do_not_fit_or_are_none_leave_it_to_the_token_loop(lens):
 @pytest.mark.parametrize("lens", [[65, 0], [0, 300, 1], [32] * 5, [31] * 9, [1, 200, 64], [20]])
 def test_bounds_hold_what_there_is(lens):
     exact, bound = ops.Portions.of(lens, 32), ops.Portions.bound(sum(lens), len(lens), None, 32)
-    assert all(b >= e for b, e in zip(bound[:5], exact[:5])) and bound.rest_longest >= min(exact.rest_longest, 31)
+    assert all(b >= e for b, e in zip(bound[:4], exact[:4])) or bound.count == 0
+    assert bound.rest >= exact.rest and bound.rest_longest >= min(exact.rest_longest, 31)

@@ -64,6 +64,21 @@ def test_a_request_shorter_than_the_bound_is_not_left_out(monkeypatch, memory, l
 
 
 @pytest.mark.parametrize("memory", [True, False])
+@pytest.mark.parametrize("most", [1, 40, 64, 1000])
+def test_a_request_longer_than_was_said_is_taken_whole(monkeypatch, memory, most):
+    _pays(monkeypatch)
+    step = _Step(memory, [150, 3])
+    out, state = step.run(max_new_tokens=most)
+    for r, rows in enumerate((slice(0, 150), slice(150, 153))):
+        want, left = step.alone(r)
+        # (by the loop or by the chunks: 150 terms of like size, each rounding at most 2^-24 of a partial sum, on either way; the memory's outputs are quotients, whose
+        # denominators may be small: its states show that every token was taken)
+        assert float((state[r] - left[0]).norm()) <= 300 * 2.0 ** -24 * float(left.norm()) and bool(torch.isfinite(out[rows]).all())
+        if not memory:
+            assert float((out[rows] - want).norm()) <= 300 * 2.0 ** -24 * float(want.norm())
+
+
+@pytest.mark.parametrize("memory", [True, False])
 @pytest.mark.parametrize("where", ["query", "key", "value", "input gate"])
 @pytest.mark.parametrize("token", [0, 5, 40, 63, 64, 100])
 def test_infinities_and_nans_do_not_reach_the_tokens_before_them(monkeypatch, memory, where, token):

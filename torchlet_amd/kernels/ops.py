@@ -971,6 +971,7 @@ class Portions(NamedTuple):
     rest: int
     rest_tokens: int
     rest_longest: int
+    likely: int = 0             # where `longest` is a bound: the most tokens that a request will have brought
 
     @classmethod
     def of(cls, lengths, least: int) -> "Portions":
@@ -979,14 +980,13 @@ class Portions(NamedTuple):
 
     @classmethod
     def bound(cls, tokens: int, requests: int, longest: int | None, least: int) -> "Portions":
-        """For callers that know their rows and requests alone, and maybe a bound on a request's tokens: no fewer of
-        anything than there are, or none for the chunks where there will hardly be any."""
+        """For callers that know their rows and requests alone, and maybe about how many tokens a request brings (``longest``): no fewer of anything than there are,
+        whatever ``longest`` says, or none for the chunks where there will hardly be any."""
         likely = tokens - requests + 1 if longest is None else longest      # (none of them empty)
-        longest = tokens if longest is None else longest
         if likely < least:
-            return cls(0, 0, 0, 0, requests, tokens, longest)
+            return cls(0, 0, 0, 0, requests, tokens, likely)
         count = min(requests, tokens // least)
-        return cls(count, tokens, tokens // 64 + count, longest, requests, 0, least - 1)
+        return cls(count, tokens, tokens // 64 + count, tokens, requests, 0, least - 1, min(likely, tokens))
 
 
 class _Chunks(NamedTuple):
@@ -1008,7 +1008,7 @@ def _chunk_scratch(lib, memory: bool, requests: int, heads: int, dim: int, vdim:
         return None
     each = longest if portions.chunks <= fit else min(longest, fit // portions.count)
     grid = min(portions.chunks, each * portions.count)
-    if not lib.tl_chunks_pay(*(c_int(x) for x in (1 if memory else 0, portions.count, portions.tokens, portions.chunks, -(-longest // each), portions.longest,
+    if not lib.tl_chunks_pay(*(c_int(x) for x in (1 if memory else 0, portions.count, portions.tokens, portions.chunks, -(-longest // each), portions.likely or portions.longest,
                                                   portions.rest, portions.rest_tokens, portions.rest_longest, requests, heads, dim, vdim))):
         return None
     floats = -(-grid * per_chunk // 4) * 4
@@ -1031,7 +1031,7 @@ def mlstm_scan(qkv: torch.Tensor, k_off: int, v_off: int, gates: torch.Tensor, s
     ``qkv [T, >=]`` holds per token the queries at column 0 (``heads * dim``), the keys at ``k_off`` and the values at
     ``v_off`` (``heads * vdim``); ``gates`` float32 ``[T, 2 * heads]`` the raw input and forget gates (bias added);
     ``state`` float32 ``[slots, heads, dim * vdim + dim + 1]`` (S, n, m per head) is updated in place; ``out`` float32
-    ``[T, heads * vdim]`` receives ``S^T q / (max(|n.q|, exp(-m)) + denom_eps)``.  ``max_new_tokens``: no fewer tokens than any request brings; ``portions``
+    ``[T, heads * vdim]`` receives ``S^T q / (max(|n.q|, exp(-m)) + denom_eps)``.  ``max_new_tokens``: about the most tokens that a request brings; ``portions``
     (of :data:`CHUNKED_FROM` tokens or more): what the host knows of the requests' lengths, exactly."""
     T = qkv.shape[0]
     R = req_indptr.numel() - 1
@@ -1150,7 +1150,7 @@ def decay_scan(qkv: torch.Tensor, decay: torch.Tensor, state: torch.Tensor, slot
     """Linear attention with one fixed decay per head over the step's tokens, request by request from the state its slot holds: ``qkv``
     float32 ``[T, 2 * heads * dim + heads * vdim]`` (queries, keys, values, head by head), ``decay`` float32 ``[heads]``; head ``h`` of
     ``state[slot]`` (float32, laid out as :func:`delta_scan`'s) moves by ``S <- decay[h] S + k v^T`` and ``out`` float32 ``[T, heads * vdim]``
-    receives ``S^T q``.  ``max_new_tokens``: no fewer tokens than any request brings; ``portions`` (of :data:`CHUNKED_FROM` tokens or more): what
+    receives ``S^T q``.  ``max_new_tokens``: about the most tokens that a request brings; ``portions`` (of :data:`CHUNKED_FROM` tokens or more): what
     the host knows of the requests' lengths, exactly."""
     T = qkv.shape[0]
     R = req_indptr.numel() - 1
