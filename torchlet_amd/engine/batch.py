@@ -118,7 +118,10 @@ class StepContext:
 
     def tile_count(self, tq: int) -> int:
         """The number of tiles of ``tq`` tokens."""
-        return int((-(-self._host_new_lens // tq)).sum())
+        key = ("tiles", tq)
+        if key not in self._tiles:
+            self._tiles[key] = int((-(-self._host_new_lens // tq)).sum())
+        return self._tiles[key]
 
     def tiles_by_length(self, tq_short: int, tq_long: int, threshold: int):
         """Two tile lists: requests that bring fewer than ``threshold`` tokens in tiles of
