@@ -24,26 +24,6 @@ __global__ void embedding_kernel(const int* __restrict__ ids, const T* __restric
     }
 }
 
-extern "C" int tl_embedding(const void* ids, const void* table, int table_dtype, void* out,
-                            int tokens, int hidden, int vocab, float scale, const void* positions, const void* pos_table,
-                            int pos_dtype, int pos_rows, int copies, hipStream_t stream) {
-    TL_REQUIRE(tokens >= 0 && hidden > 0 && vocab > 0 && copies > 0, "embedding: bad sizes tokens=%d hidden=%d vocab=%d copies=%d", tokens, hidden, vocab, copies);
-    TL_REQUIRE(!pos_table || (positions && pos_rows > 0), "embedding: a position table needs positions and rows");
-    if (tokens == 0) return TL_OK;
-    dim3 grid(tokens), block(256);
-    const size_t copy_stride = (size_t)tokens * hidden;
-    const int pos_f32 = pos_dtype == TL_DT_F32;
-    if (table_dtype == TL_DT_F32)
-        embedding_kernel<float><<<grid, block, 0, stream>>>((const int*)ids, (const float*)table, (float*)out, hidden, vocab, scale,
-                                                            (const int*)positions, pos_table, pos_f32, pos_rows, copies, copy_stride);
-    else if (table_dtype == TL_DT_BF16)
-        embedding_kernel<bf16_t><<<grid, block, 0, stream>>>((const int*)ids, (const bf16_t*)table, (float*)out, hidden, vocab, scale,
-                                                             (const int*)positions, pos_table, pos_f32, pos_rows, copies, copy_stride);
-    else TL_REQUIRE(false, "embedding: unknown dtype %d", table_dtype);
-    TL_CHECK_LAUNCH("embedding");
-    return TL_OK;
-}
-
 // ------------------------------------------------------------------ add + RMSNorm
 // One block per output row.  r = residual[row] (+ pending[row]); if `update`, r is
 // written back to the residual; out = r * rsqrt(mean(r^2) + eps) * weight.
@@ -944,29 +924,6 @@ __global__ void last_token_kernel(const int* __restrict__ ids, const int* __rest
     if (b > a) last_token[slots[r]] = ids[b - 1];
 }
 
-extern "C" int tl_bigram_embedding(const void* ids, const void* table, void* out, int tokens, int hidden, int vocab, float scale,
-                                   const void* token_req, const void* req_indptr, int requests, const void* positions, const void* slots,
-                                   void* last_token, const void* bigram, int buckets, long mul_prev, long mul_cur, int copies, int dtype,
-                                   hipStream_t stream) {
-    TL_REQUIRE(tokens >= 0 && hidden > 0 && vocab > 0 && copies > 0 && buckets > 0 && requests >= 0, "bigram_embedding: bad sizes");
-    TL_REQUIRE(token_req && req_indptr && positions && slots && last_token && bigram, "bigram_embedding: a null operand");
-    if (tokens == 0) return TL_OK;
-    const size_t copy_stride = (size_t)tokens * hidden;
-    if (dtype == TL_DT_F32)
-        bigram_embedding_kernel<float><<<tokens, 256, 0, stream>>>((const int*)ids, (const float*)table, (float*)out, hidden, vocab, scale,
-            (const int*)token_req, (const int*)req_indptr, (const int*)positions, (const int*)slots, (const int*)last_token, (const float*)bigram,
-            buckets, mul_prev, mul_cur, copies, copy_stride);
-    else if (dtype == TL_DT_BF16)
-        bigram_embedding_kernel<bf16_t><<<tokens, 256, 0, stream>>>((const int*)ids, (const bf16_t*)table, (float*)out, hidden, vocab, scale,
-            (const int*)token_req, (const int*)req_indptr, (const int*)positions, (const int*)slots, (const int*)last_token, (const bf16_t*)bigram,
-            buckets, mul_prev, mul_cur, copies, copy_stride);
-    else TL_REQUIRE(false, "bigram_embedding: unknown dtype %d", dtype);
-    TL_CHECK_LAUNCH("bigram_embedding");
-    last_token_kernel<<<(requests + 63) / 64, 64, 0, stream>>>((const int*)ids, (const int*)req_indptr, (const int*)slots, (int*)last_token, requests);
-    TL_CHECK_LAUNCH("last_token");
-    return TL_OK;
-}
-
 // ------------------------------------------------------------------ rows in pieces of four numbers
 __device__ __forceinline__ float4 load4(const float* p) { return *(const float4*)p; }
 __device__ __forceinline__ float4 load4(const bf16_t* p) {
@@ -1061,6 +1018,170 @@ static RowPlan plan_row(int hidden) {
     const int n = hidden / 4;
     const int threads = n <= 64 ? 64 : n <= 128 ? 128 : n <= 256 ? 256 : n <= 512 ? 512 : 1024;
     return RowPlan{threads, (n + threads - 1) / threads};
+}
+
+// ------------------------------------------------------------------ embedding rows in pieces
+// The embedding kernels above with a row's pieces in registers: every fetch of a row (and of its position's or bigram's row) is requested before the first
+// is used, where the loops over single numbers paid a trip to memory each (a decode step of 4 rows: 2048 wide, four copies 8.2 -> 3.4 us; with a bigram row 8.8 -> 4.2, and 4.1 of its second launch; normed, 4096 wide,
+// 14.4 -> 4.0 us).
+template <typename T, int NP>
+__global__ void __launch_bounds__(1024)
+embedding_rows_kernel(const int* __restrict__ ids, const T* __restrict__ table, float* __restrict__ out, int hidden, int vocab, float scale,
+                      const int* __restrict__ positions, const void* __restrict__ pos_table, int pos_f32, int pos_rows, int copies, size_t copy_stride) {
+    const int t = blockIdx.x;
+    int id = ids[t], p = pos_table ? positions[t] : 0;
+    if (id < 0 || id >= vocab) id = 0;  // ids are checked on the host; never read out of bounds
+    if (p < 0 || p >= pos_rows) p = 0;
+    RowPieces<NP> r, e;
+    load_row<NP>(table + (size_t)id * hidden, hidden, r);
+    if (pos_table) {
+        if (pos_f32) load_row<NP>((const float*)pos_table + (size_t)p * hidden, hidden, e);
+        else load_row<NP>((const bf16_t*)pos_table + (size_t)p * hidden, hidden, e);
+    }
+#pragma unroll
+    for (int n = 0; n < NP; ++n)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            r.v[n][v] *= scale;
+            if (pos_table) r.v[n][v] += e.v[n][v];
+        }
+    for (int c = 0; c < copies; ++c) store_row<NP>(out + c * copy_stride + (size_t)t * hidden, hidden, r);
+}
+
+template <typename T, int NP>
+__global__ void __launch_bounds__(1024)
+embedding_norm_rows_kernel(const int* __restrict__ ids, const T* __restrict__ table, float* __restrict__ out, int hidden, int vocab,
+                           float scale, const float* __restrict__ weight, float eps) {
+    __shared__ float red[16];
+    const int t = blockIdx.x;
+    int id = ids[t];
+    if (id < 0 || id >= vocab) id = 0;
+    RowPieces<NP> r, w;
+    load_row<NP>(table + (size_t)id * hidden, hidden, r);
+    load_row<NP>(weight, hidden, w);
+#pragma unroll
+    for (int n = 0; n < NP; ++n)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) r.v[n][v] *= scale;
+    const float inv = rsqrtf(block_sum(row_squares(r), red) / (float)hidden + eps);
+#pragma unroll
+    for (int n = 0; n < NP; ++n)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) r.v[n][v] = r.v[n][v] * inv * w.v[n][v];
+    store_row<NP>(out + (size_t)t * hidden, hidden, r);
+}
+
+// OWN: a work-group takes all tokens of one request and leaves the request's last token itself (steps with as many tokens as requests, where a launch
+// more would be all that last_token_kernel is); otherwise one token.
+template <typename T, int NP, bool OWN>
+__global__ void __launch_bounds__(1024)
+bigram_embedding_rows_kernel(const int* __restrict__ ids, const T* __restrict__ table, float* __restrict__ out, int hidden, int vocab,
+                             float scale, const int* __restrict__ token_req, const int* __restrict__ req_indptr,
+                             const int* __restrict__ positions, const int* __restrict__ slots, int* __restrict__ last_token,
+                             const T* __restrict__ bigram, int buckets, long long mul_prev, long long mul_cur, int copies, size_t copy_stride) {
+    const int r = OWN ? (int)blockIdx.x : token_req[blockIdx.x];
+    const int tok0 = req_indptr[r], first = OWN ? tok0 : (int)blockIdx.x, last = OWN ? req_indptr[r + 1] : first + 1;
+    int* kept = last_token + slots[r];
+    int before = *kept;                                  // (read before this work-group, or the launch behind this one, writes it)
+    for (int t = first; t < last; ++t) {
+        int id = ids[t], prev = t > tok0 ? ids[t - 1] : before;
+        if (id < 0 || id >= vocab) id = 0;
+        if (prev < 0 || prev >= vocab) prev = 0;
+        int row = buckets;
+        if (positions[t] > 0) {
+            long long h = ((long long)prev * mul_prev + (long long)id * mul_cur) % buckets;
+            if (h < 0) h += buckets;
+            row = (int)h;
+        }
+        RowPieces<NP> x, b;
+        load_row<NP>(table + (size_t)id * hidden, hidden, x);
+        load_row<NP>(bigram + (size_t)row * hidden, hidden, b);
+#pragma unroll
+        for (int n = 0; n < NP; ++n)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) x.v[n][v] = fmaf(x.v[n][v], scale, b.v[n][v]);
+        for (int c = 0; c < copies; ++c) store_row<NP>(out + c * copy_stride + (size_t)t * hidden, hidden, x);
+    }
+    if (OWN) {
+        __syncthreads();                                 // every thread has read what was kept
+        if (threadIdx.x == 0 && last > first) *kept = ids[last - 1];
+    }
+}
+
+// Rows that can be held in pieces: a multiple of four numbers, 16-byte aligned, up to 12288 of them.
+static bool rows_in_pieces(int hidden, uintptr_t bits) { return hidden % 4 == 0 && hidden <= 12288 && bits % 16 == 0; }
+#define TL_ROWS(CALL)                                                           \
+    const RowPlan plan = plan_row(hidden);                                      \
+    if (plan.pieces == 1) { CALL(1); } else if (plan.pieces == 2) { CALL(2); } else { CALL(3); }
+
+extern "C" int tl_embedding(const void* ids, const void* table, int table_dtype, void* out,
+                            int tokens, int hidden, int vocab, float scale, const void* positions, const void* pos_table,
+                            int pos_dtype, int pos_rows, int copies, hipStream_t stream) {
+    TL_REQUIRE(tokens >= 0 && hidden > 0 && vocab > 0 && copies > 0, "embedding: bad sizes tokens=%d hidden=%d vocab=%d copies=%d", tokens, hidden, vocab, copies);
+    TL_REQUIRE(!pos_table || (positions && pos_rows > 0), "embedding: a position table needs positions and rows");
+    if (tokens == 0) return TL_OK;
+    dim3 grid(tokens), block(256);
+    const size_t copy_stride = (size_t)tokens * hidden;
+    const int pos_f32 = pos_dtype == TL_DT_F32;
+    TL_REQUIRE(table_dtype == TL_DT_F32 || table_dtype == TL_DT_BF16, "embedding: unknown dtype %d", table_dtype);
+    if (rows_in_pieces(hidden, (uintptr_t)table | (uintptr_t)out | (uintptr_t)pos_table)) {
+#define TL_EMB(T, N) embedding_rows_kernel<T, N><<<tokens, plan.threads, 0, stream>>>((const int*)ids, (const T*)table, (float*)out, hidden, vocab, scale, \
+        (const int*)positions, pos_table, pos_f32, pos_rows, copies, copy_stride)
+#define TL_EMB_N(N) if (table_dtype == TL_DT_F32) TL_EMB(float, N); else TL_EMB(bf16_t, N)
+        TL_ROWS(TL_EMB_N)
+#undef TL_EMB_N
+#undef TL_EMB
+        TL_CHECK_LAUNCH("embedding");
+        return TL_OK;
+    }
+    if (table_dtype == TL_DT_F32)
+        embedding_kernel<float><<<grid, block, 0, stream>>>((const int*)ids, (const float*)table, (float*)out, hidden, vocab, scale,
+                                                            (const int*)positions, pos_table, pos_f32, pos_rows, copies, copy_stride);
+    else if (table_dtype == TL_DT_BF16)
+        embedding_kernel<bf16_t><<<grid, block, 0, stream>>>((const int*)ids, (const bf16_t*)table, (float*)out, hidden, vocab, scale,
+                                                             (const int*)positions, pos_table, pos_f32, pos_rows, copies, copy_stride);
+    else TL_REQUIRE(false, "embedding: unknown dtype %d", table_dtype);
+    TL_CHECK_LAUNCH("embedding");
+    return TL_OK;
+}
+
+extern "C" int tl_bigram_embedding(const void* ids, const void* table, void* out, int tokens, int hidden, int vocab, float scale,
+                                   const void* token_req, const void* req_indptr, int requests, const void* positions, const void* slots,
+                                   void* last_token, const void* bigram, int buckets, long mul_prev, long mul_cur, int copies, int dtype,
+                                   hipStream_t stream) {
+    TL_REQUIRE(tokens >= 0 && hidden > 0 && vocab > 0 && copies > 0 && buckets > 0 && requests >= 0, "bigram_embedding: bad sizes");
+    TL_REQUIRE(token_req && req_indptr && positions && slots && last_token && bigram, "bigram_embedding: a null operand");
+    if (tokens == 0) return TL_OK;
+    const size_t copy_stride = (size_t)tokens * hidden;
+    TL_REQUIRE(dtype == TL_DT_F32 || dtype == TL_DT_BF16, "bigram_embedding: unknown dtype %d", dtype);
+    if (rows_in_pieces(hidden, (uintptr_t)table | (uintptr_t)out | (uintptr_t)bigram)) {
+        const bool own = tokens == requests;
+#define TL_BIG(T, N, OWN) bigram_embedding_rows_kernel<T, N, OWN><<<tokens, plan.threads, 0, stream>>>((const int*)ids, (const T*)table, (float*)out, hidden, vocab, \
+        scale, (const int*)token_req, (const int*)req_indptr, (const int*)positions, (const int*)slots, (int*)last_token, (const T*)bigram, buckets, mul_prev, mul_cur, \
+        copies, copy_stride)
+#define TL_BIG_N(N) if (dtype == TL_DT_F32) { if (own) TL_BIG(float, N, true); else TL_BIG(float, N, false); } else if (own) TL_BIG(bf16_t, N, true); else TL_BIG(bf16_t, N, false)
+        TL_ROWS(TL_BIG_N)
+#undef TL_BIG_N
+#undef TL_BIG
+        TL_CHECK_LAUNCH("bigram_embedding");
+        if (own) return TL_OK;
+        last_token_kernel<<<(requests + 63) / 64, 64, 0, stream>>>((const int*)ids, (const int*)req_indptr, (const int*)slots, (int*)last_token, requests);
+        TL_CHECK_LAUNCH("last_token");
+        return TL_OK;
+    }
+    if (dtype == TL_DT_F32)
+        bigram_embedding_kernel<float><<<tokens, 256, 0, stream>>>((const int*)ids, (const float*)table, (float*)out, hidden, vocab, scale,
+            (const int*)token_req, (const int*)req_indptr, (const int*)positions, (const int*)slots, (const int*)last_token, (const float*)bigram,
+            buckets, mul_prev, mul_cur, copies, copy_stride);
+    else if (dtype == TL_DT_BF16)
+        bigram_embedding_kernel<bf16_t><<<tokens, 256, 0, stream>>>((const int*)ids, (const bf16_t*)table, (float*)out, hidden, vocab, scale,
+            (const int*)token_req, (const int*)req_indptr, (const int*)positions, (const int*)slots, (const int*)last_token, (const bf16_t*)bigram,
+            buckets, mul_prev, mul_cur, copies, copy_stride);
+    else TL_REQUIRE(false, "bigram_embedding: unknown dtype %d", dtype);
+    TL_CHECK_LAUNCH("bigram_embedding");
+    last_token_kernel<<<(requests + 63) / 64, 64, 0, stream>>>((const int*)ids, (const int*)req_indptr, (const int*)slots, (int*)last_token, requests);
+    TL_CHECK_LAUNCH("last_token");
+    return TL_OK;
 }
 
 // ------------------------------------------------------------------ norm of the branch output, addition, norm of the sum
@@ -1203,10 +1324,53 @@ __global__ void normed_sum_kernel(const T* __restrict__ x, int branches, size_t 
     }
 }
 
+// The same with all branches' rows in registers and their sums of squares joined at one barrier: one trip to memory a row (4 rows of two branches of 2048
+// numbers 12.5 -> 3.6 us).
+template <typename T, int NP, int B>
+__global__ void __launch_bounds__(1024)
+normed_sum_rows_kernel(const T* __restrict__ x, size_t branch_stride, const float* __restrict__ w, float eps, T* __restrict__ out, int hidden) {
+    __shared__ float red[B][16];
+    const size_t at = (size_t)blockIdx.x * hidden;
+    RowPieces<NP> r[B], wr[B];
+#pragma unroll
+    for (int b = 0; b < B; ++b) load_row<NP>(x + b * branch_stride + at, hidden, r[b]);
+#pragma unroll
+    for (int b = 0; b < B; ++b) load_row<NP>(w + (size_t)b * hidden, hidden, wr[b]);
+    const int wave = threadIdx.x / TL_WAVE, waves = blockDim.x / TL_WAVE;
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+        const float ss = wave_sum(row_squares(r[b]));
+        if (threadIdx.x % TL_WAVE == 0) red[b][wave] = ss;
+    }
+    __syncthreads();
+    RowPieces<NP> y;
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+        float ss = 0.f;
+        for (int i = 0; i < waves; ++i) ss += red[b][i];
+        const float inv = rsqrtf(ss / (float)hidden + eps);
+#pragma unroll
+        for (int n = 0; n < NP; ++n)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) y.v[n][v] = b == 0 ? r[b].v[n][v] * inv * wr[b].v[n][v] : fmaf(r[b].v[n][v] * inv, wr[b].v[n][v], y.v[n][v]);
+    }
+    store_row<NP>(out + at, hidden, y);
+}
+
 extern "C" int tl_normed_sum(const void* x, int branches, int rows, int hidden, const void* w, float eps, void* out, int dtype, hipStream_t stream) {
     TL_REQUIRE(branches > 0 && branches <= NS_MAX_BRANCHES && rows >= 0 && hidden > 0, "normed_sum: bad sizes (up to %d branches)", NS_MAX_BRANCHES);
     if (rows == 0) return TL_OK;
     const size_t stride = (size_t)rows * hidden;
+    TL_REQUIRE(dtype == TL_DT_F32 || dtype == TL_DT_BF16, "normed_sum: unknown dtype %d", dtype);
+    if (branches == 2 && rows_in_pieces(hidden, (uintptr_t)x | (uintptr_t)w | (uintptr_t)out)) {      // (two: what a mixer of two branches sums)
+#define TL_NS(T, N) normed_sum_rows_kernel<T, N, 2><<<rows, plan.threads, 0, stream>>>((const T*)x, stride, (const float*)w, eps, (T*)out, hidden)
+#define TL_NS_N(N) if (dtype == TL_DT_F32) TL_NS(float, N); else TL_NS(bf16_t, N)
+        TL_ROWS(TL_NS_N)
+#undef TL_NS_N
+#undef TL_NS
+        TL_CHECK_LAUNCH("normed_sum");
+        return TL_OK;
+    }
     if (dtype == TL_DT_F32) normed_sum_kernel<float><<<rows, 256, 0, stream>>>((const float*)x, branches, stride, (const float*)w, eps, (float*)out, hidden);
     else if (dtype == TL_DT_BF16) normed_sum_kernel<bf16_t><<<rows, 256, 0, stream>>>((const bf16_t*)x, branches, stride, (const float*)w, eps, (bf16_t*)out, hidden);
     else TL_REQUIRE(false, "normed_sum: unknown dtype %d", dtype);
@@ -1242,6 +1406,16 @@ extern "C" int tl_embedding_norm(const void* ids, const void* table, int table_d
     TL_REQUIRE(tokens >= 0 && hidden > 0 && hidden <= 12288 && vocab > 0 && weight, "embedding_norm: bad sizes tokens=%d hidden=%d vocab=%d", tokens, hidden, vocab);
     if (tokens == 0) return TL_OK;
     const size_t smem = sizeof(float) * hidden;
+    TL_REQUIRE(table_dtype == TL_DT_F32 || table_dtype == TL_DT_BF16, "embedding_norm: unknown dtype %d", table_dtype);
+    if (rows_in_pieces(hidden, (uintptr_t)table | (uintptr_t)out | (uintptr_t)weight)) {
+#define TL_EN(T, N) embedding_norm_rows_kernel<T, N><<<tokens, plan.threads, 0, stream>>>((const int*)ids, (const T*)table, (float*)out, hidden, vocab, scale, (const float*)weight, eps)
+#define TL_EN_N(N) if (table_dtype == TL_DT_F32) TL_EN(float, N); else TL_EN(bf16_t, N)
+        TL_ROWS(TL_EN_N)
+#undef TL_EN_N
+#undef TL_EN
+        TL_CHECK_LAUNCH("embedding_norm");
+        return TL_OK;
+    }
     if (table_dtype == TL_DT_F32)
         embedding_norm_kernel<float><<<tokens, 256, smem, stream>>>((const int*)ids, (const float*)table, (float*)out, hidden, vocab, scale, (const float*)weight, eps);
     else if (table_dtype == TL_DT_BF16)
