@@ -57,8 +57,8 @@ __device__ __forceinline__ void wait_direct_loads() { asm volatile("s_waitcnt vm
 
 // Rows of one slab in shared memory: the BM rows of x and the BN rows of w, rounded up to what the waves'
 // load instructions (64 lanes x 16 bytes each) fill between them.
-constexpr int dl_slab_rows(int bm, int bn, int waves, int tk) {
-    const int per = (64 / (tk / 8)) * waves;
+constexpr int dl_slab_rows(int bm, int bn, int waves) {
+    const int per = 8 * waves;
     return (bm + bn + per - 1) / per * per;
 }
 
@@ -68,10 +68,10 @@ template <int ACT>
 __device__ __forceinline__ float activated(float v) { return activate(v, ACT); }
 
 template <int ACT, int BM, int BN, int WM, int WN, int FM, int FN, int ROOM, bool PAIRS>
-__device__ __forceinline__ void store_expert_tile_as(const f32x16_t (&acc)[FM][FN], bf16_t* stage, bf16_t* out, int r0, int c0, int M, int N, int ldo) {
+__device__ __forceinline__ void store_expert_tile_as(const f32x4_t (&acc)[FM][FN], bf16_t* stage, bf16_t* out, int r0, int c0, int M, int N, int ldo) {
     constexpr int WNO = PAIRS ? WN / 2 : WN;
     static_assert(BM * (PAIRS ? BN / 2 : BN) <= ROOM, "the result tile must fit the slab buffers");
-    const int lane = threadIdx.x & 63, lm = lane & 31, half = lane >> 5;
+    const int lane = threadIdx.x & 63, lm = lane & 15, quad = lane >> 4;
     const int cols = PAIRS ? N / 2 : N, co = PAIRS ? c0 / 2 : c0;
     const bool whole = cols % 8 == 0 && ldo % 8 == 0 && ((uintptr_t)out % 16) == 0;
     constexpr int C = WNO / 8, CX = C & -C;
@@ -80,28 +80,26 @@ __device__ __forceinline__ void store_expert_tile_as(const f32x16_t (&acc)[FM][F
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int j = 0; j < FN; ++j)
+        for (int j = 0; j < FN; ++j) {
+            constexpr int V = PAIRS ? 2 : 4;              // output columns of a lane's four
+            bf16_t h[V];
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                constexpr int V = PAIRS ? 2 : 4;              // output columns of a lane's four
-                bf16_t h[V];
-#pragma unroll
-                for (int e = 0; e < V; ++e) {
-                    if constexpr (PAIRS) h[e] = from_float<bf16_t>(activated<ACT>(acc[i][j][4 * g + 2 * e]) * acc[i][j][4 * g + 2 * e + 1]);
-                    else h[e] = from_float<bf16_t>(activated<ACT>(acc[i][j][4 * g + e]));
-                }
-                const int n = (j * 32 + 8 * g + 4 * half) / (PAIRS ? 2 : 1), row = i * 32 + lm;
-                if (whole) {
-                    bf16_t* dst = stage + row * WNO + (((n >> 3) ^ (row & (CX - 1))) * 8) + (n & 7);
-                    const uint32_t a = (uint32_t)h[0].bits | ((uint32_t)h[1].bits << 16);
-                    if constexpr (PAIRS) *(uint32_t*)dst = a;
-                    else *(uint2*)dst = make_uint2(a, (uint32_t)h[V - 2].bits | ((uint32_t)h[V - 1].bits << 16));
-                } else if (r0 + row < M) {
-#pragma unroll
-                    for (int e = 0; e < V; ++e)
-                        if (co + n + e < cols) out[(size_t)(r0 + row) * ldo + co + n + e] = h[e];
-                }
+            for (int e = 0; e < V; ++e) {
+                if constexpr (PAIRS) h[e] = from_float<bf16_t>(activated<ACT>(acc[i][j][2 * e]) * acc[i][j][2 * e + 1]);
+                else h[e] = from_float<bf16_t>(activated<ACT>(acc[i][j][e]));
             }
+            const int n = (j * 16 + 4 * quad) / (PAIRS ? 2 : 1), row = i * 16 + lm;
+            if (whole) {
+                bf16_t* dst = stage + row * WNO + (((n >> 3) ^ (row & (CX - 1))) * 8) + (n & 7);
+                const uint32_t a = (uint32_t)h[0].bits | ((uint32_t)h[1].bits << 16);
+                if constexpr (PAIRS) *(uint32_t*)dst = a;
+                else *(uint2*)dst = make_uint2(a, (uint32_t)h[V - 2].bits | ((uint32_t)h[V - 1].bits << 16));
+            } else if (r0 + row < M) {
+#pragma unroll
+                for (int e = 0; e < V; ++e)
+                    if (co + n + e < cols) out[(size_t)(r0 + row) * ldo + co + n + e] = h[e];
+            }
+        }
     if (!whole) return;
     // (one wave's shared-memory accesses are carried out in order: no wait in between)
 #pragma unroll
@@ -113,7 +111,7 @@ __device__ __forceinline__ void store_expert_tile_as(const f32x16_t (&acc)[FM][F
 }
 
 template <int BM, int BN, int WM, int WN, int FM, int FN, int ROOM, bool PAIRS>
-__device__ __forceinline__ void store_expert_tile(const f32x16_t (&acc)[FM][FN], bf16_t* stage, bf16_t* out, int r0, int c0, int M, int N, int ldo, int act) {
+__device__ __forceinline__ void store_expert_tile(const f32x4_t (&acc)[FM][FN], bf16_t* stage, bf16_t* out, int r0, int c0, int M, int N, int ldo, int act) {
     switch (act & ~ACT_PAIRS) {         // (one switch for the tile, not one for every number)
     case ACT_RELU2: return store_expert_tile_as<ACT_RELU2, BM, BN, WM, WN, FM, FN, ROOM, PAIRS>(acc, stage, out, r0, c0, M, N, ldo);
     case ACT_SILU: return store_expert_tile_as<ACT_SILU, BM, BN, WM, WN, FM, FN, ROOM, PAIRS>(acc, stage, out, r0, c0, M, N, ldo);
@@ -138,7 +136,7 @@ struct ExpertRows {
 template <typename GS> struct IsExpertRows { static constexpr bool value = false, pairs = false; };
 template <bool P> struct IsExpertRows<ExpertRows<P>> { static constexpr bool value = true, pairs = P; };
 
-template <int BM, int BN, int WGM, int WGN, int STAGES, typename TOut, int SW = 0, int TK = 64, typename GS = GroupStride>
+template <int BM, int BN, int WGM, int WGN, int STAGES, typename TOut, int SW = 0, typename GS = GroupStride>
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm_dl_tile_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                                       const void* __restrict__ bias, int bias_f32,
                                                                       TOut* __restrict__ out, int M, int N, int K, int ldx, int ldo,
@@ -146,13 +144,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_dl_tile_kernel(const bf16
     constexpr bool EX = IsExpertRows<GS>::value;
     static_assert(!EX || (!SW && sizeof(TOut) == 2), "groups of rows: bfloat16 results with an activation of their own");
     static_assert(!SW || (BN / WGN) % 64 == 0, "the fused gate needs whole 64-row blocks per wave");
-    static_assert(TK == 64 || TK == 32, "slabs of 64 or 32 columns");
-    // A slab row holds PPR pieces of 16 bytes; one load instruction of a wave fills RPL rows.  With
-    // slabs of 32 columns a row is 64 bytes and piece c of row r lies in slot c ^ ((r >> 2) & 3): the
-    // sixteen rows a quarter-wave reads then fall on all 64 banks as well.  Half the slab is half the
-    // shared memory per stage: twice as many stages fit, and a request has twice as long to arrive.
-    constexpr int PPR = TK / 8, RPL = 64 / PPR;
-#define DL_SWZ(r) (TK == 64 ? (((r) >> 1) & 7) : (((r) >> 2) & 3))
+    // A slab row holds PPR pieces of 16 bytes; one load instruction of a wave fills RPL rows.
+    constexpr int TK = 64, PPR = TK / 8, RPL = 64 / PPR;
     // Split K (k_per_split > 0, a multiple of 64): blockIdx.y owns the columns [y * k_per_split, ...) of
     // x and w and writes its own [M, ldo] slab of partial sums to out; whoever reads them adds the slabs up.
     const int ldw = K;
@@ -170,9 +163,9 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_dl_tile_kernel(const bf16
     }
     constexpr int NW = WGM * WGN;
     constexpr int WM = BM / WGM, WN = BN / WGN;          // wave tile
-    constexpr int FM = WM / 32, FN = WN / 32;            // 32x32 blocks per wave
+    constexpr int FM = WM / 16, FN = WN / 16;            // 16x16 blocks per wave
     constexpr int ROWS = BM + BN;
-    constexpr int LROWS = dl_slab_rows(BM, BN, NW, TK);  // a slab's rows in shared memory: ROWS, rounded up so that ...
+    constexpr int LROWS = dl_slab_rows(BM, BN, NW);  // a slab's rows in shared memory: ROWS, rounded up so that ...
     constexpr int LOADS = LROWS / RPL / NW;              // ... every wave issues as many load instructions per slab (RPL rows each)
     static_assert(LOADS * (STAGES - 1) < 64, "outstanding loads must fit the counter");
     extern __shared__ __attribute__((aligned(16))) bf16_t lds_raw[];   // [STAGES][LROWS][TK]
@@ -250,7 +243,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_dl_tile_kernel(const bf16
     for (int j = 0; j < LOADS; ++j) {
         const int base_row = RPL * (wave + j * NW);
         const int row = min(base_row + lane / PPR, ROWS - 1);      // (rows of the rounding: copies of the last row, never read)
-        const int c = (lane % PPR) ^ DL_SWZ(row);
+        const int c = (lane % PPR) ^ ((row >> 1) & 7);
         if (row < BM) {
             int m = min(m0 + row, M - 1);
             if constexpr (EX) m = gs.src ? gs.src[m] : m;
@@ -265,39 +258,43 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_dl_tile_kernel(const bf16
     const bf16_t* wt = w + (size_t)n0 * ldw;
     const unsigned lds_base = (unsigned)(uintptr_t)((void __attribute__((address_space(3)))*)lds_raw);
 
-    f32x16_t acc[FM][FN];
+    f32x4_t acc[FM][FN];
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+            for (int v = 0; v < 4; ++v) acc[i][j][v] = 0.f;
 
-    const int slabs = K / TK;
-    const int fr = lane & 31, fh = lane >> 5;
-    int arow[FM], brow[FN], akey[FM], bkey[FN];
-#pragma unroll
-    for (int i = 0; i < FM; ++i) { arow[i] = wm * WM + i * 32 + fr; akey[i] = DL_SWZ(arow[i]); }
-#pragma unroll
-    for (int j = 0; j < FN; ++j) { brow[j] = BM + wn * WN + j * 32 + fr; bkey[j] = DL_SWZ(brow[j]); }
-#undef DL_SWZ
-
-    // The loop is a hand-laid pipeline; scheduling fences keep the compiler from undoing it.  A step
-    // of TK columns has TK / 16 phases of FM * FN products.  A phase's memory instructions go between
-    // its products, one product first: the operand reads of the next phase into the other register set,
-    // so a read has a whole phase to arrive, and the wait before a phase's first product is for operands
-    // asked for a phase ago with nothing younger outstanding.  (All reads first and then all products,
-    // the wait at the loop's head came out as one for every read, the ones just issued too, and the 7B's fused
-    // gate/up product at 2048 rows took 537 us instead of 487.)  The last phase of a step first waits for the
-    // next slab and meets the other waves at the barrier (they have all read their last operands of this
-    // slab by then); between its products go the first half of the requests for the slab STAGES - 1 ahead, into
-    // the buffer just given up, and then the reads of the first operands of the next slab.  The other half of
-    // the requests goes into the first phase of the next step: a compute unit's 64 requests in one phase hold
-    // its waves up, whatever they fetch (requests of 4 bytes a lane cost the same; without any the loop ran a
-    // sixth faster), and in two phases less so (2048 x 3584 x 18944: 392 -> 353 us; spread over three phases the
-    // last ones arrive too late).  Past the end the last slab is requested again (nobody reads it), so the count
+    // Products of 16 x 16 x 32: lane l holds eight columns of K, 8 (l / 16) .. + 7 of a phase's 32, of row l % 16 of a block.  They do the work of a 32 x 32 x
+    // 16 product in as many cycles and move half as much of the accumulators, and the power that this takes is what sets the clock of a large product (8192 x 8192 x 8192:
+    // 2650 cycles a slab at 1.67 GHz with the larger blocks, 2610 at 1.8 with these: 846 -> 778 us; 2048 x 37888 x 3584 468 -> 446, 2048 x 8192 x 2048 60 -> 56).
+    //
+    // The loop is a hand-laid pipeline; scheduling fences keep the compiler from undoing it.  A step of TK columns has two phases of FM * FN products.  A phase's
+    // memory instructions go between its products, one product first: the operand reads of the next phase, so that a read has a whole phase to arrive.  (All
+    // reads first and then all products, the wait at the loop's head came out as one for every read, the ones just issued too.)  Both operands
+    // have two sets of registers; where these and the sums do not fit (the waves of 64 x 160), the operand with more blocks (`rolled`) has one set, each
+    // block read anew once the last product that needs it is under way (in a wave of 128 x 64, where both ways fit, it costs a fortieth: 778 against 796 us).
+    //
+    // The last phase of a step waits for the next slab and meets the other waves at the barrier (they have all read their last operands of this
+    // slab by then): at its start, or with many products halfway through it, which leaves the slab that much longer to arrive (8192 x 8192 x 8192: 863 us at the
+    // start, 778 halfway).  Behind the barrier go the first half of the requests for the slab STAGES - 1 ahead, into
+    // the buffer just given up, and the reads of the first operands of the next slab.  The other half of the requests goes into the first phase of the next
+    // step: a compute unit's 64 requests in one phase hold its waves up, whatever they fetch (requests of 4 bytes a lane cost the same; without any the loop ran a
+    // sixth faster), and in two phases less so (all of them behind the reads: 857 us).  Past the end the last slab is requested again (nobody reads it), so the count
     // of requests in flight is the same in every step, which the wait relies on.
-    Frag16 af[2][FM], bfr[2][FN];
+    constexpr int PHASES = TK / 32, NM = FM * FN;
+    constexpr bool MANY = NM > 16, ROLL_X = FM >= FN;
+    constexpr bool ROLL = 4 * NM + 8 * (FM + FN) > (NW > 4 ? 232 : 464);      // registers of the products and of two sets of operands
+    constexpr int FR = ROLL_X ? FM : FN, FD = ROLL_X ? FN : FM;       // blocks of the rolled operand (the outer index of the products) and of the other
+    constexpr int BARRIER_AT = MANY ? NM * 3 / 4 : 0;                    // products of the last phase ahead of its barrier
+    Frag16 rolled[ROLL ? 1 : 2][FR], paired[2][FD];
+    const int slabs = K / TK;
+    const int fr = lane & 15, fq = lane >> 4;
+    // where this lane's first block lies in a slab (rows are 64 elements; a block's rows are 1024 further on, its slots' order the same)
+    const int x_at = (wm * WM + fr) * TK, w_at = (BM + wn * WN + fr) * TK;
+    const int roll_at = ROLL_X ? x_at : w_at, pair_at = ROLL_X ? w_at : x_at;
+    const int slot[PHASES] = {(fq ^ ((fr >> 1) & 7)) * 8, ((fq + 4) ^ ((fr >> 1) & 7)) * 8};
     // requests of a slab issued in the last phase of a step; the rest in the next step's first.  (Not for the smallest tile,
     // four requests a wave and slab: split in two they made the decode step's products over K a fiftieth slower.)
     constexpr int L_LAST = LOADS >= 6 ? (LOADS + 1) / 2 : LOADS;
@@ -316,91 +313,73 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_dl_tile_kernel(const bf16
 #pragma unroll
     for (int j = 0; j < L_LAST; ++j) request(STAGES - 1, j);
 #pragma unroll
-    for (int i = 0; i < FM; ++i) af[0][i].u = *(const uint4*)(lds_raw + arow[i] * TK + ((fh ^ akey[i]) * 8));
+    for (int d = 0; d < FD; ++d) paired[0][d].u = *(const uint4*)(lds_raw + pair_at + d * 16 * TK + slot[0]);
 #pragma unroll
-    for (int j = 0; j < FN; ++j) bfr[0][j].u = *(const uint4*)(lds_raw + brow[j] * TK + ((fh ^ bkey[j]) * 8));
+    for (int r = 0; r < FR; ++r) rolled[0][r].u = *(const uint4*)(lds_raw + roll_at + r * 16 * TK + slot[0]);
     __builtin_amdgcn_sched_barrier(0);
 
-    constexpr int PHASES = TK / 16;
-    constexpr int NM = FM * FN, NR = FM + FN;               // products and operand reads of a phase
     for (int sl = 0; sl < slabs; ++sl) {
-        const bf16_t* cb = lds_raw + (sl % STAGES) * LROWS * TK;
 #pragma unroll
         for (int kk = 0; kk < PHASES; ++kk) {
             const int cur = kk & 1, nxt = cur ^ 1;
             const bool last = kk + 1 == PHASES;
-            const bf16_t* nb = last ? lds_raw + ((sl + 1) % STAGES) * LROWS * TK : cb;      // where the next phase's operands lie
-            const int c = (last ? 0 : 2 * (kk + 1)) + fh;
+            const bf16_t* nb = lds_raw + ((sl + (last ? 1 : 0)) % STAGES) * LROWS * TK + slot[last ? 0 : kk + 1];      // where the next phase's operands lie
             // this phase's requests [lfirst, lend) and the slab they fetch: in the last phase the slab that gets the
             // buffer given up now, in the first the rest of the slab that got the buffer given up a step ago
             const int lfirst = last ? 0 : L_LAST, lend = last ? L_LAST : kk == 0 ? LOADS : L_LAST;
             const int slab_of = last ? sl + STAGES : sl - 1 + STAGES;
             const int nl = lend - lfirst;
-            const int ops = nl + NR;                                                         // memory instructions of this phase ...
-            const int per = (ops + NM - 1) / NM;                                             // ... and how many follow each product
-            if (last) {
-                wait_direct_loads<(STAGES - 2) * LOADS>();
-                __syncthreads();
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            if constexpr (NM == 1) {
-                // One product a phase (the smallest tile): a phase's memory instructions first, then its product, which
-                // covers them; but for the step's first phase, whose product comes first so that the wait at the loop's
-                // head is for that product's operands alone.
-                if (kk == 0) {
-                    acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[cur][0].v, af[cur][0].v, acc[0][0], 0, 0, 0);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-#pragma unroll
-                for (int op = 0; op < ops; ++op) {
-                    const int r = op - nl;
-                    if (r < 0) request(slab_of, lfirst + op);
-                    else if (r < FM) af[nxt][r].u = *(const uint4*)(nb + arow[r] * TK + ((c ^ akey[r]) * 8));
-                    else bfr[nxt][r - FM].u = *(const uint4*)(nb + brow[r - FM] * TK + ((c ^ bkey[r - FM]) * 8));
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                if (kk > 0) {
-                    acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[cur][0].v, af[cur][0].v, acc[0][0], 0, 0, 0);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                continue;
-            }
+            const int start = last ? BARRIER_AT : 0;                                         // the first product that memory instructions follow
+            const int ops = nl + FD + FR;                                                    // memory instructions of this phase ...
+            const int least = (ops + NM - start - 1) / (NM - start), per = MANY && !ROLL && least < 2 ? 2 : least;      // ... and how many follow each product
+            auto issue = [&](int op) {
+                if (op < nl) request(slab_of, lfirst + op);
+                else if (op < nl + FD) paired[nxt][op - nl].u = *(const uint4*)(nb + pair_at + (op - nl) * 16 * TK);
+                else rolled[ROLL ? 0 : nxt][op - nl - FD].u = *(const uint4*)(nb + roll_at + (op - nl - FD) * 16 * TK);
+            };
             int op = 0;
 #pragma unroll
             for (int q = 0; q < NM; ++q) {
-                acc[q / FN][q % FN] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[cur][q % FN].v, af[cur][q / FN].v, acc[q / FN][q % FN], 0, 0, 0);
+                if (last && q == start) {
+                    wait_direct_loads<(STAGES - 2) * LOADS>();
+                    __syncthreads();
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                const int r = q / FD, d = q % FD, i = ROLL_X ? r : d, j = ROLL_X ? d : r;
+                const Frag16 &fx = ROLL_X ? rolled[ROLL ? 0 : cur][r] : paired[cur][d], &fw = ROLL_X ? paired[cur][d] : rolled[ROLL ? 0 : cur][r];
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw.v, fx.v, acc[i][j], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
+                if (q < start) continue;
 #pragma unroll
-                for (int e = 0; e < per; ++e, ++op) {
-                    if (op >= ops) break;
-                    const int r = op - nl;
-                    if (r < 0) request(slab_of, lfirst + op);
-                    else if (r < FM) af[nxt][r].u = *(const uint4*)(nb + arow[r] * TK + ((c ^ akey[r]) * 8));
-                    else bfr[nxt][r - FM].u = *(const uint4*)(nb + brow[r - FM] * TK + ((c ^ bkey[r - FM]) * 8));
+                for (int e = 0; e < per; ++e) {
+                    if (op >= ops || (ROLL && op >= nl + FD && q < (op - nl - FD + 1) * FD - 1)) break;      // (a rolled block that products to come still need stays)
+                    issue(op++);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
+#pragma unroll
+            for (; op < ops; ++op) issue(op);
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
     wait_direct_loads<0>();
 
-    // The products are taken as weight block times x block, so of a 32x32 block a lane holds one
-    // row of x, m = lane % 32, and sixteen output columns n = 8 (v / 4) + 4 (lane / 32) + v % 4:
-    // four neighbours at a time.  With the fused gate, even blocks hold gate columns and the next
-    // block the up columns of the same 32 outputs.
-    const int lm = lane & 31, half = lane >> 5;
+    // The products are taken as weight block times x block, so of a 16x16 block a lane holds one row of x, m = lane % 16, and four neighbouring
+    // output columns, 4 (lane / 16) and up.  With the fused gate, of every four blocks of columns the first two hold gate columns and the
+    // other two the up columns of the same 32 outputs.
+    const int lm = lane & 15, quad = lane >> 4;
     if constexpr (EX) {
         store_expert_tile<BM, BN, WM, WN, FM, FN, STAGES * ROWS * TK, IsExpertRows<GS>::pairs>(acc, lds_raw + wave * (WM * (IsExpertRows<GS>::pairs ? WN / 2 : WN)),
             out, m0 + wm * WM, n0 + wn * WN, M, N, ldo, gs.act);
         return;
     }
     constexpr int WNO = SW ? WN / 2 : WN;                   // output columns of a wave tile
-    constexpr int FNO = SW ? FN / 2 : FN;                   // and its blocks of 32 of them
+    constexpr int FNO = SW ? FN / 2 : FN;                   // and its blocks of 16 of them
     const int cols = SW ? out_cols : N;                     // output columns in all
     const int c0 = (SW ? n0 / 2 : n0) + wn * WNO;           // first output column and row of this wave
     const int r0 = m0 + wm * WM;
     auto value = [&](int i, int jo, int v) -> float {
-        if constexpr (SW) return gate_mul<SW>(acc[i][2 * jo][v], acc[i][2 * jo + 1][v]);
+        if constexpr (SW) return gate_mul<SW>(acc[i][jo / 2 * 4 + jo % 2][v], acc[i][jo / 2 * 4 + 2 + jo % 2][v]);
         else return acc[i][jo][v];
     };
     auto bias_at = [&](int n) -> float { return (!SW && bias && n < cols) ? load_vec(bias, bias_f32, n) : 0.f; };
@@ -420,19 +399,16 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_dl_tile_kernel(const bf16
 #pragma unroll
             for (int i = 0; i < FM; ++i)
 #pragma unroll
-                for (int jo = 0; jo < FNO; ++jo)
+                for (int jo = 0; jo < FNO; ++jo) {
+                    const int n = jo * 16 + 4 * quad, row = i * 16 + lm;
+                    bf16_t h[4];
 #pragma unroll
-                    for (int g = 0; g < 4; ++g) {
-                        const int n = jo * 32 + 8 * g + 4 * half;
-                        bf16_t h[4];
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) h[e] = from_float<bf16_t>(value(i, jo, 4 * g + e) + bias_at(c0 + n + e));
-                        uint2 packed;
-                        packed.x = (uint32_t)h[0].bits | ((uint32_t)h[1].bits << 16);
-                        packed.y = (uint32_t)h[2].bits | ((uint32_t)h[3].bits << 16);
-                        const int row = i * 32 + lm;
-                        *(uint2*)(stage + row * WNO + (((n >> 3) ^ (row & (CX - 1))) * 8) + (n & 4)) = packed;
-                    }
+                    for (int e = 0; e < 4; ++e) h[e] = from_float<bf16_t>(value(i, jo, e) + bias_at(c0 + n + e));
+                    uint2 packed;
+                    packed.x = (uint32_t)h[0].bits | ((uint32_t)h[1].bits << 16);
+                    packed.y = (uint32_t)h[2].bits | ((uint32_t)h[3].bits << 16);
+                    *(uint2*)(stage + row * WNO + (((n >> 3) ^ (row & (CX - 1))) * 8) + (n & 4)) = packed;
+                }
             // (one wave's shared-memory accesses are carried out in order: no wait in between)
 #pragma unroll
             for (int q = 0; q < WM * C / 64; ++q) {
@@ -448,28 +424,25 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_dl_tile_kernel(const bf16
     const bool quads = sizeof(TOut) == 4 && cols % 4 == 0 && ldo % 4 == 0 && ((uintptr_t)out % 16) == 0;
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
-        const int m = r0 + i * 32 + lm;
+        const int m = r0 + i * 16 + lm;
         if (m >= M) continue;
 #pragma unroll
-        for (int jo = 0; jo < FNO; ++jo)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int n = c0 + jo * 32 + 8 * g + 4 * half;
-                if (quads) {
-                    if (n < cols) {
-                        float4 f;
-                        f.x = value(i, jo, 4 * g) + bias_at(n);
-                        f.y = value(i, jo, 4 * g + 1) + bias_at(n + 1);
-                        f.z = value(i, jo, 4 * g + 2) + bias_at(n + 2);
-                        f.w = value(i, jo, 4 * g + 3) + bias_at(n + 3);
-                        *(float4*)((float*)out + (size_t)m * ldo + n) = f;
-                    }
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (n + e < cols) out[(size_t)m * ldo + n + e] = from_float<TOut>(value(i, jo, 4 * g + e) + bias_at(n + e));
+        for (int jo = 0; jo < FNO; ++jo) {
+            const int n = c0 + jo * 16 + 4 * quad;
+            if (quads) {
+                if (n < cols) {
+                    float4 f;
+                    f.x = value(i, jo, 0) + bias_at(n);
+                    f.y = value(i, jo, 1) + bias_at(n + 1);
+                    f.z = value(i, jo, 2) + bias_at(n + 2);
+                    f.w = value(i, jo, 3) + bias_at(n + 3);
+                    *(float4*)((float*)out + (size_t)m * ldo + n) = f;
                 }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < cols) out[(size_t)m * ldo + n + e] = from_float<TOut>(value(i, jo, e) + bias_at(n + e));
             }
+        }
     }
 }
-

@@ -317,8 +317,8 @@ static int launch_experts_few(const ExpertsCall& c, hipStream_t stream) {
 
 template <int BM, int BN, int WGM, int WGN, int STAGES, bool PAIRS>
 static int launch_experts_tile_t(const ExpertsCall& c, hipStream_t stream) {
-    constexpr size_t lds = (size_t)STAGES * dl_slab_rows(BM, BN, WGM * WGN, 64) * 64 * sizeof(bf16_t);
-    auto kernel = gemm_dl_tile_kernel<BM, BN, WGM, WGN, STAGES, bf16_t, 0, 64, ExpertRows<PAIRS>>;
+    constexpr size_t lds = (size_t)STAGES * dl_slab_rows(BM, BN, WGM * WGN) * 64 * sizeof(bf16_t);
+    auto kernel = gemm_dl_tile_kernel<BM, BN, WGM, WGN, STAGES, bf16_t, 0, ExpertRows<PAIRS>>;
     static hipError_t allowed = allow_lds(kernel, lds);
     if (allowed != hipSuccess) {
         tl_set_error("experts_tile: cannot get %zu bytes of shared memory: %s", lds, hipGetErrorString(allowed));
@@ -345,7 +345,7 @@ static int launch_experts(int which, const ExpertsCall& c, hipStream_t stream) {
     case EX_TILE_64x128: rc = launch_experts_tile<64, 128, 1, 2, 3>(c, stream); break;
     case EX_TILE_128x128: rc = launch_experts_tile<128, 128, 2, 2, 2>(c, stream); break;
     case EX_TILE_128x256: rc = launch_experts_tile<128, 256, 2, 4, 3>(c, stream); break;
-    case EX_TILE_256x256: rc = launch_experts_tile<256, 256, 4, 2, 2>(c, stream); break;
+    case EX_TILE_256x256: rc = launch_experts_tile<256, 256, 2, 4, 2>(c, stream); break;
     default: TL_REQUIRE(false, "experts_gemm: no kernel %d", which);
     }
     if (rc != TL_OK) return rc;

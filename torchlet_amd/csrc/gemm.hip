@@ -1218,109 +1218,141 @@ static int launch_mfma_tile(const void* x, const void* w, const void* bias, int 
 // Tile shapes of the direct-load kernel and which one a product gets.  Estimate per shape: the
 // tiles are dealt to 256 compute units, each works through ceil(tiles / 256) of them one after
 // the other; a tile takes a fixed time (filling the pipeline, storing the result) plus its
-// products at the rate one compute unit reaches with that shape (fitted to measurements at
-// 2048 rows against the Qwen2.5-7B and 14B matrices, K from 3584 to 18944).
-// (DL_128x128_S4: 128 x 128 with four slabs in shared memory, one work-group to a compute unit: for products of up
-// to 128 rows split over K, where what counts is how many bytes of weights a work-group has on their way; measured
-// at 128 rows against the best other tile: 3584 x 18944 48.8 -> 37.1 us, 3584 x 3584 18.6 -> 15.8, 5120 x 5120 29.7 -> 21.4)
-// (DL_256x320: eight waves of 64 x 160, 246 registers, 144 KB of slabs; float slabs of a split K only, since a bfloat16
+// products at the rate one compute unit reaches with that shape.  The figures are fitted to measurements of every shape at 16 to 8192 rows
+// against 27 matrices (the Qwen2.5 models' and those 2048 to 16384 wide of the other designs), whole and split: a product gets a shape whose time is 1.005 of the
+// fastest shape's on average over those 320 sizes, 1.14 at most (1.07 and 1.8 with the figures fitted to 2048 rows alone).
+// (DL_128x128_S4: 128 x 128 with four slabs in shared memory, one work-group to a compute unit: where the tiles are one round of work-groups, what
+// counts is how many bytes a work-group has on their way: 2048 x 2048 x 8192 69.6 us against 102.7 with two slabs, 2048 x 2048 x 2048 21.1 against 25.9, 400 x 7168 x 5120
+// 1.8 times as fast; with more tiles than units two work-groups of two slabs each share a unit: 2048 x 8192 x 2048 65.5 us against 75.2)
+// (DL_256x320: eight waves of 64 x 160, 250 registers, 144 KB of slabs; float slabs of a split K only, since a bfloat16
 // result tile of 160 KB does not fit its slab buffers.  It is there for thousands of rows against a matrix 5120 wide:
 // 2048 rows are 160 tiles of 256 x 256, which leave 96 of 256 compute units idle, and 128 of these, which with K in
-// two halves are one round of 256 work-groups.  Measured at 2048 rows, slabs written: 5120 x 27648 504 us against
-// 651 whole and 573 in three parts of 256 x 256; 5120 x 13824 263 against 324 and 306; 5120 x 5120 112 against 140
-// and 132.  Its rate here is the one it reaches with all compute units busy, lower than a tile's that runs on 160.)
+// two halves are one round of 256 work-groups.  Measured at 2048 rows, slabs written: 5120 x 27648 430 us against
+// 480 in three parts of 256 x 256 and 546 in two of 256 x 160; 5120 x 13824 218 against 259 and 280.)
 // (DL_256x160: four waves of 64 x 160, for matrices 5120 wide as well: 2048 rows are 256 tiles, one to a compute
 // unit, and 4096 rows two rounds of them where tiles of 256 x 256 take one and a quarter.  A compute unit gets through
 // a slab of it hardly faster than through one of 256 x 256 (what a slab costs is mostly its requests, 52 against 64,
-// not its products, 40 against 64), so it wins only where it fills rounds that the square tile leaves part empty.
-// Measured, whole products: 2048 x 5120 x 13824 261 us against 274-296; 2048 x 5120 x 5120 97 against 106; at 4096
-// rows 499 against 585 and 202 against 239; 4096 x 4608 x 3584 130 against 158.  Eight waves of 32 x 160: 265, 99.)
+// not its products, 40 against 64), so it wins only where it fills rounds that the square tile leaves part empty.)
+// (Tiles of 256 x 224, which fill the rounds of matrices 3584 and 7168 wide, are at most 4 % faster than the best of these anywhere: a chip with
+// idle compute units runs the others at a higher clock.)
 enum DlTile { DL_64x64, DL_64x256, DL_128x128, DL_128x256, DL_256x128, DL_192x256, DL_256x192, DL_256x256, DL_64x128, DL_128x128_S4, DL_64x192, DL_128x192, DL_64x320, DL_256x320, DL_256x160, DL_TILES };
 static const int DL_BM[DL_TILES] = {64, 64, 128, 128, 256, 192, 256, 256, 64, 128, 64, 128, 64, 256, 256};
 static const int DL_BN[DL_TILES] = {64, 256, 128, 256, 128, 256, 192, 256, 128, 128, 192, 192, 320, 320, 160};
-static const double DL_RATE[DL_TILES] = {2.45e12, 3.3e12, 4.2e12, 4.6e12, 4.8e12, 5.2e12, 5.2e12, 6.1e12, 2.1e12, 4.2e12, 3.0e12, 4.4e12, 3.5e12, 5.5e12, 4.3e12};   // FLOP/s of one compute unit
-static const double DL_FIXED[DL_TILES] = {2.7e-6, 11.5e-6, 5.5e-6, 11e-6, 15e-6, 6e-6, 8e-6, 14e-6, 5e-6, 4.5e-6, 9e-6, 9e-6, 12e-6, 10e-6, 10e-6};       // seconds per tile
 
 // Seconds for `groups` work-groups of tile t over k columns each.  The two smallest tiles run two
 // to a compute unit: each then works at half the unit's rate, and one that has a unit to itself
-// (not more work-groups than units) at about 0.62 of it.  With few rows the products wait for the
-// operands: a compute unit fills its shared memory at about 40 GB/s, and a work-group draws its BN
+// (not more work-groups than units) at about 0.87 of it.  With few rows the products wait for the
+// operands: a compute unit fills its shared memory at about 69 GB/s, and a work-group draws its BN
 // rows of weights and its BM rows of x alike (x as often as there are tiles along N: with 64 x 64 tiles
-// as many bytes of x as of weights).  Measured at 17-64 rows: on the 14B's gate/up matrix 108 work-groups
-// of 64 x 256 take 81 us, 216 of 64 x 128 take 56-59, 432 of 64 x 64 (two to a unit) 59-68; on the 7B's
-// 148 of 64 x 256 take 55-60 and 592 of 64 x 64 take 57-66; on the LM head at 128 rows 594 of 128 x 256
-// take 239 and 1188 of 128 x 128 take 266.  `weights_only`: the estimates of plan_dl_split (whether and how to
-// split K over work-groups, a few hundred rows against a narrow matrix) count the weights alone, at 32 GB/s,
-// which is what its plans were fitted with: with x counted they came out a tenth slower at 512 rows against
-// the down projections (87 against 82 us on the 7B's).
-static double dl_estimate(DlTile t, long groups, int k, bool weights_only = false) {
+// as many bytes of x as of weights).  Measured at 64 rows: on the 14B's gate/up matrix 108 work-groups
+// of 64 x 256 take 80 us, 216 of 64 x 128 59, 432 of 64 x 64 (two to a unit) 68.
+struct DlFigures {
+    double rate[DL_TILES], fixed[DL_TILES];      // FLOP/s of one compute unit; seconds per tile
+    double stream, alone, lag;                   // bytes per second of a compute unit; see above; a factor on single rounds of 128 x 128
+    bool x_counts;                               // whether the rows of x count as bytes that a work-group draws
+};
+static double dl_estimate(const DlFigures& f, DlTile t, long groups, int k) {
     const bool pairs = t == DL_64x64 || t == DL_128x128;
     const double products = 2.0 * DL_BM[t] * DL_BN[t] * k;
-    const double stream = weights_only ? 2.0 * DL_BN[t] * k / 32e9 : 2.0 * (DL_BN[t] + DL_BM[t]) * k / 40e9;
+    const double stream = 2.0 * (DL_BN[t] + (f.x_counts ? DL_BM[t] : 0)) * k / f.stream;
     const int cus = TL_COMPUTE_UNITS;
-    if (!pairs) return (double)((groups + cus - 1) / cus) * fmax(products / DL_RATE[t] + DL_FIXED[t], stream);
-    const double rate = groups > cus ? DL_RATE[t] / 2 : DL_RATE[t] * 0.62;
-    // (a single round of 128 x 128 tiles runs a tenth behind this estimate: measured on the fused gate/up
-    // products of the 7B, 14B and 32B at 96 to 512 rows, where it otherwise displaced 128 x 256 tiles
-    // that were up to a fifth faster)
-    const double lag = (t == DL_128x128 && groups <= 2 * cus) ? 1.1 : 1.0;
-    return lag * (double)((groups + 2 * cus - 1) / (2 * cus)) * fmax(products / rate + DL_FIXED[t], groups > cus ? 2 * stream : stream);
+    if (!pairs) return (double)((groups + cus - 1) / cus) * fmax(products / f.rate[t] + f.fixed[t], stream);
+    const double rate = f.rate[t] * (groups > cus ? 0.5 : f.alone);
+    const double lag = t == DL_128x128 && groups <= 2 * cus ? f.lag : 1.0;
+    return lag * (double)((groups + 2 * cus - 1) / (2 * cus)) * fmax(products / rate + f.fixed[t], groups > cus ? 2 * stream : stream);
 }
+static const DlFigures DL_NOW = {
+    {2.52e12, 2.82e12, 3.71e12, 4.41e12, 5.38e12, 4.34e12, 5.27e12, 6.23e12, 1.89e12, 4.01e12, 3.0e12, 4.83e12, 3.5e12, 5.5e12, 4.48e12},
+    {2.7e-6, 9.5e-6, 5.5e-6, 11e-6, 8.4e-6, 11e-6, 9.1e-6, 15.4e-6, 3.1e-6, 5.2e-6, 9.7e-6, 10.6e-6, 12e-6, 5.1e-6, 10.6e-6}, 68.8e9, 0.87, 1.0, true};
+// The figures of the rule by which a product's result stays in 32 bits (gives_slabs below): those of slower kernels, and kept as they are, since what a
+// consumer reads in 32 bits is not to depend on how fast a tile has become.
+static const DlFigures DL_SLAB_RULE = {
+    {2.45e12, 3.3e12, 4.2e12, 4.6e12, 4.8e12, 5.2e12, 5.2e12, 6.1e12, 2.1e12, 4.2e12, 3.0e12, 4.4e12, 3.5e12, 5.5e12, 4.3e12},
+    {2.7e-6, 11.5e-6, 5.5e-6, 11e-6, 15e-6, 6e-6, 8e-6, 14e-6, 5e-6, 4.5e-6, 9e-6, 9e-6, 12e-6, 10e-6, 10e-6}, 32e9, 0.62, 1.1, false};
 
-static DlTile pick_dl_tile(int M, int N, int K, bool sw, double* estimate = nullptr, bool weights_only = false, int products = 1) {
+static long dl_tiles(DlTile t, int M, int N) { return (long)((M + DL_BM[t] - 1) / DL_BM[t]) * ((N + DL_BN[t] - 1) / DL_BN[t]); }
+
+static DlTile pick_dl_tile(int M, int N, int K, bool sw, int products = 1) {
     DlTile best = DL_128x128;
     double best_t = 1e30;
     for (int t = 0; t < DL_TILES; ++t) {
         if (sw && (t == DL_64x64 || t == DL_256x192 || t == DL_64x320 || t == DL_256x160)) continue;      // a wave of the fused gate needs whole 64-row blocks of weights
         if (t == DL_256x320) continue;      // float slabs of partial sums only: a bfloat16 result tile of 160 KB does not fit its slab buffers
-        const long tiles = (long)((M + DL_BM[t] - 1) / DL_BM[t]) * ((N + DL_BN[t] - 1) / DL_BN[t]) * products;
-        if (t == DL_128x128_S4 && (tiles > TL_COMPUTE_UNITS || M > 128)) continue;      // one round of work-groups, every weight drawn once
-        // (the split planner's unsplit baseline is fitted without the 192-wide tiles: with them it kept 512 rows against the
-        // 14B's query/key/value matrix whole, 74.8 us, where it used to split K, 53.9 us)
-        if (weights_only && (t == DL_64x192 || t == DL_128x192 || t == DL_64x320)) continue;
-        const double est = dl_estimate((DlTile)t, tiles, K, weights_only);
+        const long tiles = dl_tiles((DlTile)t, M, N) * products;
+        if (t == DL_128x128_S4 && tiles > TL_COMPUTE_UNITS) continue;      // one round of work-groups
+        const double est = dl_estimate(DL_NOW, (DlTile)t, tiles, K);
         if (est < best_t) { best_t = est; best = (DlTile)t; }
     }
-    if (estimate) *estimate = best_t;
     return best;
+}
+
+// K in `parts` ranges of k_per columns (a multiple of 64), none of them empty; 0 if there is no such split.
+static int dl_k_per(int K, int parts) {
+    const int k_per = ((K / 64 + parts - 1) / parts) * 64;
+    return (K + k_per - 1) / k_per == parts ? k_per : 0;
+}
+static const DlTile DL_ALONE[] = {DL_128x128_S4, DL_128x256, DL_256x128, DL_192x256, DL_256x192, DL_256x256, DL_256x320, DL_64x64};      // a compute unit to themselves
+static bool dl_can_split(DlTile t, int M, int N, int parts, int small_rows) {
+    const bool one_round = dl_tiles(t, M, N) * parts <= TL_COMPUTE_UNITS;
+    // (the small tile as for up to 64 rows, one work-group to a compute unit: 128 rows against the 7B's output
+    // projection 13.0 us in two parts where four parts of 128 x 128 take 17.0)
+    return t == DL_128x128_S4 ? one_round : t == DL_64x64 ? one_round && M <= small_rows : true;
+}
+
+// Whether a product of more than 64 rows whose consumer can add slabs up gives it float slabs: where K split over work-groups pays against a bfloat16
+// result, the slabs counted at their bytes once written and once read.
+static bool gives_slabs(int M, int N, int K) {
+    double whole = 1e30;
+    for (int t = 0; t < DL_TILES; ++t) {
+        if (t == DL_256x320 || t == DL_64x192 || t == DL_128x192 || t == DL_64x320) continue;
+        const long tiles = dl_tiles((DlTile)t, M, N);
+        if (t == DL_128x128_S4 && (tiles > TL_COMPUTE_UNITS || M > 128)) continue;
+        whole = fmin(whole, dl_estimate(DL_SLAB_RULE, (DlTile)t, tiles, K));
+    }
+    whole += (double)M * N * 2 * 2 / 3e12;
+    for (DlTile t : DL_ALONE)
+        for (int P = 2; P <= 8 && K / P >= 512; ++P) {
+            const int k_per = dl_k_per(K, P);
+            if (k_per && dl_can_split(t, M, N, P, 128) &&
+                1.1 * dl_estimate(DL_SLAB_RULE, t, dl_tiles(t, M, N) * P, k_per) + (double)P * M * N * 4 * 2 / 3e12 < whole) return true;
+        }
+    return false;
 }
 
 // More than 64 rows against a matrix whose output tiles leave compute units idle (a few hundred rows
 // of a prompt portion against the down projection, say): K split over `parts` work-groups per tile
-// into float slabs that the consumer adds up.  Only the tiles that have a compute unit to themselves
-// are considered; the slabs cost their bytes once written and once read.  parts == 1: no split pays.
+// into float slabs that the consumer adds up, or one float slab where a tile's own rounds fill the chip better (1457 x 2048 x 5632: 45.7 us in four parts of 192 x
+// 256, 37.2 in one of 128 x 128 with four slabs; 400 x 7168 x 5120 53 and 41).  Split, only the tiles that have a compute unit to themselves
+// are considered; the slabs cost their bytes once written and once read.  parts == 0: a bfloat16 result.
+// Fitted like the tiles' figures, with the slabs' reading counted at 4 TB/s: the choice takes 1.01 of the fastest's time on average.
 struct DlSplit { DlTile tile; int parts; int k_per; };
 static DlSplit plan_dl_split(int M, int N, int K) {
-    double best_t;
-    DlSplit best{pick_dl_tile(M, N, K, false, &best_t, true), 1, 0};
-    best_t += (double)M * N * 2 * 2 / 3e12;
-    const int steps = K / 64;
-    static const DlTile alone[] = {DL_128x128_S4, DL_128x256, DL_256x128, DL_192x256, DL_256x192, DL_256x256, DL_256x320, DL_64x64};
-    for (DlTile t : alone) {
-        const long tiles = (long)((M + DL_BM[t] - 1) / DL_BM[t]) * ((N + DL_BN[t] - 1) / DL_BN[t]);
+    DlSplit best{DL_128x128, 0, 0};
+    if (!gives_slabs(M, N, K)) return best;
+    double best_t = 1e30;
+    auto consider = [&](DlTile t, int P, int k_per) {
+        // (a tenth on top: float slabs leave the kernel more slowly than the estimate's bfloat16 rows)
+        const double est = 1.11 * dl_estimate(DL_NOW, t, dl_tiles(t, M, N) * P, k_per) + (double)P * M * N * 5.9 / 3e12;
+        if (est < best_t) { best_t = est; best = DlSplit{t, P, k_per}; }
+    };
+    for (int t = 0; t < DL_TILES; ++t)
+        if (t != DL_128x128_S4 || dl_tiles((DlTile)t, M, N) <= TL_COMPUTE_UNITS) consider((DlTile)t, 1, K);
+    for (DlTile t : DL_ALONE)
         for (int P = 2; P <= 8 && K / P >= 512; ++P) {
-            const int k_per = ((steps + P - 1) / P) * 64;
-            if ((K + k_per - 1) / k_per != P) continue;
-            if (t == DL_128x128_S4 && tiles * P > TL_COMPUTE_UNITS) continue;       // measured in one round of work-groups only
-            // (the small tile as for up to 64 rows, one work-group to a compute unit: 128 rows against the 7B's output
-            // projection 13.0 us in two parts where four parts of 128 x 128 take 17.0)
-            if (t == DL_64x64 && (M > 128 || tiles * P > TL_COMPUTE_UNITS)) continue;
-            // (a tenth on top: float slabs leave the kernel more slowly than the estimate's bfloat16 rows)
-            const double est = 1.1 * dl_estimate(t, tiles * P, k_per, true) + (double)P * M * N * 4 * 2 / 3e12;
-            if (est < best_t) { best_t = est; best = DlSplit{t, P, k_per}; }
+            const int k_per = dl_k_per(K, P);
+            if (k_per && dl_can_split(t, M, N, P, 256)) consider(t, P, k_per);
         }
-    }
     return best;
 }
 
 // parts > 1 (float results only): K is split into `parts` ranges of k_per columns and out holds that many [M, ldo] slabs.
-template <int BM, int BN, int WGM, int WGN, int STAGES, typename TOut, int SW, int TK = 64>
+template <int BM, int BN, int WGM, int WGN, int STAGES, typename TOut, int SW>
 static int launch_dl_tile_t(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int N, int K,
                             int ldx, int ldo, int out_cols, hipStream_t stream, int parts = 1, int k_per = 0, Groups gr = Groups{}) {
-    constexpr size_t lds = (size_t)STAGES * dl_slab_rows(BM, BN, WGM * WGN, TK) * TK * sizeof(bf16_t);
+    constexpr size_t lds = (size_t)STAGES * dl_slab_rows(BM, BN, WGM * WGN) * 64 * sizeof(bf16_t);
     // (a lane's offset from its tile's first row is kept in 32 bits)
     TL_REQUIRE((long)(BM > BN ? BM : BN) * (ldx > K ? ldx : K) * 2 < (1L << 31), "gemm_dl_tile: rows of %d elements are too long", ldx > K ? ldx : K);
-    auto kernel = gemm_dl_tile_kernel<BM, BN, WGM, WGN, STAGES, TOut, SW, TK>;
+    auto kernel = gemm_dl_tile_kernel<BM, BN, WGM, WGN, STAGES, TOut, SW>;
     static hipError_t allowed = allow_lds(kernel, lds);
     if (allowed != hipSuccess) {
         tl_set_error("gemm_dl_tile: cannot get %zu bytes of shared memory: %s", lds, hipGetErrorString(allowed));
@@ -1354,7 +1386,7 @@ static int launch_dl_tile(DlTile tile, const void* x, const void* w, const void*
     case DL_256x192:
         if constexpr (!SW) return launch_dl_tile_t<256, 192, 4, 2, 2, TOut, false>(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, out_cols, stream, parts, k_per, gr);
         else break;
-    case DL_256x256: return launch_dl_tile_t<256, 256, 4, 2, 2, TOut, SW>(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, out_cols, stream, parts, k_per, gr);
+    case DL_256x256: return launch_dl_tile_t<256, 256, 2, 4, 2, TOut, SW>(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, out_cols, stream, parts, k_per, gr);
     case DL_256x160:
         if constexpr (!SW) return launch_dl_tile_t<256, 160, 4, 1, 2, TOut, false>(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, out_cols, stream, parts, k_per, gr);
         else break;
@@ -1686,7 +1718,10 @@ extern "C" int tl_gemm_partials_pay(int M, int N, int K);
 
 // How many parts tl_gemm_partials would use.
 extern "C" int tl_gemm_partials_parts(int M, int N, int K) {
-    if (M > 64 && K % 64 == 0) return plan_dl_split(M, N, K).parts;
+    if (M > 64 && K % 64 == 0) {
+        const int parts = plan_dl_split(M, N, K).parts;
+        return parts > 0 ? parts : 1;
+    }
     if (partials_on_tiles(M, N, K)) {
         const long tiles = (long)((M + 63) / 64) * ((N + 63) / 64);
         int P = (int)(TL_COMPUTE_UNITS / tiles);          // about one work-group per compute unit
@@ -1701,6 +1736,7 @@ extern "C" int tl_gemm_partials_parts(int M, int N, int K) {
 }
 
 extern "C" int tl_gemm_partials_pay(int M, int N, int K) {
+    if (M > 64 && K % 64 == 0) return gives_slabs(M, N, K);
     return partials_on_tiles(M, N, K) && tl_gemm_partials_parts(M, N, K) > 1;
 }
 
@@ -1710,7 +1746,8 @@ extern "C" int tl_gemm_partials(const void* x, const void* w, void* out, int M, 
     TL_REQUIRE(K % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0,
                "gemm_partials: needs K and the row stride of x to be multiples of 8 and 16-byte aligned operands");
     if (M > 64 && K % 64 == 0) {
-        const DlSplit plan = plan_dl_split(M, N, K);
+        DlSplit plan = plan_dl_split(M, N, K);
+        if (plan.parts == 0) plan = DlSplit{pick_dl_tile(M, N, K, false), 1, 0};
         *parts = plan.parts;
         const int rc = launch_dl_tile<float, false>(plan.tile, x, w, nullptr, 0, out, M, N, K, ldx, N, 0, stream, plan.parts, plan.k_per);
         if (rc != TL_OK) return rc;
@@ -1760,7 +1797,7 @@ extern "C" int tl_gemm_groups(const void* x, long x_group, const void* w, void* 
     gr.stride = GroupStride{x_group, (long)N * K, out_group};
     const bool aligned = K % 8 == 0 && ldx % 8 == 0 && x_group % 8 == 0 && out_group % 8 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0;
     if (dtype == TL_DT_BF16 && aligned && K % 64 == 0 && (M > 32 || (M > 8 && (long)N * groups >= 16384))) {
-        const DlTile tile = pick_dl_tile(M, N, K, false, nullptr, false, groups);
+        const DlTile tile = pick_dl_tile(M, N, K, false, groups);
         const int rc = out_f32 ? launch_dl_tile<float, false>(tile, x, w, nullptr, 0, out, M, N, K, ldx, ldo, 0, stream, 1, 0, gr)
                                : launch_dl_tile<bf16_t, false>(tile, x, w, nullptr, 0, out, M, N, K, ldx, ldo, 0, stream, 1, 0, gr);
         if (rc != TL_OK) return rc;
