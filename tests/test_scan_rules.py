@@ -46,3 +46,14 @@ def test_fixed_decays_take_the_faster_way(lib, lens, heads, dim, vdim, want):
     ([1] * 63 + [64], 2, 128, 128, True), ([1] * 31 + [64] * 4, 2, 128, 128, False), ([256], 2, 128, 128, True), ([1] * 200 + [256], 2, 128, 128, True)])
 def test_the_matrix_memory_takes_the_faster_way(lib, lens, heads, dim, vdim, want):
     assert _pays(lib, 1, lens, heads, dim, vdim) == want
+
+
+# the delta rule (1) and the selective recurrence (2): steps whose two ways differ by a tenth or more where both were measured
+@pytest.mark.parametrize("mode, lens, heads, dim, vdim, want", [
+    (1, [256], 16, 128, 128, True), (1, [2048], 16, 128, 128, True), (1, [175, 250, 325, 400], 16, 128, 128, True), (1, [1] * 15 + [256], 16, 128, 128, True),
+    (1, [128] * 16, 32, 128, 128, False), (1, [275, 550, 825, 1100], 32, 128, 128, True), (1, [512], 4, 64, 64, True), (1, [128], 8, 256, 256, True),
+    (2, [512], 128, 128, 64, True), (2, [275, 550, 825, 1100], 128, 128, 64, True), (2, [256], 64, 128, 64, True)])
+def test_blocks_where_they_are_the_faster_way(lib, mode, lens, heads, dim, vdim, want):
+    from torchlet_amd.kernels import ops
+    p = ops.Portions.of(lens, ops.BLOCKS_FROM)
+    assert bool(lib.tl_blocks_pay(*(c_int(x) for x in (mode, p.tokens, p.longest, p.rest, heads, dim, vdim)))) == want

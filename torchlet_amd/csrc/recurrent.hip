@@ -4,6 +4,7 @@
 #include <limits.h>
 
 #include "common.h"
+#include <type_traits>
 
 // A barrier that orders shared memory only: __syncthreads() also waits for every fetch from memory that is on its
 // way (its fence covers global memory), which would end a prefetch at the first barrier after it.
@@ -1038,14 +1039,455 @@ static int launch_delta_scan(const void* qkv, const void* gates, const void* hea
     return TL_OK;
 }
 
+// ------------------------------------------------------------------ long portions in blocks: the delta rule and the selective recurrence
+// The token loop above is a chain of some 500 cycles a token, whatever else the GPU does (one prompt of 2048 tokens, 16 heads: 412 us on 128 work-groups).  Over a block of
+// 16 tokens the recurrence is a few products of small matrices, with S the state before the block, g the decays, G_i = prod_{l <= i} g_l and D_ij = prod_{j < l <= i} g_l:
+//   L_ij = beta_i (k_i . k_j) D_ij below the diagonal;   U = (1 + L)^-1 diag(beta) (V - diag(G) K S);   O = diag(G) Q S + (Q K^T o D) U;   S <- G_16 S + K^T diag(w) U,  w_j = D_16,j
+// (the selective recurrence: U = diag(beta) V).  What does not need the state, T = (1 + L)^-1 diag(beta), P = Q K^T o D, G and w, is made for all blocks at once by
+// block_matrices_kernel (the inverse by substitution, and the decays' products, in 64 bits; no quotients, so a decay of zero is one); block_scan_kernel then walks a request's
+// blocks with the state in registers: products in true 32-bit on v_mfma_f32_16x16x4_f32, whose result layout (lane l: rows 4 (l / 16) + v of column l % 16) is the
+// layout of its right operand, so state, U and V never change lanes.  A work-group owns 16 columns, each of four waves a quarter of their rows: one barrier a block, for the
+// quarters' shares of K S and Q S; a fifth wave makes the outputs, a block behind.  What bounds it: a block's chain of products (29 matrix instructions of 32 cycles a wave, four of them one after the other for U), the exchange and a wait for operands, some 2700 cycles for
+// 16 tokens: 2048 tokens, 16 heads of 128 x 128 413 -> 162 us.  Errors against 64 bits (1500 tokens, whole outputs; loop / blocks): slow decays 1.5e-7 to 1.75e-7 / 1.0e-7, fast ones 7.0e-8 / 6.5e-8, selective 1.1e-7 / 0.8e-7.
+// Requests of few tokens in the step stay with the token loop, whose bits do not depend on how a request is cut into steps; blocks are counted from the step's first token of the request.
+#define BL_T 16                 // tokens of a block
+
+typedef float bl_f32x4 __attribute__((ext_vector_type(4)));
+
+// A block's and head's numbers in scratch.
+template <int MODE> struct BlockPlaces {
+    static constexpr int P = 0, G = 256, W = 272, PD = 288, TD = 304, T = 320, FLOATS = MODE == 1 ? 576 : 304;      // (PD, TD: the diagonals, zero in P and T)
+};
+
+__device__ __forceinline__ int bl_blocks(const int* __restrict__ req_indptr, int r, int least) {
+    const int n = req_indptr[r + 1] - req_indptr[r];
+    return n >= least ? (n + BL_T - 1) / BL_T : 0;
+}
+
+// One wave for a block, the heads that share its keys four at a time.
+template <int MODE>
+__global__ void __launch_bounds__(64)
+block_matrices_kernel(const float* __restrict__ qkv, const float* __restrict__ gates, const int* __restrict__ req_indptr, float* __restrict__ scratch,
+                      int requests, int heads, int kv_heads, int dim, int vdim, int least) {
+    __shared__ double skk[BL_T][BL_T + 1], sqk[BL_T][BL_T + 1], sl[4][BL_T][BL_T + 1];
+    __shared__ float sg[4][BL_T], sb[4][BL_T];
+    const int lane = threadIdx.x, quad = lane >> 4, c = lane & 15;
+    int first = 0, req = -1, block0 = 0;
+    for (int base = 0; base < requests && req < 0; base += TL_WAVE) {
+        const int r = base + lane;
+        const int mine = r < requests ? bl_blocks(req_indptr, r, least) : 0;
+        int upto = mine;
+#pragma unroll
+        for (int o = 1; o < TL_WAVE; o <<= 1) {
+            const int t = __shfl_up(upto, o, TL_WAVE);
+            if (lane >= o) upto += t;
+        }
+        const unsigned long long past = __ballot(first + upto > (int)blockIdx.x);
+        if (past) {
+            const int l = __builtin_amdgcn_readfirstlane(__ffsll(past) - 1);
+            req = base + l;
+            block0 = first + __builtin_amdgcn_readlane(upto, l) - __builtin_amdgcn_readlane(mine, l);
+        }
+        first += __builtin_amdgcn_readlane(upto, TL_WAVE - 1);
+    }
+    if (req < 0) return;                                   // (the grid is an upper bound)
+    const int tok0 = req_indptr[req] + ((int)blockIdx.x - block0) * BL_T, nt = min(BL_T, req_indptr[req + 1] - tok0);
+    const int C = 2 * kv_heads * dim + heads * vdim, share = heads / kv_heads;
+    const int parts = (share + 3) / 4, kv = blockIdx.y / parts, in_share = (blockIdx.y % parts) * 4 + quad;
+    const bool live = in_share < share;
+    const int head = kv * share + min(in_share, share - 1);
+    const float* row = qkv + (size_t)(tok0 + min(c, nt - 1)) * C + kv * dim + 4 * quad;
+    // (sums of eight products each, joined in 64 bits: 128 of them in one chain double the error of what the block's own tokens contribute)
+    double kk[4] = {0.0, 0.0, 0.0, 0.0}, qk[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 2
+    for (int d0 = 0; d0 < dim; d0 += 32) {
+        bl_f32x4 ks[4], qs[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) ks[v] = qs[v] = bl_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int d = d0; d < d0 + 32; d += 16) {
+            float4 q = make_float4(0.f, 0.f, 0.f, 0.f), k = q;
+            if (d + 4 * quad < dim) {
+                q = *(const float4*)(row + d);
+                k = *(const float4*)(row + kv_heads * dim + d);
+            }
+            const float qa[4] = {q.x, q.y, q.z, q.w}, ka[4] = {k.x, k.y, k.z, k.w};
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                if (MODE == 1) ks[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[v], ka[v], ks[v], 0, 0, 0);
+                qs[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[v], ka[v], qs[v], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            if (MODE == 1) kk[v] += ((double)ks[0][v] + ks[1][v]) + ((double)ks[2][v] + ks[3][v]);
+            qk[v] += ((double)qs[0][v] + qs[1][v]) + ((double)qs[2][v] + qs[3][v]);
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        if (MODE == 1) skk[4 * quad + v][c] = kk[v];
+        sqk[4 * quad + v][c] = qk[v];
+    }
+    // (beyond the request's last token: beta = 0 and a decay of 1)
+    const float* gate = gates + (size_t)(tok0 + min(c, nt - 1)) * 2 * heads + head;
+    sb[quad][c] = c < nt ? gate[0] : 0.f;
+    sg[quad][c] = c < nt ? gate[heads] : 1.f;
+    shared_barrier();
+    float* to = scratch + ((size_t)blockIdx.x * heads + head) * BlockPlaces<MODE>::FLOATS;
+    const float beta = sb[quad][c];
+    double d = 1.0, all = sg[quad][0];                      // D_ic, and G_i
+#pragma unroll
+    for (int i = 0; i < BL_T; ++i) {
+        const double g = sg[quad][i];
+        if (i > 0) all *= g;
+        if (i > c) d *= g;
+        const float p = i >= c ? (float)(sqk[i][c] * d * (MODE == 1 ? 1.0 : (double)beta)) : 0.f;
+        if (live) to[BlockPlaces<MODE>::P + i * BL_T + c] = i > c ? p : 0.f;
+        if (live && i == c) to[BlockPlaces<MODE>::PD + c] = p;
+        if (MODE == 1) sl[quad][i][c] = i > c ? sb[quad][i] * skk[i][c] * d : 0.0;
+        if (live && c == 0) to[BlockPlaces<MODE>::G + i] = (float)all;
+    }
+    if (live) to[BlockPlaces<MODE>::W + c] = (float)(MODE == 1 ? d : d * beta);
+    if (MODE == 1) {
+        if (live) to[BlockPlaces<MODE>::TD + c] = beta;
+        shared_barrier();
+        double x[BL_T];                                     // column c of the inverse, times beta_c
+#pragma unroll
+        for (int i = 0; i < BL_T; ++i) {
+            double s = i == c ? (double)beta : 0.0;
+#pragma unroll
+            for (int l = 0; l < i; ++l) s -= sl[quad][i][l] * x[l];
+            x[i] = i >= c ? s : 0.0;
+            if (live) to[BlockPlaces<MODE>::T + i * BL_T + c] = i > c ? (float)x[i] : 0.f;
+        }
+    }
+}
+
+// sum_j m_ij r_j of a lane's rows i = 4 quad + v over j < i alone, number by number, with m as the matrix instruction's left operand (lane l: row l % 16, columns 4 (l / 16) and
+// up): where a later token's row of r is an infinity or a NaN, which the instruction would multiply by the zeros above the diagonal.  (From registers: a load here would make
+// the compiler wait for all that are on their way, on the usual path too.)
+__device__ __forceinline__ bl_f32x4 bl_lower_product(bl_f32x4 m, bl_f32x4 r) {
+    const int lane = threadIdx.x & 63, quad = lane >> 4, c = lane & 15;
+    bl_f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int j = 0; j < BL_T; ++j) {
+        const float rj = (j & 2) ? ((j & 1) ? r[3] : r[2]) : ((j & 1) ? r[1] : r[0]), mj = (j & 2) ? ((j & 1) ? m[3] : m[2]) : ((j & 1) ? m[1] : m[0]);
+        const float x = __shfl(rj, (j >> 2) * 16 + c, TL_WAVE);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const float y = __shfl(mj, (j >> 2) * 16 + 4 * quad + v, TL_WAVE);
+            if (j < 4 * quad + v) s[v] = fmaf(y, x, s[v]);
+        }
+    }
+    return s;
+}
+
+// MODE as the token loop's (1 or 2).  NT: a wave's rows in tiles of 16, 64 NT >= dim; WHOLE: 64 NT == dim.
+template <int MODE, int NT, bool WHOLE>
+__global__ void __launch_bounds__(320, NT <= 2 ? 3 : 2)
+block_scan_kernel(const float* __restrict__ qkv, const float* __restrict__ scratch, const float* __restrict__ head_skip, float* __restrict__ state, size_t slot_stride,
+                  const int* __restrict__ slots, const int* __restrict__ req_indptr, float* __restrict__ out, int heads, int kv_heads, int dim, int vdim, int least, int blocks) {
+    __shared__ bl_f32x4 part[3][2][4][TL_WAVE];              // the waves' shares of K S and Q S, of three blocks in turn: at a barrier the fifth wave still reads those of the block before
+    __shared__ bl_f32x4 su[2][TL_WAVE];                      // U
+    typedef BlockPlaces<MODE> Places;
+    // neighbouring heads, which share keys and queries, and all columns of a head on one XCD where that deals out evenly: what one work-group fetches the others find in its L2
+    const int req = blockIdx.z, head = heads % 8 == 0 ? (int)(blockIdx.x % 8) * (heads / 8) + (int)blockIdx.x / 8 : (int)blockIdx.x;
+    const int tok0 = req_indptr[req], tok1 = req_indptr[req + 1];
+    if (tok1 - tok0 < least) return;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TL_WAVE), lane = threadIdx.x % TL_WAVE, quad = lane >> 4, c = lane & 15;
+    int first = 0;
+    for (int base = 0; base < req; base += TL_WAVE) {
+        int mine = base + lane < req ? bl_blocks(req_indptr, base + lane, least) : 0;
+#pragma unroll
+        for (int o = TL_WAVE / 2; o > 0; o >>= 1) mine += __shfl_xor(mine, o, TL_WAVE);
+        first += mine;
+    }
+    first = __builtin_amdgcn_readfirstlane(first);
+    const int full = (tok1 - tok0) / BL_T, left = (tok1 - tok0) % BL_T;
+    if (first + full + (left > 0) > blocks) return;        // (more than the caller counted: nothing is read beyond the scratch)
+    const int C = 2 * kv_heads * dim + heads * vdim, kv = head / (heads / kv_heads), col = blockIdx.y * BL_T + c;
+    const float* q_base = qkv + (size_t)tok0 * C + kv * dim;
+    const float* k_base = q_base + kv_heads * dim;
+    const float* v_base = qkv + (size_t)tok0 * C + 2 * kv_heads * dim + (size_t)head * vdim;
+    const float* m_base = scratch + ((size_t)first * heads + head) * Places::FLOATS;
+    float* o_base = out + ((size_t)tok0 * heads + head) * vdim;
+    const int count = full + (left > 0);
+    auto total = [&](int block, int which) {
+        const bl_f32x4(&x)[4][TL_WAVE] = part[block % 3][which];
+        return (x[0][lane] + x[1][lane]) + (x[2][lane] + x[3][lane]);
+    };
+    auto odd = [&](const bl_f32x4& x) {
+        const float most = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
+        const float sum = (x[0] + x[1]) + (x[2] + x[3]);   // (a maximum passes a NaN over, a sum does not)
+        return __ballot(!(most <= 3.402823466e38f) || sum != sum) != 0;
+    };
+
+    if (wave == 4) {                                       // the outputs, a block behind the others
+        const float skip = MODE == 2 ? head_skip[head] : 0.f;
+        const unsigned value_at = (unsigned)min(col, vdim - 1);
+        struct { bl_f32x4 P, Pd, G, value; } ops[4];       // of four blocks, each requested when its place is free
+        auto fetch = [&](int place, int block) {
+            const float* m = m_base + (size_t)block * heads * Places::FLOATS;
+            ops[place].P = *(const bl_f32x4*)(m + Places::P + c * BL_T + 4 * quad);
+            ops[place].Pd = *(const bl_f32x4*)(m + Places::PD + 4 * quad);
+            ops[place].G = *(const bl_f32x4*)(m + Places::G + 4 * quad);
+            if (MODE == 2) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) ops[place].value[v] = v_base[(size_t)min(block * BL_T + 4 * quad + v, tok1 - tok0 - 1) * C + value_at];
+            }
+        };
+#pragma unroll
+        for (int i = 0; i < 4; ++i) fetch(i, min(i, count - 1));
+        shared_barrier();
+        auto outputs = [&](int i, int block) {
+            shared_barrier();                              // (the others' next block, or their end)
+            bl_f32x4 u, before = total(block, 1);
+            if (MODE == 1) u = su[block & 1][lane];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) if (MODE == 2) u[v] = block * BL_T + 4 * quad + v < tok1 - tok0 ? ops[i].value[v] : 0.f;
+            bl_f32x4 o = {0.f, 0.f, 0.f, 0.f};
+            if (odd(u)) o = bl_lower_product(ops[i].P, u);
+            else {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) o = __builtin_amdgcn_mfma_f32_16x16x4f32(ops[i].P[v], u[v], o, 0, 0, 0);
+            }
+            float* to = o_base + (size_t)block * BL_T * heads * vdim;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const float x = fmaf(ops[i].Pd[v], u[v], fmaf(ops[i].G[v], before[v], o[v]));
+                if (col < vdim && block * BL_T + 4 * quad + v < tok1 - tok0) to[(unsigned)((4 * quad + v) * heads * vdim + col)] = MODE == 2 ? fmaf(skip, u[v], x) : x;
+            }
+            fetch(i, min(block + 4, count - 1));
+        };
+        int block = 0;
+        for (; block + 3 < count; block += 4) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) outputs(i, block + i);
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            if (block + i < count) outputs(i, block + i);
+        return;
+    }
+
+    const int row0 = wave * 16 * NT;
+    float* st = state + (size_t)slots[req] * slot_stride + (size_t)head * vdim * dim + (size_t)min(col, vdim - 1) * dim;
+    bl_f32x4 S[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int r = row0 + 16 * t + 4 * quad;
+        S[t] = bl_f32x4{0.f, 0.f, 0.f, 0.f};
+        if (r < dim && col < vdim) S[t] = *(const bl_f32x4*)(st + r);
+    }
+
+    // A block's operands: keys and queries of token c as left operands of the products with S, keys of tokens 4 quad + v as that of the state's update, the block's matrices,
+    // values.  They are requested two blocks ahead (a trip to memory takes as long as a block's work), by a base that the wave shares and offsets of the lane's
+    // that never change and without a branch (behind one the compiler waits for every request on its way): rows beyond dim are copies, whose share of the state's update is
+    // zeroed, and the blocks are whole; a request's last, broken one has a fetch of its own.
+    struct Operands { bl_f32x4 k[NT], q[NT], T, G, w, Td; float kt[NT][4], v[4], all; } ops[2];
+    unsigned row_at[NT], turned_at[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        row_at[t] = (unsigned)(c * C + (WHOLE ? row0 + 16 * t + 4 * quad : min(row0 + 16 * t + 4 * quad, dim - 4)));
+        turned_at[t] = (unsigned)(4 * quad * C + (WHOLE ? row0 + 16 * t + c : min(row0 + 16 * t + c, dim - 1)));
+    }
+    const unsigned value_at = (unsigned)(4 * quad * C + min(col, vdim - 1));
+    auto fetch_rows = [&](Operands& n, int block) {
+        const float* kb = k_base + (size_t)block * BL_T * C;
+        const float* qb = q_base + (size_t)block * BL_T * C;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            if (MODE == 1) n.k[t] = *(const bl_f32x4*)(kb + row_at[t]);
+            n.q[t] = *(const bl_f32x4*)(qb + row_at[t]);
+        }
+    };
+    auto fetch_matrices = [&](Operands& n, int block) {
+        const float* m = m_base + (size_t)block * heads * Places::FLOATS;
+        if (MODE == 1) {
+            n.G = *(const bl_f32x4*)(m + Places::G + 4 * quad);
+            n.T = *(const bl_f32x4*)(m + Places::T + c * BL_T + 4 * quad);
+            n.Td = *(const bl_f32x4*)(m + Places::TD + 4 * quad);
+        }
+        n.w = *(const bl_f32x4*)(m + Places::W + 4 * quad);
+        n.all = m[Places::G + BL_T - 1];
+    };
+    auto fetch_rest = [&](Operands& n, int block) {
+        const float* kb = k_base + (size_t)block * BL_T * C;
+        const float* vb = v_base + (size_t)block * BL_T * C;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            n.v[v] = (vb + v * C)[value_at];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) n.kt[t][v] = (kb + v * C)[turned_at[t]];
+        }
+        fetch_matrices(n, block);
+    };
+    auto fetch_broken = [&](Operands& n, int block) {       // `left` tokens; the others' keys, queries and values are zeros (and their step sizes)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            n.k[t] = n.q[t] = bl_f32x4{0.f, 0.f, 0.f, 0.f};
+            if (c < left) {
+                if (MODE == 1) n.k[t] = *(const bl_f32x4*)(k_base + (size_t)block * BL_T * C + row_at[t]);
+                n.q[t] = *(const bl_f32x4*)(q_base + (size_t)block * BL_T * C + row_at[t]);
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const bool in = 4 * quad + v < left;
+            n.v[v] = in ? v_base[(size_t)(block * BL_T + v) * C + value_at] : 0.f;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) n.kt[t][v] = in ? k_base[(size_t)(block * BL_T + v) * C + turned_at[t]] : 0.f;
+        }
+        fetch_matrices(n, block);
+    };
+    // ahead: the block to request next, whole; broken: whether this is the last block of `left` tokens, behind which nothing is requested
+    auto work = [&](Operands& n, int block, int ahead, auto broken) {
+        // K S, then Q S, four sums each; K S is exchanged while Q S is made
+        bl_f32x4 a[4], b[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) a[v] = b[v] = bl_f32x4{0.f, 0.f, 0.f, 0.f};
+        if (MODE == 1) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) a[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(n.k[t][v], S[t][v], a[v], 0, 0, 0);
+        }
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) b[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(n.q[t][v], S[t][v], b[v], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        bl_f32x4(&shares)[2][4][TL_WAVE] = part[block % 3];
+        if (MODE == 1) {
+            shares[0][wave][lane] = (a[0] + a[1]) + (a[2] + a[3]);
+            shared_barrier();
+        }
+        const bl_f32x4 value = {n.v[0], n.v[1], n.v[2], n.v[3]};
+        bl_f32x4 u = value, r = value;
+        if (MODE == 1) {
+            const bl_f32x4 sum = total(block, 0);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                r[v] = fmaf(-n.G[v], sum[v], value[v]);
+                if (broken && 4 * quad + v >= left) r[v] = 0.f;
+            }
+            // (the diagonal's share, the largest, goes in last and once: in the matrix instruction every small one after it would be rounded at its size)
+            u = bl_f32x4{0.f, 0.f, 0.f, 0.f};
+            if (odd(r)) u = bl_lower_product(n.T, r);
+            else {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) u = __builtin_amdgcn_mfma_f32_16x16x4f32(n.T[v], r[v], u, 0, 0, 0);
+            }
+        }
+        if (!broken) fetch_rows(n, ahead);
+        shares[1][wave][lane] = (b[0] + b[1]) + (b[2] + b[3]);      // (for the fifth wave, behind the next barrier)
+        if (MODE == 1) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                u[v] = fmaf(n.Td[v], r[v], u[v]);
+                if (broken && 4 * quad + v >= left) u[v] = 0.f;
+            }
+            if (wave == 0) su[block & 1][lane] = u;
+        }
+        bl_f32x4 more[NT];                                  // (apart from S, which is rounded once a block)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) more[t] = bl_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const float wu = n.w[v] * u[v];
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+                more[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(WHOLE || row0 + 16 * t + c < dim ? n.kt[t][v] : 0.f, wu, more[t], 0, 0, 0);
+        }
+        const float all = n.all;
+        if (!broken) fetch_rest(n, ahead);
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) S[t][v] = fmaf(all, S[t][v], more[t][v]);
+        if (MODE == 2) shared_barrier();
+    };
+    if (full > 0) {
+        fetch_rows(ops[0], 0);
+        fetch_rest(ops[0], 0);
+        fetch_rows(ops[1], min(1, full - 1));
+        fetch_rest(ops[1], min(1, full - 1));
+    }
+    int block = 0;
+    for (; block + 1 < full; block += 2) {                  // (no way past one of the two: behind it the compiler would wait for what the other requests)
+        work(ops[0], block, min(block + 2, full - 1), std::false_type{});
+        work(ops[1], block + 1, min(block + 3, full - 1), std::false_type{});
+    }
+    if (block < full) work(ops[0], block, full - 1, std::false_type{});
+    if (left > 0) {
+        fetch_broken(ops[0], full);
+        work(ops[0], full, full, std::true_type{});
+    }
+    shared_barrier();                                       // the last block's outputs
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int r = row0 + 16 * t + 4 * quad;
+        if (r < dim && col < vdim) *(bl_f32x4*)(st + r) = S[t];
+    }
+}
+
+// Numbers of scratch for so many blocks.
+extern "C" long tl_blocks_floats(int mode, int blocks, int heads) { return (long)blocks * heads * (mode == 1 ? BlockPlaces<1>::FLOATS : BlockPlaces<2>::FLOATS); }
+
+// Whether a step's long portions (`tokens` in all, the longest of so many) go through the blocks, beside `rest` requests of a few tokens: two estimates in us, fitted to the device's times
+// below.  The loop's and the blocks' time is a chain along the longest portion and, where the work-groups outnumber the chip, about the same work on both ways; the
+// matrices are what the blocks cost more.
+// Measured (us, loop / blocks): the delta rule, 16 heads of 128 x 128: 128 tokens 28 / 27, 256 51 / 32, 512 107 / 49, 2048 413 / 162; 175 to 400 tokens 97 / 66, 275 to 1100 247 / 139, 16 x 128 107 / 114;
+// 32 heads: 2048 423 / 169, 16 x 128 183 / 208; 4 heads of 64 x 64: 512 73 / 36, 2048 283 / 116; 8 heads of 256 x 256: 128 68 / 32, 2048 1103 / 251; the selective recurrence, 128 heads of 128 x 64: 512 101 / 50, 2048 395 / 160, 275 to 1100 405 / 263, 16 x 128 243 / 220.
+extern "C" int tl_blocks_pay(int mode, int tokens, int longest, int rest, int heads, int dim, int vdim) {
+    const double groups = (double)heads * ((vdim + BL_T - 1) / BL_T), rows = (dim + 63) / 64;
+    const double work = tokens * groups * 256.0 / tl_mlstm_units * fmax(1.0, rows / 2);
+    const double loop = 5 + hypot(longest * (rows > 3 ? 0.53 : 0.07 + 0.065 * rows), work * (mode == 1 ? 3.7e-4 : 2.3e-4));
+    const double blocks = 14 + tokens * (double)heads * (mode == 1 ? 1.2e-4 : 0.6e-4) + (rest > 0 ? 8 : 0) + hypot(longest * (0.03 + 0.024 * rows), work * (mode == 1 ? 3.5e-4 : 1.85e-4));
+    return blocks < loop;
+}
+
+// Whether the requests of `least` tokens and more can go through the blocks: whole pieces of four numbers, and scratch for all of them.
+static bool blocks_fit(int mode, const void* qkv, int heads, int kv_heads, int dim, int vdim, const void* state, long slot_stride, int blocks, const void* scratch, long floats) {
+    return scratch && blocks > 0 && floats >= tl_blocks_floats(mode, blocks, heads) && dim % 4 == 0 && (2 * kv_heads * dim + heads * vdim) % 4 == 0 && ((uintptr_t)qkv & 15) == 0 &&
+           ((uintptr_t)state & 15) == 0 && slot_stride % 4 == 0 && ((uintptr_t)scratch & 15) == 0 && (long)kv_heads * ((heads / kv_heads + 3) / 4) <= 65535;
+}
+
+template <int MODE>
+static void launch_blocks(const void* qkv, const void* gates, const void* skip, void* state, long slot_stride, const void* slots, const void* req_indptr, void* out,
+                          int requests, int heads, int kv_heads, int dim, int vdim, int least, int blocks, void* scratch, hipStream_t stream) {
+    const dim3 mgrid(blocks, kv_heads * ((heads / kv_heads + 3) / 4)), grid(heads, (vdim + BL_T - 1) / BL_T, requests);
+    block_matrices_kernel<MODE><<<mgrid, 64, 0, stream>>>((const float*)qkv, (const float*)gates, (const int*)req_indptr, (float*)scratch, requests, heads, kv_heads, dim, vdim, least);
+#define TL_BLOCKS_W(N, W) block_scan_kernel<MODE, N, W><<<grid, 320, 0, stream>>>((const float*)qkv, (const float*)scratch, (const float*)skip, (float*)state, (size_t)slot_stride, \
+        (const int*)slots, (const int*)req_indptr, (float*)out, heads, kv_heads, dim, vdim, least, blocks)
+#define TL_BLOCKS(N) if (dim == 64 * N) TL_BLOCKS_W(N, true); else TL_BLOCKS_W(N, false)
+    if (dim <= 64) { TL_BLOCKS(1); }
+    else if (dim <= 128) { TL_BLOCKS(2); }
+    else if (dim <= 192) { TL_BLOCKS(3); }
+    else { TL_BLOCKS(4); }
+#undef TL_BLOCKS_W
+#undef TL_BLOCKS
+}
+
+// With scratch (null: the token loop alone) requests of at least `least` tokens go through the blocks where the rows allow it (`blocks`: no fewer than they make), and the
+// token loop takes the others (rest: how many there are, or more if the caller cannot tell; 0 only if there are none), of about rest_longest tokens at most.
 extern "C" int tl_delta_scan(const void* qkv, const void* gates, void* state, long slot_stride, const void* slots, const void* req_indptr,
-                             void* out, int requests, int heads, int kv_heads, int dim, int vdim, int tokens, int longest, hipStream_t stream) {
+                             void* out, int requests, int heads, int kv_heads, int dim, int vdim, int tokens, int longest, int least, int blocks, int rest,
+                             int rest_longest, void* scratch, long scratch_floats, hipStream_t stream) {
     TL_REQUIRE(requests >= 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && dim > 0 && vdim > 0, "delta_scan: bad sizes");
     TL_REQUIRE(dim <= DELTA_L * 16, "delta_scan: built for up to %d query/key dimensions per head, got %d", DELTA_L * 16, dim);
     TL_REQUIRE(slot_stride >= (long)heads * dim * vdim, "delta_scan: the state rows are too short");
     TL_REQUIRE(requests <= 65535 && heads <= 65535, "delta_scan: too many requests or heads for one launch");
     if (requests == 0) return TL_OK;
-    launch_delta_scan<1>(qkv, gates, nullptr, state, slot_stride, slots, req_indptr, out, requests, heads, kv_heads, dim, vdim, tokens, longest, INT_MAX, stream);
+    const bool through = blocks_fit(1, qkv, heads, kv_heads, dim, vdim, state, slot_stride, blocks, scratch, scratch_floats);
+    if (through) {
+        launch_blocks<1>(qkv, gates, nullptr, state, slot_stride, slots, req_indptr, out, requests, heads, kv_heads, dim, vdim, least, blocks, scratch, stream);
+        TL_CHECK_LAUNCH("delta_blocks");
+        if (rest == 0) return TL_OK;
+    }
+    launch_delta_scan<1>(qkv, gates, nullptr, state, slot_stride, slots, req_indptr, out, requests, heads, kv_heads, dim, vdim, through ? rest * rest_longest : tokens,
+                         through ? rest_longest : longest, through ? least : INT_MAX, stream);
     TL_CHECK_LAUNCH("delta_scan");
     return TL_OK;
 }
@@ -1999,13 +2441,21 @@ extern "C" int tl_decay_scan(const void* qkv, const void* decay, void* state, lo
 // state + heads * vdim] as selective_prepare leaves it (C, B, x), gates float [T, 2 * heads] (dt, decay), skip float [heads] (D); the
 // state as the delta rule's ([vdim][state] per head), out float [T, heads * vdim].
 extern "C" int tl_selective_scan(const void* qkv, const void* gates, const void* skip, void* state, long slot_stride, const void* slots,
-                                 const void* req_indptr, void* out, int requests, int heads, int groups, int dim, int vdim, int tokens, int longest, hipStream_t stream) {
+                                 const void* req_indptr, void* out, int requests, int heads, int groups, int dim, int vdim, int tokens, int longest, int least, int blocks,
+                                 int rest, int rest_longest, void* scratch, long scratch_floats, hipStream_t stream) {
     TL_REQUIRE(requests >= 0 && heads > 0 && groups > 0 && heads % groups == 0 && dim > 0 && vdim > 0 && gates && skip, "selective_scan: bad sizes");
     TL_REQUIRE(dim <= DELTA_L * 16, "selective_scan: built for states of up to %d numbers per column, got %d", DELTA_L * 16, dim);
     TL_REQUIRE(slot_stride >= (long)heads * dim * vdim, "selective_scan: the state rows are too short");
     TL_REQUIRE(requests <= 65535 && heads <= 65535, "selective_scan: too many requests or heads for one launch");
     if (requests == 0) return TL_OK;
-    launch_delta_scan<2>(qkv, gates, skip, state, slot_stride, slots, req_indptr, out, requests, heads, groups, dim, vdim, tokens, longest, INT_MAX, stream);
+    const bool through = blocks_fit(2, qkv, heads, groups, dim, vdim, state, slot_stride, blocks, scratch, scratch_floats);
+    if (through) {
+        launch_blocks<2>(qkv, gates, skip, state, slot_stride, slots, req_indptr, out, requests, heads, groups, dim, vdim, least, blocks, scratch, stream);
+        TL_CHECK_LAUNCH("selective_blocks");
+        if (rest == 0) return TL_OK;
+    }
+    launch_delta_scan<2>(qkv, gates, skip, state, slot_stride, slots, req_indptr, out, requests, heads, groups, dim, vdim, through ? rest * rest_longest : tokens,
+                         through ? rest_longest : longest, through ? least : INT_MAX, stream);
     TL_CHECK_LAUNCH("selective_scan");
     return TL_OK;
 }

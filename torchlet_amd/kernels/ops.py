@@ -44,6 +44,8 @@ def _lib(name: str) -> ctypes.CDLL:
         _libs[name] = lib
         if name == "gemm" and torch.cuda.is_available():
             lib.tl_gemm_set_compute_units(c_int(compute_units()))
+        if name == "recurrent":
+            lib.tl_blocks_floats.restype = ctypes.c_long
         if name == "recurrent" and torch.cuda.is_available():
             lib.tl_mlstm_set_compute_units(c_int(compute_units()))
         if name == "experts" and torch.cuda.is_available():
@@ -1120,12 +1122,32 @@ def delta_prepare(proj: torch.Tensor, conv_w: torch.Tensor, gates: torch.Tensor,
                                      c_float(qscale), c_float(unit_eps), c_int(_dt(proj, "delta_prepare")), _stream()))
 
 
+# Portions of at least so many tokens go through blocks of 16 tokens in the delta rule and the selective recurrence, where a step's sizes make that the faster
+# way; the blocks' matrices stand in scratch of at most CHUNK_SCRATCH numbers (a step with more is the token loop's).
+BLOCKS_FROM = 128
+
+
+def _block_args(lib, mode: int, portions: Portions | None, T: int, R: int, heads: int, dim: int, vdim: int, max_new_tokens: int | None, device):
+    """Of the C entries: the tokens by which the loop alone sizes its batches, what goes through the blocks, what is left for the loop, the scratch (which the caller holds
+    until the launch)."""
+    most = max(1, T - R + 1) if max_new_tokens is None else max_new_tokens
+    portions = portions or Portions.bound(T, R, max_new_tokens, BLOCKS_FROM)
+    if portions.count and lib.tl_blocks_pay(*(c_int(x) for x in (mode, portions.tokens, portions.likely or portions.longest, portions.rest, heads, dim, vdim))):
+        blocks = portions.tokens // 16 + portions.count
+        floats = lib.tl_blocks_floats(c_int(mode), c_int(blocks), c_int(heads))
+        if floats <= CHUNK_SCRATCH:
+            scratch = torch.empty(floats, dtype=torch.float32, device=device)
+            return scratch, (c_int(most), c_int(BLOCKS_FROM), c_int(blocks), c_int(portions.rest), c_int(portions.rest_longest), _ptr(scratch), ctypes.c_long(floats))
+    return None, (c_int(most), c_int(BLOCKS_FROM), c_int(0), c_int(0), c_int(0), c_void_p(0), ctypes.c_long(0))
+
+
 def delta_scan(qkv: torch.Tensor, gates: torch.Tensor, state: torch.Tensor, slots: torch.Tensor, req_indptr: torch.Tensor, out: torch.Tensor,
-               heads: int, kv_heads: int, dim: int, vdim: int, max_new_tokens: int | None = None) -> None:
+               heads: int, kv_heads: int, dim: int, vdim: int, max_new_tokens: int | None = None, portions: Portions | None = None) -> None:
     """The gated delta rule over the step's tokens, request by request from the state its slot holds: ``qkv`` float32 ``[T, C]`` as
     :func:`delta_prepare` left it (queries, keys, values), ``gates`` float32 ``[T, 2 * heads]`` (beta, decay); head ``h`` of ``state[slot]``
     (float32, ``dim x vdim`` numbers from ``h * dim * vdim`` on, column by column: ``[vdim][dim]``) moves by ``S <- g S; u = beta (v - S^T k); S <- S + k u^T`` and ``out`` float32
-    ``[T, heads * vdim]`` receives ``S^T q``."""
+    ``[T, heads * vdim]`` receives ``S^T q``.  ``max_new_tokens``: about the most tokens that a request brings; ``portions`` (of :data:`BLOCKS_FROM`
+    tokens or more): what the host knows of the requests' lengths, exactly."""
     T = qkv.shape[0]
     R = req_indptr.numel() - 1
     C = 2 * kv_heads * dim + heads * vdim
@@ -1140,9 +1162,9 @@ def delta_scan(qkv: torch.Tensor, gates: torch.Tensor, state: torch.Tensor, slot
     _i32(slots, "slots", R)
     _i32(req_indptr, "req_indptr", R + 1)
     lib = _lib("recurrent")
+    scratch, blocks = _block_args(lib, 1, portions, T, R, heads, dim, vdim, max_new_tokens, qkv.device)
     _check(lib, lib.tl_delta_scan(_ptr(qkv), _ptr(gates), _ptr(state), ctypes.c_long(state.stride(0)), _ptr(slots), _ptr(req_indptr), _ptr(out),
-                                  c_int(R), c_int(heads), c_int(kv_heads), c_int(dim), c_int(vdim), c_int(T),
-                                  c_int(max(1, T - R + 1) if max_new_tokens is None else max_new_tokens), _stream()))
+                                  c_int(R), c_int(heads), c_int(kv_heads), c_int(dim), c_int(vdim), c_int(T), *blocks, _stream()))
 
 
 def decay_scan(qkv: torch.Tensor, decay: torch.Tensor, state: torch.Tensor, slots: torch.Tensor, req_indptr: torch.Tensor, out: torch.Tensor,
@@ -1209,12 +1231,12 @@ def selective_prepare(proj: torch.Tensor, x_off: int, conv_w: torch.Tensor, conv
 
 
 def selective_scan(qkv: torch.Tensor, gates: torch.Tensor, skip: torch.Tensor, state: torch.Tensor, slots: torch.Tensor, req_indptr: torch.Tensor,
-                   out: torch.Tensor, heads: int, groups: int, dim: int, vdim: int, max_new_tokens: int | None = None) -> None:
+                   out: torch.Tensor, heads: int, groups: int, dim: int, vdim: int, max_new_tokens: int | None = None, portions: Portions | None = None) -> None:
     """A selective state-space recurrence over the step's tokens, request by request from the state its slot holds: ``qkv`` float32 ``[T, 2 *
     groups * dim + heads * vdim]`` as :func:`selective_prepare` left it (C, B, x), ``gates`` float32 ``[T, 2 * heads]`` (dt, decay), ``skip``
     float32 ``[heads]``; head ``h`` (reading B and C of group ``h // (heads / groups)``) of ``state[slot]`` (float32, ``dim x vdim`` numbers from ``h *
     dim * vdim`` on, column by column: ``[vdim][dim]``) moves by ``S <- decay S + dt B x^T`` and ``out`` float32 ``[T, heads * vdim]`` receives
-    ``S^T C + skip[h] x``."""
+    ``S^T C + skip[h] x``.  ``max_new_tokens`` and ``portions`` as :func:`delta_scan`'s."""
     T = qkv.shape[0]
     R = req_indptr.numel() - 1
     C = 2 * groups * dim + heads * vdim
@@ -1231,9 +1253,9 @@ def selective_scan(qkv: torch.Tensor, gates: torch.Tensor, skip: torch.Tensor, s
     _i32(slots, "slots", R)
     _i32(req_indptr, "req_indptr", R + 1)
     lib = _lib("recurrent")
+    scratch, blocks = _block_args(lib, 2, portions, T, R, heads, dim, vdim, max_new_tokens, qkv.device)
     _check(lib, lib.tl_selective_scan(_ptr(qkv), _ptr(gates), _ptr(skip), _ptr(state), ctypes.c_long(state.stride(0)), _ptr(slots), _ptr(req_indptr),
-                                      _ptr(out), c_int(R), c_int(heads), c_int(groups), c_int(dim), c_int(vdim), c_int(T),
-                                      c_int(max(1, T - R + 1) if max_new_tokens is None else max_new_tokens), _stream()))
+                                      _ptr(out), c_int(R), c_int(heads), c_int(groups), c_int(dim), c_int(vdim), c_int(T), *blocks, _stream()))
 
 
 def silu_float(x: torch.Tensor, out: torch.Tensor) -> None:

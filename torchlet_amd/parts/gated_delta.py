@@ -94,7 +94,8 @@ class GatedDelta(StagedMixer):
         ops.delta_prepare(proj, self.w_conv, gates, self.a_log, self.dt_bias, cache.state, self.state_floats, ctx.slots, ctx.req_indptr,
                           ctx.token_req, qkv, self.heads, self.kv_heads, self.dim, self.vdim, self.taps, self.qscale, float(self.spec.unit_eps))
         o = torch.empty((T, self.v_width), dtype=torch.float32, device=h.device)
+        lengths = {"portions": ctx.portions(ops.BLOCKS_FROM)} if h.is_cuda else {}      # (which kernels take the step's requests)
         ops.delta_scan(qkv, gates, cache.state, ctx.slots, ctx.req_indptr, o, self.heads, self.kv_heads, self.dim, self.vdim,
-                       max_new_tokens=ctx.max_new_tokens)
+                       max_new_tokens=ctx.max_new_tokens, **lengths)
         ops.gated_head_norm(o, proj[:, self.channels:], self.w_norm, float(self.spec.norm_eps), out, self.heads, self.vdim,
                             gate="silu", gain=gain)

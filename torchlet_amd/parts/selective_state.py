@@ -82,8 +82,9 @@ class SelectiveState(StagedMixer):
         ops.selective_prepare(proj, self.inner, self.w_conv, self.b_conv, gates, self.a_log, self.dt_bias, cache.state, self.state_floats,
                               ctx.slots, ctx.req_indptr, ctx.token_req, cbx, self.heads, self.inner, self.gn, self.taps)
         y = torch.empty((T, self.inner), dtype=torch.float32, device=h.device)
+        lengths = {"portions": ctx.portions(ops.BLOCKS_FROM)} if h.is_cuda else {}      # (which kernels take the step's requests)
         ops.selective_scan(cbx, gates, self.skip, cache.state, ctx.slots, ctx.req_indptr, y, self.heads, self.groups, self.state, self.vdim,
-                           max_new_tokens=ctx.max_new_tokens)
+                           max_new_tokens=ctx.max_new_tokens, **lengths)
         # the gate comes before the norm, and the norm runs over norm_groups equal parts of the row
         ops.gated_head_norm(y, proj[:, : self.inner], self.w_norm, float(self.spec.norm_eps), out, self.spec.norm_groups,
                             self.inner // self.spec.norm_groups, gate="silu", gain=gain, gate_first=True)
