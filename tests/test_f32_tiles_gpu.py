@@ -1,0 +1,39 @@
+"""The 32-bit tile kernel's sizes of tiles give the same bits, and the elementwise activation in whole pieces those of the numbers one by one."""
+import math
+
+import pytest
+import torch
+
+from torchlet_amd.kernels import ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M", [17, 63, 64, 65, 129, 300])
+@pytest.mark.parametrize("N, K", [(64, 4), (65, 36), (127, 64), (130, 100), (516, 252)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_every_tile_gives_the_same_bits(M, N, K, bias):
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x, w = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda") / math.sqrt(K)
+    b = torch.randn(N, generator=g, device="cuda") if bias else None
+    out = {}
+    for tile in (4, 5, 6):
+        out[tile] = torch.full((M, N + 4), 7.0, device="cuda")
+        ops.linear_f32_variant(x, w, b, out[tile][:, :N], tile)
+        assert bool((out[tile][:, N:] == 7.0).all())
+    by_rule = torch.empty(M, N, device="cuda")
+    ops.linear(x, w, b, by_rule)
+    assert torch.equal(out[4], out[5]) and torch.equal(out[4], out[6]) and torch.equal(out[4][:, :N], by_rule)
+    want = x.double() @ w.double().T + (b.double() if bias else 0.0)
+    torch.testing.assert_close(by_rule.double(), want, rtol=2e-5, atol=8 * 2 ** -24 * math.sqrt(K))
+
+
+@pytest.mark.parametrize("n", [1, 7, 8, 2048, 2056, 2051, 256 * 8 * 3 + 8])
+@pytest.mark.parametrize("kind", ["relu2", "silu", "gelu_tanh", "gelu"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_activation_in_pieces(n, kind, dtype):
+    x = (torch.randn(n + 1, generator=torch.Generator().manual_seed(n)) * 2).to(dtype).cuda()
+    pieces, single = x[:n].clone(), torch.cat((x[:1], x[:n])).clone()[1:]          # (the second one begins off a 16-byte boundary)
+    ops.activation(pieces, kind)
+    ops.activation(single, kind)
+    assert torch.equal(pieces, single)

@@ -292,8 +292,8 @@ static void launch_gemv_f32(const void* x, const void* w, const void* bias, int 
 //
 // v_mfma_f32_32x32x2_f32 multiplies 32-bit operands and adds in 32-bit: it is no reduced-precision mode
 // (nothing is rounded to a shorter format on the way), and it runs at four times the rate of the
-// v_fma_f32 tile kernel above.  A work-group of four waves owns a tile of BM x 128 outputs (BM = 64 or
-// 128), a wave 32 FMB x 64 of them; slabs of 16 columns of both operands go through registers into shared
+// v_fma_f32 tile kernel above.  A work-group of four waves owns a tile of 64 FMB x 64 FNB outputs, a wave
+// 32 FMB x 32 FNB of them; slabs of 16 columns of both operands go through registers into shared
 // memory (two buffers, one barrier per slab).  A lane reads four neighbouring k of its row at once; lanes
 // 0-31 take k = 8c .. 8c+3 and lanes 32-63 k = 8c+4 .. 8c+7 of a chunk of eight, so instruction e of a chunk
 // multiplies k = 8c + e and 8c + 4 + e: which k meet in one instruction is free as long as both operands
@@ -301,15 +301,14 @@ static void launch_gemv_f32(const void* x, const void* w, const void* bias, int 
 // lies in its tile, so a row's result does not depend on the batch; it differs from the other 32-bit
 // kernels' by rounding (another order of the same sum).  Needs K % 4 == 0 and 16-byte aligned rows.
 typedef float gf_f32x16_t __attribute__((ext_vector_type(16)));
-#define GF_BN 128
 #define GF_TK 16
 #define GF_LD (GF_TK + 4)          // floats between rows in shared memory: 16-byte reads of 16 rows fall on all banks
-template <int FMB>
+template <int FMB, int FNB>
 __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                             const void* __restrict__ bias, int bias_f32,
                                                             float* __restrict__ out, int M, int N, int K, int ldx, int ldo) {
-    constexpr int BM = 64 * FMB;
-    constexpr int XL = BM * 4 / 256;                       // 16-byte pieces of x a thread moves per slab (1 or 2)
+    constexpr int BM = 64 * FMB, GF_BN = 64 * FNB;
+    constexpr int XL = BM * 4 / 256, WL = GF_BN * 4 / 256; // 16-byte pieces of x and of w a thread moves per slab
     __shared__ __attribute__((aligned(16))) float xs[2][BM * GF_LD];
     __shared__ __attribute__((aligned(16))) float ws[2][GF_BN * GF_LD];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -317,9 +316,9 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
     const int lr = lane & 31, lh = lane >> 5;
     const int m0 = blockIdx.y * BM, n0 = blockIdx.x * GF_BN;
 
-    gf_f32x16_t acc[2][FMB];
+    gf_f32x16_t acc[FNB][FMB];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < FNB; ++i)
 #pragma unroll
         for (int j = 0; j < FMB; ++j)
 #pragma unroll
@@ -327,7 +326,7 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
 
     // piece p of a slab: row p / 4, columns 4 (p % 4) .. + 4; rows past the end read the last row (never stored),
     // columns past K read the last whole piece and count as zero
-    float4 gx[XL], gw[2];
+    float4 gx[XL], gw[WL];
     auto fetch = [&](int k0) {
 #pragma unroll
         for (int i = 0; i < XL; ++i) {
@@ -336,7 +335,7 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
             if (k >= K) gx[i] = make_float4(0.f, 0.f, 0.f, 0.f);
         }
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < WL; ++i) {
             const int p = tid + 256 * i, k = k0 + 4 * (p & 3);
             gw[i] = *(const float4*)(w + (size_t)min(n0 + (p >> 2), N - 1) * K + min(k, K - 4));
             if (k >= K) gw[i] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -349,7 +348,7 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
             *(float4*)(&xs[buf][(p >> 2) * GF_LD + 4 * (p & 3)]) = gx[i];
         }
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < WL; ++i) {
             const int p = tid + 256 * i;
             *(float4*)(&ws[buf][(p >> 2) * GF_LD + 4 * (p & 3)]) = gw[i];
         }
@@ -364,13 +363,13 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
         const float* wb = ws[s & 1];
 #pragma unroll
         for (int c = 0; c < GF_TK / 8; ++c) {
-            float4 a[2], b[FMB];
+            float4 a[FNB], b[FMB];
 #pragma unroll
-            for (int i = 0; i < 2; ++i) a[i] = *(const float4*)(wb + (wn * 64 + i * 32 + lr) * GF_LD + 8 * c + 4 * lh);
+            for (int i = 0; i < FNB; ++i) a[i] = *(const float4*)(wb + (wn * 32 * FNB + i * 32 + lr) * GF_LD + 8 * c + 4 * lh);
 #pragma unroll
             for (int j = 0; j < FMB; ++j) b[j] = *(const float4*)(xb + (wm * 32 * FMB + j * 32 + lr) * GF_LD + 8 * c + 4 * lh);
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < FNB; ++i)
 #pragma unroll
                 for (int j = 0; j < FMB; ++j) {
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i].x, b[j].x, acc[i][j], 0, 0, 0);
@@ -390,10 +389,10 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
         const int m = m0 + wm * 32 * FMB + j * 32 + lr;
         if (m >= M) continue;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < FNB; ++i)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const int n = n0 + wn * 64 + i * 32 + 8 * g + 4 * lh;
+                const int n = n0 + wn * 32 * FNB + i * 32 + 8 * g + 4 * lh;
                 float v[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] = acc[i][j][4 * g + e] + ((bias && n + e < N) ? load_vec(bias, bias_f32, n + e) : 0.f);
@@ -412,21 +411,33 @@ static bool gemm_f32_mfma_fits(const void* x, const void* w, int M, int K, int l
     return M > 16 && K >= 4 && K % 4 == 0 && ldx % 4 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0;
 }
 
+// `tile`: 0 by the rule, 1 64 x 64, 2 64 x 128, 3 128 x 128 (tests cover each; tuning times them).
 static void launch_gemm_f32_mfma(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int N, int K,
-                                 int ldx, int ldo, hipStream_t stream) {
-    // tiles of 64 rows where those of 128 would leave most compute units without one
-    const long tiles128 = (long)((M + 127) / 128) * ((N + GF_BN - 1) / GF_BN);
-    if (M <= 64 || tiles128 < 256) {
-        dim3 grid((N + GF_BN - 1) / GF_BN, (M + 63) / 64);
-        gemm_f32_mfma_kernel<1><<<grid, dim3(256), 0, stream>>>((const float*)x, (const float*)w, bias, bias_f32, (float*)out, M, N, K, ldx, ldo);
-    } else {
-        dim3 grid((N + GF_BN - 1) / GF_BN, (M + 127) / 128);
-        gemm_f32_mfma_kernel<2><<<grid, dim3(256), 0, stream>>>((const float*)x, (const float*)w, bias, bias_f32, (float*)out, M, N, K, ldx, ldo);
+                                 int ldx, int ldo, hipStream_t stream, int tile = 0) {
+    auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    if (tile == 0) {
+        // Seconds per column of K: a start and a round of work-groups, up to TL_COMPUTE_UNITS of them at once (the smaller tiles' rounds overlap on a unit).  Fitted to 17 to 2048
+        // rows against nine matrices 2048 to 152064 wide; the sums are the same whichever is taken.  Measured (us; 64 x 64 / 64 x 128 / 128 x 128): 100 x 3584 x 3584 104 / 166 / 275,
+        // 753 x 3584 x 18944 1160 / 1373 / 1440, 1200 x 3584 x 3584 358 / 393 / 474, 301 x 37888 x 3584 930 / 863 / 1011, 753 x 37888 x 3584 2248 / 1977 / 1803.
+        // (Two sizes alone, 64 x 128 up to one round of 128 x 128 tiles, took 1.6 times as long up to 256 rows.)
+        static const struct { int bm, bn; double start, round; } sizes[] = {{64, 64, 0.0065, 0.0207}, {64, 128, 0.0085, 0.0365}, {128, 128, 0.0055, 0.0705}};
+        double best = 1e30;
+        for (int t = 0; t < 3; ++t) {
+            const double est = sizes[t].start + sizes[t].round * ((tiles(sizes[t].bm, sizes[t].bn) + TL_COMPUTE_UNITS - 1) / TL_COMPUTE_UNITS);
+            if (est < best) { best = est; tile = t + 1; }
+        }
     }
+#define GF_LAUNCH(FMB, FNB)                                                                                                                        \
+    gemm_f32_mfma_kernel<FMB, FNB><<<dim3((N + 64 * FNB - 1) / (64 * FNB), (M + 64 * FMB - 1) / (64 * FMB)), dim3(256), 0, stream>>>(                \
+        (const float*)x, (const float*)w, bias, bias_f32, (float*)out, M, N, K, ldx, ldo)
+    if (tile == 1) GF_LAUNCH(1, 1);
+    else if (tile == 2) GF_LAUNCH(1, 2);
+    else GF_LAUNCH(2, 2);
+#undef GF_LAUNCH
 }
 
 // One named kernel of the 32-bit products (for tests and tuning): 0 the general tile kernel (v_fma_f32), 1 the matrix-core
-// tile kernel, 2 and 3 the kernels for up to 16 rows on multiply-adds and on the matrix cores.
+// tile kernel, 2 and 3 the kernels for up to 16 rows on multiply-adds and on the matrix cores, 4 to 6 the matrix-core tile kernel with tiles of 64 x 64, 64 x 128, 128 x 128.
 extern "C" int tl_gemm_f32_variant(const void* x, const void* w, const void* bias, int bias_f32, void* out,
                                    int M, int N, int K, int ldx, int ldo, int matrix_cores, hipStream_t stream) {
     TL_REQUIRE(M > 0 && N > 0 && K > 0 && ldx >= K && ldo >= N, "gemm_f32: bad sizes M=%d N=%d K=%d ldx=%d ldo=%d", M, N, K, ldx, ldo);
@@ -435,7 +446,7 @@ extern "C" int tl_gemm_f32_variant(const void* x, const void* w, const void* bia
         launch_gemv_f32(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, stream, matrix_cores - 2);
     } else if (matrix_cores) {
         TL_REQUIRE(gemm_f32_mfma_fits(x, w, 17, K, ldx), "gemm_f32: the matrix-core kernel needs K %% 4 == 0 and 16-byte aligned rows");
-        launch_gemm_f32_mfma(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, stream);
+        launch_gemm_f32_mfma(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, stream, matrix_cores > 3 ? matrix_cores - 3 : 0);
     } else {
         launch_gemm_tile<float, float>(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, stream);
     }
