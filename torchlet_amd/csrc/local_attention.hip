@@ -1159,13 +1159,27 @@ pool_blocks_kernel(const T* __restrict__ k_plane, const T* __restrict__ v_plane,
     if (e >= dim + vdim) return;
     const bool is_key = e < dim;
     const int d = is_key ? e : e - dim;
+    // (sixteen positions' pages, then their numbers, are requested together: one after the other a block's 64 positions were a chain of 64 trips to memory: 2048 tokens, 4 heads 30.7 -> 13.3 us.  A
+    // position without a page reads the sentinel's and is left out)
+    constexpr int AHEAD = 16;
     float sum = 0.f;
-    for (int j = 0; j < pool; ++j) {
-        const int key = b * pool + j, blk = key / page_size, slot = key % page_size;
-        const int page = blk < table_width ? table[blk] : 0;
-        if (page <= 0 || page >= pages) continue;          // (a block's tokens are all held when its last one arrives)
-        sum += is_key ? to_float(k_plane[(((size_t)page * kv_heads + g) * page_size + slot) * dim + d])
-                      : to_float(v_plane[(((size_t)page * kv_heads + g) * vdim + d) * page_size + slot]);
+    for (int j0 = 0; j0 < pool; j0 += AHEAD) {
+        int at[AHEAD];
+        T x[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            const int blk = (b * pool + j0 + u) / page_size;
+            at[u] = j0 + u < pool && blk < table_width ? table[blk] : 0;
+            if (at[u] < 0 || at[u] >= pages) at[u] = 0;
+        }
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            const int slot = (b * pool + j0 + u) % page_size;
+            x[u] = is_key ? k_plane[(((size_t)at[u] * kv_heads + g) * page_size + slot) * dim + d] : v_plane[(((size_t)at[u] * kv_heads + g) * vdim + d) * page_size + slot];
+        }
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u)
+            if (at[u] > 0) sum += to_float(x[u]);          // (a block's tokens are all held when its last one arrives)
     }
     const float mean = sum / (float)pool;
     if (is_key) pk_plane[(((size_t)ppage * kv_heads + g) * page_size + pslot) * dim + d] = from_float<T>(mean);
