@@ -37,3 +37,13 @@ def test_activation_in_pieces(n, kind, dtype):
     ops.activation(pieces, kind)
     ops.activation(single, kind)
     assert torch.equal(pieces, single)
+
+
+def test_more_rows_than_a_launch_has_of_the_smallest_tiles():
+    M, N, K = 65535 * 64 + 3, 64, 4
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x, w = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda")
+    out = torch.empty(M, N, device="cuda")
+    ops.linear(x, w, None, out)
+    for part in (slice(0, 130), slice(M - 130, M)):
+        torch.testing.assert_close(out[part].double(), x[part].double() @ w.double().T, rtol=2e-5, atol=8 * 2 ** -24 * math.sqrt(K))

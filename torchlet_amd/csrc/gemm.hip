@@ -411,22 +411,30 @@ static bool gemm_f32_mfma_fits(const void* x, const void* w, int M, int K, int l
     return M > 16 && K >= 4 && K % 4 == 0 && ldx % 4 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0;
 }
 
-// `tile`: 0 by the rule, 1 64 x 64, 2 64 x 128, 3 128 x 128 (tests cover each; tuning times them).
+// The size of tiles of a 32-bit product: 1 64 x 64, 2 64 x 128, 3 128 x 128.
+//
+// Microseconds per column of K: a start and a round of work-groups, up to TL_COMPUTE_UNITS of them at once (the smaller tiles' rounds overlap on a unit).  Fitted to 17 to 2048
+// rows against nine matrices 2048 to 152064 wide; the sums are the same whichever is taken.  Measured (us; 64 x 64 / 64 x 128 / 128 x 128): 100 x 3584 x 3584 104 / 166 / 275,
+// 753 x 3584 x 18944 1160 / 1373 / 1440, 1200 x 3584 x 3584 358 / 393 / 474, 301 x 37888 x 3584 930 / 863 / 1011, 753 x 37888 x 3584 2248 / 1977 / 1803.
+// (Two sizes alone, 64 x 128 up to one round of 128 x 128 tiles, took 1.6 times as long up to 256 rows.)
+// A size whose rows of tiles are more than a launch has in y is not considered: beyond 4.19 million rows the tiles are 128 high.
+extern "C" int tl_gemm_f32_tile(int M, int N) {
+    static const struct { int bm, bn; double start, round; } sizes[] = {{64, 64, 0.0065, 0.0207}, {64, 128, 0.0085, 0.0365}, {128, 128, 0.0055, 0.0705}};
+    double best = 1e30;
+    int tile = 3;
+    for (int t = 0; t < 3; ++t) {
+        const long rows = ((long)M + sizes[t].bm - 1) / sizes[t].bm, tiles = rows * (((long)N + sizes[t].bn - 1) / sizes[t].bn);
+        if (rows > 65535) continue;
+        const double est = sizes[t].start + sizes[t].round * ((tiles + TL_COMPUTE_UNITS - 1) / TL_COMPUTE_UNITS);
+        if (est < best) { best = est; tile = t + 1; }
+    }
+    return tile;
+}
+
+// `tile`: 0 by the rule above, else one of its sizes (tests cover each; tuning times them).
 static void launch_gemm_f32_mfma(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int N, int K,
                                  int ldx, int ldo, hipStream_t stream, int tile = 0) {
-    auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-    if (tile == 0) {
-        // Seconds per column of K: a start and a round of work-groups, up to TL_COMPUTE_UNITS of them at once (the smaller tiles' rounds overlap on a unit).  Fitted to 17 to 2048
-        // rows against nine matrices 2048 to 152064 wide; the sums are the same whichever is taken.  Measured (us; 64 x 64 / 64 x 128 / 128 x 128): 100 x 3584 x 3584 104 / 166 / 275,
-        // 753 x 3584 x 18944 1160 / 1373 / 1440, 1200 x 3584 x 3584 358 / 393 / 474, 301 x 37888 x 3584 930 / 863 / 1011, 753 x 37888 x 3584 2248 / 1977 / 1803.
-        // (Two sizes alone, 64 x 128 up to one round of 128 x 128 tiles, took 1.6 times as long up to 256 rows.)
-        static const struct { int bm, bn; double start, round; } sizes[] = {{64, 64, 0.0065, 0.0207}, {64, 128, 0.0085, 0.0365}, {128, 128, 0.0055, 0.0705}};
-        double best = 1e30;
-        for (int t = 0; t < 3; ++t) {
-            const double est = sizes[t].start + sizes[t].round * ((tiles(sizes[t].bm, sizes[t].bn) + TL_COMPUTE_UNITS - 1) / TL_COMPUTE_UNITS);
-            if (est < best) { best = est; tile = t + 1; }
-        }
-    }
+    if (tile == 0) tile = tl_gemm_f32_tile(M, N);
 #define GF_LAUNCH(FMB, FNB)                                                                                                                        \
     gemm_f32_mfma_kernel<FMB, FNB><<<dim3((N + 64 * FNB - 1) / (64 * FNB), (M + 64 * FMB - 1) / (64 * FMB)), dim3(256), 0, stream>>>(                \
         (const float*)x, (const float*)w, bias, bias_f32, (float*)out, M, N, K, ldx, ldo)
