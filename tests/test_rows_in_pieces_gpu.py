@@ -76,3 +76,46 @@ def test_embedding_and_branches(hidden, dtype):
         ops.normed_sum(x.cuda(), w.cuda(), 1e-5, out)
         want = (x.double() / torch.sqrt(x.double().pow(2).mean(-1, keepdim=True) + 1e-5) * w.double()[:, None]).sum(0)
         torch.testing.assert_close(out.cpu().double(), want, rtol=2 ** -8 if dtype == torch.bfloat16 else 2e-5, atol=1e-5)
+
+
+def _graph_us(fn):
+    fn()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        fn()
+    times = []
+    for _ in range(5):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        graph.replay()
+        b.record()
+        torch.cuda.synchronize()
+        times.append(a.elapsed_time(b) * 1e3)
+    return min(times)
+
+
+def test_bigram_rows_of_one_request_beside_empty_ones():
+    """As many tokens as requests, all of them one request's: the rows, the token that is kept, and a time that no walk from token to token fits in."""
+    T, hidden, V, ids = 2048, 256, 50, torch.randint(0, 50, (2048,), generator=torch.Generator().manual_seed(1), dtype=torch.int32)
+    g = torch.Generator().manual_seed(2)
+    table, big = torch.randn(V, hidden, generator=g), torch.randn(8, hidden, generator=g)
+    at = 1000                                                # the request's number; those before it end at token 0, those behind it at T
+    indptr = torch.tensor([0] * (at + 1) + [T] * (T - at), dtype=torch.int32)
+    req = torch.full((T,), at, dtype=torch.int32)
+    positions, slots = torch.arange(3, 3 + T, dtype=torch.int32), torch.arange(T, dtype=torch.int32)
+    last = torch.full((T, 1), 9, dtype=torch.int32).cuda()
+    out = torch.empty(T, hidden).cuda()
+    args = [t.cuda() for t in (big, req, indptr, positions, slots, ids, table)]
+    big_d, req_d, indptr_d, positions_d, slots_d, ids_d, table_d = args
+
+    def run():
+        ops.bigram_embedding(ids_d, table_d, out, 0.5, big_d, 7, 5, 3, req_d, indptr_d, positions_d, slots_d, last)
+    run()
+    before = torch.cat((torch.tensor([9]), ids[:-1].long()))
+    want = table.double()[ids.long()] * 0.5 + big.double()[(before * 5 + ids.long() * 3) % 7]
+    torch.testing.assert_close(out.cpu().double(), want, rtol=1e-6, atol=1e-6)
+    kept = torch.full((T,), 9, dtype=torch.int32)
+    kept[at] = ids[-1]
+    assert torch.equal(last.cpu()[:, 0], kept)
+    assert _graph_us(run) < 300                              # (tens of us; 2048 rows one after the other are a millisecond)
