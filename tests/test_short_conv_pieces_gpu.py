@@ -18,8 +18,8 @@ def _shift(t, by):
     return wide.cuda()[:, by: by + t.shape[1]]
 
 
-# one token each; as many tokens as requests, but two and none; portions in runs of two; portions in runs of eight that cross requests' ends
-PLANS = [[1, 1, 1], [2, 0, 1, 1], [5, 1, 3, 2], [700, 3, 1, 2, 1001, 8]]
+# one token each; as many tokens as requests, but two and none, or none to seven; portions in runs of two; portions in runs of eight that cross requests' ends
+PLANS = [[1, 1, 1], [2, 0, 1, 1], [0, 0, 7, 0, 1, 3, 0, 0, 4, 0, 1, 2, 1, 1, 0, 2, 4, 0, 0, 0, 0, 4, 0, 0, 0, 0, 1, 0, 0, 0, 0], [5, 1, 3, 2], [700, 3, 1, 2, 1001, 8]]
 
 
 @pytest.mark.parametrize("lens", PLANS)
@@ -64,3 +64,30 @@ def test_selective(lens, dtype, heads, inner, gn):
         ops.selective_prepare(wide, 4 + by, conv.cuda(), conv_b.cuda(), gd, a_log.cuda(), bias.cuda(), state, 8, slots, _i32(indptr), req, out, heads, inner, gn, 4)
         got.append((out.cpu(), gd.cpu(), state.cpu()))
     assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+def test_one_request_beside_empty_ones_is_not_walked_token_by_token():
+    heads, kv, dim, vdim, T = 16, 8, 128, 128, 2048
+    C = 2 * kv * dim + heads * vdim
+    g = torch.Generator().manual_seed(5)
+    proj, conv, gates, a_log = (torch.randn(T, C, generator=g).bfloat16().cuda(), torch.randn(C, 4, generator=g).cuda(), torch.randn(T, 2 * heads, generator=g).cuda(),
+                                torch.zeros(heads).cuda())
+    indptr, req, slots = _i32([0] * 6 + [T] * (T - 5)), _i32([5] * T), _i32(list(range(T)))
+    state, qkv = torch.zeros(T, 3 * C + 8).cuda(), torch.empty(T, C).cuda()
+
+    def run():
+        ops.delta_prepare(proj, conv, gates, a_log, a_log, state, 8, slots, indptr, req, qkv, heads, kv, dim, vdim, 4, 0.3, 1e-6)
+    run()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run()
+    times = []
+    for _ in range(5):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        graph.replay()
+        b.record()
+        torch.cuda.synchronize()
+        times.append(a.elapsed_time(b) * 1e3)
+    assert min(times) < 400                                  # (tens of us; 2048 tokens one after the other are more than a millisecond)

@@ -586,8 +586,10 @@ __global__ void delta_tail_kernel(const T* __restrict__ proj, int ld, float* __r
 // What delta_prepare_kernel and selective_prepare_kernel (MODE 1) make, for four taps and channels that come in whole pieces of four: a thread owns four
 // neighbouring channels of a run of RUN tokens (their taps, and the window of the three inputs before the current token, stay in registers), so an input is
 // fetched once instead of once per tap, 8 or 16 bytes at a time, and the run's inputs are requested together.  A head's unit norm is shared by the dim / 4
-// neighbouring lanes that hold it.  OWN: a work-group takes all tokens of one request and moves its tail on itself (its threads own the channels they read),
-// which saves the tail's launch; for steps with as many tokens as requests, whatever tokens each of them brings.
+// neighbouring lanes that hold it.  OWN: for steps with as many tokens as requests (decode steps), without the tail's launch: a work-group takes the first three tokens of the
+// request of its own number, the only ones that read its tail, moves the tail on (its threads own the channels they read), and takes the token of its own number if that
+// is a later one of its request: whatever a request brings, nobody walks its tokens one after the other (one request of 2048 tokens of 4096 channels beside 2047 empty ones
+// 1830 us when the request's work-group did, 18.7 now; 16 requests of one token 3.4 both ways).
 // Bound by its bytes on prompts (2048 tokens of 4096 channels 53 -> 20 us, 3000 of 8448 163 -> 43 us), by launch and one trip to memory in decode steps (with the tail's kernel
 // 11.3 -> 4.5 us).
 struct ConvArgs {
@@ -609,11 +611,12 @@ __global__ void __launch_bounds__(256)
 short_conv_kernel(const T* __restrict__ proj, ConvArgs a) {
     const int p = blockIdx.y * 256 + threadIdx.x, pieces = a.C / 4, gate0 = (pieces + TL_WAVE - 1) / TL_WAVE * TL_WAVE;
     const int first = OWN ? a.req_indptr[blockIdx.x] : (int)blockIdx.x * RUN;
-    const int last = OWN ? a.req_indptr[blockIdx.x + 1] : min(first + RUN, a.tokens);
+    const int end = OWN ? a.req_indptr[blockIdx.x + 1] : min(first + RUN, a.tokens), last = OWN ? min(first + 3, end) : end;
+    const bool more = OWN && (int)blockIdx.x - a.req_indptr[a.token_req[blockIdx.x]] >= 3;
     if (p >= gate0) {                                  // (whole waves) the gates of the tokens' heads
         const int h = p - gate0;
         if (h >= a.heads) return;
-        for (int t = first; t < last; ++t) {
+        for (int t = OWN ? (int)blockIdx.x : first; t < (OWN ? (int)blockIdx.x + 1 : last); ++t) {
             float* g = a.gates + (size_t)t * 2 * a.heads;
             if (MODE == 0) {
                 const float b = g[h], v = g[a.heads + h];
@@ -638,6 +641,26 @@ short_conv_kernel(const T* __restrict__ proj, ConvArgs a) {
     float4 win[3];
     int req = -1;
     float* tail = nullptr;
+    auto convolve = [&](int t, const float4& now) {
+        float4 y = bias;
+#define TL_TAP(f, e) y.f = fmaf(tap[e].w, now.f, fmaf(tap[e].z, win[2].f, fmaf(tap[e].y, win[1].f, fmaf(tap[e].x, win[0].f, y.f))))
+        TL_TAP(x, 0); TL_TAP(y, 1); TL_TAP(z, 2); TL_TAP(w, 3);
+#undef TL_TAP
+        y = make_float4(silu_f(y.x), silu_f(y.y), silu_f(y.z), silu_f(y.w));
+        int to = c;
+        if (MODE == 0) {
+            float ss = fmaf(y.w, y.w, fmaf(y.z, y.z, fmaf(y.y, y.y, y.x * y.x)));
+            for (int k = a.unit_lanes / 2; k > 0; k >>= 1) ss += __shfl_xor(ss, k, TL_WAVE);
+            if (c < a.unit_end) {
+                float factor = 1.f / sqrtf(ss + a.unit_eps);
+                if (c < a.q_end) factor *= a.qscale;
+                y = make_float4(y.x * factor, y.y * factor, y.z * factor, y.w * factor);
+            }
+        } else {
+            to = c < a.inner ? 2 * a.gn + c : (c < a.inner + a.gn ? a.gn + (c - a.inner) : c - a.inner - a.gn);
+        }
+        if (live) store4(a.out + (size_t)t * a.C + to, y);
+    };
     for (int base = first; base < last; base += RUN) {
         Piece x[RUN];
 #pragma unroll
@@ -659,30 +682,19 @@ short_conv_kernel(const T* __restrict__ proj, ConvArgs a) {
                 }
             }
             const float4 now = widen4(x[u]);
-            float4 y = bias;
-#define TL_TAP(f, e) y.f = fmaf(tap[e].w, now.f, fmaf(tap[e].z, win[2].f, fmaf(tap[e].y, win[1].f, fmaf(tap[e].x, win[0].f, y.f))))
-            TL_TAP(x, 0); TL_TAP(y, 1); TL_TAP(z, 2); TL_TAP(w, 3);
-#undef TL_TAP
-            y = make_float4(silu_f(y.x), silu_f(y.y), silu_f(y.z), silu_f(y.w));
-            int to = c;
-            if (MODE == 0) {
-                float ss = fmaf(y.w, y.w, fmaf(y.z, y.z, fmaf(y.y, y.y, y.x * y.x)));
-                for (int k = a.unit_lanes / 2; k > 0; k >>= 1) ss += __shfl_xor(ss, k, TL_WAVE);
-                if (c < a.unit_end) {
-                    float factor = 1.f / sqrtf(ss + a.unit_eps);
-                    if (c < a.q_end) factor *= a.qscale;
-                    y = make_float4(y.x * factor, y.y * factor, y.z * factor, y.w * factor);
-                }
-            } else {
-                to = c < a.inner ? 2 * a.gn + c : (c < a.inner + a.gn ? a.gn + (c - a.inner) : c - a.inner - a.gn);
-            }
-            if (live) store4(a.out + (size_t)t * a.C + to, y);
+            convolve(t, now);
             win[0] = win[1]; win[1] = win[2]; win[2] = now;
         }
     }
-    if (OWN && live && last > first) {
+    if (OWN && live && end > first) {
 #pragma unroll
-        for (int j = 0; j < 3; ++j) store4(tail + (size_t)j * a.C, win[j]);
+        for (int j = 0; j < 3; ++j) store4(tail + (size_t)j * a.C, end - first > 3 ? widen4(*(const Piece*)(col + (size_t)(end - 3 + j) * a.ld)) : win[j]);
+    }
+    if (more) {                                        // (a wave together)
+        const int t = blockIdx.x;
+#pragma unroll
+        for (int j = 0; j < 3; ++j) win[j] = widen4(*(const Piece*)(col + (size_t)(t - 3 + j) * a.ld));
+        convolve(t, widen4(*(const Piece*)(col + (size_t)t * a.ld)));
     }
 }
 
