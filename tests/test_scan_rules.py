@@ -57,3 +57,13 @@ def test_blocks_where_they_are_the_faster_way(lib, mode, lens, heads, dim, vdim,
     from torchlet_amd.kernels import ops
     p = ops.Portions.of(lens, ops.BLOCKS_FROM)
     assert bool(lib.tl_blocks_pay(*(c_int(x) for x in (mode, p.tokens, p.longest, p.rest, heads, dim, vdim)))) == want
+
+
+# many portions whose work-groups outnumber the chip: the delta rule's loop is ahead, the selective recurrence's is not
+@pytest.mark.parametrize("mode, lens, heads, dim, vdim, want", [
+    (1, [128] * 64, 32, 128, 128, False), (1, [256] * 32, 32, 128, 128, False), (1, [128] * 64, 16, 128, 128, False), (1, [512] * 4, 32, 128, 128, True),
+    (1, [128, 300, 500, 900], 32, 128, 128, True), (1, [512] * 4, 16, 128, 128, True), (2, [128] * 16, 128, 128, 64, True), (2, [256] * 32, 128, 128, 64, True)])
+def test_blocks_of_crowded_steps(lib, mode, lens, heads, dim, vdim, want):
+    from torchlet_amd.kernels import ops
+    p = ops.Portions.of(lens, ops.BLOCKS_FROM)
+    assert bool(lib.tl_blocks_pay(*(c_int(x) for x in (mode, p.tokens, p.longest, p.rest, heads, dim, vdim)))) == want

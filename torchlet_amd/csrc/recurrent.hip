@@ -1447,16 +1447,20 @@ block_scan_kernel(const float* __restrict__ qkv, const float* __restrict__ scrat
 // Numbers of scratch for so many blocks.
 extern "C" long tl_blocks_floats(int mode, int blocks, int heads) { return (long)blocks * heads * (mode == 1 ? BlockPlaces<1>::FLOATS : BlockPlaces<2>::FLOATS); }
 
-// Whether a step's long portions (`tokens` in all, the longest of so many) go through the blocks, beside `rest` requests of a few tokens: two estimates in us, fitted to the device's times
-// below.  The loop's and the blocks' time is a chain along the longest portion and, where the work-groups outnumber the chip, about the same work on both ways; the
-// matrices are what the blocks cost more.
-// Measured (us, loop / blocks): the delta rule, 16 heads of 128 x 128: 128 tokens 28 / 27, 256 51 / 32, 512 107 / 49, 2048 413 / 162; 175 to 400 tokens 97 / 66, 275 to 1100 247 / 139, 16 x 128 107 / 114;
-// 32 heads: 2048 423 / 169, 16 x 128 183 / 208; 4 heads of 64 x 64: 512 73 / 36, 2048 283 / 116; 8 heads of 256 x 256: 128 68 / 32, 2048 1103 / 251; the selective recurrence, 128 heads of 128 x 64: 512 101 / 50, 2048 395 / 160, 275 to 1100 405 / 263, 16 x 128 243 / 220.
+// Whether a step's long portions (`tokens` in all, the longest of so many) go through the blocks, beside `rest` requests of a few tokens: two estimates in us, fitted to both ways'
+// times over 1600 steps of 128 to 9000 tokens at 2 to 128 heads and held against 600 others: the way it takes is 1.010 times the faster one's time on average, 13 of the 600 go through
+// blocks that the loop would be more than 3 % ahead of, 26 stay with a loop more than 8 % behind.  The loop's and the blocks' time is a chain along the longest portion and, where the
+// work-groups outnumber the chip, the work: about the same on both ways, but for the matrices, which the blocks cost more, so that the delta rule's steps of many thousand tokens in many
+// portions stay with the loop.
+// Measured (us, loop / blocks): the delta rule, 16 heads of 128 x 128: 128 tokens 27 / 22, 256 50 / 30, 512 106 / 48, 2048 413 / 162; 128 to 900 tokens of four requests 196 / 105,
+// 16 x 128 102 / 109, 4 x 512 127 / 91, 64 x 128 351 / 420; 32 heads: 512 109 / 52, 16 x 128 178 / 206, 64 x 128 676 / 872, 32 x 256 666 / 776, 16 x 512 673 / 724; 4 heads of
+// 64 x 64: 512 73 / 37; 8 heads of 256 x 256: 128 72 / 32, 512 291 / 76; the selective recurrence, 128 heads of 128 x 64: 128 28 / 21, 512 99 / 49, 16 x 128 241 / 213, 64 x 128 972 / 903.
 extern "C" int tl_blocks_pay(int mode, int tokens, int longest, int rest, int heads, int dim, int vdim) {
     const double groups = (double)heads * ((vdim + BL_T - 1) / BL_T), rows = (dim + 63) / 64;
     const double work = tokens * groups * 256.0 / tl_mlstm_units * fmax(1.0, rows / 2);
-    const double loop = 5 + hypot(longest * (rows > 3 ? 0.53 : 0.07 + 0.065 * rows), work * (mode == 1 ? 3.7e-4 : 2.3e-4));
-    const double blocks = 14 + tokens * (double)heads * (mode == 1 ? 1.2e-4 : 0.6e-4) + (rest > 0 ? 8 : 0) + hypot(longest * (0.03 + 0.024 * rows), work * (mode == 1 ? 3.5e-4 : 1.85e-4));
+    const double loop = 0.7 + hypot(longest * (rows > 3 ? 0.62 : 0.099 + 0.057 * rows), work * (mode == 1 ? 3.57e-4 : 2.55e-4));
+    const double blocks = 10.3 + tokens * (double)heads * rows * (mode == 1 ? 3.35e-4 : 0.16e-4) + (rest > 0 ? 12 : 0) +
+                          hypot(longest * (0.036 + 0.010 * rows), work * (rows > 1 ? 1.0 : 0.84) * (mode == 1 ? 2.73e-4 : 1.84e-4));
     return blocks < loop;
 }
 
