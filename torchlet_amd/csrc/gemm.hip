@@ -1299,10 +1299,25 @@ static DlTile pick_dl_tile(int M, int N, int K, bool sw, int products = 1) {
         if (t == DL_256x320) continue;      // float slabs of partial sums only: a bfloat16 result tile of 160 KB does not fit its slab buffers
         const long tiles = dl_tiles((DlTile)t, M, N) * products;
         if (t == DL_128x128_S4 && tiles > TL_COMPUTE_UNITS) continue;      // one round of work-groups
-        const double est = dl_estimate(DL_NOW, (DlTile)t, tiles, K);
+        double est = dl_estimate(DL_NOW, (DlTile)t, tiles, K);
+        // One row of tiles: no weight is drawn twice, all come from memory and none from the L2s, and there the small tile with two work-groups on some of the units, and the deep one with
+        // the fused gate, fall behind their estimates.  Measured (us; 64 x 64 / 64 x 128 / 128 x 128 with four slabs): 63 x 18944 x 5120 62.5 / 52.9 / 52.5, 63 x 18944 x 3584 40.7 / 37.1 /
+        // 36.3, 33 x 22528 x 5120 57.4 / 51.4 / 50.6; where rows of w lie multiples of 4 KB apart, or are short, the small tile stays ahead (33 x 27648 x 8192 91 / 105 / 102, x 768 12.4 / 13.0 / 13.0); the gate, 128 x
+        // 5632 x 13824 - / 113 / 137, 128 x 6912 x 5120 - / 48.7 / 58.0.  (Without these two lines 94 of 1134 sizes of 33 to 700 rows took more than 3 % longer, up to 19 %, than
+        // with the shapes that the rule before the figures above chose, with them 55, up to 14 %; of 427 with the gate 15, up to 21 %, and 6, up to 13 %.)
+        if (t == DL_64x64 && M <= 64 && tiles > TL_COMPUTE_UNITS && K > 2048 && K % 2048) est *= 1.4;
+        if (t == DL_128x128_S4 && sw && M > 64 && M <= 128) est *= 1.05;
         if (est < best_t) { best_t = est; best = (DlTile)t; }
     }
     return best;
+}
+
+// The tile of a whole product (gated: with the fused gate, N rows of its interleaved matrix), by its rows, columns and slabs in shared memory; tests ask for it.
+extern "C" void tl_gemm_direct_choice(int M, int N, int K, int gated, int* rows, int* columns, int* slabs4) {
+    const DlTile t = pick_dl_tile(M, N, K, gated != 0);
+    *rows = DL_BM[t];
+    *columns = DL_BN[t];
+    *slabs4 = t == DL_128x128_S4;
 }
 
 // K in `parts` ranges of k_per columns (a multiple of 64), none of them empty; 0 if there is no such split.
