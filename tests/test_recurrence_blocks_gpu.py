@@ -57,9 +57,10 @@ def _run(kind, x, gates, skip, state, lens, H, G, dim, vdim, **more):
 
 
 # lengths: the fewest that go through blocks, one short of them, whole and broken blocks, single tokens and an empty request beside them; sizes: whole tiles, broken
-# ones, every number of tiles a wave, rows that cannot be read in pieces (which stay with the token loop)
+# ones, every number of tiles a wave, rows that cannot be read in pieces (which stay with the token loop), and numbers of heads that are dealt out over the XCDs
 @pytest.mark.parametrize("kind", ["delta", "selective"])
-@pytest.mark.parametrize("H, G, dim, vdim", [(4, 2, 128, 128), (5, 1, 64, 40), (2, 2, 100, 36), (6, 1, 36, 20), (1, 1, 256, 24), (2, 1, 132, 16), (2, 1, 30, 17)])
+@pytest.mark.parametrize("H, G, dim, vdim", [(4, 2, 128, 128), (5, 1, 64, 40), (2, 2, 100, 36), (6, 1, 36, 20), (1, 1, 256, 24), (2, 1, 132, 16), (2, 1, 30, 17),
+                                               (8, 4, 64, 40), (16, 8, 128, 36)])
 @pytest.mark.parametrize("lens", [[128], [127], [1, 128, 0, 161, 15, 144], [259, 129]])
 @pytest.mark.parametrize("exact", [True, False])
 def test_blocks_against_the_recurrence(kind, H, G, dim, vdim, lens, exact):

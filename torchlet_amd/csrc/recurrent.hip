@@ -774,8 +774,9 @@ extern "C" int tl_delta_prepare(const void* proj, int ld, const void* conv_w, vo
 // by dim alone) of it in registers for all tokens of the step, so the lanes' pieces of q and k lie side by side in shared memory and those of
 // the state side by side in memory ([vdim][dim] per head), and they add their sums with four exchanges inside the row (pairs, quads, halves,
 // the row: every lane gets the same bits).  k . q, which all columns share, is made once a token.  The order of every sum is fixed by dim, so a
-// token's result in this loop depends neither on how its request was cut into steps nor on what else the step holds (fixed decays leave it for long portions: see the
-// chunks below).  A wave has 4 CPL columns, a work-group
+// token's result in this loop depends neither on how its request was cut into steps nor on what else the step holds.  (Long portions leave it, fixed decays for chunks of 64 tokens and the other
+// two for blocks of 16, see below, where a step's sizes make that the faster way: from CHUNKED_FROM or BLOCKS_FROM tokens on a portion's rounding depends on where it was cut and, through
+// that choice, on what else the step holds.)  A wave has 4 CPL columns, a work-group
 // of four waves 16 CPL.  Tokens are taken TB at a time (1, 4 or 16, by the longest portion of the step): their q, k, v, beta and g are fetched
 // into registers one batch ahead, as whole pieces of four where the rows allow it, and go to shared memory; a request's last batch is filled up
 // with tokens that change nothing (k = 0, beta = 0, decay 1), so the loop has no branch.
@@ -1053,13 +1054,14 @@ static int launch_delta_scan(const void* qkv, const void* gates, const void* hea
 
 // ------------------------------------------------------------------ long portions in blocks: the delta rule and the selective recurrence
 // The token loop above is a chain of some 500 cycles a token, whatever else the GPU does (one prompt of 2048 tokens, 16 heads: 412 us on 128 work-groups).  Over a block of
-// 16 tokens the recurrence is a few products of small matrices, with S the state before the block, g the decays, G_i = prod_{l <= i} g_l and D_ij = prod_{j < l <= i} g_l:
+// 16 tokens the recurrence is a few products of small matrices (the compact form of a product of Householder-like steps, Bischof and Van Loan's WY representation, as "Parallelizing Linear
+// Transformers with the Delta Rule over Sequence Length", Yang et al. 2024, use it), with S the state before the block, g the decays, G_i = prod_{l <= i} g_l and D_ij = prod_{j < l <= i} g_l:
 //   L_ij = beta_i (k_i . k_j) D_ij below the diagonal;   U = (1 + L)^-1 diag(beta) (V - diag(G) K S);   O = diag(G) Q S + (Q K^T o D) U;   S <- G_16 S + K^T diag(w) U,  w_j = D_16,j
 // (the selective recurrence: U = diag(beta) V).  What does not need the state, T = (1 + L)^-1 diag(beta), P = Q K^T o D, G and w, is made for all blocks at once by
 // block_matrices_kernel (the inverse by substitution, and the decays' products, in 64 bits; no quotients, so a decay of zero is one); block_scan_kernel then walks a request's
 // blocks with the state in registers: products in true 32-bit on v_mfma_f32_16x16x4_f32, whose result layout (lane l: rows 4 (l / 16) + v of column l % 16) is the
 // layout of its right operand, so state, U and V never change lanes.  A work-group owns 16 columns, each of four waves a quarter of their rows: one barrier a block, for the
-// quarters' shares of K S and Q S; a fifth wave makes the outputs, a block behind.  What bounds it: a block's chain of products (29 matrix instructions of 32 cycles a wave, four of them one after the other for U), the exchange and a wait for operands, some 2700 cycles for
+// quarters' shares of K S and Q S; a fifth wave makes the outputs, a block behind.  What bounds it: a block's chain of products (28 matrix instructions of 32 cycles a wave at 128 x 128, four of them one after the other for U), the exchange and a wait for operands, some 2700 cycles for
 // 16 tokens: 2048 tokens, 16 heads of 128 x 128 413 -> 162 us.  Errors against 64 bits (1500 tokens, whole outputs; loop / blocks): slow decays 1.5e-7 to 1.75e-7 / 1.0e-7, fast ones 7.0e-8 / 6.5e-8, selective 1.1e-7 / 0.8e-7.
 // Requests of few tokens in the step stay with the token loop, whose bits do not depend on how a request is cut into steps; blocks are counted from the step's first token of the request.
 #define BL_T 16                 // tokens of a block

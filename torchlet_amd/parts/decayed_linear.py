@@ -4,8 +4,10 @@ Per token ``q = silu(W_q h)`` and ``k = silu(W_k h)`` (``heads x dim``) and ``v 
 its state ``S [dim, vdim]`` by ``S <- decay_i S + k v^T`` and gives ``o = S^T q``.  The heads' outputs side by side are divided by their root
 mean square (all of them together), multiplied by a weight vector and by ``sigmoid(W_g h)``, and projected by ``W_o``.  A request's slot
 holds the states of all heads in 32-bit, zero when the slot is handed out; activations of the projections, state, outputs and norm are
-32-bit under every engine.  The recurrence runs in the delta rule's kernel without that rule's correction term, token by token from where
-the state stands, so a portion of n tokens is n single steps by construction.
+32-bit under every engine.  The recurrence runs in the delta rule's kernel without that rule's correction term from where the state stands:
+token by token, where a portion of n tokens is n single steps to the bit, or, for portions of ``ops.CHUNKED_FROM`` tokens and more where the step's
+sizes make it the faster way, in chunks of 64 tokens, which round in another order, so that such a portion's rounding depends on where its
+request was cut and on what else the step holds.
 """
 from __future__ import annotations
 

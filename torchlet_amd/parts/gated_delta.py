@@ -10,8 +10,10 @@ softplus(W_a h + dt_bias))`` per head.  Head ``i`` (reading q/k head ``i // (hea
 and the mixer's output is ``W_o (concat_heads(o / rms(o) * w_norm) * silu(W_g h))``.  A request's slot holds the states of all
 heads and the last ``conv - 1`` inputs of every convolved channel, in 32-bit, zero when the slot is handed out.  The unit norms, the
 gates, the decays, the state and the per-head norm are 32-bit under every engine; the projections run in the compute dtype (the two
-per-head gates leave their product in 32-bit).  One kernel runs the recurrence for every request of the step from where its state
-stands, token by token, so a portion of n tokens is n single steps by construction.
+per-head gates leave their product in 32-bit).  The recurrence runs for every request of the step from where its state stands: token by
+token, where a portion of n tokens is n single steps to the bit, or, for portions of ``ops.BLOCKS_FROM`` tokens and more where the step's sizes
+make it the faster way, in blocks of 16 tokens, which count from the portion's first and round in another order.  So the rounding of
+such a portion depends on where its request was cut and on what else the step holds.
 """
 from __future__ import annotations
 

@@ -9,8 +9,10 @@ running maximum ``m`` (all zero for a new request) move token by token::
 
 and the mixer's output is ``W_o (concat_heads(o / rms(o)) * w_norm * sigmoid(W_g h))``.  The state lives in 32-bit in the
 cache manager's slot of the request; gates, decays and the quotient are 32-bit under every engine, the projections run in
-the compute dtype.  One kernel runs the recurrence for every request of the step from where its state stands, so a
-portion of n tokens is n single steps by construction.
+the compute dtype.  The recurrence runs for every request of the step from where its state stands: token by token, where a
+portion of n tokens is n single steps to the bit, or, for portions of ``ops.CHUNKED_FROM`` tokens and more where the step's sizes
+make it the faster way, in chunks of 64 tokens, which round in another order, so that such a portion's rounding depends on
+where its request was cut and on what else the step holds.
 """
 from __future__ import annotations
 

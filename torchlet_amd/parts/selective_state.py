@@ -10,8 +10,10 @@ and the mixer's output is ``W_o (norm(y * silu(z)) * w_norm)``, the norm a root-
 ``inner`` numbers, the gate before it.  A request's slot holds the states of all heads and the last ``conv - 1`` inputs of every convolved
 channel, in 32-bit, zero when the slot is handed out.  The convolution's output, step sizes, decays, the state and the gated norm are
 32-bit under every engine; the projections run in the compute dtype.  The recurrence is the delta rule's kernel without that rule's
-correction term, with B as its keys, C as its queries, dt as its step size and x as its values, so it runs token by token from where the
-state stands and a portion of n tokens is n single steps by construction.
+correction term, with B as its keys, C as its queries, dt as its step size and x as its values: token by token from where the state
+stands, where a portion of n tokens is n single steps to the bit, or, for portions of ``ops.BLOCKS_FROM`` tokens and more where the step's sizes
+make it the faster way, in blocks of 16 tokens, which count from the portion's first and round in another order.  So the rounding of
+such a portion depends on where its request was cut and on what else the step holds.
 """
 from __future__ import annotations
 
