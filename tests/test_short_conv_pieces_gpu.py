@@ -1,4 +1,4 @@
-"""Short convolutions over whole pieces of four channels against the same numbers in rows that do not allow pieces (which the general kernels take)."""
+"""Short convolutions over whole pieces of four channels against the same numbers in rows that do not allow pieces (which the general kernels take), and against 64 bits."""
 import pytest
 import torch
 
@@ -9,6 +9,22 @@ pytestmark = pytest.mark.gpu
 
 def _i32(x):
     return torch.tensor(x, dtype=torch.int32).cuda()
+
+
+def _convolved(proj, conv, bias, tails, lens):
+    """In 64 bits: silu of the convolution over each request's inputs behind its tail (``tails [requests, 3, C]``), and the tails behind them."""
+    out, after, at = [], [], 0
+    for r, n in enumerate(lens):
+        rows = torch.cat((tails[r].double(), proj[at: at + n].double()))
+        y = bias.double() + sum(rows[j: j + n] * conv.double()[:, j] for j in range(4))
+        out.append(y / (1 + torch.exp(-y)))
+        after.append(rows[n:])
+        at += n
+    return torch.cat(out), torch.stack(after)
+
+
+# what a 32-bit convolution, silu and norm of numbers of order one make of 64 bits: a few roundings
+CLOSE = dict(rtol=2e-6, atol=2e-6)
 
 
 def _shift(t, by):
@@ -43,6 +59,17 @@ def test_delta(lens, dtype, heads, kv, dim, vdim):
     torch.testing.assert_close(got[0][0], got[1][0], rtol=2e-6, atol=1e-7)
     assert torch.equal(got[0][0][:, 2 * kv * dim:], got[1][0][:, 2 * kv * dim:])
     assert torch.equal(got[0][1], got[1][1]) and torch.equal(got[0][2], got[1][2])
+    y, tails = _convolved(proj, conv, torch.zeros(C), start[slots.cpu().long(), 8:].view(R, 3, C), lens)
+    unit = y[:, : 2 * kv * dim].view(T, 2 * kv, dim)
+    unit = unit / torch.sqrt((unit * unit).sum(-1, keepdim=True) + 1e-6)
+    unit[:, :kv] *= 0.3
+    torch.testing.assert_close(got[0][0].double(), torch.cat((unit.flatten(1), y[:, 2 * kv * dim:]), 1), **CLOSE)
+    z = gates.double()
+    decay = torch.exp(-torch.exp(a_log.double()) * torch.nn.functional.softplus(z[:, heads:] + bias.double()))
+    torch.testing.assert_close(got[0][1].double(), torch.cat((torch.sigmoid(z[:, :heads]), decay), 1), **CLOSE)
+    want = start.clone()
+    want[slots.cpu().long(), 8:] = tails.float().reshape(R, -1)      # (inputs as they are: no rounding)
+    assert torch.equal(got[0][2], want)
 
 
 @pytest.mark.parametrize("lens", PLANS)
@@ -64,6 +91,13 @@ def test_selective(lens, dtype, heads, inner, gn):
         ops.selective_prepare(wide, 4 + by, conv.cuda(), conv_b.cuda(), gd, a_log.cuda(), bias.cuda(), state, 8, slots, _i32(indptr), req, out, heads, inner, gn, 4)
         got.append((out.cpu(), gd.cpu(), state.cpu()))
     assert all(torch.equal(a, b) for a, b in zip(*got))
+    y, tails = _convolved(proj[:, :C], conv, conv_b, start[slots.cpu().long(), 8:].view(R, 3, C), lens)
+    torch.testing.assert_close(got[0][0].double(), torch.cat((y[:, inner + gn:], y[:, inner: inner + gn], y[:, :inner]), 1), **CLOSE)
+    dt = torch.nn.functional.softplus(proj[:, C: C + heads].double() + bias.double())
+    torch.testing.assert_close(got[0][1].double(), torch.cat((dt, torch.exp(-torch.exp(a_log.double()) * dt)), 1), **CLOSE)
+    want = start.clone()
+    want[slots.cpu().long(), 8:] = tails.float().reshape(R, -1)
+    assert torch.equal(got[0][2], want)
 
 
 def test_one_request_beside_empty_ones_is_not_walked_token_by_token():

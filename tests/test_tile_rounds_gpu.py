@@ -30,11 +30,12 @@ def test_one_round_of_tiles(M, N, K, result):
     assert (out[:, N:] == 7.0).all()
 
 
-# one slab and several, by whichever the plan takes: the slabs' sum is the product, and 32 bits are kept
-@pytest.mark.parametrize("M,N,K", [(1457, 2048, 5632), (400, 7168, 5120), (1457, 2048, 4096), (200, 3584, 3584), (513, 5120, 5120), (100, 4608, 3584)])
-def test_float_slabs(M, N, K):
+# one slab (of 64 x 64 and of 128 x 128 tiles) and several: the slabs' sum is the product, and 32 bits are kept
+@pytest.mark.parametrize("M,N,K,slabs", [(200, 3584, 3584, 1), (400, 7168, 3584, 1), (1457, 2048, 5632, 2), (400, 7168, 5120, 2), (1457, 2048, 4096, 2), (513, 5120, 5120, 2), (512, 5120, 13824, 3),
+                                         (100, 4608, 3584, 7)])
+def test_float_slabs(M, N, K, slabs):
     assert ops.linear_partials_pay(M, N, K)
     x, w, ref = _operands(M, N, K)
-    slabs = ops.linear_partials(x, w)
-    assert slabs.dtype == torch.float32 and slabs.shape[1:] == (M, N)
-    torch.testing.assert_close(slabs.double().sum(0), ref, rtol=2e-5, atol=8 * 2 ** -24 * math.sqrt(K))
+    got = ops.linear_partials(x, w)
+    assert got.dtype == torch.float32 and got.shape == (slabs, M, N)
+    torch.testing.assert_close(got.double().sum(0), ref, rtol=2e-5, atol=8 * 2 ** -24 * math.sqrt(K))
