@@ -267,18 +267,18 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_dl_tile_kernel(const bf16
             for (int v = 0; v < 4; ++v) acc[i][j][v] = 0.f;
 
     // Products of 16 x 16 x 32: lane l holds eight columns of K, 8 (l / 16) .. + 7 of a phase's 32, of row l % 16 of a block.  They do the work of a 32 x 32 x
-    // 16 product in as many cycles and move half as much of the accumulators, and the power that this takes is what sets the clock of a large product (8192 x 8192 x 8192:
-    // 2650 cycles a slab at 1.67 GHz with the larger blocks, 2610 at 1.8 with these: 846 -> 778 us; 2048 x 37888 x 3584 468 -> 446, 2048 x 8192 x 2048 60 -> 56).
+    // 16 product in as many cycles and move half as much of the accumulators, and the power that this takes is what sets the clock of a large product (2650 cycles a slab at
+    // 1.67 GHz with the larger blocks, 2610 at 1.8 with these; with all that follows 8192 x 8192 x 8192 850 -> 766 us, 2048 x 37888 x 3584 475 -> 431, 2048 x 8192 x 2048 62 -> 54).
     //
     // The loop is a hand-laid pipeline; scheduling fences keep the compiler from undoing it.  A step of TK columns has two phases of FM * FN products.  A phase's
     // memory instructions go between its products, one product first: the operand reads of the next phase, so that a read has a whole phase to arrive.  (All
     // reads first and then all products, the wait at the loop's head came out as one for every read, the ones just issued too.)  Both operands
     // have two sets of registers; where these and the sums do not fit (the waves of 64 x 160), the operand with more blocks (`rolled`) has one set, each
-    // block read anew once the last product that needs it is under way (in a wave of 128 x 64, where both ways fit, it costs a fortieth: 778 against 796 us).
+    // block read anew once the last product that needs it is under way (in a wave of 128 x 64, where both ways fit, it costs a fortieth).
     //
     // The last phase of a step waits for the next slab and meets the other waves at the barrier (they have all read their last operands of this
-    // slab by then): at its start, or with many products halfway through it, which leaves the slab that much longer to arrive (8192 x 8192 x 8192: 863 us at the
-    // start, 778 halfway).  Behind the barrier go the first half of the requests for the slab STAGES - 1 ahead, into
+    // slab by then): at its start, or with many products three quarters through it, which leaves the slab that much longer to arrive (8192 x 8192 x 8192: 863 us at the
+    // start, 780 halfway, 775 at three quarters; 766 with two memory instructions behind a product).  Behind the barrier go the first half of the requests for the slab STAGES - 1 ahead, into
     // the buffer just given up, and the reads of the first operands of the next slab.  The other half of the requests goes into the first phase of the next
     // step: a compute unit's 64 requests in one phase hold its waves up, whatever they fetch (requests of 4 bytes a lane cost the same; without any the loop ran a
     // sixth faster), and in two phases less so (all of them behind the reads: 857 us).  Past the end the last slab is requested again (nobody reads it), so the count

@@ -358,16 +358,17 @@ static int launch_experts(int which, const ExpertsCall& c, hipStream_t stream) {
 // Up to 8 slots a group on average (4 where K is beyond 2048: a strip's rows of x, read once per strip, outgrow the caches) the weights' stream
 // sets the time: the few-rows kernel, with waves enough to leave each a few steps of K.  Measured (us; few rows with 8 waves / with 4 / the
 // tiles of 64 x 128; groups x N x K, every call on other weights):
-//   16 x 1024 x 2048, 16 slots 11.8 / 13.8 / 20.9, 128 slots 17.7 / 20.9 / 22.1, 256 slots 26.4 / 26.7 / 22.5
-//   16 x 2048 x 1024, 16 slots 15.7 / 9.8 / 13.6, 64 slots 25.2 / 15.0 / 16.0, 128 slots 28.2 / 17.0 / 16.1, 256 slots 43.9 / 26.3 / 16.0
-//   32 x 4096 x 4096, 16 slots 77 / 82 / 84, 128 slots 181 / 191 / 178, 256 slots 208 / 213 / 179 (229 us at the rate of a large copy)
+//   16 x 1024 x 2048, 16 slots 13.9 / 14.9 / 20.4, 128 slots 19.7 / 21.7 / 21.6, 256 slots 25.6 / 24.6 / 21.6
+//   16 x 2048 x 1024, 16 slots 16.9 / 11.8 / 14.6, 64 slots 25.3 / 15.2 / 15.9, 128 slots 30.0 / 17.9 / 15.9, 256 slots 42.6 / 25.0 / 16.1
+//   32 x 4096 x 4096, 16 slots 68 / 73 / 74, 128 slots 183 / 190 / 176, 256 slots 210 / 212 / 178 (229 us at the rate of a large copy)
 // (the kernel without shared memory, which had these calls, took 37 us for the first and 134 at 4096 slots, where the tiles take 37).
 //
 // Beyond that, tiles: rounds of work-groups (two of the two smaller tiles to a compute unit) times a tile's time, fitted to single rounds at K of
-// 1024 and 2048; every group ends in a tile that is half empty on average.  Measured (us; 64 x 128 / 128 x 128 / 128 x 256 / 256 x 256):
-//   16 x 1024 x 2048, 2048 slots 35 / 36 / 37 / 50, 4096 slots 49 / 42 / 37 / 53, 16384 slots 121 / 110 / 92 / 107
-//   16 x 2048 x 1024, 2048 slots 31 / 25 / 23 / 31, 4096 slots 45 / 47 / 43 / 34, 16384 slots 134 / 110 / 104 / 95
-//   32 x 4096 x 4096, 2048 slots 219 / 192 / 190 / 254, 16384 slots 873 / 693 / 630 / 654
+// 1024 and 2048; every group ends in a tile that is half empty on average.  The figures were fitted to tiles of 32 x 32 x 16 products and hold for today's: over 37 sizes of 16 to 16384
+// slots the kernel chosen takes 1.01 of the fastest one's time on average, 1.13 at most.  Measured (us; 64 x 128 / 128 x 128 / 128 x 256 / 256 x 256):
+//   16 x 1024 x 2048, 2048 slots 33 / 35 / 34 / 46, 4096 slots 47 / 38 / 34 / 49, 16384 slots 119 / 103 / 90 / 101
+//   16 x 2048 x 1024, 2048 slots 31 / 26 / 22 / 29, 4096 slots 45 / 44 / 39 / 32, 16384 slots 143 / 108 / 96 / 92
+//   32 x 4096 x 4096, 2048 slots 228 / 190 / 190 / 250, 16384 slots 830 / 680 / 587 / 613
 static int pick_experts(const ExpertsCall& c) {
     if ((long)c.rows <= (c.K > 2048 ? 4L : 8L) * c.groups) return c.K < 2048 ? EX_FEW_4 : EX_FEW_8;
     static const struct { int kernel, bm, bn, per_unit; double fixed, per_k; } tiles[] = {

@@ -1238,8 +1238,9 @@ static int launch_mfma_tile(const void* x, const void* w, const void* bias, int 
 // tiles are dealt to 256 compute units, each works through ceil(tiles / 256) of them one after
 // the other; a tile takes a fixed time (filling the pipeline, storing the result) plus its
 // products at the rate one compute unit reaches with that shape.  The figures are fitted to measurements of every shape at 16 to 8192 rows
-// against 27 matrices (the Qwen2.5 models' and those 2048 to 16384 wide of the other designs), whole and split: a product gets a shape whose time is 1.005 of the
-// fastest shape's on average over those 320 sizes, 1.14 at most (1.07 and 1.8 with the figures fitted to 2048 rows alone).
+// against 27 matrices (the Qwen2.5 models' and those 2048 to 16384 wide of the other designs; the rates of 64 x 192, 64 x 320 and 256 x 320 came out as they were): a whole
+// product gets a shape whose time is 1.005 of the fastest shape's on average over those 341 sizes, 1.13 at most, and 1.008 over 160 others, 1.14 at most
+// (1.07 and 1.8 with the figures fitted to 2048 rows alone).
 // (DL_128x128_S4: 128 x 128 with four slabs in shared memory, one work-group to a compute unit: where the tiles are one round of work-groups, what
 // counts is how many bytes a work-group has on their way: 2048 x 2048 x 8192 69.6 us against 102.7 with two slabs, 2048 x 2048 x 2048 21.1 against 25.9, 400 x 7168 x 5120
 // 1.8 times as fast; with more tiles than units two work-groups of two slabs each share a unit: 2048 x 8192 x 2048 65.5 us against 75.2)
@@ -1283,8 +1284,8 @@ static double dl_estimate(const DlFigures& f, DlTile t, long groups, int k) {
 static const DlFigures DL_NOW = {
     {2.52e12, 2.82e12, 3.71e12, 4.41e12, 5.38e12, 4.34e12, 5.27e12, 6.23e12, 1.89e12, 4.01e12, 3.0e12, 4.83e12, 3.5e12, 5.5e12, 4.48e12},
     {2.7e-6, 9.5e-6, 5.5e-6, 11e-6, 8.4e-6, 11e-6, 9.1e-6, 15.4e-6, 3.1e-6, 5.2e-6, 9.7e-6, 10.6e-6, 12e-6, 5.1e-6, 10.6e-6}, 68.8e9, 0.87, 1.0, true};
-// The figures of the rule by which a product's result stays in 32 bits (gives_slabs below): those of slower kernels, and kept as they are, since what a
-// consumer reads in 32 bits is not to depend on how fast a tile has become.
+// The numbers of the rule by which a product's result stays in 32 bits (gives_slabs below).  They are no kernel's: they were the estimates of slower kernels when the line was drawn, and stay, since
+// a result that a consumer has read in 32 bits is not to lose them because a tile has become faster.
 static const DlFigures DL_SLAB_RULE = {
     {2.45e12, 3.3e12, 4.2e12, 4.6e12, 4.8e12, 5.2e12, 5.2e12, 6.1e12, 2.1e12, 4.2e12, 3.0e12, 4.4e12, 3.5e12, 5.5e12, 4.3e12},
     {2.7e-6, 11.5e-6, 5.5e-6, 11e-6, 15e-6, 6e-6, 8e-6, 14e-6, 5e-6, 4.5e-6, 9e-6, 9e-6, 12e-6, 10e-6, 10e-6}, 32e9, 0.62, 1.1, false};
@@ -1333,8 +1334,10 @@ static bool dl_can_split(DlTile t, int M, int N, int parts, int small_rows) {
     return t == DL_128x128_S4 ? one_round : t == DL_64x64 ? one_round && M <= small_rows : true;
 }
 
-// Whether a product of more than 64 rows whose consumer can add slabs up gives it float slabs: where K split over work-groups pays against a bfloat16
-// result, the slabs counted at their bytes once written and once read.
+// Whether a product of more than 64 rows whose consumer can add slabs up gives it float slabs: a line between the sizes whose sums reach the consumer in 32 bits and those that are rounded
+// to bfloat16 first, drawn where K split over work-groups was ahead of a bfloat16 result.  What it costs by today's times, product and reading against the best whole product with a bfloat16 result:
+// 512 rows against 5120 x 13824 0.67, 5120 x 5120 0.84, 7168 x 5120 0.99; over 574 sizes on its yes side 0.84 on average; 75 of them are more than 5 % behind, up to 1.35 (1457 x 2048 x 4096),
+// mostly where the plan below splits what one slab would do faster.
 static bool gives_slabs(int M, int N, int K) {
     double whole = 1e30;
     for (int t = 0; t < DL_TILES; ++t) {
@@ -1355,10 +1358,11 @@ static bool gives_slabs(int M, int N, int K) {
 
 // More than 64 rows against a matrix whose output tiles leave compute units idle (a few hundred rows
 // of a prompt portion against the down projection, say): K split over `parts` work-groups per tile
-// into float slabs that the consumer adds up, or one float slab where a tile's own rounds fill the chip better (1457 x 2048 x 5632: 45.7 us in four parts of 192 x
-// 256, 37.2 in one of 128 x 128 with four slabs; 400 x 7168 x 5120 53 and 41).  Split, only the tiles that have a compute unit to themselves
+// into float slabs that the consumer adds up, or one float slab where a tile's own rounds fill the chip better (400 x 7168 x 3584: 34.2 us in two parts of 256 x 128, 29.7 in one of
+// 128 x 128 with four slabs in shared memory; 133 x 4608 x 3584 16.5 in three parts, 14.6 in one of 64 x 64).  Split, only the tiles that have a compute unit to themselves
 // are considered; the slabs cost their bytes once written and once read.  parts == 0: a bfloat16 result.
-// Fitted like the tiles' figures, with the slabs' reading counted at 4 TB/s: the choice takes 1.01 of the fastest's time on average.
+// With the slabs' reading counted at 4 TB/s the choice takes 1.026 of the fastest plan's time on average over 123 of the fitted sizes, 1.28 at most, and 1.078 over 51 others, 1.54 at most:
+// it undervalues one slab of 128 x 128 (1457 x 2048 x 4096 34.6 in two parts, 28.6 in one).
 struct DlSplit { DlTile tile; int parts; int k_per; };
 static DlSplit plan_dl_split(int M, int N, int K) {
     DlSplit best{DL_128x128, 0, 0};
