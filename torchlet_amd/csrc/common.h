@@ -26,6 +26,20 @@ __device__ __forceinline__ float load_vec(const void* p, int is_f32, size_t i) {
     return is_f32 ? ((const float*)p)[i] : to_float(((const bf16_t*)p)[i]);
 }
 
+// Four neighbouring numbers (16-byte aligned floats, 8-byte aligned bfloat16).
+__device__ __forceinline__ float4 load4(const float* p) { return *(const float4*)p; }
+__device__ __forceinline__ float4 load4(const bf16_t* p) {
+    const uint2 t = *(const uint2*)p;
+    return make_float4(__uint_as_float(t.x << 16), __uint_as_float(t.x & 0xffff0000u), __uint_as_float(t.y << 16), __uint_as_float(t.y & 0xffff0000u));
+}
+__device__ __forceinline__ void store4(float* p, float4 v) { *(float4*)p = v; }
+__device__ __forceinline__ void store4(bf16_t* p, float4 v) {
+    uint2 t;
+    t.x = (uint32_t)from_float<bf16_t>(v.x).bits | ((uint32_t)from_float<bf16_t>(v.y).bits << 16);
+    t.y = (uint32_t)from_float<bf16_t>(v.z).bits | ((uint32_t)from_float<bf16_t>(v.w).bits << 16);
+    *(uint2*)p = t;
+}
+
 // ---------------------------------------------------------------- reductions
 #define TL_WAVE 64
 

@@ -925,18 +925,6 @@ __global__ void last_token_kernel(const int* __restrict__ ids, const int* __rest
 }
 
 // ------------------------------------------------------------------ rows in pieces of four numbers
-__device__ __forceinline__ float4 load4(const float* p) { return *(const float4*)p; }
-__device__ __forceinline__ float4 load4(const bf16_t* p) {
-    const uint2 t = *(const uint2*)p;
-    return make_float4(__uint_as_float(t.x << 16), __uint_as_float(t.x & 0xffff0000u), __uint_as_float(t.y << 16), __uint_as_float(t.y & 0xffff0000u));
-}
-__device__ __forceinline__ void store4(float* p, float4 v) { *(float4*)p = v; }
-__device__ __forceinline__ void store4(bf16_t* p, float4 v) {
-    uint2 t;
-    t.x = (uint32_t)from_float<bf16_t>(v.x).bits | ((uint32_t)from_float<bf16_t>(v.y).bits << 16);
-    t.y = (uint32_t)from_float<bf16_t>(v.z).bits | ((uint32_t)from_float<bf16_t>(v.w).bits << 16);
-    *(uint2*)p = t;
-}
 // Up to four neighbouring numbers: all four at once where rows are multiples of four (VEC 4), one otherwise.
 template <int VEC, typename T> __device__ __forceinline__ void load_piece(const T* p, float (&v)[VEC]) {
     if constexpr (VEC == 4) { const float4 f = load4(p); v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w; }

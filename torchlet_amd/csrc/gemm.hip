@@ -1362,7 +1362,9 @@ static bool gives_slabs(int M, int N, int K) {
 // 128 x 128 with four slabs in shared memory; 133 x 4608 x 3584 16.5 in three parts, 14.6 in one of 64 x 64).  Split, only the tiles that have a compute unit to themselves
 // are considered; the slabs cost their bytes once written and once read.  parts == 0: a bfloat16 result.
 // With the slabs' reading counted at 4 TB/s the choice takes 1.026 of the fastest plan's time on average over 123 of the fitted sizes, 1.28 at most, and 1.078 over 51 others, 1.54 at most:
-// it undervalues one slab of 128 x 128 (1457 x 2048 x 4096 34.6 in two parts, 28.6 in one).
+// it undervalues one slab of 128 x 128 (1457 x 2048 x 4096 34.6 in two parts, 28.6 in one).  Against the plans before the tiles' figures were refitted, the norm that adds the slabs up included: 0.97 on average over
+// 410 sizes of 65 to 700 rows, 33 of them more than 3 % slower, up to 1.16 (133 x 4608 x 8192: seven parts of 256 x 128 where three of 128 x 128 would take 0.82 of that); no factor on one shape or on one
+// slab that mends those leaves the others as they are.
 struct DlSplit { DlTile tile; int parts; int k_per; };
 static DlSplit plan_dl_split(int M, int N, int K) {
     DlSplit best{DL_128x128, 0, 0};

@@ -366,17 +366,13 @@ gated_row_norm_kernel(const float* __restrict__ o, const T* __restrict__ gate, i
 // The same with a stretch's numbers in registers: LANES threads to a stretch (part of a wave, a wave, or a work-group of its own), NP pieces of four
 // neighbouring numbers to a thread, all requested before the first is used, so that a stretch costs one trip to memory instead of one per number
 // of a thread and pass.  What bounds it is its bytes on prompts and its launch and that one trip in decode steps: 4 tokens of 4096 numbers 15.3 -> 4.0 us, of
-// 8192 27.5 -> 5.4 us (one number a thread and trip before).
+// 8192 27.5 -> 5.4 us (one number a thread and trip before).  (Four: a piece as it is stored, widened where it is used: half the registers of one on its way.)
 template <typename T> struct Four;
 template <> struct Four<float> { typedef float4 type; };
 template <> struct Four<bf16_t> { typedef ushort4 type; };
 __device__ __forceinline__ float4 widen4(float4 v) { return v; }
 __device__ __forceinline__ float4 widen4(ushort4 v) {
     return make_float4(to_float(bf16_t{v.x}), to_float(bf16_t{v.y}), to_float(bf16_t{v.z}), to_float(bf16_t{v.w}));
-}
-__device__ __forceinline__ void store4(float* p, float4 v) { *(float4*)p = v; }
-__device__ __forceinline__ void store4(bf16_t* p, float4 v) {
-    *(ushort4*)p = make_ushort4(from_float<bf16_t>(v.x).bits, from_float<bf16_t>(v.y).bits, from_float<bf16_t>(v.z).bits, from_float<bf16_t>(v.w).bits);
 }
 
 template <typename T, int NP, int LANES>
@@ -1667,12 +1663,6 @@ extern "C" int tl_channel_decay(const void* z, const void* w2t, const void* w0, 
 // step), fetched into registers one batch ahead; a request's last batch is filled up with tokens that change nothing (k = 0, w = 1).
 // `last_rows` (optional, float [tokens, row_width]): the row of the request's last token goes to its slot from tail_off on (what the next
 // portion's first token finds of the token before it).
-template <typename T> __device__ __forceinline__ float4 wkv_load4(const T* p);
-template <> __device__ __forceinline__ float4 wkv_load4<float>(const float* p) { return *(const float4*)p; }
-template <> __device__ __forceinline__ float4 wkv_load4<bf16_t>(const bf16_t* p) {
-    const uint2 t = *(const uint2*)p;
-    return make_float4(__uint_as_float(t.x << 16), __uint_as_float(t.x & 0xffff0000u), __uint_as_float(t.y << 16), __uint_as_float(t.y & 0xffff0000u));
-}
 
 template <typename T, int RPL, int TB>
 __global__ void __launch_bounds__(256)
@@ -1722,8 +1712,8 @@ wkv_scan_kernel(const T* __restrict__ rkv, int ld, int k_off, int v_off, const f
                 const T* row = rkv + (size_t)(base + t) * ld + head * dim + e;
                 const float* wrow = decay + ((size_t)(base + t) * heads + head) * dim + e;
                 if (vec) {
-                    pr[j] = wkv_load4<T>(row);
-                    pk[j] = wkv_load4<T>(row + k_off);
+                    pr[j] = load4(row);
+                    pk[j] = load4(row + k_off);
                     pw[j] = *(const float4*)wrow;
                 } else {
                     float a[4], b[4], c[4];
@@ -1916,7 +1906,6 @@ __device__ __forceinline__ int ck_find(const ChunkArgs& a, int want, int& first_
     return -1;
 }
 
-template <typename T> __device__ __forceinline__ float4 ck_load4(const T* p) { return wkv_load4<T>(p); }
 
 // MEMORY: the matrix memory (b, g and the running maximum per token; outputs over max(|n . q|, exp(-m)) + denom_eps); otherwise fixed decays.
 template <typename T, bool MEMORY>
@@ -1959,7 +1948,7 @@ chunk_states_kernel(ChunkArgs a) {
         const int idx = tid + j * 256, t = idx / (CK_V / 4), c = (idx % (CK_V / 4)) * 4;
         float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
         if (t < nt && v0 + c < a.vdim) {
-            x = ck_load4<T>(vsrc + (size_t)t * a.ld + c);
+            x = load4(vsrc + (size_t)t * a.ld + c);
             const float w = sw[t];
             x.x *= w; x.y *= w; x.z *= w; x.w *= w;
         }
@@ -1972,7 +1961,7 @@ chunk_states_kernel(ChunkArgs a) {
 #pragma unroll
         for (int j = 0; j < CK_T * CK_D / 4 / 256; ++j) {
             const int idx = tid + j * 256, t = idx / (CK_D / 4), c = (idx % (CK_D / 4)) * 4;
-            *(float4*)(sk + t * CK_LD + c) = t < nt && d0 + c < a.dim ? ck_load4<T>(ksrc + (size_t)t * a.ld + d0 + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+            *(float4*)(sk + t * CK_LD + c) = t < nt && d0 + c < a.dim ? load4(ksrc + (size_t)t * a.ld + d0 + c) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
         __syncthreads();
         if (v0 + wave * 32 < a.vdim) {
@@ -2165,8 +2154,8 @@ chunk_outputs_kernel(ChunkArgs a) {
             const int idx = tid + j * 256, t = idx / (CK_D / 4), c = (idx % (CK_D / 4)) * 4;
             float4 x = make_float4(0.f, 0.f, 0.f, 0.f), y = x;
             if (t < nt && d0 + c < a.dim) {
-                x = ck_load4<T>(qsrc + (size_t)t * a.ld + d0 + c);
-                y = ck_load4<T>(ksrc + (size_t)t * a.ld + d0 + c);
+                x = load4(qsrc + (size_t)t * a.ld + d0 + c);
+                y = load4(ksrc + (size_t)t * a.ld + d0 + c);
                 x.x *= a.qscale; x.y *= a.qscale; x.z *= a.qscale; x.w *= a.qscale;
             }
             *(float4*)(sq + t * CK_LD + c) = x;
@@ -2223,7 +2212,7 @@ chunk_outputs_kernel(ChunkArgs a) {
 #pragma unroll
     for (int j = 0; j < CK_T * CK_V / 4 / 256; ++j) {
         const int idx = tid + j * 256, t = idx / (CK_V / 4), c = (idx % (CK_V / 4)) * 4;
-        const float4 x = t < nt && v0 + c < a.vdim ? ck_load4<T>(vsrc + (size_t)t * a.ld + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+        const float4 x = t < nt && v0 + c < a.vdim ? load4(vsrc + (size_t)t * a.ld + c) : make_float4(0.f, 0.f, 0.f, 0.f);
         *(float4*)(ss + t * CK_LV + c) = x;
         if (fmaf(x.x, 0.f, fmaf(x.y, 0.f, fmaf(x.z, 0.f, x.w * 0.f))) != 0.f) *odd = 1;      // an infinity or a NaN
     }
