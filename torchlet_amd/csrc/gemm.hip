@@ -7,7 +7,7 @@
 // product of the 32-bit path and the fallback of the bfloat16 path for shapes that
 // the matrix-core kernels refuse.  The sum over K runs in one fixed order for every
 // output element, whatever M is, so a row's result does not depend on the batch.
-#include "direct_tile.h"
+#include "row_ring.h"
 
 // The compute units of the GPU the library runs on: the caller tells it once (tl_gemm_set_compute_units, from
 // the device's properties); 256, the MI355X on which every plan below was measured, until it does.
@@ -481,7 +481,8 @@ extern "C" int tl_gemm_f32_variant(const void* x, const void* w, const void* bia
 // of which then walks a run of outputs of its own, strip after strip, and requests the first
 // steps of its next strip before it adds up the sums of this one (measured at M = 8, 7B sizes:
 // gate/up 57 -> 51 us, LM head 207 -> 189 us).
-// Needs K % 8 == 0 and 16-byte aligned rows; other shapes go to the general kernel.
+// Needs K % 8 == 0 and 16-byte aligned rows; other shapes go to the general kernel.  With K a multiple of 64 it serves one row against more than 32768 columns and the products that
+// make their norm themselves; gemm_ring_kernel the others.
 #define SK_KOFF(lg) (16 * (lg))     // a lane reads 32 contiguous bytes per step (other splits measured the same)
 #define SK_SECOND 8
 #define SK_LOAD(p) (*(const uint4*)(p))
@@ -527,6 +528,40 @@ struct RopeArgs {
     bf16_t* v_plane;           // [pages, kv_heads, head_dim, page]
     int bt_stride, page, q_heads, kv_heads, head_dim;
 };
+
+// Four neighbouring columns n .. n + 3 of row m, those below n_end: two pairs (pair layout: one frequency turns a pair; a run of columns ends between pairs or not at all), the query
+// and key heads' turned by the row's position `pos`; queries go to out, keys and values to page `page`.
+__device__ __forceinline__ void rope_store(const RopeArgs& ra, const f32x4_t& sum, int n, int n_end, int m, int pos, int page, bf16_t* out, int ldo) {
+#pragma unroll
+    for (int pr = 0; pr < 2; ++pr) {
+        const int np = n + 2 * pr;
+        if (np + 1 >= n_end) continue;                 // runs hold an even number of columns
+        float y1 = sum[2 * pr], y2 = sum[2 * pr + 1];
+        const int head = np / ra.head_dim, dd = np - head * ra.head_dim;
+        if (head < ra.q_heads + ra.kv_heads) {
+            const float angle = (float)pos * ra.inv_freq[dd / 2];
+            const float c = cosf(angle), sn = sinf(angle);
+            const float t1 = y1 * c - y2 * sn;
+            const float t2 = y2 * c + y1 * sn;
+            y1 = t1;
+            y2 = t2;
+        }
+        const uint16_t e1 = from_float<bf16_t>(y1).bits, e2 = from_float<bf16_t>(y2).bits;
+        const uint32_t both = (uint32_t)e1 | ((uint32_t)e2 << 16);
+        if (head < ra.q_heads || !ra.k_plane) {
+            *(uint32_t*)(out + (size_t)m * ldo + np) = both;
+        } else if (page != 0) {     // page 0 is the sentinel (a padding row's): never written
+            const int kvh = (head - ra.q_heads) % ra.kv_heads, off = pos % ra.page;
+            const size_t base = ((size_t)page * ra.kv_heads + kvh) * ra.page * ra.head_dim;
+            if (head < ra.q_heads + ra.kv_heads) {
+                *(uint32_t*)(ra.k_plane + base + (size_t)off * ra.head_dim + dd) = both;
+            } else {
+                ra.v_plane[base + (size_t)dd * ra.page + off].bits = e1;
+                ra.v_plane[base + (size_t)(dd + 1) * ra.page + off].bits = e2;
+            }
+        }
+    }
+}
 
 // Eight neighbouring elements as floats, from float or bfloat16 memory and back.
 __device__ __forceinline__ void load8(const float* p, float* v) {
@@ -866,39 +901,11 @@ __global__ __launch_bounds__(KS * 64) void gemm_skinny_kernel(const bf16_t* __re
                 const int m = t * 16 + li;
                 const int n = n0 + r * 16 + 4 * lg;
                 if (RP) {
-                    // two pairs of neighbouring columns per lane (pair layout: one frequency turns a pair); a strip
-                    // of a number of rows that is no multiple of four may end between them
-                    if (m >= M) continue;
+                    if (bias) {
 #pragma unroll
-                    for (int pr = 0; pr < 2; ++pr) {
-                        const int np = n + 2 * pr;
-                        if (np + 1 >= n_end) continue;                 // strips hold an even number of rows
-                        float y1 = sum[2 * pr] + (bias ? load_vec(bias, bias_f32, np) : 0.f);
-                        float y2 = sum[2 * pr + 1] + (bias ? load_vec(bias, bias_f32, np + 1) : 0.f);
-                        const int head = np / ra.head_dim, dd = np - head * ra.head_dim;
-                        if (head < ra.q_heads + ra.kv_heads) {
-                            const float angle = (float)rp_pos * ra.inv_freq[dd / 2];
-                            const float c = cosf(angle), sn = sinf(angle);
-                            const float t1 = y1 * c - y2 * sn;
-                            const float t2 = y2 * c + y1 * sn;
-                            y1 = t1;
-                            y2 = t2;
-                        }
-                        const uint16_t e1 = from_float<bf16_t>(y1).bits, e2 = from_float<bf16_t>(y2).bits;
-                        const uint32_t both = (uint32_t)e1 | ((uint32_t)e2 << 16);
-                        if (head < ra.q_heads || !ra.k_plane) {
-                            *(uint32_t*)((bf16_t*)out + (size_t)m * ldo + np) = both;
-                        } else if (rp_page != 0) {     // page 0 is the sentinel (a padding row's): never written
-                            const int kvh = (head - ra.q_heads) % ra.kv_heads, off = rp_pos % ra.page;
-                            const size_t base = ((size_t)rp_page * ra.kv_heads + kvh) * ra.page * ra.head_dim;
-                            if (head < ra.q_heads + ra.kv_heads) {
-                                *(uint32_t*)(ra.k_plane + base + (size_t)off * ra.head_dim + dd) = both;
-                            } else {
-                                ra.v_plane[base + (size_t)dd * ra.page + off].bits = e1;
-                                ra.v_plane[base + (size_t)(dd + 1) * ra.page + off].bits = e2;
-                            }
-                        }
+                        for (int v = 0; v < 4; ++v) sum[v] += load_vec(bias, bias_f32, min(n + v, N - 1));
                     }
+                    if (m < M) rope_store(ra, sum, n, n_end, m, rp_pos, rp_page, (bf16_t*)out, ldo);
                     continue;
                 }
                 if (m < M) {
@@ -1028,6 +1035,156 @@ static void pick_skinny(const void* x, const void* w, const void* bias, int bias
         else if (strips >= 1024) launch_skinny<2, MT, 2>(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, out_f32, stream, 0, gr);
         else launch_skinny<1, MT, 8>(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, out_f32, stream, 0, gr);
     }
+}
+
+// ------------------------------------------------------------------ few rows through rings in shared memory (K a multiple of 64)
+// See row_ring.h.  Work-group (i, y, z): outputs i * rps .. of product z (gs), or the y-th range of K of a product split over K (k_per_split columns each, a
+// slab [M, ldo] of partial sums each).  SW: the gate's activation as in gemm_skinny_kernel (out_cols outputs, gate and up rows interleaved in blocks of 32); RP: its rotation and
+// cache write.
+template <int WJ, int XH, typename TOut, int SW = 0, bool RP = false>
+__global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const void* __restrict__ bias, int bias_f32,
+                                                        TOut* __restrict__ out, int M, int N, int K, int ldx, int ldo, int out_cols, int k_per_split, int rps,
+                                                        RopeArgs ra, GroupStride gs) {
+    constexpr int HALVES = SW ? 2 : 1;
+    using S = RingShape<WJ, XH, HALVES>;
+    static_assert(!RP || (!SW && S::MT == 1 && sizeof(TOut) == 2), "the rotation is built for up to 16 rows");
+    extern __shared__ __attribute__((aligned(16))) char ring[];
+    const int ldw = K;
+    x += blockIdx.z * gs.x;
+    w += blockIdx.z * gs.w;
+    out += blockIdx.z * gs.out;
+    if (k_per_split > 0) {
+        const int kb = blockIdx.y * k_per_split;
+        x += kb;
+        w += kb;
+        out += (size_t)blockIdx.y * M * ldo;
+        K = min(K - kb, k_per_split);
+    }
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 15, kg = lane >> 4;
+    const int n0 = blockIdx.x * rps, n_end = min(SW ? out_cols : N, n0 + rps);
+    // (the waves that turn and write: their rows' positions and pages ahead of the weights, so that no wait for them lies behind the ring's)
+    int rp_pos = 0, rp_page = 0;
+    if (RP && wave < S::STRIPS) {
+        const int row = min(li, M - 1);
+        rp_pos = ra.positions[row];
+        if (ra.k_plane) rp_page = ra.block_table[(size_t)ra.token_req[row] * ra.bt_stride + rp_pos / ra.page];
+    }
+    // the matrix's row of an output's gate (or of the output itself); its up row lies 32 further on
+    auto row_of = [](int o) { return SW ? (o >> 5) * 64 + (o & 31) : o; };
+    unsigned woff[WJ], xoff[XH];
+#pragma unroll
+    for (int j = 0; j < WJ; ++j) {
+        const int r = 8 * j + lane / 8, c = (lane % 8) ^ ((r >> 1) & 7), half = r / S::HR;
+        woff[j] = (unsigned)((row_of(min(n0 + r - half * S::HR, n_end - 1)) - row_of(n0) + 32 * half) * ldw + c * 8) * 2;
+    }
+#pragma unroll
+    for (int j = 0; j < XH; ++j) {
+        const int r = 8 * (WJ + j) + lane / 8, c = (lane % 8) ^ ((r >> 1) & 7);
+        xoff[j] = (unsigned)(min(r - 8 * WJ, M - 1) * ldx + c * 8) * 2;
+    }
+    ring_products<WJ, XH, HALVES>(w + (size_t)row_of(n0) * ldw, woff, x, xoff, K / 64, ring, wave, ldw % 2048 == 0);
+    const bool quads = ldo % 4 == 0 && n0 % 4 == 0 && ((uintptr_t)out % (4 * sizeof(TOut))) == 0;
+    for (int q = wave; q < S::SH * S::MT; q += S::NW) {
+        const int s = q / S::MT, t = q % S::MT, m = 16 * t + li, n = n0 + 16 * s + 4 * kg;
+        f32x4_t sum = ring_sum<WJ, XH, HALVES>(ring, s, t);
+        if constexpr (SW) {
+            const f32x4_t up = ring_sum<WJ, XH, HALVES>(ring, S::SH + s, t);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) sum[v] = gate_mul<SW>(sum[v], up[v]);
+        } else if (bias) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) sum[v] += load_vec(bias, bias_f32, min(n + v, N - 1));
+        }
+        if (m >= M) continue;
+        if constexpr (RP) {
+            rope_store(ra, sum, n, n_end, m, rp_pos, rp_page, (bf16_t*)out, ldo);
+        } else if (quads && n + 3 < n_end) {
+            store4(out + (size_t)m * ldo + n, make_float4(sum[0], sum[1], sum[2], sum[3]));
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if (n + v < n_end) out[(size_t)m * ldo + n + v] = from_float<TOut>(sum[v]);
+        }
+    }
+}
+
+// What the rings take: whole slabs, 16-byte aligned rows, offsets inside a work-group's rows (of the interleaved matrix 128 apart at most) that fit 32 bits.
+static bool ring_fits(const void* x, const void* w, int M, int K, int ldx) {
+    return M > 0 && M <= 64 && K % 64 == 0 && ldx % 8 == 0 && K < (1 << 23) && ldx < (1 << 23) && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0;
+}
+
+// Where a product of up to 64 rows goes through the rings: against the tile kernel and, one row, the few-rows kernel that fetches into registers (us, the other / this):
+// 64 rows, 2048 x 2048 8.5 / 6.0, 18432 x 4096 48 / 39, 32000 x 2048 34.2 / 33.9, 152064 x 3584 214 / 254 (the tiles' work-groups share what they fetch of x);
+// 12 rows, 152064 x 3584 190 / 194, 8 rows 197 / 187, 1 row 175 / 183, 1 row, 32000 x 4096 42.5 / 42.8.
+static bool ring_pays(int M, long columns) { return M <= 64 && (columns <= 32768 || (M >= 2 && M <= 8)); }
+
+struct RingCall {
+    const void *x, *w, *bias;
+    int bias_f32;
+    void* out;
+    int M, N, K, ldx, ldo, out_cols;       // out_cols > 0: the fused gate's outputs
+    int parts = 1, k_per = 0;
+    Groups gr = Groups{};
+    RopeArgs ra = RopeArgs{};
+};
+
+template <int WJ, int XH, typename TOut, int SW, bool RP>
+static int launch_ring_t(const RingCall& c, int rows, hipStream_t stream) {
+    using S = RingShape<WJ, XH, SW ? 2 : 1>;
+    auto kernel = gemm_ring_kernel<WJ, XH, TOut, SW, RP>;
+    static hipError_t allowed = allow_lds(kernel, S::LDS);
+    TL_REQUIRE(allowed == hipSuccess, "gemm_ring: cannot get %zu bytes of shared memory", S::LDS);
+    const int total = SW ? c.out_cols : c.N;
+    kernel<<<dim3((total + rows - 1) / rows, c.parts, c.gr.count), 256, S::LDS, stream>>>((const bf16_t*)c.x, (const bf16_t*)c.w, c.bias, c.bias_f32, (TOut*)c.out, c.M, c.N, c.K,
+                                                                                      c.ldx, c.ldo, c.out_cols, c.k_per, rows, c.ra, c.gr.stride);
+    TL_CHECK_LAUNCH("gemm_ring");
+    return TL_OK;
+}
+
+template <int XH, typename TOut, int SW, bool RP>
+static int launch_ring_x(const RingCall& c, RingPlan p, hipStream_t stream) {
+    switch (p.wj) {
+    case 2: return launch_ring_t<2, XH, TOut, SW, RP>(c, p.rows, stream);
+    case 4: return launch_ring_t<4, XH, TOut, SW, RP>(c, p.rows, stream);
+    case 6: return launch_ring_t<6, XH, TOut, SW, RP>(c, p.rows, stream);
+    case 8: return launch_ring_t<8, XH, TOut, SW, RP>(c, p.rows, stream);
+    }
+    if constexpr (!SW) {
+        if (p.wj == 1) return launch_ring_t<1, XH, TOut, SW, RP>(c, p.rows, stream);
+        if (p.wj == 3) return launch_ring_t<3, XH, TOut, SW, RP>(c, p.rows, stream);
+    }
+    TL_REQUIRE(false, "gemm_ring: no shape of %d requests", p.wj);
+}
+
+// `p.wj` 0: the plan is made here.
+template <typename TOut, int SW, bool RP>
+static int launch_ring(const RingCall& c, hipStream_t stream, RingPlan p = RingPlan{0, 0}) {
+    if (p.wj == 0) p = plan_ring(SW ? c.out_cols : c.N, c.M, SW ? 2 : 1, TL_COMPUTE_UNITS / (c.parts * c.gr.count), RP);
+    if (c.M <= 8) return launch_ring_x<1, TOut, SW, RP>(c, p, stream);
+    if (c.M <= 16) return launch_ring_x<2, TOut, SW, RP>(c, p, stream);
+    if constexpr (!RP) {
+        if (c.M <= 32) return launch_ring_x<4, TOut, SW, RP>(c, p, stream);
+        return launch_ring_x<8, TOut, SW, RP>(c, p, stream);
+    }
+    TL_REQUIRE(false, "gemm_ring: too many rows (%d)", c.M);
+}
+
+// One shape of the kernel above (for tests and tuning): 8 wj weight rows a work-group (with `gate`, 1 + the gate's number, half gate and half up rows), `rows` outputs of which
+// are used; parts > 1: K split into ranges of k_per columns, float slabs.  wj 0: as the dispatch would.
+extern "C" int tl_gemm_ring_variant(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int N, int K, int ldx, int ldo, int out_f32, int gate, int wj,
+                                    int rows, int parts, int k_per, hipStream_t stream) {
+    const int total = gate ? ldo : N, halves = gate ? 2 : 1;
+    TL_REQUIRE(ring_fits(x, w, M, K, ldx) && N > 0 && ldo >= (gate ? 1 : N) && gate >= 0 && gate <= 3 && (!gate || (!out_f32 && N == (ldo + 31) / 32 * 64)),
+               "gemm_ring: bad sizes M=%d N=%d K=%d", M, N, K);
+    TL_REQUIRE(wj == 0 || (wj > 0 && wj <= 8 && rows > 0 && rows <= 8 * wj / halves), "gemm_ring: %d outputs do not fit %d requests", rows, wj);
+    TL_REQUIRE(parts == 1 || (parts > 1 && out_f32 && !bias && k_per > 0 && k_per % 64 == 0 && (long)k_per * (parts - 1) < K && (long)k_per * parts >= K),
+               "gemm_ring: %d ranges of %d columns are not a split of %d", parts, k_per, K);
+    RingCall c{x, w, bias, bias_f32, out, M, N, K, ldx, ldo, gate ? total : 0, parts, parts > 1 ? k_per : 0};
+    const RingPlan p{wj, rows};
+    if (gate == 1) return launch_ring<bf16_t, 1, false>(c, stream, p);
+    if (gate == 2) return launch_ring<bf16_t, 2, false>(c, stream, p);
+    if (gate == 3) return launch_ring<bf16_t, 3, false>(c, stream, p);
+    return out_f32 ? launch_ring<float, 0, false>(c, stream, p) : launch_ring<bf16_t, 0, false>(c, stream, p);
 }
 
 // One named instance of the few-rows kernel, of those the dispatch below can pick (for tests and tuning);
@@ -1512,11 +1669,12 @@ static bool skinny_fits(const void* x, const void* w, int M, int K, int ldx) {
 }
 
 // out = x w^T (+ bias) in the engine's dtype: picks the kernel for the shape.
-//   bfloat16, aligned, M <= 64  -> gemm_skinny (matrix cores, weight streaming), except that
-//                                  33..64 rows against a wide matrix go to the tile kernel
-//   bfloat16, aligned, K a multiple of 64, M > 32 (M > 8 against a wide matrix) -> gemm_dl_tile
-//                                  (matrix cores, operands straight into shared memory)
-//   bfloat16, aligned, M > 64   -> gemm_mfma_tile (matrix cores, shared-memory tiles)
+//   bfloat16, aligned, K a multiple of 64:
+//     up to 64 rows against up to 32768 columns, 2 to 8 rows against more -> gemm_ring (see ring_pays)
+//     one row against more        -> gemm_skinny (matrix cores, weight streaming)
+//     everything else             -> gemm_dl_tile (matrix cores, operands straight into shared memory)
+//   bfloat16, aligned, other K, M <= 64 -> gemm_skinny, except that 33..64 rows against a wide matrix go to the tile kernel
+//   bfloat16, aligned, other K, M > 64  -> gemm_mfma_tile (matrix cores, shared-memory tiles)
 //   32-bit, aligned, M <= 16    -> gemv_f32 (true 32-bit arithmetic, weight streaming)
 //   32-bit, aligned, M > 16     -> gemm_f32_mfma (true 32-bit arithmetic on the matrix cores)
 //   everything else             -> gemm_tile (true 32-bit arithmetic)
@@ -1525,9 +1683,11 @@ extern "C" int tl_gemm(const void* x, const void* w, const void* bias, int bias_
     TL_REQUIRE(M >= 0 && N > 0 && K > 0 && ldx >= K && ldo >= N, "gemm: bad sizes M=%d N=%d K=%d ldx=%d ldo=%d", M, N, K, ldx, ldo);
     if (M == 0) return TL_OK;
     const bool aligned = K % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0;
-    // (measured at 17-32 rows: against a wide matrix the tile kernel is far ahead, 60 against 85-107 us
-    // on gate/up and 200 against 310-400 us on the LM head; against a narrow one the skinny kernel wins)
-    if (dtype == TL_DT_BF16 && aligned && K % 64 == 0 && (M > 32 || (M > 8 && N >= 16384))) {
+    if (dtype == TL_DT_BF16 && ring_fits(x, w, M, K, ldx) && ring_pays(M, N)) {
+        const RingCall c{x, w, bias, bias_f32, out, M, N, K, ldx, ldo, 0};
+        return out_f32 ? launch_ring<float, 0, false>(c, stream) : launch_ring<bf16_t, 0, false>(c, stream);
+    }
+    if (dtype == TL_DT_BF16 && aligned && K % 64 == 0 && M > 8) {
         int rc = out_f32 ? launch_dl_tile<float, false>(pick_dl_tile(M, N, K, false), x, w, bias, bias_f32, out, M, N, K, ldx, ldo, 0, stream)
                          : launch_dl_tile<bf16_t, false>(pick_dl_tile(M, N, K, false), x, w, bias, bias_f32, out, M, N, K, ldx, ldo, 0, stream);
         if (rc != TL_OK) return rc;
@@ -1594,15 +1754,20 @@ extern "C" int tl_gemm_rope(const void* x, const void* w, const void* bias, int 
                "gemm_rope: the cache write needs both planes, the block table and the requests of the rows");
     TL_REQUIRE(N == (q_heads + (k_plane ? 2 * kv_heads : 0)) * head_dim, "gemm_rope: %d output columns do not match the heads", N);
     const int strips = (N + 15) / 16, ks = strips >= 1024 ? 16 : 8;
-    // (from 9 rows on the product split over K on the tile kernel plus the rotation kernel that adds its slabs up
-    // is ahead where that split is to be had: 4608 x 3584 at 16 rows 14.5 against 17.0 us, at 8 rows 14.8 against 14.0)
-    if (M > 16 || (M > 8 && tl_gemm_partials_pay(M, N, K)) || !skinny_fits(x, w, M, K, ldx) || N % 16 || ldo % 4 || ((uintptr_t)out % 8) || K / 64 / ks >= 16 ||
+    const bool rings = ring_fits(x, w, M, K, ldx);
+    // (from 9 rows on the product split over K plus the rotation kernel that adds its slabs up stands beside it where that split is to be had)
+    if (M > 16 || (M > 8 && tl_gemm_partials_pay(M, N, K)) || !skinny_fits(x, w, M, K, ldx) || N % 16 || ldo % 4 || ((uintptr_t)out % 8) || (!rings && K / 64 / ks >= 16) ||
         (k_plane && (((uintptr_t)k_plane % 8) || head_dim % 4)))
         return TL_NOT_FUSED;
     RopeArgs ra;
     ra.positions = (const int*)positions; ra.inv_freq = (const float*)inv_freq; ra.token_req = (const int*)token_req;
     ra.block_table = (const int*)block_table; ra.k_plane = (bf16_t*)k_plane; ra.v_plane = (bf16_t*)v_plane;
     ra.bt_stride = bt_stride; ra.page = page > 0 ? page : 1; ra.q_heads = q_heads; ra.kv_heads = k_plane ? kv_heads : 0; ra.head_dim = head_dim;
+    if (rings) {
+        RingCall c{x, w, bias, bias_f32, out, M, N, K, ldx, ldo, 0};
+        c.ra = ra;
+        return launch_ring<bf16_t, 0, true>(c, stream);
+    }
     const bool xl = M > 1 && (size_t)M * (K + 8) * 2 <= SKINNY_XL_MAX_BYTES;
     int blocks = 1;
     const int rows = ks == 8 ? balanced_rows(N, &blocks) : 0;
@@ -1701,10 +1866,10 @@ static int gemm_gated(const void* x, const void* w, void* out, int M, int I, int
     const bf16_t* xb = (const bf16_t*)x;
     const bf16_t* wb = (const bf16_t*)w;
     bf16_t* ob = (bf16_t*)out;
-    // the few-rows kernel where its copy of x fits shared memory (else every wave fetches x as often
-    // as its weights: 32B sizes, 16 rows, 20.2 against 18.9 ms a step)
-    const bool x_fits = M == 1 || (size_t)16 * 1024 + (size_t)M * (K + 8) * 2 <= 156 * 1024;
-    if ((M <= 16 && (x_fits || K % 64 != 0)) || (M <= 32 && K % 64 != 0)) {
+    // through the rings up to 16 rows, up to 64 against up to 24576 rows of the matrix (us, tiles / rings: 32 rows, 22528 x 4096 46 / 34, 27648 x 5120 51.1 / 51.3,
+    // 37888 x 3584 49.9 / 52.3; 64 rows, 2048 x 2048 15.6 / 6.3, 22528 x 4096 47 / 43, 27648 x 5120 56 / 62)
+    if (ring_fits(x, w, M, K, ldx) && (M <= 16 || N <= 24576)) return launch_ring<bf16_t, GATE, false>(RingCall{x, w, nullptr, 0, out, M, N, K, ldx, ldo, I}, stream);
+    if (M <= 32 && K % 64 != 0) {
         if (M <= 16) launch_skinny_t<1, 1, 16, bf16_t, GATE>(xb, wb, nullptr, 0, ob, M, N, K, ldx, ldo, I, stream);
         else launch_skinny_t<1, 2, 16, bf16_t, GATE>(xb, wb, nullptr, 0, ob, M, N, K, ldx, ldo, I, stream);
     } else if (K % 64 == 0) {
@@ -1736,9 +1901,8 @@ extern "C" int tl_gemm_swiglu(const void* x, const void* w, void* out, int M, in
 // units busy; whoever reads the slabs adds them up.  Returns P through `parts` (the caller sizes
 // `out` for tl_gemm_partials_max()).  More than 64 rows: see plan_dl_split (measured at 512 rows:
 // 3584 x 18944 147 -> 82 us, 5120 x 13824 179 -> 82 us, 5120 x 27648 348 -> 150 us, the norm's sum
-// included).  Up to 64 rows, where it pays (see partials_on_tiles), the direct-load tile
-// kernel runs with 64 x 64 tiles (measured at 64 rows, 3584 x 18944: 31 us with four parts against
-// 90 us whole; 3584 x 3584: 9.5 against 20 us); for other K the skinny kernel
+// included).  Up to 64 rows, where it pays (see partials_on_tiles), the rings or, from 33 rows on
+// with K below 8192, the direct-load tile kernel with 64 x 64 tiles; for other K the skinny kernel
 // with R = 4 strips per work-group, which share every x fetch.
 extern "C" int tl_gemm_partials_max() { return 8; }
 
@@ -1799,6 +1963,10 @@ extern "C" int tl_gemm_partials(const void* x, const void* w, void* out, int M, 
     const int k_per = ((steps + P - 1) / P) * 64;
     P = (K + k_per - 1) / k_per;
     *parts = P;
+    // (the rings against the tiles, us: 16 rows, 2048 x 2048 4.4 / 3.5, 4096 x 8192 17.9 / 13.5, 3584 x 18944 26.8 / 24.4; 64 rows, 4096 x 8192 19.4 / 18.1, 3584 x 18944
+    // 36.6 / 33.9, 4096 x 4096 11.1 / 11.4, 3584 x 3584 at 48 rows 9.4 / 9.9)
+    if (partials_on_tiles(M, N, K) && ring_fits(x, w, M, K, ldx) && (M <= 32 || K >= 8192))
+        return launch_ring<float, 0, false>(RingCall{x, w, nullptr, 0, out, M, N, K, ldx, N, 0, P, k_per}, stream);
     if (partials_on_tiles(M, N, K)) {
         auto kernel = gemm_dl_tile_kernel<64, 64, 2, 2, 4, float, false>;
         constexpr size_t lds = (size_t)4 * 128 * 64 * sizeof(bf16_t);
@@ -1836,7 +2004,12 @@ extern "C" int tl_gemm_groups(const void* x, long x_group, const void* w, void* 
     gr.count = groups;
     gr.stride = GroupStride{x_group, (long)N * K, out_group};
     const bool aligned = K % 8 == 0 && ldx % 8 == 0 && x_group % 8 == 0 && out_group % 8 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0;
-    if (dtype == TL_DT_BF16 && aligned && K % 64 == 0 && (M > 32 || (M > 8 && (long)N * groups >= 16384))) {
+    if (dtype == TL_DT_BF16 && x_group % 8 == 0 && ring_fits(x, w, M, K, ldx) && ring_pays(M, (long)N * groups)) {
+        RingCall c{x, w, nullptr, 0, out, M, N, K, ldx, ldo, 0};
+        c.gr = gr;
+        return out_f32 ? launch_ring<float, 0, false>(c, stream) : launch_ring<bf16_t, 0, false>(c, stream);
+    }
+    if (dtype == TL_DT_BF16 && aligned && K % 64 == 0 && M > 8) {
         const DlTile tile = pick_dl_tile(M, N, K, false, groups);
         const int rc = out_f32 ? launch_dl_tile<float, false>(tile, x, w, nullptr, 0, out, M, N, K, ldx, ldo, 0, stream, 1, 0, gr)
                                : launch_dl_tile<bf16_t, false>(tile, x, w, nullptr, 0, out, M, N, K, ldx, ldo, 0, stream, 1, 0, gr);

@@ -1,0 +1,163 @@
+// Products of few rows against a matrix that is streamed once: every wave keeps a ring of slabs of its own in shared memory.  Shared by the plain products
+// (gemm.hip) and the products over groups of rows (experts.hip).
+#pragma once
+#include "direct_tile.h"
+
+// A work-group of four waves owns 8 WJ weight rows and all rows of x (8 XH at most).  K is dealt to its waves in slabs of 64 columns, slab s to wave s % 4; a wave
+// requests its slabs (the weight rows' and x's 128 bytes each) straight into its own part of shared memory, D of them ahead, waits for its own requests alone and
+// takes the products of a slab when it is there.  No barrier until the end, where the waves' sums meet in shared memory.
+//
+// Such a product takes as long as a compute unit needs to draw its share of the weights and its copy of x, and it draws at the rate of what it has on its way: a kernel
+// whose waves fetch weight rows into registers (two steps of K each) behind a copy of x into shared memory had 16 to 32 KB on their way, fetched with sixteen rows to an
+// instruction, and waited for x before the first product.  Here it is 64 to 80 KB a work-group, two work-groups to a unit where the plan has so many, each
+// instruction fetches eight whole lines, and x arrives beside the weights.  Measured against that kernel (us, launch included, weights from memory; rows of x, N x K):
+//   1 row: 2048 x 2048 3.8 -> 3.2, 4608 x 3584 8.1 -> 7.4;  8 rows: 256 x 2048 4.1 -> 3.1, 2048 x 2048 5.0 -> 3.5, 6144 x 2048 9.1 -> 6.5, 4096 x 4096 11.8 -> 7.6, gate and up
+//   of 2 x 18944 x 3584 50.6 -> 46.9;  16 rows: 34 x 4096 8.9 -> 4.2, 2048 x 2048 6.2 -> 3.7, gate and up of 2 x 11264 x 4096 38.9 -> 32.0;  32 rows: 4608 x 3584 21.8 -> 10.8
+//
+// HALVES 2: the weight rows are two halves of 4 WJ rows (the gate's and the up matrix's rows of the same outputs).
+template <int WJ, int XH, int HALVES = 1>
+struct RingShape {
+    static constexpr int NW = 4;
+    static constexpr int SLOT = (WJ + XH) * 1024;                          // bytes of a slab: 8 (WJ + XH) rows of 128
+    static constexpr int FIT = 80 * 1024 / (NW * SLOT), D = FIT < 2 ? 2 : FIT > 4 ? 4 : FIT;
+    static constexpr int HR = 8 * WJ / HALVES, SH = (HR + 15) / 16;        // weight rows of a half, and the blocks of 16 they make
+    static constexpr int STRIPS = HALVES * SH, MT = (XH + 1) / 2;          // blocks of 16 weight rows and of 16 rows of x
+    static constexpr int SETS = XH <= 2 ? 2 : 1;                           // sets of sums a wave keeps: see ring_products
+    static constexpr size_t LDS = (size_t)NW * D * SLOT;
+    static_assert(WJ % HALVES == 0 && (HALVES - 1) * HR + 16 * SH <= 8 * (WJ + XH), "a block that is not full reads on in its own slab");
+    static_assert(SETS * STRIPS * MT * 1024 <= D * SLOT, "a wave's sums fit its own ring");
+    static_assert((WJ + XH) * (D - 1) < 64 && LDS <= 160 * 1024, "requests on their way fit the counter, rings the shared memory");
+};
+
+// The products of `slabs` slabs: request j of a slab fetches eight rows of 128 bytes at w + woff[j] (x + xoff[j]), bytes, moved on by 128 a slab.  `wave` is uniform.
+// On return every wave's sums lie in its ring (see ring_sum) and all waves have met.
+//
+// Up to 16 rows of x the numbers are summed as gemm_skinny_kernel with eight waves sums them, to the bit (the product that makes its norm itself runs there, and a request must
+// not notice which of the two served it): slab s belongs to sum s % 8, so a wave keeps two sets, and lane group g holds the columns 16 g .. + 15 of a slab.
+//
+// `spread`: the weight rows lie a multiple of 4 KB apart.  Work-groups in step then ask the same few channels of the memory for all their rows, so they begin at different
+// slabs; this order spreads both neighbours and the work-groups of an XCD (us, in step -> spread: 16 rows, 8144 x 4096 16.3 -> 13.7, 32000 x 4096 48 -> 41, 4096 x 16384
+// 33 -> 22, 11264 x 2048 10.9 -> 9.9; with other pitches, 4608 x 3584 8.1 -> 8.5, 2048 x 5632 8.4 -> 8.4).  With few slabs a wave has them all on their way from the
+// start, and 4096 columns by 1024 of K took 8.3 instead of 7.6.
+template <int WJ, int XH, int HALVES>
+__device__ __forceinline__ void ring_products(const bf16_t* w, const unsigned (&woff)[WJ], const bf16_t* x, const unsigned (&xoff)[XH], int slabs, char* ring, int wave, bool spread) {
+    using S = RingShape<WJ, XH, HALVES>;
+    constexpr int NW = S::NW, D = S::D, LPS = WJ + XH, MT = S::MT;
+    const int lane = threadIdx.x & 63, li = lane & 15, kg = lane >> 4;
+    char* own = ring + wave * (D * S::SLOT);
+    const unsigned own_at = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)((void __attribute__((address_space(3)))*)own));
+    const int mine = slabs > wave ? (slabs - wave + NW - 1) / NW : 0;
+    const int from = spread && mine >= 8 ? (int)((blockIdx.x + blockIdx.x / 8) % (unsigned)mine) : 0;
+    auto request = [&](int i) {
+        const int turned = i + from < mine ? i + from : i + from - mine;
+        const int k = 64 * (wave + turned * NW);
+        const unsigned at = own_at + (unsigned)((i % D) * S::SLOT);
+#pragma unroll
+        for (int j = 0; j < WJ; ++j) load_to_lds_at(w + k, woff[j], at + j * 1024);
+#pragma unroll
+        for (int j = 0; j < XH; ++j) load_to_lds_at(x + k, xoff[j], at + (WJ + j) * 1024);
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (d < mine) request(d);
+    // where this lane's two pieces of a block lie in a slab
+    int wat[S::STRIPS][2], xat[MT][2];
+#pragma unroll
+    for (int s = 0; s < S::STRIPS; ++s) {
+        const int row = (s / S::SH) * S::HR + (s % S::SH) * 16 + li;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) wat[s][h] = row * 128 + (((2 * kg + h) ^ ((row >> 1) & 7)) * 16);
+    }
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        const int row = 8 * WJ + 16 * t + (XH == 1 ? li & 7 : li);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) xat[t][h] = row * 128 + (((2 * kg + h) ^ ((row >> 1) & 7)) * 16);
+    }
+    f32x4_t acc[S::SETS][S::STRIPS][MT];
+#pragma unroll
+    for (int u = 0; u < S::SETS; ++u)
+#pragma unroll
+        for (int s = 0; s < S::STRIPS; ++s)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) acc[u][s][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    auto products = [&](int i, f32x4_t (&sums)[S::STRIPS][MT]) {
+        const int after = mine - 1 - i;                 // slabs requested behind this one: D - 1 at most
+        if (after >= D - 1) wait_direct_loads<(D - 1) * LPS>();
+        else if (D > 3 && after == 2) wait_direct_loads<(D > 3 ? 2 : 0) * LPS>();
+        else if (D > 2 && after == 1) wait_direct_loads<(D > 2 ? 1 : 0) * LPS>();
+        else wait_direct_loads<0>();
+        const char* slab = own + (i % D) * S::SLOT;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            Frag16 wf[S::STRIPS], xf[MT];
+#pragma unroll
+            for (int t = 0; t < MT; ++t) xf[t].u = *(const uint4*)(slab + xat[t][h]);
+#pragma unroll
+            for (int s = 0; s < S::STRIPS; ++s) wf[s].u = *(const uint4*)(slab + wat[s][h]);
+#pragma unroll
+            for (int s = 0; s < S::STRIPS; ++s)
+#pragma unroll
+                for (int t = 0; t < MT; ++t) sums[s][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[s].v, xf[t].v, sums[s][t], 0, 0, 0);
+        }
+        if (i + D < mine) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // this slab has been read: its place is filled anew
+            request(i + D);
+        }
+    };
+    // (the last slab of an odd number stands behind the loop, not in it: with a way out between the two sets the compiler copied a set's registers from pass to pass, and
+    // read one of them before the matrix instruction that writes it was through)
+    int i = 0;
+    for (; i + S::SETS <= mine; i += S::SETS) {
+        products(i, acc[0]);
+        if constexpr (S::SETS == 2) products(i + 1, acc[1]);
+    }
+    if (S::SETS == 2 && i < mine) products(i, acc[0]);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_nop 15" ::: "memory");      // (and the last products through, whichever way led here)
+#pragma unroll
+    for (int u = 0; u < S::SETS; ++u)
+#pragma unroll
+        for (int s = 0; s < S::STRIPS; ++s)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) *(f32x4_t*)(own + ((u * S::STRIPS + s) * MT + t) * 1024 + lane * 16) = acc[u][s][t];
+    __syncthreads();
+}
+
+// The waves' sums of block s of weight rows and block t of x: element v is weight row 16 (s % SH) + 4 (lane / 16) + v of half s / SH against x row 16 t + lane % 16.
+template <int WJ, int XH, int HALVES>
+__device__ __forceinline__ f32x4_t ring_sum(const char* ring, int s, int t) {
+    using S = RingShape<WJ, XH, HALVES>;
+    f32x4_t sum = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < S::SETS; ++u)
+#pragma unroll
+        for (int v = 0; v < S::NW; ++v) sum += *(const f32x4_t*)(ring + v * (S::D * S::SLOT) + ((u * S::STRIPS + s) * S::MT + t) * 1024 + (threadIdx.x & 63) * 16);
+    return sum;
+}
+
+// The shapes that are built, and how outputs are dealt out: `wj` of the shape, `rows` outputs to a work-group (8 wj / halves at most).
+struct RingPlan {
+    int wj, rows;
+};
+
+// `units` compute units share `total` outputs: the shape with the least of (rounds of work-groups) x (rows a work-group draws, x's among them, and a third of eight rows for its
+// start and end), then equal shares for all work-groups of these rounds: a launch is as slow as its busiest unit (4608 rows at 18 a unit 8.0 us, at 24 8.6, at
+// 16 and two rounds 9.3).  No fewer than eight rows: one request fetches as many.
+static RingPlan plan_ring(int total, int M, int halves, int units, bool even) {
+    const int xh = M <= 8 ? 1 : M <= 16 ? 2 : M <= 32 ? 4 : 8;
+    if (units < 1) units = 1;
+    RingPlan best{0, 0};
+    double least = 1e30;
+    for (int wj : {1, 2, 3, 4, 6, 8}) {
+        if (wj % halves) continue;
+        const long per = 8 * wj / halves, rounds = ((total + per - 1) / per + units - 1) / units;
+        const double cost = rounds * (wj + 0.5 * xh + 0.3);
+        if (cost >= least) continue;
+        least = cost;
+        const long groups = rounds * units;
+        int rows = (int)((total + groups - 1) / groups), floor = 8 / halves;
+        if (even) rows += rows & 1;
+        best = RingPlan{wj, rows < floor ? floor : rows > per ? (int)per : rows};
+    }
+    return best;
+}

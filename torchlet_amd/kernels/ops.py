@@ -440,6 +440,24 @@ def linear_few_rows_variant(x, weight, bias, out, strips_per_wave: int, waves_al
                                            c_int(waves_along_k), c_int(rows_per_strip), _stream()))
 
 
+def linear_ring_variant(x, weight, bias, out, requests: int = 0, rows: int = 0, parts: int = 1, activation: str | None = None) -> None:
+    """One shape of the kernel whose waves keep rings of slabs in shared memory (for tests and tuning): ``8 * requests`` weight rows a work-group, of which
+    ``rows`` outputs are used (``requests`` 0: as the library would choose); K a multiple of 64, up to 64 rows.  ``parts`` > 1: float32 slabs ``out [parts, M, N]``
+    of ranges of K.  ``activation``: the gated product of :func:`linear_swiglu`."""
+    M, K = x.shape
+    gate = 0 if activation is None else 1 + GATE_ACTIVATIONS[activation]
+    N = weight.shape[0] if not gate else out.shape[1]
+    if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.shape[1] != K or not weight.is_contiguous() or x.stride(1) != 1 or out.stride(-1) != 1 \
+            or out.shape != ((M, N) if parts == 1 else (parts, M, N)) or (parts > 1 and not out.is_contiguous()) \
+            or (gate and (weight.shape[0] != -(-N // 32) * 64 or not out.is_contiguous() or bias is not None)):
+        raise KernelError("linear_ring_variant: bfloat16 operands and fitting shapes only")
+    bf = _vec(bias, N, "linear bias")
+    lib = _lib("gemm")
+    _check(lib, lib.tl_gemm_ring_variant(_ptr(x), _ptr(weight), _ptr(bias), c_int(bf), _ptr(out), c_int(M), c_int(weight.shape[0]), c_int(K), c_int(x.stride(0)),
+                                         c_int(out.stride(-2)), c_int(1 if out.dtype == torch.float32 else 0), c_int(gate), c_int(requests), c_int(rows), c_int(parts),
+                                         c_int(-(-(K // 64) // parts) * 64), _stream()))
+
+
 def linear_many_rows_variant(x, weight, bias, out, tile_m: int, tile_n: int, slab: int = 32) -> None:
     """One named tile shape of the many-rows matrix-core kernel (for tests and tuning)."""
     M, K = x.shape
