@@ -742,44 +742,80 @@ streams_norm_kernel(float* __restrict__ x, int S, int total_rows, int hidden, co
     }
 }
 
+// p += the N slabs' four numbers at src, src + stride, ...: all requested, then added in their order.
+template <int N>
+__device__ __forceinline__ void add_slabs4(const float* src, size_t stride, float4& p) {
+    float4 b[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) b[u] = *(const float4*)(src + u * stride);
+#pragma unroll
+    for (int u = 0; u < N; ++u) { p.x += b[u].x; p.y += b[u].y; p.z += b[u].z; p.w += b[u].w; }
+}
+
 // The same with a row in registers (rows of a multiple of 4 numbers, up to 16384, and 1, 2 or 4 copies): a thread holds N pieces of four numbers,
 // every copy's piece and the pending output's are requested together, and the passes over u (mean, squared deviations, output) read registers.
 // What bounds it: a decode step's few rows the trip to memory and the two sums over the work-group, a prompt's rows the bytes (each copy once in
 // and once out).  Measured against the kernel above (four copies, a pending output of bfloat16, layer norm): see tl_streams_norm.
+// One trip to memory: the copies, the pending output, the norm's vectors and the numbers of the mix are all requested before the first is used, slabs of partial sums four at a time (one after
+// the other, and the vectors behind the two sums, 8 rows of four copies of 2048 with four slabs took 5.1 us, with this 4.1; 8 rows of 8192 10.0 / 7.0).
 template <typename T, int S, int N>
 __global__ void __launch_bounds__(1024)
 streams_norm_reg_kernel(float* __restrict__ x, int total_rows, int hidden, const void* __restrict__ pending, int parts, const float* __restrict__ mix,
                         const float* __restrict__ gate, const float* __restrict__ read, int kind, const void* __restrict__ weight, int weight_f32,
                         const void* __restrict__ bias, int bias_f32, float eps, float gain, T* __restrict__ out, const int* __restrict__ rows) {
-    __shared__ float red[16];
+    constexpr bool EARLY = S * N <= 8;               // the norm's vectors in registers from the start, where there is room for them
+    __shared__ float red[2][16];
     const int orow = blockIdx.x;
     const int srow = rows ? rows[orow] : orow;
     const size_t copy_stride = (size_t)total_rows * hidden;
     float* xr = x + (size_t)srow * hidden;
-    float4 xs[S][N], p[N], u[N];
+    float m[S][S], g[S], rd[S];
+#pragma unroll
+    for (int b = 0; b < S; ++b) {
+        g[b] = gate ? gate[b] : 1.f;
+        rd[b] = read ? read[b] : 1.f;
+#pragma unroll
+        for (int a = 0; a < S; ++a) m[a][b] = mix ? mix[a * S + b] : (a == b ? 1.f : 0.f);
+    }
+    float4 xs[S][N], p[N], u[N], w[EARLY ? N : 1], sh[EARLY ? N : 1];
+    auto vec4 = [](const void* v, int is_f32, int i) { return is_f32 ? load4((const float*)v + i) : load4((const bf16_t*)v + i); };
+    // (beyond the row: its last piece again, kept out of the sums and the stores)
+    auto at = [&](int j) { return min(4 * (int)(threadIdx.x + j * blockDim.x), hidden - 4); };
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-        const int i = 4 * (threadIdx.x + j * blockDim.x);
+        const int i = at(j);
 #pragma unroll
-        for (int a = 0; a < S; ++a) xs[a][j] = i < hidden ? *(const float4*)(xr + a * copy_stride + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int a = 0; a < S; ++a) xs[a][j] = *(const float4*)(xr + a * copy_stride + i);
         p[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (pending && i < hidden) {
-            if (parts == 0) {
-                const T* pen = (const T*)pending + (size_t)srow * hidden + i;
-                if constexpr (sizeof(T) == 4) p[j] = *(const float4*)pen;
-                else {
-                    const uint2 b = *(const uint2*)pen;
-                    p[j] = make_float4(__uint_as_float(b.x << 16), __uint_as_float(b.x & 0xffff0000u), __uint_as_float(b.y << 16), __uint_as_float(b.y & 0xffff0000u));
-                }
-            } else {
-                const float* slab = (const float*)pending + (size_t)srow * hidden + i;
-                for (int q = 0; q < parts; ++q) {
-                    const float4 b = *(const float4*)(slab + q * copy_stride);
-                    p[j].x += b.x; p[j].y += b.y; p[j].z += b.z; p[j].w += b.w;
-                }
-            }
+        if (pending && parts == 0) p[j] = load4((const T*)pending + (size_t)srow * hidden + i);
+    }
+    if (EARLY) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            w[j] = vec4(weight, weight_f32, at(j));
+            if (kind == 1) sh[j] = vec4(bias, bias_f32, at(j));
         }
     }
+    if (pending && parts > 0) {                      // slabs in their order, four requested together
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const float* slab = (const float*)pending + (size_t)srow * hidden + at(j);
+            int q = 0;
+            for (; q + 4 <= parts; q += 4) add_slabs4<4>(slab + q * copy_stride, copy_stride, p[j]);
+            if (parts - q == 3) add_slabs4<3>(slab + q * copy_stride, copy_stride, p[j]);
+            else if (parts - q == 2) add_slabs4<2>(slab + q * copy_stride, copy_stride, p[j]);
+            else if (parts - q == 1) add_slabs4<1>(slab + q * copy_stride, copy_stride, p[j]);
+        }
+    }
+    const int lane = threadIdx.x % TL_WAVE, wave = threadIdx.x / TL_WAVE, waves = blockDim.x / TL_WAVE;
+    auto row_sum = [&](float v, float* place) {
+        v = wave_sum(v);
+        if (lane == 0) place[wave] = v;
+        __syncthreads();
+        float t = 0.f;
+        for (int i = 0; i < waves; ++i) t += place[i];
+        return t;
+    };
     float sum = 0.f;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
@@ -789,19 +825,17 @@ streams_norm_reg_kernel(float* __restrict__ x, int total_rows, int hidden, const
 #pragma unroll
             for (int b = 0; b < S; ++b) {
                 nb[b] = make_float4(0.f, 0.f, 0.f, 0.f);
-                const float gb = gate ? gate[b] : 1.f;
 #pragma unroll
                 for (int a = 0; a < S; ++a) {
-                    const float m = mix ? mix[a * S + b] : (a == b ? 1.f : 0.f);
-                    nb[b].x = fmaf(m, xs[a][j].x, nb[b].x);
-                    nb[b].y = fmaf(m, xs[a][j].y, nb[b].y);
-                    nb[b].z = fmaf(m, xs[a][j].z, nb[b].z);
-                    nb[b].w = fmaf(m, xs[a][j].w, nb[b].w);
+                    nb[b].x = fmaf(m[a][b], xs[a][j].x, nb[b].x);
+                    nb[b].y = fmaf(m[a][b], xs[a][j].y, nb[b].y);
+                    nb[b].z = fmaf(m[a][b], xs[a][j].z, nb[b].z);
+                    nb[b].w = fmaf(m[a][b], xs[a][j].w, nb[b].w);
                 }
-                nb[b].x = fmaf(gb, p[j].x, nb[b].x);
-                nb[b].y = fmaf(gb, p[j].y, nb[b].y);
-                nb[b].z = fmaf(gb, p[j].z, nb[b].z);
-                nb[b].w = fmaf(gb, p[j].w, nb[b].w);
+                nb[b].x = fmaf(g[b], p[j].x, nb[b].x);
+                nb[b].y = fmaf(g[b], p[j].y, nb[b].y);
+                nb[b].z = fmaf(g[b], p[j].z, nb[b].z);
+                nb[b].w = fmaf(g[b], p[j].w, nb[b].w);
             }
 #pragma unroll
             for (int b = 0; b < S; ++b) {
@@ -812,16 +846,15 @@ streams_norm_reg_kernel(float* __restrict__ x, int total_rows, int hidden, const
         u[j] = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int b = 0; b < S; ++b) {
-            const float rd = read ? read[b] : 1.f;
-            u[j].x = fmaf(rd, xs[b][j].x, u[j].x);
-            u[j].y = fmaf(rd, xs[b][j].y, u[j].y);
-            u[j].z = fmaf(rd, xs[b][j].z, u[j].z);
-            u[j].w = fmaf(rd, xs[b][j].w, u[j].w);
+            u[j].x = fmaf(rd[b], xs[b][j].x, u[j].x);
+            u[j].y = fmaf(rd[b], xs[b][j].y, u[j].y);
+            u[j].z = fmaf(rd[b], xs[b][j].z, u[j].z);
+            u[j].w = fmaf(rd[b], xs[b][j].w, u[j].w);
         }
-        sum += (u[j].x + u[j].y) + (u[j].z + u[j].w);
+        if (i < hidden) sum += (u[j].x + u[j].y) + (u[j].z + u[j].w);
     }
     float mean = 0.f;
-    if (kind == 1) mean = block_sum(sum, red) / (float)hidden;
+    if (kind == 1) mean = row_sum(sum, red[0]) / (float)hidden;
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
@@ -830,22 +863,21 @@ streams_norm_reg_kernel(float* __restrict__ x, int total_rows, int hidden, const
             ss = fmaf(u[j].x, u[j].x, fmaf(u[j].y, u[j].y, fmaf(u[j].z, u[j].z, fmaf(u[j].w, u[j].w, ss))));
         }
     }
-    ss = block_sum(ss, red);
+    ss = row_sum(ss, red[1]);
     const float inv = 1.f / sqrtf(ss / (float)hidden + eps);
 #pragma unroll
     for (int j = 0; j < N; ++j) {
         const int i = 4 * (threadIdx.x + j * blockDim.x);
         if (i >= hidden) continue;
-        const float d[4] = {u[j].x * inv, u[j].y * inv, u[j].z * inv, u[j].w * inv};
-        T y[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float w = load_vec(weight, weight_f32, i + e);
-            y[e] = from_float<T>(kind == 1 ? (d[e] * w + load_vec(bias, bias_f32, i + e)) * gain : d[e] * gain * w);
+        const float4 wj = EARLY ? w[EARLY ? j : 0] : vec4(weight, weight_f32, i);
+        float4 y;
+        if (kind == 1) {
+            const float4 bj = EARLY ? sh[EARLY ? j : 0] : vec4(bias, bias_f32, i);
+            y = make_float4((u[j].x * inv * wj.x + bj.x) * gain, (u[j].y * inv * wj.y + bj.y) * gain, (u[j].z * inv * wj.z + bj.z) * gain, (u[j].w * inv * wj.w + bj.w) * gain);
+        } else {
+            y = make_float4(u[j].x * inv * gain * wj.x, u[j].y * inv * gain * wj.y, u[j].z * inv * gain * wj.z, u[j].w * inv * gain * wj.w);
         }
-        T* dst = out + (size_t)orow * hidden + i;
-        if constexpr (sizeof(T) == 4) *(float4*)dst = make_float4(y[0], y[1], y[2], y[3]);
-        else *(uint2*)dst = make_uint2((uint32_t)y[0].bits | ((uint32_t)y[1].bits << 16), (uint32_t)y[2].bits | ((uint32_t)y[3].bits << 16));
+        store4(out + (size_t)orow * hidden + i, y);
     }
 }
 
@@ -857,9 +889,9 @@ extern "C" int tl_streams_norm(void* x, int streams, int total_rows, int hidden,
     TL_REQUIRE((size_t)hidden * sizeof(float) <= 60 * 1024, "streams_norm: rows of %d numbers do not fit the shared memory", hidden);
     TL_REQUIRE((mix == nullptr) == (gate == nullptr), "streams_norm: mix and gate come together");
     if (n_out == 0) return TL_OK;
-    // Rows in registers wherever a piece of four numbers can be fetched whole (us, this kernel / the one above: 8 rows of 2048 under 9 / 15.4, 8 rows of 8192 10 / 45, 2048 rows of
-    // 2048 27.5 / 44.8 and of 4096 50.8 / 78.2; the short ones are bound by their launch).
-    const bool pieces = hidden % 4 == 0 && hidden <= 16384 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)pending % 16) == 0 && ((uintptr_t)out % 16) == 0;
+    // Rows in registers wherever a piece of four numbers can be fetched whole (us, this kernel / the one above: 8 rows of 2048 4.0 / 15.4, 8 rows of 8192 7.0 / 45, 2048 rows of
+    // 2048 25.3 / 44.8 and of 4096 48.3 / 78.2; the short ones are bound by their launch).
+    const bool pieces = hidden % 4 == 0 && hidden <= 16384 && (((uintptr_t)x | (uintptr_t)pending | (uintptr_t)out | (uintptr_t)weight | (uintptr_t)bias) % 16) == 0;
     if (pieces && (streams == 1 || streams == 2 || streams == 4) && (act_dtype == TL_DT_F32 || act_dtype == TL_DT_BF16)) {
         const int n = hidden <= 4096 ? 1 : hidden <= 8192 ? 2 : 4, threads = ((hidden / 4 + n - 1) / n + TL_WAVE - 1) / TL_WAVE * TL_WAVE;
 #define TL_SN_T(T, S, N) streams_norm_reg_kernel<T, S, N><<<n_out, threads, 0, stream>>>((float*)x, total_rows, hidden, pending, parts, (const float*)mix, \
