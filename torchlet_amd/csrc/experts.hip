@@ -455,12 +455,17 @@ extern "C" int tl_grouped_gemm(const void* a, int a_ld, int a_group, const void*
 //           experts' scores divided by their sum plus weight_eps.
 // In every mode the weights are multiplied by weight_scale at the end.  group_size > 0: the experts lie in groups of that many neighbours, a
 // group counts as much as the best of its experts (by what the choice goes by), and only the group_keep best groups' experts can be chosen.
-__global__ void route_topk_kernel(const float* __restrict__ logits, int experts, int top, int mode, const float* __restrict__ bias,
-                                  int* __restrict__ chosen, float* __restrict__ weights, int tokens, float weight_scale, float weight_eps, int group_size,
-                                  int group_keep) {
-    const int t = blockIdx.x * (blockDim.x / TL_WAVE) + threadIdx.x / TL_WAVE, lane = threadIdx.x % TL_WAVE;
-    if (t >= tokens) return;
-    const float* z = logits + (size_t)t * experts;
+struct RouteRule {
+    int experts, top, mode;
+    const float* bias;
+    float weight_scale, weight_eps;
+    int group_size, group_keep;
+};
+
+// One token's choice by one wave: z its logits, chosen and weights its `top` places.
+__device__ __forceinline__ void route_token(const float* z, const RouteRule& r, int* chosen, float* weights) {
+    const int lane = threadIdx.x % TL_WAVE, experts = r.experts, mode = r.mode;
+    const float* bias = r.bias;
     float zmax = 0.f, den = 1.f;
     if (mode == 1) {
         float mx = -INFINITY;
@@ -492,48 +497,138 @@ __global__ void route_topk_kernel(const float* __restrict__ logits, int experts,
         return min(at, experts - 1);                    // (outputs that are no numbers choose nothing: the last expert stands in)
     };
     unsigned long long taken = 0;                       // the experts that are chosen already, or whose group is not kept
-    if (group_size > 0) {
+    if (r.group_size > 0) {
         unsigned long long kept = 0;                    // the best expert outside the kept groups tells the next best group
-        for (int j = 0; j < group_keep; ++j) {
+        for (int j = 0; j < r.group_keep; ++j) {
             float best, score;
-            const int g = pick(kept, best, score) / group_size;
+            const int g = pick(kept, best, score) / r.group_size;
             for (int e = lane, i = 0; e < experts; e += TL_WAVE, ++i)
-                if (e / group_size == g) kept |= 1ull << i;
+                if (e / r.group_size == g) kept |= 1ull << i;
         }
         taken = ~kept;
     }
-    for (int j = 0; j < top; ++j) {
+    for (int j = 0; j < r.top; ++j) {
         float best, score;
         const int at = pick(taken, best, score);
         if (at % TL_WAVE == lane) taken |= 1ull << (at / TL_WAVE);
         if (j == 0) first = best;
         const float p = mode != 0 ? score : expf(best - first);
         sum += p;
-        if (lane == j) { chosen[(size_t)t * top + j] = at; mine = p; }
+        if (lane == j) { chosen[j] = at; mine = p; }
     }
-    if (lane < top) weights[(size_t)t * top + lane] = (mode == 1 ? mine : mode == 2 ? mine / (sum + weight_eps) : mine / sum) * weight_scale;
+    if (lane < r.top) weights[lane] = (mode == 1 ? mine : mode == 2 ? mine / (sum + r.weight_eps) : mine / sum) * r.weight_scale;
+}
+
+// The same for up to 64 experts, one to a lane: what the choice goes by stays in a register, and the best lane is found by its value's maximum and a ballot (the lowest lane of
+// those that have it), where the walk above carries value, score and index through every exchange.  The same choices and weights, to the bit.
+__device__ __forceinline__ void route_token_lanes(const float* z, const RouteRule& r, int* chosen, float* weights) {
+    const int lane = threadIdx.x % TL_WAVE, experts = r.experts, mode = r.mode;
+    const bool real = lane < experts;
+    const float mine_z = real ? z[lane] : -INFINITY;
+    float v = mine_z, score = 0.f;
+    if (mode == 1) {
+        const float zmax = wave_max(fmaxf(-INFINITY, mine_z));
+        const float den = wave_sum(real ? expf(mine_z - zmax) : 0.f);
+        score = expf(mine_z - zmax) / den;
+    } else if (mode == 2) {
+        score = 1.f / (1.f + expf(-mine_z));
+    }
+    if (mode != 0) v = r.bias && real ? score + r.bias[lane] : score;
+    bool open = real && v == v;                         // (an output that is no number is not chosen)
+    auto pick = [&](bool among, float& best, float& s) {
+        best = wave_max(among ? v : -INFINITY);
+        const unsigned long long have = __ballot(among && v == best);
+        const int at = have ? __builtin_amdgcn_readfirstlane(__ffsll(have) - 1) : experts - 1;      // (none: the last expert stands in)
+        s = have ? __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(score), at)) : 0.f;
+        return at;
+    };
+    if (r.group_size > 0) {
+        bool kept = false;
+        for (int j = 0; j < r.group_keep; ++j) {
+            float best, s;
+            const int g = pick(open && !kept, best, s) / r.group_size;
+            kept = kept || lane / r.group_size == g;
+        }
+        open = open && kept;
+    }
+    float first = 0.f, sum = 0.f, mine = 0.f;
+    int mine_at = 0;
+    for (int j = 0; j < r.top; ++j) {
+        float best, s;
+        const int at = pick(open, best, s);
+        if (lane == at) open = false;
+        if (j == 0) first = best;
+        const float p = mode != 0 ? s : expf(best - first);
+        sum += p;
+        if (lane == j) { mine_at = at; mine = p; }
+    }
+    if (lane < r.top) {
+        chosen[lane] = mine_at;
+        weights[lane] = (mode == 1 ? mine : mode == 2 ? mine / (sum + r.weight_eps) : mine / sum) * r.weight_scale;
+    }
+}
+
+__global__ void route_topk_kernel(const float* __restrict__ logits, RouteRule rule, int* __restrict__ chosen, float* __restrict__ weights, int tokens) {
+    const int t = blockIdx.x * (blockDim.x / TL_WAVE) + threadIdx.x / TL_WAVE;
+    if (t >= tokens) return;
+    if (rule.experts <= TL_WAVE) route_token_lanes(logits + (size_t)t * rule.experts, rule, chosen + (size_t)t * rule.top, weights + (size_t)t * rule.top);
+    else route_token(logits + (size_t)t * rule.experts, rule, chosen + (size_t)t * rule.top, weights + (size_t)t * rule.top);
 }
 
 // Sort of the (token, choice) pairs by expert, by one work-group: offsets[e] .. offsets[e + 1] - 1 are the slots of
-// expert e, slot_token[slot] the token a slot reads, pair_slot[token * top + j] where the pair's output row lies.
-__global__ void __launch_bounds__(1024)
-route_sort_kernel(const int* __restrict__ chosen, int pairs, int top, int experts, int* __restrict__ offsets,
-                  int* __restrict__ slot_token, int* __restrict__ pair_slot) {
-    extern __shared__ int cursor[];                     // [experts + 1]
+// expert e, slot_token[slot] the token a slot reads, pair_slot[token * top + j] where the pair's output row lies.  cursor: [experts + 1] in shared memory.
+__device__ __forceinline__ void route_sort(const int* chosen, int pairs, int top, int experts, int* cursor, int* __restrict__ offsets, int* __restrict__ slot_token,
+                                           int* __restrict__ pair_slot) {
     for (int e = threadIdx.x; e <= experts; e += blockDim.x) cursor[e] = 0;
     __syncthreads();
     for (int i = threadIdx.x; i < pairs; i += blockDim.x) atomicAdd(&cursor[chosen[i] + 1], 1);
     __syncthreads();
-    if (threadIdx.x == 0)
-        for (int e = 0; e < experts; ++e) cursor[e + 1] += cursor[e];
-    __syncthreads();
-    for (int e = threadIdx.x; e <= experts; e += blockDim.x) offsets[e] = cursor[e];
+    if (threadIdx.x < TL_WAVE) {                        // running sums, 64 experts at a time
+        int before = 0;
+        for (int base = 0; base < experts; base += TL_WAVE) {
+            const int e = base + (int)threadIdx.x;
+            int upto = e < experts ? cursor[e + 1] : 0;
+#pragma unroll
+            for (int o = 1; o < TL_WAVE; o <<= 1) {
+                const int t = __shfl_up(upto, o, TL_WAVE);
+                if ((int)threadIdx.x >= o) upto += t;
+            }
+            upto += before;
+            if (e < experts) {
+                cursor[e + 1] = upto;
+                offsets[e + 1] = upto;
+            }
+            before = __shfl(upto, TL_WAVE - 1, TL_WAVE);
+        }
+        if (threadIdx.x == 0) offsets[0] = 0;
+    }
     __syncthreads();
     for (int i = threadIdx.x; i < pairs; i += blockDim.x) {
         const int slot = atomicAdd(&cursor[chosen[i]], 1);
         slot_token[slot] = i / top;
         pair_slot[i] = slot;
     }
+}
+
+__global__ void __launch_bounds__(1024)
+route_sort_kernel(const int* __restrict__ chosen, int pairs, int top, int experts, int* __restrict__ offsets, int* __restrict__ slot_token, int* __restrict__ pair_slot) {
+    extern __shared__ int cursor[];                     // [experts + 1]
+    route_sort(chosen, pairs, top, experts, cursor, offsets, slot_token, pair_slot);
+}
+
+// Choice and sort of a decode step's tokens in one launch: a wave to a token, the choices stay in shared memory.  Both are chains of exchanges that hardly touch memory: what
+// counts is their length and the launches (us: two kernels, each exchange with value, score and index, a running sum by one thread / this; 8 tokens, 2 of 16 by their logits 5.2 / 3.0,
+// 2 of 18 by biased softmax 6.3 / 3.4, 4 of 32 by sigmoid 7.8 / 3.9, 2 of 16 in 4 groups 8.3 / 4.1).  Beyond 16 tokens the waves of one work-group would take turns: 32 tokens, 4 of 32
+// 6.3 in one launch, 5.8 (at 64 tokens) in two.
+#define ROUTE_FEW 16
+__global__ void __launch_bounds__(1024)
+route_few_kernel(const float* __restrict__ logits, RouteRule rule, float* __restrict__ weights, int tokens, int* __restrict__ offsets, int* __restrict__ slot_token,
+                 int* __restrict__ pair_slot) {
+    extern __shared__ int cursor[];                     // [experts + 1], then the choices [tokens * top]
+    int* chosen = cursor + rule.experts + 1;
+    const int t = threadIdx.x / TL_WAVE;                // (as many waves as tokens)
+    route_token_lanes(logits + (size_t)t * rule.experts, rule, chosen + t * rule.top, weights + (size_t)t * rule.top);
+    route_sort(chosen, tokens * rule.top, rule.top, rule.experts, cursor, offsets, slot_token, pair_slot);
 }
 
 extern "C" int tl_route(const void* logits, int tokens, int experts, int top, int mode, const void* bias, void* chosen, void* weights,
@@ -545,8 +640,14 @@ extern "C" int tl_route(const void* logits, int tokens, int experts, int top, in
     TL_REQUIRE(groups >= 0 && (groups == 0 || (experts % groups == 0 && groups_kept > 0 && groups_kept <= groups && top <= groups_kept * (experts / groups))),
                "route: %d of %d groups of %d experts do not hold %d choices", groups_kept, groups, experts, top);
     if (tokens == 0) return TL_OK;
-    route_topk_kernel<<<(tokens + 3) / 4, 4 * TL_WAVE, 0, stream>>>((const float*)logits, experts, top, mode, (const float*)bias, (int*)chosen, (float*)weights, tokens,
-                                                                    weight_scale, weight_eps, groups > 0 ? experts / groups : 0, groups_kept);
+    const RouteRule rule{experts, top, mode, (const float*)bias, weight_scale, weight_eps, groups > 0 ? experts / groups : 0, groups_kept};
+    if (tokens <= ROUTE_FEW && experts <= TL_WAVE) {
+        route_few_kernel<<<1, tokens * TL_WAVE, (experts + 1 + tokens * top) * sizeof(int), stream>>>((const float*)logits, rule, (float*)weights, tokens, (int*)offsets,
+                                                                                                  (int*)slot_token, (int*)pair_slot);
+        TL_CHECK_LAUNCH("route_few");
+        return TL_OK;
+    }
+    route_topk_kernel<<<(tokens + 3) / 4, 4 * TL_WAVE, 0, stream>>>((const float*)logits, rule, (int*)chosen, (float*)weights, tokens);
     TL_CHECK_LAUNCH("route_topk");
     route_sort_kernel<<<1, 1024, (experts + 1) * sizeof(int), stream>>>((const int*)chosen, tokens * top, top, experts, (int*)offsets,
                                                                        (int*)slot_token, (int*)pair_slot);
