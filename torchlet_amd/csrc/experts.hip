@@ -1,7 +1,7 @@
 // Matrix products over groups (one weight matrix per group: an expert and the tokens routed to it, or a head and
 // its slice of every token's row), the router's choice of experts, the sort of tokens by expert, the weighted sum
 // of the chosen experts' outputs, and the elementwise activation of a dense feed-forward.  Sums are float.
-#include "direct_tile.h"
+#include "row_ring.h"
 
 // ------------------------------------------------------------------ grouped product
 // out[row(m), g_out + n] = act(sum_k a[src(m), g_a + k] * w[g][n][k]) for the rows m of group g, in tiles of 64 x 64
@@ -198,7 +198,7 @@ grouped_gemm_mfma_kernel(const bf16_t* __restrict__ a, int a_ld, int a_group, co
 }
 
 // ------------------------------------------------------------------ products over the experts' rows (bfloat16, K a multiple of 64)
-// Two kernels beside the one above, which keeps the heads' products of many rows and what these refuse.
+// Three kernels beside the one above, which keeps the heads' products of many rows and what these refuse.
 //
 // Few rows per expert (a decode step): what counts is the stream of the weights, and a stream needs work-groups enough to have tens of KB on their
 // way from every compute unit.  A work-group owns a strip of 16 weight rows of one expert and up to 16 of its slots; its waves deal K out
@@ -214,18 +214,17 @@ struct HeadColumns {
     int gate_ld;
 };
 
-template <int FEW_WAVES, bool HEADS>
-__global__ void __launch_bounds__(FEW_WAVES * 64)
-experts_few_rows_kernel(const bf16_t* __restrict__ a, int a_ld, const int* __restrict__ src, const bf16_t* __restrict__ w, bf16_t* __restrict__ out,
-                        int out_ld, const int* __restrict__ offsets, int groups, int N, int K, int act, HeadColumns heads) {
-    __shared__ __attribute__((aligned(16))) float red[FEW_WAVES][256];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, kg = lane >> 4;
-    // this work-group's tile among the groups', found by a prefix sum over the lanes
-    int g = HEADS ? blockIdx.z : -1, m0 = HEADS ? blockIdx.y * 16 : 0, m_end = HEADS ? heads.rows : 0, first = 0;
-    for (int base = 0; !HEADS && base < groups && g < 0; base += TL_WAVE) {
+// This work-group's tile (blockIdx.y) among the groups' tiles of `height` rows, found by a prefix sum over the lanes: the group (-1: none), its tile's first row and the group's end.
+struct GroupTile {
+    int g, m0, m_end;
+};
+__device__ __forceinline__ GroupTile find_tile(const int* offsets, int groups, int height) {
+    const int lane = threadIdx.x & 63;
+    int first = 0;
+    for (int base = 0; base < groups; base += TL_WAVE) {
         const int e = base + lane;
         const int from = e < groups ? offsets[e] : 0, to = e < groups ? offsets[e + 1] : 0;
-        const int mine = (to - from + 15) / 16;
+        const int mine = (to - from + height - 1) / height;
         int upto = mine;
 #pragma unroll
         for (int o = 1; o < TL_WAVE; o <<= 1) {
@@ -235,13 +234,22 @@ experts_few_rows_kernel(const bf16_t* __restrict__ a, int a_ld, const int* __res
         const unsigned long long past = __ballot(first + upto > (int)blockIdx.y);
         if (past) {
             const int l = __builtin_amdgcn_readfirstlane(__ffsll(past) - 1);
-            g = base + l;
             const int before = first + __builtin_amdgcn_readlane(upto, l) - __builtin_amdgcn_readlane(mine, l);
-            m0 = __builtin_amdgcn_readlane(from, l) + ((int)blockIdx.y - before) * 16;
-            m_end = __builtin_amdgcn_readlane(to, l);
+            return GroupTile{base + l, __builtin_amdgcn_readlane(from, l) + ((int)blockIdx.y - before) * height, __builtin_amdgcn_readlane(to, l)};
         }
         first += __builtin_amdgcn_readlane(upto, TL_WAVE - 1);
     }
+    return GroupTile{-1, 0, 0};
+}
+
+template <int FEW_WAVES, bool HEADS>
+__global__ void __launch_bounds__(FEW_WAVES * 64)
+experts_few_rows_kernel(const bf16_t* __restrict__ a, int a_ld, const int* __restrict__ src, const bf16_t* __restrict__ w, bf16_t* __restrict__ out,
+                        int out_ld, const int* __restrict__ offsets, int groups, int N, int K, int act, HeadColumns heads) {
+    __shared__ __attribute__((aligned(16))) float red[FEW_WAVES][256];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, kg = lane >> 4;
+    const GroupTile tile = HEADS ? GroupTile{(int)blockIdx.z, (int)blockIdx.y * 16, heads.rows} : find_tile(offsets, groups, 16);
+    const int g = tile.g, m0 = tile.m0, m_end = tile.m_end;
     if (g < 0) return;
     const int n0 = blockIdx.x * 16;
     const bf16_t* wrow = w + ((size_t)g * N + min(n0 + li, N - 1)) * K + 16 * kg;
@@ -293,6 +301,47 @@ experts_few_rows_kernel(const bf16_t* __restrict__ a, int a_ld, const int* __res
     }
 }
 
+// Few rows per expert through rings in shared memory (see row_ring.h): a work-group owns rps weight rows of one expert (8 WJ at most) and 8 XH of its slots.
+template <int WJ, int XH>
+__global__ void __launch_bounds__(256)
+experts_ring_kernel(const bf16_t* __restrict__ a, int a_ld, const int* __restrict__ src, const bf16_t* __restrict__ w, bf16_t* __restrict__ out, int out_ld,
+                    const int* __restrict__ offsets, int groups, int N, int K, int act, int rps) {
+    using S = RingShape<WJ, XH>;
+    extern __shared__ __attribute__((aligned(16))) char ring[];
+    const GroupTile tile = find_tile(offsets, groups, 8 * XH);
+    if (tile.g < 0) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 15, kg = lane >> 4;
+    const int n0 = blockIdx.x * rps, n_end = min(N, n0 + rps);
+    unsigned woff[WJ], xoff[XH];
+#pragma unroll
+    for (int j = 0; j < XH; ++j) {
+        const int r = 8 * (WJ + j) + lane / 8, c = (lane % 8) ^ ((r >> 1) & 7), slot = min(tile.m0 + r - 8 * WJ, tile.m_end - 1);
+        xoff[j] = (unsigned)((src ? src[slot] : slot) * a_ld + c * 8) * 2;
+    }
+#pragma unroll
+    for (int j = 0; j < WJ; ++j) {
+        const int r = 8 * j + lane / 8, c = (lane % 8) ^ ((r >> 1) & 7);
+        woff[j] = (unsigned)((min(n0 + r, n_end - 1) - n0) * K + c * 8) * 2;
+    }
+    ring_products<WJ, XH, 1>(w + ((size_t)tile.g * N + n0) * K, woff, a, xoff, K / 64, ring, wave, K % 2048 == 0);
+    const int base_act = act & ~ACT_PAIRS;
+    for (int q = wave; q < S::SH * S::MT; q += S::NW) {
+        const int s = q / S::MT, t = q % S::MT, m = tile.m0 + 16 * t + li, n = n0 + 16 * s + 4 * kg;
+        const f32x4_t sum = ring_sum<WJ, XH, 1>(ring, s, t);
+        if (16 * t + li >= 8 * XH || m >= tile.m_end) continue;
+        bf16_t* orow = out + (size_t)m * out_ld;
+        if (act & ACT_PAIRS) {
+#pragma unroll
+            for (int v = 0; v < 4; v += 2)
+                if (n + v + 1 < n_end) orow[(n + v) / 2] = from_float<bf16_t>(activate(sum[v], base_act) * sum[v + 1]);
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if (n + v < n_end) orow[n + v] = from_float<bf16_t>(activate(sum[v], base_act));
+        }
+    }
+}
+
 // Many rows per expert (a prompt): the tile kernel with operands fetched straight into shared memory, over groups of rows.
 static int experts_units = 256;       // compute units the tiles are dealt to
 extern "C" void tl_experts_set_compute_units(int units) { if (units > 0) experts_units = units; }
@@ -308,10 +357,21 @@ struct ExpertsCall {
     int groups, rows, x_rows, N, K, act;      // rows: of out; x_rows: of a
 };
 
-template <int WAVES>
 static int launch_experts_few(const ExpertsCall& c, hipStream_t stream) {
     const dim3 grid((c.N + 15) / 16, c.rows / 16 + (c.groups < c.rows ? c.groups : c.rows));
-    experts_few_rows_kernel<WAVES, false><<<grid, WAVES * 64, 0, stream>>>(c.a, c.a_ld, c.src, c.w, c.out, c.out_ld, c.offsets, c.groups, c.N, c.K, c.act, HeadColumns{});
+    experts_few_rows_kernel<4, false><<<grid, 4 * 64, 0, stream>>>(c.a, c.a_ld, c.src, c.w, c.out, c.out_ld, c.offsets, c.groups, c.N, c.K, c.act, HeadColumns{});
+    return TL_OK;
+}
+
+template <int WJ, int XH>
+static int launch_experts_ring(const ExpertsCall& c, hipStream_t stream) {
+    using S = RingShape<WJ, XH>;
+    constexpr int rows = 8 * WJ;
+    auto kernel = experts_ring_kernel<WJ, XH>;
+    static hipError_t allowed = allow_lds(kernel, S::LDS);
+    TL_REQUIRE(allowed == hipSuccess, "experts_ring: cannot get %zu bytes of shared memory", S::LDS);
+    const dim3 grid((c.N + rows - 1) / rows, c.rows / (8 * XH) + (c.groups < c.rows ? c.groups : c.rows));
+    kernel<<<grid, 256, S::LDS, stream>>>(c.a, c.a_ld, c.src, c.w, c.out, c.out_ld, c.offsets, c.groups, c.N, c.K, c.act, rows);
     return TL_OK;
 }
 
@@ -335,13 +395,14 @@ static int launch_experts_tile(const ExpertsCall& c, hipStream_t stream) {
     return c.act & ACT_PAIRS ? launch_experts_tile_t<BM, BN, WGM, WGN, STAGES, true>(c, stream) : launch_experts_tile_t<BM, BN, WGM, WGN, STAGES, false>(c, stream);
 }
 
-enum ExpertsKernel { EX_FEW_8, EX_FEW_4, EX_TILE_64x128, EX_TILE_128x128, EX_TILE_128x256, EX_TILE_256x256, EX_KERNELS };
+enum ExpertsKernel { EX_RING_8, EX_FEW_4, EX_TILE_64x128, EX_TILE_128x128, EX_TILE_128x256, EX_TILE_256x256, EX_RING_16, EX_KERNELS };
 
 static int launch_experts(int which, const ExpertsCall& c, hipStream_t stream) {
     int rc = TL_OK;
     switch (which) {
-    case EX_FEW_8: rc = launch_experts_few<8>(c, stream); break;
-    case EX_FEW_4: rc = launch_experts_few<4>(c, stream); break;
+    case EX_RING_8: rc = launch_experts_ring<2, 1>(c, stream); break;
+    case EX_RING_16: rc = launch_experts_ring<4, 2>(c, stream); break;
+    case EX_FEW_4: rc = launch_experts_few(c, stream); break;
     case EX_TILE_64x128: rc = launch_experts_tile<64, 128, 1, 2, 3>(c, stream); break;
     case EX_TILE_128x128: rc = launch_experts_tile<128, 128, 2, 2, 2>(c, stream); break;
     case EX_TILE_128x256: rc = launch_experts_tile<128, 256, 2, 4, 3>(c, stream); break;
@@ -355,13 +416,13 @@ static int launch_experts(int which, const ExpertsCall& c, hipStream_t stream) {
 
 // Which kernel a call gets, by what the host knows: the slots of all groups together (how they are dealt to the groups only the GPU knows).
 //
-// Up to 8 slots a group on average (4 where K is beyond 2048: a strip's rows of x, read once per strip, outgrow the caches) the weights' stream
-// sets the time: the few-rows kernel, with waves enough to leave each a few steps of K.  Measured (us; few rows with 8 waves / with 4 / the
-// tiles of 64 x 128; groups x N x K, every call on other weights):
-//   16 x 1024 x 2048, 16 slots 13.9 / 14.9 / 20.4, 128 slots 19.7 / 21.7 / 21.6, 256 slots 25.6 / 24.6 / 21.6
-//   16 x 2048 x 1024, 16 slots 16.9 / 11.8 / 14.6, 64 slots 25.3 / 15.2 / 15.9, 128 slots 30.0 / 17.9 / 15.9, 256 slots 42.6 / 25.0 / 16.1
-//   32 x 4096 x 4096, 16 slots 68 / 73 / 74, 128 slots 183 / 190 / 176, 256 slots 210 / 212 / 178 (229 us at the rate of a large copy)
-// (the kernel without shared memory, which had these calls, took 37 us for the first and 134 at 4096 slots, where the tiles take 37).
+// Up to 12 slots a group on average (8 with K below 2048, where a wave has few slabs to keep on their way) the weights' stream sets the time: the rings, 16 weight rows and 8 slots a
+// work-group up to 4 slots a group, 32 rows and 16 slots beyond; below 2048 columns of K and up to 4 slots a group the few-rows kernel, which has all its requests out at once.
+// Measured (us; few rows with 8 waves / with 4 / rings of 16 rows and 8 slots / of 32 and 16 / tiles of 64 x 128; groups x N x K, every call on other weights):
+//   16 x 2048 x 2048, 16 slots 19.8 / 21.8 / 18.5 / 18.6 / 28.4, 64 slots 28.1 / 30.8 / 24.4 / 25.4 / 37.2, 256 slots 44.0 / 44.0 / 38.5 / 29.2 / 37.0
+//   16 x 2048 x 1024, 16 slots 18.1 / 11.1 / 12.1 / 11.4 / 14.1, 64 slots 26.5 / 15.3 / 16.1 / 15.3 / 16.0, 128 slots 28.6 / 17.4 / 18.1 / 15.7 / 16.2, 256 slots 41.9 / 23.5 / 27.0 / 18.9 / 16.6
+//   32 x 4096 x 4096, 16 slots 76 / 81 / 75 / 81 / 83, 128 slots 181 / 187 / 170 / 175 / 180, 256 slots 209 / 211 / 194 / 176 / 181, 512 slots - / 308 / 262 / 197 / 182
+//   32 x 4096 x 2048, 16 slots 43 / 43 / 39 / 41 / 55, 256 slots 113 / 115 / 104 / 90 / 119
 //
 // Beyond that, tiles: rounds of work-groups (two of the two smaller tiles to a compute unit) times a tile's time, fitted to single rounds at K of
 // 1024 and 2048; every group ends in a tile that is half empty on average.  The figures were fitted to tiles of 32 x 32 x 16 products and hold for today's: over 37 sizes of 16 to 16384
@@ -370,7 +431,7 @@ static int launch_experts(int which, const ExpertsCall& c, hipStream_t stream) {
 //   16 x 2048 x 1024, 2048 slots 31 / 26 / 22 / 29, 4096 slots 45 / 44 / 39 / 32, 16384 slots 143 / 108 / 96 / 92
 //   32 x 4096 x 4096, 2048 slots 228 / 190 / 190 / 250, 16384 slots 830 / 680 / 587 / 613
 static int pick_experts(const ExpertsCall& c) {
-    if ((long)c.rows <= (c.K > 2048 ? 4L : 8L) * c.groups) return c.K < 2048 ? EX_FEW_4 : EX_FEW_8;
+    if ((long)c.rows <= (c.K < 2048 ? 8L : 12L) * c.groups) return (long)c.rows > 4L * c.groups ? EX_RING_16 : c.K < 2048 ? EX_FEW_4 : EX_RING_8;
     static const struct { int kernel, bm, bn, per_unit; double fixed, per_k; } tiles[] = {
         {EX_TILE_64x128, 64, 128, 2, 9e-6, 6.5e-6}, {EX_TILE_128x128, 128, 128, 2, 7e-6, 13e-6},
         {EX_TILE_128x256, 128, 256, 1, 8e-6, 10.2e-6}, {EX_TILE_256x256, 256, 256, 1, 9e-6, 20e-6}};       // seconds of a tile: fixed, and per 1024 columns of K

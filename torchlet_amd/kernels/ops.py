@@ -1823,7 +1823,8 @@ def experts_linear(x: torch.Tensor, slot_token: torch.Tensor | None, weight: tor
 
 def experts_linear_variant(x: torch.Tensor, slot_token: torch.Tensor | None, weight: torch.Tensor, offsets: torch.Tensor, out: torch.Tensor,
                            activation: str, which: int) -> None:
-    """:func:`experts_linear` with the kernel named (0, 1: few rows with 8 or 4 waves; 2 to 5: tiles of 64 x 128, 128 x 128, 128 x 256, 256 x 256),
+    """:func:`experts_linear` with the kernel named (0: rings of 16 weight rows and 8 slots; 1: few rows; 2 to 5: tiles of 64 x 128, 128 x 128, 128 x 256, 256 x 256; 6: rings of
+    32 weight rows and 16 slots),
     for tests and tuning: bfloat16, K a multiple of 64."""
     G, N, K = weight.shape
     S, pairs = out.shape[0], ACTIVATIONS[activation] >= 16
