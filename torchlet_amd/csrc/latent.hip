@@ -87,6 +87,85 @@ __global__ void latent_prepare_kernel(const T* __restrict__ down, int ld, int q_
     for (int i = threadIdx.x; i < steps; i += blockDim.x) turn_part(kr, dst + rank)(i);
 }
 
+// The same for fewer than 512 tokens, with a work-group for each thing that there is to do (`roles`: bit 0 the page row, bit 1 the query latent, bit 2 the queries' rotated parts; blockIdx.y
+// counts those that are set), so that a decode step waits for one of them and not for all in turn.  Each asks for its numbers and its norm's weights before it uses the first.
+// (us, all in turn / this: one token, a query latent of 1536 5.4 / 3.3, of 768 4.7 / 3.3, 16 heads' rotated parts 3.8 / 3.3; 511 tokens 6.4 / 4.5, 5.5 / 4.1, 4.7 / 4.1.  Of more tokens
+// the chip holds no more work-groups at once: 2048 tokens 9.9 / 11.4.)
+template <typename T>
+__global__ void __launch_bounds__(256)
+latent_prepare_few_kernel(const T* __restrict__ down, int ld, int q_rank, int kv_off, int rank, int rot, int rot_dims,
+                          const void* __restrict__ wq, int wq_f32, const void* __restrict__ wkv, int wkv_f32, float eps,
+                          const int* __restrict__ positions, const float* __restrict__ inv_freq,
+                          const int* __restrict__ token_req, const int* __restrict__ block_table, int bt_stride,
+                          T* __restrict__ plane, int page_size, T* __restrict__ cq, int halves, T* __restrict__ rows, QueryParts parts, int roles) {
+    __shared__ float red[16];
+    __shared__ float cs[LAT_MAX_PAIRS], sn[LAT_MAX_PAIRS];      // the token's angles, by which all heads turn
+    constexpr int KEEP = 8;                                     // numbers of a row that a thread keeps; a longer row's others are read again
+    const int t = blockIdx.x, half = rot_dims / 2, steps = rot - half;      // (steps: pairs, then single numbers)
+    const T* row = down + (size_t)t * ld;
+    // number j of a rotated part: its partner lies as far on as the pair is wide
+    auto turn_part = [&](const T* src, T* dst, int j, float c, float sine) {
+        if (j < half) {
+            const int a = halves ? j : 2 * j, b = halves ? j + half : 2 * j + 1;
+            const float u = to_float(src[a]), v = to_float(src[b]);
+            dst[a] = from_float<T>(u * c - v * sine);
+            dst[b] = from_float<T>(v * c + u * sine);
+        } else {
+            dst[half + j] = src[half + j];                      // (what lies beyond the rotated dimensions passes)
+        }
+    };
+    auto work = [&](int role) {
+        if (role == 2) {
+            for (int i = threadIdx.x; i < half; i += 256) sincosf((float)positions[t] * inv_freq[i], &sn[i], &cs[i]);
+            __syncthreads();
+            for (int i = threadIdx.x; i < parts.heads * steps; i += 256) {
+                const int h = i / steps, j = i % steps;
+                turn_part(row + (size_t)h * parts.head + parts.plain, rows + (size_t)t * parts.rows_ld + (size_t)h * (rank + rot) + rank, j, j < half ? cs[j] : 0.f, j < half ? sn[j] : 0.f);
+            }
+            return;
+        }
+        const T* src = role == 0 ? row + kv_off : row;
+        const void* w = role == 0 ? wkv : wq;
+        const int n = role == 0 ? rank : q_rank, w_f32 = role == 0 ? wkv_f32 : wq_f32;
+        float x[KEEP], wx[KEEP];
+#pragma unroll
+        for (int j = 0; j < KEEP; ++j) {
+            const int i = threadIdx.x + 256 * j;
+            x[j] = i < n ? to_float(src[i]) : 0.f;
+            wx[j] = i < n ? load_vec(w, w_f32, i) : 0.f;
+        }
+        T* dst = cq + (size_t)t * q_rank;
+        if (role == 0) {
+            const int pos = positions[t], page = block_table[(size_t)token_req[t] * bt_stride + pos / page_size];
+            if (page == 0) return;                                  // (the whole work-group)
+            dst = plane + ((size_t)page * page_size + pos % page_size) * (rank + rot);
+            for (int i = threadIdx.x; i < steps; i += 256) {
+                float c = 0.f, sine = 0.f;
+                if (i < half) sincosf((float)pos * inv_freq[i], &sine, &c);
+                turn_part(src + rank, dst + rank, i, c, sine);
+            }
+        }
+        float ss = 0.f;
+#pragma unroll
+        for (int j = 0; j < KEEP; ++j) ss = fmaf(x[j], x[j], ss);
+        for (int i = threadIdx.x + 256 * KEEP; i < n; i += 256) { const float v = to_float(src[i]); ss = fmaf(v, v, ss); }
+        ss = block_sum(ss, red);
+        const float inv = 1.f / sqrtf(ss / (float)n + eps);
+#pragma unroll
+        for (int j = 0; j < KEEP; ++j) {
+            const int i = threadIdx.x + 256 * j;
+            if (i < n) dst[i] = from_float<T>(x[j] * inv * wx[j]);
+        }
+        for (int i = threadIdx.x + 256 * KEEP; i < n; i += 256) dst[i] = from_float<T>(to_float(src[i]) * inv * load_vec(w, w_f32, i));
+    };
+    int next = blockIdx.y;
+    for (int role = 0; role < 3; ++role) {
+        if (!((roles >> role) & 1)) continue;
+        if (next == 0) work(role);
+        --next;
+    }
+}
+
 extern "C" int tl_latent_prepare(const void* down, int ld, int q_rank, int kv_off, int rank, int rot, int rot_dims, const void* wq, int wq_f32,
                                  const void* wkv, int wkv_f32, float eps, const void* positions, const void* inv_freq,
                                  const void* token_req, const void* block_table, int bt_stride, void* plane, int page_size,
@@ -100,12 +179,19 @@ extern "C" int tl_latent_prepare(const void* down, int ld, int q_rank, int kv_of
     TL_REQUIRE(q_rank == 0 || (wq && cq), "latent_prepare: a query latent needs its norm's weight and a place to go");
     TL_REQUIRE(plane == nullptr || (page_size > 0 && block_table != nullptr && token_req != nullptr), "latent_prepare: a cache write needs the block table");
     if (tokens == 0) return TL_OK;
-    dim3 grid(tokens), block(256);
+    const int roles = (plane ? 1 : 0) | (q_rank > 0 ? 2 : 0) | (rows ? 4 : 0);
+    if (roles == 0) return TL_OK;
+    const bool few = tokens < 512;
+    dim3 grid(tokens, few ? (roles & 1) + (roles >> 1 & 1) + (roles >> 2) : 1), block(256);
 #define TL_ARGS(T) (const T*)down, ld, q_rank, kv_off, rank, rot, rot_dims, wq, wq_f32, wkv, wkv_f32, eps, (const int*)positions, (const float*)inv_freq, \
                    (const int*)token_req, (const int*)block_table, bt_stride, (T*)plane, page_size, (T*)cq, halves, (T*)rows, QueryParts{q_heads, q_head, q_plain, rows_ld}
-    if (dtype == TL_DT_F32) latent_prepare_kernel<float><<<grid, block, 0, stream>>>(TL_ARGS(float));
-    else if (dtype == TL_DT_BF16) latent_prepare_kernel<bf16_t><<<grid, block, 0, stream>>>(TL_ARGS(bf16_t));
+#define TL_PREPARE(T)                                                                            \
+    if (few) latent_prepare_few_kernel<T><<<grid, block, 0, stream>>>(TL_ARGS(T), roles);        \
+    else latent_prepare_kernel<T><<<grid, block, 0, stream>>>(TL_ARGS(T))
+    if (dtype == TL_DT_F32) { TL_PREPARE(float); }
+    else if (dtype == TL_DT_BF16) { TL_PREPARE(bf16_t); }
     else TL_REQUIRE(false, "latent_prepare: unknown dtype %d", dtype);
+#undef TL_PREPARE
 #undef TL_ARGS
     TL_CHECK_LAUNCH("latent_prepare");
     return TL_OK;
