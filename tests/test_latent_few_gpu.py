@@ -1,4 +1,4 @@
-"""The latents' norms, rotation and cache write on both sides of 512 tokens (below: a work-group for each of them), against plain 64-bit formulas."""
+"""The latents' norms, rotation and cache write on both sides of 512 tokens (below: a work-group for each of them) and the merge of a decoded token's parts, against plain 64-bit formulas."""
 from __future__ import annotations
 
 import pytest
@@ -48,3 +48,27 @@ def test_prepare_on_both_sides_of_the_line(tokens, q_rank, rank, rot, dims, head
         got = rows[:, h * (rank + rot): (h + 1) * (rank + rot)].cpu().double()
         torch.testing.assert_close(got[:, rank:], turned(x[:, h * head + plain: h * head + plain + rot]), **tol)
         assert bool((got[:, :rank] == 7.0).all())
+
+
+@pytest.mark.parametrize("vdim", [64, 128])
+@pytest.mark.parametrize("splits", [2, 3, 9, 32])
+def test_merge_of_a_decoded_tokens_parts(vdim, splits, monkeypatch):
+    from torchlet_amd.kernels import ops
+    heads, kv, dim, page, ctx, scale = 4, 1, 64, 8, [600, 0, 75], 0.1
+    monkeypatch.setattr(ops, "local_decode_splits", lambda *a: splits)
+    g = torch.Generator().manual_seed(vdim + splits)
+    bl = 80
+    k, v = (torch.randn(1 + 3 * bl, kv, page, n, generator=g).bfloat16() for n in (dim, vdim))
+    table = (1 + torch.randperm(3 * bl, generator=g)).int().view(3, bl)
+    q = torch.randn(3, heads * dim, generator=g).bfloat16()
+    sink = torch.linspace(-1, 5, heads)
+    out = torch.empty(3, heads * vdim, dtype=torch.bfloat16, device="cuda")
+    i32 = lambda t: torch.tensor(t, dtype=torch.int32, device="cuda")
+    tiles = (i32([0, 1, 2, 3]), i32(ctx), i32([0, 1, 2]), i32([0, 0, 0]), 3)
+    ops.local_attention(q.cuda(), out, k.cuda(), v.transpose(2, 3).contiguous().cuda(), table.cuda(), i32([0, 1, 2]), i32(ctx), heads, kv, dim, vdim, page, scale, tiles=tiles, sink=sink.cuda())
+    for r in range(3):
+        keys, values = (p[table[r].long()][:, 0].reshape(bl * page, -1)[: ctx[r] + 1].double() for p in (k, v))
+        s = q[r].double().view(heads, dim) @ keys.T * scale
+        w = torch.exp(s - torch.cat((s, sink.double()[:, None]), 1).logsumexp(1, keepdim=True))
+        bound = 2.0 ** -7 * (w @ values.abs()) + 1e-4          # (as above)
+        assert bool(((out[r].cpu().double().view(heads, vdim) - w @ values).abs() <= bound).all())

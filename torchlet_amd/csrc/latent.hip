@@ -443,17 +443,28 @@ latent_attention_kernel(const T* __restrict__ q, int q_ld, T* __restrict__ out, 
     }
 }
 
-// out[row] = sum_s exp(m_s - M) acc_s / sum_s exp(m_s - M) l_s over the parts of a row, in the order of the parts.
-// The parts' weights are worked out once per row (by the first wave, a part a lane, into shared memory), then every thread sums its
-// columns, VEC neighbours of one part to a load (four where rank is a multiple of four), eight parts requested before the first is added: the trips to memory are
-// what it costs (one token's heads, 512 numbers each in 62 parts, 22.3 -> 8.6 us).
+// out[row] = sum_s exp(m_s - M) acc_s / sum_s exp(m_s - M) l_s over the parts of a row, in a fixed order: four runs of neighbouring parts, each in the order of its parts.
+// A work-group owns 32 pieces of a row, VEC neighbouring numbers each (four where rank is a multiple of four); a quarter of its threads takes a run of parts.  One trip to
+// memory is what it costs: every thread asks for all its parts (16 at most) before the parts' weights are worked out, by the first wave, a part a lane.  (A work-group to a
+// row, eight parts requested at a time behind the weights: one token's heads, 512 numbers each in 62 parts, with the attention 30.5 us, so 24.5.)
 #define LAT_MAX_SPLITS 64
+#define LAT_MERGE_COLS 32
 template <typename T, int VEC>
-__global__ void latent_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml, T* __restrict__ out,
-                                    int rows, int rank, int splits, const T* __restrict__ gate, int gate_ld, int heads) {
+__global__ void __launch_bounds__(4 * LAT_MERGE_COLS)
+latent_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml, T* __restrict__ out,
+                    int rows, int rank, int splits, const T* __restrict__ gate, int gate_ld, int heads) {
+    constexpr int RUN = LAT_MAX_SPLITS / 4;
+    struct __attribute__((aligned(4 * VEC))) Piece { float v[VEC]; };
     __shared__ float wgt[LAT_MAX_SPLITS];
     __shared__ float inv_s;
-    const int row = blockIdx.x;
+    __shared__ Piece sums[4][LAT_MERGE_COLS];
+    const int row = blockIdx.x, c = threadIdx.x % LAT_MERGE_COLS, run = threadIdx.x / LAT_MERGE_COLS;
+    const int col = (blockIdx.y * LAT_MERGE_COLS + c) * VEC, each = (splits + 3) / 4, s0 = run * each, s1 = min(splits, s0 + each);
+    const float* po = part_o + (size_t)row * splits * rank + min(col, rank - VEC);
+    Piece p[RUN];
+#pragma unroll
+    for (int u = 0; u < RUN; ++u)
+        if (u < each) p[u] = *(const Piece*)(po + (size_t)min(s0 + u, splits - 1) * rank);      // (beyond the run: fetched, not added)
     const float* ml = part_ml + (size_t)row * splits * 2;
     if (threadIdx.x < TL_WAVE) {
         const int s = threadIdx.x;
@@ -461,9 +472,7 @@ __global__ void latent_merge_kernel(const float* __restrict__ part_o, const floa
         const float M = wave_max(ms);
         const float w = (s < splits && ms != -INFINITY) ? expf(ms - M) : 0.f;
         if (s < splits) wgt[s] = w;
-        float den = 0.f;
-        for (int i = 0; i < splits; ++i)               // in the order of the parts
-            den += __shfl(w, i, TL_WAVE) * __shfl(ls, i, TL_WAVE);
+        const float den = wave_sum(w * ls);
         if (s == 0) {
             float inv0 = den > 0.f ? 1.f / den : 0.f;
             if (gate) inv0 *= 1.f / (1.f + expf(-to_float(gate[(size_t)(row / heads) * gate_ld + row % heads])));
@@ -471,36 +480,30 @@ __global__ void latent_merge_kernel(const float* __restrict__ part_o, const floa
         }
     }
     __syncthreads();
+    Piece a;
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) a.v[v] = 0.f;
+#pragma unroll
+    for (int u = 0; u < RUN; ++u)
+        if (s0 + u < s1) {
+#pragma unroll
+            for (int v = 0; v < VEC; ++v) a.v[v] = fmaf(wgt[s0 + u], p[u].v[v], a.v[v]);
+        }
+    sums[run][c] = a;
+    __syncthreads();
+    if (run > 0 || col >= rank) return;
     const float inv = inv_s;
-    const float* po = part_o + (size_t)row * splits * rank;
-    struct __attribute__((aligned(4 * VEC))) Piece { float v[VEC]; };
-    for (int c = threadIdx.x * VEC; c < rank; c += blockDim.x * VEC) {
-        float a[VEC] = {};
-        int s = 0;
-        for (; s + 8 <= splits; s += 8) {
-            Piece p[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) p[u] = *(const Piece*)(po + (size_t)(s + u) * rank + c);
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-#pragma unroll
-                for (int v = 0; v < VEC; ++v) a[v] = fmaf(wgt[s + u], p[u].v[v], a[v]);
-        }
-        for (; s < splits; ++s) {
-            const Piece p = *(const Piece*)(po + (size_t)s * rank + c);
-#pragma unroll
-            for (int v = 0; v < VEC; ++v) a[v] = fmaf(wgt[s], p.v[v], a[v]);
-        }
-#pragma unroll
-        for (int v = 0; v < VEC; ++v) out[(size_t)row * rank + c + v] = from_float<T>(a[v] * inv);
-    }
+    for (int v = 0; v < VEC; ++v) out[(size_t)row * rank + col + v] = from_float<T>((((a.v[v] + sums[1][c].v[v]) + sums[2][c].v[v]) + sums[3][c].v[v]) * inv);
 }
 
 template <typename T>
 static void launch_latent_merge(const void* part_o, const void* part_ml, void* out, int rows, int rank, int splits, const void* gate, int gate_ld, int heads,
                                 hipStream_t stream) {
-    auto kernel = rank % 4 == 0 && ((uintptr_t)part_o & 15) == 0 ? latent_merge_kernel<T, 4> : latent_merge_kernel<T, 1>;
-    kernel<<<rows, 128, 0, stream>>>((const float*)part_o, (const float*)part_ml, (T*)out, rows, rank, splits, (const T*)gate, gate_ld, heads);
+    const bool fours = rank % 4 == 0 && ((uintptr_t)part_o & 15) == 0;
+    auto kernel = fours ? latent_merge_kernel<T, 4> : latent_merge_kernel<T, 1>;
+    const int pieces = fours ? rank / 4 : rank;
+    kernel<<<dim3(rows, (pieces + LAT_MERGE_COLS - 1) / LAT_MERGE_COLS), 4 * LAT_MERGE_COLS, 0, stream>>>((const float*)part_o, (const float*)part_ml, (T*)out, rows, rank, splits, (const T*)gate, gate_ld, heads);
 }
 
 // ------------------------------------------------------------------ attention on the matrix cores (bfloat16)
