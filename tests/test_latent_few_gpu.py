@@ -1,4 +1,5 @@
-"""The latents' norms, rotation and cache write on both sides of 512 tokens (below: a work-group for each of them) and the merge of a decoded token's parts, against plain 64-bit formulas."""
+"""The latents' norms, rotation and cache write on both sides of 512 tokens (below: a work-group for each of them), the attention at the sizes that have kernels of their own (latents of
+512 numbers beside 64 or no rotated ones) and the merges of parts, against plain 64-bit formulas."""
 from __future__ import annotations
 
 import pytest
@@ -48,6 +49,37 @@ def test_prepare_on_both_sides_of_the_line(tokens, q_rank, rank, rot, dims, head
         got = rows[:, h * (rank + rot): (h + 1) * (rank + rot)].cpu().double()
         torch.testing.assert_close(got[:, rank:], turned(x[:, h * head + plain: h * head + plain + rot]), **tol)
         assert bool((got[:, :rank] == 7.0).all())
+
+
+@pytest.mark.parametrize("rot", [0, 32, 64])                    # (32: the kernel by sizes that come with the call)
+@pytest.mark.parametrize("tile_rows,new", [(16, 1), (32, 2), (64, 5)])
+@pytest.mark.parametrize("splits", [1, 2, 3, 63, 64])
+@pytest.mark.parametrize("sink,window", [(True, 0), (False, 45)])
+def test_attention_over_latents_of_512_numbers(rot, tile_rows, new, splits, sink, window):
+    from torchlet_amd.kernels import ops
+    g = torch.Generator().manual_seed(rot + splits)
+    heads, rank, page, ctx, scale = 16, 512, 8, [0, 31, 333], 0.05
+    D, bl = rank + rot, 44
+    plane = (torch.randn(1 + 3 * bl, 1, page, D, generator=g)).bfloat16()
+    table = (1 + torch.randperm(3 * bl, generator=g)).int().view(3, bl)
+    T, tq = 3 * new, ops.latent_tile_tokens(heads, tile_rows)
+    q = torch.randn(T, heads * D, generator=g).bfloat16()
+    sinks = torch.linspace(-2, 4, heads) if sink else None
+    tiles = [(r, t) for r in range(3) for t in range(0, new, tq)]
+    out = torch.empty(T, heads * rank, dtype=torch.bfloat16, device="cuda")
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    ops.latent_attention(q.cuda(), out, plane.cuda(), table.cuda(), i32([0, new, 2 * new, 3 * new]), i32(ctx), i32([r for r, _ in tiles]), i32([t for _, t in tiles]), len(tiles), tq, heads, rank, rot,
+                         page, scale, None if sinks is None else sinks.cuda(), splits, max_new_tokens=new, window=window)
+    for r in range(3):
+        for i in range(new):
+            n = ctx[r] + i + 1
+            keys = plane[table[r].long()].reshape(-1, D)[max(0, n - window) if window else 0: n].double()
+            s = q[r * new + i].double().view(heads, D) @ keys.T * scale
+            den = torch.cat((s, sinks.double()[:, None]), 1) if sink else s
+            w = torch.exp(s - den.logsumexp(1, keepdim=True))
+            # the weights go to the product in bfloat16 and the result is rounded once: 2^-8 (half a unit in the last of 8 binary places) each, of the sum of magnitudes
+            bound = 2.0 ** -7 * (w @ keys[:, :rank].abs()) + 1e-4
+            assert bool(((out[r * new + i].cpu().double().view(heads, rank) - w @ keys[:, :rank]).abs() <= bound).all())
 
 
 @pytest.mark.parametrize("vdim", [64, 128])

@@ -515,6 +515,9 @@ static void launch_latent_merge(const void* part_o, const void* part_ml, void* o
 // A work-group of four waves owns RB blocks of 16 rows (row = token x head of a chunk of up to 16 heads; RB = 4, 2 or 1
 // by how many rows a tile of the step can have) and 4 / RB waves share a block: each takes all of the block's scores
 // (the softmax's state is then the same in all of them, nothing is exchanged) and its own share of the latent's columns.
+// A wave has its SIMD to itself, so the vector instructions around the products are what a step costs.  Latents of 512 numbers beside 64 or no rotated ones have kernels of their own,
+// in which every piece of a row is known to be there: a step of 32 keys with one block 5.1 us by sizes that come with the call, 2.8 by known ones (one token, 16 heads: 64 keys
+// 15.4 / 10.8 us, 512 keys in 8 parts 18.3 / 13.9, 4000 keys in 62 parts 24.6 / 18.4).
 #define LM_KEYS 32                    // keys of a step
 #define LM_DC_MAX 20                  // 32-number pieces of a cache row (rows of up to 640 numbers)
 #define LM_LOG2E 1.4426950408889634f
@@ -528,16 +531,19 @@ union LmFrag {
     lm_bf16x8 v;
 };
 
-template <int RB>
+template <int RB, int RANK = 0, int ROT = 0>
 __global__ void __launch_bounds__(256)
 latent_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __restrict__ out, const bf16_t* __restrict__ plane,
                              const int* __restrict__ block_table, int bt_stride, const int* __restrict__ req_indptr,
                              const int* __restrict__ ctx_lens, const int* __restrict__ tile_req, const int* __restrict__ tile_tok0,
-                             int tile_tokens, int heads, int rank, int rot, int page_size, float scale, const float* __restrict__ sink,
+                             int tile_tokens, int heads, int any_rank, int any_rot, int page_size, float scale, const float* __restrict__ sink,
                              int splits, float* __restrict__ part_o, float* __restrict__ part_ml, int window, const bf16_t* __restrict__ gate,
                              int gate_ld) {
+    const int rank = RANK ? RANK : any_rank, rot = RANK ? ROT : any_rot;
+    constexpr int DC = RANK ? (RANK + ROT) / 32 : LM_DC_MAX, ROUNDS = RANK ? (RANK + ROT + 63) / 64 : LM_DC_MAX / 2;      // 32-number pieces of a row, and rounds of eight lanes' pieces
     constexpr int WPR = 4 / RB;                      // waves that share a block of rows
     constexpr int NT = 32 / WPR;                     // most blocks of 16 latent columns a wave sums (latents of up to 512 numbers)
+    constexpr bool WHOLE = RANK == 512;              // every wave has that many
     extern __shared__ __align__(16) unsigned char lm_smem[];
     const int D = rank + rot, dc = D / 32, ldk = D + 8, ldt = LM_KEYS + 4;
     bf16_t* sk = (bf16_t*)lm_smem;                   // [32 keys][D + 8]: rows as they lie in the cache
@@ -558,9 +564,9 @@ latent_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __r
     const int tok = first + tok0 + rt, qpos = ctx + tok0 + rt;
     const int qfirst = window > 0 ? max(0, qpos - window + 1) : 0;      // the first key this query reads
     const int tile_first = window > 0 ? max(0, ctx + tok0 - window + 1) : 0;      // ... and the first one any query of the tile reads
-    LmFrag qf[LM_DC_MAX];
+    LmFrag qf[DC];
 #pragma unroll
-    for (int c = 0; c < LM_DC_MAX; ++c)
+    for (int c = 0; c < DC; ++c)
         qf[c].u = (c < dc && row_ok) ? *(const uint4*)(q + (size_t)tok * q_ld + (size_t)rh * D + 32 * c + 8 * g) : make_uint4(0, 0, 0, 0);
     // blocks of 16 latent columns of this wave: t0 .. t0 + nt - 1 (the last wave of a block of rows may have fewer than the others, or none)
     const int t_each = (rank / 16 + WPR - 1) / WPR, t0 = share * t_each, nt = min(t_each, rank / 16 - t0);
@@ -589,25 +595,25 @@ latent_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __r
     __syncthreads();
     constexpr bool TWO = RB < 4;                     // steps requested ahead: two where the registers allow it
     const int stride = splits * LM_KEYS, ahead = TWO ? 2 * stride : stride;
-    uint4 stage0[LM_DC_MAX / 2], stage1[TWO ? LM_DC_MAX / 2 : 1];
+    uint4 stage0[ROUNDS], stage1[TWO ? ROUNDS : 1];
     // where this lane's pieces go in shared memory does not change from step to step
     bf16_t* const sk_mine = sk + kk * ldk + 8 * pg;
     uint32_t* const st_mine = (uint32_t*)(st + (8 * pg + (odd ? 4 : 0)) * ldt + (kk & ~1));
     const int page_shift = (page_size & (page_size - 1)) == 0 ? __ffs(page_size) - 1 : -1;
     // (every lane fetches, from a clamped place where its own lies beyond the keys or the row: a fetch under a condition
     // would be waited for on the spot; what must be zero is cleared when the pieces are written to shared memory)
-    auto request = [&](uint4 (&stage)[LM_DC_MAX / 2], int at) {
+    auto request = [&](uint4 (&stage)[ROUNDS], int at) {
         const int pos = max(min(at + kk, last), tile_first);
         const int blk = page_shift >= 0 ? pos >> page_shift : pos / page_size;
         const bf16_t* src = plane + ((size_t)tbl[blk] * page_size + (pos - blk * page_size)) * D;
 #pragma unroll
-        for (int i = 0; i < LM_DC_MAX / 2; ++i)
+        for (int i = 0; i < ROUNDS; ++i)
             if (i < rounds) stage[i] = *(const uint4*)(src + 8 * min(pg + 8 * i, pieces - 1));
     };
-    auto step = [&](uint4 (&stage)[LM_DC_MAX / 2], int k0) {
+    auto step = [&](uint4 (&stage)[ROUNDS], int k0) {
         shared_barrier();                             // the products of the step before have read shared memory
 #pragma unroll
-        for (int i = 0; i < LM_DC_MAX / 2; ++i) {
+        for (int i = 0; i < ROUNDS; ++i) {
             if (i < rounds) {
                 const int col = 64 * i + 8 * pg;
                 const uint4 x = (k0 + kk <= last && k0 + kk >= tile_first && col < D) ? stage[i] : make_uint4(0, 0, 0, 0);
@@ -643,7 +649,7 @@ latent_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __r
                 const bf16_t* krow0 = sk + (32 * j + li) * ldk + 8 * g;
                 const bf16_t* krow1 = krow0 + 16 * ldk;
 #pragma unroll
-                for (int c = 0; c < LM_DC_MAX; c += 2) {
+                for (int c = 0; c < DC; c += 2) {
                     if (c < dc) {
                         LmFrag k0f, k1f;
                         k0f.u = *(const uint4*)(krow0 + 32 * c);
@@ -651,12 +657,12 @@ latent_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __r
                         s00 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0f.v, qf[c].v, s00, 0, 0, 0);
                         s10 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1f.v, qf[c].v, s10, 0, 0, 0);
                     }
-                    if (c + 1 < dc) {
+                    if (c + 1 < DC && c + 1 < dc) {
                         LmFrag k0f, k1f;
                         k0f.u = *(const uint4*)(krow0 + 32 * (c + 1));
                         k1f.u = *(const uint4*)(krow1 + 32 * (c + 1));
-                        s01 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0f.v, qf[c + 1].v, s01, 0, 0, 0);
-                        s11 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1f.v, qf[c + 1].v, s11, 0, 0, 0);
+                        s01 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0f.v, qf[c + 1 < DC ? c + 1 : c].v, s01, 0, 0, 0);
+                        s11 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1f.v, qf[c + 1 < DC ? c + 1 : c].v, s11, 0, 0, 0);
                     }
                 }
                 s00 += s01;
@@ -686,15 +692,18 @@ latent_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __r
             }
             l = l * alpha + psum;
             m = m_new;
+            if (moved) {
+#pragma unroll
+                for (int t = 0; t < NT; ++t) acc[t] *= alpha;
+            }
             // ---- O^T += L^T P^T over this wave's share of the latent's columns
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                if (t < nt) {
+                if (WHOLE || t < nt) {
                     const bf16_t* lrow = st + (16 * (t0 + t) + li) * ldt + 32 * j + 4 * g;
                     LmFrag vf;
                     vf.h[0] = *(const uint2*)lrow;
                     vf.h[1] = *(const uint2*)(lrow + 16);
-                    if (moved) acc[t] *= alpha;
                     acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, pf.v, acc[t], 0, 0, 0);
                 }
             }
@@ -721,7 +730,7 @@ latent_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __r
         bf16_t* o = out + ((size_t)tok * heads + rh) * rank;
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            if (t < nt) {
+            if (WHOLE || t < nt) {
                 union { uint2 u; uint16_t e[4]; } pk;
 #pragma unroll
                 for (int v = 0; v < 4; ++v) pk.e[v] = from_float<bf16_t>(acc[t][v] * inv).bits;
@@ -733,7 +742,7 @@ latent_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __r
         float* o = part_o + prow * rank;
 #pragma unroll
         for (int t = 0; t < NT; ++t)
-            if (t < nt) *(lm_f32x4*)(o + 16 * (t0 + t) + 4 * g) = acc[t];
+            if (WHOLE || t < nt) *(lm_f32x4*)(o + 16 * (t0 + t) + 4 * g) = acc[t];
         if (share == 0 && g == 0) { part_ml[prow * 2] = m / LM_LOG2E; part_ml[prow * 2 + 1] = l; }       // the merge works in base e
     }
 }
@@ -748,14 +757,14 @@ static bool lm_fits(int rank, int rot, int q_ld, const void* q, const void* plan
            ((uintptr_t)q % 16) == 0 && ((uintptr_t)plane % 16) == 0 && lm_smem_bytes(rank, rot) <= 160 * 1024;
 }
 
-template <int RB>
+template <int RB, int RANK, int ROT>
 static int launch_lm(const void* q, int q_ld, void* out, const void* plane, const void* block_table, int bt_stride, const void* req_indptr,
                      const void* ctx_lens, const void* tile_req, const void* tile_tok0, int num_tiles, int tile_tokens, int heads, int rank,
                      int rot, int page_size, float scale, const void* sink, int splits, void* part_o, void* part_ml, int window, const void* gate,
                      int gate_ld, hipStream_t stream) {
     static size_t allowed = 48 * 1024;               // (per instance of the template)
     const size_t smem = lm_smem_bytes(rank, rot);
-    auto kernel = latent_attention_mfma_kernel<RB>;
+    auto kernel = latent_attention_mfma_kernel<RB, RANK, ROT>;
     if (smem > allowed) {
         if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
             tl_set_error("latent_attention: cannot get %zu bytes of shared memory", smem); return TL_ERR_HIP;
@@ -795,10 +804,12 @@ extern "C" int tl_latent_attention(const void* q, int q_ld, void* out, const voi
     if (dtype == TL_DT_BF16 && !general && lm_fits(rank, rot, q_ld, q, plane, bt_stride)) {
         TL_REQUIRE(tile_tokens * min(heads, 16) <= 64, "latent_attention: a tile of %d tokens and %d heads has more than 64 rows", tile_tokens, heads);
         int rc;
-#define TL_LM(RB) rc = launch_lm<RB>(q, q_ld, out, plane, block_table, bt_stride, req_indptr, ctx_lens, tile_req, tile_tok0, num_tiles, tile_tokens, \
+#define TL_LM_AS(RB, RANK, ROT) rc = launch_lm<RB, RANK, ROT>(q, q_ld, out, plane, block_table, bt_stride, req_indptr, ctx_lens, tile_req, tile_tok0, num_tiles, tile_tokens, \
                                      heads, rank, rot, page_size, scale, sink, splits, part_o, part_ml, window, gate, gate_ld, stream)
-        if (tile_rows <= 16) TL_LM(1); else if (tile_rows <= 32) TL_LM(2); else TL_LM(4);
+#define TL_LM(RB) if (rank == 512 && rot == 64) TL_LM_AS(RB, 512, 64); else if (rank == 512 && rot == 0) TL_LM_AS(RB, 512, 0); else TL_LM_AS(RB, 0, 0)
+        if (tile_rows <= 16) { TL_LM(1); } else if (tile_rows <= 32) { TL_LM(2); } else { TL_LM(4); }
 #undef TL_LM
+#undef TL_LM_AS
         if (rc != TL_OK) return rc;
         if (splits > 1) {
             const int rows = tokens * heads;
