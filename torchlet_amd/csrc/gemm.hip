@@ -7,6 +7,7 @@
 // product of the 32-bit path and the fallback of the bfloat16 path for shapes that
 // the matrix-core kernels refuse.  The sum over K runs in one fixed order for every
 // output element, whatever M is, so a row's result does not depend on the batch.
+#include "activation.h"
 #include "row_ring.h"
 
 // The compute units of the GPU the library runs on: the caller tells it once (tl_gemm_set_compute_units, from
@@ -1039,15 +1040,24 @@ static void pick_skinny(const void* x, const void* w, const void* bias, int bias
 
 // ------------------------------------------------------------------ few rows through rings in shared memory (K a multiple of 64)
 // See row_ring.h.  Work-group (i, y, z): outputs i * rps .. of product z (gs), or the y-th range of K of a product split over K (k_per_split columns each, a
-// slab [M, ldo] of partial sums each).  SW: the gate's activation as in gemm_skinny_kernel (out_cols outputs, gate and up rows interleaved in blocks of 32); RP: its rotation and
-// cache write.
-template <int WJ, int XH, typename TOut, int SW = 0, bool RP = false>
+// slab [M, ldo] of partial sums each).  SW: the gate's activation as in gemm_skinny_kernel (out_cols outputs, gate and up rows interleaved in blocks of 32); END: what becomes of the
+// sums: END_ROTATE its rotation and cache write, END_TOKEN an activation and the product with the row's token's own numbers (16 rows, 256 x 2048: 5.6 us in two launches, 4.4 in one).
+#define END_STORE 0
+#define END_ROTATE 1
+#define END_TOKEN 2
+struct TokenRow {
+    const int* ids;
+    const bf16_t* table;      // row ids[m] holds N numbers; rows ld apart; what is no row leaves its outputs as they are
+    int ld, vocab, act;
+};
+template <int WJ, int XH, typename TOut, int SW = 0, int END = END_STORE>
 __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const void* __restrict__ bias, int bias_f32,
                                                         TOut* __restrict__ out, int M, int N, int K, int ldx, int ldo, int out_cols, int k_per_split, int rps,
-                                                        RopeArgs ra, GroupStride gs) {
+                                                        RopeArgs ra, TokenRow tk, GroupStride gs) {
+    constexpr bool RP = END == END_ROTATE, TK = END == END_TOKEN;
     constexpr int HALVES = SW ? 2 : 1;
     using S = RingShape<WJ, XH, HALVES>;
-    static_assert(!RP || (!SW && S::MT == 1 && sizeof(TOut) == 2), "the rotation is built for up to 16 rows");
+    static_assert(END == END_STORE || (!SW && S::MT == 1 && sizeof(TOut) == 2), "the rotation and the tokens' rows are built for up to 16 rows");
     extern __shared__ __attribute__((aligned(16))) char ring[];
     const int ldw = K;
     x += blockIdx.z * gs.x;
@@ -1069,6 +1079,7 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict
         rp_pos = ra.positions[row];
         if (ra.k_plane) rp_page = ra.block_table[(size_t)ra.token_req[row] * ra.bt_stride + rp_pos / ra.page];
     }
+    const int tk_id = TK ? tk.ids[min(li, M - 1)] : 0;
     // the matrix's row of an output's gate (or of the output itself); its up row lies 32 further on
     auto row_of = [](int o) { return SW ? (o >> 5) * 64 + (o & 31) : o; };
     unsigned woff[WJ], xoff[XH];
@@ -1086,6 +1097,12 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict
     const bool quads = ldo % 4 == 0 && n0 % 4 == 0 && ((uintptr_t)out % (4 * sizeof(TOut))) == 0;
     for (int q = wave; q < S::SH * S::MT; q += S::NW) {
         const int s = q / S::MT, t = q % S::MT, m = 16 * t + li, n = n0 + 16 * s + 4 * kg;
+        const bool known = !TK || (tk_id >= 0 && tk_id < tk.vocab);
+        float own[4];
+        if constexpr (TK) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) own[v] = known ? to_float(tk.table[(size_t)tk_id * tk.ld + min(n + v, N - 1)]) : 0.f;
+        }
         f32x4_t sum = ring_sum<WJ, XH, HALVES>(ring, s, t);
         if constexpr (SW) {
             const f32x4_t up = ring_sum<WJ, XH, HALVES>(ring, S::SH + s, t);
@@ -1095,7 +1112,11 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict
 #pragma unroll
             for (int v = 0; v < 4; ++v) sum[v] += load_vec(bias, bias_f32, min(n + v, N - 1));
         }
-        if (m >= M) continue;
+        if (m >= M || !known) continue;
+        if constexpr (TK) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) sum[v] = activate(sum[v], tk.act) * own[v];
+        }
         if constexpr (RP) {
             rope_store(ra, sum, n, n_end, m, rp_pos, rp_page, (bf16_t*)out, ldo);
         } else if (quads && n + 3 < n_end) {
@@ -1126,45 +1147,46 @@ struct RingCall {
     int parts = 1, k_per = 0;
     Groups gr = Groups{};
     RopeArgs ra = RopeArgs{};
+    TokenRow tk = TokenRow{};
 };
 
-template <int WJ, int XH, typename TOut, int SW, bool RP>
+template <int WJ, int XH, typename TOut, int SW, int END>
 static int launch_ring_t(const RingCall& c, int rows, hipStream_t stream) {
     using S = RingShape<WJ, XH, SW ? 2 : 1>;
-    auto kernel = gemm_ring_kernel<WJ, XH, TOut, SW, RP>;
+    auto kernel = gemm_ring_kernel<WJ, XH, TOut, SW, END>;
     static hipError_t allowed = allow_lds(kernel, S::LDS);
     TL_REQUIRE(allowed == hipSuccess, "gemm_ring: cannot get %zu bytes of shared memory", S::LDS);
     const int total = SW ? c.out_cols : c.N;
     kernel<<<dim3((total + rows - 1) / rows, c.parts, c.gr.count), 256, S::LDS, stream>>>((const bf16_t*)c.x, (const bf16_t*)c.w, c.bias, c.bias_f32, (TOut*)c.out, c.M, c.N, c.K,
-                                                                                      c.ldx, c.ldo, c.out_cols, c.k_per, rows, c.ra, c.gr.stride);
+                                                                                      c.ldx, c.ldo, c.out_cols, c.k_per, rows, c.ra, c.tk, c.gr.stride);
     TL_CHECK_LAUNCH("gemm_ring");
     return TL_OK;
 }
 
-template <int XH, typename TOut, int SW, bool RP>
+template <int XH, typename TOut, int SW, int END>
 static int launch_ring_x(const RingCall& c, RingPlan p, hipStream_t stream) {
     switch (p.wj) {
-    case 2: return launch_ring_t<2, XH, TOut, SW, RP>(c, p.rows, stream);
-    case 4: return launch_ring_t<4, XH, TOut, SW, RP>(c, p.rows, stream);
-    case 6: return launch_ring_t<6, XH, TOut, SW, RP>(c, p.rows, stream);
-    case 8: return launch_ring_t<8, XH, TOut, SW, RP>(c, p.rows, stream);
+    case 2: return launch_ring_t<2, XH, TOut, SW, END>(c, p.rows, stream);
+    case 4: return launch_ring_t<4, XH, TOut, SW, END>(c, p.rows, stream);
+    case 6: return launch_ring_t<6, XH, TOut, SW, END>(c, p.rows, stream);
+    case 8: return launch_ring_t<8, XH, TOut, SW, END>(c, p.rows, stream);
     }
     if constexpr (!SW) {
-        if (p.wj == 1) return launch_ring_t<1, XH, TOut, SW, RP>(c, p.rows, stream);
-        if (p.wj == 3) return launch_ring_t<3, XH, TOut, SW, RP>(c, p.rows, stream);
+        if (p.wj == 1) return launch_ring_t<1, XH, TOut, SW, END>(c, p.rows, stream);
+        if (p.wj == 3) return launch_ring_t<3, XH, TOut, SW, END>(c, p.rows, stream);
     }
     TL_REQUIRE(false, "gemm_ring: no shape of %d requests", p.wj);
 }
 
 // `p.wj` 0: the plan is made here.
-template <typename TOut, int SW, bool RP>
+template <typename TOut, int SW, int END>
 static int launch_ring(const RingCall& c, hipStream_t stream, RingPlan p = RingPlan{0, 0}) {
-    if (p.wj == 0) p = plan_ring(SW ? c.out_cols : c.N, c.M, SW ? 2 : 1, TL_COMPUTE_UNITS / (c.parts * c.gr.count), RP);
-    if (c.M <= 8) return launch_ring_x<1, TOut, SW, RP>(c, p, stream);
-    if (c.M <= 16) return launch_ring_x<2, TOut, SW, RP>(c, p, stream);
-    if constexpr (!RP) {
-        if (c.M <= 32) return launch_ring_x<4, TOut, SW, RP>(c, p, stream);
-        return launch_ring_x<8, TOut, SW, RP>(c, p, stream);
+    if (p.wj == 0) p = plan_ring(SW ? c.out_cols : c.N, c.M, SW ? 2 : 1, TL_COMPUTE_UNITS / (c.parts * c.gr.count), END == END_ROTATE);
+    if (c.M <= 8) return launch_ring_x<1, TOut, SW, END>(c, p, stream);
+    if (c.M <= 16) return launch_ring_x<2, TOut, SW, END>(c, p, stream);
+    if constexpr (END == END_STORE) {
+        if (c.M <= 32) return launch_ring_x<4, TOut, SW, END>(c, p, stream);
+        return launch_ring_x<8, TOut, SW, END>(c, p, stream);
     }
     TL_REQUIRE(false, "gemm_ring: too many rows (%d)", c.M);
 }
@@ -1181,10 +1203,10 @@ extern "C" int tl_gemm_ring_variant(const void* x, const void* w, const void* bi
                "gemm_ring: %d ranges of %d columns are not a split of %d", parts, k_per, K);
     RingCall c{x, w, bias, bias_f32, out, M, N, K, ldx, ldo, gate ? total : 0, parts, parts > 1 ? k_per : 0};
     const RingPlan p{wj, rows};
-    if (gate == 1) return launch_ring<bf16_t, 1, false>(c, stream, p);
-    if (gate == 2) return launch_ring<bf16_t, 2, false>(c, stream, p);
-    if (gate == 3) return launch_ring<bf16_t, 3, false>(c, stream, p);
-    return out_f32 ? launch_ring<float, 0, false>(c, stream, p) : launch_ring<bf16_t, 0, false>(c, stream, p);
+    if (gate == 1) return launch_ring<bf16_t, 1, END_STORE>(c, stream, p);
+    if (gate == 2) return launch_ring<bf16_t, 2, END_STORE>(c, stream, p);
+    if (gate == 3) return launch_ring<bf16_t, 3, END_STORE>(c, stream, p);
+    return out_f32 ? launch_ring<float, 0, END_STORE>(c, stream, p) : launch_ring<bf16_t, 0, END_STORE>(c, stream, p);
 }
 
 // One named instance of the few-rows kernel, of those the dispatch below can pick (for tests and tuning);
@@ -1685,7 +1707,7 @@ extern "C" int tl_gemm(const void* x, const void* w, const void* bias, int bias_
     const bool aligned = K % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0;
     if (dtype == TL_DT_BF16 && ring_fits(x, w, M, K, ldx) && ring_pays(M, N)) {
         const RingCall c{x, w, bias, bias_f32, out, M, N, K, ldx, ldo, 0};
-        return out_f32 ? launch_ring<float, 0, false>(c, stream) : launch_ring<bf16_t, 0, false>(c, stream);
+        return out_f32 ? launch_ring<float, 0, END_STORE>(c, stream) : launch_ring<bf16_t, 0, END_STORE>(c, stream);
     }
     if (dtype == TL_DT_BF16 && aligned && K % 64 == 0 && M > 8) {
         int rc = out_f32 ? launch_dl_tile<float, false>(pick_dl_tile(M, N, K, false), x, w, bias, bias_f32, out, M, N, K, ldx, ldo, 0, stream)
@@ -1766,7 +1788,7 @@ extern "C" int tl_gemm_rope(const void* x, const void* w, const void* bias, int 
     if (rings) {
         RingCall c{x, w, bias, bias_f32, out, M, N, K, ldx, ldo, 0};
         c.ra = ra;
-        return launch_ring<bf16_t, 0, true>(c, stream);
+        return launch_ring<bf16_t, 0, END_ROTATE>(c, stream);
     }
     const bool xl = M > 1 && (size_t)M * (K + 8) * 2 <= SKINNY_XL_MAX_BYTES;
     int blocks = 1;
@@ -1792,6 +1814,19 @@ static NormArgs norm_args(const void* residual, void* residual_out, const void* 
     na.weight = weight; na.part_stride = (size_t)part_stride; na.parts = parts; na.weight_f32 = weight_f32; na.eps = eps;
     return na;
 }
+
+// out[m, n] = act((x w^T)[m, n]) * table[ids[m], n] of up to 16 rows in bfloat16, the product and what follows in float (a row whose id is no row of the table keeps what it
+// holds).  Returns TL_NOT_FUSED (nothing launched) for shapes it is not built for.
+extern "C" int tl_gemm_token_gate(const void* x, const void* w, const void* ids, const void* table, int table_ld, int vocab, void* out, int M, int N, int K, int ldx, int ldo, int act,
+                                  hipStream_t stream) {
+    TL_REQUIRE(M > 0 && N > 0 && K > 0 && ldx >= K && ldo >= N && table_ld >= N && vocab > 0 && ids && table, "gemm_token_gate: bad sizes M=%d N=%d K=%d", M, N, K);
+    TL_REQUIRE(known_activation(act) && !(act & ACT_PAIRS), "gemm_token_gate: unknown activation %d", act);
+    if (M > 16 || !ring_fits(x, w, M, K, ldx) || !ring_pays(M, N)) return TL_NOT_FUSED;
+    RingCall c{x, w, nullptr, 0, out, M, N, K, ldx, ldo, 0};
+    c.tk = TokenRow{(const int*)ids, (const bf16_t*)table, table_ld, vocab, act};
+    return launch_ring<bf16_t, 0, END_TOKEN>(c, stream);
+}
+
 
 // tl_gemm_rope for one row whose x is the norm of the residual stream, made inside the kernel (see NormArgs):
 // pending is bfloat16 [K] (parts == 0), float [parts][part_stride] or null.  Returns TL_NOT_FUSED (nothing
@@ -1868,7 +1903,7 @@ static int gemm_gated(const void* x, const void* w, void* out, int M, int I, int
     bf16_t* ob = (bf16_t*)out;
     // through the rings up to 16 rows, up to 64 against up to 24576 rows of the matrix (us, tiles / rings: 32 rows, 22528 x 4096 46 / 34, 27648 x 5120 51.1 / 51.3,
     // 37888 x 3584 49.9 / 52.3; 64 rows, 2048 x 2048 15.6 / 6.3, 22528 x 4096 47 / 43, 27648 x 5120 56 / 62)
-    if (ring_fits(x, w, M, K, ldx) && (M <= 16 || N <= 24576)) return launch_ring<bf16_t, GATE, false>(RingCall{x, w, nullptr, 0, out, M, N, K, ldx, ldo, I}, stream);
+    if (ring_fits(x, w, M, K, ldx) && (M <= 16 || N <= 24576)) return launch_ring<bf16_t, GATE, END_STORE>(RingCall{x, w, nullptr, 0, out, M, N, K, ldx, ldo, I}, stream);
     if (M <= 32 && K % 64 != 0) {
         if (M <= 16) launch_skinny_t<1, 1, 16, bf16_t, GATE>(xb, wb, nullptr, 0, ob, M, N, K, ldx, ldo, I, stream);
         else launch_skinny_t<1, 2, 16, bf16_t, GATE>(xb, wb, nullptr, 0, ob, M, N, K, ldx, ldo, I, stream);
@@ -1966,7 +2001,7 @@ extern "C" int tl_gemm_partials(const void* x, const void* w, void* out, int M, 
     // (the rings against the tiles, us: 16 rows, 2048 x 2048 4.4 / 3.5, 4096 x 8192 17.9 / 13.5, 3584 x 18944 26.8 / 24.4; 64 rows, 4096 x 8192 19.4 / 18.1, 3584 x 18944
     // 36.6 / 33.9, 4096 x 4096 11.1 / 11.4, 3584 x 3584 at 48 rows 9.4 / 9.9)
     if (partials_on_tiles(M, N, K) && ring_fits(x, w, M, K, ldx) && (M <= 32 || K >= 8192))
-        return launch_ring<float, 0, false>(RingCall{x, w, nullptr, 0, out, M, N, K, ldx, N, 0, P, k_per}, stream);
+        return launch_ring<float, 0, END_STORE>(RingCall{x, w, nullptr, 0, out, M, N, K, ldx, N, 0, P, k_per}, stream);
     if (partials_on_tiles(M, N, K)) {
         auto kernel = gemm_dl_tile_kernel<64, 64, 2, 2, 4, float, false>;
         constexpr size_t lds = (size_t)4 * 128 * 64 * sizeof(bf16_t);
@@ -2007,7 +2042,7 @@ extern "C" int tl_gemm_groups(const void* x, long x_group, const void* w, void* 
     if (dtype == TL_DT_BF16 && x_group % 8 == 0 && ring_fits(x, w, M, K, ldx) && ring_pays(M, (long)N * groups)) {
         RingCall c{x, w, nullptr, 0, out, M, N, K, ldx, ldo, 0};
         c.gr = gr;
-        return out_f32 ? launch_ring<float, 0, false>(c, stream) : launch_ring<bf16_t, 0, false>(c, stream);
+        return out_f32 ? launch_ring<float, 0, END_STORE>(c, stream) : launch_ring<bf16_t, 0, END_STORE>(c, stream);
     }
     if (dtype == TL_DT_BF16 && aligned && K % 64 == 0 && M > 8) {
         const DlTile tile = pick_dl_tile(M, N, K, false, groups);

@@ -1907,6 +1907,25 @@ def token_gate(z: torch.Tensor, token_ids: torch.Tensor, table: torch.Tensor, ou
                                   c_int(ACTIVATIONS[activation]), c_int(_dt(out, "token_gate")), _stream()))
 
 
+def linear_token_gate(x: torch.Tensor, weight: torch.Tensor, token_ids: torch.Tensor, table: torch.Tensor, out: torch.Tensor, activation: str = "gelu_tanh") -> None:
+    """``out[t] = act(weight @ x[t]) * table[token_ids[t]]``: :func:`linear` into 32-bit numbers and :func:`token_gate`, in one launch for up to 16 rows in bfloat16 where the
+    library has the shape."""
+    (M, K), N = x.shape, weight.shape[0]
+    if x.is_cuda and M <= 16 and x.dtype == weight.dtype == table.dtype == out.dtype == torch.bfloat16 and M > 0:
+        if weight.shape != (N, K) or out.shape != (M, N) or not out.is_contiguous() or not weight.is_contiguous() or x.stride(1) != 1 or table.dim() != 2 or table.shape[1] != N \
+                or table.stride(1) != 1 or ACTIVATIONS[activation] >= 16:
+            raise KernelError("linear_token_gate: shapes do not fit")
+        _i32(token_ids, "token_ids", M)
+        lib = _lib("gemm")
+        rc = lib.tl_gemm_token_gate(_ptr(x), _ptr(weight), _ptr(token_ids), _ptr(table), c_int(table.stride(0)), c_int(table.shape[0]), _ptr(out), c_int(M), c_int(N), c_int(K),
+                                    c_int(x.stride(0)), c_int(N), c_int(ACTIVATIONS[activation]), _stream())
+        if rc != 100:          # (100: not built for this shape)
+            return _check(lib, rc)
+    z = torch.empty((M, N), dtype=torch.float32, device=x.device)
+    linear(x, weight, None, z)
+    token_gate(z, token_ids, table, out, activation)
+
+
 def activation(x: torch.Tensor, kind: str) -> None:
     """The elementwise activation ``kind`` (``relu2``: the square of relu) on contiguous ``x``, in place."""
     if not x.is_contiguous():

@@ -46,8 +46,6 @@ class TokenSide(Part):
     def forward(self, x: torch.Tensor, ctx) -> torch.Tensor:
         """``x [T, hidden]`` -> ``y``: ``[T, hidden]``, or float32 slabs of partial sums ``[P, T, hidden]``."""
         T = x.shape[0]
-        z = torch.empty((T, self.dim), dtype=torch.float32, device=x.device)
-        ops.linear(x, self.w_gate, None, z)
         g = torch.empty((T, self.dim), dtype=self.dtype, device=x.device)
-        ops.token_gate(z, ctx.token_ids, self.table, g, self.spec.activation)
+        ops.linear_token_gate(x, self.w_gate, ctx.token_ids, self.table, g, self.spec.activation)
         return project_out(g, self.w_proj, self.dtype)
