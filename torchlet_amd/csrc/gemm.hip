@@ -1041,10 +1041,18 @@ static void pick_skinny(const void* x, const void* w, const void* bias, int bias
 // ------------------------------------------------------------------ few rows through rings in shared memory (K a multiple of 64)
 // See row_ring.h.  Work-group (i, y, z): outputs i * rps .. of product z (gs), or the y-th range of K of a product split over K (k_per_split columns each, a
 // slab [M, ldo] of partial sums each).  SW: the gate's activation as in gemm_skinny_kernel (out_cols outputs, gate and up rows interleaved in blocks of 32); END: what becomes of the
-// sums: END_ROTATE its rotation and cache write, END_TOKEN an activation and the product with the row's token's own numbers (16 rows, 256 x 2048: 5.6 us in two launches, 4.4 in one).
+// sums: END_ROTATE its rotation and cache write, END_TOKEN an activation and the product with the row's token's own numbers (16 rows, 256 x 2048: 5.6 us in two launches, 4.4 in one);
+// END_BESIDE: as END_STORE, and behind the products of gs comes one more (blockIdx.z == be.z), of other columns and into float, eight of them to a work-group: it shares its compute
+// unit with another one (16 rows, 4 x 2048 x 2048 and 64 x 2048: 12.9 us in two launches, 10.7 in one, 11.8 with as many columns to a work-group as the others have).
 #define END_STORE 0
 #define END_ROTATE 1
 #define END_TOKEN 2
+#define END_BESIDE 3
+struct Beside {
+    const bf16_t *x, *w;      // rows of x as far apart as the others'
+    float* out;               // [M, N]
+    int N, z;
+};
 struct TokenRow {
     const int* ids;
     const bf16_t* table;      // row ids[m] holds N numbers; rows ld apart; what is no row leaves its outputs as they are
@@ -1053,16 +1061,28 @@ struct TokenRow {
 template <int WJ, int XH, typename TOut, int SW = 0, int END = END_STORE>
 __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const void* __restrict__ bias, int bias_f32,
                                                         TOut* __restrict__ out, int M, int N, int K, int ldx, int ldo, int out_cols, int k_per_split, int rps,
-                                                        RopeArgs ra, TokenRow tk, GroupStride gs) {
-    constexpr bool RP = END == END_ROTATE, TK = END == END_TOKEN;
+                                                        RopeArgs ra, TokenRow tk, Beside be, GroupStride gs) {
+    constexpr bool RP = END == END_ROTATE, TK = END == END_TOKEN, BE = END == END_BESIDE;
     constexpr int HALVES = SW ? 2 : 1;
     using S = RingShape<WJ, XH, HALVES>;
-    static_assert(END == END_STORE || (!SW && S::MT == 1 && sizeof(TOut) == 2), "the rotation and the tokens' rows are built for up to 16 rows");
+    static_assert(END == END_STORE || END == END_BESIDE || (!SW && S::MT == 1 && sizeof(TOut) == 2), "the rotation and the tokens' rows are built for up to 16 rows");
     extern __shared__ __attribute__((aligned(16))) char ring[];
     const int ldw = K;
-    x += blockIdx.z * gs.x;
-    w += blockIdx.z * gs.w;
-    out += blockIdx.z * gs.out;
+    const bool beside = BE && (int)blockIdx.z == be.z;
+    if (BE) {
+        if (beside) {
+            x = be.x;
+            w = be.w;
+            N = be.N;
+            rps = min(rps, 8);
+        }
+        if ((int)blockIdx.x * rps >= N) return;        // (the whole work-group: the grid is as wide as the widest product)
+    }
+    if (!beside) {
+        x += blockIdx.z * gs.x;
+        w += blockIdx.z * gs.w;
+        out += blockIdx.z * gs.out;
+    }
     if (k_per_split > 0) {
         const int kb = blockIdx.y * k_per_split;
         x += kb;
@@ -1117,6 +1137,12 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict
 #pragma unroll
             for (int v = 0; v < 4; ++v) sum[v] = activate(sum[v], tk.act) * own[v];
         }
+        if (beside) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if (n + v < n_end) be.out[(size_t)m * be.N + n + v] = sum[v];
+            continue;
+        }
         if constexpr (RP) {
             rope_store(ra, sum, n, n_end, m, rp_pos, rp_page, (bf16_t*)out, ldo);
         } else if (quads && n + 3 < n_end) {
@@ -1148,6 +1174,7 @@ struct RingCall {
     Groups gr = Groups{};
     RopeArgs ra = RopeArgs{};
     TokenRow tk = TokenRow{};
+    Beside be = Beside{};
 };
 
 template <int WJ, int XH, typename TOut, int SW, int END>
@@ -1156,9 +1183,9 @@ static int launch_ring_t(const RingCall& c, int rows, hipStream_t stream) {
     auto kernel = gemm_ring_kernel<WJ, XH, TOut, SW, END>;
     static hipError_t allowed = allow_lds(kernel, S::LDS);
     TL_REQUIRE(allowed == hipSuccess, "gemm_ring: cannot get %zu bytes of shared memory", S::LDS);
-    const int total = SW ? c.out_cols : c.N;
-    kernel<<<dim3((total + rows - 1) / rows, c.parts, c.gr.count), 256, S::LDS, stream>>>((const bf16_t*)c.x, (const bf16_t*)c.w, c.bias, c.bias_f32, (TOut*)c.out, c.M, c.N, c.K,
-                                                                                      c.ldx, c.ldo, c.out_cols, c.k_per, rows, c.ra, c.tk, c.gr.stride);
+    const int total = SW ? c.out_cols : c.N, least = min(rows, 8), wide = max((total + rows - 1) / rows, (c.be.N + least - 1) / least);      // (be.N: 0 without a product beside)
+    kernel<<<dim3(wide, c.parts, c.gr.count + (END == END_BESIDE)), 256, S::LDS, stream>>>((const bf16_t*)c.x, (const bf16_t*)c.w, c.bias, c.bias_f32, (TOut*)c.out, c.M, c.N, c.K,
+                                                                                      c.ldx, c.ldo, c.out_cols, c.k_per, rows, c.ra, c.tk, c.be, c.gr.stride);
     TL_CHECK_LAUNCH("gemm_ring");
     return TL_OK;
 }
@@ -2066,4 +2093,18 @@ extern "C" int tl_gemm_groups(const void* x, long x_group, const void* w, void* 
         if (rc != TL_OK) return rc;
     }
     return TL_OK;
+}
+
+// The same in bfloat16 for up to 16 rows, and beside them one more product of the same K: out2 [M, N2] (float) = x2 w2^T, rows of x2 ldx apart.  Returns TL_NOT_FUSED (nothing
+// launched) for shapes it is not built for.
+extern "C" int tl_gemm_groups_beside(const void* x, long x_group, const void* w, void* out, long out_group, int groups, int M, int N, int K, int ldx, int ldo, const void* x2,
+                                     const void* w2, void* out2, int N2, hipStream_t stream) {
+    TL_REQUIRE(groups > 0 && groups <= 64 && M > 0 && N > 0 && N2 > 0 && K > 0 && ldx >= K && ldo >= N && x_group >= 0 && out_group >= 0,
+               "gemm_groups_beside: bad sizes groups=%d M=%d N=%d/%d K=%d", groups, M, N, N2, K);
+    if (M > 16 || x_group % 8 || !ring_fits(x, w, M, K, ldx) || !ring_fits(x2, w2, M, K, ldx) || !ring_pays(M, (long)N * groups) || N2 > N) return TL_NOT_FUSED;
+    RingCall c{x, w, nullptr, 0, out, M, N, K, ldx, ldo, 0};
+    c.gr.count = groups;
+    c.gr.stride = GroupStride{x_group, (long)N * K, out_group};
+    c.be = Beside{(const bf16_t*)x2, (const bf16_t*)w2, (float*)out2, N2, groups};
+    return launch_ring<bf16_t, 0, END_BESIDE>(c, stream);
 }

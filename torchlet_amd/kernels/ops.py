@@ -410,6 +410,24 @@ def linear_groups(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor) -> N
                                    c_int(K), c_int(out.stride(0)), c_int(_dt(x, "linear_groups")), c_int(1 if out.dtype == torch.float32 else 0), _stream()))
 
 
+def linear_groups_beside(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, x2: torch.Tensor, weight2: torch.Tensor, out2: torch.Tensor) -> None:
+    """:func:`linear_groups` of ``x``, and :func:`linear` of ``x2 [T, K]`` and ``weight2 [n, K]`` into ``out2 [T, n]`` (float32): one launch for up to 16 rows in bfloat16 where the
+    library has the shape."""
+    G, T, K = x.shape
+    N, n = weight.shape[1], weight2.shape[0]
+    if x.is_cuda and 0 < T <= 16 and x.dtype == weight.dtype == out.dtype == x2.dtype == weight2.dtype == torch.bfloat16 and out2.dtype == torch.float32:
+        if weight.shape != (G, N, K) or out.shape != (T, G * N) or not x.is_contiguous() or not weight.is_contiguous() or out.stride(1) != 1 or x2.shape != (T, K) \
+                or not x2.is_contiguous() or weight2.shape != (n, K) or not weight2.is_contiguous() or out2.shape != (T, n) or not out2.is_contiguous():
+            raise KernelError("linear_groups_beside: shapes do not fit")
+        lib = _lib("gemm")
+        rc = lib.tl_gemm_groups_beside(_ptr(x), ctypes.c_long(T * K), _ptr(weight), _ptr(out), ctypes.c_long(N), c_int(G), c_int(T), c_int(N), c_int(K), c_int(K),
+                                       c_int(out.stride(0)), _ptr(x2), _ptr(weight2), _ptr(out2), c_int(n), _stream())
+        if rc != 100:          # (100: not built for this shape)
+            return _check(lib, rc)
+    linear_groups(x, weight, out)
+    linear(x2, weight2, None, out2)
+
+
 def linear_f32_variant(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, out: torch.Tensor, matrix_cores) -> None:
     """One named kernel of the 32-bit products (for tests and tuning): 0 / False the general tile kernel (``v_fma_f32``),
     1 / True the matrix-core tile kernel (``v_mfma_f32_32x32x2_f32``, K a multiple of 4), 2 and 3 the kernels for up to 16

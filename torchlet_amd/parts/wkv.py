@@ -99,13 +99,12 @@ class WKV(Mixer):
         stream.residual, stream.pending, stream.post = x, None, None
         K, V = self.k_width, self.v_width
         proj = torch.empty((T, 2 * K + 2 * V), dtype=self.dtype, device=dev)          # r | k | v | gate
+        z = torch.empty((T, self.w1.shape[0]), dtype=torch.float32, device=dev)
         if self.w_rkvg is not None:
-            ops.linear_groups(mixes[:4], self.w_rkvg, proj)
+            ops.linear_groups_beside(mixes[:4], self.w_rkvg, proj, mixes[4], self.w1, z)
         else:
             ops.linear_groups(mixes[:2], self.w_rk, proj[:, : 2 * K])
-            ops.linear_groups(mixes[2:4], self.w_vg, proj[:, 2 * K:])
-        z = torch.empty((T, self.w1.shape[0]), dtype=torch.float32, device=dev)
-        ops.linear(mixes[4], self.w1, None, z)
+            ops.linear_groups_beside(mixes[2:4], self.w_vg, proj[:, 2 * K:], mixes[4], self.w1, z)
         decay = torch.empty((T, K), dtype=torch.float32, device=dev)
         ops.channel_decay(z, self.w2t, self.w0, decay)
         o = torch.empty((T, V), dtype=torch.float32, device=dev)
