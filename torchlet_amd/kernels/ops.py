@@ -424,7 +424,10 @@ def linear_groups_beside(x: torch.Tensor, weight: torch.Tensor, out: torch.Tenso
                                        c_int(out.stride(0)), _ptr(x2), _ptr(weight2), _ptr(out2), c_int(n), _stream())
         if rc != 100:          # (100: not built for this shape)
             return _check(lib, rc)
-    linear_groups(x, weight, out)
+    if G == 1:
+        linear(x[0], weight[0], None, out)
+    else:
+        linear_groups(x, weight, out)
     linear(x2, weight2, None, out2)
 
 

@@ -352,6 +352,7 @@ class StagedMixer(Mixer):
     w_o: torch.Tensor | None = None
     b_in: torch.Tensor | None = None      # biases of the two projections (a mixer that stands alone may have them; branches of a
     b_o: torch.Tensor | None = None       # mixer that stacks several projections into one may not)
+    w_side: torch.Tensor | None = None    # [n, hidden]: what the mixer projects into 32-bit numbers beside ``w_in``; ``mix`` is handed the result as ``side``
 
     def mix(self, proj: torch.Tensor, h: torch.Tensor, ctx, cache, out: torch.Tensor, gain: float = 1.0) -> None:
         """``proj [T, in_width]`` (a row-strided view of ``h @ w_in.T``) and ``h`` itself (for what the mixer projects on its own,
@@ -359,13 +360,28 @@ class StagedMixer(Mixer):
         raise NotImplementedError
 
     def forward(self, h, ctx, cache):
-        from ..kernels import ops
         T = h.shape[0]
         proj = torch.empty((T, self.in_width), dtype=self.dtype, device=h.device)
-        ops.linear(h, self.w_in, self.b_in, proj)
+        more = project_in(h, self.w_in, self.b_in, proj, self)
         mixed = torch.empty((T, self.mix_width), dtype=self.dtype, device=h.device)
-        self.mix(proj, h, ctx, cache, mixed)
+        self.mix(proj, h, ctx, cache, mixed, **more)
         return project_out(mixed, self.w_o, self.dtype, self.b_o)
+
+
+def project_in(h: torch.Tensor, w_in: torch.Tensor, b_in: torch.Tensor | None, proj: torch.Tensor, mixer: StagedMixer | None) -> dict:
+    """``proj = h @ w_in.T (+ b_in)``, and what ``mixer`` projects beside it: few rows in one launch.  The latter as the keyword argument of its ``mix``."""
+    from ..kernels import ops
+    w_side = mixer.w_side if mixer is not None else None
+    if w_side is None:
+        ops.linear(h, w_in, b_in, proj)
+        return {}
+    side = torch.empty((h.shape[0], w_side.shape[0]), dtype=torch.float32, device=h.device)
+    if b_in is None and h.is_contiguous():
+        ops.linear_groups_beside(h[None], w_in[None], proj, h, w_side, side)
+    else:
+        ops.linear(h, w_in, b_in, proj)
+        ops.linear(h, w_side, None, side)
+    return {"side": side}
 
 
 def project_out(mixed: torch.Tensor, w_o: torch.Tensor, dtype: torch.dtype, bias: torch.Tensor | None = None) -> torch.Tensor:

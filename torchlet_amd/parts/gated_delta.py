@@ -87,10 +87,16 @@ class GatedDelta(StagedMixer):
         self.w_norm = self._place(tensors["norm"], KEEP_FLOAT32)
         self.w_o = self._place(tensors["o"], KEEP_COMPUTE)
 
-    def mix(self, proj, h, ctx, cache, out, gain=1.0):
+    @property
+    def w_side(self):
+        return self.w_gates
+
+    def mix(self, proj, h, ctx, cache, out, gain=1.0, side=None):
         T = h.shape[0]
-        gates = torch.empty((T, 2 * self.heads), dtype=torch.float32, device=h.device)
-        ops.linear(h, self.w_gates, None, gates)
+        gates = side
+        if gates is None:
+            gates = torch.empty((T, 2 * self.heads), dtype=torch.float32, device=h.device)
+            ops.linear(h, self.w_gates, None, gates)
         qkv = torch.empty((T, self.channels), dtype=torch.float32, device=h.device)
         # convolutions (from the slot's tails, which move on), silu, unit vectors; the raw gates become beta and the decay in place
         ops.delta_prepare(proj, self.w_conv, gates, self.a_log, self.dt_bias, cache.state, self.state_floats, ctx.slots, ctx.req_indptr,

@@ -15,7 +15,7 @@ import torch
 
 from ..config.base import ConfigError
 from ..kernels import ops
-from .base import KEEP_COMPUTE, KEEP_FLOAT32, MIXERS, Mixer, StagedMixer, WeightSpec, join_name, project_out, under
+from .base import KEEP_COMPUTE, KEEP_FLOAT32, MIXERS, Mixer, StagedMixer, WeightSpec, join_name, project_in, project_out, under
 
 
 @MIXERS.register("parallel")
@@ -79,13 +79,14 @@ class ParallelMixer(Mixer):
     def forward(self, h, ctx, cache):
         T = h.shape[0]
         proj = torch.empty((T, self.w_in.shape[0]), dtype=self.dtype, device=h.device)
-        ops.linear(h, self.w_in, None, proj)
+        beside = next((b for b in self.branches if b.w_side is not None), None)
+        more = project_in(h, self.w_in, None, proj, beside)
         if self.normed:
             outs = torch.empty((len(self.branches), T, self.hidden), dtype=self.dtype, device=h.device)
             at_in = 0
             for i, b in enumerate(self.branches):
                 mixed = torch.empty((T, b.mix_width), dtype=self.dtype, device=h.device)
-                b.mix(proj[:, at_in: at_in + b.in_width], h, ctx, cache, mixed)
+                b.mix(proj[:, at_in: at_in + b.in_width], h, ctx, cache, mixed, **(more if b is beside else {}))
                 ops.linear(mixed, self.w_outs[i], None, outs[i])
                 at_in += b.in_width
             y = torch.empty((T, self.hidden), dtype=self.dtype, device=h.device)
@@ -94,7 +95,7 @@ class ParallelMixer(Mixer):
         mixed = torch.empty((T, self.w_o.shape[1]), dtype=self.dtype, device=h.device)
         at_in = at_out = 0
         for b, scale in zip(self.branches, self.scales):
-            b.mix(proj[:, at_in: at_in + b.in_width], h, ctx, cache, mixed[:, at_out: at_out + b.mix_width], scale)
+            b.mix(proj[:, at_in: at_in + b.in_width], h, ctx, cache, mixed[:, at_out: at_out + b.mix_width], scale, **(more if b is beside else {}))
             at_in += b.in_width
             at_out += b.mix_width
         return project_out(mixed, self.w_o, self.dtype)
