@@ -60,3 +60,27 @@ def test_chosen_rows_kinds_and_float_output(S, width, kind, gain):
             want = u / torch.sqrt((u * u).mean(-1, keepdim=True) + eps) * gain * w.double()
         # (32-bit sums of some ten terms, a mean over the row and a handful of products: a few units of 2^-24 each)
         torch.testing.assert_close(out.cpu().double(), want, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("S,width,rows", [(1, 2048, 3), (4, 2048, 300), (1, 8196, 256), (2, 8192, 257), (4, 8192, 300), (1, 15360, 300), (2, 15360, 3)])
+@pytest.mark.parametrize("kind", ["layernorm", "rmsnorm"])
+@pytest.mark.parametrize("slabs", [0, 3, 9])
+def test_vectors_at_any_address_and_any_number_of_rows_give_the_same_bits(S, width, rows, kind, slabs):
+    """The norm's vectors behind one more number (no whole pieces to fetch them in), and rows beyond those that have a compute unit each: the registers' kernel all the same, number by number
+    and later instead of in whole pieces and at once, with the same sums."""
+    from torchlet_amd.kernels import ops
+    g = torch.Generator().manual_seed(width + rows)
+    x, pending = torch.randn(S, rows, width, generator=g), torch.randn(*((slabs,) if slabs else ()), rows, width, generator=g)
+    pending = (pending if slabs else pending.bfloat16()).cuda()
+    vectors = [torch.randn(width + 8, generator=g).to(torch.bfloat16 if kind == "layernorm" else torch.float32).cuda() for _ in range(2)]
+
+    def norm(n, at):
+        w, b = (torch.cat((v[:at], v)).cuda()[at: at + width] for v in vectors)
+        copies, out = x[:, :n].contiguous().cuda(), torch.empty(n, width, dtype=torch.bfloat16, device="cuda")
+        ops.streams_norm(copies, (pending[:, :n] if slabs else pending[:n]).contiguous(), None, None, kind, w, b if kind == "layernorm" else None, 1e-5, out)
+        return copies, out
+
+    copies, want = norm(rows, 0)
+    for n, at in ((rows, 1), (rows, 4), (2, 0), (2, 3)):
+        got = norm(n, at)
+        assert torch.equal(got[1], want[:n]) and torch.equal(got[0], copies[:, :n])

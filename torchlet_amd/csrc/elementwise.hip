@@ -762,7 +762,7 @@ template <typename T, int S, int N>
 __global__ void __launch_bounds__(1024)
 streams_norm_reg_kernel(float* __restrict__ x, int total_rows, int hidden, const void* __restrict__ pending, int parts, const float* __restrict__ mix,
                         const float* __restrict__ gate, const float* __restrict__ read, int kind, const void* __restrict__ weight, int weight_f32,
-                        const void* __restrict__ bias, int bias_f32, float eps, float gain, T* __restrict__ out, const int* __restrict__ rows) {
+                        const void* __restrict__ bias, int bias_f32, float eps, float gain, T* __restrict__ out, const int* __restrict__ rows, bool whole) {
     constexpr bool EARLY = S * N <= 8;               // the norm's vectors in registers from the start, where there is room for them
     __shared__ float red[2][16];
     const int orow = blockIdx.x;
@@ -778,7 +778,11 @@ streams_norm_reg_kernel(float* __restrict__ x, int total_rows, int hidden, const
         for (int a = 0; a < S; ++a) m[a][b] = mix ? mix[a * S + b] : (a == b ? 1.f : 0.f);
     }
     float4 xs[S][N], p[N], u[N], w[EARLY ? N : 1], sh[EARLY ? N : 1];
-    auto vec4 = [](const void* v, int is_f32, int i) { return is_f32 ? load4((const float*)v + i) : load4((const bf16_t*)v + i); };
+    // (`whole`: both vectors lie where four numbers can be fetched at once)
+    auto vec4 = [&](const void* v, int is_f32, int i) {
+        if (!whole) return make_float4(load_vec(v, is_f32, i), load_vec(v, is_f32, i + 1), load_vec(v, is_f32, i + 2), load_vec(v, is_f32, i + 3));
+        return is_f32 ? load4((const float*)v + i) : load4((const bf16_t*)v + i);
+    };
     // (beyond the row: its last piece again, kept out of the sums and the stores)
     auto at = [&](int j) { return min(4 * (int)(threadIdx.x + j * blockDim.x), hidden - 4); };
 #pragma unroll
@@ -891,11 +895,13 @@ extern "C" int tl_streams_norm(void* x, int streams, int total_rows, int hidden,
     if (n_out == 0) return TL_OK;
     // Rows in registers wherever a piece of four numbers can be fetched whole (us, this kernel / the one above: 8 rows of 2048 4.0 / 15.4, 8 rows of 8192 7.0 / 45, 2048 rows of
     // 2048 25.3 / 44.8 and of 4096 48.3 / 78.2; the short ones are bound by their launch).
-    const bool pieces = hidden % 4 == 0 && hidden <= 16384 && (((uintptr_t)x | (uintptr_t)pending | (uintptr_t)out | (uintptr_t)weight | (uintptr_t)bias) % 16) == 0;
+    const bool pieces = hidden % 4 == 0 && hidden <= 16384 && (((uintptr_t)x | (uintptr_t)pending | (uintptr_t)out) % 16) == 0;
+    // (the vectors number by number where they lie elsewhere: 8 rows of four copies of 2048 4.7 us, 64 rows of 8192 7.3; by the kernel above 16.3 and 32)
+    const bool whole = (uintptr_t)weight % (weight_f32 ? 16 : 8) == 0 && (uintptr_t)bias % (bias_f32 ? 16 : 8) == 0;
     if (pieces && (streams == 1 || streams == 2 || streams == 4) && (act_dtype == TL_DT_F32 || act_dtype == TL_DT_BF16)) {
         const int n = hidden <= 4096 ? 1 : hidden <= 8192 ? 2 : 4, threads = ((hidden / 4 + n - 1) / n + TL_WAVE - 1) / TL_WAVE * TL_WAVE;
 #define TL_SN_T(T, S, N) streams_norm_reg_kernel<T, S, N><<<n_out, threads, 0, stream>>>((float*)x, total_rows, hidden, pending, parts, (const float*)mix, \
-        (const float*)gate, (const float*)read, kind, weight, weight_f32, bias, bias_f32, eps, gain, (T*)out, (const int*)rows)
+        (const float*)gate, (const float*)read, kind, weight, weight_f32, bias, bias_f32, eps, gain, (T*)out, (const int*)rows, whole)
 #define TL_SN_N(T, S) (n == 1 ? TL_SN_T(T, S, 1) : n == 2 ? TL_SN_T(T, S, 2) : TL_SN_T(T, S, 4))
 #define TL_SN(T) (streams == 1 ? TL_SN_N(T, 1) : streams == 2 ? TL_SN_N(T, 2) : TL_SN_N(T, 4))
         if (act_dtype == TL_DT_F32) TL_SN(float); else TL_SN(bf16_t);
