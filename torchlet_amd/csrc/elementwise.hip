@@ -756,28 +756,32 @@ __device__ __forceinline__ void add_slabs4(const float* src, size_t stride, floa
 // every copy's piece and the pending output's are requested together, and the passes over u (mean, squared deviations, output) read registers.
 // What bounds it: a decode step's few rows the trip to memory and the two sums over the work-group, a prompt's rows the bytes (each copy once in
 // and once out).  Measured against the kernel above (four copies, a pending output of bfloat16, layer norm): see tl_streams_norm.
-// One trip to memory: the copies, the pending output, the norm's vectors and the numbers of the mix are all requested before the first is used, slabs of partial sums four at a time (one after
-// the other, and the vectors behind the two sums, 8 rows of four copies of 2048 with four slabs took 5.1 us, with this 4.1; 8 rows of 8192 10.0 / 7.0).
-template <typename T, int S, int N>
+// EARLY, one trip to memory: the copies, the pending output, the norm's vectors and the numbers of the mix are all requested before the first is used, slabs of partial sums four at a
+// time (one after the other, and the vectors behind the two sums, 8 rows of four copies of 2048 with four slabs took 5.1 us, with this 4.1; 8 rows of 8192 10.0 / 7.0).  That takes up to
+// 118 registers where the rest needs 18 to 105: see tl_streams_norm for who gets it.
+template <typename T, int S, int N, bool EARLY>
 __global__ void __launch_bounds__(1024)
 streams_norm_reg_kernel(float* __restrict__ x, int total_rows, int hidden, const void* __restrict__ pending, int parts, const float* __restrict__ mix,
                         const float* __restrict__ gate, const float* __restrict__ read, int kind, const void* __restrict__ weight, int weight_f32,
                         const void* __restrict__ bias, int bias_f32, float eps, float gain, T* __restrict__ out, const int* __restrict__ rows, bool whole) {
-    constexpr bool EARLY = S * N <= 8;               // the norm's vectors in registers from the start, where there is room for them
+    constexpr bool VECTORS = EARLY && S * N <= 8;    // the norm's vectors in registers from the start, where there is room for them
     __shared__ float red[2][16];
     const int orow = blockIdx.x;
     const int srow = rows ? rows[orow] : orow;
     const size_t copy_stride = (size_t)total_rows * hidden;
     float* xr = x + (size_t)srow * hidden;
     float m[S][S], g[S], rd[S];
+    auto fetch_mix = [&]() {
 #pragma unroll
-    for (int b = 0; b < S; ++b) {
-        g[b] = gate ? gate[b] : 1.f;
-        rd[b] = read ? read[b] : 1.f;
+        for (int b = 0; b < S; ++b) {
+            g[b] = gate ? gate[b] : 1.f;
+            rd[b] = read ? read[b] : 1.f;
 #pragma unroll
-        for (int a = 0; a < S; ++a) m[a][b] = mix ? mix[a * S + b] : (a == b ? 1.f : 0.f);
-    }
-    float4 xs[S][N], p[N], u[N], w[EARLY ? N : 1], sh[EARLY ? N : 1];
+            for (int a = 0; a < S; ++a) m[a][b] = mix ? mix[a * S + b] : (a == b ? 1.f : 0.f);
+        }
+    };
+    if (EARLY) fetch_mix();
+    float4 xs[S][N], p[N], u[N], w[VECTORS ? N : 1], sh[VECTORS ? N : 1];
     // (`whole`: both vectors lie where four numbers can be fetched at once)
     auto vec4 = [&](const void* v, int is_f32, int i) {
         if (!whole) return make_float4(load_vec(v, is_f32, i), load_vec(v, is_f32, i + 1), load_vec(v, is_f32, i + 2), load_vec(v, is_f32, i + 3));
@@ -793,24 +797,27 @@ streams_norm_reg_kernel(float* __restrict__ x, int total_rows, int hidden, const
         p[j] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (pending && parts == 0) p[j] = load4((const T*)pending + (size_t)srow * hidden + i);
     }
-    if (EARLY) {
+    if (VECTORS) {
 #pragma unroll
         for (int j = 0; j < N; ++j) {
             w[j] = vec4(weight, weight_f32, at(j));
             if (kind == 1) sh[j] = vec4(bias, bias_f32, at(j));
         }
     }
-    if (pending && parts > 0) {                      // slabs in their order, four requested together
+    if (pending && parts > 0) {                      // slabs in their order
 #pragma unroll
         for (int j = 0; j < N; ++j) {
             const float* slab = (const float*)pending + (size_t)srow * hidden + at(j);
             int q = 0;
-            for (; q + 4 <= parts; q += 4) add_slabs4<4>(slab + q * copy_stride, copy_stride, p[j]);
-            if (parts - q == 3) add_slabs4<3>(slab + q * copy_stride, copy_stride, p[j]);
-            else if (parts - q == 2) add_slabs4<2>(slab + q * copy_stride, copy_stride, p[j]);
-            else if (parts - q == 1) add_slabs4<1>(slab + q * copy_stride, copy_stride, p[j]);
+            if (EARLY)
+                for (; q + 4 <= parts; q += 4) add_slabs4<4>(slab + q * copy_stride, copy_stride, p[j]);
+            if (EARLY && parts - q == 3) add_slabs4<3>(slab + q * copy_stride, copy_stride, p[j]);
+            else if (EARLY && parts - q == 2) add_slabs4<2>(slab + q * copy_stride, copy_stride, p[j]);
+            else
+                for (; q < parts; ++q) add_slabs4<1>(slab + q * copy_stride, copy_stride, p[j]);
         }
     }
+    if (!EARLY) fetch_mix();
     const int lane = threadIdx.x % TL_WAVE, wave = threadIdx.x / TL_WAVE, waves = blockDim.x / TL_WAVE;
     auto row_sum = [&](float v, float* place) {
         v = wave_sum(v);
@@ -873,10 +880,10 @@ streams_norm_reg_kernel(float* __restrict__ x, int total_rows, int hidden, const
     for (int j = 0; j < N; ++j) {
         const int i = 4 * (threadIdx.x + j * blockDim.x);
         if (i >= hidden) continue;
-        const float4 wj = EARLY ? w[EARLY ? j : 0] : vec4(weight, weight_f32, i);
+        const float4 wj = VECTORS ? w[VECTORS ? j : 0] : vec4(weight, weight_f32, i);
         float4 y;
         if (kind == 1) {
-            const float4 bj = EARLY ? sh[EARLY ? j : 0] : vec4(bias, bias_f32, i);
+            const float4 bj = VECTORS ? sh[VECTORS ? j : 0] : vec4(bias, bias_f32, i);
             y = make_float4((u[j].x * inv * wj.x + bj.x) * gain, (u[j].y * inv * wj.y + bj.y) * gain, (u[j].z * inv * wj.z + bj.z) * gain, (u[j].w * inv * wj.w + bj.w) * gain);
         } else {
             y = make_float4(u[j].x * inv * gain * wj.x, u[j].y * inv * gain * wj.y, u[j].z * inv * gain * wj.z, u[j].w * inv * gain * wj.w);
@@ -898,16 +905,21 @@ extern "C" int tl_streams_norm(void* x, int streams, int total_rows, int hidden,
     const bool pieces = hidden % 4 == 0 && hidden <= 16384 && (((uintptr_t)x | (uintptr_t)pending | (uintptr_t)out) % 16) == 0;
     // (the vectors number by number where they lie elsewhere: 8 rows of four copies of 2048 4.7 us, 64 rows of 8192 7.3; by the kernel above 16.3 and 32)
     const bool whole = (uintptr_t)weight % (weight_f32 ? 16 : 8) == 0 && (uintptr_t)bias % (bias_f32 ? 16 : 8) == 0;
+    // EARLY for as many rows as the GPU has compute units, and for rows of up to 4096 numbers: beyond, the registers it takes leave a unit one row at a time instead of two (us, EARLY / not:
+    // 2048 rows of two copies of 8192, layer norm, 72 / 54; of one of 15360 77 / 59; 300 rows of four of 8192 22.5 / 18.5; 2048 rows of one of 4096, vectors number by number, 28 / 25).
+    const bool early = n_out <= 256 || (whole && hidden <= 4096);
     if (pieces && (streams == 1 || streams == 2 || streams == 4) && (act_dtype == TL_DT_F32 || act_dtype == TL_DT_BF16)) {
         const int n = hidden <= 4096 ? 1 : hidden <= 8192 ? 2 : 4, threads = ((hidden / 4 + n - 1) / n + TL_WAVE - 1) / TL_WAVE * TL_WAVE;
-#define TL_SN_T(T, S, N) streams_norm_reg_kernel<T, S, N><<<n_out, threads, 0, stream>>>((float*)x, total_rows, hidden, pending, parts, (const float*)mix, \
+#define TL_SN_E(T, S, N, EARLY) streams_norm_reg_kernel<T, S, N, EARLY><<<n_out, threads, 0, stream>>>((float*)x, total_rows, hidden, pending, parts, (const float*)mix, \
         (const float*)gate, (const float*)read, kind, weight, weight_f32, bias, bias_f32, eps, gain, (T*)out, (const int*)rows, whole)
+#define TL_SN_T(T, S, N) (early ? TL_SN_E(T, S, N, true) : TL_SN_E(T, S, N, false))
 #define TL_SN_N(T, S) (n == 1 ? TL_SN_T(T, S, 1) : n == 2 ? TL_SN_T(T, S, 2) : TL_SN_T(T, S, 4))
 #define TL_SN(T) (streams == 1 ? TL_SN_N(T, 1) : streams == 2 ? TL_SN_N(T, 2) : TL_SN_N(T, 4))
         if (act_dtype == TL_DT_F32) TL_SN(float); else TL_SN(bf16_t);
 #undef TL_SN
 #undef TL_SN_N
 #undef TL_SN_T
+#undef TL_SN_E
         TL_CHECK_LAUNCH("streams_norm");
         return TL_OK;
     }
