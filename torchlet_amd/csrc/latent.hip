@@ -692,7 +692,7 @@ latent_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __r
             }
             l = l * alpha + psum;
             m = m_new;
-            if (moved) {
+            if (WHOLE && moved) {
 #pragma unroll
                 for (int t = 0; t < NT; ++t) acc[t] *= alpha;
             }
@@ -704,6 +704,7 @@ latent_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __r
                     LmFrag vf;
                     vf.h[0] = *(const uint2*)lrow;
                     vf.h[1] = *(const uint2*)(lrow + 16);
+                    if (!WHOLE && moved) acc[t] *= alpha;
                     acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, pf.v, acc[t], 0, 0, 0);
                 }
             }
