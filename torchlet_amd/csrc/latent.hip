@@ -88,10 +88,12 @@ __global__ void latent_prepare_kernel(const T* __restrict__ down, int ld, int q_
 }
 
 // The same for fewer than 512 tokens, with a work-group for each thing that there is to do (`roles`: bit 0 the page row, bit 1 the query latent, bit 2 the queries' rotated parts; blockIdx.y
-// counts those that are set), so that a decode step waits for one of them and not for all in turn.  Each asks for its numbers and its norm's weights before it uses the first.
+// counts those that are set), so that a decode step waits for one of them and not for all in turn.  Each asks for its numbers and its norm's weights before it uses the first, the page row's for
+// its page as well, and looks whether that is the sentinel when its sum is there.  KEEP 2 for rows of up to 512 numbers, 8 for others: places a row does not fill are asked for all the same.
+// (A page row without rotated numbers, alone, 512 numbers: in turn 3.8, with the page looked at first and eight places 4.2, so 3.8.)
 // (us, all in turn / this: one token, a query latent of 1536 5.4 / 3.3, of 768 4.7 / 3.3, 16 heads' rotated parts 3.8 / 3.3; 511 tokens 6.4 / 4.5, 5.5 / 4.1, 4.7 / 4.1.  Of more tokens
 // the chip holds no more work-groups at once: 2048 tokens 9.9 / 11.4.)
-template <typename T>
+template <typename T, int KEEP>                                 // KEEP: numbers of a row that a thread keeps; a longer row's others are read again
 __global__ void __launch_bounds__(256)
 latent_prepare_few_kernel(const T* __restrict__ down, int ld, int q_rank, int kv_off, int rank, int rot, int rot_dims,
                           const void* __restrict__ wq, int wq_f32, const void* __restrict__ wkv, int wkv_f32, float eps,
@@ -100,18 +102,19 @@ latent_prepare_few_kernel(const T* __restrict__ down, int ld, int q_rank, int kv
                           T* __restrict__ plane, int page_size, T* __restrict__ cq, int halves, T* __restrict__ rows, QueryParts parts, int roles) {
     __shared__ float red[16];
     __shared__ float cs[LAT_MAX_PAIRS], sn[LAT_MAX_PAIRS];      // the token's angles, by which all heads turn
-    constexpr int KEEP = 8;                                     // numbers of a row that a thread keeps; a longer row's others are read again
     const int t = blockIdx.x, half = rot_dims / 2, steps = rot - half;      // (steps: pairs, then single numbers)
     const T* row = down + (size_t)t * ld;
-    // number j of a rotated part: its partner lies as far on as the pair is wide
-    auto turn_part = [&](const T* src, T* dst, int j, float c, float sine) {
+    // number j of a rotated part: its partner lies as far on as the pair is wide; what lies beyond the rotated dimensions passes, as it is
+    struct Two { T u, v; };
+    auto first_of = [&](int j) { return j >= half ? half + j : halves ? j : 2 * j; };
+    auto fetch_two = [&](const T* src, int j) { return Two{src[first_of(j)], src[j >= half ? half + j : halves ? j + half : 2 * j + 1]}; };
+    auto put_turned = [&](T* dst, int j, Two x, float c, float sine) {
         if (j < half) {
-            const int a = halves ? j : 2 * j, b = halves ? j + half : 2 * j + 1;
-            const float u = to_float(src[a]), v = to_float(src[b]);
-            dst[a] = from_float<T>(u * c - v * sine);
-            dst[b] = from_float<T>(v * c + u * sine);
+            const float u = to_float(x.u), v = to_float(x.v);
+            dst[first_of(j)] = from_float<T>(u * c - v * sine);
+            dst[halves ? j + half : 2 * j + 1] = from_float<T>(v * c + u * sine);
         } else {
-            dst[half + j] = src[half + j];                      // (what lies beyond the rotated dimensions passes)
+            dst[half + j] = x.u;
         }
     };
     auto work = [&](int role) {
@@ -120,7 +123,8 @@ latent_prepare_few_kernel(const T* __restrict__ down, int ld, int q_rank, int kv
             __syncthreads();
             for (int i = threadIdx.x; i < parts.heads * steps; i += 256) {
                 const int h = i / steps, j = i % steps;
-                turn_part(row + (size_t)h * parts.head + parts.plain, rows + (size_t)t * parts.rows_ld + (size_t)h * (rank + rot) + rank, j, j < half ? cs[j] : 0.f, j < half ? sn[j] : 0.f);
+                put_turned(rows + (size_t)t * parts.rows_ld + (size_t)h * (rank + rot) + rank, j, fetch_two(row + (size_t)h * parts.head + parts.plain, j), j < half ? cs[j] : 0.f,
+                           j < half ? sn[j] : 0.f);
             }
             return;
         }
@@ -135,14 +139,17 @@ latent_prepare_few_kernel(const T* __restrict__ down, int ld, int q_rank, int kv
             wx[j] = i < n ? load_vec(w, w_f32, i) : 0.f;
         }
         T* dst = cq + (size_t)t * q_rank;
-        if (role == 0) {
-            const int pos = positions[t], page = block_table[(size_t)token_req[t] * bt_stride + pos / page_size];
-            if (page == 0) return;                                  // (the whole work-group)
+        int pos = 0, page = 1;
+        Two two;
+        float c = 0.f, sine = 0.f;
+        auto angle = [&](int i) { if (i < half) sincosf((float)pos * inv_freq[i], &sine, &c); };
+        if (role == 0) {                                            // the page and this thread's first pair are fetched beside the row, looked at when its sum is there
+            pos = positions[t];
+            page = block_table[(size_t)token_req[t] * bt_stride + pos / page_size];
             dst = plane + ((size_t)page * page_size + pos % page_size) * (rank + rot);
-            for (int i = threadIdx.x; i < steps; i += 256) {
-                float c = 0.f, sine = 0.f;
-                if (i < half) sincosf((float)pos * inv_freq[i], &sine, &c);
-                turn_part(src + rank, dst + rank, i, c, sine);
+            if ((int)threadIdx.x < steps) {
+                two = fetch_two(src + rank, threadIdx.x);
+                angle(threadIdx.x);
             }
         }
         float ss = 0.f;
@@ -150,7 +157,15 @@ latent_prepare_few_kernel(const T* __restrict__ down, int ld, int q_rank, int kv
         for (int j = 0; j < KEEP; ++j) ss = fmaf(x[j], x[j], ss);
         for (int i = threadIdx.x + 256 * KEEP; i < n; i += 256) { const float v = to_float(src[i]); ss = fmaf(v, v, ss); }
         ss = block_sum(ss, red);
+        if (page == 0) return;                                      // (the whole work-group)
         const float inv = 1.f / sqrtf(ss / (float)n + eps);
+        if (role == 0) {
+            if ((int)threadIdx.x < steps) put_turned(dst + rank, threadIdx.x, two, c, sine);
+            for (int i = threadIdx.x + 256; i < steps; i += 256) {
+                angle(i);
+                put_turned(dst + rank, i, fetch_two(src + rank, i), c, sine);
+            }
+        }
 #pragma unroll
         for (int j = 0; j < KEEP; ++j) {
             const int i = threadIdx.x + 256 * j;
@@ -186,7 +201,8 @@ extern "C" int tl_latent_prepare(const void* down, int ld, int q_rank, int kv_of
 #define TL_ARGS(T) (const T*)down, ld, q_rank, kv_off, rank, rot, rot_dims, wq, wq_f32, wkv, wkv_f32, eps, (const int*)positions, (const float*)inv_freq, \
                    (const int*)token_req, (const int*)block_table, bt_stride, (T*)plane, page_size, (T*)cq, halves, (T*)rows, QueryParts{q_heads, q_head, q_plain, rows_ld}
 #define TL_PREPARE(T)                                                                            \
-    if (few) latent_prepare_few_kernel<T><<<grid, block, 0, stream>>>(TL_ARGS(T), roles);        \
+    if (few && max(q_rank, rank) <= 512) latent_prepare_few_kernel<T, 2><<<grid, block, 0, stream>>>(TL_ARGS(T), roles);        \
+    else if (few) latent_prepare_few_kernel<T, 8><<<grid, block, 0, stream>>>(TL_ARGS(T), roles);        \
     else latent_prepare_kernel<T><<<grid, block, 0, stream>>>(TL_ARGS(T))
     if (dtype == TL_DT_F32) { TL_PREPARE(float); }
     else if (dtype == TL_DT_BF16) { TL_PREPARE(bf16_t); }
