@@ -104,3 +104,30 @@ def test_merge_of_a_decoded_tokens_parts(vdim, splits, monkeypatch):
         w = torch.exp(s - torch.cat((s, sink.double()[:, None]), 1).logsumexp(1, keepdim=True))
         bound = 2.0 ** -7 * (w @ values.abs()) + 1e-4          # (as above)
         assert bool(((out[r].cpu().double().view(heads, vdim) - w @ values).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("rank", [64, 80, 128, 192, 256, 320, 384, 448, 512])        # (80: the kernel by sizes that come with the call)
+@pytest.mark.parametrize("rot", [0, 32, 64, 96, 16])                                 # (as 96; with 16 only rows of whole pieces of 32, so 80 alone)
+@pytest.mark.parametrize("tile_rows,new,splits", [(16, 1, 1), (16, 1, 3), (32, 2, 1), (64, 5, 1), (64, 5, 2)])
+def test_attention_at_every_size_that_has_a_kernel(rank, rot, tile_rows, new, splits):
+    from torchlet_amd.kernels import ops
+    D = rank + rot
+    if D % 32:
+        return
+    g = torch.Generator().manual_seed(D + splits)
+    heads, page, ctx, scale, bl = 16, 8, [3, 77], 0.08, 12
+    plane = torch.randn(1 + 2 * bl, 1, page, D, generator=g).bfloat16()
+    table = (1 + torch.randperm(2 * bl, generator=g)).int().view(2, bl)
+    T, tq = 2 * new, ops.latent_tile_tokens(heads, tile_rows)
+    q = torch.randn(T, heads * D, generator=g).bfloat16()
+    tiles = [(r, t) for r in range(2) for t in range(0, new, tq)]
+    out = torch.empty(T, heads * rank, dtype=torch.bfloat16, device="cuda")
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    ops.latent_attention(q.cuda(), out, plane.cuda(), table.cuda(), i32([0, new, 2 * new]), i32(ctx), i32([r for r, _ in tiles]), i32([t for _, t in tiles]), len(tiles), tq, heads, rank, rot,
+                         page, scale, None, splits, max_new_tokens=new, window=0)
+    for r in range(2):
+        for i in range(new):
+            keys = plane[table[r].long()].reshape(-1, D)[: ctx[r] + i + 1].double()
+            w = torch.softmax(q[r * new + i].double().view(heads, D) @ keys.T * scale, 1)
+            bound = 2.0 ** -7 * (w @ keys[:, :rank].abs()) + 1e-4          # (as above)
+            assert bool(((out[r * new + i].cpu().double().view(heads, rank) - w @ keys[:, :rank]).abs() <= bound).all())

@@ -531,9 +531,11 @@ static void launch_latent_merge(const void* part_o, const void* part_ml, void* o
 // A work-group of four waves owns RB blocks of 16 rows (row = token x head of a chunk of up to 16 heads; RB = 4, 2 or 1
 // by how many rows a tile of the step can have) and 4 / RB waves share a block: each takes all of the block's scores
 // (the softmax's state is then the same in all of them, nothing is exchanged) and its own share of the latent's columns.
-// A wave has its SIMD to itself, so the vector instructions around the products are what a step costs.  Latents of 512 numbers beside 64 or no rotated ones have kernels of their own,
-// in which every piece of a row is known to be there: a step of 32 keys with one block 5.1 us by sizes that come with the call, 2.8 by known ones (one token, 16 heads: 64 keys
-// 15.4 / 10.8 us, 512 keys in 8 parts 18.3 / 13.9, 4000 keys in 62 parts 24.6 / 18.4).
+// A wave has few others on its SIMD, so the vector instructions around the products are what a step costs.  Where the latent is a multiple of 64 numbers, which gives all waves that share
+// a block of rows the same number of columns, and the rotated part 0, 32 or 64 (RANK, ROT), the kernel is built for the sizes: which pieces of a row there are is then no comparison any more, and
+// the registers are as many as it needs.  (us, by sizes that come with the call / known; one token, 16 heads: 512 beside 64, 64 keys 15.4 / 10.8, 512 keys in 8 parts 18.3 / 13.9, 4000 keys in 62
+// parts 24.6 / 18.4, 384 beside 64, 4000 keys 29.7 / 17.8, 256 beside 64, 500 keys 21.3 / 14.6; prompts, four times 64 tokens behind 500: 512 beside 32 109 / 84, 256 beside 64 77 / 52, 64 beside 64
+// 47 / 28.)  Other sizes keep the kernel that takes them with the call (RANK 0).
 #define LM_KEYS 32                    // keys of a step
 #define LM_DC_MAX 20                  // 32-number pieces of a cache row (rows of up to 640 numbers)
 #define LM_LOG2E 1.4426950408889634f
@@ -558,8 +560,8 @@ latent_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __r
     const int rank = RANK ? RANK : any_rank, rot = RANK ? ROT : any_rot;
     constexpr int DC = RANK ? (RANK + ROT) / 32 : LM_DC_MAX, ROUNDS = RANK ? (RANK + ROT + 63) / 64 : LM_DC_MAX / 2;      // 32-number pieces of a row, and rounds of eight lanes' pieces
     constexpr int WPR = 4 / RB;                      // waves that share a block of rows
-    constexpr int NT = 32 / WPR;                     // most blocks of 16 latent columns a wave sums (latents of up to 512 numbers)
-    constexpr bool WHOLE = RANK == 512;              // every wave has that many
+    constexpr int NT = (RANK ? RANK / 16 : 32) / WPR;   // most blocks of 16 latent columns a wave sums (latents of up to 512 numbers)
+    constexpr bool WHOLE = RANK > 0;                 // every wave has that many
     extern __shared__ __align__(16) unsigned char lm_smem[];
     const int D = rank + rot, dc = D / 32, ldk = D + 8, ldt = LM_KEYS + 4;
     bf16_t* sk = (bf16_t*)lm_smem;                   // [32 keys][D + 8]: rows as they lie in the cache
@@ -823,9 +825,13 @@ extern "C" int tl_latent_attention(const void* q, int q_ld, void* out, const voi
         int rc;
 #define TL_LM_AS(RB, RANK, ROT) rc = launch_lm<RB, RANK, ROT>(q, q_ld, out, plane, block_table, bt_stride, req_indptr, ctx_lens, tile_req, tile_tok0, num_tiles, tile_tokens, \
                                      heads, rank, rot, page_size, scale, sink, splits, part_o, part_ml, window, gate, gate_ld, stream)
-#define TL_LM(RB) if (rank == 512 && rot == 64) TL_LM_AS(RB, 512, 64); else if (rank == 512 && rot == 0) TL_LM_AS(RB, 512, 0); else TL_LM_AS(RB, 0, 0)
-        if (tile_rows <= 16) { TL_LM(1); } else if (tile_rows <= 32) { TL_LM(2); } else { TL_LM(4); }
+#define TL_LM_ROT(RB, ROT) switch (rank) { \
+        case 64: TL_LM_AS(RB, 64, ROT); break; case 128: TL_LM_AS(RB, 128, ROT); break; case 192: TL_LM_AS(RB, 192, ROT); break; case 256: TL_LM_AS(RB, 256, ROT); break; \
+        case 320: TL_LM_AS(RB, 320, ROT); break; case 384: TL_LM_AS(RB, 384, ROT); break; case 448: TL_LM_AS(RB, 448, ROT); break; default: TL_LM_AS(RB, 512, ROT); }
+#define TL_LM(RB) if (rank % 64 != 0 || rot > 64) { TL_LM_AS(RB, 0, 0); } else if (rot == 0) { TL_LM_ROT(RB, 0) } else if (rot == 32) { TL_LM_ROT(RB, 32) } else { TL_LM_ROT(RB, 64) }
+        if (tile_rows <= 16) { TL_LM(1) } else if (tile_rows <= 32) { TL_LM(2) } else { TL_LM(4) }
 #undef TL_LM
+#undef TL_LM_ROT
 #undef TL_LM_AS
         if (rc != TL_OK) return rc;
         if (splits > 1) {
