@@ -28,3 +28,14 @@ def test_tiles_of_products_with_few_rows(lib, M, N, K, gated, ahead):
     rows, columns, slabs = c_int(), c_int(), c_int()
     lib.tl_gemm_direct_choice(c_int(M), c_int(N), c_int(K), c_int(gated), ctypes.byref(rows), ctypes.byref(columns), ctypes.byref(slabs))
     assert (rows.value, columns.value) in ahead
+
+
+# 0: rings of slabs, 1: the few-rows kernel that fetches into registers, 2: tiles; sizes on both sides of each line, measured 4 % and more apart
+@pytest.mark.parametrize("M, N, K, gated, want", [
+    (1, 32768, 768, 0, 0), (1, 152064, 3584, 0, 1), (8, 152064, 3584, 0, 0), (9, 152064, 3584, 0, 2), (16, 32768, 64, 0, 0),
+    (32, 24576, 64, 0, 0), (24, 28672, 128, 0, 2), (32, 27648, 1024, 0, 2), (32, 27648, 2048, 0, 0), (17, 32832, 4096, 0, 2),
+    (64, 8192, 64, 0, 0), (56, 32000, 128, 0, 2), (48, 16384, 768, 0, 2), (64, 20480, 256, 0, 2), (33, 24576, 2048, 0, 0), (64, 27648, 5120, 0, 2), (64, 29392, 6848, 0, 2), (40, 32768, 4096, 0, 0),
+    (8, 20480, 256, 1, 1), (1, 20480, 768, 1, 0), (8, 20480, 1024, 1, 0), (16, 16384, 64, 1, 0), (32, 12288, 64, 1, 0), (32, 13312, 4096, 1, 2), (64, 8192, 64, 1, 0), (48, 10240, 192, 1, 2),
+    (64, 12288, 1536, 1, 2), (33, 12288, 2048, 1, 0)])
+def test_few_rows_go_where_they_were_faster(lib, M, N, K, gated, want):
+    assert lib.tl_gemm_few_rows_choice(c_int(M), c_int(N), c_int(K), c_int(gated)) == want

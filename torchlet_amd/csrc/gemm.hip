@@ -1160,10 +1160,26 @@ static bool ring_fits(const void* x, const void* w, int M, int K, int ldx) {
     return M > 0 && M <= 64 && K % 64 == 0 && ldx % 8 == 0 && K < (1 << 23) && ldx < (1 << 23) && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0;
 }
 
-// Where a product of up to 64 rows goes through the rings: against the tile kernel and, one row, the few-rows kernel that fetches into registers (us, the other / this):
-// 64 rows, 2048 x 2048 8.5 / 6.0, 18432 x 4096 48 / 39, 32000 x 2048 34.2 / 33.9, 152064 x 3584 214 / 254 (the tiles' work-groups share what they fetch of x);
-// 12 rows, 152064 x 3584 190 / 194, 8 rows 197 / 187, 1 row 175 / 183, 1 row, 32000 x 4096 42.5 / 42.8.
-static bool ring_pays(int M, long columns) { return M <= 64 && (columns <= 32768 || (M >= 2 && M <= 8)); }
+// Where a product of up to 64 rows goes through the rings, K a multiple of 64: measured against what it took before them, the tiles or the few-rows kernel that fetches into registers, over a grid
+// of widths and depths (us, the other / this).
+//   Up to 16 rows up to 32768 columns, 2 to 8 rows any number: 12 rows, 152064 x 3584 190 / 194, 8 rows 197 / 187, 1 row 179 / 187, 2 rows 151936 x 896 53 / 50.
+//   17 to 32 rows up to 24576, deep ones up to 32768 (32 rows: 24576 x 1024 13.8 / 11.9, 28672 x 256 6.1 / 7.6, 27648 x 1024 14.3 / 15.9, x 2048 28.4 / 25.4).
+//   33 to 64 rows fetch as much of x as of the weights, and the tiles' work-groups share it: up to 8192 columns (64 rows, 2048 x 2048 8.5 / 6.0, 8192 x 1024 8.2 / 6.7, x 256 4.4 / 4.2), up to 24576
+//   where K is deep (18432 x 4096 48 / 39, 24576 x 2048 28.5 / 25.4, 16384 x 1024 9.5 / 10.6, 24576 x 256 6.4 / 8.2), with rows of weights multiples of 4 KB apart, whose order the rings turn,
+//   up to 32768 (30000 x 4096 55.6 / 54.0, x 5120 64 / 72).
+static bool ring_pays(int M, long columns, int K) {
+    if (M <= 16) return columns <= 32768 || (M >= 2 && M <= 8);
+    if (M <= 32) return columns <= 24576 || (columns <= 32768 && K >= 2048);
+    return M <= 64 && (columns <= 8192 || (K >= 2048 && (columns <= 24576 || (columns <= 32768 && K % 2048 == 0))));
+}
+
+// The same for a fused gate, `outputs` of which there are (us, the other / this): up to 16 rows but for wide and shallow ones, where the few-rows kernel's work-groups walk many strips each (8 rows,
+// 20480 outputs, K 256 7.5 / 8.8, 768 14.1 / 14.8, 1536 25.7 / 23.7; one row, K 768 15.4 / 14.6); 17 to 32 rows up to 12288 outputs (32 rows, 11264 x 4096 46 / 34, 18944 x 3584 50 / 52); 33 to 64
+// rows up to 8192, deep ones up to 12288 (64 rows: 8192 x 512 9.1 / 7.2, 11264 x 4096 47 / 44, x 1024 14.8 / 16.5, 12288 x 256 7.2 / 9.4).
+static bool ring_pays_gated(int M, int outputs, int K) {
+    if (M <= 16) return M == 1 || outputs <= 16384 || K >= 1024;
+    return M <= 64 && (outputs <= (M <= 32 ? 12288 : 8192) || (outputs <= 12288 && K >= 2048));
+}
 
 struct RingCall {
     const void *x, *w, *bias;
@@ -1216,6 +1232,13 @@ static int launch_ring(const RingCall& c, hipStream_t stream, RingPlan p = RingP
         return launch_ring_x<8, TOut, SW, END>(c, p, stream);
     }
     TL_REQUIRE(false, "gemm_ring: too many rows (%d)", c.M);
+}
+
+// Which kernel a bfloat16 product of aligned operands and up to 64 rows gets, K a multiple of 64 (for tests): 0 the rings, 1 the few-rows kernel that fetches into registers, 2 tiles.
+// `gated`: N outputs of the fused gate.
+extern "C" int tl_gemm_few_rows_choice(int M, int N, int K, int gated) {
+    if (gated) return ring_pays_gated(M, N, K) ? 0 : M <= 16 ? 1 : 2;
+    return ring_pays(M, N, K) ? 0 : M > 8 ? 2 : 1;
 }
 
 // One shape of the kernel above (for tests and tuning): 8 wj weight rows a work-group (with `gate`, 1 + the gate's number, half gate and half up rows), `rows` outputs of which
@@ -1719,7 +1742,7 @@ static bool skinny_fits(const void* x, const void* w, int M, int K, int ldx) {
 
 // out = x w^T (+ bias) in the engine's dtype: picks the kernel for the shape.
 //   bfloat16, aligned, K a multiple of 64:
-//     up to 64 rows against up to 32768 columns, 2 to 8 rows against more -> gemm_ring (see ring_pays)
+//     up to 64 rows as ring_pays says -> gemm_ring
 //     one row against more        -> gemm_skinny (matrix cores, weight streaming)
 //     everything else             -> gemm_dl_tile (matrix cores, operands straight into shared memory)
 //   bfloat16, aligned, other K, M <= 64 -> gemm_skinny, except that 33..64 rows against a wide matrix go to the tile kernel
@@ -1732,7 +1755,7 @@ extern "C" int tl_gemm(const void* x, const void* w, const void* bias, int bias_
     TL_REQUIRE(M >= 0 && N > 0 && K > 0 && ldx >= K && ldo >= N, "gemm: bad sizes M=%d N=%d K=%d ldx=%d ldo=%d", M, N, K, ldx, ldo);
     if (M == 0) return TL_OK;
     const bool aligned = K % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0;
-    if (dtype == TL_DT_BF16 && ring_fits(x, w, M, K, ldx) && ring_pays(M, N)) {
+    if (dtype == TL_DT_BF16 && ring_fits(x, w, M, K, ldx) && ring_pays(M, N, K)) {
         const RingCall c{x, w, bias, bias_f32, out, M, N, K, ldx, ldo, 0};
         return out_f32 ? launch_ring<float, 0, END_STORE>(c, stream) : launch_ring<bf16_t, 0, END_STORE>(c, stream);
     }
@@ -1848,7 +1871,7 @@ extern "C" int tl_gemm_token_gate(const void* x, const void* w, const void* ids,
                                   hipStream_t stream) {
     TL_REQUIRE(M > 0 && N > 0 && K > 0 && ldx >= K && ldo >= N && table_ld >= N && vocab > 0 && ids && table, "gemm_token_gate: bad sizes M=%d N=%d K=%d", M, N, K);
     TL_REQUIRE(known_activation(act) && !(act & ACT_PAIRS), "gemm_token_gate: unknown activation %d", act);
-    if (M > 16 || !ring_fits(x, w, M, K, ldx) || !ring_pays(M, N)) return TL_NOT_FUSED;
+    if (M > 16 || !ring_fits(x, w, M, K, ldx) || !ring_pays(M, N, K)) return TL_NOT_FUSED;
     RingCall c{x, w, nullptr, 0, out, M, N, K, ldx, ldo, 0};
     c.tk = TokenRow{(const int*)ids, (const bf16_t*)table, table_ld, vocab, act};
     return launch_ring<bf16_t, 0, END_TOKEN>(c, stream);
@@ -1928,10 +1951,8 @@ static int gemm_gated(const void* x, const void* w, void* out, int M, int I, int
     const bf16_t* xb = (const bf16_t*)x;
     const bf16_t* wb = (const bf16_t*)w;
     bf16_t* ob = (bf16_t*)out;
-    // through the rings up to 16 rows, up to 64 against up to 24576 rows of the matrix (us, tiles / rings: 32 rows, 22528 x 4096 46 / 34, 27648 x 5120 51.1 / 51.3,
-    // 37888 x 3584 49.9 / 52.3; 64 rows, 2048 x 2048 15.6 / 6.3, 22528 x 4096 47 / 43, 27648 x 5120 56 / 62)
-    if (ring_fits(x, w, M, K, ldx) && (M <= 16 || N <= 24576)) return launch_ring<bf16_t, GATE, END_STORE>(RingCall{x, w, nullptr, 0, out, M, N, K, ldx, ldo, I}, stream);
-    if (M <= 32 && K % 64 != 0) {
+    if (ring_fits(x, w, M, K, ldx) && ring_pays_gated(M, I, K)) return launch_ring<bf16_t, GATE, END_STORE>(RingCall{x, w, nullptr, 0, out, M, N, K, ldx, ldo, I}, stream);
+    if (M <= 16 || (M <= 32 && K % 64 != 0)) {
         if (M <= 16) launch_skinny_t<1, 1, 16, bf16_t, GATE>(xb, wb, nullptr, 0, ob, M, N, K, ldx, ldo, I, stream);
         else launch_skinny_t<1, 2, 16, bf16_t, GATE>(xb, wb, nullptr, 0, ob, M, N, K, ldx, ldo, I, stream);
     } else if (K % 64 == 0) {
@@ -2066,7 +2087,7 @@ extern "C" int tl_gemm_groups(const void* x, long x_group, const void* w, void* 
     gr.count = groups;
     gr.stride = GroupStride{x_group, (long)N * K, out_group};
     const bool aligned = K % 8 == 0 && ldx % 8 == 0 && x_group % 8 == 0 && out_group % 8 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0;
-    if (dtype == TL_DT_BF16 && x_group % 8 == 0 && ring_fits(x, w, M, K, ldx) && ring_pays(M, (long)N * groups)) {
+    if (dtype == TL_DT_BF16 && x_group % 8 == 0 && ring_fits(x, w, M, K, ldx) && ring_pays(M, (long)N * groups, K)) {
         RingCall c{x, w, nullptr, 0, out, M, N, K, ldx, ldo, 0};
         c.gr = gr;
         return out_f32 ? launch_ring<float, 0, END_STORE>(c, stream) : launch_ring<bf16_t, 0, END_STORE>(c, stream);
@@ -2101,7 +2122,7 @@ extern "C" int tl_gemm_groups_beside(const void* x, long x_group, const void* w,
                                      const void* w2, void* out2, int N2, hipStream_t stream) {
     TL_REQUIRE(groups > 0 && groups <= 64 && M > 0 && N > 0 && N2 > 0 && K > 0 && ldx >= K && ldo >= N && x_group >= 0 && out_group >= 0,
                "gemm_groups_beside: bad sizes groups=%d M=%d N=%d/%d K=%d", groups, M, N, N2, K);
-    if (M > 16 || x_group % 8 || !ring_fits(x, w, M, K, ldx) || !ring_fits(x2, w2, M, K, ldx) || !ring_pays(M, (long)N * groups) || N2 > N) return TL_NOT_FUSED;
+    if (M > 16 || x_group % 8 || !ring_fits(x, w, M, K, ldx) || !ring_fits(x2, w2, M, K, ldx) || !ring_pays(M, (long)N * groups, K) || N2 > N) return TL_NOT_FUSED;
     RingCall c{x, w, nullptr, 0, out, M, N, K, ldx, ldo, 0};
     c.gr.count = groups;
     c.gr.stride = GroupStride{x_group, (long)N * K, out_group};
