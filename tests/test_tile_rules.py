@@ -39,3 +39,14 @@ def test_tiles_of_products_with_few_rows(lib, M, N, K, gated, ahead):
     (64, 12288, 1536, 1, 2), (33, 12288, 2048, 1, 0)])
 def test_few_rows_go_where_they_were_faster(lib, M, N, K, gated, want):
     assert lib.tl_gemm_few_rows_choice(c_int(M), c_int(N), c_int(K), c_int(gated)) == want
+
+
+# a unit's work-groups: 4 requests twice where 8 (a gate's rows up to 8 also 6) would have it to themselves with two slabs on their way; shares of all outputs by equal numbers
+@pytest.mark.parametrize("total, M, halves, even, want", [
+    (16384, 1, 1, 0, (4, 32)), (14336, 16, 1, 0, (4, 28)), (12288, 8, 1, 0, (6, 48)), (8192, 2, 2, 0, (4, 16)), (5120, 8, 2, 0, (4, 10)), (5120, 9, 2, 0, (6, 20)), (8192, 16, 2, 0, (4, 16)),
+    (16384, 17, 1, 0, (8, 64)), (4608, 1, 1, 1, (3, 18)), (16640, 3, 1, 0, (3, 22)), (100, 1, 1, 0, (1, 8)), (13568, 8, 1, 1, (4, 28))])
+def test_shares_of_the_rings(lib, total, M, halves, even, want):
+    wj, rows = c_int(), c_int()
+    lib.tl_gemm_ring_plan(c_int(total), c_int(M), c_int(halves), c_int(256), c_int(even), ctypes.byref(wj), ctypes.byref(rows))
+    assert (wj.value, rows.value) == want
+    assert rows.value <= 8 * wj.value // halves and (not even or rows.value % 2 == 0)

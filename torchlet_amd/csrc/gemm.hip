@@ -1241,6 +1241,13 @@ extern "C" int tl_gemm_few_rows_choice(int M, int N, int K, int gated) {
     return ring_pays(M, N, K) ? 0 : M > 8 ? 2 : 1;
 }
 
+// The plan of a whole product through the rings (for tests): `halves` 2 for the fused gate.
+extern "C" void tl_gemm_ring_plan(int total, int M, int halves, int units, int even, int* wj, int* rows) {
+    const RingPlan p = plan_ring(total, M, halves, units, even != 0);
+    *wj = p.wj;
+    *rows = p.rows;
+}
+
 // One shape of the kernel above (for tests and tuning): 8 wj weight rows a work-group (with `gate`, 1 + the gate's number, half gate and half up rows), `rows` outputs of which
 // are used; parts > 1: K split into ranges of k_per columns, float slabs.  wj 0: as the dispatch would.
 extern "C" int tl_gemm_ring_variant(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int N, int K, int ldx, int ldo, int out_f32, int gate, int wj,

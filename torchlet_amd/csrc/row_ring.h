@@ -140,24 +140,32 @@ struct RingPlan {
     int wj, rows;
 };
 
-// `units` compute units share `total` outputs: the shape with the least of (rounds of work-groups) x (rows a work-group draws, x's among them, and a third of eight rows for its
-// start and end), then equal shares for all work-groups of these rounds: a launch is as slow as its busiest unit (4608 rows at 18 a unit 8.0 us, at 24 8.6, at
-// 16 and two rounds 9.3).  No fewer than eight rows: one request fetches as many.
+// `units` compute units share `total` outputs: the shape with the least of (rounds of work-groups) x (requests of a work-group's weights, half of x's, which other work-groups have fetched into
+// the caches as well, and a third of one for its start and end), then equal shares for all work-groups of these rounds: a launch is as slow as its busiest unit (4608 rows at 18 a unit 8.0 us, at
+// 24 8.6, at 16 and two rounds 9.3).  No fewer than eight rows: one request fetches as many.
+// A shape of six or eight requests has two slabs on its way, 56 to 80 KB, and with one work-group a unit that is all.  Up to 16 rows of x, where eight requests would fill a unit, two work-groups
+// of four share it with 144 or 160 KB on their way; up to 8 rows of x also in a gate's place of six (us, one row: 16384 x 768 7.0 -> 6.7, x 2048 15.5 -> 13.6; gates, two rows: 8192 x 768
+// 7.7 -> 7.1, x 3584 23.0 -> 22.4, 5120 x 768 5.7 -> 5.6; 16 rows, 5120 x 3584 15.5 -> 16.3, 8192 x 3584 22.9 -> 22.5).
 static RingPlan plan_ring(int total, int M, int halves, int units, bool even) {
-    const int xh = M <= 8 ? 1 : M <= 16 ? 2 : M <= 32 ? 4 : 8;
+    const int xh = M <= 8 ? 1 : M <= 16 ? 2 : M <= 32 ? 4 : 8, floor = 8 / halves;
     if (units < 1) units = 1;
+    auto share = [&](long groups, long per) {
+        int rows = (int)((total + groups - 1) / groups);
+        if (even) rows += rows & 1;
+        return rows < floor ? floor : rows > per ? (int)per : rows;
+    };
     RingPlan best{0, 0};
     double least = 1e30;
+    long best_rounds = 0;
     for (int wj : {1, 2, 3, 4, 6, 8}) {
         if (wj % halves) continue;
         const long per = 8 * wj / halves, rounds = ((total + per - 1) / per + units - 1) / units;
         const double cost = rounds * (wj + 0.5 * xh + 0.3);
         if (cost >= least) continue;
         least = cost;
-        const long groups = rounds * units;
-        int rows = (int)((total + groups - 1) / groups), floor = 8 / halves;
-        if (even) rows += rows & 1;
-        best = RingPlan{wj, rows < floor ? floor : rows > per ? (int)per : rows};
+        best_rounds = rounds;
+        best = RingPlan{wj, share(rounds * units, per)};
     }
+    if (best_rounds == 1 && (best.wj == 8 ? xh <= 2 : best.wj == 6 && xh == 1 && halves == 2)) best = RingPlan{4, share(2L * units, 32 / halves)};
     return best;
 }
