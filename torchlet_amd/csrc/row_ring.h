@@ -36,7 +36,8 @@ struct RingShape {
 // not notice which of the two served it): slab s belongs to sum s % 8, so a wave keeps two sets, and lane group g holds the columns 16 g .. + 15 of a slab.
 //
 // `spread`: the weight rows lie a multiple of 4 KB apart.  Work-groups in step then ask the same few channels of the memory for all their rows, so they begin at different
-// slabs; this order spreads both neighbours and the work-groups of an XCD (us, in step -> spread: 16 rows, 8144 x 4096 16.3 -> 13.7, 32000 x 4096 48 -> 41, 4096 x 16384
+// slabs: 5 b + b / 8 spreads both neighbours and the work-groups of an XCD (over 88 sizes by 1, 8 and 16 rows 1.018 of the best of seven such rules on average, 1.12 at most; b + b / 8 1.028 and
+// 1.45: 4608 x 4096, one row, 11.6 -> 9.2, where the kernel before took 10.1) (us, in step -> spread: 16 rows, 8144 x 4096 16.3 -> 13.7, 32000 x 4096 48 -> 41, 4096 x 16384
 // 33 -> 22, 11264 x 2048 10.9 -> 9.9; with other pitches, 4608 x 3584 8.1 -> 8.5, 2048 x 5632 8.4 -> 8.4).  With few slabs a wave has them all on their way from the
 // start, and 4096 columns by 1024 of K took 8.3 instead of 7.6.
 template <int WJ, int XH, int HALVES>
@@ -47,7 +48,7 @@ __device__ __forceinline__ void ring_products(const bf16_t* w, const unsigned (&
     char* own = ring + wave * (D * S::SLOT);
     const unsigned own_at = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)((void __attribute__((address_space(3)))*)own));
     const int mine = slabs > wave ? (slabs - wave + NW - 1) / NW : 0;
-    const int from = spread && mine >= 8 ? (int)((blockIdx.x + blockIdx.x / 8) % (unsigned)mine) : 0;
+    const int from = spread && mine >= 8 ? (int)((5 * blockIdx.x + blockIdx.x / 8) % (unsigned)mine) : 0;
     auto request = [&](int i) {
         const int turned = i + from < mine ? i + from : i + from - mine;
         const int k = 64 * (wave + turned * NW);
