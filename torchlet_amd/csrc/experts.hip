@@ -323,7 +323,7 @@ experts_ring_kernel(const bf16_t* __restrict__ a, int a_ld, const int* __restric
         const int r = 8 * j + lane / 8, c = (lane % 8) ^ ((r >> 1) & 7);
         woff[j] = (unsigned)((min(n0 + r, n_end - 1) - n0) * K + c * 8) * 2;
     }
-    ring_products<WJ, XH, 1>(w + ((size_t)tile.g * N + n0) * K, woff, a, xoff, K / 64, ring, wave, K % 2048 == 0);
+    ring_products<WJ, XH, 1>(w + ((size_t)tile.g * N + n0) * K, woff, a, xoff, K / 64, ring, wave, ring_spread(K));
     const int base_act = act & ~ACT_PAIRS;
     for (int q = wave; q < S::SH * S::MT; q += S::NW) {
         const int s = q / S::MT, t = q % S::MT, m = tile.m0 + 16 * t + li, n = n0 + 16 * s + 4 * kg;

@@ -615,9 +615,10 @@ struct NormArgs {
     size_t part_stride;
     int parts, weight_f32;
     float eps;
+    int share, strips, shares;      // TURN: see gemm_skinny_kernel
 };
 
-template <int R, int MT, int KS, typename TOut, int SW = 0, bool XL = false, int D = 2, bool RP = false, bool NF = false>
+template <int R, int MT, int KS, typename TOut, int SW = 0, bool XL = false, int D = 2, bool RP = false, bool NF = false, bool TURN = false>
 __global__ __launch_bounds__(KS * 64) void gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                               const void* __restrict__ bias, int bias_f32,
                                                               TOut* __restrict__ out, int M, int N, int K, int ldx, int ldo,
@@ -659,17 +660,31 @@ __global__ __launch_bounds__(KS * 64) void gemm_skinny_kernel(const bf16_t* __re
     // their 32 up rows), and the sums of both meet in shared memory.
     constexpr int KW = SW ? KS / 2 : KS;       // waves along K per strip
     const int kwave = SW ? wave % KW : wave;
+    static_assert(!TURN || (NF && !SW && KS == 8), "the rings' order is kept by eight waves along K");
+    // The columns that step i of this wave begins at.  TURN: in the order in which gemm_ring_kernel takes them, which begins elsewhere in each of its work-groups (its wave v takes slabs v, v + 4,
+    // ... from its start on, for two sums in turn: those are this kernel's waves v and v + 4).
+    const int per_wave = K / 256;
+    int from = 0;                              // (of the strip at hand)
+    auto step_at = [&](int i) {
+        if (!TURN) return 64 * (kwave + i * KW);
+        const int t = (kwave >> 2) + 2 * i + from;
+        return 64 * ((kwave & 3) + 4 * (t < per_wave ? t : t - per_wave));
+    };
     const int total = SW ? out_cols : N;
     const int rps = rows_per_strip > 0 ? rows_per_strip : 16 * R;
     const int run_begin = blockIdx.x * ((XL && rows_per_group > 0) ? rows_per_group : rps);
     const int run_end = min(total, run_begin + ((XL && rows_per_group > 0) ? rows_per_group : rps));
-    auto strip_begin = [&](int i) { return run_begin + i * rps; };
-    auto strip_end = [&](int i) { return min(run_begin + i * rps + rps, run_end); };
+    // TURN: the run is na.shares of what gemm_ring_kernel's work-groups have each (na.share outputs), every one of them na.strips strips; the strip's number is then 256 times the share's and its own in it
+    auto strip_begin = [&](int i) { return TURN ? run_begin + (i >> 8) * na.share + (i & 255) * rps : run_begin + i * rps; };
+    auto strip_end = [&](int i) { return min(TURN ? min(strip_begin(i) + rps, run_begin + ((i >> 8) + 1) * na.share) : run_begin + i * rps + rps, run_end); };
+    auto strip_after = [&](int i) { return !TURN || (i & 255) + 1 < na.strips ? i + 1 : (i | 255) + 1; };
+    auto turn_to = [&](int i) { if (TURN) from = ring_start(blockIdx.x * na.shares + (i >> 8), per_wave); };
     auto lane_row = [&](int i, int r) {        // the weight row this lane fetches for block r of strip i
         const int o = min(strip_begin(i) + r * 16 + li, strip_end(i) - 1);
         return SW ? (o >> 5) * 64 + (wave / KW) * 32 + (o & 31) : o;
     };
     int strip = 0;
+    turn_to(strip);
     int rp_pos = 0, rp_page = 0;               // RP: this lane's row (li), fetched now, used in the epilogue
     if (RP) {
         const int row = min(li, M - 1);
@@ -696,7 +711,7 @@ __global__ __launch_bounds__(KS * 64) void gemm_skinny_kernel(const bf16_t* __re
     Frag16 wa0[D][R], wa1[D][R], wb0[D][MT], wb1[D][MT];
 #define SK_ISSUE(d, i)                                                                              \
     {                                                                                               \
-        const int k_ = 64 * (kwave + (i) * KW) + SK_KOFF(lg);                                       \
+        const int k_ = step_at(i) + SK_KOFF(lg);                                                    \
         _Pragma("unroll") for (int r = 0; r < R; ++r) {                                             \
             wa0[d][r].u = SK_LOAD(wrow[r] + k_);                                                    \
             wa1[d][r].u = SK_LOAD(wrow[r] + k_ + SK_SECOND);                                        \
@@ -796,7 +811,7 @@ __global__ __launch_bounds__(KS * 64) void gemm_skinny_kernel(const bf16_t* __re
             for (int d = 0; d < D; ++d) {
                 if (i + d < mine) {
                     if (XL) {
-                        const int k = 64 * (kwave + (i + d) * KW) + SK_KOFF(lg);
+                        const int k = step_at(i + d) + SK_KOFF(lg);
 #pragma unroll
                         for (int t = 0; t < MT; ++t) {
                             wb0[d][t].u = *(const uint4*)(&xs[xoff[t] + k]);
@@ -847,10 +862,12 @@ __global__ __launch_bounds__(KS * 64) void gemm_skinny_kernel(const bf16_t* __re
                     acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[r].v, b1[t].v, acc[r][t], 0, 0, 0);
                 }
         }
-        const bool more = XL && strip_begin(strip + 1) < run_end;   // without the copy of x: one strip per work-group
+        const int next = strip_after(strip);
+        const bool more = XL && strip_begin(next) < run_end;        // without the copy of x: one strip per work-group
         if (more) {                            // the next strip's first steps, before this strip's sums
 #pragma unroll
-            for (int r = 0; r < R; ++r) wrow[r] = w + (size_t)lane_row(strip + 1, r) * ldw;
+            for (int r = 0; r < R; ++r) wrow[r] = w + (size_t)lane_row(next, r) * ldw;
+            turn_to(next);
 #pragma unroll
             for (int d = 0; d < D; ++d)
                 if (d < mine) SK_ISSUE(d, d)
@@ -922,7 +939,7 @@ __global__ __launch_bounds__(KS * 64) void gemm_skinny_kernel(const bf16_t* __re
             }
         }
         if (!more) break;
-        ++strip;
+        strip = next;
         if (KS > 1) lds_barrier();             // the sums are read until here; the next strip's overwrite them
     }
 #undef SK_ISSUE
@@ -936,6 +953,12 @@ struct StripPlan {
     int groups, per_group, per_strip;
 };
 
+// A run of outputs in equal strips of at most `cap` (a multiple of 16; `even`: of an even number).
+static int equal_strips(int run, int cap, bool even) {
+    const int count = (run + cap - 1) / cap, rows = (run + count - 1) / count;
+    return even ? rows + (rows & 1) : rows;
+}
+
 // Equal runs for up to `most` work-groups, each walked in equal strips of at most `cap` outputs (a multiple of
 // 16); `even` keeps both numbers even (the fused rotation turns pairs of neighbouring outputs).
 static StripPlan plan_strips(int total, int most, int cap, bool even) {
@@ -943,9 +966,7 @@ static StripPlan plan_strips(int total, int most, int cap, bool even) {
     p.per_group = (total + most - 1) / most;
     if (p.per_group < 4) p.per_group = 4;                     // a strip of fewer rows wastes most of its fetches
     if (even) p.per_group += p.per_group & 1;
-    const int count = (p.per_group + cap - 1) / cap;
-    p.per_strip = (p.per_group + count - 1) / count;
-    if (even) p.per_strip += p.per_strip & 1;
+    p.per_strip = equal_strips(p.per_group, cap, even);
     p.groups = (total + p.per_group - 1) / p.per_group;
     return p;
 }
@@ -1113,7 +1134,7 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict
         const int r = 8 * (WJ + j) + lane / 8, c = (lane % 8) ^ ((r >> 1) & 7);
         xoff[j] = (unsigned)(min(r - 8 * WJ, M - 1) * ldx + c * 8) * 2;
     }
-    ring_products<WJ, XH, HALVES>(w + (size_t)row_of(n0) * ldw, woff, x, xoff, K / 64, ring, wave, ldw % 2048 == 0);
+    ring_products<WJ, XH, HALVES>(w + (size_t)row_of(n0) * ldw, woff, x, xoff, K / 64, ring, wave, ring_spread(ldw));
     const bool quads = ldo % 4 == 0 && n0 % 4 == 0 && ((uintptr_t)out % (4 * sizeof(TOut))) == 0;
     for (int q = wave; q < S::SH * S::MT; q += S::NW) {
         const int s = q / S::MT, t = q % S::MT, m = 16 * t + li, n = n0 + 16 * s + 4 * kg;
@@ -1224,7 +1245,7 @@ static int launch_ring_x(const RingCall& c, RingPlan p, hipStream_t stream) {
 // `p.wj` 0: the plan is made here.
 template <typename TOut, int SW, int END>
 static int launch_ring(const RingCall& c, hipStream_t stream, RingPlan p = RingPlan{0, 0}) {
-    if (p.wj == 0) p = plan_ring(SW ? c.out_cols : c.N, c.M, SW ? 2 : 1, TL_COMPUTE_UNITS / (c.parts * c.gr.count), END == END_ROTATE);
+    if (p.wj == 0) p = plan_ring(SW ? c.out_cols : c.N, c.M, SW ? 2 : 1, TL_COMPUTE_UNITS / (c.parts * c.gr.count), END == END_ROTATE, ring_spread(c.K));
     if (c.M <= 8) return launch_ring_x<1, TOut, SW, END>(c, p, stream);
     if (c.M <= 16) return launch_ring_x<2, TOut, SW, END>(c, p, stream);
     if constexpr (END == END_STORE) {
@@ -1242,8 +1263,8 @@ extern "C" int tl_gemm_few_rows_choice(int M, int N, int K, int gated) {
 }
 
 // The plan of a whole product through the rings (for tests): `halves` 2 for the fused gate.
-extern "C" void tl_gemm_ring_plan(int total, int M, int halves, int units, int even, int* wj, int* rows) {
-    const RingPlan p = plan_ring(total, M, halves, units, even != 0);
+extern "C" void tl_gemm_ring_plan(int total, int M, int K, int halves, int units, int even, int* wj, int* rows) {
+    const RingPlan p = plan_ring(total, M, halves, units, even != 0, ring_spread(K));
     *wj = p.wj;
     *rows = p.rows;
 }
@@ -1833,7 +1854,7 @@ extern "C" int tl_gemm_rope(const void* x, const void* w, const void* bias, int 
                "gemm_rope: the cache write needs both planes, the block table and the requests of the rows");
     TL_REQUIRE(N == (q_heads + (k_plane ? 2 * kv_heads : 0)) * head_dim, "gemm_rope: %d output columns do not match the heads", N);
     const int strips = (N + 15) / 16, ks = strips >= 1024 ? 16 : 8;
-    const bool rings = ring_fits(x, w, M, K, ldx);
+    const bool rings = ring_fits(x, w, M, K, ldx) && ks == 8;      // (ks 16: as tl_gemm_rope_normed sums there)
     // (from 9 rows on the product split over K plus the rotation kernel that adds its slabs up stands beside it where that split is to be had)
     if (M > 16 || (M > 8 && tl_gemm_partials_pay(M, N, K)) || !skinny_fits(x, w, M, K, ldx) || N % 16 || ldo % 4 || ((uintptr_t)out % 8) || (!rings && K / 64 / ks >= 16) ||
         (k_plane && (((uintptr_t)k_plane % 8) || head_dim % 4)))
@@ -1868,8 +1889,18 @@ static NormArgs norm_args(const void* residual, void* residual_out, const void* 
                           const void* weight, int weight_f32, float eps) {
     NormArgs na;
     na.residual = (const float*)residual; na.residual_out = (float*)residual_out; na.pending = pending;
-    na.weight = weight; na.part_stride = (size_t)part_stride; na.parts = parts; na.weight_f32 = weight_f32; na.eps = eps;
+    na.weight = weight; na.part_stride = (size_t)part_stride; na.parts = parts; na.weight_f32 = weight_f32; na.eps = eps; na.share = na.strips = na.shares = 0;
     return na;
+}
+
+// The work-groups of a projection of one row that keeps the order of gemm_ring_kernel's, whose work-groups have `share` outputs each: up to two to a compute unit, for as many shares each.  Returns
+// the outputs of a strip (see equal_strips).
+static int keep_shares(NormArgs& na, int share, int total) {
+    const int rows = equal_strips(share, 32, true), count = (total + share - 1) / share;
+    na.share = share;
+    na.strips = (share + rows - 1) / rows;
+    na.shares = (count + 2 * TL_COMPUTE_UNITS - 1) / (2 * TL_COMPUTE_UNITS);
+    return rows;
 }
 
 // out[m, n] = act((x w^T)[m, n]) * table[ids[m], n] of up to 16 rows in bfloat16, the product and what follows in float (a row whose id is no row of the table keeps what it
@@ -1899,7 +1930,7 @@ extern "C" int tl_gemm_rope_normed(const void* residual, void* residual_out, con
     TL_REQUIRE((k_plane == nullptr) == (v_plane == nullptr) && (!k_plane || (token_req && block_table && page > 0 && bt_stride > 0)),
                "gemm_rope_normed: the cache write needs both planes, the block table and the request of the row");
     TL_REQUIRE(N == (q_heads + (k_plane ? 2 * kv_heads : 0)) * head_dim, "gemm_rope_normed: %d output columns do not match the heads", N);
-    const NormArgs na = norm_args(residual, residual_out, pending, parts, part_stride, norm_weight, norm_weight_f32, eps);
+    NormArgs na = norm_args(residual, residual_out, pending, parts, part_stride, norm_weight, norm_weight_f32, eps);
     const int strips = (N + 15) / 16, ks = strips >= 1024 ? 16 : 8;
     if (!norm_fits(na, K, ks * 64) || ((uintptr_t)w % 16) || N % 16 || ldo % 4 || ((uintptr_t)out % 8) || K / 64 / ks >= 16 ||
         (k_plane && (((uintptr_t)k_plane % 8) || head_dim % 4)))
@@ -1909,15 +1940,20 @@ extern "C" int tl_gemm_rope_normed(const void* residual, void* residual_out, con
     ra.block_table = (const int*)block_table; ra.k_plane = (bf16_t*)k_plane; ra.v_plane = (bf16_t*)v_plane;
     ra.bt_stride = bt_stride; ra.page = page > 0 ? page : 1; ra.q_heads = q_heads; ra.kv_heads = k_plane ? kv_heads : 0; ra.head_dim = head_dim;
     int blocks = 1;
-    const int rows = ks == 8 ? balanced_rows(N, &blocks) : 0;
-    dim3 grid(rows > 0 ? (N + rows - 1) / rows : strips);
+    int rows = ks == 8 ? balanced_rows(N, &blocks) : 0, run = 0;
+    if (ks == 8 && ring_spread(K)) {             // shares as tl_gemm_rope deals them (see ring_products), in equal strips of up to two blocks: the same bits, and with rows of weights a multiple of
+                                                 // 4 KB apart the order is as good here (us, in step / turned: 2560 x 2048 7.6 / 7.8, 6144 x 4096 16.6 / 16.1, 9216 x 2048 19.9 / 15.4)
+        rows = keep_shares(na, plan_ring(N, 1, 1, TL_COMPUTE_UNITS, true, true).rows, N);
+        blocks = rows > 16 ? 2 : 1;
+        run = na.shares * na.share;
+    }
+    dim3 grid(run > 0 ? (N + run - 1) / run : rows > 0 ? (N + rows - 1) / rows : strips);
     const size_t lds = (size_t)ks * blocks * 1024 + (size_t)(K + 8) * 2;
-    if (rows > 0 && blocks == 2)
-        gemm_skinny_kernel<2, 1, 8, bf16_t, false, true, 2, true, true><<<grid, dim3(8 * 64), lds, stream>>>(
-            nullptr, (const bf16_t*)w, bias, bias_f32, (bf16_t*)out, 1, N, K, K, ldo, 0, 0, rows, 0, ra, na, GroupStride{});
-    else if (ks == 8)
-        gemm_skinny_kernel<1, 1, 8, bf16_t, false, true, 2, true, true><<<grid, dim3(8 * 64), lds, stream>>>(
-            nullptr, (const bf16_t*)w, bias, bias_f32, (bf16_t*)out, 1, N, K, K, ldo, 0, 0, rows, 0, ra, na, GroupStride{});
+#define TL_NORMED_ROPE(R, TURN) gemm_skinny_kernel<R, 1, 8, bf16_t, false, true, 2, true, true, TURN><<<grid, dim3(8 * 64), lds, stream>>>( \
+            nullptr, (const bf16_t*)w, bias, bias_f32, (bf16_t*)out, 1, N, K, K, ldo, 0, 0, rows, run, ra, na, GroupStride{})
+    if (rows > 0 && blocks == 2) { if (run > 0) TL_NORMED_ROPE(2, true); else TL_NORMED_ROPE(2, false); }
+    else if (ks == 8) { if (run > 0) TL_NORMED_ROPE(1, true); else TL_NORMED_ROPE(1, false); }
+#undef TL_NORMED_ROPE
     else
         gemm_skinny_kernel<1, 1, 16, bf16_t, false, true, 2, true, true><<<grid, dim3(16 * 64), lds, stream>>>(
             nullptr, (const bf16_t*)w, bias, bias_f32, (bf16_t*)out, 1, N, K, K, ldo, 0, 0, 0, 0, ra, na, GroupStride{});

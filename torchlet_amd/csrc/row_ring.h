@@ -32,14 +32,21 @@ struct RingShape {
 // The products of `slabs` slabs: request j of a slab fetches eight rows of 128 bytes at w + woff[j] (x + xoff[j]), bytes, moved on by 128 a slab.  `wave` is uniform.
 // On return every wave's sums lie in its ring (see ring_sum) and all waves have met.
 //
-// Up to 16 rows of x the numbers are summed as gemm_skinny_kernel with eight waves sums them, to the bit (the product that makes its norm itself runs there, and a request must
-// not notice which of the two served it): slab s belongs to sum s % 8, so a wave keeps two sets, and lane group g holds the columns 16 g .. + 15 of a slab.
+// Up to 16 rows of x a product's numbers are summed in one order, whatever their number: slab s belongs to sum s % 8, so a wave keeps two sets, and lane group g holds the columns 16 g .. + 15 of a
+// slab.  gemm_skinny_kernel with eight waves along K sums the same way, to the bit: the query/key/value projection of one row that makes its norm itself runs there, and a request must not notice
+// which of the two served it.  With more rows a wave keeps one set.
 //
-// `spread`: the weight rows lie a multiple of 4 KB apart.  Work-groups in step then ask the same few channels of the memory for all their rows, so they begin at different
-// slabs: 5 b + b / 8 spreads both neighbours and the work-groups of an XCD (over 88 sizes by 1, 8 and 16 rows 1.018 of the best of seven such rules on average, 1.12 at most; b + b / 8 1.028 and
-// 1.45: 4608 x 4096, one row, 11.6 -> 9.2, where the kernel before took 10.1) (us, in step -> spread: 16 rows, 8144 x 4096 16.3 -> 13.7, 32000 x 4096 48 -> 41, 4096 x 16384
-// 33 -> 22, 11264 x 2048 10.9 -> 9.9; with other pitches, 4608 x 3584 8.1 -> 8.5, 2048 x 5632 8.4 -> 8.4).  With few slabs a wave has them all on their way from the
-// start, and 4096 columns by 1024 of K took 8.3 instead of 7.6.
+// `spread`: the weight rows lie a multiple of 4 KB apart.  Work-groups in step then ask the same few channels of the memory for all their rows, so they begin at different slabs (see ring_start) and
+// take them in turn from there.  The order of a sum then hangs on which work-group has the output, so up to 16 rows plan_ring deals such a product out alike whatever their number, and that
+// projection does as it says (the gate of one row that makes its norm itself goes in step and is equal to rounding there: in these orders 18944 x 4096 took 70 us instead of 62).
+// (us, in step -> spread: 16 rows, 8144 x 4096 16.3 -> 13.7, 32000 x 4096 48 -> 41, 4096 x 16384 33 -> 22, 11264 x 2048 10.9 -> 9.9; with other pitches, 4608 x 3584 8.1 -> 8.5, 2048 x 5632
+// 8.4 -> 8.4.  Ranges of 512 columns in four orders, summed by pairs so that it would not hang on the work-group: 8144 x 4096 16.1, 4096 x 16384 34.  With few slabs a wave has them all on their
+// way from the start, and 4096 columns by 1024 of K took 8.3 instead of 7.6.)
+// Where a work-group begins: 5 b + b / 8 spreads neighbours and the work-groups of an XCD (over 88 sizes by 1, 8 and 16 rows 1.018 of the best of seven such rules on average, 1.12 at most; b + b / 8
+// 1.028 and 1.45: 4608 x 4096, one row, 11.6 -> 9.2, 2304 x 8192 1.45 -> 1.12 times the best).
+__host__ __device__ inline bool ring_spread(int pitch) { return pitch % 2048 == 0; }
+__device__ __forceinline__ int ring_start(unsigned group, int slabs_of_a_wave) { return (int)((5 * group + group / 8) % (unsigned)slabs_of_a_wave); }
+
 template <int WJ, int XH, int HALVES>
 __device__ __forceinline__ void ring_products(const bf16_t* w, const unsigned (&woff)[WJ], const bf16_t* x, const unsigned (&xoff)[XH], int slabs, char* ring, int wave, bool spread) {
     using S = RingShape<WJ, XH, HALVES>;
@@ -48,7 +55,7 @@ __device__ __forceinline__ void ring_products(const bf16_t* w, const unsigned (&
     char* own = ring + wave * (D * S::SLOT);
     const unsigned own_at = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)((void __attribute__((address_space(3)))*)own));
     const int mine = slabs > wave ? (slabs - wave + NW - 1) / NW : 0;
-    const int from = spread && mine >= 8 ? (int)((5 * blockIdx.x + blockIdx.x / 8) % (unsigned)mine) : 0;
+    const int from = spread && mine >= 8 ? ring_start(blockIdx.x, mine) : 0;
     auto request = [&](int i) {
         const int turned = i + from < mine ? i + from : i + from - mine;
         const int k = 64 * (wave + turned * NW);
@@ -147,8 +154,9 @@ struct RingPlan {
 // A shape of six or eight requests has two slabs on its way, 56 to 80 KB, and with one work-group a unit that is all.  Up to 16 rows of x, where eight requests would fill a unit, two work-groups
 // of four share it with 144 or 160 KB on their way; up to 8 rows of x also in a gate's place of six (us, one row: 16384 x 768 7.0 -> 6.7, x 2048 15.5 -> 13.6; gates, two rows: 8192 x 768
 // 7.7 -> 7.1, x 3584 23.0 -> 22.4, 5120 x 768 5.7 -> 5.6; 16 rows, 5120 x 3584 15.5 -> 16.3, 8192 x 3584 22.9 -> 22.5).
-static RingPlan plan_ring(int total, int M, int halves, int units, bool even) {
-    const int xh = M <= 8 ? 1 : M <= 16 ? 2 : M <= 32 ? 4 : 8, floor = 8 / halves;
+// `spread` (see ring_products): up to 16 rows the same plan, that of 16.
+static RingPlan plan_ring(int total, int M, int halves, int units, bool even, bool spread) {
+    const int xh = M <= 8 && !spread ? 1 : M <= 16 ? 2 : M <= 32 ? 4 : 8, floor = 8 / halves;
     if (units < 1) units = 1;
     auto share = [&](long groups, long per) {
         int rows = (int)((total + groups - 1) / groups);
