@@ -41,3 +41,17 @@ def test_the_dispatch_around_the_rings(K, slots):
     ops.experts_linear(x, None, w, offsets, got)
     ops.experts_linear(x, None, w, offsets, want, general=True)
     torch.testing.assert_close(got.float(), want.float(), rtol=2.0 ** -7, atol=4 * K * 2.0 ** -24)
+
+
+def test_more_groups_than_a_launch_has_tiles_of_eight_slots():
+    from torchlet_amd.kernels import ops
+    g = torch.Generator().manual_seed(2)
+    G, N, K, slots = 52000, 8, 2048, 4 * 52000
+    w = torch.randn(G, N, K, device="cuda", dtype=torch.bfloat16) / K ** 0.5
+    x, src = torch.randn(64, K, generator=g).bfloat16().cuda(), torch.randint(0, 64, (slots,), generator=g, dtype=torch.int32).cuda()
+    offsets = (4 * torch.arange(G + 1)).int().cuda()
+    got = torch.empty(slots, N, dtype=torch.bfloat16, device="cuda")
+    ops.experts_linear(x, src, w, offsets, got)
+    for e in (0, 1, 43700, 51999):
+        want = x[src[4 * e: 4 * e + 4].long()].double() @ w[e].double().T
+        torch.testing.assert_close(got[4 * e: 4 * e + 4].double(), want, rtol=2.0 ** -8, atol=1e-4)

@@ -431,7 +431,8 @@ static int launch_experts(int which, const ExpertsCall& c, hipStream_t stream) {
 //   16 x 2048 x 1024, 2048 slots 31 / 26 / 22 / 29, 4096 slots 45 / 44 / 39 / 32, 16384 slots 143 / 108 / 96 / 92
 //   32 x 4096 x 4096, 2048 slots 228 / 190 / 190 / 250, 16384 slots 830 / 680 / 587 / 613
 static int pick_experts(const ExpertsCall& c) {
-    if ((long)c.rows <= (c.K < 2048 ? 8L : 12L) * c.groups) return (long)c.rows > 4L * c.groups ? EX_RING_16 : c.K < 2048 ? EX_FEW_4 : EX_RING_8;
+    const bool eights = c.rows / 8 + (c.groups < c.rows ? c.groups : c.rows) <= 65535;      // a launch has that many tiles of 8 slots (experts_fit has counted those of 16)
+    if ((long)c.rows <= (c.K < 2048 ? 8L : 12L) * c.groups) return (long)c.rows > 4L * c.groups ? EX_RING_16 : c.K < 2048 ? EX_FEW_4 : eights ? EX_RING_8 : EX_RING_16;
     static const struct { int kernel, bm, bn, per_unit; double fixed, per_k; } tiles[] = {
         {EX_TILE_64x128, 64, 128, 2, 9e-6, 6.5e-6}, {EX_TILE_128x128, 128, 128, 2, 7e-6, 13e-6},
         {EX_TILE_128x256, 128, 256, 1, 8e-6, 10.2e-6}, {EX_TILE_256x256, 256, 256, 1, 9e-6, 20e-6}};       // seconds of a tile: fixed, and per 1024 columns of K
@@ -450,6 +451,13 @@ static bool experts_fit(const ExpertsCall& c) {
     // (a lane's offset from the first row of x, and of w from its tile's, is kept in 32 bits)
     return c.K % 64 == 0 && c.a_ld % 8 == 0 && ((uintptr_t)c.a % 16) == 0 && ((uintptr_t)c.w % 16) == 0 && (long)c.x_rows * c.a_ld * 2 < (1L << 31) &&
            256L * c.K * 2 < (1L << 31) && (long)(c.rows / 16 + c.groups) <= 65535;
+}
+
+// The kernel that a call of fitting operands gets, by its number (for tests).
+extern "C" int tl_experts_choice(int groups, int rows, int N, int K) {
+    ExpertsCall c{};
+    c.groups = groups; c.rows = rows; c.N = N; c.K = K;
+    return pick_experts(c);
 }
 
 // One kernel of ExpertsKernel by its number (tests cover each; tuning times them).
