@@ -482,8 +482,9 @@ extern "C" int tl_gemm_f32_variant(const void* x, const void* w, const void* bia
 // of which then walks a run of outputs of its own, strip after strip, and requests the first
 // steps of its next strip before it adds up the sums of this one (measured at M = 8, 7B sizes:
 // gate/up 57 -> 51 us, LM head 207 -> 189 us).
-// Needs K % 8 == 0 and 16-byte aligned rows; other shapes go to the general kernel.  With K a multiple of 64 it serves one row against more than 32768 columns and the products that
-// make their norm themselves; gemm_ring_kernel the others.
+// Needs K % 8 == 0 and 16-byte aligned rows; other shapes go to the general kernel.  Products with K a multiple of 64, which the figures here were measured on, are gemm_ring_kernel's by now but for:
+// one row against more than 32768 columns, the products of one row that make their norm themselves, the slabs of one row against up to 4096 columns, projections with their rotation of 16384
+// columns and more, gates of 2 to 16 rows with more than 16384 outputs and K below 1024.  The rules below (balanced_rows, plan_strips, pick_skinny, the copy of x) serve those and every other K.
 #define SK_KOFF(lg) (16 * (lg))     // a lane reads 32 contiguous bytes per step (other splits measured the same)
 #define SK_SECOND 8
 #define SK_LOAD(p) (*(const uint4*)(p))
@@ -1037,7 +1038,7 @@ static int balanced_rows(int N, int* blocks) {
 template <int MT>
 static void pick_skinny(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int N, int K,
                         int ldx, int ldo, int out_f32, hipStream_t stream, Groups gr = Groups{}) {
-    // Measured on MI355X at Qwen2.5-7B sizes (weights streamed from HBM, M = 8 and 64):
+    // Measured on MI355X at Qwen2.5-7B sizes (weights streamed from HBM, M = 8 and 64; K a multiple of 64, which but for one row against many columns the rings take by now):
     // with up to 32 rows one strip of 16 weight rows per work-group is best throughout, with
     // 16 waves along K for wide matrices (gate_up, LM head: 4.7-5.0 TB/s) and 8 for narrow
     // ones (qkv, o, down); with 64 rows the x operand weighs more and several strips per wave
@@ -2027,19 +2028,17 @@ extern "C" int tl_gemm_swiglu(const void* x, const void* w, void* out, int M, in
 // units busy; whoever reads the slabs adds them up.  Returns P through `parts` (the caller sizes
 // `out` for tl_gemm_partials_max()).  More than 64 rows: see plan_dl_split (measured at 512 rows:
 // 3584 x 18944 147 -> 82 us, 5120 x 13824 179 -> 82 us, 5120 x 27648 348 -> 150 us, the norm's sum
-// included).  Up to 64 rows, where it pays (see partials_on_tiles), the rings or, from 33 rows on
+// included).  Up to 64 rows, where it pays (see gives_few_row_slabs), the rings or, from 33 rows on
 // with K below 8192, the direct-load tile kernel with 64 x 64 tiles; for other K the skinny kernel
 // with R = 4 strips per work-group, which share every x fetch.
 extern "C" int tl_gemm_partials_max() { return 8; }
 
-// Whether the tile kernel does the split: from 2 rows on, and for one row where the few-rows kernel
-// has more than 256 strips of 16 weight rows to deal out.  Measured with the consumer's sum left out
-// (us, few-rows kernel against split tiles): 3584 x 3584: 1 row 7.0 / 7.4, 2 rows 8.0 / 7.4, 8 rows 9.1 / 7.5,
-// 16 rows 10.6 / 7.6; 5120 x 5120: 1 row 16.2 / 13.2, 8 rows 19.0 / 12.7, 16 rows 22.5 / 13.1;
-// 3584 x 18944: 1 row 28.2 / 27.2, 8 rows 31.6 / 26.1, 16 rows 38.2 / 26.6; 5120 x 27648, one row: 70.8 / 53
-// (320 strips, one work-group of eight waves with eight steps in flight per compute unit: two rounds,
-// the second nearly empty).
-static bool partials_on_tiles(int M, int N, int K) {
+// Whether a product of up to 64 rows is given in slabs, K dealt to the work-groups of a narrow matrix: from 2 rows on, and for one row against more than 4096 columns on 256 units.  The line was drawn
+// when its other side were the few-rows kernel's strips (3584 x 3584, 8 rows 9.1 / 7.5 us, 5120 x 27648, one row 70.8 / 53).  Between a whole product and slabs through the rings it would lie elsewhere
+// (us with the norm that adds them up, whole / slabs: 2 rows, 3584 x 3584 10.4 / 11.2, 5120 x 5120 15.5 / 16.5, 4096 x 4096 11.1 / 12.9, 3584 x 18944 29.3 / 29.9, 2048 x 5632 10.2 / 10.1; 16 rows,
+// 3584 x 3584 11.3 / 11.6, 4096 x 4096 11.9 / 13.7, 3584 x 18944 33.0 / 31.8; 32 rows, 3584 x 3584 13.0 / 12.6, 3584 x 18944 41 / 31; 64 rows 16.3 / 14.2 and 56 / 35), but what a consumer has read
+// in 32 bits it goes on reading in 32 bits, and a whole product is rounded to bfloat16.
+static bool gives_few_row_slabs(int M, int N, int K) {
     return K % 64 == 0 && (M >= 2 || N > 16 * TL_COMPUTE_UNITS);
 }
 
@@ -2052,7 +2051,7 @@ extern "C" int tl_gemm_partials_parts(int M, int N, int K) {
         const int parts = plan_dl_split(M, N, K).parts;
         return parts > 0 ? parts : 1;
     }
-    if (partials_on_tiles(M, N, K)) {
+    if (gives_few_row_slabs(M, N, K)) {
         const long tiles = (long)((M + 63) / 64) * ((N + 63) / 64);
         int P = (int)(TL_COMPUTE_UNITS / tiles);          // about one work-group per compute unit
         const int by_k = K / 512;                         // at least eight slabs of 64 per part
@@ -2067,7 +2066,7 @@ extern "C" int tl_gemm_partials_parts(int M, int N, int K) {
 
 extern "C" int tl_gemm_partials_pay(int M, int N, int K) {
     if (M > 64 && K % 64 == 0) return gives_slabs(M, N, K);
-    return partials_on_tiles(M, N, K) && tl_gemm_partials_parts(M, N, K) > 1;
+    return gives_few_row_slabs(M, N, K) && tl_gemm_partials_parts(M, N, K) > 1;
 }
 
 extern "C" int tl_gemm_partials(const void* x, const void* w, void* out, int M, int N, int K, int ldx, int* parts,
@@ -2091,9 +2090,9 @@ extern "C" int tl_gemm_partials(const void* x, const void* w, void* out, int M, 
     *parts = P;
     // (the rings against the tiles, us: 16 rows, 2048 x 2048 4.4 / 3.5, 4096 x 8192 17.9 / 13.5, 3584 x 18944 26.8 / 24.4; 64 rows, 4096 x 8192 19.4 / 18.1, 3584 x 18944
     // 36.6 / 33.9, 4096 x 4096 11.1 / 11.4, 3584 x 3584 at 48 rows 9.4 / 9.9)
-    if (partials_on_tiles(M, N, K) && ring_fits(x, w, M, K, ldx) && (M <= 32 || K >= 8192))
+    if (gives_few_row_slabs(M, N, K) && ring_fits(x, w, M, K, ldx) && (M <= 32 || K >= 8192))
         return launch_ring<float, 0, END_STORE>(RingCall{x, w, nullptr, 0, out, M, N, K, ldx, N, 0, P, k_per}, stream);
-    if (partials_on_tiles(M, N, K)) {
+    if (gives_few_row_slabs(M, N, K)) {
         auto kernel = gemm_dl_tile_kernel<64, 64, 2, 2, 4, float, false>;
         constexpr size_t lds = (size_t)4 * 128 * 64 * sizeof(bf16_t);
         static hipError_t allowed = allow_lds(kernel, lds);

@@ -9,8 +9,9 @@
 //
 // Such a product takes as long as a compute unit needs to draw its share of the weights and its copy of x, and it draws at the rate of what it has on its way: a kernel
 // whose waves fetch weight rows into registers (two steps of K each) behind a copy of x into shared memory had 16 to 32 KB on their way, fetched with sixteen rows to an
-// instruction, and waited for x before the first product.  Here it is 64 to 80 KB a work-group, two work-groups to a unit where the plan has so many, each
-// instruction fetches eight whole lines, and x arrives beside the weights.  Measured against that kernel (us, launch included, weights from memory; rows of x, N x K):
+// instruction, and waited for x before the first product.  Here it is 4 D (WJ + XH) KB a work-group: 32 (one request of weights, up to 8 rows of x) to 80, up to which two work-groups
+// fit a unit, and with 32 or 64 rows of x up to 128.  Each instruction fetches eight whole lines, and x arrives beside the weights.  Measured against that kernel (us, launch included,
+// weights from memory; rows of x, N x K):
 //   1 row: 2048 x 2048 3.8 -> 3.2, 4608 x 3584 8.1 -> 7.4;  8 rows: 256 x 2048 4.1 -> 3.1, 2048 x 2048 5.0 -> 3.5, 6144 x 2048 9.1 -> 6.5, 4096 x 4096 11.8 -> 7.6, gate and up
 //   of 2 x 18944 x 3584 50.6 -> 46.9;  16 rows: 34 x 4096 8.9 -> 4.2, 2048 x 2048 6.2 -> 3.7, gate and up of 2 x 11264 x 4096 38.9 -> 32.0;  32 rows: 4608 x 3584 21.8 -> 10.8
 //
