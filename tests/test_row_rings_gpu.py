@@ -170,3 +170,15 @@ def test_projection_of_one_row_that_makes_its_norm_itself_in_turned_orders(ops, 
     exact = h.double() @ w.double().T
     torch.testing.assert_close(v1[1, :, :, 9].reshape(-1).double(), exact[0, (nh + nkv) * hd:], rtol=2 ** -8, atol=1e-4)
 
+
+
+@pytest.mark.parametrize("M", [1, 9, 17])
+def test_rows_too_far_apart_for_the_rings_offsets(ops, M):
+    N, K, apart = 130, 128, 1 << 24            # (the bytes between rows, by a tile's rows, are beyond 32 bits)
+    x, w = _operands(M, N, K, M)
+    wide = torch.zeros(M, apart, dtype=torch.bfloat16, device="cuda")
+    wide[:, :K] = x
+    ref = x.double() @ w.double().T
+    out = torch.full((M, N), float("nan"), device="cuda")
+    ops.linear(wide[:, :K], w, None, out)
+    torch.testing.assert_close(out.double(), ref, **_tol32(ref, K))

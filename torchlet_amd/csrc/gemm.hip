@@ -1772,7 +1772,7 @@ static bool skinny_fits(const void* x, const void* w, int M, int K, int ldx) {
 // out = x w^T (+ bias) in the engine's dtype: picks the kernel for the shape.
 //   bfloat16, aligned, K a multiple of 64:
 //     up to 64 rows as ring_pays says -> gemm_ring
-//     one row against more        -> gemm_skinny (matrix cores, weight streaming)
+//     one row against more, and up to 32 rows 2^23 numbers apart -> gemm_skinny (matrix cores, weight streaming)
 //     everything else             -> gemm_dl_tile (matrix cores, operands straight into shared memory)
 //   bfloat16, aligned, other K, M <= 64 -> gemm_skinny, except that 33..64 rows against a wide matrix go to the tile kernel
 //   bfloat16, aligned, other K, M > 64  -> gemm_mfma_tile (matrix cores, shared-memory tiles)
@@ -1788,7 +1788,7 @@ extern "C" int tl_gemm(const void* x, const void* w, const void* bias, int bias_
         const RingCall c{x, w, bias, bias_f32, out, M, N, K, ldx, ldo, 0};
         return out_f32 ? launch_ring<float, 0, END_STORE>(c, stream) : launch_ring<bf16_t, 0, END_STORE>(c, stream);
     }
-    if (dtype == TL_DT_BF16 && aligned && K % 64 == 0 && M > 8) {
+    if (dtype == TL_DT_BF16 && aligned && K % 64 == 0 && (M > 32 || (M > 8 && N >= 16384))) {      // (up to 32 rows of fewer columns: the rings', but for rows too far apart for their offsets and the tiles')
         int rc = out_f32 ? launch_dl_tile<float, false>(pick_dl_tile(M, N, K, false), x, w, bias, bias_f32, out, M, N, K, ldx, ldo, 0, stream)
                          : launch_dl_tile<bf16_t, false>(pick_dl_tile(M, N, K, false), x, w, bias, bias_f32, out, M, N, K, ldx, ldo, 0, stream);
         if (rc != TL_OK) return rc;
@@ -2134,7 +2134,7 @@ extern "C" int tl_gemm_groups(const void* x, long x_group, const void* w, void* 
         c.gr = gr;
         return out_f32 ? launch_ring<float, 0, END_STORE>(c, stream) : launch_ring<bf16_t, 0, END_STORE>(c, stream);
     }
-    if (dtype == TL_DT_BF16 && aligned && K % 64 == 0 && M > 8) {
+    if (dtype == TL_DT_BF16 && aligned && K % 64 == 0 && (M > 32 || (M > 8 && (long)N * groups >= 16384))) {
         const DlTile tile = pick_dl_tile(M, N, K, false, groups);
         const int rc = out_f32 ? launch_dl_tile<float, false>(tile, x, w, nullptr, 0, out, M, N, K, ldx, ldo, 0, stream, 1, 0, gr)
                                : launch_dl_tile<bf16_t, false>(tile, x, w, nullptr, 0, out, M, N, K, ldx, ldo, 0, stream, 1, 0, gr);
