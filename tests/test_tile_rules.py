@@ -47,7 +47,7 @@ def test_few_rows_go_where_they_were_faster(lib, M, N, K, gated, want):
     (16384, 17, 1, 0, (8, 64)), (4608, 1, 1, 1, (3, 18)), (16640, 3, 1, 0, (3, 22)), (100, 1, 1, 0, (1, 8)), (13568, 8, 1, 1, (4, 28))])
 def test_shares_of_the_rings(lib, total, M, halves, even, want):
     wj, rows = c_int(), c_int()
-    lib.tl_gemm_ring_plan(c_int(total), c_int(M), c_int(3584), c_int(halves), c_int(256), c_int(even), ctypes.byref(wj), ctypes.byref(rows))
+    lib.tl_gemm_ring_plan(c_int(total), c_int(M), c_int(3584), c_int(halves), c_int(256), c_int(even), c_int(1), ctypes.byref(wj), ctypes.byref(rows))
     assert (wj.value, rows.value) == want
     assert rows.value <= 8 * wj.value // halves and (not even or rows.value % 2 == 0)
 
@@ -59,6 +59,14 @@ def test_shares_do_not_hang_on_the_number_of_rows_where_the_order_of_the_sums_ha
                 plans = set()
                 for M in range(1, 17):
                     wj, rows = c_int(), c_int()
-                    lib.tl_gemm_ring_plan(c_int(total), c_int(M), c_int(K), c_int(halves), c_int(256), c_int(even), ctypes.byref(wj), ctypes.byref(rows))
+                    lib.tl_gemm_ring_plan(c_int(total), c_int(M), c_int(K), c_int(halves), c_int(256), c_int(even), c_int(1), ctypes.byref(wj), ctypes.byref(rows))
                     plans.add((wj.value, rows.value))
                 assert len(plans) == 1, (total, K, halves, even)
+
+
+# ranges of K: a unit's work-group of eight requests stays alone
+@pytest.mark.parametrize("total, M, K, parts, want", [(3584, 8, 18944, 4, (8, 56)), (4096, 1, 4096, 4, (8, 64)), (5120, 16, 13824, 3, (8, 61)), (2048, 8, 8192, 8, (8, 64)), (2048, 8, 2048, 4, (4, 32))])
+def test_shares_of_the_rings_with_k_split(lib, total, M, K, parts, want):
+    wj, rows = c_int(), c_int()
+    lib.tl_gemm_ring_plan(c_int(total), c_int(M), c_int(K), c_int(1), c_int(256), c_int(0), c_int(parts), ctypes.byref(wj), ctypes.byref(rows))
+    assert (wj.value, rows.value) == want

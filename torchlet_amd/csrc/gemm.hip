@@ -1246,7 +1246,7 @@ static int launch_ring_x(const RingCall& c, RingPlan p, hipStream_t stream) {
 // `p.wj` 0: the plan is made here.
 template <typename TOut, int SW, int END>
 static int launch_ring(const RingCall& c, hipStream_t stream, RingPlan p = RingPlan{0, 0}) {
-    if (p.wj == 0) p = plan_ring(SW ? c.out_cols : c.N, c.M, SW ? 2 : 1, TL_COMPUTE_UNITS / (c.parts * c.gr.count), END == END_ROTATE, ring_spread(c.K));
+    if (p.wj == 0) p = plan_ring(SW ? c.out_cols : c.N, c.M, SW ? 2 : 1, TL_COMPUTE_UNITS / (c.parts * c.gr.count), END == END_ROTATE, ring_spread(c.K), c.parts > 1);
     if (c.M <= 8) return launch_ring_x<1, TOut, SW, END>(c, p, stream);
     if (c.M <= 16) return launch_ring_x<2, TOut, SW, END>(c, p, stream);
     if constexpr (END == END_STORE) {
@@ -1263,9 +1263,9 @@ extern "C" int tl_gemm_few_rows_choice(int M, int N, int K, int gated) {
     return ring_pays(M, N, K) ? 0 : M > 8 ? 2 : 1;
 }
 
-// The plan of a whole product through the rings (for tests): `halves` 2 for the fused gate.
-extern "C" void tl_gemm_ring_plan(int total, int M, int K, int halves, int units, int even, int* wj, int* rows) {
-    const RingPlan p = plan_ring(total, M, halves, units, even != 0, ring_spread(K));
+// The plan of a product through the rings (for tests): `halves` 2 for the fused gate; K in `parts` ranges.
+extern "C" void tl_gemm_ring_plan(int total, int M, int K, int halves, int units, int even, int parts, int* wj, int* rows) {
+    const RingPlan p = plan_ring(total, M, halves, units / parts, even != 0, ring_spread(K), parts > 1);
     *wj = p.wj;
     *rows = p.rows;
 }
@@ -1944,7 +1944,7 @@ extern "C" int tl_gemm_rope_normed(const void* residual, void* residual_out, con
     int rows = ks == 8 ? balanced_rows(N, &blocks) : 0, run = 0;
     if (ks == 8 && ring_spread(K)) {             // shares as tl_gemm_rope deals them (see ring_products), in equal strips of up to two blocks: the same bits, and with rows of weights a multiple of
                                                  // 4 KB apart the order is as good here (us, in step / turned: 2560 x 2048 7.6 / 7.8, 6144 x 4096 16.6 / 16.1, 9216 x 2048 19.9 / 15.4)
-        rows = keep_shares(na, plan_ring(N, 1, 1, TL_COMPUTE_UNITS, true, true).rows, N);
+        rows = keep_shares(na, plan_ring(N, 1, 1, TL_COMPUTE_UNITS, true, true, false).rows, N);
         blocks = rows > 16 ? 2 : 1;
         run = na.shares * na.share;
     }

@@ -155,8 +155,10 @@ struct RingPlan {
 // A shape of six or eight requests has two slabs on its way, 56 to 80 KB, and with one work-group a unit that is all.  Up to 16 rows of x, where eight requests would fill a unit, two work-groups
 // of four share it with 144 or 160 KB on their way; up to 8 rows of x also in a gate's place of six (us, one row: 16384 x 768 7.0 -> 6.7, x 2048 15.5 -> 13.6; gates, two rows: 8192 x 768
 // 7.7 -> 7.1, x 3584 23.0 -> 22.4, 5120 x 768 5.7 -> 5.6; 16 rows, 5120 x 3584 15.5 -> 16.3, 8192 x 3584 22.9 -> 22.5).
+// Not where K is split over work-groups (8 rows, one of eight / two of four, each 56 to 64 outputs of one range of K: 4096 x 4096 8.2 / 9.4, 3584 x 18944 25.3 / 26.6, 3072 x 8192 11.4 / 12.0,
+// 5120 x 13824 28.0 / 28.2, 3584 x 3584 7.1 / 7.0).
 // `spread` (see ring_products): up to 16 rows the same plan, that of 16.
-static RingPlan plan_ring(int total, int M, int halves, int units, bool even, bool spread) {
+static RingPlan plan_ring(int total, int M, int halves, int units, bool even, bool spread, bool split) {
     const int xh = M <= 8 && !spread ? 1 : M <= 16 ? 2 : M <= 32 ? 4 : 8, floor = 8 / halves;
     if (units < 1) units = 1;
     auto share = [&](long groups, long per) {
@@ -176,6 +178,6 @@ static RingPlan plan_ring(int total, int M, int halves, int units, bool even, bo
         best_rounds = rounds;
         best = RingPlan{wj, share(rounds * units, per)};
     }
-    if (best_rounds == 1 && (best.wj == 8 ? xh <= 2 : best.wj == 6 && xh == 1 && halves == 2)) best = RingPlan{4, share(2L * units, 32 / halves)};
+    if (!split && best_rounds == 1 && (best.wj == 8 ? xh <= 2 : best.wj == 6 && xh == 1 && halves == 2)) best = RingPlan{4, share(2L * units, 32 / halves)};
     return best;
 }
