@@ -905,9 +905,10 @@ extern "C" int tl_streams_norm(void* x, int streams, int total_rows, int hidden,
     const bool pieces = hidden % 4 == 0 && hidden <= 16384 && (((uintptr_t)x | (uintptr_t)pending | (uintptr_t)out) % 16) == 0;
     // (the vectors number by number where they lie elsewhere: 8 rows of four copies of 2048 4.7 us, 64 rows of 8192 7.3; by the kernel above 16.3 and 32)
     const bool whole = (uintptr_t)weight % (weight_f32 ? 16 : 8) == 0 && (uintptr_t)bias % (bias_f32 ? 16 : 8) == 0;
-    // EARLY for as many rows as the GPU has compute units, and for rows of up to 4096 numbers: beyond, the registers it takes leave a unit one row at a time instead of two (us, EARLY / not:
-    // 2048 rows of two copies of 8192, layer norm, 72 / 54; of one of 15360 77 / 59; 300 rows of four of 8192 22.5 / 18.5; 2048 rows of one of 4096, vectors number by number, 28 / 25).
-    const bool early = n_out <= 256 || (whole && hidden <= 4096);
+    // EARLY for as many rows as the GPU has compute units.  Beyond, the other rows' requests hide the trips, and what counts is how many rows a unit holds, which the registers it takes make fewer
+    // (us, EARLY / not, pending outputs of bfloat16: 1000 rows of 3584, one copy 15.0 / 12.2, four 27.8 / 26.1, 2048 rows of four of 2052 29.9 / 27.3, 2048 rows of two of 8192 72 / 54), but for
+    // slabs in rows of up to 4096 numbers, where there is more to ask for ahead (2048 rows of 3072 with three slabs, 0.85 / 0.96 of the time before EARLY, 1000 of two copies of 4096 0.86 / 0.94).
+    const bool early = n_out <= 256 || (parts > 0 && whole && hidden <= 4096);
     if (pieces && (streams == 1 || streams == 2 || streams == 4) && (act_dtype == TL_DT_F32 || act_dtype == TL_DT_BF16)) {
         const int n = hidden <= 4096 ? 1 : hidden <= 8192 ? 2 : 4, threads = ((hidden / 4 + n - 1) / n + TL_WAVE - 1) / TL_WAVE * TL_WAVE;
 #define TL_SN_E(T, S, N, EARLY) streams_norm_reg_kernel<T, S, N, EARLY><<<n_out, threads, 0, stream>>>((float*)x, total_rows, hidden, pending, parts, (const float*)mix, \
