@@ -41,6 +41,13 @@ def test_few_rows_go_where_they_were_faster(lib, M, N, K, gated, want):
     assert lib.tl_gemm_few_rows_choice(c_int(M), c_int(N), c_int(K), c_int(gated)) == want
 
 
+# slabs of K in ranges, sizes on both sides of each line, measured 3 % and more apart
+@pytest.mark.parametrize("M, N, K, want", [(32, 3072, 8192, 0), (2, 2048, 2048, 0), (33, 4096, 4096, 2), (64, 3072, 8192, 2), (48, 2048, 8192, 2), (33, 2304, 9728, 2), (64, 5120, 8192, 2), (64, 4096, 9728, 2),
+                                           (64, 3584, 8192, 0), (33, 6144, 13824, 0), (64, 1536, 9728, 0), (64, 768, 27648, 0), (64, 4096, 8192, 0), (48, 2048, 16384, 0), (48, 8192, 16384, 0)])
+def test_slabs_of_few_rows_come_from_what_was_faster(lib, M, N, K, want):
+    assert lib.tl_gemm_slabs_choice(c_int(M), c_int(N), c_int(K)) == want
+
+
 # a unit's work-groups: 4 requests twice where 8 (a gate's rows up to 8 also 6) would have it to themselves with two slabs on their way; shares of all outputs by equal numbers
 @pytest.mark.parametrize("total, M, halves, even, want", [
     (16384, 1, 1, 0, (4, 32)), (14336, 16, 1, 0, (4, 28)), (12288, 8, 1, 0, (6, 48)), (8192, 2, 2, 0, (4, 16)), (5120, 8, 2, 0, (4, 10)), (5120, 9, 2, 0, (6, 20)), (8192, 16, 2, 0, (4, 16)),

@@ -2028,8 +2028,8 @@ extern "C" int tl_gemm_swiglu(const void* x, const void* w, void* out, int M, in
 // units busy; whoever reads the slabs adds them up.  Returns P through `parts` (the caller sizes
 // `out` for tl_gemm_partials_max()).  More than 64 rows: see plan_dl_split (measured at 512 rows:
 // 3584 x 18944 147 -> 82 us, 5120 x 13824 179 -> 82 us, 5120 x 27648 348 -> 150 us, the norm's sum
-// included).  Up to 64 rows, where it pays (see gives_few_row_slabs), the rings or, from 33 rows on
-// with K below 8192, the direct-load tile kernel with 64 x 64 tiles; for other K the skinny kernel
+// included).  Up to 64 rows, where it pays (see gives_few_row_slabs), the rings or the
+// direct-load tile kernel with 64 x 64 tiles (see slabs_by_rings); for other K the skinny kernel
 // with R = 4 strips per work-group, which share every x fetch.
 extern "C" int tl_gemm_partials_max() { return 8; }
 
@@ -2069,6 +2069,23 @@ extern "C" int tl_gemm_partials_pay(int M, int N, int K) {
     return gives_few_row_slabs(M, N, K) && tl_gemm_partials_parts(M, N, K) > 1;
 }
 
+// Whether those slabs come from the rings or from tiles of 64 x 64.  Up to 32 rows the rings (us, tiles / rings: 16 rows, 2048 x 2048 4.4 / 3.5, 4096 x 8192 17.9 / 13.5, 3584 x 18944 26.8 / 24.4).
+// 33 to 64 rows, with K long enough: where their equal shares give a unit an eighth fewer weight rows than a tile has (64 rows, 6144 x 13824 0.86 of the tiles' time, 3584 x 8192 0.89), or where
+// every unit has 64 on both sides and the rings' order is turned (4096 x 8192 0.88, 2048 x 16384, 48 rows, 0.90).  Otherwise a work-group draws as much either way, and tiles, whose waves read a
+// row of x once for 64 columns, are ahead (64 rows, 3072 x 8192 14.9 / 16.2, 2048 x 11008 13.8 / 14.9, 5120 x 8192 21.5 / 22.9, 4096 x 4096 11.1 / 11.4).
+static bool slabs_by_rings(int M, int N, int K, int parts, int k_per) {
+    if (M <= 32) return true;
+    if (K < 8192) return false;
+    const bool every_unit = N % 64 == 0 && N / 64 * parts == TL_COMPUTE_UNITS, turned = ring_spread(K) && k_per >= 2048;      // (2048: eight slabs a wave)
+    return (every_unit && turned) || plan_ring(N, M, 1, TL_COMPUTE_UNITS / parts, false, ring_spread(K), parts > 1).rows <= 56;
+}
+
+// The same for tests: 0 the rings, 2 tiles.
+extern "C" int tl_gemm_slabs_choice(int M, int N, int K) {
+    const int steps = (K + 63) / 64, P = tl_gemm_partials_parts(M, N, K), k_per = ((steps + P - 1) / P) * 64;
+    return slabs_by_rings(M, N, K, (K + k_per - 1) / k_per, k_per) ? 0 : 2;
+}
+
 extern "C" int tl_gemm_partials(const void* x, const void* w, void* out, int M, int N, int K, int ldx, int* parts,
                                 hipStream_t stream) {
     TL_REQUIRE(M > 0 && N > 0 && K > 0 && ldx >= K, "gemm_partials: bad sizes M=%d N=%d K=%d", M, N, K);
@@ -2088,9 +2105,7 @@ extern "C" int tl_gemm_partials(const void* x, const void* w, void* out, int M, 
     const int k_per = ((steps + P - 1) / P) * 64;
     P = (K + k_per - 1) / k_per;
     *parts = P;
-    // (the rings against the tiles, us: 16 rows, 2048 x 2048 4.4 / 3.5, 4096 x 8192 17.9 / 13.5, 3584 x 18944 26.8 / 24.4; 64 rows, 4096 x 8192 19.4 / 18.1, 3584 x 18944
-    // 36.6 / 33.9, 4096 x 4096 11.1 / 11.4, 3584 x 3584 at 48 rows 9.4 / 9.9)
-    if (gives_few_row_slabs(M, N, K) && ring_fits(x, w, M, K, ldx) && (M <= 32 || K >= 8192))
+    if (gives_few_row_slabs(M, N, K) && ring_fits(x, w, M, K, ldx) && slabs_by_rings(M, N, K, P, k_per))
         return launch_ring<float, 0, END_STORE>(RingCall{x, w, nullptr, 0, out, M, N, K, ldx, N, 0, P, k_per}, stream);
     if (gives_few_row_slabs(M, N, K)) {
         auto kernel = gemm_dl_tile_kernel<64, 64, 2, 2, 4, float, false>;
