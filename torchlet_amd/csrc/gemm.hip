@@ -1943,7 +1943,7 @@ extern "C" int tl_gemm_rope_normed(const void* residual, void* residual_out, con
     int blocks = 1;
     int rows = ks == 8 ? balanced_rows(N, &blocks) : 0, run = 0;
     if (ks == 8 && ring_spread(K)) {             // shares as tl_gemm_rope deals them (see ring_products), in equal strips of up to two blocks: the same bits, and with rows of weights a multiple of
-                                                 // 4 KB apart the order is as good here (us, in step / turned: 2560 x 2048 7.1 / 7.4, 6144 x 4096 15.8 / 14.9, 10240 x 2048 18.9 / 15.8)
+                                                 // 4 KB apart the order is as good here (us, in step / turned: 2560 x 2048 7.1 / 7.2, 6144 x 4096 15.8 / 14.9, 10240 x 2048 18.9 / 15.8)
         rows = keep_shares(na, plan_ring(N, 1, 1, TL_COMPUTE_UNITS, true, true, false).rows, N);
         blocks = rows > 16 ? 2 : 1;
         run = na.shares * na.share;

@@ -43,11 +43,14 @@ struct RingShape {
 // (us, in step -> spread: 16 rows, 8144 x 4096 16.3 -> 13.7, 32000 x 4096 48 -> 41, 4096 x 16384 33 -> 22, 11264 x 2048 10.9 -> 9.9; with other pitches, 4608 x 3584 8.1 -> 8.5, 2048 x 5632
 // 8.4 -> 8.4.  Ranges of 512 columns in four orders, summed by pairs so that it would not hang on the work-group: 8144 x 4096 16.1, 4096 x 16384 34.  With few slabs a wave has them all on their
 // way from the start, and 4096 columns by 1024 of K took 8.3 instead of 7.6.)
-// Where a work-group begins: an eighth of the way on from its neighbour, which runs on the next XCD, and every eighth three slabs on.  Over 131 sizes by 1, 2 to 8 and 16 rows, gates among them,
-// 1.014 of the best of five such rules on average and 1.10 at most, 5 b + b / 8 1.020 and 1.24: where its steps fall in with the pitch of the work-groups' rows (us, that / this / the kernel
-// that fetches into registers: 20000 x 8192, one row, 67.7 / 58.6 / 60.4, 10240 x 8192, 2 rows, 37.7 / 31.8 / 34.8, gate 24640 x 8192, 4 rows, 160 / 139 / 147; 2048 x 6144, 2 rows, 7.9 / 8.5 / 9.3).
+// Where a work-group begins: with up to 16 slabs a wave at 5 b + b / 8, beyond an eighth of the way on from its neighbour, which runs on the next XCD, and every eighth three slabs on.  With many
+// slabs the first rule falls in with the pitch of the work-groups' rows at some sizes (us, first / second / the kernel that fetches into registers: 20000 x 8192, one row, 67.7 / 58.6 / 60.4,
+// 10240 x 8192, 2 rows, 37.7 / 31.8 / 34.8, gate 24640 x 8192, 4 rows, 160 / 139 / 147; over 44 sizes of K 8192 and more the second takes 0.98 of the first), with few it is a little ahead
+// (2560 x 2048, 16 rows, 4.5 / 4.7; over 22 sizes of K up to 4096 and up to 6144 columns 0.996).
 __host__ __device__ inline bool ring_spread(int pitch) { return pitch % 2048 == 0; }
-__device__ __forceinline__ int ring_start(unsigned group, unsigned slabs_of_a_wave) { return (int)((group % 8 * slabs_of_a_wave / 8 + 3 * (group / 8)) % slabs_of_a_wave); }
+__device__ __forceinline__ int ring_start(unsigned group, unsigned slabs_of_a_wave) {
+    return (int)((slabs_of_a_wave <= 16 ? 5 * group + group / 8 : group % 8 * slabs_of_a_wave / 8 + 3 * (group / 8)) % slabs_of_a_wave);
+}
 
 template <int WJ, int XH, int HALVES>
 __device__ __forceinline__ void ring_products(const bf16_t* w, const unsigned (&woff)[WJ], const bf16_t* x, const unsigned (&xoff)[XH], int slabs, char* ring, int wave, bool spread) {
