@@ -1,5 +1,5 @@
 """The latents' norms, rotation and cache write on both sides of 512 tokens (below: a work-group for each of them), the attention at the sizes that have kernels of their own (latents of
-512 numbers beside 64 or no rotated ones) and the merges of parts, against plain 64-bit formulas."""
+a multiple of 64 numbers beside 0, 32 or 64 rotated ones) and at others, and the merges of parts, against plain 64-bit formulas."""
 from __future__ import annotations
 
 import pytest
@@ -51,7 +51,7 @@ def test_prepare_on_both_sides_of_the_line(tokens, q_rank, rank, rot, dims, head
         assert bool((got[:, :rank] == 7.0).all())
 
 
-@pytest.mark.parametrize("rot", [0, 32, 64])                    # (32: the kernel by sizes that come with the call)
+@pytest.mark.parametrize("rot", [0, 32, 64])
 @pytest.mark.parametrize("tile_rows,new", [(16, 1), (32, 2), (64, 5)])
 @pytest.mark.parametrize("splits", [1, 2, 3, 63, 64])
 @pytest.mark.parametrize("sink,window", [(True, 0), (False, 45)])
