@@ -47,3 +47,29 @@ def test_more_rows_than_a_launch_has_of_the_smallest_tiles():
     ops.linear(x, w, None, out)
     for part in (slice(0, 130), slice(M - 130, M)):
         torch.testing.assert_close(out[part].double(), x[part].double() @ w.double().T, rtol=2e-5, atol=8 * 2 ** -24 * math.sqrt(K))
+
+
+@pytest.mark.parametrize("M", [17, 31, 32, 33, 97, 130])
+@pytest.mark.parametrize("N, K", [(31, 28), (33, 32), (64, 60), (100, 224), (130, 1028)])
+def test_tiles_of_small_blocks_and_of_large_ones_give_the_same_bits(M, N, K):
+    """One slab or none, a rest of a slab, more slabs than are in flight; rows of x wider than K, rows of the result wider than N."""
+    g = torch.Generator(device="cuda").manual_seed(M * K + N)
+    x, w = torch.randn(M, K + 8, generator=g, device="cuda")[:, :K], torch.randn(N, K, generator=g, device="cuda") / math.sqrt(K)
+    out = {}
+    for tile in (4, 5, 6, 7, 8):
+        out[tile] = torch.full((M, N + 3), 7.0, device="cuda")
+        ops.linear_f32_variant(x, w, None, out[tile][:, :N], tile)
+        assert torch.equal(out[tile], out[4])
+    assert bool((out[4][:, N:] == 7.0).all())
+    torch.testing.assert_close(out[4][:, :N].double(), x.double() @ w.double().T, rtol=2e-5, atol=8 * 2 ** -24 * math.sqrt(K))
+
+
+def test_what_lies_beyond_a_row_reaches_no_sum():
+    """Columns past K, rows past M and N: infinities there leave every result finite."""
+    M, N, K = 40, 40, 36
+    x, w = torch.full((M + 1, K + 28), math.inf, device="cuda"), torch.full((N + 8, K), math.inf, device="cuda")
+    x[:M, :K], w[:N] = 1.0, 2.0
+    for tile in (4, 5, 6, 7, 8):
+        out = torch.empty(M, N, device="cuda")
+        ops.linear_f32_variant(x[:M, :K], w[:N], None, out, tile)
+        assert torch.equal(out, torch.full_like(out, 2.0 * K))

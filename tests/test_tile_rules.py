@@ -77,3 +77,10 @@ def test_shares_of_the_rings_with_k_split(lib, total, M, K, parts, want):
     wj, rows = c_int(), c_int()
     lib.tl_gemm_ring_plan(c_int(total), c_int(M), c_int(K), c_int(1), c_int(256), c_int(0), c_int(parts), ctypes.byref(wj), ctypes.byref(rows))
     assert (wj.value, rows.value) == want
+
+
+# tiles of blocks of 16 (4: 64 x 32, 5: 32 x 32) beside those of blocks of 32, sizes measured 5 % and more apart from the next
+@pytest.mark.parametrize("M, N, want", [(17, 4608, 5), (33, 2052, 5), (40, 288, 5), (100, 3584, 4), (200, 2048, 4), (64, 5632, 4), (753, 3584, 1), (753, 4608, 2), (301, 37888, 2), (753, 37888, 3),
+                                        (65535 * 32, 32, 4), (65535 * 64 + 1, 32, 3), (65535 * 128, 64, 3)])
+def test_32_bit_tiles_of_small_blocks(lib, M, N, want):
+    assert lib.tl_gemm_f32_any_tile(c_int(M), c_int(N)) == want

@@ -291,109 +291,166 @@ static void launch_gemv_f32(const void* x, const void* w, const void* bias, int 
 // =====================================================================================
 // True 32-bit on the matrix cores, more than 16 rows: the prompt steps of the 32-bit engine.
 //
-// v_mfma_f32_32x32x2_f32 multiplies 32-bit operands and adds in 32-bit: it is no reduced-precision mode
-// (nothing is rounded to a shorter format on the way), and it runs at four times the rate of the
-// v_fma_f32 tile kernel above.  A work-group of four waves owns a tile of 64 FMB x 64 FNB outputs, a wave
-// 32 FMB x 32 FNB of them; slabs of 16 columns of both operands go through registers into shared
-// memory (two buffers, one barrier per slab).  A lane reads four neighbouring k of its row at once; lanes
-// 0-31 take k = 8c .. 8c+3 and lanes 32-63 k = 8c+4 .. 8c+7 of a chunk of eight, so instruction e of a chunk
-// multiplies k = 8c + e and 8c + 4 + e: which k meet in one instruction is free as long as both operands
-// agree.  The sum of an output element runs in that one fixed order whatever M is and wherever the element
-// lies in its tile, so a row's result does not depend on the batch; it differs from the other 32-bit
-// kernels' by rounding (another order of the same sum).  Needs K % 4 == 0 and 16-byte aligned rows.
-typedef float gf_f32x16_t __attribute__((ext_vector_type(16)));
-#define GF_TK 16
-#define GF_LD (GF_TK + 4)          // floats between rows in shared memory: 16-byte reads of 16 rows fall on all banks
-template <int FMB, int FNB>
-__global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restrict__ x, const float* __restrict__ w,
+// v_mfma_f32_32x32x2_f32 and v_mfma_f32_16x16x4_f32 multiply 32-bit operands and add in 32-bit: they are no reduced-precision mode
+// (nothing is rounded to a shorter format on the way), and they run at four times the rate of the
+// v_fma_f32 tile kernel above.  A work-group of four waves owns a tile of 2 B FMB x 2 B FNB outputs, a wave
+// FMB x FNB blocks of B x B of them.
+//
+// What bounds it is the matrix instruction (64 cycles for a block of 32, 32 for one of 16, against 8 of shared memory for a wave's 16-byte read), so all else has to
+// stay out of its way: slabs of 32 columns of both operands go straight into shared memory, laid out and requested as in direct_tile.h (a row of a slab is 128 bytes
+// there too), STAGES of them in flight or in use, and the operands of the next phase (PHASE times eight columns) are read while this one's are multiplied.  The last
+// phase of a slab waits for the next slab and meets the other waves halfway through its products; behind that barrier go the first reads of the next slab and the
+// requests into the buffer just given up.  Measured against slabs of 16 columns through registers with a barrier each (us; the matrix instruction's 157 TFLOP/s alone
+// would take the last figure): 753 x 37888 x 3584 1772 -> 1443 (1303), 753 x 3584 x 18944 1098 -> 863 (651), 753 x 3584 x 3584 212 -> 166 (123), 301 x 37888 x 3584
+// 832 -> 631 (521), 2048 x 2048 x 2048 167 -> 124 (109).  What is left is the last round of tiles and the clock.
+//
+// A lane holds four neighbouring k of its row: with blocks of 32 lanes 0-31 k = 8c .. 8c+3 and lanes 32-63 k = 8c+4 .. 8c+7 of a chunk of eight, so instruction e
+// of a chunk multiplies k = 8c + e and 8c + 4 + e: which k meet in one instruction is free as long as both operands agree.  With blocks of 16 an instruction takes the k of two of these
+// in the same order (8c, 8c + 4, 8c + 1, 8c + 5 and then the two further on), and its sums come out the same to the last bit.  The sum of an output element
+// runs in that one fixed order whatever M is, whichever tile is taken and wherever the element lies in it, so a row's result does not depend on the batch; it differs from the
+// other 32-bit kernels' by rounding (another order of the same sum).  Needs K % 4 == 0 and 16-byte aligned rows; what K has beyond whole slabs goes through
+// registers, columns past K as zeros.
+#define GF_TK 32
+template <int B, int FMB, int FNB, int STAGES, int WAVES_PER_SIMD, int PHASE>
+__global__ __launch_bounds__(256, WAVES_PER_SIMD) void gemm_f32_mfma_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                             const void* __restrict__ bias, int bias_f32,
                                                             float* __restrict__ out, int M, int N, int K, int ldx, int ldo) {
-    constexpr int BM = 64 * FMB, GF_BN = 64 * FNB;
-    constexpr int XL = BM * 4 / 256, WL = GF_BN * 4 / 256; // 16-byte pieces of x and of w a thread moves per slab
-    __shared__ __attribute__((aligned(16))) float xs[2][BM * GF_LD];
-    __shared__ __attribute__((aligned(16))) float ws[2][GF_BN * GF_LD];
+    constexpr int BM = 2 * B * FMB, BN = 2 * B * FNB, ROWS = BM + BN;
+    constexpr int E = B == 32 ? 4 : 2, V = B * B / 64;      // instructions of a chunk and block, results of a lane and block
+    typedef float sums_t __attribute__((ext_vector_type(V)));
+    typedef float operand_t __attribute__((ext_vector_type(E)));
+    constexpr int LOADS = ROWS / 32;                        // requests of a wave per slab: eight rows each, BM / 32 of them of x
+    constexpr int SLAB = ROWS * GF_TK;                      // floats
+    extern __shared__ __attribute__((aligned(16))) float gf_lds[];     // [STAGES][ROWS][GF_TK]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
-    const int lr = lane & 31, lh = lane >> 5;
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * GF_BN;
+    const int lr = lane % B, lh = lane / B;
 
-    gf_f32x16_t acc[FNB][FMB];
+    // tile order as in direct_tile.h: each XCD walks 8 x 8 blocks of tiles out of its own L2
+    int m0, n0;
+    {
+        const int tiles_n = gridDim.x, tiles_m = gridDim.y, total = tiles_n * tiles_m, id = blockIdx.y * tiles_n + blockIdx.x;
+        const int xcd = id % 8, lid = xcd * (total / 8) + min(xcd, total % 8) + id / 8;
+        const int per_group = 8 * tiles_n, first_m = (lid / per_group) * 8, rows = min(tiles_m - first_m, 8);
+        m0 = (first_m + (lid % per_group) % rows) * BM;
+        n0 = ((lid % per_group) / rows) * BN;
+    }
+
+    sums_t acc[FNB][FMB];
 #pragma unroll
     for (int i = 0; i < FNB; ++i)
 #pragma unroll
         for (int j = 0; j < FMB; ++j)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+            for (int v = 0; v < V; ++v) acc[i][j][v] = 0.f;
 
-    // piece p of a slab: row p / 4, columns 4 (p % 4) .. + 4; rows past the end read the last row (never stored),
-    // columns past K read the last whole piece and count as zero
-    float4 gx[XL], gw[WL];
-    auto fetch = [&](int k0) {
+    // request j of this wave fills the rows 8 (wave + 4 j) .. + 7 of the stacked [x rows; w rows] slab; piece c of row r lies in slot c ^ ((r >> 1) & 7).
+    // Rows past the end read the last row (never stored).
+    unsigned soff[LOADS];
+    int ldst[LOADS];
 #pragma unroll
-        for (int i = 0; i < XL; ++i) {
-            const int p = tid + 256 * i, k = k0 + 4 * (p & 3);
-            gx[i] = *(const float4*)(x + (size_t)min(m0 + (p >> 2), M - 1) * ldx + min(k, K - 4));
-            if (k >= K) gx[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-#pragma unroll
-        for (int i = 0; i < WL; ++i) {
-            const int p = tid + 256 * i, k = k0 + 4 * (p & 3);
-            gw[i] = *(const float4*)(w + (size_t)min(n0 + (p >> 2), N - 1) * K + min(k, K - 4));
-            if (k >= K) gw[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-    };
-    auto park = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < XL; ++i) {
-            const int p = tid + 256 * i;
-            *(float4*)(&xs[buf][(p >> 2) * GF_LD + 4 * (p & 3)]) = gx[i];
-        }
-#pragma unroll
-        for (int i = 0; i < WL; ++i) {
-            const int p = tid + 256 * i;
-            *(float4*)(&ws[buf][(p >> 2) * GF_LD + 4 * (p & 3)]) = gw[i];
-        }
-    };
-    fetch(0);
-    park(0);
-    __syncthreads();
-    const int slabs = (K + GF_TK - 1) / GF_TK;
-    for (int s = 0; s < slabs; ++s) {
-        if (s + 1 < slabs) fetch((s + 1) * GF_TK);          // on their way while this slab is multiplied
-        const float* xb = xs[s & 1];
-        const float* wb = ws[s & 1];
-#pragma unroll
-        for (int c = 0; c < GF_TK / 8; ++c) {
-            float4 a[FNB], b[FMB];
-#pragma unroll
-            for (int i = 0; i < FNB; ++i) a[i] = *(const float4*)(wb + (wn * 32 * FNB + i * 32 + lr) * GF_LD + 8 * c + 4 * lh);
-#pragma unroll
-            for (int j = 0; j < FMB; ++j) b[j] = *(const float4*)(xb + (wm * 32 * FMB + j * 32 + lr) * GF_LD + 8 * c + 4 * lh);
-#pragma unroll
-            for (int i = 0; i < FNB; ++i)
-#pragma unroll
-                for (int j = 0; j < FMB; ++j) {
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i].x, b[j].x, acc[i][j], 0, 0, 0);
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i].y, b[j].y, acc[i][j], 0, 0, 0);
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i].z, b[j].z, acc[i][j], 0, 0, 0);
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i].w, b[j].w, acc[i][j], 0, 0, 0);
-                }
-        }
-        if (s + 1 < slabs) park((s + 1) & 1);               // everyone left that buffer before the last barrier
-        __syncthreads();
+    for (int j = 0; j < LOADS; ++j) {
+        const int row = 8 * (wave + 4 * j) + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
+        soff[j] = j < BM / 32 ? (unsigned)((min(m0 + row, M - 1) - m0) * ldx + c * 4) * 4u : (unsigned)((min(n0 + row - BM, N - 1) - n0) * K + c * 4) * 4u;
+        ldst[j] = __builtin_amdgcn_readfirstlane(8 * (wave + 4 * j) * GF_TK * 4);
     }
-    // weight block times x block: a lane holds row m = lane % 32 of x and the output columns
-    // n = 8 (v / 4) + 4 (lane / 32) + v % 4 of a 32 x 32 block, four neighbours at a time
+    const float *xt = x + (size_t)m0 * ldx, *wt = w + (size_t)n0 * K;
+    const unsigned lds_base = (unsigned)(uintptr_t)((void __attribute__((address_space(3)))*)gf_lds);
+    const int slabs = K / GF_TK, rest = K % GF_TK;
+
+    // a chunk's operands (blocks are 16 or 32 rows apart, which leaves the slots' order as it is)
+    const int x_at = (wm * B * FMB + lr) * GF_TK, w_at = (BM + wn * B * FNB + lr) * GF_TK, turn = (lr >> 1) & 7;
+    operand_t a[2][PHASE][FNB], b[2][PHASE][FMB];
+    auto read = [&](const float* slab, int phase, int set, int op) {
+        const int h = op / (FMB + FNB), o = op % (FMB + FNB), c = phase * PHASE + h;
+        const float* row = slab + (o < FNB ? w_at + o * B * GF_TK : x_at + (o - FNB) * B * GF_TK);
+        operand_t& to = o < FNB ? a[set][h][o] : b[set][h][o - FNB];
+        if constexpr (B == 32) {
+            to = *(const operand_t*)(row + ((2 * c + lh) ^ turn) * 4);
+        } else {
+            const float* at = row + ((2 * c + (lh & 1)) ^ turn) * 4 + (lh >> 1);
+            to[0] = at[0];
+            to[1] = at[2];
+        }
+    };
+    auto product = [&](int set, int q) {
+        const int h = q / (E * FMB * FNB), e = q / (FMB * FNB) % E, i = q % (FMB * FNB) / FMB, j = q % FMB;
+        if constexpr (B == 32) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[set][h][i][e], b[set][h][j][e], acc[i][j], 0, 0, 0);
+        else acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[set][h][i][e], b[set][h][j][e], acc[i][j], 0, 0, 0);
+    };
+    static_assert(GF_TK / 8 / PHASE % 2 == 0, "two sets of operands in turn");
+    constexpr int READS = PHASE * (FMB + FNB), PHASES = GF_TK / 8 / PHASE, NM = PHASE * E * FMB * FNB, BARRIER_AT = NM / 2;
+    if (slabs > 0) {
+        // (past the end the last slab is requested again, which nobody reads: the count of requests in flight is the same in every step)
+        auto request = [&](int slab, int j) {
+            load_to_lds_at((j < BM / 32 ? xt : wt) + min(slab, slabs - 1) * GF_TK, soff[j], lds_base + (slab % STAGES) * (SLAB * 4) + ldst[j]);
+        };
+#pragma unroll
+        for (int st = 0; st < STAGES; ++st)
+#pragma unroll
+            for (int j = 0; j < LOADS; ++j) request(st, j);
+        wait_direct_loads<(STAGES - 1) * LOADS>();
+        __syncthreads();
+#pragma unroll
+        for (int op = 0; op < READS; ++op) read(gf_lds, 0, 0, op);
+        __builtin_amdgcn_sched_barrier(0);
+        for (int sl = 0; sl < slabs; ++sl) {
+            const float *here = gf_lds + (sl % STAGES) * SLAB, *next = gf_lds + ((sl + 1) % STAGES) * SLAB;
+#pragma unroll
+            for (int c = 0; c < PHASES; ++c) {
+                const bool last = c + 1 == PHASES;
+                const int start = last ? BARRIER_AT : 0, ops = READS + (last ? LOADS : 0), per = (ops + NM - start - 1) / (NM - start);
+                int op = 0;
+#pragma unroll
+                for (int q = 0; q < NM; ++q) {
+                    if (last && q == start) {
+                        wait_direct_loads<(STAGES - 2) * LOADS>();
+                        __syncthreads();
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    product(c & 1, q);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (q < start) continue;
+#pragma unroll
+                    for (int e = 0; e < per; ++e, ++op) {
+                        if (op < READS) read(last ? next : here, last ? 0 : c + 1, (c + 1) & 1, op);
+                        else if (op < ops) request(sl + STAGES, op - READS);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        }
+        wait_direct_loads<0>();
+    }
+    if (rest) {
+        __syncthreads();                                    // (all direct loads have landed and all operands are read)
+#pragma unroll
+        for (int j = 0; j < LOADS; ++j) {
+            const int row = 8 * (wave + 4 * j) + (lane >> 3), piece = lane & 7, k = slabs * GF_TK + 4 * piece;
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (k < K) v = *(const float4*)(row < BM ? x + (size_t)min(m0 + row, M - 1) * ldx + k : w + (size_t)min(n0 + row - BM, N - 1) * K + k);
+            *(float4*)(gf_lds + row * GF_TK + ((piece ^ ((row >> 1) & 7)) * 4)) = v;
+        }
+        __syncthreads();
+        for (int c = 0; 8 * PHASE * c < rest; ++c) {
+#pragma unroll
+            for (int op = 0; op < READS; ++op) read(gf_lds, c, 0, op);
+#pragma unroll
+            for (int q = 0; q < NM; ++q) product(0, q);
+        }
+    }
+    // weight block times x block: a lane holds row m = lane % B of x and the output columns
+    // n = 8 (v / 4) + 4 (lane / 32) + v % 4 of a 32 x 32 block, 4 (lane / 16) + v of a 16 x 16 block, four neighbours at a time
     const bool quads = N % 4 == 0 && ldo % 4 == 0 && ((uintptr_t)out % 16) == 0;
 #pragma unroll
     for (int j = 0; j < FMB; ++j) {
-        const int m = m0 + wm * 32 * FMB + j * 32 + lr;
+        const int m = m0 + wm * B * FMB + j * B + lr;
         if (m >= M) continue;
 #pragma unroll
         for (int i = 0; i < FNB; ++i)
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int n = n0 + wn * 32 * FNB + i * 32 + 8 * g + 4 * lh;
+            for (int g = 0; g < V / 4; ++g) {
+                const int n = n0 + wn * B * FNB + i * B + 8 * g + 4 * lh;
                 float v[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] = acc[i][j][4 * g + e] + ((bias && n + e < N) ? load_vec(bias, bias_f32, n + e) : 0.f);
@@ -408,22 +465,24 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
     }
 }
 
+// (a lane's offset from its tile's first row is kept in 32 bits)
 static bool gemm_f32_mfma_fits(const void* x, const void* w, int M, int K, int ldx) {
-    return M > 16 && K >= 4 && K % 4 == 0 && ldx % 4 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0;
+    return M > 16 && K >= 4 && K % 4 == 0 && ldx % 4 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0 && ldx < (1 << 22) && K < (1 << 22);
 }
 
-// The size of tiles of a 32-bit product: 1 64 x 64, 2 64 x 128, 3 128 x 128.
+// The size of tiles of a 32-bit product: 1 64 x 64, 2 64 x 128, 3 128 x 128 of blocks of 32; 4 64 x 32 and 5 32 x 32 of blocks of 16, which move twice the operands per product
+// but leave few rows against a narrow matrix more work-groups and a shorter chain each.
 //
 // Microseconds per column of K: a start and a round of work-groups, up to TL_COMPUTE_UNITS of them at once (the smaller tiles' rounds overlap on a unit).  Fitted to 17 to 2048
-// rows against nine matrices 2048 to 152064 wide; the sums are the same whichever is taken.  Measured (us; 64 x 64 / 64 x 128 / 128 x 128): 100 x 3584 x 3584 104 / 166 / 275,
-// 753 x 3584 x 18944 1160 / 1373 / 1440, 1200 x 3584 x 3584 358 / 393 / 474, 301 x 37888 x 3584 930 / 863 / 1011, 753 x 37888 x 3584 2248 / 1977 / 1803.
-// (Two sizes alone, 64 x 128 up to one round of 128 x 128 tiles, took 1.6 times as long up to 256 rows.)
+// rows against thirteen matrices 288 to 37888 wide, within a tenth of each; the sums are the same whichever is taken.  Measured (us; 64 x 64 / 64 x 128 / 128 x 128 / 64 x 32 / 32 x 32):
+// 17 x 4608 x 3584 65 / 113 / 211 / 45 / 33, 100 x 3584 x 3584 66 / 114 / 214 / 45 / 52, 301 x 3584 x 18944 578 / 586 / 1111 / 600 / 659, 753 x 3584 x 18944 863 / 1084 / 1117 / 1191 / 1443,
+// 753 x 4608 x 3584 225 / 210 / 216 / 267 / 350, 301 x 37888 x 3584 675 / 631 / 816 / 894 / 1164, 753 x 37888 x 3584 1618 / 1472 / 1443 / 2096 / 2744.
 // A size whose rows of tiles are more than a launch has in y is not considered: beyond 4.19 million rows the tiles are 128 high.
-extern "C" int tl_gemm_f32_tile(int M, int N) {
-    static const struct { int bm, bn; double start, round; } sizes[] = {{64, 64, 0.0065, 0.0207}, {64, 128, 0.0085, 0.0365}, {128, 128, 0.0055, 0.0705}};
+static int f32_tile(int M, int N, int sizes_considered) {
+    static const struct { int bm, bn; double start, round; } sizes[] = {{64, 64, 0.002, 0.0155}, {64, 128, 0.001, 0.0293}, {128, 128, 0.003, 0.0573}, {64, 32, 0.002, 0.0105}, {32, 32, 0.0025, 0.0068}};
     double best = 1e30;
     int tile = 3;
-    for (int t = 0; t < 3; ++t) {
+    for (int t = 0; t < sizes_considered; ++t) {
         const long rows = ((long)M + sizes[t].bm - 1) / sizes[t].bm, tiles = rows * (((long)N + sizes[t].bn - 1) / sizes[t].bn);
         if (rows > 65535) continue;
         const double est = sizes[t].start + sizes[t].round * ((tiles + TL_COMPUTE_UNITS - 1) / TL_COMPUTE_UNITS);
@@ -431,22 +490,30 @@ extern "C" int tl_gemm_f32_tile(int M, int N) {
     }
     return tile;
 }
+extern "C" int tl_gemm_f32_tile(int M, int N) { return f32_tile(M, N, 3); }            // the choice among the blocks of 32 ...
+extern "C" int tl_gemm_f32_any_tile(int M, int N) { return f32_tile(M, N, 5); }        // ... and among all, which a product takes
 
-// `tile`: 0 by the rule above, else one of its sizes (tests cover each; tuning times them).
+template <int B, int FMB, int FNB, int STAGES, int WAVES_PER_SIMD, int PHASE>
+static void launch_gemm_f32_tile(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int N, int K, int ldx, int ldo, hipStream_t stream) {
+    constexpr int BM = 2 * B * FMB, BN = 2 * B * FNB;
+    constexpr size_t lds = (size_t)STAGES * (BM + BN) * GF_TK * sizeof(float);
+    static_assert(lds <= 65536, "no more shared memory than a kernel has unasked");
+    gemm_f32_mfma_kernel<B, FMB, FNB, STAGES, WAVES_PER_SIMD, PHASE><<<dim3((N + BN - 1) / BN, (M + BM - 1) / BM), dim3(256), lds, stream>>>(
+        (const float*)x, (const float*)w, bias, bias_f32, (float*)out, M, N, K, ldx, ldo);
+}
+
+// `tile`: 0 by the rule above, else one of its sizes (tests cover each; tuning times them).  Two work-groups of the larger tiles (64 and 48 KB) and three of 64 x 64 fit a compute unit.
 static void launch_gemm_f32_mfma(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int N, int K,
                                  int ldx, int ldo, hipStream_t stream, int tile = 0) {
-    if (tile == 0) tile = tl_gemm_f32_tile(M, N);
-#define GF_LAUNCH(FMB, FNB)                                                                                                                        \
-    gemm_f32_mfma_kernel<FMB, FNB><<<dim3((N + 64 * FNB - 1) / (64 * FNB), (M + 64 * FMB - 1) / (64 * FMB)), dim3(256), 0, stream>>>(                \
-        (const float*)x, (const float*)w, bias, bias_f32, (float*)out, M, N, K, ldx, ldo)
-    if (tile == 1) GF_LAUNCH(1, 1);
-    else if (tile == 2) GF_LAUNCH(1, 2);
-    else GF_LAUNCH(2, 2);
-#undef GF_LAUNCH
+    if (tile == 0) tile = tl_gemm_f32_any_tile(M, N);
+    auto launch = tile == 1 ? launch_gemm_f32_tile<32, 1, 1, 3, 3, 2> : tile == 2 ? launch_gemm_f32_tile<32, 1, 2, 2, 2, 1> : tile == 3 ? launch_gemm_f32_tile<32, 2, 2, 2, 2, 1>
+                : tile == 4 ? launch_gemm_f32_tile<16, 2, 1, 4, 3, 2> : launch_gemm_f32_tile<16, 1, 1, 6, 3, 2>;
+    launch(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, stream);
 }
 
 // One named kernel of the 32-bit products (for tests and tuning): 0 the general tile kernel (v_fma_f32), 1 the matrix-core
-// tile kernel, 2 and 3 the kernels for up to 16 rows on multiply-adds and on the matrix cores, 4 to 6 the matrix-core tile kernel with tiles of 64 x 64, 64 x 128, 128 x 128.
+// tile kernel, 2 and 3 the kernels for up to 16 rows on multiply-adds and on the matrix cores, 4 to 6 the matrix-core tile kernel with tiles of 64 x 64, 64 x 128, 128 x 128,
+// 7 and 8 with 64 x 32 and 32 x 32.
 extern "C" int tl_gemm_f32_variant(const void* x, const void* w, const void* bias, int bias_f32, void* out,
                                    int M, int N, int K, int ldx, int ldo, int matrix_cores, hipStream_t stream) {
     TL_REQUIRE(M > 0 && N > 0 && K > 0 && ldx >= K && ldo >= N, "gemm_f32: bad sizes M=%d N=%d K=%d ldx=%d ldo=%d", M, N, K, ldx, ldo);
