@@ -509,6 +509,194 @@ __global__ __launch_bounds__(64 * NW) void paged_attention_mfma_kernel(AttnArgs 
 }
 
 // =====================================================================================
+// The same in true 32-bit (pages of a multiple of 4 tokens): v_mfma_f32_16x16x4_f32 multiplies and adds 32-bit numbers, as in the
+// 32-bit products.
+//
+// As above a wave owns the tile's 16 rows and both products run transposed; it walks the keys in chunks of 16.  A lane holds four neighbouring d
+// of its key (16 c + 4 g .. + 3), and instruction e of a piece multiplies d = 16 c + 4 g + e of the four lane groups: which d meet in
+// one instruction is free as long as both operands agree.  The scores come out as the keys 4 g .. 4 g + 3 of the lane's row, which is the second product's B operand as
+// it is, against four neighbouring keys of a d from the transposed values.  The next chunk's keys are requested when this one's scores are
+// there, its values when these are multiplied: a chunk is 64 instructions of 32 cycles at a head size of 128, and what a work-group of one or two chunks a wave
+// waits for is two trips to memory.  The general kernel above, whose lanes fetch single numbers into shared memory and whose scores are multiply-adds over it, took
+// (heads of 128, us, merge included; now): 4 requests decoding at 75 to 308 keys, 28 heads over 4, 27.8 -> 9.5; 8 at 1200 keys, 40 heads over 8, 90 -> 21; prompts of 75 to
+// 297 tokens in one step, 28 over 4, 196 -> 48, one of 1200 1019 -> 205; 3 heads of 32 at 26 keys 7.3 -> 4.0.  (Eight waves a work-group: the same within a tenth.)
+#define ATF_DC (AT_HD / 16)
+#define ATF_WAVES 4
+__global__ __launch_bounds__(64 * ATF_WAVES) void paged_attention_f32_mfma_kernel(AttnArgs a) {
+    __shared__ float park[(ATF_WAVES / 2) * ATM_SLOT];
+    __shared__ int bt_s[ATM_BT_MAX];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int li = lane & 15, g = lane >> 4;
+
+    const int tile = blockIdx.x;
+    const int group = a.heads / a.kv_heads;
+    const int chunks_h = (group + a.gcap - 1) / a.gcap;
+    const int kvh = blockIdx.y / chunks_h;
+    const int g0 = (blockIdx.y % chunks_h) * a.gcap;
+    const int gcount = min(a.gcap, group - g0);
+
+    const bool one_each = a.tile_req == nullptr;             // (as above: nothing to look up before length, block table and query)
+    const int req = one_each ? tile : a.tile_req[tile];
+    const int* bt_g = a.block_table + (size_t)req * a.bt_stride;
+    const bool bt_local = a.bt_stride <= ATM_BT_MAX;
+    if (bt_local)
+        for (int i = threadIdx.x; i < a.bt_stride; i += 64 * ATF_WAVES) bt_s[i] = bt_g[i];
+    const int tok0 = one_each ? 0 : a.tile_tok0[tile];
+    const int first = one_each ? req : a.req_indptr[req];
+    const int n_new = one_each ? 1 : a.req_indptr[req + 1] - first;
+    const int ctx = a.ctx_lens[req];
+    const int ntok = min(a.tq, n_new - tok0);
+
+    const int r_tok = li / a.gcap, r_g = li % a.gcap;
+    const bool row_ok = r_tok < ntok && r_g < gcount;
+    const int r_pos = ctx + tok0 + r_tok;
+    const int r_lo = a.window > 0 ? r_pos - a.window + 1 : 0;
+    const int r_head = kvh * group + g0 + r_g;
+    const int r_token = first + tok0 + r_tok;
+
+    f32x4_t qf[ATF_DC];
+    {
+        const float* q = (const float*)a.q + (size_t)r_token * a.q_stride + (size_t)r_head * AT_HD;
+#pragma unroll
+        for (int c = 0; c < ATF_DC; ++c) qf[c] = row_ok ? *(const f32x4_t*)(q + 16 * c + 4 * g) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+
+    const int key_hi = ctx + tok0 + ntok;
+    const int key_lo = a.window > 0 ? max(0, ctx + tok0 - a.window + 1) : 0;
+    const int ch_first = key_lo / 16, ch_last = (key_hi + 15) / 16;
+    const int per_split = (ch_last - ch_first + a.splits - 1) / a.splits;
+    const int ch_begin = ch_first + blockIdx.z * per_split, ch_end = min(ch_last, ch_begin + per_split);
+
+    const float *kp = (const float*)a.k_plane, *vp = (const float*)a.v_plane;
+    const int page = a.page;
+    const size_t kv_stride = (size_t)a.kv_heads * page * AT_HD;      // numbers per page, all KV heads
+    const size_t kvh_off = (size_t)kvh * page * AT_HD;
+    if (bt_local) __syncthreads();
+    auto page_of = [&](int key, int& off) {
+        int blk;
+        split_key(key, page, a.page_shift, blk, off);
+        return (size_t)(bt_local ? bt_s[blk] : bt_g[blk]) * kv_stride + kvh_off;
+    };
+    f32x4_t kf[ATF_DC], vf[ATM_DT];
+    auto fetch_keys = [&](int chunk) {
+        int off;
+        const float* row = kp + page_of(min(chunk * 16 + li, key_hi - 1), off);
+#pragma unroll
+        for (int c = 0; c < ATF_DC; ++c) kf[c] = *(const f32x4_t*)(row + (size_t)off * AT_HD + 16 * c + 4 * g);
+    };
+    auto fetch_values = [&](int chunk) {
+        const int key = chunk * 16 + 4 * g, there = key_hi - key;          // written keys from this lane's first on
+        int off;
+        const float* at = vp + page_of(min(key, key_hi - 1), off);
+        off &= ~3;                                                       // (a lane whose keys are all unwritten reads the last written ones and drops them)
+#pragma unroll
+        for (int t = 0; t < ATM_DT; ++t) {
+            vf[t] = *(const f32x4_t*)(at + off + (size_t)(16 * t + li) * page);
+            if (there < 4) {                                             // what is not written yet may be anything, Inf and NaN too: zeros
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (e >= there) vf[t][e] = 0.f;
+            }
+        }
+    };
+    const int tile_pos_min = ctx + tok0;
+    const int tile_lo_max = a.window > 0 ? max(0, ctx + tok0 + ntok - a.window) : 0;
+
+    float m = -INFINITY, l = 0.f;
+    f32x4_t acc[ATM_DT];
+#pragma unroll
+    for (int t = 0; t < ATM_DT; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+    int ch = ch_begin + wave;
+    if (ch < ch_end) {
+        fetch_keys(ch);
+        fetch_values(ch);
+    }
+    for (; ch < ch_end; ch += ATF_WAVES) {
+        f32x4_t s0 = f32x4_t{0.f, 0.f, 0.f, 0.f}, s1 = s0;              // (two chains: an instruction does not wait for the one before it)
+#pragma unroll
+        for (int c = 0; c < ATF_DC; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; e += 2) {
+                s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[c][e], qf[c][e], s0, 0, 0, 0);
+                s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[c][e + 1], qf[c][e + 1], s1, 0, 0, 0);
+            }
+        const bool more = ch + ATF_WAVES < ch_end;
+        if (more) fetch_keys(ch + ATF_WAVES);
+        const int kbase = ch * 16;
+        f32x4_t s = (s0 + s1) * a.scale;
+        if (kbase + 15 > tile_pos_min || kbase < tile_lo_max) {          // (uniform: not for chunks that every row sees whole)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int key = kbase + 4 * g + v;
+                if (!(row_ok && key <= r_pos && key >= r_lo)) s[v] = -INFINITY;
+            }
+        }
+        const float mloc = max_across_halves(max_across_rows(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]))));
+        const float m_new = fmaxf(m, mloc);
+        const float alpha = (m == -INFINITY) ? 0.f : expf(m - m_new);
+        f32x4_t p;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) p[v] = (s[v] == -INFINITY) ? 0.f : expf(s[v] - m_new);
+        l = l * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
+        const bool moved = __any(m_new != m);
+        m = m_new;
+#pragma unroll
+        for (int t = 0; t < ATM_DT; ++t) {
+            if (moved) acc[t] *= alpha;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int t = 0; t < ATM_DT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][e], p[e], acc[t], 0, 0, 0);
+        if (more) fetch_values(ch + ATF_WAVES);
+    }
+
+    // ---- merge the waves: the upper half of those left hands its state to the lower half, until one is left
+#pragma unroll
+    for (int half = ATF_WAVES / 2; half >= 1; half >>= 1) {
+        __syncthreads();
+        if (wave >= half && wave < 2 * half) {
+            float* dst = park + (size_t)(wave - half) * ATM_SLOT;
+#pragma unroll
+            for (int t = 0; t < ATM_DT; ++t) *(f32x4_t*)(dst + (t * 64 + lane) * 4) = acc[t];
+            dst[ATM_DT * 256 + lane] = m;
+            dst[ATM_DT * 256 + 64 + lane] = l;
+        }
+        __syncthreads();
+        if (wave < half) {
+            const float* src = park + (size_t)wave * ATM_SLOT;
+            const float mo = src[ATM_DT * 256 + lane], lo = src[ATM_DT * 256 + 64 + lane];
+            const float mm = fmaxf(m, mo);
+            const float sa = (m == -INFINITY) ? 0.f : expf(m - mm);
+            const float sb = (mo == -INFINITY) ? 0.f : expf(mo - mm);
+#pragma unroll
+            for (int t = 0; t < ATM_DT; ++t) acc[t] = acc[t] * sa + *(const f32x4_t*)(src + (t * 64 + lane) * 4) * sb;
+            l = l * sa + lo * sb;
+            m = mm;
+        }
+    }
+    if (wave != 0) return;
+    l += __shfl_xor(l, 16, TL_WAVE);
+    l += __shfl_xor(l, 32, TL_WAVE);
+    if (!row_ok) return;
+    const size_t pr = (size_t)r_token * a.heads + r_head;
+    if (a.splits == 1) {
+        const float inv = 1.f / l;
+#pragma unroll
+        for (int t = 0; t < ATM_DT; ++t) *(f32x4_t*)((float*)a.out + pr * AT_HD + 16 * t + 4 * g) = acc[t] * inv;
+    } else {
+        float* o = a.part_o + (pr * a.splits + blockIdx.z) * AT_HD;
+#pragma unroll
+        for (int t = 0; t < ATM_DT; ++t) *(f32x4_t*)(o + 16 * t + 4 * g) = acc[t];
+        if (g == 0) {
+            a.part_ml[(pr * a.splits + blockIdx.z) * 2] = m;
+            a.part_ml[(pr * a.splits + blockIdx.z) * 2 + 1] = l;
+        }
+    }
+}
+
+// =====================================================================================
 // Prompt portions on the matrix cores: 64 rows per work-group, keys and values through
 // shared memory.
 //
@@ -1340,7 +1528,9 @@ extern "C" int tl_paged_attention(const void* q, int q_stride, void* out, const 
     dim3 grid(tiles, kv_heads * chunks, splits), block(256);
     const bool aligned = ((uintptr_t)q % 16) == 0 && q_stride % 8 == 0 && ((uintptr_t)out % 8) == 0 &&
                          ((uintptr_t)k_plane % 16) == 0 && ((uintptr_t)v_plane % 8) == 0;
-    if (dtype == TL_DT_F32) paged_attention_kernel<float><<<grid, block, 0, stream>>>(a);
+    const bool whole = ((uintptr_t)q % 16) == 0 && q_stride % 4 == 0 && ((uintptr_t)out % 16) == 0 && ((uintptr_t)k_plane % 16) == 0 && ((uintptr_t)v_plane % 16) == 0;
+    if (dtype == TL_DT_F32 && page % 4 == 0 && whole && !general && head_dim == AT_HD) paged_attention_f32_mfma_kernel<<<grid, dim3(64 * ATF_WAVES), 0, stream>>>(a);
+    else if (dtype == TL_DT_F32) paged_attention_kernel<float><<<grid, block, 0, stream>>>(a);
     else if (dtype == TL_DT_BF16 && page % 4 == 0 && aligned && !general && head_dim == AT_HD) {
         if (waves == 8) paged_attention_mfma_kernel<8><<<grid, dim3(512), 0, stream>>>(a);
         else paged_attention_mfma_kernel<4><<<grid, block, 0, stream>>>(a);

@@ -23,6 +23,7 @@ from .base import KEEP_COMPUTE, KEEP_STORED, MIXERS, POSITION_ENCODINGS, LazyNor
 # (``ops.compute_units()``), the thresholds in keys and tokens were measured on an MI355X (256 units).
 _MIN_KEYS_PER_SPLIT = 256
 _MIN_KEYS_PER_SPLIT_32BIT = 64
+_MIN_NUMBERS_TO_SPLIT_32BIT = 160 * 128  # where the matrix cores run it: a head's keys times their size (300 keys of 128 take 14.4 us whole and 9.5 in 8 parts and their merge, 150 of 32 6.0 and 6.6)
 _PORTION_MIN_TOKENS = 16     # requests that bring at least this many tokens go to a prompt-portion kernel: the
                              # 128-row one where it is built (head size 64 or 128, pages of 8, 16, 32, ...
                              # tokens; measured on MI355X at 28/4 heads of 128: 2048 new tokens 222 -> 110 us,
@@ -129,7 +130,7 @@ class GQAttention(Mixer):
         self.w_o = self._place(tensors["o_proj.weight"], KEEP_COMPUTE)
 
     # -- the step -----------------------------------------------------------------
-    def _splits(self, ctx, tiles: int, longest: int | None = None) -> tuple[int, int]:
+    def _splits(self, ctx, tiles: int, longest: int | None = None, page_size: int = 16) -> tuple[int, int]:
         """(parts of every request's keys, waves of a work-group) for the 16-row kernel: work-groups of eight waves
         while one per tile and head group leaves compute units idle, with as many parts as give each unit one
         work-group; from there on work-groups of four waves, two to a unit, and no parts beyond that."""
@@ -138,12 +139,15 @@ class GQAttention(Mixer):
         base = max(1, tiles * self.kv_heads * chunks)
         units = self.compute_units
         waves = 8 if base <= units and self.dtype == torch.bfloat16 else 4      # (the 32-bit kernel has work-groups of four)
-        by_fill = -(-(units if waves == 8 else 2 * units) // base)      # four waves: enough work-groups to fill the units twice
+        # the 32-bit matrix-core kernel fills the units once (64 tiles of 1200 keys: 20.7 us in 4 parts, 21.7 in 8)
+        cores32 = self.dtype == torch.float32 and self.head_dim % 16 == 0 and page_size % 4 == 0
+        by_fill = -(-(units if waves == 8 or cores32 else 2 * units) // base)      # four waves: enough work-groups to fill the units twice
         longest = ctx.max_total_len if longest is None else longest
         longest = longest if self.window is None else min(longest, self.window + ctx.max_new_tokens)
-        # (the 32-bit engine's kernel walks its keys 32 at a time through shared memory, one work-group of four waves
-        # on a part: parts of 64 keys keep the compute units busy where 256 left most of them idle)
-        by_keys = max(1, longest // (_MIN_KEYS_PER_SPLIT if self.dtype == torch.bfloat16 else _MIN_KEYS_PER_SPLIT_32BIT))
+        # (the 32-bit engine's kernels have work-groups of four waves: parts of 64 keys keep the compute units busy where 256 left most of them idle)
+        by_keys = longest // (_MIN_KEYS_PER_SPLIT if self.dtype == torch.bfloat16 else _MIN_KEYS_PER_SPLIT_32BIT)
+        if cores32 and longest * self.head_dim < _MIN_NUMBERS_TO_SPLIT_32BIT:
+            by_keys = 1
         return max(1, min(by_fill, by_keys, 64)), waves
 
     takes_lazy_norm = True
@@ -245,7 +249,7 @@ class GQAttention(Mixer):
                 extra = dict(max_total_len=ctx.max_total_len, splits=splits, merge_tokens=(long[3], long[4]))
             kernel(q, out, k_plane, v_plane, table, ctx.req_indptr, ctx.ctx_lens, long[0], long[1], long[2], tq, *common, **extra)
             if short[2]:     # split over their keys; the merge of the parts is kept to the rows of these requests
-                splits, waves = self._splits(ctx, short[2], short[5])
+                splits, waves = self._splits(ctx, short[2], short[5], cache.page_size)
                 ops.paged_attention(q, out, k_plane, v_plane, table, ctx.req_indptr, ctx.ctx_lens,
                                     short[0], short[1], short[2], self.tile_tokens, *common,
                                     splits, merge_tokens=(short[3], short[4]), waves=waves)
@@ -253,7 +257,7 @@ class GQAttention(Mixer):
             tile_req, tile_tok0, tiles = ctx.tiles(self.tile_tokens)
             if ctx.decode_only and tiles == T:      # one token per request: no tile list to look up
                 tile_req = tile_tok0 = None
-            splits, waves = self._splits(ctx, tiles)
+            splits, waves = self._splits(ctx, tiles, page_size=cache.page_size)
             ops.paged_attention(q, out, k_plane, v_plane, table, ctx.req_indptr, ctx.ctx_lens,
                                 tile_req, tile_tok0, tiles, self.tile_tokens, *common, splits, waves=waves)
         return out
