@@ -120,3 +120,9 @@ def test_the_matrix_memory_in_chunks(monkeypatch, dtype, lens, H, dim, vdim):
             assert bool((off <= (8 * n + dim + 16) * 2.0 ** -24 * size + 1e-12).all()), (name, float((off / size).max() * 2.0 ** 24))
             torch.testing.assert_close(state[slots[r]].double(), left, rtol=1e-4, atol=1e-4)
     assert all(torch.equal(state[0], start[0]) for _, state in results.values())
+
+
+@pytest.mark.parametrize("lens", [[1024, 63, 2050], [1025, 1023]])
+def test_the_matrix_memory_over_several_rounds_of_its_gates(monkeypatch, lens):
+    """A work-group takes 16 stretches of 64 tokens a round: whole rounds, one more token and one less, and a short request beside."""
+    test_the_matrix_memory_in_chunks(monkeypatch, torch.float32, lens, 2, 20, 24)
