@@ -259,17 +259,6 @@ union FragK {
 #define ATM_BT_MAX 2048                    // block-table entries a work-group keeps in shared memory
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-// The larger of a lane's value and that of lane ^ 32 (lane ^ 16): the halves (the rows of 16 lanes) change places in
-// the vector unit, where a shuffle would go through shared memory and the step would wait for the trip.
-__device__ __forceinline__ float max_across_halves(float x) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float max_across_rows(float x) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void paged_attention_mfma_kernel(AttnArgs a) {
     __shared__ float park[(NW / 2) * ATM_SLOT];
@@ -483,8 +472,7 @@ __global__ __launch_bounds__(64 * NW) void paged_attention_mfma_kernel(AttnArgs 
         }
     }
     if (wave != 0) return;
-    l += __shfl_xor(l, 16, TL_WAVE);
-    l += __shfl_xor(l, 32, TL_WAVE);
+    l = sum_across_halves(sum_across_rows(l));
     if (!row_ok) return;
     if (a.splits == 1) {
         bf16_t* o = (bf16_t*)a.out + (size_t)r_token * a.heads * AT_HD + (size_t)r_head * AT_HD;
@@ -677,8 +665,7 @@ __global__ __launch_bounds__(64 * ATF_WAVES) void paged_attention_f32_mfma_kerne
         }
     }
     if (wave != 0) return;
-    l += __shfl_xor(l, 16, TL_WAVE);
-    l += __shfl_xor(l, 32, TL_WAVE);
+    l = sum_across_halves(sum_across_rows(l));
     if (!row_ok) return;
     const size_t pr = (size_t)r_token * a.heads + r_head;
     if (a.splits == 1) {
@@ -919,8 +906,7 @@ __global__ __launch_bounds__(256) void paged_attention_prefill_kernel(AttnArgs a
 #undef ATP_FETCH
 #undef ATP_PARK
 #undef ATP_PAGE_OF
-    l += __shfl_xor(l, 16, TL_WAVE);
-    l += __shfl_xor(l, 32, TL_WAVE);
+    l = sum_across_halves(sum_across_rows(l));
     if (!row_ok) return;
     bf16_t* o = (bf16_t*)a.out + (size_t)r_token * a.heads * AT_HD + (size_t)r_head * AT_HD;
     const float inv = 1.f / l;
@@ -1385,7 +1371,7 @@ __global__ __launch_bounds__(256, 2) void paged_attention_prompt_kernel(AttnArgs
         __syncthreads();
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    l += __shfl_xor(l, 32, TL_WAVE);
+    l = sum_across_halves(l);
     if (!row_ok) return;
     // lane holds d = 32 b + 8 q + 4 h + v of its row
     if (a.splits > 1) {

@@ -43,15 +43,51 @@ __device__ __forceinline__ void store4(bf16_t* p, float4 v) {
 // ---------------------------------------------------------------- reductions
 #define TL_WAVE 64
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = TL_WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, TL_WAVE);
+// A lane's value and that of lane ^ 32 (lane ^ 16), joined: the halves (the rows of 16 lanes) change places in the vector unit, where a shuffle would go through shared
+// memory and the step would wait for the trip.  All lanes of the wave take part.
+__device__ __forceinline__ float sum_across_halves(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float sum_across_rows(float v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float max_across_halves(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float max_across_rows(float v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+// The value of the lane BY places on in its row of 16, in a circle.
+template <int BY>
+__device__ __forceinline__ float row_turned(float v) {
+    const int i = __float_as_int(v);
+    return __int_as_float(__builtin_amdgcn_update_dpp(i, i, 0x120 + BY, 0xF, 0xF, false));
+}
+// Sums over neighbouring LANES (a power of two) and maxima over the wave, the same in each of the lanes.  The sums are those of a butterfly of exchanges with lane ^ 32, ^ 16, .. ^ 1, to
+// the bit: once the halves of a row hold the same sums, the lane 4 places on holds what lane ^ 4 does, and so on.  (As a butterfly of six shuffles a sum took 0.25 us longer: a
+// decode step's norm of 16 rows of 2048 numbers, which takes two, 4.1 -> 3.6 us, launch included.)
+template <int LANES>
+__device__ __forceinline__ float lanes_sum(float v) {
+    if constexpr (LANES > 32) v = sum_across_halves(v);
+    if constexpr (LANES > 16) v = sum_across_rows(v);
+    static_assert(LANES >= 16, "whole rows of the wave");
+    v += row_turned<8>(v);
+    v += row_turned<4>(v);
+    v += row_turned<2>(v);
+    v += row_turned<1>(v);
     return v;
 }
+__device__ __forceinline__ float wave_sum(float v) { return lanes_sum<TL_WAVE>(v); }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = TL_WAVE / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, TL_WAVE));
-    return v;
+    v = max_across_rows(max_across_halves(v));
+    v = fmaxf(v, row_turned<8>(v));
+    v = fmaxf(v, row_turned<4>(v));
+    v = fmaxf(v, row_turned<2>(v));
+    return fmaxf(v, row_turned<1>(v));
 }
 
 __device__ __forceinline__ float sigmoid(float v) { return 1.f / (1.f + expf(-v)); }

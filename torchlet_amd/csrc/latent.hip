@@ -695,8 +695,7 @@ latent_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __r
             float mloc = sc[0];
 #pragma unroll
             for (int i = 1; i < 8; ++i) mloc = fmaxf(mloc, sc[i]);
-            mloc = fmaxf(mloc, __shfl_xor(mloc, 16, 64));
-            mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
+            mloc = max_across_halves(max_across_rows(mloc));
             const float m_new = fmaxf(m, mloc);
             const float alpha = (m == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m - m_new);     // (m_new may still be -inf: a step wholly before this query's window)
             const bool moved = __any(m_new != m);    // the sums are rescaled only when some query's maximum moved
@@ -740,8 +739,7 @@ latent_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __r
     } else {
         for (int k0 = kfirst; k0 <= last; k0 += stride) step(stage0, k0);
     }
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    l = sum_across_halves(sum_across_rows(l));
     if (!row_ok) return;
     if (splits == 1) {
         float inv = l > 0.f ? 1.f / l : 0.f;

@@ -336,8 +336,7 @@ local_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __re
                 sc[e] = (key <= my_last && key >= my_first) ? cap_score_fast(raw, cap, inv_cap) * LA_LOG2E : -INFINITY;
                 mx = fmaxf(mx, sc[e]);
             }
-            mx = fmaxf(mx, __shfl_xor(mx, 16, TL_WAVE));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, TL_WAVE));
+            mx = max_across_halves(max_across_rows(mx));
             const float m_new = fmaxf(m, mx);
             const float m_use = m_new == -INFINITY ? 0.f : m_new;   // a token that has seen no key yet
             const float keep = __builtin_amdgcn_exp2f(m - m_use);   // (0 while m is -inf)
@@ -387,8 +386,7 @@ local_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __re
     }
     // the first token reads furthest back; pages before may be gone
     run(k_plane, v_plane, table, table_width, mask.first(p0), p_last, my_lo, my_p);
-    l += __shfl_xor(l, 16, TL_WAVE);
-    l += __shfl_xor(l, 32, TL_WAVE);
+    l = sum_across_halves(sum_across_rows(l));
     // ---- the four waves' shares are joined: per token the maxima, the sums and the outputs, in the order of the waves
     float* sm_m = la_smem;                              // [4][16], in units of log 2
     float* sm_l = sm_m + LAM_WAVES * LAM_TOKENS;        // [4][16]
@@ -933,7 +931,7 @@ local_prompt_kernel(LocalArgs a) {
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
-    l += __shfl_xor(l, 32, TL_WAVE);
+    l = sum_across_halves(l);
     if (!row_ok) return;
     // lane holds column 32 b + 8 q + 4 h + v of its row
     float norm = a.gain;

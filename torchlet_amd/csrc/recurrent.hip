@@ -408,11 +408,8 @@ gated_norm_pieces_kernel(const float* __restrict__ o, const T* __restrict__ gate
             ss = fmaf(v.x, v.x, ss); ss = fmaf(v.y, v.y, ss); ss = fmaf(v.z, v.z, ss); ss = fmaf(v.w, v.w, ss);
         }
     }
-    if (LANES > TL_WAVE) ss = block_sum(ss, red);
-    else {
-#pragma unroll
-        for (int k = LANES / 2; k > 0; k >>= 1) ss += __shfl_xor(ss, k, TL_WAVE);
-    }
+    if constexpr (LANES > TL_WAVE) ss = block_sum(ss, red);
+    else ss = lanes_sum<LANES>(ss);
     const float inv = 1.f / sqrtf(ss / (float)vdim + eps);
     if (!live) return;
     T* dst = out + (size_t)t * out_ld + (size_t)h * vdim;
