@@ -40,6 +40,15 @@ __device__ __forceinline__ void store4(bf16_t* p, float4 v) {
     *(uint2*)p = t;
 }
 
+// Four: four neighbouring numbers as they are stored, widened where they are used (half the registers of a piece on its way).
+template <typename T> struct Four;
+template <> struct Four<float> { typedef float4 type; };
+template <> struct Four<bf16_t> { typedef ushort4 type; };
+__device__ __forceinline__ float4 widen4(float4 v) { return v; }
+__device__ __forceinline__ float4 widen4(ushort4 v) {
+    return make_float4(to_float(bf16_t{v.x}), to_float(bf16_t{v.y}), to_float(bf16_t{v.z}), to_float(bf16_t{v.w}));
+}
+
 // ---------------------------------------------------------------- reductions
 #define TL_WAVE 64
 

@@ -1,6 +1,8 @@
 // Row-wise kernels: embedding gather, residual add + RMSNorm, rotary position
 // encoding fused with the write of keys and values into cache pages, SwiGLU gate.
 // Each is templated on the activation type (float or bfloat16); all arithmetic is float.
+#include <limits.h>
+
 #include "common.h"
 
 // ------------------------------------------------------------------ embedding
@@ -115,66 +117,106 @@ __device__ __forceinline__ void add_slab_pairs(const float* src, size_t stride, 
         for (int v = 0; v < 4; ++v) { lo[v] += p[u][v]; hi[v] += q[u][v]; }
 }
 
-template <typename T, int IT>
-__global__ void add_rmsnorm_reg_kernel(float* __restrict__ residual, const void* __restrict__ pending, int parts, size_t part_stride,
-                                       const void* __restrict__ weight, int weight_f32, float eps, float gain,
-                                       T* __restrict__ out, const int* __restrict__ rows, int hidden) {
+// What a branch left for a row, fetched without a question on the way: PC 0 a row of T, 1, 2, 3, 4 or 8 that many float slabs, BRANCH_ANY more than four (four ahead, the others
+// four at a time where they are added), BRANCH_LATE any number (none ahead), BRANCH_NONE nothing.  Where the kind is known at run time alone, every answer ends in a wait for what
+// was requested before it, and a decode step's norm is little but its trips to memory: kind and types are the template's, and pieces beyond the row's end are its last piece
+// again, kept out of sums and stores.
+// (us after the kernel that wrote the slabs, kind at run time -> by template: add_rmsnorm, 8 rows of 3584 with four slabs 4.0 -> 3.4, one row of 2048 with eight 3.75 -> 2.9, 16 of 5120
+// with three 4.5 -> 4.1, 512 of 5120 with three 15.9 -> 14.6; scaled_add_rmsnorm, one row of 2048 2.4 -> 2.1, 4 of 4096 with four slabs 3.6 -> 3.2, 2048 of 2048 11.3 -> 10.3; sandwich_norm, 16 of 2048
+// with four 3.7 -> 3.3.  What is asked for ahead takes registers: with more rows than compute units and many slabs fewer rows share a unit, and 2048 of 2048 with four slabs took
+// add_rmsnorm 19.9 instead of 18.6: late there.)
+#define BRANCH_NONE (-1)
+#define BRANCH_ANY 9
+#define BRANCH_LATE 10
+template <typename T, int PC, int NP>
+struct Branch {
+    static constexpr int N = PC == BRANCH_ANY ? 4 : PC == BRANCH_LATE ? 0 : PC;
+    float4 z[NP][N > 0 ? N : 1];
+    typename Four<T>::type row[NP];
+    const float* slabs;
+    size_t stride;
+    int parts;
+    __device__ __forceinline__ void fetch(const void* pending, int count, size_t part_stride, size_t off, const int (&at)[NP]) {
+        slabs = (const float*)pending + off;
+        stride = part_stride;
+        parts = count;
+#pragma unroll
+        for (int n = 0; n < NP; ++n) {
+            if constexpr (PC == 0) row[n] = *(const typename Four<T>::type*)((const T*)pending + off + at[n]);
+#pragma unroll
+            for (int u = 0; u < N; ++u) z[n][u] = *(const float4*)(slabs + u * stride + at[n]);
+        }
+    }
+    // piece n of the row, or the slabs in their order, on top of r
+    __device__ __forceinline__ void add(int n, int at, float (&r)[4]) const {
+        if constexpr (PC == 0) {
+            const float4 y = widen4(row[n]);
+            r[0] += y.x; r[1] += y.y; r[2] += y.z; r[3] += y.w;
+        }
+#pragma unroll
+        for (int u = 0; u < N; ++u) { r[0] += z[n][u].x; r[1] += z[n][u].y; r[2] += z[n][u].z; r[3] += z[n][u].w; }
+        if constexpr (PC == BRANCH_ANY || PC == BRANCH_LATE) {
+            int q = N;
+            for (; q + 4 <= parts; q += 4) add_slabs<4>(slabs + q * stride + at, stride, r);
+            if (parts - q == 3) add_slabs<3>(slabs + q * stride + at, stride, r);
+            else if (parts - q == 2) add_slabs<2>(slabs + q * stride + at, stride, r);
+            else if (parts - q == 1) add_slabs<1>(slabs + q * stride + at, stride, r);
+        }
+    }
+};
+// F with the kind of a branch as its template's number; `late`: the least number of slabs that are not asked for ahead; EIGHT: eight are asked for at once.
+#define TL_BRANCH(pending, parts, late, EIGHT, F)             \
+    do {                                                      \
+        if (!(pending)) { F(BRANCH_NONE); }                   \
+        else if ((parts) == 0) { F(0); }                      \
+        else if ((parts) >= (late)) { F(BRANCH_LATE); }       \
+        else if ((parts) == 1) { F(1); }                      \
+        else if ((parts) == 2) { F(2); }                      \
+        else if ((parts) == 3) { F(3); }                      \
+        else if ((parts) == 4) { F(4); }                      \
+        else if ((EIGHT) && (parts) == 8) { F(((EIGHT) ? 8 : BRANCH_ANY)); } \
+        else { F(BRANCH_ANY); }                               \
+    } while (0)
+
+template <typename T, typename W, int IT, int PC>
+__global__ void __launch_bounds__(1024)
+add_rmsnorm_reg_kernel(float* __restrict__ residual, const void* __restrict__ pending, int parts, size_t part_stride, const W* __restrict__ weight, float eps, float gain,
+                       T* __restrict__ out, const int* __restrict__ rows, int hidden) {
     __shared__ float red[16];
-    const int orow = blockIdx.x;
-    const int srow = rows ? rows[orow] : orow;
-    float* res = residual + (size_t)srow * hidden;
-    const T* pen = (pending && parts == 0) ? (const T*)pending + (size_t)srow * hidden : nullptr;
-    const float* pparts = (pending && parts > 0) ? (const float*)pending + (size_t)srow * hidden : nullptr;
-    const bool update = (pending != nullptr) && (rows == nullptr);
-    float r[IT][4], wv[IT][4];
+    const int srow = rows ? rows[blockIdx.x] : blockIdx.x;
+    const size_t off = (size_t)srow * hidden;
+    int at[IT];
+    float4 x[IT];
+    typename Four<W>::type wv[IT];
+    Branch<T, PC, IT> branch;
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+        at[it] = min((int)(it * blockDim.x + threadIdx.x) * 4, hidden - 4);
+        x[it] = *(const float4*)(residual + off + at[it]);
+    }
+    branch.fetch(pending, parts, part_stride, off, at);
+#pragma unroll
+    for (int it = 0; it < IT; ++it) wv[it] = *(const typename Four<W>::type*)(weight + at[it]);
+    float r[IT][4];
     float ss = 0.f;
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-        const int i = (it * blockDim.x + threadIdx.x) * 4;
-        if (i < hidden) {
-            Vec4<float>::load(res + i, r[it]);
-            if (pen) {
-                float p[4];
-                Vec4<T>::load(pen + i, p);
-#pragma unroll
-                for (int v = 0; v < 4; ++v) r[it][v] += p[v];
-            }
-            if (pparts) {
-                // four slabs at a time, all requested before the first is added (a loop over a count known
-                // only at run time fetches one slab after the other: a trip to memory each); the sums are
-                // added in the order of the slabs either way.  The last two or three slabs are a group as well
-                // (three slabs, as for the matrices 5120 wide, were three trips).
-                int q = 0;
-                for (; q + 4 <= parts; q += 4) add_slabs<4>(pparts + q * part_stride + i, part_stride, r[it]);
-                if (parts - q == 3) add_slabs<3>(pparts + q * part_stride + i, part_stride, r[it]);
-                else if (parts - q == 2) add_slabs<2>(pparts + q * part_stride + i, part_stride, r[it]);
-                else if (parts - q == 1) add_slabs<1>(pparts + q * part_stride + i, part_stride, r[it]);
-            }
-            if (weight_f32) Vec4<float>::load((const float*)weight + i, wv[it]);
-            else Vec4<bf16_t>::load((const bf16_t*)weight + i, wv[it]);
+        r[it][0] = x[it].x; r[it][1] = x[it].y; r[it][2] = x[it].z; r[it][3] = x[it].w;
+        branch.add(it, at[it], r[it]);
+        if ((int)(it * blockDim.x + threadIdx.x) * 4 < hidden) {
 #pragma unroll
             for (int v = 0; v < 4; ++v) ss += r[it][v] * r[it][v];
-        }
-    }
-    if (update) {
-#pragma unroll
-        for (int it = 0; it < IT; ++it) {
-            const int i = (it * blockDim.x + threadIdx.x) * 4;
-            if (i < hidden) Vec4<float>::store(res + i, r[it]);
+            if (PC != BRANCH_NONE && !rows) store4(residual + off + at[it], make_float4(r[it][0], r[it][1], r[it][2], r[it][3]));
         }
     }
     ss = block_sum(ss, red);
     const float inv = rsqrtf(ss / (float)hidden + eps) * gain;
-    T* dst = out + (size_t)orow * hidden;
+    T* dst = out + (size_t)blockIdx.x * hidden;
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-        const int i = (it * blockDim.x + threadIdx.x) * 4;
-        if (i < hidden) {
-            float o[4];
-#pragma unroll
-            for (int v = 0; v < 4; ++v) o[v] = r[it][v] * inv * wv[it][v];
-            Vec4<T>::store(dst + i, o);
-        }
+        if ((int)(it * blockDim.x + threadIdx.x) * 4 >= hidden) continue;
+        const float4 w = widen4(wv[it]);
+        store4(dst + at[it], make_float4(r[it][0] * inv * w.x, r[it][1] * inv * w.y, r[it][2] * inv * w.z, r[it][3] * inv * w.w));
     }
 }
 
@@ -184,18 +226,29 @@ static void launch_add_rmsnorm(float* residual, const void* pending, int parts, 
     const bool aligned = hidden % 4 == 0 && ((uintptr_t)residual % 16) == 0 && ((uintptr_t)out % 16) == 0 &&
                          ((uintptr_t)pending % 16) == 0 && ((uintptr_t)weight % 16) == 0;
     dim3 grid(out_rows);
-    if (aligned && hidden <= 1024)
-        add_rmsnorm_reg_kernel<T, 1><<<grid, 256, 0, stream>>>(residual, pending, parts, part_stride, weight, weight_f32, eps, gain, out, rows, hidden);
-    else if (aligned && hidden <= 2048)
-        add_rmsnorm_reg_kernel<T, 2><<<grid, 256, 0, stream>>>(residual, pending, parts, part_stride, weight, weight_f32, eps, gain, out, rows, hidden);
-    else if (aligned && hidden <= 4096)
-        add_rmsnorm_reg_kernel<T, 2><<<grid, 512, 0, stream>>>(residual, pending, parts, part_stride, weight, weight_f32, eps, gain, out, rows, hidden);
-    else if (aligned && hidden <= 8192)
-        add_rmsnorm_reg_kernel<T, 4><<<grid, 512, 0, stream>>>(residual, pending, parts, part_stride, weight, weight_f32, eps, gain, out, rows, hidden);
-    else if (aligned && hidden <= 16384)
-        add_rmsnorm_reg_kernel<T, 4><<<grid, 1024, 0, stream>>>(residual, pending, parts, part_stride, weight, weight_f32, eps, gain, out, rows, hidden);
-    else
+    const int late = out_rows > 256 ? 5 : INT_MAX;
+#define TL_AR_W(W, IT, THREADS, PC) add_rmsnorm_reg_kernel<T, W, IT, PC><<<grid, THREADS, 0, stream>>>(residual, pending, parts, part_stride, (const W*)weight, eps, gain, out, rows, hidden)
+#define TL_AR_1(PC) do { if (weight_f32) TL_AR_W(float, 1, 256, PC); else TL_AR_W(bf16_t, 1, 256, PC); } while (0)
+#define TL_AR_2(PC) do { if (weight_f32) TL_AR_W(float, 2, threads, PC); else TL_AR_W(bf16_t, 2, threads, PC); } while (0)
+#define TL_AR_3(PC) do { if (weight_f32) TL_AR_W(float, 3, threads, PC); else TL_AR_W(bf16_t, 3, threads, PC); } while (0)
+#define TL_AR_4(PC) do { if (weight_f32) TL_AR_W(float, 4, threads, PC); else TL_AR_W(bf16_t, 4, threads, PC); } while (0)
+    if (aligned && hidden <= 1024) TL_BRANCH(pending, parts, late, true, TL_AR_1);
+    else if (aligned && hidden <= 4096) {
+        const int threads = hidden <= 2048 ? 256 : 512;
+        TL_BRANCH(pending, parts, late, true, TL_AR_2);
+    } else if (aligned && hidden <= 6144) {
+        const int threads = 512;
+        TL_BRANCH(pending, parts, late, false, TL_AR_3);
+    } else if (aligned && hidden <= 16384) {
+        const int threads = hidden <= 8192 ? 512 : 1024;
+        TL_BRANCH(pending, parts, late, false, TL_AR_4);
+    } else
         add_rmsnorm_kernel<T><<<grid, hidden >= 2048 ? 512 : 256, 0, stream>>>(residual, pending, parts, part_stride, weight, weight_f32, eps, gain, out, rows, hidden);
+#undef TL_AR_4
+#undef TL_AR_3
+#undef TL_AR_2
+#undef TL_AR_1
+#undef TL_AR_W
 }
 
 // parts == 0: `pending` is [rows, hidden] of the activation type (or null); parts > 0: `pending` is
@@ -586,49 +639,44 @@ __global__ void scaled_add_rmsnorm_kernel(float* __restrict__ residual, const vo
 // The same with a row in registers, four neighbouring numbers to a piece and IT pieces to a thread: everything a row needs is requested at once (slabs four at a
 // time, added up in their order), where the kernel above fetches the row again after the sum and the slabs one after the other.  Measured, rows of 2048
 // numbers: one row 5.2 -> 2.4 us, with four slabs 7.4 -> 2.5; 2048 rows 11.4 -> 7.9, with four slabs 22.4 -> 17.3.
-template <typename T, int IT>
-__global__ void scaled_add_rmsnorm_reg_kernel(float* __restrict__ residual, const void* __restrict__ pending, int parts, size_t part_stride, float alpha,
-                                              const void* __restrict__ weight, int weight_f32, float eps, T* __restrict__ out, int hidden) {
+template <typename T, typename W, int IT, int PC>
+__global__ void __launch_bounds__(1024)
+scaled_add_rmsnorm_reg_kernel(float* __restrict__ residual, const void* __restrict__ pending, int parts, size_t part_stride, float alpha, const W* __restrict__ weight, float eps,
+                              T* __restrict__ out, int hidden) {
     __shared__ float red[16];
-    const size_t at = (size_t)blockIdx.x * hidden;
-    float r[IT][4], wv[IT][4];
+    const size_t off = (size_t)blockIdx.x * hidden;
+    int at[IT];
+    float4 x[IT];
+    typename Four<W>::type wv[IT];
+    Branch<T, PC, IT> branch;
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+        at[it] = min((int)(it * blockDim.x + threadIdx.x) * 4, hidden - 4);
+        x[it] = *(const float4*)(residual + off + at[it]);
+    }
+    branch.fetch(pending, parts, part_stride, off, at);
+#pragma unroll
+    for (int it = 0; it < IT; ++it) wv[it] = *(const typename Four<W>::type*)(weight + at[it]);
+    float r[IT][4];
     float ss = 0.f;
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-        const int i = (it * blockDim.x + threadIdx.x) * 4;
-        if (i < hidden) {
-            float x[4], y[4] = {0.f, 0.f, 0.f, 0.f};
-            Vec4<float>::load(residual + at + i, x);
-            if (weight_f32) Vec4<float>::load((const float*)weight + i, wv[it]);
-            else Vec4<bf16_t>::load((const bf16_t*)weight + i, wv[it]);
-            if (pending && parts == 0) Vec4<T>::load((const T*)pending + at + i, y);
-            if (pending && parts > 0) {
-                const float* slabs = (const float*)pending + at + i;
-                int q = 0;
-                for (; q + 4 <= parts; q += 4) add_slabs<4>(slabs + q * part_stride, part_stride, y);
-                if (parts - q == 3) add_slabs<3>(slabs + q * part_stride, part_stride, y);
-                else if (parts - q == 2) add_slabs<2>(slabs + q * part_stride, part_stride, y);
-                else if (parts - q == 1) add_slabs<1>(slabs + q * part_stride, part_stride, y);
-            }
+        float y[4] = {0.f, 0.f, 0.f, 0.f};
+        branch.add(it, at[it], y);
+        r[it][0] = alpha * x[it].x + y[0]; r[it][1] = alpha * x[it].y + y[1]; r[it][2] = alpha * x[it].z + y[2]; r[it][3] = alpha * x[it].w + y[3];
+        if ((int)(it * blockDim.x + threadIdx.x) * 4 < hidden) {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                r[it][v] = alpha * x[v] + y[v];
-                ss = fmaf(r[it][v], r[it][v], ss);
-            }
+            for (int v = 0; v < 4; ++v) ss = fmaf(r[it][v], r[it][v], ss);
         }
     }
     ss = block_sum(ss, red);
     const float inv = 1.f / sqrtf(ss / (float)hidden + eps);
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-        const int i = (it * blockDim.x + threadIdx.x) * 4;
-        if (i < hidden) {
-            float y[4];
-#pragma unroll
-            for (int v = 0; v < 4; ++v) y[v] = r[it][v] * inv * wv[it][v];
-            Vec4<float>::store(residual + at + i, y);
-            if (out) Vec4<T>::store(out + at + i, y);
-        }
+        if ((int)(it * blockDim.x + threadIdx.x) * 4 >= hidden) continue;
+        const float4 w = widen4(wv[it]), y = make_float4(r[it][0] * inv * w.x, r[it][1] * inv * w.y, r[it][2] * inv * w.z, r[it][3] * inv * w.w);
+        store4(residual + off + at[it], y);
+        if (out) store4(out + off + at[it], y);
     }
 }
 
@@ -637,16 +685,24 @@ template <typename T>
 static void launch_scaled_add_rmsnorm(float* residual, const void* pending, int parts, size_t part_stride, float alpha, const void* weight, int weight_f32,
                                       float eps, T* out, int rows, int hidden, hipStream_t stream) {
     const bool aligned = hidden % 4 == 0 && (((uintptr_t)residual | (uintptr_t)pending | (uintptr_t)weight | (uintptr_t)out) & 15) == 0;
-#define TL_SAR(IT, THREADS) scaled_add_rmsnorm_reg_kernel<T, IT><<<rows, THREADS, 0, stream>>>(residual, pending, parts, part_stride, alpha, weight, weight_f32, eps, out, hidden)
-    if (aligned && hidden <= 1024) TL_SAR(1, 256);
-    else if (aligned && hidden <= 2048) TL_SAR(1, 512);
-    else if (aligned && hidden <= 4096) TL_SAR(2, 512);
-    else if (aligned && hidden <= 8192) TL_SAR(4, 512);
-    else if (aligned && hidden <= 16384) TL_SAR(4, 1024);
+#define TL_SAR_W(W, IT, PC) scaled_add_rmsnorm_reg_kernel<T, W, IT, PC><<<rows, threads, 0, stream>>>(residual, pending, parts, part_stride, alpha, (const W*)weight, eps, out, hidden)
+#define TL_SAR_1(PC) do { if (weight_f32) TL_SAR_W(float, 1, PC); else TL_SAR_W(bf16_t, 1, PC); } while (0)
+#define TL_SAR_2(PC) do { if (weight_f32) TL_SAR_W(float, 2, PC); else TL_SAR_W(bf16_t, 2, PC); } while (0)
+#define TL_SAR_3(PC) do { if (weight_f32) TL_SAR_W(float, 3, PC); else TL_SAR_W(bf16_t, 3, PC); } while (0)
+#define TL_SAR_4(PC) do { if (weight_f32) TL_SAR_W(float, 4, PC); else TL_SAR_W(bf16_t, 4, PC); } while (0)
+    const int threads = hidden <= 1024 ? 256 : hidden <= 8192 ? 512 : 1024, late = rows > 256 ? 5 : INT_MAX;
+    if (aligned && hidden <= 2048) TL_BRANCH(pending, parts, late, true, TL_SAR_1);
+    else if (aligned && hidden <= 4096) TL_BRANCH(pending, parts, late, true, TL_SAR_2);
+    else if (aligned && hidden <= 6144) TL_BRANCH(pending, parts, late, false, TL_SAR_3);
+    else if (aligned && hidden <= 16384) TL_BRANCH(pending, parts, late, false, TL_SAR_4);
     else
         scaled_add_rmsnorm_kernel<T><<<rows, hidden <= 512 ? 128 : hidden <= 2048 ? 256 : 512, 0, stream>>>(residual, pending, parts, part_stride, alpha, weight, weight_f32,
                                                                                                          eps, out, hidden);
-#undef TL_SAR
+#undef TL_SAR_4
+#undef TL_SAR_3
+#undef TL_SAR_2
+#undef TL_SAR_1
+#undef TL_SAR_W
 }
 
 extern "C" int tl_scaled_add_rmsnorm(void* residual, const void* pending, int parts, int total_rows, float alpha, const void* weight,
@@ -1315,6 +1371,62 @@ sandwich_norm_rows_kernel(float* __restrict__ residual, const void* __restrict__
     store_row<NP>(out + (size_t)blockIdx.x * hidden, hidden, r);
 }
 
+// The same where the branch's kind is known (see Branch) and the norms' weights are vectors: what is optional is fetched from the residual's row instead where it is not there, and left out of the sums.
+template <typename T, int NP, int PC>
+__global__ void __launch_bounds__(1024)
+sandwich_norm_branch_kernel(float* __restrict__ residual, const void* __restrict__ pending, int parts, size_t part_stride, const float* __restrict__ post, float post_eps, float branch_gain,
+                            const float* __restrict__ extra, const float* __restrict__ weight, float eps, float gain, T* __restrict__ out, const int* __restrict__ rows, int hidden) {
+    __shared__ float red[16];
+    const int srow = rows ? rows[blockIdx.x] : blockIdx.x;
+    const size_t off = (size_t)srow * hidden;
+    const float *post_at = post ? post : residual + off, *extra_at = extra ? extra + off : residual + off, *weight_at = weight ? weight : residual + off;
+    int at[NP];
+    float4 x[NP], pw[NP], ex[NP], w[NP];
+    Branch<T, PC, NP> branch;
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+        at[n] = min((int)(threadIdx.x + n * blockDim.x) * 4, hidden - 4);
+        x[n] = *(const float4*)(residual + off + at[n]);
+    }
+    branch.fetch(pending, parts, part_stride, off, at);
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+        ex[n] = *(const float4*)(extra_at + at[n]);
+        pw[n] = *(const float4*)(post_at + at[n]);
+        w[n] = *(const float4*)(weight_at + at[n]);
+    }
+    RowPieces<NP> r, y;
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+        const bool in = (int)(threadIdx.x + n * blockDim.x) * 4 < hidden;
+        float s[4] = {0.f, 0.f, 0.f, 0.f};
+        branch.add(n, at[n], s);
+        const float xs[4] = {x[n].x, x[n].y, x[n].z, x[n].w};
+#pragma unroll
+        for (int v = 0; v < 4; ++v) { y.v[n][v] = in ? s[v] : 0.f; r.v[n][v] = in ? xs[v] : 0.f; }
+    }
+    const float inv_y = branch_gain * (post ? rsqrtf(block_sum(row_squares(y), red) / (float)hidden + post_eps) : 1.f);
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+        const bool in = (int)(threadIdx.x + n * blockDim.x) * 4 < hidden;
+        const float e4[4] = {ex[n].x, ex[n].y, ex[n].z, ex[n].w}, p4[4] = {pw[n].x, pw[n].y, pw[n].z, pw[n].w};
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            if (extra && in) r.v[n][v] += e4[v];
+            r.v[n][v] += post ? y.v[n][v] * inv_y * p4[v] : y.v[n][v] * inv_y;
+        }
+    }
+    if (!rows) store_row<NP>(residual + off, hidden, r);
+    const float inv = weight ? rsqrtf(block_sum(row_squares(r), red) / (float)hidden + eps) * gain : gain;
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+        const float w4[4] = {w[n].x, w[n].y, w[n].z, w[n].w};
+#pragma unroll
+        for (int v = 0; v < 4; ++v) r.v[n][v] = weight ? r.v[n][v] * inv * w4[v] : r.v[n][v] * inv;
+    }
+    store_row<NP>(out + (size_t)blockIdx.x * hidden, hidden, r);
+}
+
 extern "C" int tl_sandwich_norm(void* residual, const void* pending, int parts, int part_rows, const void* post, int post_n, float post_eps,
                                 float branch_gain, const void* extra, const void* weight, int weight_n, float eps, float gain, void* out, const void* rows,
                                 int out_rows, int hidden, int act_dtype, hipStream_t stream) {
@@ -1326,6 +1438,15 @@ extern "C" int tl_sandwich_norm(void* residual, const void* pending, int parts, 
     const uintptr_t bits = (uintptr_t)residual | (uintptr_t)pending | (uintptr_t)post | (uintptr_t)extra | (uintptr_t)weight | (uintptr_t)out;
     if (hidden % 4 == 0 && bits % 16 == 0) {
         const RowPlan plan = plan_row(hidden);
+        // (rows of one piece a thread: with two, 16 rows of 5120 with three slabs took 5.9 us instead of 5.2; eight slabs asked for at once 4.5 instead of 3.8.  A hidden size of one has no rows here)
+        if (pending && act_dtype == TL_DT_BF16 && plan.pieces == 1 && (!post || post_n != 1) && (!weight || weight_n != 1)) {
+#define TL_SB(PC) sandwich_norm_branch_kernel<bf16_t, 1, PC><<<out_rows, plan.threads, 0, stream>>>((float*)residual, pending, parts, part_stride, (const float*)post, post_eps, branch_gain, \
+        (const float*)extra, (const float*)weight, eps, gain, (bf16_t*)out, (const int*)rows, hidden)
+            TL_BRANCH(pending, parts, INT_MAX, false, TL_SB);
+#undef TL_SB
+            TL_CHECK_LAUNCH("sandwich_norm");
+            return TL_OK;
+        }
 #define TL_SN(T, N)                                                                                                                               \
     sandwich_norm_rows_kernel<T, N><<<out_rows, plan.threads, 0, stream>>>((float*)residual, pending, parts, part_stride, (const float*)post, post_n, post_eps, \
         branch_gain, (const float*)extra, (const float*)weight, weight_n, eps, gain, (T*)out, (const int*)rows, hidden)

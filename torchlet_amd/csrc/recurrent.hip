@@ -366,15 +366,7 @@ gated_row_norm_kernel(const float* __restrict__ o, const T* __restrict__ gate, i
 // The same with a stretch's numbers in registers: LANES threads to a stretch (part of a wave, a wave, or a work-group of its own), NP pieces of four
 // neighbouring numbers to a thread, all requested before the first is used, so that a stretch costs one trip to memory instead of one per number
 // of a thread and pass.  What bounds it is its bytes on prompts and its launch and that one trip in decode steps: 4 tokens of 4096 numbers 15.3 -> 4.0 us, of
-// 8192 27.5 -> 5.4 us (one number a thread and trip before).  (Four: a piece as it is stored, widened where it is used: half the registers of one on its way.)
-template <typename T> struct Four;
-template <> struct Four<float> { typedef float4 type; };
-template <> struct Four<bf16_t> { typedef ushort4 type; };
-__device__ __forceinline__ float4 widen4(float4 v) { return v; }
-__device__ __forceinline__ float4 widen4(ushort4 v) {
-    return make_float4(to_float(bf16_t{v.x}), to_float(bf16_t{v.y}), to_float(bf16_t{v.z}), to_float(bf16_t{v.w}));
-}
-
+// 8192 27.5 -> 5.4 us (one number a thread and trip before). 
 template <typename T, int NP, int LANES>
 __global__ void __launch_bounds__(LANES > 256 ? LANES : 256)
 gated_norm_pieces_kernel(const float* __restrict__ o, const T* __restrict__ gate, int gate_ld, const void* __restrict__ weight, int weight_f32,
