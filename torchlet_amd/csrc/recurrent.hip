@@ -1835,6 +1835,162 @@ extern "C" int tl_wkv_scan(const void* rkv, int ld, int k_off, int v_off, const 
     return TL_OK;
 }
 
+// The same with what stands before and behind it, for steps of one token a request: the decays are made from their low-rank sums (channel_decay above), and the output goes through the norm of its
+// head and the gate (gated_head_norm) before it is stored, all in the sums' order there.  A work-group has a whole head of a request: sixteen lanes a column and CG columns to each, whose states
+// are all requested at the start, beside the token's numbers and the matrix of the decays; what a step waits for is then one trip to the state and the chain of tanh, the 64 products of a decay, the
+// recurrence and the norm.  In three launches (decays, scan by four work-groups a head, norm) 16 requests with 32 heads of 64 x 64 took 6.8 + 9.2 + 4.1 us; now 11.9.
+// Work-groups hold dim x vdim numbers of state: up to 128 x 128.
+template <typename T, int RPL, int CG>
+__global__ void __launch_bounds__(256)
+wkv_token_kernel(const T* __restrict__ rkv, int ld, int k_off, int v_off, int gate_off, const float* __restrict__ z, const float* __restrict__ w2t, const float* __restrict__ w0, int rank,
+                 const float* __restrict__ bonus, float* __restrict__ state, size_t slot_stride, const int* __restrict__ slots, const int* __restrict__ req_indptr,
+                 const float* __restrict__ norm, float eps, T* __restrict__ out, int heads, int dim, int vdim, const float* __restrict__ last_rows, int row_width, size_t tail_off) {
+    constexpr int ROWS = DELTA_L * RPL, Q = RPL / 4, AHEAD = 64, LANES = CG <= 4 ? 16 : 32;
+    __shared__ __attribute__((aligned(16))) float sr[ROWS], sk[ROWS], sw[ROWS], so[CG * 16];
+    extern __shared__ __attribute__((aligned(16))) float wt_tanh[];          // [rank]
+    const int req = blockIdx.y, head = blockIdx.x;
+    const int slot_at = slots[req], tok0 = req_indptr[req], tok1 = req_indptr[req + 1];
+    if (tok0 >= tok1) return;
+    const int tid = threadIdx.x, wave = tid / TL_WAVE, lane = tid % TL_WAVE;
+    const int rg = lane & 15, cw = wave * 4 + (lane >> 4);       // the lane's place in its columns, and the first of them
+    const int channels = heads * dim, n = head * dim + min(tid, dim - 1);
+    float* slot = state + (size_t)slot_at * slot_stride;
+    float* st = slot + (size_t)head * vdim * dim;
+    float S[CG][RPL];
+#pragma unroll
+    for (int c = 0; c < CG; ++c)
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int row = 64 * q + 4 * rg, col = 16 * c + cw;
+            const float4 x = col < vdim && row < dim ? *(const float4*)(st + (size_t)col * dim + row) : make_float4(0.f, 0.f, 0.f, 0.f);
+            S[c][4 * q] = x.x; S[c][4 * q + 1] = x.y; S[c][4 * q + 2] = x.z; S[c][4 * q + 3] = x.w;
+        }
+    float ub[RPL], ahead[AHEAD];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int row = 64 * q + 4 * rg;
+        const float4 x = row < dim ? *(const float4*)(bonus + head * dim + row) : make_float4(0.f, 0.f, 0.f, 0.f);
+        ub[4 * q] = x.x; ub[4 * q + 1] = x.y; ub[4 * q + 2] = x.z; ub[4 * q + 3] = x.w;
+    }
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) ahead[j] = w2t[(size_t)min(j, rank - 1) * channels + n];
+    const float start = w0[n];
+    for (int t = tok0; t < tok1; ++t) {
+        const T* row = rkv + (size_t)t * ld;
+        if (tid < ROWS / 4) {
+            const bool ok = 4 * tid < dim;
+            *(float4*)(sr + 4 * tid) = ok ? load4(row + head * dim + 4 * tid) : make_float4(0.f, 0.f, 0.f, 0.f);
+            *(float4*)(sk + 4 * tid) = ok ? load4(row + k_off + head * dim + 4 * tid) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        if (tid < ROWS) sw[tid] = 1.f;
+        T v[CG];
+#pragma unroll
+        for (int c = 0; c < CG; ++c) v[c] = row[v_off + head * vdim + min(16 * c + cw, vdim - 1)];
+        const int g_at = min(4 * (tid % LANES), vdim - 4);
+        const typename Four<T>::type gate = *(const typename Four<T>::type*)(row + gate_off + head * vdim + g_at);
+        const float4 nw = *(const float4*)(norm + head * vdim + g_at);
+        for (int j = tid; j < rank; j += 256) wt_tanh[j] = tanhf(z[(size_t)t * rank + j]);
+        __syncthreads();
+        if (tid < dim) {
+            float a = start;
+#pragma unroll
+            for (int j = 0; j < AHEAD; ++j)
+                if (j < rank) a = fmaf(ahead[j], wt_tanh[j], a);
+#pragma unroll 16
+            for (int j = AHEAD; j < rank; ++j) a = fmaf(w2t[(size_t)j * channels + n], wt_tanh[j], a);
+            sw[tid] = expf(-expf(a));
+        }
+        __syncthreads();
+        float4 r4[Q], k4[Q], w4[Q];
+        float b4[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int at = 64 * q + 4 * rg;
+            r4[q] = *(const float4*)(sr + at);
+            k4[q] = *(const float4*)(sk + at);
+            w4[q] = *(const float4*)(sw + at);
+            b4[0] = fmaf(k4[q].x * ub[4 * q], r4[q].x, b4[0]);
+            b4[1] = fmaf(k4[q].y * ub[4 * q + 1], r4[q].y, b4[1]);
+            b4[2] = fmaf(k4[q].z * ub[4 * q + 2], r4[q].z, b4[2]);
+            b4[3] = fmaf(k4[q].w * ub[4 * q + 3], r4[q].w, b4[3]);
+        }
+        const float b = row16_sum((b4[0] + b4[1]) + (b4[2] + b4[3]));
+#pragma unroll
+        for (int c = 0; c < CG; ++c) {
+            const float vt = to_float(v[c]);
+            float o4[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                float* s4 = S[c] + 4 * q;
+                o4[0] = fmaf(r4[q].x, s4[0], o4[0]);
+                o4[1] = fmaf(r4[q].y, s4[1], o4[1]);
+                o4[2] = fmaf(r4[q].z, s4[2], o4[2]);
+                o4[3] = fmaf(r4[q].w, s4[3], o4[3]);
+                s4[0] = fmaf(w4[q].x, s4[0], k4[q].x * vt);
+                s4[1] = fmaf(w4[q].y, s4[1], k4[q].y * vt);
+                s4[2] = fmaf(w4[q].z, s4[2], k4[q].z * vt);
+                s4[3] = fmaf(w4[q].w, s4[3], k4[q].w * vt);
+            }
+            const float o = fmaf(b, vt, row16_sum((o4[0] + o4[1]) + (o4[2] + o4[3])));
+            if (rg == 0) so[16 * c + cw] = o;
+        }
+        __syncthreads();
+        if (wave == 0) {                                // the norm of the head and its gate, LANES lanes (the others do the same again and store nothing)
+            const float4 u = *(const float4*)(so + g_at), g = widen4(gate);
+            float ss = 0.f;
+            if (4 * (lane % LANES) < vdim) { ss = fmaf(u.x, u.x, ss); ss = fmaf(u.y, u.y, ss); ss = fmaf(u.z, u.z, ss); ss = fmaf(u.w, u.w, ss); }
+            const float inv = 1.f / sqrtf(lanes_sum<LANES>(ss) / (float)vdim + eps);
+            const float4 s = make_float4(1.f / (1.f + expf(-g.x)), 1.f / (1.f + expf(-g.y)), 1.f / (1.f + expf(-g.z)), 1.f / (1.f + expf(-g.w)));
+            if (4 * lane < vdim)
+                store4(out + ((size_t)t * heads + head) * vdim + 4 * lane, make_float4(u.x * (g.x * s.x) * inv * nw.x, u.y * (g.y * s.y) * inv * nw.y,
+                                                                                       u.z * (g.z * s.z) * inv * nw.z, u.w * (g.w * s.w) * inv * nw.w));
+        }
+        if (t + 1 < tok1) __syncthreads();              // (a request that brings more: its next token's numbers go where these were)
+    }
+#pragma unroll
+    for (int c = 0; c < CG; ++c)
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int row = 64 * q + 4 * rg, col = 16 * c + cw;
+            if (col < vdim && row < dim) *(float4*)(st + (size_t)col * dim + row) = make_float4(S[c][4 * q], S[c][4 * q + 1], S[c][4 * q + 2], S[c][4 * q + 3]);
+        }
+    if (last_rows)                                      // the heads share the row
+        for (int i = head * 256 + tid; i < row_width; i += heads * 256) slot[tail_off + i] = last_rows[(size_t)(tok1 - 1) * row_width + i];
+}
+
+// Whether wkv_token_kernel is built for these sizes and places: heads in whole pieces of four numbers, on the places where they can be fetched.
+extern "C" int tl_wkv_token_fits(const void* rkv, int ld, int k_off, int v_off, int gate_off, const void* bonus, const void* state, long slot_stride, const void* norm, const void* out, int dim,
+                                 int vdim, int rank, int dtype) {
+    const size_t piece = dtype == TL_DT_F32 ? 16 : 8;
+    return (dtype == TL_DT_F32 || dtype == TL_DT_BF16) && dim > 0 && vdim > 0 && dim % 4 == 0 && vdim % 4 == 0 && dim <= 128 && vdim <= 128 && rank > 0 && rank <= 1024 &&
+           (ld | k_off | v_off | gate_off) % 4 == 0 && slot_stride % 4 == 0 && ((uintptr_t)rkv | (uintptr_t)out) % piece == 0 && ((uintptr_t)bonus | (uintptr_t)state | (uintptr_t)norm) % 16 == 0;
+}
+
+// Operands as tl_wkv_scan and tl_channel_decay take them; the gate's numbers lie in the rows of rkv from gate_off on; norm float [heads * vdim]; out [tokens, heads * vdim] of rkv's type.
+extern "C" int tl_wkv_token(const void* rkv, int ld, int k_off, int v_off, int gate_off, const void* z, const void* w2t, const void* w0, int rank, const void* bonus, void* state, long slot_stride,
+                            const void* slots, const void* req_indptr, const void* norm, float eps, void* out, int requests, int heads, int dim, int vdim, const void* last_rows, int row_width,
+                            long tail_off, int dtype, hipStream_t stream) {
+    TL_REQUIRE(requests >= 0 && heads > 0 && ld > 0 && k_off >= 0 && v_off >= 0 && gate_off >= 0 && z && w2t && w0, "wkv_token: bad sizes");
+    TL_REQUIRE(tl_wkv_token_fits(rkv, ld, k_off, v_off, gate_off, bonus, state, slot_stride, norm, out, dim, vdim, rank, dtype), "wkv_token: not built for heads of %d x %d or for these places", dim, vdim);
+    TL_REQUIRE(slot_stride >= (long)heads * dim * vdim, "wkv_token: the state rows are too short");
+    TL_REQUIRE(!last_rows || (row_width > 0 && tail_off >= (long)heads * dim * vdim && slot_stride >= tail_off + row_width),
+               "wkv_token: the slots do not hold a row of %d numbers behind the states", row_width);
+    TL_REQUIRE(requests <= 65535, "wkv_token: too many requests for one launch");
+    if (requests == 0) return TL_OK;
+#define TL_WT(T, R, C)                                                                                                                                                          \
+    wkv_token_kernel<T, R, C><<<dim3(heads, requests), 256, sizeof(float) * rank, stream>>>((const T*)rkv, ld, k_off, v_off, gate_off, (const float*)z, (const float*)w2t, \
+        (const float*)w0, rank, (const float*)bonus, (float*)state, (size_t)slot_stride, (const int*)slots, (const int*)req_indptr, (const float*)norm, eps, (T*)out, heads, dim, vdim, \
+        (const float*)last_rows, row_width, (size_t)tail_off)
+#define TL_WT_R(T, R) if (vdim <= 64) TL_WT(T, R, 4); else TL_WT(T, R, 8)
+#define TL_WT_T(T) if (dim <= 64) { TL_WT_R(T, 4); } else { TL_WT_R(T, 8); }
+    if (dtype == TL_DT_F32) { TL_WT_T(float); } else { TL_WT_T(bf16_t); }
+#undef TL_WT_T
+#undef TL_WT_R
+#undef TL_WT
+    TL_CHECK_LAUNCH("wkv_token");
+    return TL_OK;
+}
+
 // ------------------------------------------------------------------ long portions in chunks: recurrences with one decay per head and token
 // S <- g S + b k v^T, o = S^T q (the matrix memory; the decayed linear attention) over the tokens of a long portion.
 // Token by token the work of a head is a chain that a few compute units walk (four heads of 256 x 512 over 2048 tokens: 1.2 ms, a prompt's

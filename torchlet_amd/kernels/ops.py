@@ -1366,6 +1366,38 @@ def wkv_scan(rkv: torch.Tensor, k_off: int, v_off: int, decay: torch.Tensor, bon
                                 ctypes.c_long(tail_off), c_int(_dt(rkv, "wkv_scan")), _stream()))
 
 
+def wkv_token(proj: torch.Tensor, k_off: int, v_off: int, gate_off: int, z: torch.Tensor, w2t: torch.Tensor, w0: torch.Tensor, bonus: torch.Tensor, state: torch.Tensor,
+              slots: torch.Tensor, req_indptr: torch.Tensor, norm: torch.Tensor, eps: float, out: torch.Tensor, heads: int, dim: int, vdim: int, last_rows: torch.Tensor,
+              tail_off: int) -> bool:
+    """:func:`channel_decay`, :func:`wkv_scan` and :func:`gated_head_norm` (``silu``, a weight per number) in one launch, for steps in which every request brings one token
+    (any number is right, one is fast): operands as there, the gate's numbers from ``gate_off`` on in the rows of ``proj``, the decays' low-rank sums in ``z``; ``out`` ``[T, heads *
+    vdim]`` of ``proj``'s dtype receives what the norm leaves.  False, and nothing done, where the kernel is not built for the sizes or the places (or off the GPU)."""
+    if not proj.is_cuda:
+        return False
+    T, R, rank = proj.shape[0], req_indptr.numel() - 1, z.shape[1]
+    if proj.dim() != 2 or proj.stride(1) != 1 or proj.shape[1] < max(heads * dim, k_off + heads * dim, v_off + heads * vdim, gate_off + heads * vdim):
+        raise KernelError("wkv_token: the rows do not hold r, k, v and the gate at the given columns")
+    for t, shape, what in ((z, (T, rank), "z"), (w2t, (rank, heads * dim), "w2t"), (w0, (heads * dim,), "w0"), (bonus, (heads * dim,), "bonus"), (norm, (heads * vdim,), "norm")):
+        if t.dtype != torch.float32 or t.shape != shape or not t.is_contiguous():
+            raise KernelError(f"wkv_token: {what} must be contiguous float32 {list(shape)}")
+    if out.shape != (T, heads * vdim) or out.dtype != proj.dtype or not out.is_contiguous():
+        raise KernelError(f"wkv_token: out must be contiguous [{T}, {heads * vdim}] of the projections' dtype")
+    width = last_rows.shape[1]
+    if state.dtype != torch.float32 or state.dim() != 2 or state.stride(1) != 1 or state.shape[1] < tail_off + width or tail_off < heads * dim * vdim \
+            or last_rows.dtype != torch.float32 or last_rows.shape[0] != T or not last_rows.is_contiguous():
+        raise KernelError(f"wkv_token: state {tuple(state.shape)} does not hold {heads} states of {dim} x {vdim} and a row of {width}, or the rows are not contiguous float32 [T, H]")
+    _i32(slots, "slots", R)
+    _i32(req_indptr, "req_indptr", R + 1)
+    lib = _lib("recurrent")
+    at = (_ptr(proj), c_int(proj.stride(0)), c_int(k_off), c_int(v_off), c_int(gate_off))
+    if not lib.tl_wkv_token_fits(*at, _ptr(bonus), _ptr(state), ctypes.c_long(state.stride(0)), _ptr(norm), _ptr(out), c_int(dim), c_int(vdim), c_int(rank), c_int(_dt(proj, "wkv_token"))):
+        return False
+    _check(lib, lib.tl_wkv_token(*at, _ptr(z), _ptr(w2t), _ptr(w0), c_int(rank), _ptr(bonus), _ptr(state), ctypes.c_long(state.stride(0)), _ptr(slots), _ptr(req_indptr), _ptr(norm),
+                                 c_float(eps), _ptr(out), c_int(R), c_int(heads), c_int(dim), c_int(vdim), _ptr(last_rows), c_int(width), ctypes.c_long(tail_off),
+                                 c_int(_dt(proj, "wkv_token")), _stream()))
+    return True
+
+
 # ------------------------------------------------------------- attention with two head sizes, a cap and a local mask
 
 LOCAL_ATTENTION_MAX_DIM = 256

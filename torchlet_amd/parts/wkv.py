@@ -105,11 +105,13 @@ class WKV(Mixer):
         else:
             ops.linear_groups(mixes[:2], self.w_rk, proj[:, : 2 * K])
             ops.linear_groups_beside(mixes[2:4], self.w_vg, proj[:, 2 * K:], mixes[4], self.w1, z)
-        decay = torch.empty((T, K), dtype=torch.float32, device=dev)
-        ops.channel_decay(z, self.w2t, self.w0, decay)
-        o = torch.empty((T, V), dtype=torch.float32, device=dev)
-        ops.wkv_scan(proj, K, 2 * K, decay, self.bonus, cache.state, ctx.slots, ctx.req_indptr, o, self.heads, self.dim, self.vdim,
-                     max_new_tokens=ctx.max_new_tokens, last_rows=x, tail_off=self.state_floats)
         mixed = torch.empty((T, V), dtype=self.dtype, device=dev)
-        ops.gated_head_norm(o, proj[:, 2 * K + V:], self.w_norm, float(self.spec.norm_eps), mixed, self.heads, self.vdim, gate="silu")
+        if not (ctx.max_new_tokens == 1 and ops.wkv_token(proj, K, 2 * K, 2 * K + V, z, self.w2t, self.w0, self.bonus, cache.state, ctx.slots, ctx.req_indptr, self.w_norm,
+                                                          float(self.spec.norm_eps), mixed, self.heads, self.dim, self.vdim, x, self.state_floats)):
+            decay = torch.empty((T, K), dtype=torch.float32, device=dev)
+            ops.channel_decay(z, self.w2t, self.w0, decay)
+            o = torch.empty((T, V), dtype=torch.float32, device=dev)
+            ops.wkv_scan(proj, K, 2 * K, decay, self.bonus, cache.state, ctx.slots, ctx.req_indptr, o, self.heads, self.dim, self.vdim,
+                         max_new_tokens=ctx.max_new_tokens, last_rows=x, tail_off=self.state_floats)
+            ops.gated_head_norm(o, proj[:, 2 * K + V:], self.w_norm, float(self.spec.norm_eps), mixed, self.heads, self.vdim, gate="silu")
         return project_out(mixed, self.w_o, self.dtype)
