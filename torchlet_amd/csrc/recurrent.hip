@@ -1037,6 +1037,184 @@ static int launch_delta_scan(const void* qkv, const void* gates, const void* hea
     return TL_OK;
 }
 
+// ------------------------------------------------------------------ the delta rule's single tokens: convolution, recurrence, norm and gate in one launch
+// For steps of one token a request: what short_conv_kernel (four taps), delta_scan_kernel and gated_norm_pieces_kernel (silu, one weight for all heads) make in three launches, in the same
+// order of every sum.  A work-group has a key head of a request with the value heads that share it, so the channels it convolves, and the tail it moves on, are its own.  It asks for
+// its states first, sixteen lanes a column and CG columns to each; while they are on their way the convolution's inputs arrive, its threads make q, k, v and the heads' gates and leave them in
+// shared memory, then all lanes move the states, and the first ones take the outputs through the norm.  What bounds it: a compute unit draws the states of its work-group at 64 bytes a clock, 128 KB
+// for two value heads of 128 x 128, and gives them back as fast.  8 requests, 16 heads of 128 x 128 over 8: 4.5 + 6.8 + 4.1 us in three launches, 9.3 in one.
+// Built for key heads of 64 or 128 channels with up to 256 value channels between them.
+#define DT_THREADS 512                          // (sixteen waves leave a wave 128 registers, which 256 columns of 128 do not fit)
+#define DT_COLS (DT_THREADS / DELTA_L)           // columns at a time
+struct DeltaToken {
+    int ld, gate_off;
+    const float *w, *gates, *a_log, *dt_bias;
+    float* state;
+    size_t slot_stride, tail_off;
+    const int *slots, *req_indptr;
+    const float* norm;
+    float eps, gain, qscale, unit_eps;
+    int out_ld, heads, kv_heads, vdim;
+};
+template <typename T, int RPL, int CG>
+__global__ void __launch_bounds__(DT_THREADS)
+delta_token_kernel(const T* __restrict__ proj, T* __restrict__ out, DeltaToken a) {
+    constexpr int dim = DELTA_L * RPL, Q = RPL / 4, U = dim / 4;         // U: lanes of a key head's channels
+    __shared__ __attribute__((aligned(16))) float sq[dim], sk[dim], sv[CG * DT_COLS], so[CG * DT_COLS], sg[2 * CG * DT_COLS];
+    const int req = blockIdx.y, kv = blockIdx.x;
+    const int slot_at = a.slots[req], tok0 = a.req_indptr[req], tok1 = a.req_indptr[req + 1];
+    if (tok0 >= tok1) return;
+    const int tid = threadIdx.x, rg = tid & 15, cw = tid >> 4, vdim = a.vdim, hpk = a.heads / a.kv_heads, cols = hpk * vdim, head0 = kv * hpk;
+    const int C = 2 * a.kv_heads * dim + a.heads * vdim;
+    float* slot = a.state + (size_t)slot_at * a.slot_stride;
+    float* st = slot + (size_t)head0 * vdim * dim;                  // the value heads' columns, one behind the other
+    float4 S[CG][Q];
+#pragma unroll
+    for (int c = 0; c < CG; ++c)
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int col = c * DT_COLS + cw;
+            S[c][q] = *(const float4*)(st + (size_t)min(col, cols - 1) * dim + 64 * q + 4 * rg);
+        }
+    // the convolution's threads: four neighbouring channels each, queries, keys, then values
+    const int pieces = 2 * U + cols / 4;
+    const bool conv = tid < pieces;
+    const int p = min(tid, pieces - 1);
+    const int ch = p < U ? kv * dim + 4 * p : p < 2 * U ? (a.kv_heads + kv) * dim + 4 * (p - U) : 2 * a.kv_heads * dim + head0 * vdim + 4 * (p - 2 * U);
+    float* tail = slot + a.tail_off + ch;
+    const bool conv_wave = tid < (pieces + TL_WAVE - 1) / TL_WAVE * TL_WAVE;      // (its last lanes make the last piece again and store nothing)
+    float4 tap[4], win[3];
+    if (conv_wave) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) win[j] = *(const float4*)(tail + (size_t)j * C);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tap[e] = *(const float4*)(a.w + (size_t)(ch + e) * 4);
+    }
+    // the norm's threads: LANES lanes to a value head
+    const int lanes = vdim <= 64 ? 16 : 32, hn = tid / lanes, n_at = tid % lanes * 4;
+    const bool norms = hn < hpk, n_ok = norms && n_at < vdim;
+    for (int t = tok0; t < tok1; ++t) {
+        const T* row = proj + (size_t)t * a.ld;
+        typename Four<T>::type gate{};
+        float4 nw = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (n_ok) {
+            gate = *(const typename Four<T>::type*)(row + a.gate_off + (head0 + hn) * vdim + n_at);
+            nw = *(const float4*)(a.norm + n_at);
+        }
+        if (tid >= DT_THREADS - hpk) {                              // (the last threads have nothing to convolve: there are at most 128 pieces, and 16 heads)
+            const int h = DT_THREADS - 1 - tid;
+            const float* g = a.gates + (size_t)t * 2 * a.heads + head0 + h;
+            sg[2 * h] = 1.f / (1.f + expf(-g[0]));
+            sg[2 * h + 1] = expf(-expf(a.a_log[head0 + h]) * softplus_f(g[a.heads] + a.dt_bias[head0 + h]));
+        }
+        if (conv_wave) {
+            const float4 now = load4(row + ch);
+            float4 y;
+#define TL_TAP(f, e) y.f = silu_f(fmaf(tap[e].w, now.f, fmaf(tap[e].z, win[2].f, fmaf(tap[e].y, win[1].f, fmaf(tap[e].x, win[0].f, 0.f)))))
+            TL_TAP(x, 0); TL_TAP(y, 1); TL_TAP(z, 2); TL_TAP(w, 3);
+#undef TL_TAP
+            const float ss = lanes_sum<U>(fmaf(y.w, y.w, fmaf(y.z, y.z, fmaf(y.y, y.y, y.x * y.x))));
+            if (p < 2 * U) {
+                float factor = 1.f / sqrtf(ss + a.unit_eps);
+                if (p < U) factor *= a.qscale;
+                y = make_float4(y.x * factor, y.y * factor, y.z * factor, y.w * factor);
+            }
+            if (conv) *(float4*)(p < U ? sq + 4 * p : p < 2 * U ? sk + 4 * (p - U) : sv + 4 * (p - 2 * U)) = y;
+            win[0] = win[1]; win[1] = win[2]; win[2] = now;
+        }
+        __syncthreads();
+        float4 k4[Q], q4[Q];
+        float c4[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            k4[q] = *(const float4*)(sk + 64 * q + 4 * rg);
+            q4[q] = *(const float4*)(sq + 64 * q + 4 * rg);
+            c4[0] = fmaf(k4[q].x, q4[q].x, c4[0]);
+            c4[1] = fmaf(k4[q].y, q4[q].y, c4[1]);
+            c4[2] = fmaf(k4[q].z, q4[q].z, c4[2]);
+            c4[3] = fmaf(k4[q].w, q4[q].w, c4[3]);
+        }
+        const float kq = row16_sum((c4[0] + c4[1]) + (c4[2] + c4[3]));
+#pragma unroll
+        for (int c = 0; c < CG; ++c) {
+            const int col = c * DT_COLS + cw;
+            if (col >= cols) break;                                 // (16 lanes together)
+            const int h = col / vdim;
+            const float vt = sv[col], beta = sg[2 * h], g = sg[2 * h + 1];
+            float a4[4] = {0.f, 0.f, 0.f, 0.f}, b4[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                const float4 x = S[c][q];
+                a4[0] = fmaf(x.x, k4[q].x, a4[0]); a4[1] = fmaf(x.y, k4[q].y, a4[1]); a4[2] = fmaf(x.z, k4[q].z, a4[2]); a4[3] = fmaf(x.w, k4[q].w, a4[3]);
+                b4[0] = fmaf(x.x, q4[q].x, b4[0]); b4[1] = fmaf(x.y, q4[q].y, b4[1]); b4[2] = fmaf(x.z, q4[q].z, b4[2]); b4[3] = fmaf(x.w, q4[q].w, b4[3]);
+            }
+            const float dot = row16_sum((a4[0] + a4[1]) + (a4[2] + a4[3])), b = row16_sum((b4[0] + b4[1]) + (b4[2] + b4[3]));
+            const float u = beta * fmaf(-g, dot, vt);
+#pragma unroll
+            for (int q = 0; q < Q; ++q)
+                S[c][q] = make_float4(fmaf(k4[q].x, u, g * S[c][q].x), fmaf(k4[q].y, u, g * S[c][q].y), fmaf(k4[q].z, u, g * S[c][q].z), fmaf(k4[q].w, u, g * S[c][q].w));
+            if (rg == 0) so[col] = fmaf(kq, u, g * b);
+        }
+        __syncthreads();
+        if (tid < (hpk * lanes + TL_WAVE - 1) / TL_WAVE * TL_WAVE) {
+            const float4 u = n_ok ? *(const float4*)(so + hn * vdim + n_at) : make_float4(0.f, 0.f, 0.f, 0.f), z = widen4(gate);
+            float ss = fmaf(u.x, u.x, 0.f);
+            ss = fmaf(u.y, u.y, ss); ss = fmaf(u.z, u.z, ss); ss = fmaf(u.w, u.w, ss);
+            ss = vdim <= 64 ? lanes_sum<16>(ss) : lanes_sum<32>(ss);
+            const float inv = 1.f / sqrtf(ss / (float)vdim + a.eps);
+            const float4 f = make_float4(z.x * (1.f / (1.f + expf(-z.x))), z.y * (1.f / (1.f + expf(-z.y))), z.z * (1.f / (1.f + expf(-z.z))), z.w * (1.f / (1.f + expf(-z.w))));
+            if (n_ok) store4(out + (size_t)t * a.out_ld + (head0 + hn) * vdim + n_at, make_float4(u.x * f.x * inv * nw.x * a.gain, u.y * f.y * inv * nw.y * a.gain,
+                                                                                                  u.z * f.z * inv * nw.z * a.gain, u.w * f.w * inv * nw.w * a.gain));
+        }
+        // (a request that brings more: the next token's q, k, v and gates go where these were read before the second barrier, its outputs where the norm's waves read behind it)
+        if (t + 1 < tok1) __syncthreads();
+    }
+#pragma unroll
+    for (int c = 0; c < CG; ++c) {
+        const int col = c * DT_COLS + cw;
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+            if (col < cols) *(float4*)(st + (size_t)col * dim + 64 * q + 4 * rg) = S[c][q];
+    }
+    if (conv) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) *(float4*)(tail + (size_t)j * C) = win[j];
+    }
+}
+
+// Whether delta_token_kernel is built for these sizes and places.
+extern "C" int tl_delta_token_fits(const void* proj, int ld, int gate_off, const void* conv_w, const void* state, long slot_stride, long tail_off, const void* norm, const void* out, int out_ld,
+                                   int heads, int kv_heads, int dim, int vdim, int taps, int dtype) {
+    const size_t piece = dtype == TL_DT_F32 ? 16 : 8;
+    return (dtype == TL_DT_F32 || dtype == TL_DT_BF16) && heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && (dim == 64 || dim == 128) && vdim >= 16 && vdim % 4 == 0 && vdim <= 128 &&
+           heads / kv_heads * vdim <= 256 && taps == 4 && (ld | gate_off | out_ld) % 4 == 0 && slot_stride % 4 == 0 && tail_off % 4 == 0 &&
+           ((uintptr_t)proj | (uintptr_t)out) % piece == 0 && ((uintptr_t)conv_w | (uintptr_t)state | (uintptr_t)norm) % 16 == 0;
+}
+
+// Operands as tl_delta_prepare, tl_delta_scan and tl_gated_head_norm take them; gates stays as it is; the output gate's numbers lie in the rows of proj from gate_off on; norm float [vdim].
+extern "C" int tl_delta_token(const void* proj, int ld, int gate_off, const void* conv_w, const void* gates, const void* a_log, const void* dt_bias, void* state, long slot_stride, long tail_off,
+                              const void* slots, const void* req_indptr, const void* norm, float eps, float gain, void* out, int out_ld, int requests, int heads, int kv_heads, int dim,
+                              int vdim, int taps, float qscale, float unit_eps, int dtype, hipStream_t stream) {
+    TL_REQUIRE(requests >= 0 && requests <= 65535 && gates && a_log && dt_bias, "delta_token: bad sizes");
+    TL_REQUIRE(tl_delta_token_fits(proj, ld, gate_off, conv_w, state, slot_stride, tail_off, norm, out, out_ld, heads, kv_heads, dim, vdim, taps, dtype),
+               "delta_token: not built for %d heads of %d x %d over %d or for these places", heads, dim, vdim, kv_heads);
+    const int C = 2 * kv_heads * dim + heads * vdim, cols = heads / kv_heads * vdim;
+    TL_REQUIRE(ld >= C && gate_off >= C && ld >= gate_off + heads * vdim && out_ld >= heads * vdim && tail_off >= (long)heads * dim * vdim && slot_stride >= tail_off + 3L * C,
+               "delta_token: rows or state too short");
+    if (requests == 0) return TL_OK;
+    const DeltaToken a{ld, gate_off, (const float*)conv_w, (const float*)gates, (const float*)a_log, (const float*)dt_bias, (float*)state, (size_t)slot_stride, (size_t)tail_off,
+                       (const int*)slots, (const int*)req_indptr, (const float*)norm, eps, gain, qscale, unit_eps, out_ld, heads, kv_heads, vdim};
+#define TL_DTK(T, R, G) delta_token_kernel<T, R, G><<<dim3(kv_heads, requests), DT_THREADS, 0, stream>>>((const T*)proj, (T*)out, a)
+#define TL_DTK_R(T, R) if (cols <= 2 * DT_COLS) TL_DTK(T, R, 2); else if (cols <= 4 * DT_COLS) TL_DTK(T, R, 4); else TL_DTK(T, R, 8)
+#define TL_DTK_T(T) if (dim == 64) { TL_DTK_R(T, 4); } else { TL_DTK_R(T, 8); }
+    if (dtype == TL_DT_F32) { TL_DTK_T(float); } else { TL_DTK_T(bf16_t); }
+#undef TL_DTK_T
+#undef TL_DTK_R
+#undef TL_DTK
+    TL_CHECK_LAUNCH("delta_token");
+    return TL_OK;
+}
+
 // ------------------------------------------------------------------ long portions in blocks: the delta rule and the selective recurrence
 // The token loop above is a chain of some 500 cycles a token, whatever else the GPU does (one prompt of 2048 tokens, 16 heads: 412 us on 128 work-groups).  Over a block of
 // 16 tokens the recurrence is a few products of small matrices (the compact form of a product of Householder-like steps, Bischof and Van Loan's WY representation, as "Parallelizing Linear

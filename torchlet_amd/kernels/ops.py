@@ -1322,6 +1322,38 @@ def silu_float(x: torch.Tensor, out: torch.Tensor) -> None:
 CHANNEL_DECAY_MAX_RANK = 1024
 
 
+def delta_token(proj: torch.Tensor, gate_off: int, conv_w: torch.Tensor, gates: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor, state: torch.Tensor, tail_off: int,
+                slots: torch.Tensor, req_indptr: torch.Tensor, norm: torch.Tensor, eps: float, out: torch.Tensor, heads: int, kv_heads: int, dim: int, vdim: int, taps: int,
+                qscale: float, unit_eps: float, gain: float = 1.0) -> bool:
+    """:func:`delta_prepare`, :func:`delta_scan` and :func:`gated_head_norm` (``silu``, a weight ``[vdim]`` for all heads) in one launch, for steps in which every request brings
+    one token (any number is right, one is fast): operands as there (``gates`` stays raw), the output gate's numbers from ``gate_off`` on in the rows of ``proj``; ``out [T, heads *
+    vdim]`` (a row-strided view of ``proj``'s dtype) receives what the norm leaves times ``gain``.  False, and nothing done, where the kernel is not built for the sizes or the places (or off
+    the GPU)."""
+    if not proj.is_cuda:
+        return False
+    T, R, C = proj.shape[0], req_indptr.numel() - 1, 2 * kv_heads * dim + heads * vdim
+    if proj.dim() != 2 or proj.stride(1) != 1 or gate_off < C or proj.shape[1] < gate_off + heads * vdim:
+        raise KernelError(f"delta_token: the projections must hold {C} channels and a gate of {heads * vdim} numbers behind them")
+    for t, shape, what in ((conv_w, (C, taps), "conv_w"), (gates, (T, 2 * heads), "gates"), (a_log, (heads,), "a_log"), (dt_bias, (heads,), "dt_bias"), (norm, (vdim,), "norm")):
+        if t.dtype != torch.float32 or t.shape != shape or not t.is_contiguous():
+            raise KernelError(f"delta_token: {what} must be contiguous float32 {list(shape)}")
+    if out.shape != (T, heads * vdim) or out.dtype != proj.dtype or out.stride(1) != 1:
+        raise KernelError(f"delta_token: out must be [{T}, {heads * vdim}] of the projections' dtype")
+    if state.dtype != torch.float32 or state.dim() != 2 or state.stride(1) != 1 or tail_off < heads * dim * vdim or state.shape[1] < tail_off + (taps - 1) * C:
+        raise KernelError(f"delta_token: state {tuple(state.shape)} does not hold {heads} states of {dim} x {vdim} and the tails behind them")
+    _i32(slots, "slots", R)
+    _i32(req_indptr, "req_indptr", R + 1)
+    lib = _lib("recurrent")
+    dt = c_int(_dt(proj, "delta_token"))
+    rows, place = (_ptr(proj), c_int(proj.stride(0)), c_int(gate_off), _ptr(conv_w)), (_ptr(state), ctypes.c_long(state.stride(0)), ctypes.c_long(tail_off))
+    sizes = (c_int(heads), c_int(kv_heads), c_int(dim), c_int(vdim), c_int(taps))
+    if not lib.tl_delta_token_fits(*rows, *place, _ptr(norm), _ptr(out), c_int(out.stride(0)), *sizes, dt):
+        return False
+    _check(lib, lib.tl_delta_token(*rows, _ptr(gates), _ptr(a_log), _ptr(dt_bias), *place, _ptr(slots), _ptr(req_indptr), _ptr(norm), c_float(eps), c_float(gain), _ptr(out),
+                                   c_int(out.stride(0)), c_int(R), *sizes, c_float(qscale), c_float(unit_eps), dt, _stream()))
+    return True
+
+
 def channel_decay(z: torch.Tensor, w2t: torch.Tensor, w0: torch.Tensor, decay: torch.Tensor) -> None:
     """``decay = exp(-exp(w0 + tanh(z) @ w2t))``: ``z`` float32 ``[T, rank]``, ``w2t`` float32 ``[rank, channels]``, ``w0`` float32 ``[channels]``,
     ``decay`` float32 ``[T, channels]``."""

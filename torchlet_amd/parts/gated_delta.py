@@ -97,6 +97,10 @@ class GatedDelta(StagedMixer):
         if gates is None:
             gates = torch.empty((T, 2 * self.heads), dtype=torch.float32, device=h.device)
             ops.linear(h, self.w_gates, None, gates)
+        if ctx.max_new_tokens == 1 and ops.delta_token(proj, self.channels, self.w_conv, gates, self.a_log, self.dt_bias, cache.state, self.state_floats, ctx.slots, ctx.req_indptr,
+                                                       self.w_norm, float(self.spec.norm_eps), out, self.heads, self.kv_heads, self.dim, self.vdim, self.taps, self.qscale,
+                                                       float(self.spec.unit_eps), gain):
+            return
         qkv = torch.empty((T, self.channels), dtype=torch.float32, device=h.device)
         # convolutions (from the slot's tails, which move on), silu, unit vectors; the raw gates become beta and the decay in place
         ops.delta_prepare(proj, self.w_conv, gates, self.a_log, self.dt_bias, cache.state, self.state_floats, ctx.slots, ctx.req_indptr,
