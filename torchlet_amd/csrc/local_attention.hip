@@ -236,10 +236,16 @@ __device__ __forceinline__ float cap_score_fast(float s, float cap, float two_lo
 // heads read their keys and values once, and with splits > 1 a tile's keys are dealt to that many work-groups, each of which leaves its sums for
 // local_merge_kernel.  Splits are what one request needs: a work-group's CU fetches at most 64 bytes a clock, 2 MB of a head's keys and values at 4000
 // tokens take it 14 us.
-template <int DK, int DV, bool HEADS>          // dim / 32 and vdim / 16
+// FRESH (with HEADS): the token's own key and value come from the projection's rows, and the wave whose keys they are among puts them into their pages, so that a decode step needs no launch for that ahead
+// (8 tokens of 4 heads of 128 and 128: 5.0 us): the step that holds the token's key takes it from there instead of from the page, and nobody else reads its place.
+struct FreshRows {
+    const bf16_t *k, *v;     // row t: token t's keys (kv_heads * dim) and values (kv_heads * vdim)
+    int k_ld, v_ld, pages;
+};
+template <int DK, int DV, bool HEADS, bool FRESH>          // dim / 32 and vdim / 16
 __global__ void __launch_bounds__(256)
-local_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __restrict__ out, int out_ld, const bf16_t* __restrict__ k_plane,
-                            const bf16_t* __restrict__ v_plane, const int* __restrict__ block_table, int table_ld, int table_width,
+local_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __restrict__ out, int out_ld, const bf16_t* k_plane,
+                            const bf16_t* v_plane, FreshRows fresh, const int* __restrict__ block_table, int table_ld, int table_width,
                             const int* __restrict__ req_indptr, const int* __restrict__ ctx_lens, const int* __restrict__ tile_req,
                             const int* __restrict__ tile_tok0, int heads, int kv_heads, int page_size, float scale, float cap,
                             LocalMask mask, float gain, const float* __restrict__ sink, const bf16_t* __restrict__ pk_plane,
@@ -283,12 +289,20 @@ local_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __re
     float m = -INFINITY, l = 0.f;
 
     const int p_last = p0 + n_tile - 1;
+    const bf16_t* fresh_k = FRESH ? fresh.k + (size_t)(first + tok0) * fresh.k_ld + g * dim : nullptr;
+    uint16_t fresh_v[FRESH ? DV : 1];                            // this lane's columns of the token's own values
+    if constexpr (FRESH) {
+        const bf16_t* row = fresh.v + (size_t)(first + tok0) * fresh.v_ld + g * vdim + li;
+#pragma unroll
+        for (int j = 0; j < DV; ++j) fresh_v[j] = row[16 * j].bits;
+    }
     // rows of the two score products that this lane fetches: keys base + 8 (li / 4) + li % 4 (+ 4)
     const int krow = 8 * (li >> 2) + (li & 3);
     // One pass over a stretch of keys lo_valid .. hi_valid of planes kp / vp (the tokens of the tile's reach, or the pooled blocks before its
     // window), of which this lane's token reads my_first .. my_last.  The running maximum, sum and output carry over from pass to pass.
-    auto run = [&](const bf16_t* __restrict__ kp, const bf16_t* __restrict__ vp, const int* __restrict__ tbl, int tbl_width, int lo_valid, int hi_valid,
-                   int my_first, int my_last) {
+    // `own`: the stretch ends with the token itself.
+    auto run = [&](const bf16_t* kp, const bf16_t* vp, const int* __restrict__ tbl, int tbl_width, int lo_valid, int hi_valid,
+                   int my_first, int my_last, bool own) {
         const int base0 = lo_valid / LAM_KEYS * LAM_KEYS;
         const int mine = base0 + LAM_KEYS * (split * LAM_WAVES + wave), stride = splits * LAM_STRIDE;      // (key steps are dealt to the splits' waves in turn)
         if (mine > hi_valid) return;
@@ -308,6 +322,10 @@ local_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __re
             const int key0 = max(min(base + krow, hi_valid), lo_valid), key1 = max(min(base + krow + 4, hi_valid), lo_valid);
             const bf16_t* k0 = kp + (((size_t)page_at(key0) * kv_heads + g) * page_size + slot_of(key0)) * dim + 8 * kq;
             const bf16_t* k1 = kp + (((size_t)page_at(key1) * kv_heads + g) * page_size + slot_of(key1)) * dim + 8 * kq;
+            if (FRESH && own) {
+                if (key0 == hi_valid) k0 = fresh_k + 8 * kq;
+                if (key1 == hi_valid) k1 = fresh_k + 8 * kq;
+            }
 #pragma unroll
             for (int s = 0; s < DK; ++s) { a0[s].u = *(const uint4*)(k0 + 32 * s); a1[s].u = *(const uint4*)(k1 + 32 * s); }
             // values, transposed: row = column of the values, k = keys base + 8 kq .. + 7 (one page: page_size % 8 == 0)
@@ -360,6 +378,13 @@ local_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __re
                     for (int e = 0; e < 8; ++e)
                         if (vkey + e > hi_valid || vkey + e < lo_valid) vf[j].e[e] = 0;
             }
+            if (FRESH && own && vkey <= hi_valid && vkey + 7 >= hi_valid) {
+#pragma unroll
+                for (int j = 0; j < DV; ++j)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (vkey + e == hi_valid) vf[j].e[e] = fresh_v[j];
+            }
             if (__any(keep != 1.f)) {                               // (the maxima settle after a tile's first steps)
 #pragma unroll
                 for (int j = 0; j < DV; ++j) { acc[j][0] *= keep; acc[j][1] *= keep; acc[j][2] *= keep; acc[j][3] *= keep; }
@@ -377,15 +402,31 @@ local_attention_mfma_kernel(const bf16_t* __restrict__ q, int q_ld, bf16_t* __re
         // the pooled blocks that lie wholly before a token's window: 0 .. (p - window + 1) / pool - 1; the tile's last token reads the most
         const int n_tile_blocks = max(0, p_last - mask.window + 1) / pool, n_my_blocks = max(0, my_p - mask.window + 1) / pool;
         if (n_tile_blocks > 0)
-            run(pk_plane, pv_plane, pool_table + (size_t)req * pool_table_ld, pool_table_width, 0, n_tile_blocks - 1, 0, n_my_blocks - 1);
+            run(pk_plane, pv_plane, pool_table + (size_t)req * pool_table_ld, pool_table_width, 0, n_tile_blocks - 1, 0, n_my_blocks - 1, false);
     }
     if (mask.keep_first > 0 && mask.window > 0) {
         // the kept first tokens that lie before a token's window: 0 .. min(keep_first, its window's start) - 1; the tile's last token reads the most
         const int n_tile_kept = min(mask.keep_first, mask.first(p_last)), n_my_kept = min(mask.keep_first, my_lo);
-        if (n_tile_kept > 0) run(k_plane, v_plane, table, table_width, 0, n_tile_kept - 1, 0, n_my_kept - 1);
+        if (n_tile_kept > 0) run(k_plane, v_plane, table, table_width, 0, n_tile_kept - 1, 0, n_my_kept - 1, false);
     }
     // the first token reads furthest back; pages before may be gone
-    run(k_plane, v_plane, table, table_width, mask.first(p0), p_last, my_lo, my_p);
+    run(k_plane, v_plane, table, table_width, mask.first(p0), p_last, my_lo, my_p, true);
+    if constexpr (FRESH) {
+        // the wave that has walked the token's own key (of the first work-group of a head's chunks) leaves it and its value in their page; page 0, the sentinel of rows that belong to no request, is never written
+        const int steps = p_last / LAM_KEYS - mask.first(p0) / LAM_KEYS;
+        if (steps % (splits * LAM_WAVES) == split * LAM_WAVES + wave && blockIdx.y % chunks == 0 && page_of(p_last) < table_width) {
+            const int page = table[page_of(p_last)], slot = slot_of(p_last);
+            if (page > 0 && page < fresh.pages) {
+                bf16_t* kd = const_cast<bf16_t*>(k_plane) + (((size_t)page * kv_heads + g) * page_size + slot) * dim;
+                bf16_t* vd = const_cast<bf16_t*>(v_plane) + ((size_t)page * kv_heads + g) * vdim * page_size + slot;
+                for (int d = lane; d < dim; d += TL_WAVE) kd[d] = fresh_k[d];
+                if (kq == 0) {
+#pragma unroll
+                    for (int j = 0; j < DV; ++j) vd[(size_t)(16 * j + li) * page_size] = bf16_t{fresh_v[j]};
+                }
+            }
+        }
+    }
     l = sum_across_halves(sum_across_rows(l));
     // ---- the four waves' shares are joined: per token the maxima, the sums and the outputs, in the order of the waves
     float* sm_m = la_smem;                              // [4][16], in units of log 2
@@ -524,23 +565,23 @@ local_merge_kernel(const float* __restrict__ part_o, const float2* __restrict__ 
     }
 }
 
-template <int DK, int DV, bool HEADS = false>
+template <int DK, int DV, bool HEADS = false, bool FRESH = false>
 static void launch_local_mfma(const void* q, int q_ld, void* out, int out_ld, const void* k_plane, const void* v_plane, const void* block_table,
                               int table_ld, int table_width, const void* req_indptr, const void* ctx_lens, const void* tile_req,
                               const void* tile_tok0, int tiles, int heads, int kv_heads, int page_size, float scale, float cap, LocalMask mask,
                               float gain, const void* sink, const void* pk_plane, const void* pv_plane, const void* pool_table, int pool_table_ld,
                               int pool_table_width, int pool, OutputTurn back, const void* gate, int gate_ld, int below, hipStream_t stream, int splits = 1, void* part_o = nullptr,
-                              void* part_ml = nullptr) {
+                              void* part_ml = nullptr, FreshRows fresh = FreshRows{}) {
     const int group = heads / kv_heads;
     dim3 grid(tiles, HEADS ? kv_heads * ((group + 15) / 16) : heads, splits), block(LAM_WAVES * TL_WAVE);
     const size_t smem = sizeof(float) * LAM_WAVES * LAM_TOKENS * (2 + DV * 16);
-    auto kernel = local_attention_mfma_kernel<DK, DV, HEADS>;
+    auto kernel = local_attention_mfma_kernel<DK, DV, HEADS, FRESH>;
     static bool raised = false;                      // (per instance of the template)
     if (smem > 48 * 1024 && !raised) {
         hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
         raised = true;
     }
-    kernel<<<grid, block, smem, stream>>>((const bf16_t*)q, q_ld, (bf16_t*)out, out_ld, (const bf16_t*)k_plane, (const bf16_t*)v_plane,
+    kernel<<<grid, block, smem, stream>>>((const bf16_t*)q, q_ld, (bf16_t*)out, out_ld, (const bf16_t*)k_plane, (const bf16_t*)v_plane, fresh,
         (const int*)block_table, table_ld, table_width, (const int*)req_indptr, (const int*)ctx_lens, (const int*)tile_req, (const int*)tile_tok0,
         heads, kv_heads, page_size, scale, cap, mask, gain, (const float*)sink, (const bf16_t*)pk_plane, (const bf16_t*)pv_plane, (const int*)pool_table,
         pool_table_ld, pool_table_width, pool, back, (const bf16_t*)gate, gate_ld, below, (float*)part_o, (float2*)part_ml);
@@ -1004,14 +1045,15 @@ static bool local_prompt_fits(const LocalArgs& a, int dim, int vdim, int pages, 
 extern "C" int tl_local_heads_fits(int dim, int vdim) { return (dim == 64 || dim == 128 || dim == 192) && (vdim == 64 || vdim == 128); }
 
 // Tiles of up to 16 consecutive tokens of one request: tile i belongs to request tile_req[i] (null: request i) and starts at that
-// request's token tile_tok0[i] of the step (null: 0).
+// request's token tile_tok0[i] of the step (null: 0).  fresh_k, fresh_v (with splits; null: they are there): the tokens' own keys and values, which go to their pages.
 extern "C" int tl_local_attention_tiles(const void* q, int q_ld, void* out, int out_ld, const void* k_plane, const void* v_plane, int pages,
                                         const void* block_table, int table_ld, int table_width, const void* req_indptr, const void* ctx_lens,
                                         const void* tile_req, const void* tile_tok0, int tiles, int heads, int kv_heads, int dim, int vdim,
                                         int page_size, float scale, float cap, int chunk, int window, float gain, const void* sink,
                                         const void* pk_plane, const void* pv_plane, const void* pool_table, int pool_table_ld, int pool_table_width,
                                         int pool, int keep_first, const void* turn_freq, int turn_dims, int turn_halves, const void* gate, int gate_ld,
-                                        int tokens, int requests, int pool_pages, int splits, void* part_o, void* part_ml, hipStream_t stream) {
+                                        int tokens, int requests, int pool_pages, int splits, void* part_o, void* part_ml, const void* fresh_k, int fresh_k_ld, const void* fresh_v,
+                                        int fresh_v_ld, hipStream_t stream) {
     TL_REQUIRE(!gate || gate_ld >= heads, "local_attention_tiles: a gate has a number per head");
     TL_REQUIRE(!turn_freq || (turn_dims > 0 && turn_dims % 2 == 0 && turn_dims <= vdim && vdim % 2 == 0), "local_attention_tiles: an output of %d columns turned over %d", vdim, turn_dims);
     TL_REQUIRE(keep_first >= 0 && (keep_first == 0 || (window > 0 && chunk == 0)), "local_attention_tiles: kept first tokens stand beside a window, without chunks");
@@ -1032,13 +1074,18 @@ extern "C" int tl_local_attention_tiles(const void* q, int q_ld, void* out, int 
                       (const int*)pool_table, pool_table_ld, pool_table_width, pool, back, (const bf16_t*)gate, gate_ld, LP_LEAST, nullptr, nullptr, nullptr, 0, 0, 0, 0u, nullptr, 0};
     if (splits > 0) {        // one token a request, its heads together
         TL_REQUIRE(tl_local_heads_fits(dim, vdim) && tiles == tokens && splits <= TL_WAVE && (splits == 1 || (part_o && part_ml)), "local_attention_tiles: not built for these splits");
-#define TL_LAH(DK, DV)                                                                                                                       \
-    launch_local_mfma<DK, DV, true>(q, q_ld, out, out_ld, k_plane, v_plane, block_table, table_ld, table_width, req_indptr, ctx_lens,         \
+        TL_REQUIRE(!fresh_k || (fresh_v && !pool && fresh_k_ld >= kv_heads * dim && fresh_v_ld >= kv_heads * vdim && fresh_k_ld % 8 == 0 && ((uintptr_t)fresh_k & 15) == 0 && ((uintptr_t)fresh_v & 1) == 0),
+                   "local_attention_tiles: the tokens' own keys lie in whole pieces, without pooled blocks");
+        const FreshRows fresh{(const bf16_t*)fresh_k, (const bf16_t*)fresh_v, fresh_k_ld, fresh_v_ld, pages};
+#define TL_LAH(DK, DV) if (fresh_k) TL_LAH_F(DK, DV, true); else TL_LAH_F(DK, DV, false)
+#define TL_LAH_F(DK, DV, FRESH)                                                                                                              \
+    launch_local_mfma<DK, DV, true, FRESH>(q, q_ld, out, out_ld, k_plane, v_plane, block_table, table_ld, table_width, req_indptr, ctx_lens,  \
                                     tile_req, tile_tok0, tiles, heads, kv_heads, page_size, scale, cap, mask, gain, sink, pk_plane, pv_plane, \
-                                    pool_table, pool_table_ld, pool_table_width, pool, back, gate, gate_ld, INT_MAX, stream, splits, part_o, part_ml)
-        if (dim == 64) { if (vdim == 64) TL_LAH(2, 4); else TL_LAH(2, 8); }
-        else if (dim == 128) { if (vdim == 64) TL_LAH(4, 4); else TL_LAH(4, 8); }
-        else { if (vdim == 64) TL_LAH(6, 4); else TL_LAH(6, 8); }
+                                    pool_table, pool_table_ld, pool_table_width, pool, back, gate, gate_ld, INT_MAX, stream, splits, part_o, part_ml, fresh)
+        if (dim == 64) { if (vdim == 64) { TL_LAH(2, 4); } else { TL_LAH(2, 8); } }
+        else if (dim == 128) { if (vdim == 64) { TL_LAH(4, 4); } else { TL_LAH(4, 8); } }
+        else { if (vdim == 64) { TL_LAH(6, 4); } else { TL_LAH(6, 8); } }
+#undef TL_LAH_F
 #undef TL_LAH
         TL_CHECK_LAUNCH("local_attention_heads");
         if (splits > 1) {
@@ -1048,6 +1095,7 @@ extern "C" int tl_local_attention_tiles(const void* q, int q_ld, void* out, int 
         }
         return TL_OK;
     }
+    TL_REQUIRE(!fresh_k, "local_attention_tiles: the tokens' own keys and values are written where a token's heads go together");
     int below = INT_MAX;
     if (tile_req && (long)tiles * LAM_TOKENS >= tokens && local_prompt_pays(a, tokens) && local_prompt_fits(a, dim, vdim, pages, pool_pages)) {
         const long most = tokens / LP_LEAST, tiles_most = tokens / (LP_ROWS / a.gcap) + (requests < most ? requests : most);

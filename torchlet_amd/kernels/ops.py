@@ -1490,7 +1490,7 @@ def local_decode_splits(tokens: int, heads: int, kv_heads: int, keys: int, units
 def local_attention(q: torch.Tensor, out: torch.Tensor, k_plane: torch.Tensor, v_plane: torch.Tensor, block_table: torch.Tensor,
                     token_req: torch.Tensor, positions: torch.Tensor, heads: int, kv_heads: int, dim: int, vdim: int, page_size: int,
                     scale: float, softcap: float = 0.0, chunk: int = 0, window: int = 0, gain: float = 1.0, tiles=None,
-                    sink: torch.Tensor | None = None, pooled=None, keep_first: int = 0, turn_back=None, gate: torch.Tensor | None = None) -> None:
+                    sink: torch.Tensor | None = None, pooled=None, keep_first: int = 0, turn_back=None, gate: torch.Tensor | None = None, fresh=None) -> None:
     """Attention of the step's queries ``q [T, heads * dim]`` over their requests' cached keys and values (which hold the step's own tokens
     already): query head ``i`` reads key/value head ``i // (heads / kv_heads)``; ``score = q . k * scale``, then (``softcap > 0``) ``softcap *
     tanh(score / softcap)``; a query at position ``p`` reads the keys ``j <= p`` with ``j // chunk == p // chunk`` (``chunk > 0``) and ``j > p -
@@ -1503,7 +1503,8 @@ def local_attention(q: torch.Tensor, out: torch.Tensor, k_plane: torch.Tensor, v
     ``keep_first`` (with a window, without chunks): a query also reads the keys at the positions ``0 .. keep_first - 1``, wherever it stands.
     ``turn_back = (inv_freq, dims, halves)``: the first ``dims`` columns of a head's output at position ``p`` turn by ``-float32(p) * inv_freq[m]``
     (float32 ``[dims / 2]``), pair ``m`` being ``2m`` and ``2m + 1`` or, ``halves``, ``m`` and ``m + dims / 2``.  ``gate [T, heads]`` (of ``q``'s dtype, rows may
-    be strided): head ``n``'s output of token ``t`` is multiplied by ``sigmoid(gate[t, n])``."""
+    be strided): head ``n``'s output of token ``t`` is multiplied by ``sigmoid(gate[t, n])``.  ``fresh = (k, v)``: the step's keys and values as :func:`kv_cache_write` takes
+    them, not in their pages yet: they are there when this returns (written by the attention's kernel itself in a step of single tokens whose heads go together)."""
     T = q.shape[0]
     if gate is not None and (gate.dtype != q.dtype or gate.shape != (T, heads) or gate.stride(1) != 1):
         raise KernelError(f"local_attention: a gate is [T, {heads}] of the queries' dtype")
@@ -1554,14 +1555,24 @@ def local_attention(q: torch.Tensor, out: torch.Tensor, k_plane: torch.Tensor, v
             if splits > 1:
                 part_o = torch.empty((T * heads * splits, vdim), dtype=torch.float32, device=q.device)
                 part_ml = torch.empty((T * heads * splits, 2), dtype=torch.float32, device=q.device)
+        fresh_args = (c_void_p(0), c_int(0), c_void_p(0), c_int(0))
+        if fresh is not None:
+            k, v = fresh
+            if splits > 0 and pooled is None and k.dtype == v.dtype == q.dtype and k.shape == (T, kv_heads * dim) and v.shape == (T, kv_heads * vdim) and k.stride(1) == v.stride(1) == 1 \
+                    and k.stride(0) % 8 == 0 and k.data_ptr() % 16 == 0:
+                fresh_args = (_ptr(k), c_int(k.stride(0)), _ptr(v), c_int(v.stride(0)))
+            else:
+                kv_cache_write(k, v, token_req, positions, block_table, k_plane, v_plane, page_size)
         _check(lib, lib.tl_local_attention_tiles(_ptr(q), c_int(q.stride(0)), _ptr(out), c_int(out.stride(0)), _ptr(k_plane), _ptr(v_plane),
                                                  c_int(k_plane.shape[0]), _ptr(block_table), c_int(block_table.stride(0)), c_int(block_table.shape[1]),
                                                  _ptr(req_indptr), _ptr(ctx_lens), _ptr(tile_req), _ptr(tile_tok0), c_int(n_tiles), c_int(heads),
                                                  c_int(kv_heads), c_int(dim), c_int(vdim), c_int(page_size), c_float(scale), c_float(softcap),
                                                  c_int(chunk), c_int(window), c_float(gain), *pool_args, c_int(pool_table.shape[1] if pool else 0),
                                                  c_int(pool), c_int(keep_first), *turn_args, *gate_args, c_int(T), c_int(R),
-                                                 c_int(pk_plane.shape[0] if pool else 0), c_int(splits), _ptr(part_o), _ptr(part_ml), _stream()))
+                                                 c_int(pk_plane.shape[0] if pool else 0), c_int(splits), _ptr(part_o), _ptr(part_ml), *fresh_args, _stream()))
         return
+    if fresh is not None:
+        kv_cache_write(*fresh, token_req, positions, block_table, k_plane, v_plane, page_size)
     _i32(token_req, "token_req", T)
     _i32(positions, "positions", T)
     _check(lib, lib.tl_local_attention(_ptr(q), c_int(q.stride(0)), _ptr(out), c_int(out.stride(0)), _ptr(k_plane), _ptr(v_plane), c_int(k_plane.shape[0]),

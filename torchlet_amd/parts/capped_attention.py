@@ -208,9 +208,12 @@ class CappedAttention(StagedMixer):
             pool_group, (pk_plane, pv_plane) = cache.more[0]
             pv_plane = pv_plane.view(pv_plane.shape[0], self.kv_heads, self.vdim, cache.page_size)
             pooled = (pk_plane, pv_plane, ctx.block_tables[pool_group], self.pool)
+        keys, more = proj[:, self.q_width: self.q_width + self.k_width], {}
         if cache.writable and not self.one_kernel:
-            ops.kv_cache_write(proj[:, self.q_width: self.q_width + self.k_width], values,
-                               ctx.token_req, ctx.positions, table, k_plane, v_plane, cache.page_size)
+            if h.is_cuda and ctx.decode_only and pooled is None:      # single tokens: their attention may put them into their pages as well
+                more["fresh"] = (keys, values)
+            else:
+                ops.kv_cache_write(keys, values, ctx.token_req, ctx.positions, table, k_plane, v_plane, cache.page_size)
         if cache.writable and pooled is not None:      # the blocks whose last token this step brings
             ops.pool_blocks(k_plane, v_plane, table, pk_plane, pv_plane, pooled[2], ctx.req_indptr, ctx.ctx_lens,
                             ctx.max_new_tokens // self.pool + 1, cache.page_size, self.pool)
@@ -221,4 +224,4 @@ class CappedAttention(StagedMixer):
         ops.local_attention(q, out, k_plane, v_plane, table, ctx.token_req, ctx.positions, self.heads, self.kv_heads, self.dim, self.vdim,
                             cache.page_size, self.scale, self.softcap, self.chunk, self.window, gain, tiles=tiles, sink=self.sink, pooled=pooled,
                             keep_first=self.keep_first, turn_back=turn_values,
-                            gate=proj[:, self.gate_at: self.gate_at + self.gate_cols] if self.gate_cols else None)
+                            gate=proj[:, self.gate_at: self.gate_at + self.gate_cols] if self.gate_cols else None, **more)
