@@ -21,6 +21,7 @@ struct Groups {
 union Frag16 {          // 16 bytes: eight bfloat16 as the MFMA wants them, or one 128-bit load
     uint4 u;
     bf16x8_t v;
+    float f[4];
 };
 
 // The gate of a fused gate/up product: GATE 1: silu(g) * u, GATE 2: relu(g) * u, GATE 3: gelu(g) * u in its tanh form (the value of SW in the

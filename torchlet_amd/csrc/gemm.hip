@@ -511,25 +511,6 @@ static void launch_gemm_f32_mfma(const void* x, const void* w, const void* bias,
     launch(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, stream);
 }
 
-// One named kernel of the 32-bit products (for tests and tuning): 0 the general tile kernel (v_fma_f32), 1 the matrix-core
-// tile kernel, 2 and 3 the kernels for up to 16 rows on multiply-adds and on the matrix cores, 4 to 6 the matrix-core tile kernel with tiles of 64 x 64, 64 x 128, 128 x 128,
-// 7 and 8 with 64 x 32 and 32 x 32.
-extern "C" int tl_gemm_f32_variant(const void* x, const void* w, const void* bias, int bias_f32, void* out,
-                                   int M, int N, int K, int ldx, int ldo, int matrix_cores, hipStream_t stream) {
-    TL_REQUIRE(M > 0 && N > 0 && K > 0 && ldx >= K && ldo >= N, "gemm_f32: bad sizes M=%d N=%d K=%d ldx=%d ldo=%d", M, N, K, ldx, ldo);
-    if (matrix_cores == 2 || matrix_cores == 3) {      // the two kernels for up to 16 rows: 2 multiply-adds, 3 matrix cores
-        TL_REQUIRE(gemv_f32_fits(x, w, M, K, ldx), "gemm_f32: the few-rows kernels need M <= 16, K %% 4 == 0 and 16-byte aligned rows");
-        launch_gemv_f32(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, stream, matrix_cores - 2);
-    } else if (matrix_cores) {
-        TL_REQUIRE(gemm_f32_mfma_fits(x, w, 17, K, ldx), "gemm_f32: the matrix-core kernel needs K %% 4 == 0 and 16-byte aligned rows");
-        launch_gemm_f32_mfma(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, stream, matrix_cores > 3 ? matrix_cores - 3 : 0);
-    } else {
-        launch_gemm_tile<float, float>(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, stream);
-    }
-    TL_CHECK_LAUNCH("gemm_f32");
-    return TL_OK;
-}
-
 // =====================================================================================
 // bfloat16 on the matrix cores, few rows (M <= 64): the decode step's products.
 //
@@ -1147,21 +1128,21 @@ struct TokenRow {
     const bf16_t* table;      // row ids[m] holds N numbers; rows ld apart; what is no row leaves its outputs as they are
     int ld, vocab, act;
 };
-template <int WJ, int XH, typename TOut, int SW = 0, int END = END_STORE>
-__global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const void* __restrict__ bias, int bias_f32,
+template <int WJ, int XH, typename TOut, int SW = 0, int END = END_STORE, typename T = bf16_t>
+__global__ __launch_bounds__((64 * ring_waves<WJ, T>())) void gemm_ring_kernel(const T* __restrict__ x, const T* __restrict__ w, const void* __restrict__ bias, int bias_f32,
                                                         TOut* __restrict__ out, int M, int N, int K, int ldx, int ldo, int out_cols, int k_per_split, int rps,
                                                         RopeArgs ra, TokenRow tk, Beside be, GroupStride gs) {
     constexpr bool RP = END == END_ROTATE, TK = END == END_TOKEN, BE = END == END_BESIDE;
     constexpr int HALVES = SW ? 2 : 1;
-    using S = RingShape<WJ, XH, HALVES>;
+    using S = RingShape<WJ, XH, HALVES, T>;
     static_assert(END == END_STORE || END == END_BESIDE || (!SW && S::MT == 1 && sizeof(TOut) == 2), "the rotation and the tokens' rows are built for up to 16 rows");
     extern __shared__ __attribute__((aligned(16))) char ring[];
     const int ldw = K;
     const bool beside = BE && (int)blockIdx.z == be.z;
     if (BE) {
         if (beside) {
-            x = be.x;
-            w = be.w;
+            x = (const T*)be.x;
+            w = (const T*)be.w;
             N = be.N;
             rps = min(rps, 8);
         }
@@ -1195,14 +1176,14 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict
 #pragma unroll
     for (int j = 0; j < WJ; ++j) {
         const int r = 8 * j + lane / 8, c = (lane % 8) ^ ((r >> 1) & 7), half = r / S::HR;
-        woff[j] = (unsigned)((row_of(min(n0 + r - half * S::HR, n_end - 1)) - row_of(n0) + 32 * half) * ldw + c * 8) * 2;
+        woff[j] = (unsigned)((row_of(min(n0 + r - half * S::HR, n_end - 1)) - row_of(n0) + 32 * half) * ldw) * (unsigned)sizeof(T) + c * 16;
     }
 #pragma unroll
     for (int j = 0; j < XH; ++j) {
         const int r = 8 * (WJ + j) + lane / 8, c = (lane % 8) ^ ((r >> 1) & 7);
-        xoff[j] = (unsigned)(min(r - 8 * WJ, M - 1) * ldx + c * 8) * 2;
+        xoff[j] = (unsigned)(min(r - 8 * WJ, M - 1) * ldx) * (unsigned)sizeof(T) + c * 16;
     }
-    ring_products<WJ, XH, HALVES>(w + (size_t)row_of(n0) * ldw, woff, x, xoff, K / 64, ring, wave, ring_spread(ldw));
+    ring_products<WJ, XH, HALVES>(w + (size_t)row_of(n0) * ldw, woff, x, xoff, K / (128 / (int)sizeof(T)), ring, wave, ring_spread<T>(ldw));
     const bool quads = ldo % 4 == 0 && n0 % 4 == 0 && ((uintptr_t)out % (4 * sizeof(TOut))) == 0;
     for (int q = wave; q < S::SH * S::MT; q += S::NW) {
         const int s = q / S::MT, t = q % S::MT, m = 16 * t + li, n = n0 + 16 * s + 4 * kg;
@@ -1212,9 +1193,9 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict
 #pragma unroll
             for (int v = 0; v < 4; ++v) own[v] = known ? to_float(tk.table[(size_t)tk_id * tk.ld + min(n + v, N - 1)]) : 0.f;
         }
-        f32x4_t sum = ring_sum<WJ, XH, HALVES>(ring, s, t);
+        f32x4_t sum = ring_sum<WJ, XH, HALVES, T>(ring, s, t);
         if constexpr (SW) {
-            const f32x4_t up = ring_sum<WJ, XH, HALVES>(ring, S::SH + s, t);
+            const f32x4_t up = ring_sum<WJ, XH, HALVES, T>(ring, S::SH + s, t);
 #pragma unroll
             for (int v = 0; v < 4; ++v) sum[v] = gate_mul<SW>(sum[v], up[v]);
         } else if (bias) {
@@ -1249,6 +1230,19 @@ static bool ring_fits(const void* x, const void* w, int M, int K, int ldx) {
     return M > 0 && M <= 64 && K % 64 == 0 && ldx % 8 == 0 && K < (1 << 23) && ldx < (1 << 23) && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0;
 }
 
+// The same in 32 bits: slabs of 32 columns, up to 16 rows.
+static bool ring_fits_f32(const void* x, const void* w, int M, int K, int ldx) {
+    return M > 0 && M <= 16 && K % 32 == 0 && ldx % 4 == 0 && K < (1 << 22) && ldx < (1 << 22) && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0;
+}
+
+// And where they are taken, against the multiply-add kernel (up to 8 rows) and the matrix-core kernel (above) that fetch into registers behind a copy of x and begin every chunk of it with an empty
+// pipe (us, those / the rings, weights from memory): 4 rows 4608 x 3584 17.8 / 14.9, 37888 x 3584 109 / 94, 3584 x 18944 61 / 47.6, 152064 x 3584 391 / 360; 8 rows 23 / 15.4, 122 / 95, 87 / 49,
+// 454 / 366; 16 rows 25 / 15.7, 131 / 100, 112 / 54, 482 / 374, 512 x 512 4.3 / 3.2.  One row keeps its sums' order whatever stands beside it, so the line does not hang on the number of rows up to 8, and
+// one or two of them lose a little against wide matrices (one row, 37888 x 3584 89.6 / 93, 152064 x 3584 346 / 352, 3584 x 18944 49.0 / 47.7, 8192 x 8192 54 / 48).  Narrow matrices want more work-groups than
+// these have (4 rows, 256 x 2048 5.2 / 5.5, 64 x 4096 7.5 / 8.3).  The sums' error against 64 bits (relative): K 2048 1.2e-7 / 1.0e-7, 3584 1.5e-7 / 1.1e-7, 18944 3.1e-7 / 1.8e-7, above 8 rows
+// 3.8e-7 / 1.1e-7; at 512 columns up to 8 rows 0.87e-7 / 0.9e-7, and so short sums stay where they are.
+static bool ring_pays_f32(int M, int N, int K) { return M > 8 || (K >= 1024 && N >= 1024); }
+
 // Where a product of up to 64 rows goes through the rings, K a multiple of 64: measured against what it took before them, the tiles or the few-rows kernel that fetches into registers, over a grid
 // of widths and depths (us, the other / this).
 //   Up to 16 rows up to 32768 columns, 2 to 8 rows any number: 12 rows, 152064 x 3584 190 / 194, 8 rows 197 / 187, 1 row 179 / 187, 2 rows 151936 x 896 53 / 50.
@@ -1282,43 +1276,43 @@ struct RingCall {
     Beside be = Beside{};
 };
 
-template <int WJ, int XH, typename TOut, int SW, int END>
+template <int WJ, int XH, typename TOut, int SW, int END, typename T>
 static int launch_ring_t(const RingCall& c, int rows, hipStream_t stream) {
-    using S = RingShape<WJ, XH, SW ? 2 : 1>;
-    auto kernel = gemm_ring_kernel<WJ, XH, TOut, SW, END>;
+    using S = RingShape<WJ, XH, SW ? 2 : 1, T>;
+    auto kernel = gemm_ring_kernel<WJ, XH, TOut, SW, END, T>;
     static hipError_t allowed = allow_lds(kernel, S::LDS);
     TL_REQUIRE(allowed == hipSuccess, "gemm_ring: cannot get %zu bytes of shared memory", S::LDS);
     const int total = SW ? c.out_cols : c.N, least = min(rows, 8), wide = max((total + rows - 1) / rows, (c.be.N + least - 1) / least);      // (be.N: 0 without a product beside)
-    kernel<<<dim3(wide, c.parts, c.gr.count + (END == END_BESIDE)), 256, S::LDS, stream>>>((const bf16_t*)c.x, (const bf16_t*)c.w, c.bias, c.bias_f32, (TOut*)c.out, c.M, c.N, c.K,
+    kernel<<<dim3(wide, c.parts, c.gr.count + (END == END_BESIDE)), 64 * S::NW, S::LDS, stream>>>((const T*)c.x, (const T*)c.w, c.bias, c.bias_f32, (TOut*)c.out, c.M, c.N, c.K,
                                                                                       c.ldx, c.ldo, c.out_cols, c.k_per, rows, c.ra, c.tk, c.be, c.gr.stride);
     TL_CHECK_LAUNCH("gemm_ring");
     return TL_OK;
 }
 
-template <int XH, typename TOut, int SW, int END>
+template <int XH, typename TOut, int SW, int END, typename T>
 static int launch_ring_x(const RingCall& c, RingPlan p, hipStream_t stream) {
     switch (p.wj) {
-    case 2: return launch_ring_t<2, XH, TOut, SW, END>(c, p.rows, stream);
-    case 4: return launch_ring_t<4, XH, TOut, SW, END>(c, p.rows, stream);
-    case 6: return launch_ring_t<6, XH, TOut, SW, END>(c, p.rows, stream);
-    case 8: return launch_ring_t<8, XH, TOut, SW, END>(c, p.rows, stream);
+    case 2: return launch_ring_t<2, XH, TOut, SW, END, T>(c, p.rows, stream);
+    case 4: return launch_ring_t<4, XH, TOut, SW, END, T>(c, p.rows, stream);
+    case 6: return launch_ring_t<6, XH, TOut, SW, END, T>(c, p.rows, stream);
+    case 8: return launch_ring_t<8, XH, TOut, SW, END, T>(c, p.rows, stream);
     }
     if constexpr (!SW) {
-        if (p.wj == 1) return launch_ring_t<1, XH, TOut, SW, END>(c, p.rows, stream);
-        if (p.wj == 3) return launch_ring_t<3, XH, TOut, SW, END>(c, p.rows, stream);
+        if (p.wj == 1) return launch_ring_t<1, XH, TOut, SW, END, T>(c, p.rows, stream);
+        if (p.wj == 3) return launch_ring_t<3, XH, TOut, SW, END, T>(c, p.rows, stream);
     }
     TL_REQUIRE(false, "gemm_ring: no shape of %d requests", p.wj);
 }
 
 // `p.wj` 0: the plan is made here.
-template <typename TOut, int SW, int END>
+template <typename TOut, int SW, int END, typename T = bf16_t>
 static int launch_ring(const RingCall& c, hipStream_t stream, RingPlan p = RingPlan{0, 0}) {
-    if (p.wj == 0) p = plan_ring(SW ? c.out_cols : c.N, c.M, SW ? 2 : 1, TL_COMPUTE_UNITS / (c.parts * c.gr.count), END == END_ROTATE, ring_spread(c.K), c.parts > 1);
-    if (c.M <= 8) return launch_ring_x<1, TOut, SW, END>(c, p, stream);
-    if (c.M <= 16) return launch_ring_x<2, TOut, SW, END>(c, p, stream);
-    if constexpr (END == END_STORE) {
-        if (c.M <= 32) return launch_ring_x<4, TOut, SW, END>(c, p, stream);
-        return launch_ring_x<8, TOut, SW, END>(c, p, stream);
+    if (p.wj == 0) p = plan_ring(SW ? c.out_cols : c.N, c.M, SW ? 2 : 1, TL_COMPUTE_UNITS / (c.parts * c.gr.count), END == END_ROTATE, ring_spread<T>(c.K), c.parts > 1);
+    if (c.M <= 8) return launch_ring_x<1, TOut, SW, END, T>(c, p, stream);
+    if (c.M <= 16) return launch_ring_x<2, TOut, SW, END, T>(c, p, stream);
+    if constexpr (END == END_STORE && sizeof(T) == 2) {
+        if (c.M <= 32) return launch_ring_x<4, TOut, SW, END, T>(c, p, stream);
+        return launch_ring_x<8, TOut, SW, END, T>(c, p, stream);
     }
     TL_REQUIRE(false, "gemm_ring: too many rows (%d)", c.M);
 }
@@ -1353,6 +1347,30 @@ extern "C" int tl_gemm_ring_variant(const void* x, const void* w, const void* bi
     if (gate == 2) return launch_ring<bf16_t, 2, END_STORE>(c, stream, p);
     if (gate == 3) return launch_ring<bf16_t, 3, END_STORE>(c, stream, p);
     return out_f32 ? launch_ring<float, 0, END_STORE>(c, stream, p) : launch_ring<bf16_t, 0, END_STORE>(c, stream, p);
+}
+
+// One named kernel of the 32-bit products (for tests and tuning): 0 the general tile kernel (v_fma_f32), 1 the matrix-core
+// tile kernel, 2 and 3 the kernels for up to 16 rows on multiply-adds and on the matrix cores, 4 to 6 the matrix-core tile kernel with tiles of 64 x 64, 64 x 128, 128 x 128,
+// 7 and 8 with 64 x 32 and 32 x 32; 9 the rings, which are what 2 (sizes that ring_pays_f32 gives them) and 3 (any) stand for where they fit, as in the dispatch.
+extern "C" int tl_gemm_f32_variant(const void* x, const void* w, const void* bias, int bias_f32, void* out,
+                                   int M, int N, int K, int ldx, int ldo, int matrix_cores, hipStream_t stream) {
+    TL_REQUIRE(M > 0 && N > 0 && K > 0 && ldx >= K && ldo >= N, "gemm_f32: bad sizes M=%d N=%d K=%d ldx=%d ldo=%d", M, N, K, ldx, ldo);
+    const bool rings = ring_fits_f32(x, w, M, K, ldx);
+    if (matrix_cores == 9 || (rings && (matrix_cores == 3 || (matrix_cores == 2 && ring_pays_f32(8, N, K))))) {
+        TL_REQUIRE(rings, "gemm_f32: the rings need M <= 16, K %% 32 == 0 and 16-byte aligned rows");
+        return launch_ring<float, 0, END_STORE, float>(RingCall{x, w, bias, bias_f32, out, M, N, K, ldx, ldo, 0}, stream);
+    }
+    if (matrix_cores == 2 || matrix_cores == 3) {      // the two kernels for up to 16 rows: 2 multiply-adds, 3 matrix cores
+        TL_REQUIRE(gemv_f32_fits(x, w, M, K, ldx), "gemm_f32: the few-rows kernels need M <= 16, K %% 4 == 0 and 16-byte aligned rows");
+        launch_gemv_f32(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, stream, matrix_cores - 2);
+    } else if (matrix_cores) {
+        TL_REQUIRE(gemm_f32_mfma_fits(x, w, 17, K, ldx), "gemm_f32: the matrix-core kernel needs K %% 4 == 0 and 16-byte aligned rows");
+        launch_gemm_f32_mfma(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, stream, matrix_cores > 3 ? matrix_cores - 3 : 0);
+    } else {
+        launch_gemm_tile<float, float>(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, stream);
+    }
+    TL_CHECK_LAUNCH("gemm_f32");
+    return TL_OK;
 }
 
 // One named instance of the few-rows kernel, of those the dispatch below can pick (for tests and tuning);
@@ -1843,6 +1861,7 @@ static bool skinny_fits(const void* x, const void* w, int M, int K, int ldx) {
 //     everything else             -> gemm_dl_tile (matrix cores, operands straight into shared memory)
 //   bfloat16, aligned, other K, M <= 64 -> gemm_skinny, except that 33..64 rows against a wide matrix go to the tile kernel
 //   bfloat16, aligned, other K, M > 64  -> gemm_mfma_tile (matrix cores, shared-memory tiles)
+//   32-bit, aligned, K a multiple of 32, M <= 16 as ring_pays_f32 says -> gemm_ring (true 32-bit arithmetic on the matrix cores)
 //   32-bit, aligned, M <= 16    -> gemv_f32 (true 32-bit arithmetic, weight streaming)
 //   32-bit, aligned, M > 16     -> gemm_f32_mfma (true 32-bit arithmetic on the matrix cores)
 //   everything else             -> gemm_tile (true 32-bit arithmetic)
@@ -1880,6 +1899,10 @@ extern "C" int tl_gemm(const void* x, const void* w, const void* bias, int bias_
         else pick_skinny<4>(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, out_f32, stream);
         TL_CHECK_LAUNCH("gemm_skinny");
         return TL_OK;
+    }
+    if (dtype == TL_DT_F32 && ring_fits_f32(x, w, M, K, ldx) && ring_pays_f32(M, N, K)) {
+        const RingCall c{x, w, bias, bias_f32, out, M, N, K, ldx, ldo, 0};
+        return launch_ring<float, 0, END_STORE, float>(c, stream);
     }
     if (dtype == TL_DT_F32 && gemv_f32_fits(x, w, M, K, ldx)) {
         launch_gemv_f32(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, stream);

@@ -15,15 +15,21 @@
 //   1 row: 2048 x 2048 3.8 -> 3.2, 4608 x 3584 8.1 -> 7.4;  8 rows: 256 x 2048 4.1 -> 3.1, 2048 x 2048 5.0 -> 3.5, 6144 x 2048 9.1 -> 6.5, 4096 x 4096 11.8 -> 7.6, gate and up
 //   of 2 x 18944 x 3584 50.6 -> 46.9;  16 rows: 34 x 4096 8.9 -> 4.2, 2048 x 2048 6.2 -> 3.7, gate and up of 2 x 11264 x 4096 38.9 -> 32.0;  32 rows: 4608 x 3584 21.8 -> 10.8
 //
+// float: a slab is 32 columns, the same 128 bytes of every row, and the products are v_mfma_f32_16x16x4_f32's, which multiply and add in 32 bits.  A slab's sums are taken two instructions at a
+// time from zero and then added to the wave's, so that a long sum has few roundings in a row.  An instruction takes 32 cycles, 256 a slab and block of weight rows: work-groups of few
+// weight rows, which have a unit to themselves, deal K to eight waves; sum s % 8 of slab s is then a wave's only one, so the order is the same.
+//
 // HALVES 2: the weight rows are two halves of 4 WJ rows (the gate's and the up matrix's rows of the same outputs).
-template <int WJ, int XH, int HALVES = 1>
+template <int WJ, typename T>
+constexpr int ring_waves() { return sizeof(T) == 4 && WJ <= 3 ? 8 : 4; }
+template <int WJ, int XH, int HALVES = 1, typename T = bf16_t>
 struct RingShape {
-    static constexpr int NW = 4;
+    static constexpr int NW = ring_waves<WJ, T>();
     static constexpr int SLOT = (WJ + XH) * 1024;                          // bytes of a slab: 8 (WJ + XH) rows of 128
     static constexpr int FIT = 80 * 1024 / (NW * SLOT), D = FIT < 2 ? 2 : FIT > 4 ? 4 : FIT;
     static constexpr int HR = 8 * WJ / HALVES, SH = (HR + 15) / 16;        // weight rows of a half, and the blocks of 16 they make
     static constexpr int STRIPS = HALVES * SH, MT = (XH + 1) / 2;          // blocks of 16 weight rows and of 16 rows of x
-    static constexpr int SETS = XH <= 2 ? 2 : 1;                           // sets of sums a wave keeps: see ring_products
+    static constexpr int SETS = XH <= 2 ? 8 / NW : 1;                           // sets of sums a wave keeps: see ring_products
     static constexpr size_t LDS = (size_t)NW * D * SLOT;
     static_assert(WJ % HALVES == 0 && (HALVES - 1) * HR + 16 * SH <= 8 * (WJ + XH), "a block that is not full reads on in its own slab");
     static_assert(SETS * STRIPS * MT * 1024 <= D * SLOT, "a wave's sums fit its own ring");
@@ -47,15 +53,16 @@ struct RingShape {
 // slabs the first rule falls in with the pitch of the work-groups' rows at some sizes (us, first / second / the kernel that fetches into registers: 20000 x 8192, one row, 67.7 / 58.6 / 60.4,
 // 10240 x 8192, 2 rows, 37.7 / 31.8 / 34.8, gate 24640 x 8192, 4 rows, 160 / 139 / 147; over 44 sizes of K 8192 and more the second takes 0.98 of the first), with few it is a little ahead
 // (2560 x 2048, 16 rows, 4.5 / 4.7; over 22 sizes of K up to 4096 and up to 6144 columns 0.996).
-__host__ __device__ inline bool ring_spread(int pitch) { return pitch % 2048 == 0; }
+template <typename T = bf16_t>
+__host__ __device__ inline bool ring_spread(int pitch) { return pitch % (4096 / (int)sizeof(T)) == 0; }
 __device__ __forceinline__ int ring_start(unsigned group, unsigned slabs_of_a_wave) {
     return (int)((slabs_of_a_wave <= 16 ? 5 * group + group / 8 : group % 8 * slabs_of_a_wave / 8 + 3 * (group / 8)) % slabs_of_a_wave);
 }
 
-template <int WJ, int XH, int HALVES>
-__device__ __forceinline__ void ring_products(const bf16_t* w, const unsigned (&woff)[WJ], const bf16_t* x, const unsigned (&xoff)[XH], int slabs, char* ring, int wave, bool spread) {
-    using S = RingShape<WJ, XH, HALVES>;
-    constexpr int NW = S::NW, D = S::D, LPS = WJ + XH, MT = S::MT;
+template <int WJ, int XH, int HALVES, typename T>
+__device__ __forceinline__ void ring_products(const T* w, const unsigned (&woff)[WJ], const T* x, const unsigned (&xoff)[XH], int slabs, char* ring, int wave, bool spread) {
+    using S = RingShape<WJ, XH, HALVES, T>;
+    constexpr int NW = S::NW, D = S::D, LPS = WJ + XH, MT = S::MT, COLS = 128 / sizeof(T);
     const int lane = threadIdx.x & 63, li = lane & 15, kg = lane >> 4;
     char* own = ring + wave * (D * S::SLOT);
     const unsigned own_at = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)((void __attribute__((address_space(3)))*)own));
@@ -63,7 +70,7 @@ __device__ __forceinline__ void ring_products(const bf16_t* w, const unsigned (&
     const int from = spread && mine >= 8 ? ring_start(blockIdx.x, mine) : 0;
     auto request = [&](int i) {
         const int turned = i + from < mine ? i + from : i + from - mine;
-        const int k = 64 * (wave + turned * NW);
+        const int k = COLS * (wave + turned * NW);
         const unsigned at = own_at + (unsigned)((i % D) * S::SLOT);
 #pragma unroll
         for (int j = 0; j < WJ; ++j) load_to_lds_at(w + k, woff[j], at + j * 1024);
@@ -101,6 +108,7 @@ __device__ __forceinline__ void ring_products(const bf16_t* w, const unsigned (&
         else if (D > 2 && after == 1) wait_direct_loads<(D > 2 ? 1 : 0) * LPS>();
         else wait_direct_loads<0>();
         const char* slab = own + (i % D) * S::SLOT;
+        f32x4_t part[2][2][S::STRIPS][MT];          // (float) a slab's sums by pairs of instructions
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             Frag16 wf[S::STRIPS], xf[MT];
@@ -108,10 +116,26 @@ __device__ __forceinline__ void ring_products(const bf16_t* w, const unsigned (&
             for (int t = 0; t < MT; ++t) xf[t].u = *(const uint4*)(slab + xat[t][h]);
 #pragma unroll
             for (int s = 0; s < S::STRIPS; ++s) wf[s].u = *(const uint4*)(slab + wat[s][h]);
+            if constexpr (sizeof(T) == 4) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int s = 0; s < S::STRIPS; ++s)
+#pragma unroll
+                        for (int t = 0; t < MT; ++t)
+                            part[h][e & 1][s][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[s].f[e], xf[t].f[e], e < 2 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : part[h][e & 1][s][t], 0, 0, 0);
+            } else {
+#pragma unroll
+                for (int s = 0; s < S::STRIPS; ++s)
+#pragma unroll
+                    for (int t = 0; t < MT; ++t) sums[s][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[s].v, xf[t].v, sums[s][t], 0, 0, 0);
+            }
+        }
+        if constexpr (sizeof(T) == 4) {
 #pragma unroll
             for (int s = 0; s < S::STRIPS; ++s)
 #pragma unroll
-                for (int t = 0; t < MT; ++t) sums[s][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[s].v, xf[t].v, sums[s][t], 0, 0, 0);
+                for (int t = 0; t < MT; ++t) sums[s][t] += (part[0][0][s][t] + part[0][1][s][t]) + (part[1][0][s][t] + part[1][1][s][t]);
         }
         if (i + D < mine) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // this slab has been read: its place is filled anew
@@ -137,9 +161,9 @@ __device__ __forceinline__ void ring_products(const bf16_t* w, const unsigned (&
 }
 
 // The waves' sums of block s of weight rows and block t of x: element v is weight row 16 (s % SH) + 4 (lane / 16) + v of half s / SH against x row 16 t + lane % 16.
-template <int WJ, int XH, int HALVES>
+template <int WJ, int XH, int HALVES, typename T = bf16_t>
 __device__ __forceinline__ f32x4_t ring_sum(const char* ring, int s, int t) {
-    using S = RingShape<WJ, XH, HALVES>;
+    using S = RingShape<WJ, XH, HALVES, T>;
     f32x4_t sum = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int u = 0; u < S::SETS; ++u)
