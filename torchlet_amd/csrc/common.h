@@ -104,6 +104,15 @@ __device__ __forceinline__ float sigmoid(float v) { return 1.f / (1.f + expf(-v)
 // z / 2 (1 + tanh(y)), y = sqrt(2 / pi) (z + 0.044715 z^3), with (1 + tanh(y)) / 2 = sigmoid(2 y).
 __device__ __forceinline__ float gelu_tanh(float z) { return z * sigmoid(1.5957691216057308f * fmaf(0.044715f * z * z, z, z)); }
 
+// One pair turned by its angle, in a fixed sequence of roundings (one product, one fused
+// multiply-add per result), so that every kernel here gives the same bits for the same input.
+__device__ __forceinline__ void rope_turn(float& x1, float& x2, float c, float sn) {
+    const float y1 = __fmaf_rn(x1, c, -__fmul_rn(x2, sn));
+    const float y2 = __fmaf_rn(x2, c, __fmul_rn(x1, sn));
+    x1 = y1;
+    x2 = y2;
+}
+
 // Sum over a block of up to 1024 threads; every thread gets the result.
 // `red` points to at least 16 floats of shared memory.
 __device__ __forceinline__ float block_sum(float v, float* red) {

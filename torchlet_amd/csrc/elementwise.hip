@@ -281,15 +281,6 @@ extern "C" int tl_add_rmsnorm(void* residual, const void* pending, int parts, in
 //     [pages, kv_heads, head_dim, page], the layout the attention kernels read.  Page 0 is the
 //     sentinel that empty block-table entries point to: a token whose page is 0 (a padding row of a
 //     step of fixed shape) has its keys and values dropped, so nothing ever writes that page.
-// One pair turned by its angle, in a fixed sequence of roundings (one product, one fused
-// multiply-add per result), so that every kernel here gives the same bits for the same input.
-__device__ __forceinline__ void rope_turn(float& x1, float& x2, float c, float sn) {
-    const float y1 = __fmaf_rn(x1, c, -__fmul_rn(x2, sn));
-    const float y2 = __fmaf_rn(x2, c, __fmul_rn(x1, sn));
-    x1 = y1;
-    x2 = y2;
-}
-
 #define ROPE_HEADS_PER_GROUP 4          // one wave per head, four heads per work-group
 template <typename T>
 __global__ __launch_bounds__(ROPE_HEADS_PER_GROUP * TL_WAVE)

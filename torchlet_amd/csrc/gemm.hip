@@ -119,17 +119,66 @@ extern "C" int tl_gemm_general(const void* x, const void* w, const void* bias, i
 // added up in a fixed butterfly order.  A row's result therefore depends on neither M nor the
 // other rows, as in the tile kernel, but its rounding differs from the tile kernel's (another
 // order of the same sum).  Needs K % 4 == 0 and 16-byte aligned rows.
+//
+// END (see F32Pairs): a wave's two rows are what a gate or a rotation joins, and its sums go on to that, with the bits that the kernels behind a plain product would leave (us, one row, two
+// launches / one, profiled: query, key and value of 5 heads of 32 from 96 columns 5.7 / 4.5; gate and up of 2 x 200 x 96 4.8 / 3.2; and a launch's gap less).
 #define GV_ROWS 8
-template <int MR>
+#define F32_PLAIN 0
+#define F32_GATE 1
+#define F32_ROTATE 2
+// Rows of the matrix by pairs: pair p is the rows a = p / span * 2 span + p % span and a + span.  The gate's: span outputs, the gate's rows and then the up rows, out[m, p] = act(a) * b.  The
+// rotation's: span is half a head, the two elements that a frequency turns (queries and keys; values are as they are); queries go to out, keys and values to their pages.
+struct F32Pairs {
+    int count, span, act;
+    const int* positions;      // [M]
+    const float* inv_freq;     // [head_dim / 2]
+    const int* token_req;      // [M] request of each row (null: no cache write)
+    const int* block_table;    // [requests, bt_stride]
+    float* k_plane;            // [pages, kv_heads, page, head_dim]
+    float* v_plane;            // [pages, kv_heads, head_dim, page]
+    int bt_stride, page, q_heads, kv_heads;
+    __host__ __device__ int row(int p) const { return p / span * 2 * span + p % span; }
+};
+__device__ __forceinline__ float f32_gate(int act, float g, float u) { return (act == 1 ? fmaxf(g, 0.f) : act == 2 ? gelu_tanh(g) : g / (1.f + expf(-g))) * u; }
+// Pair p's cosine and sine at position pos, made while the weights are on their way.
+__device__ __forceinline__ float2 f32_turn(const F32Pairs& pa, int p, int pos) {
+    const float angle = (float)pos * pa.inv_freq[min(p, pa.count - 1) % pa.span];
+    return make_float2(cosf(angle), sinf(angle));
+}
+// Pair p of row m, at position pos of page `page`.
+__device__ __forceinline__ void f32_turn_store(const F32Pairs& pa, int p, float y1, float y2, float2 turn, int m, int pos, int page, float* out, int ldo) {
+    const int half = pa.span, head = p / half, j = p - head * half, hd = 2 * half;
+    if (head < pa.q_heads + pa.kv_heads) rope_turn(y1, y2, turn.x, turn.y);
+    if (head < pa.q_heads) {
+        float* o = out + (size_t)m * ldo + head * hd + j;
+        o[0] = y1;
+        o[half] = y2;
+    } else if (page != 0) {       // page 0 is the sentinel (a padding row's): never written
+        const int off = pos % pa.page;
+        const size_t base = ((size_t)page * pa.kv_heads + (head - pa.q_heads) % pa.kv_heads) * pa.page * hd;
+        const bool key = head < pa.q_heads + pa.kv_heads;
+        float* o = key ? pa.k_plane + base + (size_t)off * hd + j : pa.v_plane + base + (size_t)j * pa.page + off;
+        o[0] = y1;
+        o[(size_t)half * (key ? 1 : pa.page)] = y2;
+    }
+}
+template <int MR, int END>
 __global__ __launch_bounds__(256) void gemv_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                        const void* __restrict__ bias, int bias_f32,
-                                                       float* __restrict__ out, int M, int N, int K, int ldx, int ldo) {
+                                                       float* __restrict__ out, int M, int N, int K, int ldx, int ldo, F32Pairs pa) {
     constexpr int KC = MR >= 8 ? 512 : 1024;       // 32 KB of x at most; at eight rows the shorter chunk keeps the kernel to 128 registers
     __shared__ float4 xs[MR][KC / 4];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int n0 = blockIdx.x * GV_ROWS + wave * 2;
-    const float* wa = w + (size_t)min(n0, N - 1) * K;        // rows past the end: read the last row, write nothing
-    const float* wb = w + (size_t)min(n0 + 1, N - 1) * K;
+    const int n0 = blockIdx.x * GV_ROWS + wave * 2, pair = n0 / 2;
+    const int first = END ? pa.row(min(pair, pa.count - 1)) : min(n0, N - 1), second = END ? first + pa.span : min(n0 + 1, N - 1);
+    const float* wa = w + (size_t)first * K;                 // rows past the end: read the last row, write nothing
+    const float* wb = w + (size_t)second * K;
+    int pos = 0, page = 0;                                   // (lane m: row m's)
+    if (END == F32_ROTATE) {
+        const int row = min(lane, M - 1);
+        pos = pa.positions[row];
+        if (pa.k_plane) page = pa.block_table[(size_t)pa.token_req[row] * pa.bt_stride + pos / pa.page];
+    }
     float acc[MR][2];
 #pragma unroll
     for (int m = 0; m < MR; ++m) acc[m][0] = acc[m][1] = 0.f;
@@ -149,6 +198,7 @@ __global__ __launch_bounds__(256) void gemv_f32_kernel(const float* __restrict__
     };
 #pragma unroll
     for (int j = 0; j < IPC; ++j) fetch(j, lane + 64 * j);
+    const float2 turn = END == F32_ROTATE ? f32_turn(pa, pair, pos) : make_float2(0.f, 0.f);
     for (int k0 = 0; k0 < K; k0 += KC) {
         const int pieces = min(KC, K - k0) / 4;
         __syncthreads();
@@ -180,6 +230,17 @@ __global__ __launch_bounds__(256) void gemv_f32_kernel(const float* __restrict__
     for (int m = 0; m < MR; ++m)
 #pragma unroll
         for (int r = 0; r < 2; ++r) acc[m][r] = wave_sum(acc[m][r]);
+    if constexpr (END != F32_PLAIN) {
+        float y1 = 0.f, y2 = 0.f;                            // lane m has row m
+#pragma unroll
+        for (int m = 0; m < MR; ++m)
+            if (lane == m) { y1 = acc[m][0]; y2 = acc[m][1]; }
+        if (lane >= M || pair >= pa.count) return;
+        if (bias) { y1 += load_vec(bias, bias_f32, first); y2 += load_vec(bias, bias_f32, second); }
+        if constexpr (END == F32_GATE) out[(size_t)lane * ldo + pair] = f32_gate(pa.act, y1, y2);
+        else f32_turn_store(pa, pair, y1, y2, turn, lane, pos, page, out, ldo);
+        return;
+    }
     if (lane < 2 && n0 + lane < N) {
         const int n = n0 + lane;
         const float b = bias ? load_vec(bias, bias_f32, n) : 0.f;
@@ -267,6 +328,18 @@ static bool gemv_f32_fits(const void* x, const void* w, int M, int K, int ldx) {
     return M <= 16 && K % 4 == 0 && ldx % 4 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0;
 }
 
+template <int END>
+static void launch_gemv_f32_fma(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int N, int K, int ldx, int ldo, const F32Pairs& pa, hipStream_t stream) {
+    dim3 grid((N + GV_ROWS - 1) / GV_ROWS), block(256);
+#define GV_LAUNCH(MR) gemv_f32_kernel<MR, END><<<grid, block, 0, stream>>>((const float*)x, (const float*)w, bias, bias_f32, (float*)out, M, N, K, ldx, ldo, pa)
+    if (M <= 1) GV_LAUNCH(1);
+    else if (M <= 2) GV_LAUNCH(2);
+    else if (M <= 4) GV_LAUNCH(4);
+    else if (M <= 8) GV_LAUNCH(8);
+    else if constexpr (END == F32_PLAIN) GV_LAUNCH(16);
+#undef GV_LAUNCH
+}
+
 // mfma: 0 the multiply-add kernel, 1 the matrix-core kernel, -1 the one that is faster for M.  Measured on the four
 // products of a 7B layer (us, multiply-adds / matrix cores): 1 row 174 / 237, 4 rows 216 / 241, 8 rows 274 / 265,
 // 16 rows 425 / 300: the matrix-core kernel's time hardly grows with the rows, but its work-groups of 16 weight rows
@@ -278,14 +351,7 @@ static void launch_gemv_f32(const void* x, const void* w, const void* bias, int 
                                                                                      (float*)out, M, N, K, ldx, ldo);
         return;
     }
-    dim3 grid((N + GV_ROWS - 1) / GV_ROWS), block(256);
-#define GV_LAUNCH(MR) gemv_f32_kernel<MR><<<grid, block, 0, stream>>>((const float*)x, (const float*)w, bias, bias_f32, (float*)out, M, N, K, ldx, ldo)
-    if (M <= 1) GV_LAUNCH(1);
-    else if (M <= 2) GV_LAUNCH(2);
-    else if (M <= 4) GV_LAUNCH(4);
-    else if (M <= 8) GV_LAUNCH(8);
-    else GV_LAUNCH(16);
-#undef GV_LAUNCH
+    launch_gemv_f32_fma<F32_PLAIN>(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, F32Pairs{}, stream);
 }
 
 // =====================================================================================
@@ -1131,11 +1197,12 @@ struct TokenRow {
 template <int WJ, int XH, typename TOut, int SW = 0, int END = END_STORE, typename T = bf16_t>
 __global__ __launch_bounds__((64 * ring_waves<WJ, T>())) void gemm_ring_kernel(const T* __restrict__ x, const T* __restrict__ w, const void* __restrict__ bias, int bias_f32,
                                                         TOut* __restrict__ out, int M, int N, int K, int ldx, int ldo, int out_cols, int k_per_split, int rps,
-                                                        RopeArgs ra, TokenRow tk, Beside be, GroupStride gs) {
+                                                        RopeArgs ra, TokenRow tk, Beside be, GroupStride gs, F32Pairs pa) {
     constexpr bool RP = END == END_ROTATE, TK = END == END_TOKEN, BE = END == END_BESIDE;
-    constexpr int HALVES = SW ? 2 : 1;
+    constexpr bool PAIRS = sizeof(T) == 4 && (SW || RP);      // float: rows by pairs (F32Pairs); out_cols counts them
+    constexpr int HALVES = SW || PAIRS ? 2 : 1;
     using S = RingShape<WJ, XH, HALVES, T>;
-    static_assert(END == END_STORE || END == END_BESIDE || (!SW && S::MT == 1 && sizeof(TOut) == 2), "the rotation and the tokens' rows are built for up to 16 rows");
+    static_assert(END == END_STORE || END == END_BESIDE || (!SW && S::MT == 1 && (sizeof(TOut) == 2 || PAIRS)), "the rotation and the tokens' rows are built for up to 16 rows");
     extern __shared__ __attribute__((aligned(16))) char ring[];
     const int ldw = K;
     const bool beside = BE && (int)blockIdx.z == be.z;
@@ -1161,22 +1228,30 @@ __global__ __launch_bounds__((64 * ring_waves<WJ, T>())) void gemm_ring_kernel(c
         K = min(K - kb, k_per_split);
     }
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 15, kg = lane >> 4;
-    const int n0 = blockIdx.x * rps, n_end = min(SW ? out_cols : N, n0 + rps);
+    const int n0 = blockIdx.x * rps, n_end = min(HALVES == 2 ? out_cols : N, n0 + rps);
     // (the waves that turn and write: their rows' positions and pages ahead of the weights, so that no wait for them lies behind the ring's)
     int rp_pos = 0, rp_page = 0;
-    if (RP && wave < S::STRIPS) {
+    float2 rp_turn[4] = {};
+    if (PAIRS && RP && wave < S::SH) {
+        const int row = min(li, M - 1);
+        rp_pos = pa.positions[row];
+        if (pa.k_plane) rp_page = pa.block_table[(size_t)pa.token_req[row] * pa.bt_stride + rp_pos / pa.page];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) rp_turn[v] = f32_turn(pa, n0 + 16 * wave + 4 * kg + v, rp_pos);
+    } else if (RP && !PAIRS && wave < S::STRIPS) {
         const int row = min(li, M - 1);
         rp_pos = ra.positions[row];
         if (ra.k_plane) rp_page = ra.block_table[(size_t)ra.token_req[row] * ra.bt_stride + rp_pos / ra.page];
     }
     const int tk_id = TK ? tk.ids[min(li, M - 1)] : 0;
-    // the matrix's row of an output's gate (or of the output itself); its up row lies 32 further on
-    auto row_of = [](int o) { return SW ? (o >> 5) * 64 + (o & 31) : o; };
+    // the matrix's row of an output's gate (or of the output itself); its up row lies 32 further on, a pair's second row a span
+    auto row_of = [&](int o) { return PAIRS ? pa.row(o) : SW ? (o >> 5) * 64 + (o & 31) : o; };
+    const int apart = PAIRS ? pa.span : 32;
     unsigned woff[WJ], xoff[XH];
 #pragma unroll
     for (int j = 0; j < WJ; ++j) {
         const int r = 8 * j + lane / 8, c = (lane % 8) ^ ((r >> 1) & 7), half = r / S::HR;
-        woff[j] = (unsigned)((row_of(min(n0 + r - half * S::HR, n_end - 1)) - row_of(n0) + 32 * half) * ldw) * (unsigned)sizeof(T) + c * 16;
+        woff[j] = (unsigned)(row_of(min(n0 + r - half * S::HR, n_end - 1)) - row_of(n0) + apart * half) * (unsigned)ldw * (unsigned)sizeof(T) + c * 16;
     }
 #pragma unroll
     for (int j = 0; j < XH; ++j) {
@@ -1194,7 +1269,20 @@ __global__ __launch_bounds__((64 * ring_waves<WJ, T>())) void gemm_ring_kernel(c
             for (int v = 0; v < 4; ++v) own[v] = known ? to_float(tk.table[(size_t)tk_id * tk.ld + min(n + v, N - 1)]) : 0.f;
         }
         f32x4_t sum = ring_sum<WJ, XH, HALVES, T>(ring, s, t);
-        if constexpr (SW) {
+        if constexpr (PAIRS) {
+            const f32x4_t up = ring_sum<WJ, XH, HALVES, T>(ring, S::SH + s, t);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                float a = sum[v], b = up[v];
+                if (SW) {
+                    sum[v] = f32_gate(pa.act, a, b);
+                } else if (m < M && n + v < n_end) {
+                    if (bias) { a += load_vec(bias, bias_f32, pa.row(n + v)); b += load_vec(bias, bias_f32, pa.row(n + v) + pa.span); }
+                    f32_turn_store(pa, n + v, a, b, rp_turn[v], m, rp_pos, rp_page, (float*)out, ldo);
+                }
+            }
+            if (RP) continue;
+        } else if constexpr (SW) {
             const f32x4_t up = ring_sum<WJ, XH, HALVES, T>(ring, S::SH + s, t);
 #pragma unroll
             for (int v = 0; v < 4; ++v) sum[v] = gate_mul<SW>(sum[v], up[v]);
@@ -1213,7 +1301,7 @@ __global__ __launch_bounds__((64 * ring_waves<WJ, T>())) void gemm_ring_kernel(c
                 if (n + v < n_end) be.out[(size_t)m * be.N + n + v] = sum[v];
             continue;
         }
-        if constexpr (RP) {
+        if constexpr (RP && !PAIRS) {
             rope_store(ra, sum, n, n_end, m, rp_pos, rp_page, (bf16_t*)out, ldo);
         } else if (quads && n + 3 < n_end) {
             store4(out + (size_t)m * ldo + n, make_float4(sum[0], sum[1], sum[2], sum[3]));
@@ -1274,17 +1362,19 @@ struct RingCall {
     RopeArgs ra = RopeArgs{};
     TokenRow tk = TokenRow{};
     Beside be = Beside{};
+    F32Pairs pa = F32Pairs{};
 };
 
 template <int WJ, int XH, typename TOut, int SW, int END, typename T>
 static int launch_ring_t(const RingCall& c, int rows, hipStream_t stream) {
-    using S = RingShape<WJ, XH, SW ? 2 : 1, T>;
+    constexpr int HALVES = SW || (END == END_ROTATE && sizeof(T) == 4) ? 2 : 1;
+    using S = RingShape<WJ, XH, HALVES, T>;
     auto kernel = gemm_ring_kernel<WJ, XH, TOut, SW, END, T>;
     static hipError_t allowed = allow_lds(kernel, S::LDS);
     TL_REQUIRE(allowed == hipSuccess, "gemm_ring: cannot get %zu bytes of shared memory", S::LDS);
-    const int total = SW ? c.out_cols : c.N, least = min(rows, 8), wide = max((total + rows - 1) / rows, (c.be.N + least - 1) / least);      // (be.N: 0 without a product beside)
+    const int total = HALVES == 2 ? c.out_cols : c.N, least = min(rows, 8), wide = max((total + rows - 1) / rows, (c.be.N + least - 1) / least);      // (be.N: 0 without a product beside)
     kernel<<<dim3(wide, c.parts, c.gr.count + (END == END_BESIDE)), 64 * S::NW, S::LDS, stream>>>((const T*)c.x, (const T*)c.w, c.bias, c.bias_f32, (TOut*)c.out, c.M, c.N, c.K,
-                                                                                      c.ldx, c.ldo, c.out_cols, c.k_per, rows, c.ra, c.tk, c.be, c.gr.stride);
+                                                                                      c.ldx, c.ldo, c.out_cols, c.k_per, rows, c.ra, c.tk, c.be, c.gr.stride, c.pa);
     TL_CHECK_LAUNCH("gemm_ring");
     return TL_OK;
 }
@@ -1297,9 +1387,11 @@ static int launch_ring_x(const RingCall& c, RingPlan p, hipStream_t stream) {
     case 6: return launch_ring_t<6, XH, TOut, SW, END, T>(c, p.rows, stream);
     case 8: return launch_ring_t<8, XH, TOut, SW, END, T>(c, p.rows, stream);
     }
-    if constexpr (!SW) {
-        if (p.wj == 1) return launch_ring_t<1, XH, TOut, SW, END, T>(c, p.rows, stream);
+    if constexpr (!SW || sizeof(T) == 4) {
         if (p.wj == 3) return launch_ring_t<3, XH, TOut, SW, END, T>(c, p.rows, stream);
+    }
+    if constexpr (!SW && !(END == END_ROTATE && sizeof(T) == 4)) {
+        if (p.wj == 1) return launch_ring_t<1, XH, TOut, SW, END, T>(c, p.rows, stream);
     }
     TL_REQUIRE(false, "gemm_ring: no shape of %d requests", p.wj);
 }
@@ -1307,7 +1399,8 @@ static int launch_ring_x(const RingCall& c, RingPlan p, hipStream_t stream) {
 // `p.wj` 0: the plan is made here.
 template <typename TOut, int SW, int END, typename T = bf16_t>
 static int launch_ring(const RingCall& c, hipStream_t stream, RingPlan p = RingPlan{0, 0}) {
-    if (p.wj == 0) p = plan_ring(SW ? c.out_cols : c.N, c.M, SW ? 2 : 1, TL_COMPUTE_UNITS / (c.parts * c.gr.count), END == END_ROTATE, ring_spread<T>(c.K), c.parts > 1);
+    constexpr bool pairs = sizeof(T) == 4 && (SW || END == END_ROTATE);
+    if (p.wj == 0) p = plan_ring(SW || pairs ? c.out_cols : c.N, c.M, SW || pairs ? 2 : 1, TL_COMPUTE_UNITS / (c.parts * c.gr.count), END == END_ROTATE && !pairs, ring_spread<T>(c.K), c.parts > 1, pairs);
     if (c.M <= 8) return launch_ring_x<1, TOut, SW, END, T>(c, p, stream);
     if (c.M <= 16) return launch_ring_x<2, TOut, SW, END, T>(c, p, stream);
     if constexpr (END == END_STORE && sizeof(T) == 2) {
@@ -2111,6 +2204,46 @@ extern "C" int tl_gemm_swiglu(const void* x, const void* w, void* out, int M, in
     TL_REQUIRE(act >= 0 && act <= 2, "gemm_swiglu: unknown gate %d", act);
     if (act == 2) return gemm_gated<3>(x, w, out, M, I, K, ldx, ldo, stream);
     return act == 1 ? gemm_gated<2>(x, w, out, M, I, K, ldx, ldo, stream) : gemm_gated<1>(x, w, out, M, I, K, ldx, ldo, stream);
+}
+
+// A 32-bit product of up to 16 rows whose matrix's rows a gate or a rotation joins by pairs (through the rings, 4 rows, us, two launches / one: gate and up of 2 x 18944 x 3584 94 + 5 / 93,
+// query, key and value 4608 x 3584 14.9 + 4.5 / 18.4): the rings where they are taken (offsets to a pair's second row in 32 bits), the multiply-add kernel up
+// to 8 rows.  Returns TL_NOT_FUSED (nothing launched) for the rest.
+template <int END>
+static int f32_pairs(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int K, int ldx, int ldo, const F32Pairs& pa, hipStream_t stream) {
+    const int N = 2 * pa.count;
+    if (M > 16 || !gemv_f32_fits(x, w, M, K, ldx)) return TL_NOT_FUSED;
+    if (ring_fits_f32(x, w, M, K, ldx) && ring_pays_f32(M, N, K) && ((size_t)pa.span + 256) * K * 4 < ((size_t)1 << 32)) {
+        RingCall c{x, w, bias, bias_f32, out, M, N, K, ldx, ldo, pa.count};
+        c.pa = pa;
+        return launch_ring<float, END == F32_GATE ? 1 : 0, END == F32_GATE ? END_STORE : END_ROTATE, float>(c, stream);
+    }
+    if (M > 8) return TL_NOT_FUSED;
+    launch_gemv_f32_fma<END>(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, pa, stream);
+    TL_CHECK_LAUNCH("gemv_f32");
+    return TL_OK;
+}
+
+// out[m, i] = act((x w^T)[m, i]) * (x w^T)[m, I + i] in 32 bits: w holds the gate's I rows, then the up rows.
+extern "C" int tl_gemm_gate_f32(const void* x, const void* w, void* out, int M, int I, int K, int ldx, int ldo, int act, hipStream_t stream) {
+    TL_REQUIRE(M > 0 && I > 0 && I < (1 << 30) && K > 0 && ldx >= K && ldo >= I && act >= 0 && act <= 2, "gemm_gate_f32: bad sizes M=%d I=%d K=%d or an unknown gate %d", M, I, K, act);
+    F32Pairs pa{};
+    pa.count = pa.span = I;
+    pa.act = act;
+    return f32_pairs<F32_GATE>(x, w, nullptr, 0, out, M, K, ldx, ldo, pa, stream);
+}
+
+// tl_gemm_rope in 32 bits: the rows of the heads as they are, frequency j turning the elements j and j + head_dim / 2.
+extern "C" int tl_gemm_rope_f32(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int N, int K, int ldx, int ldo, const void* positions, const void* inv_freq,
+                                const void* token_req, const void* block_table, int bt_stride, void* k_plane, void* v_plane, int page, int q_heads, int kv_heads, int head_dim, hipStream_t stream) {
+    TL_REQUIRE(M > 0 && N > 0 && K > 0 && ldx >= K && ldo >= q_heads * head_dim, "gemm_rope_f32: bad sizes M=%d N=%d K=%d", M, N, K);
+    TL_REQUIRE(positions && inv_freq && head_dim > 0 && head_dim % 2 == 0 && q_heads >= 0 && kv_heads >= 0, "gemm_rope_f32: needs positions, frequencies and an even head size");
+    TL_REQUIRE((k_plane == nullptr) == (v_plane == nullptr) && (!k_plane || (token_req && block_table && page > 0 && bt_stride > 0 && kv_heads > 0)),
+               "gemm_rope_f32: the cache write needs both planes, the block table and the requests of the rows");
+    TL_REQUIRE(N == (q_heads + (k_plane ? 2 * kv_heads : 0)) * head_dim, "gemm_rope_f32: %d output columns do not match the heads", N);
+    const F32Pairs pa{N / 2, head_dim / 2, 0, (const int*)positions, (const float*)inv_freq, (const int*)token_req, (const int*)block_table, (float*)k_plane, (float*)v_plane,
+                      bt_stride, page > 0 ? page : 1, q_heads, k_plane ? kv_heads : 0};
+    return f32_pairs<F32_ROTATE>(x, w, bias, bias_f32, out, M, K, ldx, ldo, pa, stream);
 }
 
 // out[P, M, N] (float) = partial sums of x w^T over P ranges of K, for a product with too few output

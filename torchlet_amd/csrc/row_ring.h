@@ -31,7 +31,7 @@ struct RingShape {
     static constexpr int STRIPS = HALVES * SH, MT = (XH + 1) / 2;          // blocks of 16 weight rows and of 16 rows of x
     static constexpr int SETS = XH <= 2 ? 8 / NW : 1;                           // sets of sums a wave keeps: see ring_products
     static constexpr size_t LDS = (size_t)NW * D * SLOT;
-    static_assert(WJ % HALVES == 0 && (HALVES - 1) * HR + 16 * SH <= 8 * (WJ + XH), "a block that is not full reads on in its own slab");
+    static_assert(8 * WJ % HALVES == 0 && (HALVES - 1) * HR + 16 * SH <= 8 * (WJ + XH), "a block that is not full reads on in its own slab");
     static_assert(SETS * STRIPS * MT * 1024 <= D * SLOT, "a wave's sums fit its own ring");
     static_assert((WJ + XH) * (D - 1) < 64 && LDS <= 160 * 1024, "requests on their way fit the counter, rings the shared memory");
 };
@@ -186,7 +186,8 @@ struct RingPlan {
 // Not where K is split over work-groups (8 rows, one of eight / two of four, each 56 to 64 outputs of one range of K: 4096 x 4096 8.2 / 9.4, 3584 x 18944 25.3 / 26.6, 3072 x 8192 11.4 / 12.0,
 // 5120 x 13824 28.0 / 28.2, 3584 x 3584 7.1 / 7.0).
 // `spread` (see ring_products): up to 16 rows the same plan, that of 16.
-static RingPlan plan_ring(int total, int M, int halves, int units, bool even, bool spread, bool split) {
+// `pairs`: the float kernel's pairs of rows, which are built for three requests as well (4608 x 3584, 4 rows, 9 pairs to a work-group: 20.9 us in shapes of four requests, 18.4 of three).
+static RingPlan plan_ring(int total, int M, int halves, int units, bool even, bool spread, bool split, bool pairs = false) {
     const int xh = M <= 8 && !spread ? 1 : M <= 16 ? 2 : M <= 32 ? 4 : 8, floor = 8 / halves;
     if (units < 1) units = 1;
     auto share = [&](long groups, long per) {
@@ -198,7 +199,7 @@ static RingPlan plan_ring(int total, int M, int halves, int units, bool even, bo
     double least = 1e30;
     long best_rounds = 0;
     for (int wj : {1, 2, 3, 4, 6, 8}) {
-        if (wj % halves) continue;
+        if (wj % halves && !(pairs && wj == 3)) continue;
         const long per = 8 * wj / halves, rounds = ((total + per - 1) / per + units - 1) / units;
         const double cost = rounds * (wj + 0.5 * xh + 0.3);
         if (cost >= least) continue;

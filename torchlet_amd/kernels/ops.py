@@ -566,6 +566,25 @@ def linear_swiglu(x: torch.Tensor, gate_up: torch.Tensor, out: torch.Tensor, act
                                    c_int(x.stride(0)), c_int(out.stride(0)), c_int(GATE_ACTIVATIONS[activation]), _stream()))
 
 
+def linear_gate_stacked(x: torch.Tensor, gate_up: torch.Tensor, out: torch.Tensor, activation: str = "silu") -> bool:
+    """``out = act(x @ gate.T) * (x @ up.T)`` in float32 with ``gate_up [2 I, K]`` the gate's rows and then the up rows, in one launch: :func:`linear`
+    and :func:`swiglu` for up to 16 rows.  ``False``, and nothing done, for what it is not built for."""
+    M, K = x.shape
+    I = out.shape[1]
+    if not (x.is_cuda and x.dtype == gate_up.dtype == out.dtype == torch.float32 and 0 < M <= 16):
+        return False
+    if gate_up.shape != (2 * I, K) or out.shape[0] != M or not gate_up.is_contiguous() or x.stride(1) != 1 or out.stride(1) != 1:
+        raise KernelError(f"linear_gate_stacked: shapes x{tuple(x.shape)} w{tuple(gate_up.shape)} out{tuple(out.shape)} do not fit")
+    if activation not in GATE_ACTIVATIONS:
+        raise KernelError(f"linear_gate_stacked: the gate's activation is one of {', '.join(GATE_ACTIVATIONS)}, not {activation!r}")
+    lib = _lib("gemm")
+    rc = lib.tl_gemm_gate_f32(_ptr(x), _ptr(gate_up), _ptr(out), c_int(M), c_int(I), c_int(K), c_int(x.stride(0)), c_int(out.stride(0)), c_int(GATE_ACTIVATIONS[activation]), _stream())
+    if rc == 100:          # not built for this shape
+        return False
+    _check(lib, rc)
+    return True
+
+
 def linear_swiglu_direct_variant(x: torch.Tensor, gate_up: torch.Tensor, out: torch.Tensor, tile_m: int, tile_n: int) -> None:
     """:func:`linear_swiglu` on one named tile shape of the kernel that fetches its operands straight into shared
     memory (K a multiple of 64; for tests and tuning)."""
@@ -636,15 +655,17 @@ def linear_rope_cache_write(x: torch.Tensor, weight: torch.Tensor, bias: torch.T
                             q_heads: int, kv_heads: int, head_dim: int, positions: torch.Tensor, inv_freq: torch.Tensor,
                             token_req: torch.Tensor | None = None, block_table: torch.Tensor | None = None,
                             k_plane: torch.Tensor | None = None, v_plane: torch.Tensor | None = None,
-                            page_size: int = 0) -> bool:
+                            page_size: int = 0, pairs: bool = True) -> bool:
     """The query/key/value projection of a decode step with the rotation and the cache write in
     its epilogue: ``out[:, :q_heads*hd]`` gets the rotated queries; with planes given, ``weight``
     has ``(q_heads + 2 kv_heads) * hd`` rows and rotated keys and values go to their pages.  The
     rows of the query and key heads are in the pair layout (:func:`pair_layout_rows`).  Built
-    for bfloat16 and up to 16 rows; returns ``False`` without doing anything for other shapes."""
+    for bfloat16 and up to 16 rows; returns ``False`` without doing anything for other shapes.
+    ``pairs=False``: the same in float32, the heads' rows as they are (frequency ``j`` turns the elements ``j`` and ``j + head_dim / 2``)."""
     M, K = x.shape
     N = weight.shape[0]
-    if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or out.dtype != torch.bfloat16 or M > 16 or M == 0 or head_dim % 4:
+    dtype = torch.bfloat16 if pairs else torch.float32
+    if x.dtype != dtype or weight.dtype != dtype or out.dtype != dtype or M > 16 or M == 0 or head_dim % (4 if pairs else 2) or not (pairs or x.is_cuda):
         return False
     if x.stride(1) != 1 or out.stride(1) != 1 or not weight.is_contiguous() or weight.shape[1] != K or out.shape[0] != M:
         raise KernelError("linear_rope_cache_write: shapes or strides do not fit")
@@ -661,10 +682,11 @@ def linear_rope_cache_write(x: torch.Tensor, weight: torch.Tensor, bias: torch.T
         raise KernelError("linear_rope_cache_write: the projection's rows do not match the heads")
     bf = _vec(bias, N, "linear bias")
     lib = _lib("gemm")
-    rc = lib.tl_gemm_rope(_ptr(x), _ptr(weight), _ptr(bias), c_int(bf), _ptr(out), c_int(M), c_int(N), c_int(K),
-                          c_int(x.stride(0)), c_int(out.stride(0)), _ptr(positions), _ptr(inv_freq), _ptr(token_req),
-                          _ptr(block_table), c_int(bt_stride), _ptr(k_plane), _ptr(v_plane), c_int(page_size),
-                          c_int(q_heads), c_int(kv_heads), c_int(head_dim), _stream())
+    entry = lib.tl_gemm_rope if pairs else lib.tl_gemm_rope_f32
+    rc = entry(_ptr(x), _ptr(weight), _ptr(bias), c_int(bf), _ptr(out), c_int(M), c_int(N), c_int(K),
+               c_int(x.stride(0)), c_int(out.stride(0)), _ptr(positions), _ptr(inv_freq), _ptr(token_req),
+               _ptr(block_table), c_int(bt_stride), _ptr(k_plane), _ptr(v_plane), c_int(page_size),
+               c_int(q_heads), c_int(kv_heads), c_int(head_dim), _stream())
     if rc == 100:          # not built for this shape
         return False
     _check(lib, rc)

@@ -203,6 +203,8 @@ class GQAttention(Mixer):
         fused = fused or (self.pair_layout and not plain and
                           ops.linear_rope_cache_write(h, w, b, qkv, self.heads, self.kv_heads, self.head_dim,
                                                       ctx.positions, inv_freq, *cache_args))
+        if self.dtype == torch.float32 and inv_freq is not None and not plain:
+            fused = ops.linear_rope_cache_write(h, w, b, qkv, self.heads, self.kv_heads, self.head_dim, ctx.positions, inv_freq, *cache_args, pairs=False)
         if not fused and not plain and self.dtype == torch.bfloat16 and (inv_freq is not None or self.position is None) \
                 and ops.linear_partials_pay(T, width, self.hidden):
             # few rows against a narrow matrix: K split over work-groups; the rotation kernel adds the slabs up

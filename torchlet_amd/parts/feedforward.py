@@ -6,7 +6,8 @@ three matrices' names come from the specification.
 product reads ``h`` once.  In bfloat16 (hidden a multiple of 8) the two are interleaved in
 blocks of 32 rows and the gate ``silu(g) * u`` is applied to the 32-bit accumulators inside
 the product's kernel, as the reference's fused kernel does (kernel/ffn_swiglu.py:139-160);
-otherwise they are stacked ``[gate; up]`` and a separate kernel applies the gate.
+otherwise they are stacked ``[gate; up]``, and a separate kernel applies the gate (in 32 bits,
+up to 16 rows, the product's own).
 """
 from __future__ import annotations
 
@@ -74,7 +75,7 @@ class SwiGLU(FeedForward):
         z = torch.empty((T, self.inter), dtype=self.dtype, device=h.device)
         if self.fused_gate:
             ops.linear_swiglu(h, self.gate_up, z, self.act)
-        else:
+        elif self.dtype != torch.float32 or not ops.linear_gate_stacked(h, self.gate_up, z, self.act):
             gu = torch.empty((T, 2 * self.inter), dtype=self.dtype, device=h.device)
             ops.linear(h, self.gate_up, None, gu)
             ops.swiglu(gu, z, self.act)
