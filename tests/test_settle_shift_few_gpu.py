@@ -30,3 +30,26 @@ def test_sum_and_mixes(lens, hidden, off, count, slabs):
             before[starts[r]] = state[R - r, off: off + hidden].double()
         torch.testing.assert_close(got.double(), x, rtol=1e-5, atol=1e-5)
         torch.testing.assert_close(mixes.double(), x + (before - x) * mu.double()[:, None], rtol=2 ** -8, atol=2e-5)      # (one rounding to bfloat16)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("hidden", [4, 1028, 2048, 2050, 4096])
+@pytest.mark.parametrize("slabs", [None, 0, 1, 2, 3, 4, 6, 8])
+def test_a_tokens_sum_and_mixes_do_not_hang_on_the_steps_size(dtype, hidden, slabs):
+    """The same tokens in steps of 40, of 256 and, on another kernel, of 257: the same bits."""
+    g = torch.Generator(device="cuda").manual_seed(hidden + 1)
+    rand = lambda *shape: torch.randn(*shape, generator=g, device="cuda")
+    T, own = 257, 40
+    res, w, mu, state = rand(T, hidden), rand(hidden), torch.rand(5, hidden, generator=g, device="cuda"), rand(3, hidden)
+    branch = None if slabs is None else rand(T, hidden).to(dtype) if slabs == 0 else rand(slabs, T, hidden)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    for post in (w, None):
+        seen = {}
+        for n in (own, 256, T):
+            lens = [own - 1, n - own + 1]
+            part = None if branch is None else branch[:n] if slabs == 0 else branch[:, :n].contiguous()
+            mixes = torch.full((5, n, hidden), float("nan"), dtype=dtype, device="cuda")
+            got = ops.settle_shift(res[:n].clone(), part, post, 1e-6, state, 0, i32([2, 1]), i32([0, lens[0], n]), i32([0] * lens[0] + [1] * lens[1]), mu, mixes)
+            seen[n] = got[:own].clone(), mixes[:, :own].clone()
+        for n in (own, 256):
+            assert torch.equal(seen[n][0], seen[T][0]) and torch.equal(seen[n][1], seen[T][1]), n

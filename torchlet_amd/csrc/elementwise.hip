@@ -1607,6 +1607,14 @@ struct ShiftArgs {
     int count, tokens, hidden, run;
 };
 
+// r + y * inv * w in three roundings of their own, so that a row's bits do not hang on which of the kernels below has the step (left to the compiler, one of them multiplied and added apart
+// and another in one rounding).
+__device__ __forceinline__ float plus_normed(float r, float y, float inv, float w) {
+#pragma clang fp contract(off)
+    const float normed = y * inv * w;
+    return r + normed;
+}
+
 template <typename T, int NP>
 __global__ void __launch_bounds__(1024)
 settle_shift_rows_kernel(ShiftArgs a, T* __restrict__ mixes) {
@@ -1624,7 +1632,7 @@ settle_shift_rows_kernel(ShiftArgs a, T* __restrict__ mixes) {
 #pragma unroll
         for (int n = 0; n < NP; ++n)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) r.v[n][v] += a.post ? y.v[n][v] * inv * pw.v[n][v] : y.v[n][v];
+            for (int v = 0; v < 4; ++v) r.v[n][v] = a.post ? plus_normed(r.v[n][v], y.v[n][v], inv, pw.v[n][v]) : r.v[n][v] + y.v[n][v];
     };
     RowPieces<NP> before, x;
     bool have = false;                                 // `before` holds the row ahead of the one at hand
@@ -1694,7 +1702,9 @@ settle_shift_few_kernel(ShiftArgs a, int tail4, T* __restrict__ mixes) {
 #pragma unroll
                 for (int v = 0; v < 4; ++v) sq.v[0][v] = in ? y[v] : 0.f;
                 const float inv = rsqrtf(block_sum(row_squares(sq), red) / (float)hidden + a.post_eps);
-                x[0] += y[0] * inv * pw.x; x[1] += y[1] * inv * pw.y; x[2] += y[2] * inv * pw.z; x[3] += y[3] * inv * pw.w;
+                const float w4[4] = {pw.x, pw.y, pw.z, pw.w};
+#pragma unroll
+                for (int v = 0; v < 4; ++v) x[v] = plus_normed(x[v], y[v], inv, w4[v]);
             } else {
 #pragma unroll
                 for (int v = 0; v < 4; ++v) x[v] += y[v];
@@ -1739,7 +1749,7 @@ settle_shift_kernel(ShiftArgs a, T* __restrict__ mixes) {
         }
         for (int i = threadIdx.x; i < hidden; i += blockDim.x) {
             float r = a.residual[at + i];
-            if (a.pending) r += a.post ? buf[i] * inv * a.post[a.post_n == 1 ? 0 : i] : buf[i];
+            if (a.pending) r = a.post ? plus_normed(r, buf[i], inv, a.post[a.post_n == 1 ? 0 : i]) : r + buf[i];
             buf[i] = r;
         }
     };
