@@ -1421,6 +1421,16 @@ def wkv_scan(rkv: torch.Tensor, k_off: int, v_off: int, decay: torch.Tensor, bon
                                 ctypes.c_long(tail_off), c_int(_dt(rkv, "wkv_scan")), _stream()))
 
 
+def wkv_token_pays(requests: int, heads: int, dim: int, vdim: int, rank: int) -> bool:
+    """Whether a step of one token a request is faster through :func:`wkv_token` than through the three launches it stands for (which leave the same bits).  A work-group
+    has a whole head, and a compute unit has two of them at once (one where both sizes are above 64): beyond that they queue, where the three launches deal a head to several.  Wide columns
+    want half the units busy, and only the first 64 rows of the decays' matrix are requested ahead.  Measured (us, three launches / one): 32 heads of 64 x 64 and rank 64, 1 request 8.3 /
+    7.8, 16 12.4 / 9.7, 32 17.4 / 17.6, 64 25.9 / 34.5; 20 requests 13.0 / 15.1; 16 heads of 128 x 128, 1 request 8.9 / 9.8, 4 9.8 / 10.2, 8 11.7 / 10.7, 16 16.1 / 11.6, 20 17.8 / 20.4;
+    32 of 64 x 128, 2 requests 8.8 / 9.3, 4 9.8 / 9.6, 16 16.3 / 12.2; rank 80, 4 requests of 32 heads 9.0 / 9.7; rank 128, 1 request 9.3 / 13.8, 16 13.6 / 15.4."""
+    groups, units = requests * heads, compute_units()
+    return rank <= 64 and groups <= (units if min(dim, vdim) > 64 else 2 * units) and (vdim <= 64 or groups >= units // 2)
+
+
 def wkv_token(proj: torch.Tensor, k_off: int, v_off: int, gate_off: int, z: torch.Tensor, w2t: torch.Tensor, w0: torch.Tensor, bonus: torch.Tensor, state: torch.Tensor,
               slots: torch.Tensor, req_indptr: torch.Tensor, norm: torch.Tensor, eps: float, out: torch.Tensor, heads: int, dim: int, vdim: int, last_rows: torch.Tensor,
               tail_off: int) -> bool:

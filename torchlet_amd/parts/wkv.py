@@ -106,8 +106,9 @@ class WKV(Mixer):
             ops.linear_groups(mixes[:2], self.w_rk, proj[:, : 2 * K])
             ops.linear_groups_beside(mixes[2:4], self.w_vg, proj[:, 2 * K:], mixes[4], self.w1, z)
         mixed = torch.empty((T, V), dtype=self.dtype, device=dev)
-        if not (ctx.max_new_tokens == 1 and ops.wkv_token(proj, K, 2 * K, 2 * K + V, z, self.w2t, self.w0, self.bonus, cache.state, ctx.slots, ctx.req_indptr, self.w_norm,
-                                                          float(self.spec.norm_eps), mixed, self.heads, self.dim, self.vdim, x, self.state_floats)):
+        if not (ctx.max_new_tokens == 1 and ops.wkv_token_pays(ctx.req_indptr.numel() - 1, self.heads, self.dim, self.vdim, z.shape[1]) and
+                ops.wkv_token(proj, K, 2 * K, 2 * K + V, z, self.w2t, self.w0, self.bonus, cache.state, ctx.slots, ctx.req_indptr, self.w_norm, float(self.spec.norm_eps), mixed, self.heads,
+                              self.dim, self.vdim, x, self.state_floats)):
             decay = torch.empty((T, K), dtype=torch.float32, device=dev)
             ops.channel_decay(z, self.w2t, self.w0, decay)
             o = torch.empty((T, V), dtype=torch.float32, device=dev)
