@@ -1,5 +1,6 @@
 """Each HIP kernel alone against a plain float64/float32 torch formula of the same
 operation, at sizes other than the tiny engines' (odd widths, many heads, long rows)."""
+import itertools
 import math
 
 import pytest
@@ -196,9 +197,9 @@ def test_linear_many_rows_in_32_bit_on_matrix_cores(ops, M, N, K, bias):
 
 
 @pytest.mark.parametrize("M", [1, 2, 3, 7, 8, 13, 16])
-@pytest.mark.parametrize("N,K", [(37, 100), (300, 1024), (129, 1028), (4608, 3584), (1, 2052), (64, 18944)])
+@pytest.mark.parametrize("N,K", [(37, 100), (300, 1024), (129, 1028), (4608, 3584), (1, 2052), (64, 18944), (4100, 1028), (4608, 3588)])
 def test_linear_few_rows_in_32_bit(ops, M, N, K):
-    """The weight-streaming kernel of the 32-bit decode step: every count of rows, an odd number
+    """The weight-streaming kernels of the 32-bit decode step: every count of rows, an odd number
     of weight rows, K of less than one, exactly one and several chunks with a tail; against a
     float64 product, and a row's result is the same whatever other rows stand beside it."""
     g = torch.Generator().manual_seed(M * 11 + N)
@@ -210,17 +211,26 @@ def test_linear_few_rows_in_32_bit(ops, M, N, K):
     out = torch.full((M, N), float("nan"), device="cuda")
     ops.linear(x, w, b, out)
     torch.testing.assert_close(out.double(), ref, **tol32)
-    # two kernels serve these row counts (multiply-adds up to 8 rows, the matrix cores' true 32-bit instruction from 9
-    # on): each agrees with float64, and in each a row's sum runs in one order whatever stands beside it (bitwise)
-    for variant in (2, 3):
+    # three kernels serve these row counts (multiply-adds up to 8 rows, the matrix cores' true 32-bit instruction behind a
+    # copy of x up to 16, and through rings of slabs where K is a multiple of 32): each agrees with float64, and in each a
+    # row's sum runs in one order whatever stands beside it (bitwise).  They are different kernels: another order of the sums
+    named = {}
+    for variant in (2, 3, 9):
         got = torch.full((M, N), float("nan"), device="cuda")
+        if (variant == 2 and M > 8) or (variant == 9 and K % 32):
+            with pytest.raises(ops.KernelError, match="need M"):
+                ops.linear_f32_variant(x, w, b, got, variant)
+            continue
         ops.linear_f32_variant(x, w, b, got, variant)
         torch.testing.assert_close(got.double(), ref, **tol32)
         alone = torch.empty(1, N, device="cuda")
         ops.linear_f32_variant(x[M - 1:], w, b, alone, variant)
         assert torch.equal(alone[0], got[M - 1]), f"variant {variant}"
-        if variant == (3 if M > 8 else 2):
-            assert torch.equal(got, out)                   # the dispatch's choice
+        named[variant] = got
+    assert torch.equal(named[ops._lib("gemm").tl_gemm_f32_few_rows_choice(M, N, K)], out)                   # the dispatch's choice
+    if N * K > 1 << 18:
+        for a, c in itertools.combinations(named.values(), 2):
+            assert not torch.equal(a, c)
     wide = torch.zeros(M, K + 24, device="cuda")          # a strided input view, a wider output
     wide[:, 8:8 + K] = x
     out2 = torch.full((M, N + 5), 3.0, device="cuda")

@@ -252,7 +252,7 @@ __global__ __launch_bounds__(256) void gemv_f32_kernel(const float* __restrict__
 
 // The same on the matrix cores, 2 to 16 rows: v_mfma_f32_16x16x4_f32 multiplies and adds in true 32-bit (as
 // v_mfma_f32_32x32x2_f32 below), and a step of several rows costs the stream of weights and little else, where the
-// kernel above spends a multiply-add per row and weight (the dispatch takes this kernel from 9 rows on).  A work-group of eight waves owns 16 weight rows; chunks of GM_KC columns of x wait in shared
+// kernel above spends a multiply-add per row and weight (the dispatch takes this kernel from 9 rows on where K is no multiple of 32, which the rings want).  A work-group of eight waves owns 16 weight rows; chunks of GM_KC columns of x wait in shared
 // memory (rows beyond M as zeros); within a chunk the waves take its pieces of 16 columns in turn.  A lane fetches
 // four neighbouring k of its weight row and of its x row at once: lane group g = lane / 16 takes k = 4 g .. 4 g + 3
 // of the piece, so instruction e of a piece multiplies k = 4 g + e of the four groups: which k meet in one instruction
@@ -329,29 +329,18 @@ static bool gemv_f32_fits(const void* x, const void* w, int M, int K, int ldx) {
 }
 
 template <int END>
-static void launch_gemv_f32_fma(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int N, int K, int ldx, int ldo, const F32Pairs& pa, hipStream_t stream) {
+static void launch_gemv_f32_fma(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int N, int K, int ldx, int ldo, const F32Pairs& pa, hipStream_t stream) {      // up to 8 rows
     dim3 grid((N + GV_ROWS - 1) / GV_ROWS), block(256);
 #define GV_LAUNCH(MR) gemv_f32_kernel<MR, END><<<grid, block, 0, stream>>>((const float*)x, (const float*)w, bias, bias_f32, (float*)out, M, N, K, ldx, ldo, pa)
     if (M <= 1) GV_LAUNCH(1);
     else if (M <= 2) GV_LAUNCH(2);
     else if (M <= 4) GV_LAUNCH(4);
-    else if (M <= 8) GV_LAUNCH(8);
-    else if constexpr (END == F32_PLAIN) GV_LAUNCH(16);
+    else GV_LAUNCH(8);
 #undef GV_LAUNCH
 }
 
-// mfma: 0 the multiply-add kernel, 1 the matrix-core kernel, -1 the one that is faster for M.  Measured on the four
-// products of a 7B layer (us, multiply-adds / matrix cores): 1 row 174 / 237, 4 rows 216 / 241, 8 rows 274 / 265,
-// 16 rows 425 / 300: the matrix-core kernel's time hardly grows with the rows, but its work-groups of 16 weight rows
-// are too few on the narrow matrices (224 for 3584 rows) to stream as fast as the other's 448 of 8.
-static void launch_gemv_f32(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int N, int K,
-                            int ldx, int ldo, hipStream_t stream, int mfma = -1) {
-    if (mfma == 1 || (mfma < 0 && M > 8)) {
-        gemv_f32_mfma_kernel<<<dim3((N + 15) / 16), dim3(GM_WAVES * 64), 0, stream>>>((const float*)x, (const float*)w, bias, bias_f32,
-                                                                                     (float*)out, M, N, K, ldx, ldo);
-        return;
-    }
-    launch_gemv_f32_fma<F32_PLAIN>(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, F32Pairs{}, stream);
+static void launch_gemv_f32_mfma(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int N, int K, int ldx, int ldo, hipStream_t stream) {
+    gemv_f32_mfma_kernel<<<dim3((N + 15) / 16), dim3(GM_WAVES * 64), 0, stream>>>((const float*)x, (const float*)w, bias, bias_f32, (float*)out, M, N, K, ldx, ldo);
 }
 
 // =====================================================================================
@@ -1330,6 +1319,10 @@ static bool ring_fits_f32(const void* x, const void* w, int M, int K, int ldx) {
 // these have (4 rows, 256 x 2048 5.2 / 5.5, 64 x 4096 7.5 / 8.3).  The sums' error against 64 bits (relative): K 2048 1.2e-7 / 1.0e-7, 3584 1.5e-7 / 1.1e-7, 18944 3.1e-7 / 1.8e-7, above 8 rows
 // 3.8e-7 / 1.1e-7; at 512 columns up to 8 rows 0.87e-7 / 0.9e-7, and so short sums stay where they are.
 static bool ring_pays_f32(int M, int N, int K) { return M > 8 || (K >= 1024 && N >= 1024); }
+// Which kernel a 32-bit product of up to 16 rows gets whose operands are aligned, by its number in tl_gemm_f32_variant: 9 the rings, 2 multiply-adds, 3 the matrix cores behind a copy of x.  The
+// last two part at 8 rows, where a row more costs a multiply-add a weight or nothing (the four products of a 7B layer, us, 2 / 3: 4 rows 216 / 241, 8 rows 274 / 265, 16 rows 425 / 300).
+static int f32_few_rows_kernel(int M, int N, int K) { return K % 32 == 0 && ring_pays_f32(M, N, K) ? 9 : M <= 8 ? 2 : 3; }
+extern "C" int tl_gemm_f32_few_rows_choice(int M, int N, int K) { return f32_few_rows_kernel(M, N, K); }
 
 // Where a product of up to 64 rows goes through the rings, K a multiple of 64: measured against what it took before them, the tiles or the few-rows kernel that fetches into registers, over a grid
 // of widths and depths (us, the other / this).
@@ -1442,20 +1435,21 @@ extern "C" int tl_gemm_ring_variant(const void* x, const void* w, const void* bi
     return out_f32 ? launch_ring<float, 0, END_STORE>(c, stream, p) : launch_ring<bf16_t, 0, END_STORE>(c, stream, p);
 }
 
-// One named kernel of the 32-bit products (for tests and tuning): 0 the general tile kernel (v_fma_f32), 1 the matrix-core
-// tile kernel, 2 and 3 the kernels for up to 16 rows on multiply-adds and on the matrix cores, 4 to 6 the matrix-core tile kernel with tiles of 64 x 64, 64 x 128, 128 x 128,
-// 7 and 8 with 64 x 32 and 32 x 32; 9 the rings, which are what 2 (sizes that ring_pays_f32 gives them) and 3 (any) stand for where they fit, as in the dispatch.
+// One named kernel of the 32-bit products (for tests and tuning), or an error where it is not built for the sizes: 0 the general tile kernel (v_fma_f32), 1 the matrix-core
+// tile kernel, 2 and 3 the kernels for few rows on multiply-adds (up to 8) and on the matrix cores (up to 16), 4 to 6 the matrix-core tile kernel with tiles of 64 x 64, 64 x 128, 128 x 128,
+// 7 and 8 with 64 x 32 and 32 x 32, 9 the rings.
 extern "C" int tl_gemm_f32_variant(const void* x, const void* w, const void* bias, int bias_f32, void* out,
                                    int M, int N, int K, int ldx, int ldo, int matrix_cores, hipStream_t stream) {
     TL_REQUIRE(M > 0 && N > 0 && K > 0 && ldx >= K && ldo >= N, "gemm_f32: bad sizes M=%d N=%d K=%d ldx=%d ldo=%d", M, N, K, ldx, ldo);
-    const bool rings = ring_fits_f32(x, w, M, K, ldx);
-    if (matrix_cores == 9 || (rings && (matrix_cores == 3 || (matrix_cores == 2 && ring_pays_f32(8, N, K))))) {
-        TL_REQUIRE(rings, "gemm_f32: the rings need M <= 16, K %% 32 == 0 and 16-byte aligned rows");
+    TL_REQUIRE(matrix_cores >= 0 && matrix_cores <= 9, "gemm_f32: no kernel %d", matrix_cores);
+    if (matrix_cores == 9) {
+        TL_REQUIRE(ring_fits_f32(x, w, M, K, ldx), "gemm_f32: the rings need M <= 16, K %% 32 == 0 and 16-byte aligned rows");
         return launch_ring<float, 0, END_STORE, float>(RingCall{x, w, bias, bias_f32, out, M, N, K, ldx, ldo, 0}, stream);
     }
-    if (matrix_cores == 2 || matrix_cores == 3) {      // the two kernels for up to 16 rows: 2 multiply-adds, 3 matrix cores
-        TL_REQUIRE(gemv_f32_fits(x, w, M, K, ldx), "gemm_f32: the few-rows kernels need M <= 16, K %% 4 == 0 and 16-byte aligned rows");
-        launch_gemv_f32(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, stream, matrix_cores - 2);
+    if (matrix_cores == 2 || matrix_cores == 3) {
+        TL_REQUIRE(gemv_f32_fits(x, w, M, K, ldx) && (matrix_cores == 3 || M <= 8), "gemm_f32: the few-rows kernels need M <= 8 or 16, K %% 4 == 0 and 16-byte aligned rows");
+        if (matrix_cores == 2) launch_gemv_f32_fma<F32_PLAIN>(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, F32Pairs{}, stream);
+        else launch_gemv_f32_mfma(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, stream);
     } else if (matrix_cores) {
         TL_REQUIRE(gemm_f32_mfma_fits(x, w, 17, K, ldx), "gemm_f32: the matrix-core kernel needs K %% 4 == 0 and 16-byte aligned rows");
         launch_gemm_f32_mfma(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, stream, matrix_cores > 3 ? matrix_cores - 3 : 0);
@@ -1954,8 +1948,8 @@ static bool skinny_fits(const void* x, const void* w, int M, int K, int ldx) {
 //     everything else             -> gemm_dl_tile (matrix cores, operands straight into shared memory)
 //   bfloat16, aligned, other K, M <= 64 -> gemm_skinny, except that 33..64 rows against a wide matrix go to the tile kernel
 //   bfloat16, aligned, other K, M > 64  -> gemm_mfma_tile (matrix cores, shared-memory tiles)
-//   32-bit, aligned, K a multiple of 32, M <= 16 as ring_pays_f32 says -> gemm_ring (true 32-bit arithmetic on the matrix cores)
-//   32-bit, aligned, M <= 16    -> gemv_f32 (true 32-bit arithmetic, weight streaming)
+//   32-bit, aligned, K a multiple of 32, M <= 16 as f32_few_rows_kernel says -> gemm_ring (true 32-bit arithmetic on the matrix cores)
+//   32-bit, aligned, M <= 16    -> gemv_f32, above 8 rows gemv_f32_mfma (true 32-bit arithmetic, weight streaming)
 //   32-bit, aligned, M > 16     -> gemm_f32_mfma (true 32-bit arithmetic on the matrix cores)
 //   everything else             -> gemm_tile (true 32-bit arithmetic)
 extern "C" int tl_gemm(const void* x, const void* w, const void* bias, int bias_f32, void* out,
@@ -1993,12 +1987,13 @@ extern "C" int tl_gemm(const void* x, const void* w, const void* bias, int bias_
         TL_CHECK_LAUNCH("gemm_skinny");
         return TL_OK;
     }
-    if (dtype == TL_DT_F32 && ring_fits_f32(x, w, M, K, ldx) && ring_pays_f32(M, N, K)) {
+    if (dtype == TL_DT_F32 && ring_fits_f32(x, w, M, K, ldx) && f32_few_rows_kernel(M, N, K) == 9) {
         const RingCall c{x, w, bias, bias_f32, out, M, N, K, ldx, ldo, 0};
         return launch_ring<float, 0, END_STORE, float>(c, stream);
     }
     if (dtype == TL_DT_F32 && gemv_f32_fits(x, w, M, K, ldx)) {
-        launch_gemv_f32(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, stream);
+        if (M <= 8) launch_gemv_f32_fma<F32_PLAIN>(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, F32Pairs{}, stream);
+        else launch_gemv_f32_mfma(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, stream);
         TL_CHECK_LAUNCH("gemv_f32");
         return TL_OK;
     }
@@ -2213,7 +2208,7 @@ template <int END>
 static int f32_pairs(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int K, int ldx, int ldo, const F32Pairs& pa, hipStream_t stream) {
     const int N = 2 * pa.count;
     if (M > 16 || !gemv_f32_fits(x, w, M, K, ldx)) return TL_NOT_FUSED;
-    if (ring_fits_f32(x, w, M, K, ldx) && ring_pays_f32(M, N, K) && ((size_t)pa.span + 256) * K * 4 < ((size_t)1 << 32)) {
+    if (ring_fits_f32(x, w, M, K, ldx) && f32_few_rows_kernel(M, N, K) == 9 && ((size_t)pa.span + 256) * K * 4 < ((size_t)1 << 32)) {
         RingCall c{x, w, bias, bias_f32, out, M, N, K, ldx, ldo, pa.count};
         c.pa = pa;
         return launch_ring<float, END == F32_GATE ? 1 : 0, END == F32_GATE ? END_STORE : END_ROTATE, float>(c, stream);

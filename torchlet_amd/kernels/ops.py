@@ -444,10 +444,10 @@ def linear_groups_beside(x: torch.Tensor, weight: torch.Tensor, out: torch.Tenso
 
 def linear_f32_variant(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, out: torch.Tensor, matrix_cores) -> None:
     """One named kernel of the 32-bit products (for tests and tuning): 0 / False the general tile kernel (``v_fma_f32``),
-    1 / True the matrix-core tile kernel (``v_mfma_f32_32x32x2_f32``, K a multiple of 4), 2 and 3 the kernels for up to 16
-    rows on multiply-adds and on the matrix cores (``v_mfma_f32_16x16x4_f32``), 4 to 6 the matrix-core tile kernel with
+    1 / True the matrix-core tile kernel (``v_mfma_f32_32x32x2_f32``, K a multiple of 4), 2 and 3 the kernels for few rows
+    on multiply-adds (up to 8) and on the matrix cores (``v_mfma_f32_16x16x4_f32``, up to 16), 4 to 6 the matrix-core tile kernel with
     tiles of 64 x 64, 64 x 128 and 128 x 128, 7 and 8 with 64 x 32 and 32 x 32, 9 the rings of
-    slabs for up to 16 rows, which 2 and 3 take as well where the library does; all multiply and add in true 32-bit."""
+    slabs for up to 16 rows (K a multiple of 32); all multiply and add in true 32-bit."""
     M, K = x.shape
     N = weight.shape[0]
     if x.dtype != torch.float32 or weight.dtype != torch.float32 or out.dtype != torch.float32 or out.shape != (M, N) \
