@@ -30,6 +30,15 @@ def test_tiles_of_products_with_few_rows(lib, M, N, K, gated, ahead):
     assert (rows.value, columns.value) in ahead
 
 
+# 32 bits, 2: multiply-adds, 3: matrix cores behind a copy of x, 9: rings; one and two rows stay with the multiply-adds wherever the rings, which take as long for one row as for eight, are behind
+@pytest.mark.parametrize("M, N, K, want", [
+    (1, 1024, 1024, 2), (1, 2048, 2048, 2), (1, 32768, 1024, 2), (1, 22016, 4096, 2), (1, 8192, 6144, 2), (1, 1536, 8192, 2), (1, 2048, 3584, 2), (1, 2560, 3584, 9), (1, 4608, 3584, 9), (1, 4096, 8192, 9),
+    (1, 2048, 18944, 9), (2, 1024, 1024, 2), (2, 2048, 2048, 2), (2, 7168, 4096, 2), (2, 2560, 2560, 2), (2, 3584, 2560, 9), (2, 4608, 3584, 9), (2, 4608, 5120, 9), (2, 1024, 6848, 2),
+    (3, 1024, 1024, 9), (4, 2048, 2048, 9), (8, 1000, 2048, 2), (8, 2048, 992, 2), (8, 2048, 1028, 2), (9, 64, 96, 9), (16, 4100, 1028, 3)])
+def test_32_bit_products_of_few_rows_go_where_they_were_faster(lib, M, N, K, want):
+    assert lib.tl_gemm_f32_few_rows_choice(c_int(M), c_int(N), c_int(K)) == want
+
+
 # 0: rings of slabs, 1: the few-rows kernel that fetches into registers, 2: tiles; sizes on both sides of each line, measured 4 % and more apart
 @pytest.mark.parametrize("M, N, K, gated, want", [
     (1, 32768, 768, 0, 0), (1, 152064, 3584, 0, 1), (8, 152064, 3584, 0, 0), (9, 152064, 3584, 0, 2), (16, 32768, 64, 0, 0),
