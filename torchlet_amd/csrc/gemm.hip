@@ -1445,14 +1445,15 @@ extern "C" int tl_gemm_ring_variant(const void* x, const void* w, const void* bi
 
 // One named kernel of the 32-bit products (for tests and tuning), or an error where it is not built for the sizes: 0 the general tile kernel (v_fma_f32), 1 the matrix-core
 // tile kernel, 2 and 3 the kernels for few rows on multiply-adds (up to 8) and on the matrix cores (up to 16), 4 to 6 the matrix-core tile kernel with tiles of 64 x 64, 64 x 128, 128 x 128,
-// 7 and 8 with 64 x 32 and 32 x 32, 9 the rings.
+// 7 and 8 with 64 x 32 and 32 x 32, 9 the rings (wj > 0: in shapes of wj requests, `rows` outputs of them used).
 extern "C" int tl_gemm_f32_variant(const void* x, const void* w, const void* bias, int bias_f32, void* out,
-                                   int M, int N, int K, int ldx, int ldo, int matrix_cores, hipStream_t stream) {
+                                   int M, int N, int K, int ldx, int ldo, int matrix_cores, int wj, int rows, hipStream_t stream) {
     TL_REQUIRE(M > 0 && N > 0 && K > 0 && ldx >= K && ldo >= N, "gemm_f32: bad sizes M=%d N=%d K=%d ldx=%d ldo=%d", M, N, K, ldx, ldo);
     TL_REQUIRE(matrix_cores >= 0 && matrix_cores <= 9, "gemm_f32: no kernel %d", matrix_cores);
     if (matrix_cores == 9) {
         TL_REQUIRE(ring_fits_f32(x, w, M, K, ldx), "gemm_f32: the rings need M <= 16, K %% 32 == 0 and 16-byte aligned rows");
-        return launch_ring<float, 0, END_STORE, float>(RingCall{x, w, bias, bias_f32, out, M, N, K, ldx, ldo, 0}, stream);
+        TL_REQUIRE(wj <= 0 || (wj <= 8 && rows > 0 && rows <= 8 * wj), "gemm_f32: %d outputs do not fit %d requests", rows, wj);
+        return launch_ring<float, 0, END_STORE, float>(RingCall{x, w, bias, bias_f32, out, M, N, K, ldx, ldo, 0}, stream, RingPlan{max(wj, 0), rows});
     }
     if (matrix_cores == 2 || matrix_cores == 3) {
         TL_REQUIRE(gemv_f32_fits(x, w, M, K, ldx) && (matrix_cores == 3 || M <= 8), "gemm_f32: the few-rows kernels need M <= 8 or 16, K %% 4 == 0 and 16-byte aligned rows");
@@ -2211,15 +2212,17 @@ extern "C" int tl_gemm_swiglu(const void* x, const void* w, void* out, int M, in
 
 // A 32-bit product of up to 16 rows whose matrix's rows a gate or a rotation joins by pairs (through the rings, 4 rows, us, two launches / one: gate and up of 2 x 18944 x 3584 94 + 5 / 93,
 // query, key and value 4608 x 3584 14.9 + 4.5 / 18.4): the rings where they are taken (offsets to a pair's second row in 32 bits), the multiply-add kernel up
-// to 8 rows.  Returns TL_NOT_FUSED (nothing launched) for the rest.
+// to 8 rows.  Returns TL_NOT_FUSED (nothing launched) for the rest.  wj (for tests and tuning) > 0: the rings in shapes of wj requests, `rows` pairs of them used; < 0: the rings as they would be dealt.
 template <int END>
-static int f32_pairs(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int K, int ldx, int ldo, const F32Pairs& pa, hipStream_t stream) {
+static int f32_pairs(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int K, int ldx, int ldo, const F32Pairs& pa, int wj, int rows, hipStream_t stream) {
     const int N = 2 * pa.count;
     if (M > 16 || !gemv_f32_fits(x, w, M, K, ldx)) return TL_NOT_FUSED;
-    if (ring_fits_f32(x, w, M, K, ldx) && f32_few_rows_kernel(M, N, K) == 9 && ((size_t)pa.span + 256) * K * 4 < ((size_t)1 << 32)) {
+    const bool rings = ring_fits_f32(x, w, M, K, ldx) && ((size_t)pa.span + 256) * K * 4 < ((size_t)1 << 32);
+    if (wj) TL_REQUIRE(rings && (wj < 0 || (wj <= 8 && rows > 0 && rows <= 4 * wj)), "gemm_f32: %d pairs do not fit %d requests, or sizes that the rings are not built for", rows, wj);
+    if (wj || (rings && f32_few_rows_kernel(M, N, K) == 9)) {
         RingCall c{x, w, bias, bias_f32, out, M, N, K, ldx, ldo, pa.count};
         c.pa = pa;
-        return launch_ring<float, END == F32_GATE ? 1 : 0, END == F32_GATE ? END_STORE : END_ROTATE, float>(c, stream);
+        return launch_ring<float, END == F32_GATE ? 1 : 0, END == F32_GATE ? END_STORE : END_ROTATE, float>(c, stream, RingPlan{max(wj, 0), rows});
     }
     if (M > 8) return TL_NOT_FUSED;
     launch_gemv_f32_fma<END>(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, pa, stream);
@@ -2228,17 +2231,18 @@ static int f32_pairs(const void* x, const void* w, const void* bias, int bias_f3
 }
 
 // out[m, i] = act((x w^T)[m, i]) * (x w^T)[m, I + i] in 32 bits: w holds the gate's I rows, then the up rows.
-extern "C" int tl_gemm_gate_f32(const void* x, const void* w, void* out, int M, int I, int K, int ldx, int ldo, int act, hipStream_t stream) {
+extern "C" int tl_gemm_gate_f32(const void* x, const void* w, void* out, int M, int I, int K, int ldx, int ldo, int act, int wj, int rows, hipStream_t stream) {
     TL_REQUIRE(M > 0 && I > 0 && I < (1 << 30) && K > 0 && ldx >= K && ldo >= I && act >= 0 && act <= 2, "gemm_gate_f32: bad sizes M=%d I=%d K=%d or an unknown gate %d", M, I, K, act);
     F32Pairs pa{};
     pa.count = pa.span = I;
     pa.act = act;
-    return f32_pairs<F32_GATE>(x, w, nullptr, 0, out, M, K, ldx, ldo, pa, stream);
+    return f32_pairs<F32_GATE>(x, w, nullptr, 0, out, M, K, ldx, ldo, pa, wj, rows, stream);
 }
 
 // tl_gemm_rope in 32 bits: the rows of the heads as they are, frequency j turning the elements j and j + head_dim / 2.
 extern "C" int tl_gemm_rope_f32(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int N, int K, int ldx, int ldo, const void* positions, const void* inv_freq,
-                                const void* token_req, const void* block_table, int bt_stride, void* k_plane, void* v_plane, int page, int q_heads, int kv_heads, int head_dim, hipStream_t stream) {
+                                const void* token_req, const void* block_table, int bt_stride, void* k_plane, void* v_plane, int page, int q_heads, int kv_heads, int head_dim, int wj, int rows,
+                                hipStream_t stream) {
     TL_REQUIRE(M > 0 && N > 0 && K > 0 && ldx >= K && ldo >= q_heads * head_dim, "gemm_rope_f32: bad sizes M=%d N=%d K=%d", M, N, K);
     TL_REQUIRE(positions && inv_freq && head_dim > 0 && head_dim % 2 == 0 && q_heads >= 0 && kv_heads >= 0, "gemm_rope_f32: needs positions, frequencies and an even head size");
     TL_REQUIRE((k_plane == nullptr) == (v_plane == nullptr) && (!k_plane || (token_req && block_table && page > 0 && bt_stride > 0 && kv_heads > 0)),
@@ -2246,7 +2250,7 @@ extern "C" int tl_gemm_rope_f32(const void* x, const void* w, const void* bias, 
     TL_REQUIRE(N == (q_heads + (k_plane ? 2 * kv_heads : 0)) * head_dim, "gemm_rope_f32: %d output columns do not match the heads", N);
     const F32Pairs pa{N / 2, head_dim / 2, 0, (const int*)positions, (const float*)inv_freq, (const int*)token_req, (const int*)block_table, (float*)k_plane, (float*)v_plane,
                       bt_stride, page > 0 ? page : 1, q_heads, k_plane ? kv_heads : 0};
-    return f32_pairs<F32_ROTATE>(x, w, bias, bias_f32, out, M, K, ldx, ldo, pa, stream);
+    return f32_pairs<F32_ROTATE>(x, w, bias, bias_f32, out, M, K, ldx, ldo, pa, wj, rows, stream);
 }
 
 // out[P, M, N] (float) = partial sums of x w^T over P ranges of K, for a product with too few output

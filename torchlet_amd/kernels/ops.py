@@ -442,12 +442,13 @@ def linear_groups_beside(x: torch.Tensor, weight: torch.Tensor, out: torch.Tenso
     linear(x2, weight2, None, out2)
 
 
-def linear_f32_variant(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, out: torch.Tensor, matrix_cores) -> None:
+def linear_f32_variant(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, out: torch.Tensor, matrix_cores, requests: int = 0, rows: int = 0) -> None:
     """One named kernel of the 32-bit products (for tests and tuning): 0 / False the general tile kernel (``v_fma_f32``),
     1 / True the matrix-core tile kernel (``v_mfma_f32_32x32x2_f32``, K a multiple of 4), 2 and 3 the kernels for few rows
     on multiply-adds (up to 8) and on the matrix cores (``v_mfma_f32_16x16x4_f32``, up to 16), 4 to 6 the matrix-core tile kernel with
     tiles of 64 x 64, 64 x 128 and 128 x 128, 7 and 8 with 64 x 32 and 32 x 32, 9 the rings of
-    slabs for up to 16 rows (K a multiple of 32); all multiply and add in true 32-bit."""
+    slabs for up to 16 rows (K a multiple of 32; ``8 * requests`` weight rows a work-group, of which ``rows`` are used, or as the library deals
+    them); all multiply and add in true 32-bit."""
     M, K = x.shape
     N = weight.shape[0]
     if x.dtype != torch.float32 or weight.dtype != torch.float32 or out.dtype != torch.float32 or out.shape != (M, N) \
@@ -456,7 +457,7 @@ def linear_f32_variant(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor
     bf = _vec(bias, N, "linear bias")
     lib = _lib("gemm")
     _check(lib, lib.tl_gemm_f32_variant(_ptr(x), _ptr(weight), _ptr(bias), c_int(bf), _ptr(out), c_int(M), c_int(N), c_int(K),
-                                        c_int(x.stride(0)), c_int(out.stride(0)), c_int(int(matrix_cores)), _stream()))
+                                        c_int(x.stride(0)), c_int(out.stride(0)), c_int(int(matrix_cores)), c_int(requests), c_int(rows), _stream()))
 
 
 def linear_few_rows_variant(x, weight, bias, out, strips_per_wave: int, waves_along_k: int, rows_per_strip: int = 0) -> None:
@@ -566,9 +567,10 @@ def linear_swiglu(x: torch.Tensor, gate_up: torch.Tensor, out: torch.Tensor, act
                                    c_int(x.stride(0)), c_int(out.stride(0)), c_int(GATE_ACTIVATIONS[activation]), _stream()))
 
 
-def linear_gate_stacked(x: torch.Tensor, gate_up: torch.Tensor, out: torch.Tensor, activation: str = "silu") -> bool:
+def linear_gate_stacked(x: torch.Tensor, gate_up: torch.Tensor, out: torch.Tensor, activation: str = "silu", rings: tuple[int, int] | None = None) -> bool:
     """``out = act(x @ gate.T) * (x @ up.T)`` in float32 with ``gate_up [2 I, K]`` the gate's rows and then the up rows, in one launch: :func:`linear`
-    and :func:`swiglu` for up to 16 rows.  ``False``, and nothing done, for what it is not built for."""
+    and :func:`swiglu` for up to 16 rows.  ``False``, and nothing done, for what it is not built for.  ``rings = (requests, pairs)`` (for tests and tuning): through the rings, so many requests and pairs of
+    rows a work-group (``-1``: as the library deals them)."""
     M, K = x.shape
     I = out.shape[1]
     if not (x.is_cuda and x.dtype == gate_up.dtype == out.dtype == torch.float32 and 0 < M <= 16):
@@ -578,7 +580,8 @@ def linear_gate_stacked(x: torch.Tensor, gate_up: torch.Tensor, out: torch.Tenso
     if activation not in GATE_ACTIVATIONS:
         raise KernelError(f"linear_gate_stacked: the gate's activation is one of {', '.join(GATE_ACTIVATIONS)}, not {activation!r}")
     lib = _lib("gemm")
-    rc = lib.tl_gemm_gate_f32(_ptr(x), _ptr(gate_up), _ptr(out), c_int(M), c_int(I), c_int(K), c_int(x.stride(0)), c_int(out.stride(0)), c_int(GATE_ACTIVATIONS[activation]), _stream())
+    rc = lib.tl_gemm_gate_f32(_ptr(x), _ptr(gate_up), _ptr(out), c_int(M), c_int(I), c_int(K), c_int(x.stride(0)), c_int(out.stride(0)), c_int(GATE_ACTIVATIONS[activation]),
+                              *map(c_int, rings or (0, 0)), _stream())
     if rc == 100:          # not built for this shape
         return False
     _check(lib, rc)
@@ -655,13 +658,14 @@ def linear_rope_cache_write(x: torch.Tensor, weight: torch.Tensor, bias: torch.T
                             q_heads: int, kv_heads: int, head_dim: int, positions: torch.Tensor, inv_freq: torch.Tensor,
                             token_req: torch.Tensor | None = None, block_table: torch.Tensor | None = None,
                             k_plane: torch.Tensor | None = None, v_plane: torch.Tensor | None = None,
-                            page_size: int = 0, pairs: bool = True) -> bool:
+                            page_size: int = 0, pairs: bool = True, rings: tuple[int, int] | None = None) -> bool:
     """The query/key/value projection of a decode step with the rotation and the cache write in
     its epilogue: ``out[:, :q_heads*hd]`` gets the rotated queries; with planes given, ``weight``
     has ``(q_heads + 2 kv_heads) * hd`` rows and rotated keys and values go to their pages.  The
     rows of the query and key heads are in the pair layout (:func:`pair_layout_rows`).  Built
     for bfloat16 and up to 16 rows; returns ``False`` without doing anything for other shapes.
-    ``pairs=False``: the same in float32, the heads' rows as they are (frequency ``j`` turns the elements ``j`` and ``j + head_dim / 2``)."""
+    ``pairs=False``: the same in float32, the heads' rows as they are (frequency ``j`` turns the elements ``j`` and ``j + head_dim / 2``), ``rings`` as :func:`linear_gate_stacked` takes
+    it."""
     M, K = x.shape
     N = weight.shape[0]
     dtype = torch.bfloat16 if pairs else torch.float32
@@ -686,7 +690,7 @@ def linear_rope_cache_write(x: torch.Tensor, weight: torch.Tensor, bias: torch.T
     rc = entry(_ptr(x), _ptr(weight), _ptr(bias), c_int(bf), _ptr(out), c_int(M), c_int(N), c_int(K),
                c_int(x.stride(0)), c_int(out.stride(0)), _ptr(positions), _ptr(inv_freq), _ptr(token_req),
                _ptr(block_table), c_int(bt_stride), _ptr(k_plane), _ptr(v_plane), c_int(page_size),
-               c_int(q_heads), c_int(kv_heads), c_int(head_dim), _stream())
+               c_int(q_heads), c_int(kv_heads), c_int(head_dim), *(() if pairs else map(c_int, rings or (0, 0))), _stream())
     if rc == 100:          # not built for this shape
         return False
     _check(lib, rc)
