@@ -12,10 +12,11 @@ def lib():
     return ctypes.CDLL(str(build.build("gemm", quiet=True)))
 
 
-# 1: 64 x 64, 2: 64 x 128, 3: 128 x 128; a launch has up to 65535 rows of tiles
-@pytest.mark.parametrize("M, N, want", [(100, 3584, 1), (301, 37888, 2), (753, 37888, 3), (65535 * 64, 64, 1), (65535 * 64 + 1, 64, 3), (65535 * 64 + 1, 192, 3), (65535 * 128, 64, 3)])
+# 1: 64 x 64, 2: 64 x 128, 3: 128 x 128, 4: 64 x 32, 5: 32 x 32; a launch has up to 65535 rows of tiles
+@pytest.mark.parametrize("M, N, want", [(65535 * 32, 32, 4), (65535 * 64, 64, 1), (65535 * 64 + 1, 32, 3), (65535 * 64 + 1, 64, 3), (65535 * 64 + 1, 192, 3), (65535 * 128, 64, 3)])
 def test_32_bit_tiles_fit_a_launch(lib, M, N, want):
     assert lib.tl_gemm_f32_tile(c_int(M), c_int(N)) == want
+    assert -(-M // {1: 64, 2: 64, 3: 128, 4: 64, 5: 32}[want]) <= 65535
 
 
 # one row of tiles against wide matrices, measured 10 % and more apart: not 64 x 64 with more work-groups than compute units unless the rows of w lie multiples of 4 KB apart or are short, and with the
@@ -89,7 +90,6 @@ def test_shares_of_the_rings_with_k_split(lib, total, M, K, parts, want):
 
 
 # tiles of blocks of 16 (4: 64 x 32, 5: 32 x 32) beside those of blocks of 32, sizes measured 5 % and more apart from the next
-@pytest.mark.parametrize("M, N, want", [(17, 4608, 5), (33, 2052, 5), (40, 288, 5), (100, 3584, 4), (200, 2048, 4), (64, 5632, 4), (753, 3584, 1), (753, 4608, 2), (301, 37888, 2), (753, 37888, 3),
-                                        (65535 * 32, 32, 4), (65535 * 64 + 1, 32, 3), (65535 * 128, 64, 3)])
+@pytest.mark.parametrize("M, N, want", [(17, 4608, 5), (33, 2052, 5), (40, 288, 5), (100, 3584, 4), (200, 2048, 4), (64, 5632, 4), (753, 3584, 1), (753, 4608, 2), (301, 37888, 2), (753, 37888, 3)])
 def test_32_bit_tiles_of_small_blocks(lib, M, N, want):
-    assert lib.tl_gemm_f32_any_tile(c_int(M), c_int(N)) == want
+    assert lib.tl_gemm_f32_tile(c_int(M), c_int(N)) == want

@@ -533,11 +533,11 @@ static bool gemm_f32_mfma_fits(const void* x, const void* w, int M, int K, int l
 // 17 x 4608 x 3584 65 / 113 / 211 / 45 / 33, 100 x 3584 x 3584 66 / 114 / 214 / 45 / 52, 301 x 3584 x 18944 578 / 586 / 1111 / 600 / 659, 753 x 3584 x 18944 863 / 1084 / 1117 / 1191 / 1443,
 // 753 x 4608 x 3584 225 / 210 / 216 / 267 / 350, 301 x 37888 x 3584 675 / 631 / 816 / 894 / 1164, 753 x 37888 x 3584 1618 / 1472 / 1443 / 2096 / 2744.
 // A size whose rows of tiles are more than a launch has in y is not considered: beyond 4.19 million rows the tiles are 128 high.
-static int f32_tile(int M, int N, int sizes_considered) {
+extern "C" int tl_gemm_f32_tile(int M, int N) {
     static const struct { int bm, bn; double start, round; } sizes[] = {{64, 64, 0.002, 0.0155}, {64, 128, 0.001, 0.0293}, {128, 128, 0.003, 0.0573}, {64, 32, 0.002, 0.0105}, {32, 32, 0.0025, 0.0068}};
     double best = 1e30;
     int tile = 3;
-    for (int t = 0; t < sizes_considered; ++t) {
+    for (int t = 0; t < 5; ++t) {
         const long rows = ((long)M + sizes[t].bm - 1) / sizes[t].bm, tiles = rows * (((long)N + sizes[t].bn - 1) / sizes[t].bn);
         if (rows > 65535) continue;
         const double est = sizes[t].start + sizes[t].round * ((tiles + TL_COMPUTE_UNITS - 1) / TL_COMPUTE_UNITS);
@@ -545,8 +545,6 @@ static int f32_tile(int M, int N, int sizes_considered) {
     }
     return tile;
 }
-extern "C" int tl_gemm_f32_tile(int M, int N) { return f32_tile(M, N, 3); }            // the choice among the blocks of 32 ...
-extern "C" int tl_gemm_f32_any_tile(int M, int N) { return f32_tile(M, N, 5); }        // ... and among all, which a product takes
 
 template <int B, int FMB, int FNB, int STAGES, int WAVES_PER_SIMD, int PHASE>
 static void launch_gemm_f32_tile(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int N, int K, int ldx, int ldo, hipStream_t stream) {
@@ -560,7 +558,7 @@ static void launch_gemm_f32_tile(const void* x, const void* w, const void* bias,
 // `tile`: 0 by the rule above, else one of its sizes (tests cover each; tuning times them).  Two work-groups of the larger tiles (64 and 48 KB) and three of 64 x 64 fit a compute unit.
 static void launch_gemm_f32_mfma(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int N, int K,
                                  int ldx, int ldo, hipStream_t stream, int tile = 0) {
-    if (tile == 0) tile = tl_gemm_f32_any_tile(M, N);
+    if (tile == 0) tile = tl_gemm_f32_tile(M, N);
     auto launch = tile == 1 ? launch_gemm_f32_tile<32, 1, 1, 3, 3, 2> : tile == 2 ? launch_gemm_f32_tile<32, 1, 2, 2, 2, 1> : tile == 3 ? launch_gemm_f32_tile<32, 2, 2, 2, 2, 1>
                 : tile == 4 ? launch_gemm_f32_tile<16, 2, 1, 4, 3, 2> : launch_gemm_f32_tile<16, 1, 1, 6, 3, 2>;
     launch(x, w, bias, bias_f32, out, M, N, K, ldx, ldo, stream);
