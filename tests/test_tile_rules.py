@@ -81,6 +81,27 @@ def test_shares_do_not_hang_on_the_number_of_rows_where_the_order_of_the_sums_ha
                 assert len(plans) == 1, (total, K, halves, even)
 
 
+# 32 bits: gates and rotations by pairs of rows, also in shapes of three requests
+@pytest.mark.parametrize("total, M, K, pairs, want", [(18944, 4, 3584, 1, (4, 15)), (27648, 4, 5120, 1, (6, 22)), (2304, 4, 3584, 1, (3, 9)), (3584, 8, 5120, 1, (4, 14)), (67, 4, 3584, 1, (2, 4)),
+                                                      (37888, 4, 3584, 0, (4, 30)), (152064, 4, 3584, 0, (8, 60)), (3584, 4, 18944, 0, (2, 14)), (4608, 12, 3584, 0, (3, 18)), (512, 16, 512, 0, (1, 8))])
+def test_shares_of_the_rings_in_32_bits(lib, total, M, K, pairs, want):
+    wj, rows = c_int(), c_int()
+    lib.tl_gemm_f32_ring_plan(c_int(total), c_int(M), c_int(K), c_int(pairs), c_int(256), ctypes.byref(wj), ctypes.byref(rows))
+    assert (wj.value, rows.value) == want
+
+
+def test_shares_in_32_bits_do_not_hang_on_the_number_of_rows_where_the_order_of_the_sums_hangs_on_the_shares(lib):
+    for total in list(range(1, 3000, 97)) + list(range(3000, 40000, 523)):
+        for K in (1024, 2048, 4096, 16384):
+            for pairs in (0, 1):
+                plans = set()
+                for M in range(1, 17):
+                    wj, rows = c_int(), c_int()
+                    lib.tl_gemm_f32_ring_plan(c_int(total), c_int(M), c_int(K), c_int(pairs), c_int(256), ctypes.byref(wj), ctypes.byref(rows))
+                    plans.add((wj.value, rows.value))
+                assert len(plans) == 1, (total, K, pairs)
+
+
 # ranges of K: a unit's work-group of eight requests stays alone
 @pytest.mark.parametrize("total, M, K, parts, want", [(3584, 8, 18944, 4, (8, 56)), (4096, 1, 4096, 4, (8, 64)), (5120, 16, 13824, 3, (8, 61)), (2048, 8, 8192, 8, (8, 64)), (2048, 8, 2048, 4, (4, 32))])
 def test_shares_of_the_rings_with_k_split(lib, total, M, K, parts, want):

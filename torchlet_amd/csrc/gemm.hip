@@ -1423,6 +1423,13 @@ extern "C" void tl_gemm_ring_plan(int total, int M, int K, int halves, int units
     *rows = p.rows;
 }
 
+// The same in 32 bits; `pairs`: rows by pairs, `total` of them.
+extern "C" void tl_gemm_f32_ring_plan(int total, int M, int K, int pairs, int units, int* wj, int* rows) {
+    const RingPlan p = plan_ring(total, M, pairs ? 2 : 1, units, false, ring_spread<float>(K), false, pairs != 0);
+    *wj = p.wj;
+    *rows = p.rows;
+}
+
 // One shape of the kernel above (for tests and tuning): 8 wj weight rows a work-group (with `gate`, 1 + the gate's number, half gate and half up rows), `rows` outputs of which
 // are used; parts > 1: K split into ranges of k_per columns, float slabs.  wj 0: as the dispatch would.
 extern "C" int tl_gemm_ring_variant(const void* x, const void* w, const void* bias, int bias_f32, void* out, int M, int N, int K, int ldx, int ldo, int out_f32, int gate, int wj,
