@@ -9,7 +9,8 @@ import pytest
 
 from torchlet_amd.kernels import build
 
-WAIT = 7              # wait states between v_mfma_f32_16x16x32_bf16 (four passes) and another kind of instruction on its result
+# wait states between a matrix instruction and another kind of instruction on its result: four passes, and eight in 32 bits
+WAITS = {"v_mfma_f32_16x16x32_bf16": 7, "v_mfma_f32_16x16x4_f32": 10}
 
 
 def _registers(operands):
@@ -42,11 +43,12 @@ def early_uses(body):
     for i, (_, text, _) in enumerate(body):
         if not text.startswith("v_mfma"):
             continue
+        wait = WAITS[text.split(None, 1)[0]]
         result = _registers(text.split(None, 1)[1].split(",")[0])
         ways, best = [(i + 1, 0)], {}
         while ways:
             p, waited = ways.pop()
-            if p >= len(body) or waited >= WAIT or best.get(p, WAIT) <= waited:
+            if p >= len(body) or waited >= wait or best.get(p, wait) <= waited:
                 continue
             best[p] = waited
             _, other, target = body[p]
@@ -75,7 +77,18 @@ def test_the_check_sees_the_short_path():
     assert early_uses(loop) == []
 
 
-@pytest.mark.parametrize("library,kernel,instances", [("gemm", "gemm_ring_kernel", 60), ("experts", "experts_ring_kernel", 2)])
+def test_the_check_waits_longer_for_32_bit_products():
+    line = [(0, "v_mfma_f32_16x16x4_f32 v[0:3], v8, v9, 0", 0), (8, "s_nop 6", 0), (12, "v_add_f32_e32 v4, v3, v4", 0), (16, "s_endpgm", 0)]
+    assert early_uses(line) == [(line[0][1], line[2][1])]
+    line[1] = (8, "s_nop 8", 0)
+    assert early_uses(line) == [(line[0][1], line[2][1])]
+    line[1] = (8, "s_nop 9", 0)
+    assert early_uses(line) == []
+
+
+# instances in bfloat16 and in 32 bits: of the latter up to 8 and up to 16 rows, six shapes of the plain product, five of the gate and five of the rotation
+@pytest.mark.parametrize("library,kernel,instances", [("gemm", "gemm_ring_kernel", {"v_mfma_f32_16x16x32_bf16": 132, "v_mfma_f32_16x16x4_f32": 32}),
+                                                      ("experts", "experts_ring_kernel", {"v_mfma_f32_16x16x32_bf16": 2})])
 def test_results_are_through_before_they_are_read(library, kernel, instances, tmp_path):
     objdump = Path(build.hipcc()).resolve().parent.parent / "llvm/bin/llvm-objdump"
     if not objdump.exists():
@@ -86,8 +99,10 @@ def test_results_are_through_before_they_are_read(library, kernel, instances, tm
     subprocess.run([objdump, "--offloading", "lib.so"], cwd=tmp_path, check=True, capture_output=True)
     code, = tmp_path.glob(f"*{build.ARCH}*")
     listing = subprocess.run([objdump, "-d", "--no-show-raw-insn", code], check=True, capture_output=True, text=True).stdout
-    names, bad = [], []
+    found, bad = dict.fromkeys(instances, 0), []
     for name, body in _functions(listing, kernel):
-        names.append(name)
+        for instruction in {text.split(None, 1)[0] for _, text, _ in body if text.startswith("v_mfma")}:
+            found[instruction] += 1
         bad += [(name, *pair) for pair in early_uses(body)]
-    assert len(names) >= instances and not bad, bad[:4]
+    assert not bad, bad[:4]
+    assert all(found[instruction] >= least for instruction, least in instances.items()), found
