@@ -44,7 +44,7 @@ def test_rotation_and_cache_write(M, heads, kv_heads, hd, K, writes, page):
     x, w, b = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda") / K ** 0.5, torch.randn(N, generator=g, device="cuda")
     freq = torch.rand(hd // 2, generator=g, device="cuda")
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
-    positions, req, table = i32([(17 * m) % 40 for m in range(M)]), i32(list(range(M))), (torch.randperm(M * 14) + 1).view(M, 14).int().cuda()
+    positions, req, table = i32([(17 * m) % 40 for m in range(M)]), i32(list(range(M))), (torch.randperm(M * 14, generator=torch.Generator().manual_seed(M)) + 1).view(M, 14).int().cuda()
     if M > 1:
         table[M - 1] = 0                      # a padding row: its keys and values are dropped
     seen = []

@@ -5,6 +5,10 @@
 
 #include "common.h"
 
+// The compute units of the GPU the library runs on: the caller tells it once; 256, the MI355X's, until then.
+static int g_compute_units = 256;
+extern "C" void tl_elementwise_set_compute_units(int n) { if (n > 0) g_compute_units = n; }
+
 // ------------------------------------------------------------------ embedding
 // out[c, t, :] = float(table[ids[t], :]) * scale (+ float(pos_table[positions[t], :])) for every copy c; the residual stream is 32-bit.
 template <typename T>
@@ -123,8 +127,9 @@ __device__ __forceinline__ void add_slab_pairs(const float* src, size_t stride, 
 // again, kept out of sums and stores.
 // (us after the kernel that wrote the slabs, kind at run time -> by template: add_rmsnorm, 8 rows of 3584 with four slabs 4.0 -> 3.4, one row of 2048 with eight 3.75 -> 2.9, 16 of 5120
 // with three 4.5 -> 4.1, 512 of 5120 with three 15.9 -> 14.6; scaled_add_rmsnorm, one row of 2048 2.4 -> 2.1, 4 of 4096 with four slabs 3.6 -> 3.2, 2048 of 2048 11.3 -> 10.3; sandwich_norm, 16 of 2048
-// with four 3.7 -> 3.3.  What is asked for ahead takes registers: with more rows than compute units and many slabs fewer rows share a unit, and 2048 of 2048 with four slabs took
-// add_rmsnorm 19.9 instead of 18.6: late there.)
+// with four 3.7 -> 3.3.  What is asked for ahead takes registers, and with more rows than compute units fewer of them share a unit: there five slabs and more are late (2048 of 2048 with eight,
+// ahead / late, add_rmsnorm 27.7 / 26.9, scaled_add_rmsnorm 28.2 / 27.2; 2048 of 1024 15.8 / 14.7, 16.1 / 14.4; of all widths 1024 to 8192 and 257 to 2048 rows alike within a hundredth), but not four
+// (512 of 4096 8.5 / 9.0, 8.7 / 9.4; 512 of 3584 6.7 / 7.0, 6.8 / 7.3; 2048 of 2048 17.2 / 17.1, 17.8 / 17.0).)
 #define BRANCH_NONE (-1)
 #define BRANCH_ANY 9
 #define BRANCH_LATE 10
@@ -226,7 +231,7 @@ static void launch_add_rmsnorm(float* residual, const void* pending, int parts, 
     const bool aligned = hidden % 4 == 0 && ((uintptr_t)residual % 16) == 0 && ((uintptr_t)out % 16) == 0 &&
                          ((uintptr_t)pending % 16) == 0 && ((uintptr_t)weight % 16) == 0;
     dim3 grid(out_rows);
-    const int late = out_rows > 256 ? 5 : INT_MAX;
+    const int late = out_rows > g_compute_units ? 5 : INT_MAX;
 #define TL_AR_W(W, IT, THREADS, PC) add_rmsnorm_reg_kernel<T, W, IT, PC><<<grid, THREADS, 0, stream>>>(residual, pending, parts, part_stride, (const W*)weight, eps, gain, out, rows, hidden)
 #define TL_AR_1(PC) do { if (weight_f32) TL_AR_W(float, 1, 256, PC); else TL_AR_W(bf16_t, 1, 256, PC); } while (0)
 #define TL_AR_2(PC) do { if (weight_f32) TL_AR_W(float, 2, threads, PC); else TL_AR_W(bf16_t, 2, threads, PC); } while (0)
@@ -681,7 +686,7 @@ static void launch_scaled_add_rmsnorm(float* residual, const void* pending, int 
 #define TL_SAR_2(PC) do { if (weight_f32) TL_SAR_W(float, 2, PC); else TL_SAR_W(bf16_t, 2, PC); } while (0)
 #define TL_SAR_3(PC) do { if (weight_f32) TL_SAR_W(float, 3, PC); else TL_SAR_W(bf16_t, 3, PC); } while (0)
 #define TL_SAR_4(PC) do { if (weight_f32) TL_SAR_W(float, 4, PC); else TL_SAR_W(bf16_t, 4, PC); } while (0)
-    const int threads = hidden <= 1024 ? 256 : hidden <= 8192 ? 512 : 1024, late = rows > 256 ? 5 : INT_MAX;
+    const int threads = hidden <= 1024 ? 256 : hidden <= 8192 ? 512 : 1024, late = rows > g_compute_units ? 5 : INT_MAX;
     if (aligned && hidden <= 2048) TL_BRANCH(pending, parts, late, true, TL_SAR_1);
     else if (aligned && hidden <= 4096) TL_BRANCH(pending, parts, late, true, TL_SAR_2);
     else if (aligned && hidden <= 6144) TL_BRANCH(pending, parts, late, false, TL_SAR_3);
@@ -1790,7 +1795,7 @@ extern "C" int tl_settle_shift(const void* residual, void* settled, const void* 
     if (hidden % 4 == 0 && bits % 16 == 0) {
         const RowPlan plan = plan_row(hidden);
         // (where a unit has more than one token the other tokens' requests hide the trips, and the mixes' vectors ahead take registers: 1303 tokens 16.2 -> 18.7 us)
-        if (run == 1 && tokens <= 256 && plan.pieces == 1 && count <= MIXES_AHEAD && (!post || post_n == hidden)) {
+        if (run == 1 && tokens <= g_compute_units && plan.pieces == 1 && count <= MIXES_AHEAD && (!post || post_n == hidden)) {
             const int tail4 = (uintptr_t)state % 16 == 0 && slot_stride % 4 == 0 && tail_off % 4 == 0;
 #define TL_SF_F(PC) settle_shift_few_kernel<float, PC><<<tokens, plan.threads, 0, stream>>>(a, tail4, (float*)mixes)
 #define TL_SF_B(PC) settle_shift_few_kernel<bf16_t, PC><<<tokens, plan.threads, 0, stream>>>(a, tail4, (bf16_t*)mixes)

@@ -48,6 +48,8 @@ def _lib(name: str) -> ctypes.CDLL:
             lib.tl_blocks_floats.restype = ctypes.c_long
         if name == "recurrent" and torch.cuda.is_available():
             lib.tl_mlstm_set_compute_units(c_int(compute_units()))
+        if name == "elementwise" and torch.cuda.is_available():
+            lib.tl_elementwise_set_compute_units(c_int(compute_units()))
         if name == "experts" and torch.cuda.is_available():
             lib.tl_experts_set_compute_units(c_int(compute_units()))
     return lib
