@@ -1042,7 +1042,7 @@ static int launch_delta_scan(const void* qkv, const void* gates, const void* hea
 // order of every sum.  A work-group has a key head of a request with the value heads that share it, so the channels it convolves, and the tail it moves on, are its own.  It asks for
 // its states first, sixteen lanes a column and CG columns to each; while they are on their way the convolution's inputs arrive, its threads make q, k, v and the heads' gates and leave them in
 // shared memory, then all lanes move the states, and the first ones take the outputs through the norm.  What bounds it: a compute unit draws the states of its work-group at 64 bytes a clock, 128 KB
-// for two value heads of 128 x 128, and gives them back as fast.  8 requests, 16 heads of 128 x 128 over 8: 4.5 + 6.8 + 4.1 us in three launches, 9.3 in one; in a captured step, gaps included, 1
+// for two value heads of 128 x 128, and gives them back as fast.  8 requests, 16 heads of 128 x 128 over 8: 4.5 + 6.8 + 4.1 us in three launches, 9.3 in one; calls one behind the other, gaps included, 1
 // request 7.9 and 6.6 us, 8 10.7 and 7.6, 32 20.6 and 12.2, 64 32.2 and 27.2, 128 52.5 and 50.6 (198 registers leave a unit one work-group; it is ahead at every size measured, up to 3072 of them).
 // Built for key heads of 64 or 128 channels with up to 256 value channels between them.
 #define DT_THREADS 512                          // (sixteen waves leave a wave 128 registers, which 256 columns of 128 do not fit)
@@ -2017,9 +2017,9 @@ extern "C" int tl_wkv_scan(const void* rkv, int ld, int k_off, int v_off, const 
 // The same with what stands before and behind it, for steps of one token a request: the decays are made from their low-rank sums (channel_decay above), and the output goes through the norm of its
 // head and the gate (gated_head_norm) before it is stored, all in the sums' order there.  A work-group has a whole head of a request: sixteen lanes a column and CG columns to each, whose states
 // are all requested at the start, beside the token's numbers and the matrix of the decays; what a step waits for is then one trip to the state and the chain of tanh, the 64 products of a decay, the
-// recurrence and the norm.  In three launches (decays, scan by four work-groups a head, norm) 16 requests with 32 heads of 64 x 64 took 6.8 + 9.2 + 4.1 us, in one 11.9; in a captured step, gaps
-// included, 12.4 and 9.7 (1 request 8.3 and 7.8).  Work-groups hold dim x vdim numbers of state, up to 128 x 128, in 169 to 272 registers: two of them share a compute unit, or none where both sizes
-// are above 64, and where more than that queue the three launches, which deal a head's columns to several, are the faster ones (32 requests 17.4 and 17.6, 64 25.9 and 34.5).
+// recurrence and the norm.  In three launches (decays, scan by four work-groups a head, norm) 16 requests with 32 heads of 64 x 64 took 6.8 + 9.2 + 4.1 us, in one 11.9.  Work-groups hold
+// dim x vdim numbers of state, up to 128 x 128, in 169 to 272 registers: two of them share a compute unit, or none, and where more than a round or two of those queue the three launches, which deal a
+// head's columns to several, are the faster ones (a decode step's call, 16 requests 6.8 us less in one launch, 32 0.8 less, 64 6.0 more).
 template <typename T, int RPL, int CG>
 __global__ void __launch_bounds__(256)
 wkv_token_kernel(const T* __restrict__ rkv, int ld, int k_off, int v_off, int gate_off, const float* __restrict__ z, const float* __restrict__ w2t, const float* __restrict__ w0, int rank,

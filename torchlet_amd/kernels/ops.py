@@ -1429,12 +1429,12 @@ def wkv_scan(rkv: torch.Tensor, k_off: int, v_off: int, decay: torch.Tensor, bon
 
 def wkv_token_pays(requests: int, heads: int, dim: int, vdim: int, rank: int) -> bool:
     """Whether a step of one token a request is faster through :func:`wkv_token` than through the three launches it stands for (which leave the same bits).  A work-group
-    has a whole head, and a compute unit has two of them at once (one where both sizes are above 64): beyond that they queue, where the three launches deal a head to several.  Wide columns
-    want half the units busy, and only the first 64 rows of the decays' matrix are requested ahead.  Measured (us, three launches / one): 32 heads of 64 x 64 and rank 64, 1 request 8.3 /
-    7.8, 16 12.4 / 9.7, 32 17.4 / 17.6, 64 25.9 / 34.5; 20 requests 13.0 / 15.1; 16 heads of 128 x 128, 1 request 8.9 / 9.8, 4 9.8 / 10.2, 8 11.7 / 10.7, 16 16.1 / 11.6, 20 17.8 / 20.4;
-    32 of 64 x 128, 2 requests 8.8 / 9.3, 4 9.8 / 9.6, 16 16.3 / 12.2; rank 80, 4 requests of 32 heads 9.0 / 9.7; rank 128, 1 request 9.3 / 13.8, 16 13.6 / 15.4."""
-    groups, units = requests * heads, compute_units()
-    return rank <= 64 and groups <= (units if min(dim, vdim) > 64 else 2 * units) and (vdim <= 64 or groups >= units // 2)
+    has a whole head, and a compute unit has two of them at once (one where both sizes are 128): beyond a round or two they queue, where the three launches deal a head to several; and only the
+    first 64 rows of the decays' matrix are requested ahead.  Measured in decode steps of a whole model (width 2048, captured; us a call that the three launches take more): 32 heads of 64 x 64,
+    rank 64, 1 request 4.1, 16 6.8, 24 0.3, 32 0.8, 40 -7.9, 64 -6.0; 64 heads, 8 requests 6.6, 16 -0.4, 32 -6.5, 64 -20; 48 heads, 16 requests 0.1, 32 -3.2; heads of 32 x 32, 512 of them 4.1,
+    1024 1.2 and -1.6, 2048 -11; 16 heads of 128 x 128, 1 request 2.7, 16 6.8, 32 5.0, 64 -2.0; 24 of 96 x 96, 16 requests 0.05, 32 -1.6; rank 80 0.4 to -1.4 up to 4 requests, 96 -6, 128 -15.  (Alone, one
+    call after the other, the three launches look better by 2 to 4 us: their starts then overlap.)"""
+    return rank <= 64 and requests * heads <= (2 if max(dim, vdim) > 64 else 4) * compute_units()
 
 
 def wkv_token(proj: torch.Tensor, k_off: int, v_off: int, gate_off: int, z: torch.Tensor, w2t: torch.Tensor, w0: torch.Tensor, bonus: torch.Tensor, state: torch.Tensor,
