@@ -33,8 +33,8 @@ def test_tiles_of_products_with_few_rows(lib, M, N, K, gated, ahead):
 
 # 32 bits, 2: multiply-adds, 3: matrix cores behind a copy of x, 9: rings; one and two rows stay with the multiply-adds wherever the rings, which take as long for one row as for eight, are behind
 @pytest.mark.parametrize("M, N, K, want", [
-    (1, 1024, 1024, 2), (1, 2048, 2048, 2), (1, 32768, 1024, 2), (1, 22016, 4096, 2), (1, 8192, 6144, 2), (1, 1536, 8192, 2), (1, 2048, 3584, 2), (1, 2560, 3584, 9), (1, 4608, 3584, 9), (1, 4096, 8192, 9),
-    (1, 2048, 18944, 9), (2, 1024, 1024, 2), (2, 2048, 2048, 2), (2, 7168, 4096, 2), (2, 2560, 2560, 2), (2, 3584, 2560, 9), (2, 4608, 3584, 9), (2, 4608, 5120, 9), (2, 1024, 6848, 2),
+    (1, 1024, 1024, 2), (1, 2048, 2048, 2), (1, 32768, 1024, 2), (1, 22016, 4096, 2), (1, 8192, 6144, 2), (1, 1536, 8192, 2), (1, 2048, 3584, 2), (1, 37888, 3584, 2), (1, 16384, 8192, 9), (1, 2560, 3584, 9), (1, 4608, 3584, 9), (1, 4096, 8192, 9),
+    (1, 2048, 18944, 9), (2, 1024, 1024, 2), (2, 2048, 2048, 2), (2, 7168, 4096, 2), (2, 2560, 2560, 2), (2, 55296, 5120, 2), (2, 10240, 5120, 9), (2, 3584, 2560, 9), (2, 4608, 3584, 9), (2, 4608, 5120, 9), (2, 1024, 6848, 2),
     (3, 1024, 1024, 9), (4, 2048, 2048, 9), (8, 1000, 2048, 2), (8, 2048, 992, 2), (8, 2048, 1028, 2), (9, 64, 96, 9), (16, 4100, 1028, 3)])
 def test_32_bit_products_of_few_rows_go_where_they_were_faster(lib, M, N, K, want):
     assert lib.tl_gemm_f32_few_rows_choice(c_int(M), c_int(N), c_int(K)) == want

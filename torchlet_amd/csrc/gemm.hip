@@ -1315,15 +1315,17 @@ static bool ring_fits_f32(const void* x, const void* w, int M, int K, int ldx) {
 // 454 / 366; 16 rows 25 / 15.7, 131 / 100, 112 / 54, 482 / 374, 512 x 512 4.3 / 3.2; 2048 x 2048 4 rows 8.0 / 6.6, 8 rows 12.4 / 6.7.  Narrow matrices want more work-groups than
 // these have (4 rows, 256 x 2048 5.2 / 5.5, 64 x 4096 7.5 / 8.3).
 // A ring takes as long for one row as for eight, the multiply-adds do not: one and two rows go to the rings where these are ahead of both, deep matrices, deeper ones where the rows lie multiples of 4 KB
-// apart, and no small ones, which come out of a cache and want their one trip short (one row, 1024 x 1024 3.0 / 4.3, 2048 x 2048 6.0 / 6.6, out of a cache 3.9 / 5.9, 8192 x 1024 8.1 / 9.4, 32768 x 1024
-// 23.4 / 28.5, 22016 x 4096 62 / 66, 3584 x 3584 11.7 / 11.4, 4608 x 3584 15.2 / 13.7, 4096 x 8192 30.0 / 26.2, 8192 x 8192 53 / 49; two rows, 1024 x 1024 3.5 / 4.3, 4096 x 3584 0.86, 2560 x 2560
-// 0.85, 7168 x 4096 1.18, 6144 x 5120 0.93 of the multiply-adds' time; 16 widths by 18 depths measured).
+// apart, and neither wide ones nor small ones, which come out of a cache and want their one trip short (one row, 1024 x 1024 3.0 / 4.3, 2048 x 2048 6.0 / 6.6, out of a cache 3.9 / 5.9, 8192 x 1024 8.1 / 9.4, 32768 x 1024
+// 23.4 / 28.5, 22016 x 4096 62 / 66, 37888 x 3584 89 / 93, 3584 x 3584 11.7 / 11.4, 4608 x 3584 15.2 / 13.7, 4096 x 8192 30.0 / 26.2, 8192 x 8192 53 / 49; two rows, 1024 x 1024 3.5 / 4.3, 4096 x 3584 0.86, 2560 x 2560
+// 0.85, 7168 x 4096 1.18, 6144 x 5120 0.93 of the multiply-adds' time; 16 widths by 18 depths measured).  Whole passes of one and two requests of fifteen models (ms, the
+// rings from 1024 x 1024 on / never / by this rule): one request, width 5120 26.0 / 25.1 / 24.8, 3584 14.6 / 14.5 / 14.4, 4096 12.2 / 12.1 / 11.8, 2048 6.20 / 5.96 / 5.93; two, 5120 28.1 / 27.6 / 27.1, 3584
+// 15.6 / 15.7 / 15.4, 4096 13.1 / 13.3 / 12.8, 2048 6.24 / 6.35 / 6.12; nowhere behind either by more than two runs differ.
 // The sums' error against 64 bits (relative): K 2048 1.2e-7 / 1.0e-7, 3584 1.5e-7 / 1.1e-7, 18944 3.1e-7 / 1.8e-7, above 8 rows
 // 3.8e-7 / 1.1e-7; at 512 columns up to 8 rows 0.87e-7 / 0.9e-7, and so short sums stay where they are.
 static bool ring_pays_f32(int M, int N, int K) {
     if (M > 2) return M > 8 || (K >= 1024 && N >= 1024);
     const bool apart = K % 1024 == 0;
-    return (long)N * K >= 9000000 && (M == 1 ? N >= 2048 && K >= (apart ? 8192 : 3584) : N >= 1536 && K >= (apart ? 5120 : 2560));
+    return (long)N * K >= 9000000 && (N <= 10240 || K >= 8192) && (M == 1 ? N >= 2048 && K >= (apart ? 8192 : 3584) : N >= 1536 && K >= (apart ? 5120 : 2560));
 }
 // Which kernel a 32-bit product of up to 16 rows gets whose operands are aligned, by its number in tl_gemm_f32_variant: 9 the rings, 2 multiply-adds, 3 the matrix cores behind a copy of x.  The
 // last two part at 8 rows, where a row more costs a multiply-add a weight or nothing (the four products of a 7B layer, us, 2 / 3: 4 rows 216 / 241, 8 rows 274 / 265, 16 rows 425 / 300).
